@@ -136,6 +136,7 @@ SYMBOLS = {
     'fa_get_clock_rate_khz': (ctypes.c_int, [ctypes.c_void_p]),
     'fa_probe_mfma_rate': (ctypes.c_int, [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p,
                                           ctypes.c_void_p, ctypes.c_void_p]),
+    'fa_write_words': (ctypes.c_int, [ctypes.c_void_p, P(ctypes.c_uint32), ctypes.c_int32, ctypes.c_void_p]),
     'fa_hip_get_last_error': (ctypes.c_int, []),
     'fa_hip_device_synchronize': (ctypes.c_int, []),
 }

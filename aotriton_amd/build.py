@@ -1,4 +1,5 @@
-"""Builds libaotriton_amd.so in-tree with hipcc for gfx950 (cross-compiles without a GPU).
+"""Builds libaotriton_amd.so (hipcc for gfx950, cross-compiles without a GPU) and _torch_host.so (the
+native host path between PyTorch and the library, host code only) in-tree.
 
 Usage: python -m aotriton_amd.build [-j N] [--force]
 """
@@ -14,6 +15,8 @@ CSRC = os.path.join(HERE, 'csrc')
 ROOT = os.path.dirname(HERE)
 OBJ = os.path.join(CSRC, 'obj')
 LIB = os.path.join(HERE, 'libaotriton_amd.so')
+HOST_SRC = os.path.join(CSRC, 'torch', 'host.cpp')
+HOST_LIB = os.path.join(HERE, '_torch_host.so')
 HIPCC = os.environ.get('HIPCC', '/opt/rocm/bin/hipcc')
 
 COMMON = [
@@ -52,25 +55,51 @@ def sources():
     return out
 
 
-def headers():
-    hs = [os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith('.h')]
-    hs.append(os.path.join(ROOT, 'include', 'aotriton_amd', 'flash.h'))
-    hs.append(os.path.join(ROOT, 'include', 'aotriton_amd', 'probe.h'))
-    return hs
+def _inputs(path, obj):
+    """The files a compilation read, from the dependency file next to its object; None without one."""
+    try:
+        text = open(obj + '.d').read()
+    except OSError:
+        return None
+    names = text.replace('\\\n', ' ').split(':', 1)[-1].split()
+    return [path] + [n for n in names if not n.startswith('/opt/')]
 
 
 def _compile(unit, force):
     src, defines, objname = unit
     obj = os.path.join(OBJ, objname)
     path = os.path.join(CSRC, src)
-    newest = max(os.path.getmtime(p) for p in [path] + headers())
-    if not force and os.path.exists(obj) and os.path.getmtime(obj) >= newest:
+    inputs = _inputs(path, obj)
+    if (not force and inputs and os.path.exists(obj) and all(os.path.exists(p) for p in inputs) and
+            os.path.getmtime(obj) >= max(os.path.getmtime(p) for p in inputs)):
         return obj, '', 0
-    cmd = [HIPCC] + COMMON + EXTRA.get(src, []) + defines + ['-x', 'hip', '-c', path, '-o', obj]
+    cmd = [HIPCC] + COMMON + EXTRA.get(src, []) + defines + ['-MD', '-MF', obj + '.d', '-x', 'hip', '-c', path, '-o', obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     # the host pass does not know the packed-fp32 feature name; that note is noise
     err = '\n'.join(l for l in r.stderr.splitlines() if 'packed-fp32-ops' not in l)
     return obj, err, r.returncode
+
+
+def build_host(force=False):
+    """The Python extension over torch's C++ API.  It links against the library next to it."""
+    newest = max(os.path.getmtime(p) for p in [HOST_SRC, os.path.join(ROOT, 'include', 'aotriton_amd', 'flash.h')])
+    if not force and os.path.exists(HOST_LIB) and os.path.getmtime(HOST_LIB) >= newest:
+        return HOST_LIB
+    import sysconfig
+    import torch
+    from torch.utils import cpp_extension
+    includes = cpp_extension.include_paths('cuda') + [sysconfig.get_paths()['include'], os.path.join(ROOT, 'include')]
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), 'lib')
+    cmd = ['g++', '-O2', '-std=c++17', '-fPIC', '-shared', '-fvisibility=hidden', '-D__HIP_PLATFORM_AMD__=1', '-DUSE_ROCM=1',
+           f'-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}', '-Wno-deprecated-declarations',
+           *[x for i in includes for x in ('-isystem', i)], HOST_SRC, '-o', HOST_LIB,
+           '-L' + HERE, '-laotriton_amd', '-Wl,-rpath,$ORIGIN', '-L' + torch_lib, '-ltorch_python', '-ltorch', '-ltorch_cpu',
+           '-ltorch_hip', '-lc10_hip', '-lc10']
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        sys.stderr.write(r.stderr)
+        raise RuntimeError('g++ failed on ' + HOST_SRC)
+    return HOST_LIB
 
 
 def build(jobs=8, force=False, verbose=True):
@@ -91,6 +120,7 @@ def build(jobs=8, force=False, verbose=True):
     if r.returncode != 0:
         sys.stderr.write(r.stderr)
         raise RuntimeError('link failed')
+    build_host(force)
     return LIB
 
 

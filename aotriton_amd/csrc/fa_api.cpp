@@ -560,6 +560,11 @@ int fa_probe_mfma_rate(int32_t random_operands, int32_t num_workgroups, int32_t 
                                 reinterpret_cast<unsigned long long*>(clocks), stream);
 }
 
+int fa_write_words(void* dst, const uint32_t* words, int32_t count, void* hip_stream) {
+  if (count < 0 || (count > 0 && (dst == nullptr || words == nullptr))) return FA_ERROR_INVALID_VALUE;
+  return (int)fa::run_write_words(static_cast<uint32_t*>(dst), words, count, static_cast<hipStream_t>(hip_stream));
+}
+
 int fa_hip_get_last_error(void) { return (int)hipGetLastError(); }
 int fa_hip_device_synchronize(void) { return (int)hipDeviceSynchronize(); }
 

@@ -93,6 +93,27 @@ hipError_t run_repack(int elem_bytes, bool unpack, const RepackArgs& a, hipStrea
   return hipGetLastError();
 }
 
+// A few words of the host (Philox seeds, the offsets of packed sequences) to device memory: they
+// travel in the kernel's argument block, so nothing is pinned, copied through a staging buffer or
+// waited for (a copy from pageable memory takes 20-30 us and synchronises).
+constexpr int kWordsPerLaunch = 240;
+struct Words { uint32_t w[kWordsPerLaunch]; };
+__global__ void write_words_kernel(uint32_t* dst, int count, const Words a) {
+  if ((int)threadIdx.x < count) dst[threadIdx.x] = a.w[threadIdx.x];
+}
+
+hipError_t run_write_words(uint32_t* dst, const uint32_t* words, int count, hipStream_t s) {
+  Words a{};
+  for (int done = 0; done < count; done += kWordsPerLaunch) {
+    const int n = count - done < kWordsPerLaunch ? count - done : kWordsPerLaunch;
+    for (int i = 0; i < n; ++i) a.w[i] = words[done + i];
+    hipLaunchKernelGGL(write_words_kernel, dim3(1), dim3(256), 0, s, dst + done, n, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
 // Register-only loop of v_mfma_f32_32x32x16_bf16 (4 independent accumulators per wave, 8 waves
 // per CU): what the matrix pipe sustains on this machine, on constant operands or on operands
 // with random mantissas (the clock under load depends on the data).  clk[0] = shader cycles,

@@ -7,6 +7,9 @@ positional entry points (attn_fwd / attn_bwd / attn_bwd_fused /
 attn_fwd_compact_varlen / attn_bwd_compact_varlen) as thin wrappers that fill the
 v3 params.  Same names, argument meaning and error behaviour (hipError_t return).
 """
+import torch  # noqa: F401  (its libraries come first: the extension links them)
+
+from . import _torch_host
 from .pyaotriton import (T0, T1, T2, T4, DType, Stream, hipError_t, get_name_suffix,  # noqa: F401
                          hipGetLastError, hipDeviceSynchronize, lazy_tensor)
 from .pyaotriton.v2.flash import debug_simulate_encoded_softmax as fa_debug_simulate_encoded_softmax
@@ -93,6 +96,25 @@ def _stream():
     return Stream()
 
 
+def _native(call, *args):
+    """A call of the native host path (csrc/torch/host.cpp): hipError_t, or None where some argument is
+    not a plain tensor of the expected rank; the views below then take it or report it."""
+    rc = call(*args)
+    return _SUCCESS if rc == 0 else None if rc is None else hipError_t(rc)
+
+
+_SUCCESS = hipError_t.hipSuccess
+
+
+def _options(extargs):
+    return (-1, False) if extargs is None else (extargs.force_backend_index, extargs.deterministic)
+
+
+def _stream_arg(stream):
+    """-1: torch's current stream, looked up natively."""
+    return -1 if stream is None else stream.native()
+
+
 def _fill_fwd(params, q, k, v, b, sm_scale, M, o, dropout_p, philox_seed, philox_offset1, philox_offset2,
               philox_seed_output, philox_offset_output, encoded_softmax, causal, atomic):
     params.Q = mk_aotensor(q)
@@ -118,6 +140,11 @@ def attn_fwd(q, k, v, b, sm_scale, M, o, dropout_p, philox_seed, philox_offset1,
              extargs=None, stream=None):
     """aotriton_flash.py:141-196 (also the v2 positional attn_fwd: is_causal -> windowed
     with top-left sentinels)."""
+    rc = _native(_torch_host.attn_fwd, q, k, v, b, sm_scale, M, o, dropout_p, philox_seed, philox_offset1,
+                 philox_offset2, philox_seed_output, philox_offset_output, encoded_softmax, *translate_causal(causal),
+                 atomic, None, None, 0, 0, None, None, 0, *_options(extargs), _stream_arg(stream))
+    if rc is not None:
+        return rc
     params = fa_forward_op_params()
     _fill_fwd(params, q, k, v, b, sm_scale, M, o, dropout_p, philox_seed, philox_offset1, philox_offset2,
               philox_seed_output, philox_offset_output, encoded_softmax, causal, atomic)
@@ -130,6 +157,12 @@ def attn_fwd_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqle
                     philox_offset1, philox_offset2, philox_seed_output, philox_offset_output,
                     encoded_softmax, causal, atomic, varlen_type, extargs=None, stream=None):
     """aotriton_flash.py:277-335."""
+    rc = _native(_torch_host.attn_fwd, q, k, v, b, sm_scale, M, o, dropout_p, philox_seed, philox_offset1,
+                 philox_offset2, philox_seed_output, philox_offset_output, encoded_softmax, *translate_causal(causal),
+                 atomic, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, seq_strides_q, seq_strides_k,
+                 IVARLEN_TYPE[varlen_type], *_options(extargs), _stream_arg(stream))
+    if rc is not None:
+        return rc
     params = fa_forward_op_params()
     _fill_fwd(params, q, k, v, b, sm_scale, M, o, dropout_p, philox_seed, philox_offset1, philox_offset2,
               philox_seed_output, philox_offset_output, encoded_softmax, causal, atomic)
@@ -169,7 +202,7 @@ def _fill_bwd(params, q, k, v, b, sm_scale, o, dout, dq, dk, dv, db, dq_acc, L, 
     params.DB = mk_aotensor(db, if_empty_then_like=q)
     params.DQ_ACC = dq_acc
     params.L = mk_aotensor(L)
-    if delta is not None and not hasattr(delta, 'c'):      # a plain tensor: wrap as eager
+    if delta is not None and not isinstance(delta, lazy_tensor.LazyTensor2):      # a plain tensor: wrap as eager
         delta = lazy_tensor.eager_delta(mk_aotensor(delta))
     params.D = delta
     params.dropout_p = float(dropout_p)
@@ -179,10 +212,23 @@ def _fill_bwd(params, q, k, v, b, sm_scale, o, dout, dq, dk, dv, db, dq_acc, L, 
     params.causal_type, params.window_left, params.window_right = translate_causal(causal)
 
 
+def _delta_arg(delta):
+    """(tensor or None, whether the native path allocates delta on demand).  A lazy tensor that stands
+    for an allocation needs no Python callback there; any other lazy tensor goes through the views."""
+    if isinstance(delta, lazy_tensor.LazyTensor2):
+        return (None, True) if delta.on_demand else (delta, False)
+    return delta, False
+
+
 def attn_bwd(q, k, v, b, sm_scale, o, dout, dq, dk, dv, db, dq_acc, L, delta, dropout_p, philox_seed,
              philox_offset1, philox_offset2, causal, extargs=None, stream=None):
     """aotriton_flash.py:198-263.  ``delta`` is a lazy tensor (lazy_delta) or a
     plain fp32 tensor; ``dq_acc`` may be None."""
+    rc = _native(_torch_host.attn_bwd, q, k, v, b, sm_scale, o, dout, dq, dk, dv, db, L, *_delta_arg(delta), dropout_p,
+                 philox_seed, philox_offset1, philox_offset2, *translate_causal(causal), None, None, 0, 0, None, None, 0,
+                 *_options(extargs), _stream_arg(stream))
+    if rc is not None:
+        return rc
     params = fa_backward_op_params()
     _fill_bwd(params, q, k, v, b, sm_scale, o, dout, dq, dk, dv, db, dq_acc, L, delta, dropout_p,
               philox_seed, philox_offset1, philox_offset2, causal)
@@ -204,6 +250,12 @@ def attn_bwd_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqle
                     philox_seed, philox_offset1, philox_offset2, causal, varlen_type, extargs=None,
                     stream=None):
     """aotriton_flash.py:337-398."""
+    rc = _native(_torch_host.attn_bwd, q, k, v, b, sm_scale, o, dout, dq, dk, dv, db, L, *_delta_arg(delta), dropout_p,
+                 philox_seed, philox_offset1, philox_offset2, *translate_causal(causal), cu_seqlens_q, cu_seqlens_k,
+                 max_seqlen_q, max_seqlen_k, seq_strides_q, seq_strides_k, IVARLEN_TYPE[varlen_type],
+                 *_options(extargs), _stream_arg(stream))
+    if rc is not None:
+        return rc
     params = fa_backward_op_params()
     _fill_bwd(params, q, k, v, b, sm_scale, o, dout, dq, dk, dv, db, dq_acc, L, delta, dropout_p,
               philox_seed, philox_offset1, philox_offset2, causal)
@@ -240,11 +292,9 @@ def check_gpu(stream=None):
 
 def lazy_dq_acc(dq):
     """aotriton_flash.py:400-403."""
-    return lazy_tensor.dq_acc(T4(dq.data_ptr(), tuple(dq.size()), dq.stride(), cast_dtype(dq.dtype)),
-                              dq.device.index)
+    return lazy_tensor.LazyTensor4(lambda: mk_aotensor(dq), dq.device.index)
 
 
 def lazy_delta(L):
     """aotriton_flash.py:405-408."""
-    return lazy_tensor.delta(T2(L.data_ptr(), tuple(L.size()), L.stride(), cast_dtype(L.dtype)),
-                             L.device.index)
+    return lazy_tensor.LazyTensor2(lambda: mk_aotensor(L), L.device.index)

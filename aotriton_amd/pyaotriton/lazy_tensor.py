@@ -7,27 +7,49 @@ from .. import _lib
 
 
 class _Lazy:
-    """Owns the ctypes struct plus the Python callbacks that keep it alive."""
+    """Owns the ctypes struct plus the Python callbacks that keep it alive.  Both are made when the
+    struct is asked for: the native host path allocates by itself and never does."""
     C = None
     ACQ = None
     DISP = None
-    VIEW = None
 
     def __init__(self, like_view, device_index, dtype=None, eager=None):
+        """``like_view``: the view whose shape the buffer takes, or a function that makes it when the
+        struct is first needed."""
+        self._like_view = like_view
+        self._device = device_index
+        self._eager = eager
+        self._held = None
+        self._c = None
+
+    @property
+    def on_demand(self):
+        """Stands for a buffer that is allocated when the operator asks for it."""
+        return self._eager is None
+
+    @property
+    def _like(self):
+        if callable(self._like_view):
+            self._like_view = self._like_view()
+        return self._like_view
+
+    @property
+    def c(self):
+        """The C struct; made, with its callbacks, on first use."""
+        if self._c is None:
+            self._c = self._make()
+        return self._c
+
+    def _make(self):
         import torch
         from . import DType
-        self._like = like_view
-        self._device = device_index
-        self._held = None
-        self.c = self.C()
-        self.c.cookie = None
-        if eager is not None:
-            self.c.eager = eager.to_c()
+        c = self.C()
+        c.cookie = None
+        if self._eager is not None:
+            c.eager = self._eager.to_c()
             self._acq = self.ACQ(0)
             self._disp = self.DISP(0)
         else:
-            view_c = self.VIEW
-
             def acquire(self_ptr, out_ptr):
                 try:
                     dev = torch.device('cuda', self._device) if self._device is not None else None
@@ -50,8 +72,9 @@ class _Lazy:
 
             self._acq = self.ACQ(acquire)
             self._disp = self.DISP(dispose)
-        self.c.acquire = self._acq
-        self.c.dispose = self._disp
+        c.acquire = self._acq
+        c.dispose = self._disp
+        return c
 
     def __bool__(self):
         return True

@@ -9,13 +9,15 @@ import math
 
 import torch
 
-from .autograd import attention, AttentionExtraArgs
+from . import _torch_host
+from .autograd import _DEFAULTS, _extra_args
 
 
 def prepare(query, key, value, attn_mask, is_causal, scale, enable_gqa):
-    """Argument checks and layout fixes shared by the SDPA-shaped entry points: returns
+    """Argument checks and layout fixes of the SDPA-shaped entry points: returns
     (q, k, v, bias, sm_scale) with unit last strides and the mask as an additive
-    (B, H, L, S) bias (None without a mask)."""
+    (B, H, L, S) bias (None without a mask).  What torch.compile traces; eager calls do the same
+    natively (csrc/torch/host.cpp)."""
     if query.dim() != 4 or key.dim() != 4 or value.dim() != 4:
         raise ValueError('expected (batch, heads, seq, head_dim) tensors')
     if is_causal and attn_mask is not None:
@@ -48,7 +50,5 @@ def scaled_dot_product_attention(query, key, value, attn_mask=None, dropout_p=0.
     (0 / -inf), and a query row that the mask hides completely yields zeros instead of NaN;
     dropout uses the operators' Philox stream (seed/offsets in `extra`), not torch's generator.
     """
-    q, k, v, bias, sm_scale = prepare(query, key, value, attn_mask, is_causal, scale, enable_gqa)
-    out, _, _ = attention(q, k, v, bias, bool(is_causal), sm_scale, float(dropout_p),
-                          extra or AttentionExtraArgs())
-    return out
+    return _torch_host.sdpa_function(query, key, value, attn_mask, dropout_p, bool(is_causal), scale, enable_gqa,
+                                     *_extra_args(extra or _DEFAULTS))

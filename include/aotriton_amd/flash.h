@@ -333,6 +333,12 @@ FA_API int fa_trim_workspace(void);
 FA_API int fa_attn_bwd_kernel(const fa_bwd_params* params, int32_t params_version,
                               void* hip_stream, int32_t kernel_slot);
 
+/* `count` 32-bit words of host memory to device memory, ordered on the stream like a kernel: they
+ * travel as kernel arguments, so the host memory is free again on return and nothing waits.  Meant
+ * for what the operators read from the device: Philox seed and offset, cu_seqlens.  No
+ * counterpart in the reference. */
+FA_API int fa_write_words(void* dst, const uint32_t* words, int32_t count, void* hip_stream);
+
 /* v2::flash::debug_simulate_encoded_softmax -- include/aotriton/flash.h:18-24,
  * modules/flash/csrc/attn_debug.cc:30-69.  r is (B, H, max_seqlen_q, max_seqlen_k). */
 FA_API int fa_debug_simulate_encoded_softmax(const fa_tensor4* r, float dropout_p,
