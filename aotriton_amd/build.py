@@ -40,7 +40,7 @@ EXTRA = {
 
 # The per-head-dim kernel files are compiled a second time with FA_PADDED=1: the copies that
 # serve head dims rounded up to the compiled one.
-PADDED_RE = re.compile(r'fa_(fwd|bwd_dkdv|bwd_dq|bwd_fused)_d\d+\.hip$')
+PADDED_RE = re.compile(r'fa_(fwd|fwd_rows|bwd_dkdv|bwd_dq|bwd_fused)_d\d+\.hip$')
 
 
 def sources():

@@ -499,6 +499,98 @@ hipError_t run_fwd(int dtype, int d, const fa::FwdArgs& a, const Shape& s, hipSt
   return hipErrorNotSupported;
 }
 
+// How a forward is cut up: the tiles of fwd_kernel as they are, the same with the keys of a tile split
+// into parts, or (rows) blocks of 32 packed rows with split keys (fa_fwd_rows.h).
+struct FwdPlan {
+  bool rows;
+  int splits;                            // 1: nothing is split and no scratch is needed
+  int row_blocks, part_rows;             // of the rows kernel
+  int64_t o_bytes, bytes;                // scratch: the parts' sums, and all of it
+};
+
+// The rule compares estimated times in microseconds.  They come from measurements on one box (bf16):
+// fwd_kernel takes a 256-row tile (128 at D = 256) through 64 keys in 1.2 / 1.9 / 2.4 us (D = 64 / 128 /
+// 256) with all CUs busy (a quarter less on an idle chip, whose clock is higher), one workgroup per
+// CU, and 6 us around that; the rows kernel takes four waves of 32 rows through 4 x 32 keys in
+// 0.9 / 1.2 / 2.6 us, two workgroups of a CU (one at D = 256) taking turns, and 4 us around that; a part's sums of 256 rows cost
+// 0.07 us of the whole chip's memory time at D = 128, the second launch 5 us.  Within 10-20 % of the
+// measured times at 24 shapes of 1-2048 queries and 64-30000 keys; the gains it decides on are larger
+// (one query, 2051 keys, Hq 32 / Hk 8: 56 -> 11 us; 32 sequences of 8190 keys: 833 -> 189; 80 queries,
+// 3216 keys: 85 -> 34; 1024 queries, 16384 keys: 398 -> 274).
+FwdPlan fwd_plan(int dtype, const Shape& s, int causal_type, int window_left, int window_right, int num_cu) {
+  FwdPlan r{};
+  r.splits = 1;
+  if (s.elementwise || !is_16bit(dtype) || s.d > 256 || s.dropout || s.max_sq <= 0 || s.max_sk <= 0 || s.batch <= 0) return r;
+  const int64_t nz = s.num_seqlens != 0 ? std::abs(s.num_seqlens) : s.batch;
+  const int group = s.hq / s.hk, bm = s.d > 128 ? 128 : 256;
+  const int m_tiles = (s.max_sq + bm - 1) / bm;
+  const int64_t tiles = nz * s.hq * m_tiles;
+  if (tiles >= 4 * num_cu && s.max_sq >= bm) return r;      // the chip is full and so are the tiles
+  const double wide = s.d / 128.0;
+
+  // the tiles as they are or split: keys of the heaviest tile and of all of them
+  int64_t most = 0, sum = 0;
+  for (int mt = 0; mt < m_tiles; ++mt) {
+    int64_t n = (s.max_sk + 63) / 64;
+    if (s.windowed) {
+      const fa::Window w = fa::parse_window(causal_type, window_left, window_right, s.max_sq, s.max_sk);
+      const fa::BlockRanges b = fa::block_ranges(true, w.left, w.right, mt * bm, s.max_sq, s.max_sk, bm, 64);
+      n = b.hi - b.lo + 1;
+    }
+    most = n > most ? n : most;
+    sum += n;
+  }
+  const double t64 = s.d == 64 ? 1.2 : s.d == 128 ? 1.9 : 2.4;
+  auto tile_time = [&](int64_t parts) {
+    const double rounds = (double)((tiles * parts + num_cu - 1) / num_cu);
+    // tiles of about the same weight go in whole rounds, uneven ones fill each other's gaps
+    const double even = (double)sum * nz * s.hq / num_cu *
+                        (sum * 5 > most * m_tiles * 4 ? rounds * num_cu / (double)(tiles * parts) : 1.0);
+    const double longest = (double)((most + parts - 1) / parts);
+    const double busy = tiles * parts < num_cu ? (double)(tiles * parts) / num_cu : 1.0;
+    return (even > longest ? even : longest) * t64 * (0.75 + 0.25 * busy) + 6 * rounds +
+           (parts > 1 ? 5 + 0.07 * wide * tiles * parts : 0.0);
+  };
+  double best = tile_time(1);
+  if (s.d <= 128 && s.num_seqlens == 0)
+    for (int64_t parts = 2; parts <= 16 && parts * 2 <= most; ++parts)
+      if (const double t = tile_time(parts); t < 0.9 * best) { best = t; r.splits = (int)parts; }
+
+  const int64_t rows = (int64_t)group * s.max_sq;
+  const int64_t items = (rows + 31) / 32 * nz * s.hk, blocks = (most * 64 + 31) / 32;
+  int64_t splits = num_cu / items;
+  const int64_t most_splits = (blocks + 3) / 4 < 64 ? (blocks + 3) / 4 : 64;
+  splits = splits > most_splits ? most_splits : splits;
+  splits = splits < 1 ? 1 : splits;      // (a window may hide every key)
+  const double steps = (double)((blocks + 4 * splits - 1) / (4 * splits));
+  const int64_t slots = (s.d > 128 ? 1 : 2) * num_cu, row_rounds = (items * splits + slots - 1) / slots;
+  const double per_cu = s.d > 128 ? (double)row_rounds : (double)(items * splits) / num_cu;
+  const double t128 = s.d == 64 ? 0.9 : s.d == 128 ? 1.2 : 2.6;
+  const double rows_time = (per_cu > 1 ? per_cu : 1) * steps * t128 + 4 * (double)row_rounds + 1 + (splits > 1 ? 4 : 0);
+  r.rows = rows_time < best;
+  int64_t stored;
+  if (r.rows) {
+    r.splits = (int)splits;
+    r.row_blocks = (int)((rows + 31) / 32);
+    r.part_rows = (int)(rows < 32 ? rows : 32);
+    stored = items * splits * r.part_rows;
+  } else {
+    stored = tiles * r.splits * bm;
+  }
+  r.o_bytes = stored * s.d * 4;
+  r.bytes = r.o_bytes + stored * 8;
+  return r;
+}
+
+hipError_t run_fwd_rows(int dtype, int d, const fa::FwdArgs& a, const Shape& s, hipStream_t stream) {
+  const bool padded = a.head_dim != d || a.head_dim_v != d;
+  switch (d) {
+    case 64: return (padded ? fa::run_fwd_rows_d64_padded : fa::run_fwd_rows_d64)(dtype, a, s.windowed, s.bias, stream);
+    case 128: return (padded ? fa::run_fwd_rows_d128_padded : fa::run_fwd_rows_d128)(dtype, a, s.windowed, s.bias, stream);
+    default: return (padded ? fa::run_fwd_rows_d256_padded : fa::run_fwd_rows_d256)(dtype, a, s.windowed, s.bias, stream);
+  }
+}
+
 fa::DropoutArgs dropout_args(float p, const fa_tensor0& seed, const fa_tensor0& off1, uint64_t off2) {
   fa::DropoutArgs d{};
   d.p = p;
@@ -736,8 +828,8 @@ int fa_debug_simulate_encoded_softmax(const fa_tensor4* r, float dropout_p, cons
   return (int)fa::run_encoded_softmax(a, stream);
 }
 
-int fa_attn_fwd(const fa_fwd_params* p, int32_t params_version, void* hip_stream,
-                const fa_options* options) {
+static int attn_fwd_impl(const fa_fwd_params* p, int32_t params_version, void* hip_stream,
+                         const fa_options* options, fa_allocator* alloc) {
   Shape s{};
   int e = validate_fwd(p, params_version, options, &s);
   if (e != FA_SUCCESS) return e;
@@ -764,7 +856,7 @@ int fa_attn_fwd(const fa_fwd_params* p, int32_t params_version, void* hip_stream
       int rc = (int)err;
       if (err == hipSuccess) {
         t_ws_nested = NestedWorkspace{true, nullptr, 0};
-        rc = fa_attn_fwd(&p2, params_version, hip_stream, options);
+        rc = attn_fwd_impl(&p2, params_version, hip_stream, options, alloc);
         t_ws_nested = NestedWorkspace{};
       }
       if (rc == FA_SUCCESS) rc = (int)repack(p->Out, p2.Out, true, stream);
@@ -797,7 +889,30 @@ int fa_attn_fwd(const fa_fwd_params* p, int32_t params_version, void* hip_stream
   FA_LOG(4, "attn_fwd: D=%d BLOCK_M=%d BLOCK_N=%d waves=%d lds=%d windowed=%d bias=%d dropout=%d nseq=%d",
          s.d, t.block_m, t.block_n, t.num_waves, t.lds_bytes, (int)s.windowed, (int)s.bias,
          (int)s.dropout, s.num_seqlens);
-  hipError_t err = run_fwd(p->Q.dtype, s.d, a, s, stream);
+  hipError_t err;
+  const FwdPlan plan = fwd_plan(p->Q.dtype, s, p->causal_type, p->window_left, p->window_right, dev->num_cu);
+  void* scratch = nullptr;
+  bool held = false;
+  if (plan.splits > 1) {
+    if (alloc != nullptr) {
+      scratch = alloc->alloc(alloc, (uint64_t)plan.bytes);
+    } else if (!t_ws_nested.active && !stream_is_capturing(stream) && plan.bytes <= ws_limit_bytes(device_index(dev))) {
+      held = ws_acquire(device_index(dev), (size_t)plan.bytes, stream, &scratch) == hipSuccess;
+      if (!held) scratch = nullptr;
+    }
+    if (scratch != nullptr) {
+      a.part_o = static_cast<float*>(scratch);
+      a.part_ml = reinterpret_cast<float*>(static_cast<char*>(scratch) + plan.o_bytes);
+    }
+  }
+  a.splits = scratch != nullptr ? plan.splits : 1;
+  if (plan.rows) {
+    a.row_blocks = plan.row_blocks; a.part_rows = plan.part_rows;
+    err = run_fwd_rows(p->Q.dtype, s.d, a, s, stream);
+  } else {
+    err = run_fwd(p->Q.dtype, s.d, a, s, stream);
+  }
+  if (held) ws_release(device_index(dev), stream);
   if (err != hipSuccess) return (int)err;
   if (p->encoded_softmax.ptr != nullptr) {
     // the forward metro chains the mask dump (modules/flash/aot/__init__.py:40-41)
@@ -806,6 +921,15 @@ int fa_attn_fwd(const fa_fwd_params* p, int32_t params_version, void* hip_stream
                                              p->philox_offset2, hip_stream);
   }
   return FA_SUCCESS;
+}
+
+int fa_attn_fwd(const fa_fwd_params* p, int32_t params_version, void* hip_stream, const fa_options* options) {
+  return attn_fwd_impl(p, params_version, hip_stream, options, nullptr);
+}
+
+int fa_attn_fwd_alloc(const fa_fwd_params* p, int32_t params_version, void* hip_stream, const fa_options* options,
+                      fa_allocator* alloc) {
+  return attn_fwd_impl(p, params_version, hip_stream, options, alloc);
 }
 
 // kernel_slot < 0: the whole backward of the chosen backend; otherwise only that

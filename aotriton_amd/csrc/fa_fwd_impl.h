@@ -19,6 +19,7 @@
 #pragma once
 #include <type_traits>
 
+#include "fa_combine.h"
 #include "fa_device.h"
 #include "fa_fwd_pipe.h"
 
@@ -36,9 +37,12 @@ struct FwdSmem {
   static constexpr int BYTES = ROWS_OFF + NW * 32 * ROW_STR;
 };
 
-// One Q tile (BM rows of head h of sequence z) against all its visible K/V tiles.
-template <typename T, int D, int NW, int BN, bool kWindowed, bool kBias, bool kDropout, bool kPad>
-__device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const int h, const int mt, char* smem_raw) {
+// One Q tile (BM rows of head h of sequence z) against all its visible K/V tiles, or with kSplit
+// against part `split` of a.splits of them: the fp32 sums and the row statistics of the part then go to
+// scratch memory, where combine_rows_kernel picks them up.
+template <typename T, int D, int NW, int BN, bool kWindowed, bool kBias, bool kDropout, bool kPad, bool kSplit>
+__device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const int h, const int mt, const int split,
+                                         char* smem_raw) {
   using Tr = Traits<T>;
   using op_t = typename Tr::op_t;
   using q4_t = typename Tr::q4_t;
@@ -77,7 +81,12 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
   // keep row +/- window inside int32
   w.left = w.left > (1 << 30) ? (1 << 30) : (w.left < -(1 << 30) ? -(1 << 30) : w.left);
   w.right = w.right > (1 << 30) ? (1 << 30) : (w.right < -(1 << 30) ? -(1 << 30) : w.right);
-  const BlockRanges br = block_ranges(kWindowed, w.left, w.right, q0, si.seqlen_q, si.seqlen_k, BM, BN);
+  BlockRanges br = block_ranges(kWindowed, w.left, w.right, q0, si.seqlen_q, si.seqlen_k, BM, BN);
+  if (kSplit && br.lo <= br.hi) {
+    const int per = (br.hi - br.lo + a.splits) / a.splits;
+    br.lo += split * per;
+    if (br.lo + per - 1 < br.hi) br.hi = br.lo + per - 1;
+  }
 
   const int hk = h / (a.hq / a.hk);                       // fwd_kernel.py:360
   const int row = q0 + wave * 32 + c;                     // this lane's query row
@@ -88,6 +97,14 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
             (int64_t)(si.q_start + row_c) * a.so.s;
   float* lse_ptr = a.lse ? a.lse + lse_offset(si, h, a.hq) : nullptr;
 
+  const int64_t part_row = kSplit ? (((int64_t)z * a.hq + h) * a.num_m_tiles + mt) * (int64_t)(a.splits * BM) + split * BM + wave * 32 + c : 0;
+  if (kSplit && br.lo > br.hi) {
+    if (row_ok && hi == 0) {
+      a.part_ml[part_row * 2] = kNegBig;
+      a.part_ml[part_row * 2 + 1] = 0.f;
+    }
+    return;
+  }
   if (br.lo > br.hi) {
     // No visible key for any row of this tile: O = 0, LSE = +inf (fwd_kernel.py:327-355)
     if (row_ok) {
@@ -519,6 +536,21 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
 
   // ---- epilogue ----------------------------------------------------------------
   const float l = cross_sum(l_i);
+  if (kSplit) {
+    if (row_ok) {
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *reinterpret_cast<f32x4*>(a.part_o + part_row * D + 32 * db + 8 * g + 4 * hi) =
+              f32x4{o[db][4 * g], o[db][4 * g + 1], o[db][4 * g + 2], o[db][4 * g + 3]};
+      if (hi == 0) {
+        a.part_ml[part_row * 2] = m_i * sc;
+        a.part_ml[part_row * 2 + 1] = l;
+      }
+    }
+    return;
+  }
   const bool alive = l > 0.f;
   float inv = alive ? 1.0f / l : 0.f;
   if (kDropout) inv *= ds.scale;          // fwd_kernel.py:573-575
@@ -556,7 +588,7 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
 // goes from one tile to the next without a relaunch.
 // QB = 0: fwd_item, NW waves of 32 rows.  QB > 0: fwd_item_pipe, 4 waves of 32 * QB rows, one wave
 // per SIMD.
-template <typename T, int D, int NW, int BN, int QB, bool kWindowed, bool kBias, bool kDropout, bool kPad>
+template <typename T, int D, int NW, int BN, int QB, bool kWindowed, bool kBias, bool kDropout, bool kPad, bool kSplit>
 __global__ __attribute__((amdgpu_flat_work_group_size(NW * 64, NW * 64)))
 __attribute__((amdgpu_waves_per_eu(D <= 128 && QB == 0 ? 2 : 1, D <= 128 && QB == 0 ? 2 : 1)))
 void fwd_kernel(const FwdArgs a) {
@@ -593,7 +625,7 @@ void fwd_kernel(const FwdArgs a) {
   else if (ragged) walk.init(a.seq, xcd, a.zh_per_xcd, a.num_zh, ratio, nseq, kRows, false);
   for (int r = 0;; ++r) {
     const int t = r * workers + ((r & 1) ? workers - 1 - p : p);
-    int z, h, mt;
+    int z, h, mt, split = 0;
     if (levels) {
       int e;
       if (!lwalk.at(t, e, mt)) break;
@@ -606,7 +638,9 @@ void fwd_kernel(const FwdArgs a) {
     } else {
       if (r * workers >= items) break;
       if (t >= items) continue;
-      const int gi = t / per_group, gr = t % per_group;
+      const int ti = kSplit ? t / a.splits : t;
+      split = kSplit ? t % a.splits : 0;
+      const int gi = ti / per_group, gr = ti % per_group;
       const int zh_local = gi * a.zh_group + gr % a.zh_group;
       const int zh = xcd * a.zh_per_xcd + zh_local;
       if (zh_local >= a.zh_per_xcd || zh >= a.num_zh) continue;
@@ -614,7 +648,7 @@ void fwd_kernel(const FwdArgs a) {
       split_zh(zh, nseq, ratio, z, h);
     }
     if constexpr (QB > 0) fwd_item_pipe<T, D, QB, BN, kWindowed, kBias, kDropout, kPad>(a, z, h, mt, smem_raw);
-    else fwd_item<T, D, NW, BN, kWindowed, kBias, kDropout, kPad>(a, z, h, mt, smem_raw);
+    else fwd_item<T, D, NW, BN, kWindowed, kBias, kDropout, kPad, kSplit>(a, z, h, mt, split, smem_raw);
   }
 }
 
@@ -646,11 +680,11 @@ template <typename T, bool kWindowed> struct FwdTile<T, 128, kWindowed> : FwdTil
 // 629 vs 510; bias + dropout + window 1024: 361 vs 333).
 template <typename T, bool kWindowed> struct FwdTile<T, 256, kWindowed> : FwdTileOf<256, 4, 32, 1> {};
 
-template <typename T, int D, bool kWindowed, bool kBias, bool kDropout, bool kPad>
+template <typename T, int D, bool kWindowed, bool kBias, bool kDropout, bool kPad, bool kSplit = false>
 hipError_t launch_fwd_variant(const FwdArgs& a, dim3 grid, hipStream_t stream) {
   using Tile = FwdTile<T, D, kWindowed>;
   constexpr int NW = Tile::NW;
-  auto kern = fwd_kernel<T, D, NW, Tile::BN, Tile::QB, kWindowed, kBias, kDropout, kPad>;
+  auto kern = fwd_kernel<T, D, NW, Tile::BN, Tile::QB, kWindowed, kBias, kDropout, kPad, kSplit>;
   constexpr int smem = Tile::LDS;
   if (grid.x == 0) return hipSuccess;      // no batch, no head or no query row: nothing to write
   if (smem > 64 * 1024) {
@@ -659,7 +693,9 @@ hipError_t launch_fwd_variant(const FwdArgs& a, dim3 grid, hipStream_t stream) {
     if (e != hipSuccess) return e;
   }
   hipLaunchKernelGGL(kern, grid, dim3(NW * 64), smem, stream, a);
-  return hipGetLastError();
+  hipError_t e = hipGetLastError();
+  if (kSplit && e == hipSuccess) e = launch_combine_rows<T, D>(a, a.num_zh, stream);
+  return e;
 }
 
 // kPad: a head dim of the tensors (FwdArgs::head_dim, head_dim_v) is smaller than D and the excess
@@ -675,11 +711,24 @@ hipError_t launch_fwd(const FwdArgs& a, bool windowed, bool bias, bool dropout, 
   b.zh_per_xcd = (b.num_zh + kNumXcd - 1) / kNumXcd;
   b.zh_group = a.hq / a.hk > 2 ? (a.hq / a.hk > 8 ? 8 : a.hq / a.hk) : 2;
   const int groups = (b.zh_per_xcd + b.zh_group - 1) / b.zh_group;
-  b.items_per_xcd = groups * b.zh_group * b.num_m_tiles;
+  // (with splits, an item is one part of the keys of a tile; only without dropout, at D <= 128)
+  const bool split = a.splits > 1;
+  b.items_per_xcd = groups * b.zh_group * b.num_m_tiles * (split ? a.splits : 1);
   int workers = a.num_cu / kNumXcd;          // one workgroup per CU
   if (workers < 1) workers = 1;
   if (workers > b.items_per_xcd) workers = b.items_per_xcd;
   dim3 grid((unsigned)(kNumXcd * workers));
+  if constexpr (D <= 128) {
+    if (split) {
+      b.part_group = 1; b.part_block = BM; b.part_rows = BM; b.row_blocks = b.num_m_tiles;
+      switch ((windowed ? 2 : 0) | (bias ? 1 : 0)) {
+        case 0: return launch_fwd_variant<T, D, false, false, false, kPad, true>(b, grid, stream);
+        case 1: return launch_fwd_variant<T, D, false, true, false, kPad, true>(b, grid, stream);
+        case 2: return launch_fwd_variant<T, D, true, false, false, kPad, true>(b, grid, stream);
+        default: return launch_fwd_variant<T, D, true, true, false, kPad, true>(b, grid, stream);
+      }
+    }
+  }
   const int key = (windowed ? 4 : 0) | (bias ? 2 : 0) | (dropout ? 1 : 0);
   switch (key) {
     case 0: return launch_fwd_variant<T, D, false, false, false, kPad>(b, grid, stream);

@@ -17,6 +17,13 @@ hipError_t run_fwd_d256(int dtype, const FwdArgs& a, bool windowed, bool bias, b
 hipError_t run_fwd_d64_padded(int dtype, const FwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
 hipError_t run_fwd_d128_padded(int dtype, const FwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
 hipError_t run_fwd_d256_padded(int dtype, const FwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
+// few query rows per K/V head: packed rows of a GQA group, keys split over workgroups (fa_fwd_rows.h)
+hipError_t run_fwd_rows_d64(int dtype, const FwdArgs& a, bool windowed, bool bias, hipStream_t s);
+hipError_t run_fwd_rows_d128(int dtype, const FwdArgs& a, bool windowed, bool bias, hipStream_t s);
+hipError_t run_fwd_rows_d256(int dtype, const FwdArgs& a, bool windowed, bool bias, hipStream_t s);
+hipError_t run_fwd_rows_d64_padded(int dtype, const FwdArgs& a, bool windowed, bool bias, hipStream_t s);
+hipError_t run_fwd_rows_d128_padded(int dtype, const FwdArgs& a, bool windowed, bool bias, hipStream_t s);
+hipError_t run_fwd_rows_d256_padded(int dtype, const FwdArgs& a, bool windowed, bool bias, hipStream_t s);
 // tile table lookups: (element type, head dim, causal / windowed)
 TileShape fwd_tile_shape(int dtype, int head_dim, bool windowed);
 

@@ -140,6 +140,26 @@ struct LazyDelta {
   static void dispose(fa_lazy_tensor2* self) { static_cast<LazyDelta*>(self->cookie)->held.reset(); }
 };
 
+// scratch memory of a forward, from torch's allocator: ordered with the stream, and a graph's own under capture
+struct Scratch {
+  fa_allocator c{};
+  Tensor held;
+  at::Device device;
+  explicit Scratch(at::Device d) : device(d) {
+    c.cookie = this;
+    c.alloc = &alloc;
+  }
+  static void* alloc(fa_allocator* self, uint64_t bytes) {
+    auto* me = static_cast<Scratch*>(self->cookie);
+    try {
+      me->held = at::empty({(int64_t)bytes}, at::TensorOptions(at::kByte).device(me->device));
+      return me->held.data_ptr();
+    } catch (...) {
+      return nullptr;
+    }
+  }
+};
+
 // ---- what `attention`, the custom ops and their backwards share -----------------------------------
 
 struct Mask { int type = 0, left = 0, right = 0; };
@@ -170,7 +190,8 @@ void fill_common(P& p, const Tensor& q, const Tensor& k, const Tensor& v, const 
 
 int run_forward(fa_fwd_params& p, const Tensor& lse, const Tensor& o, const Tensor& encoded) {
   TORCH_CHECK(view2(lse, &p.L) && view4(o, &p.Out) && view4(encoded, &p.encoded_softmax), "outputs");
-  return fa_attn_fwd(&p, FA_FWD_PARAMS_VERSION, current_stream(), nullptr);
+  Scratch scratch(o.device());
+  return fa_attn_fwd_alloc(&p, FA_FWD_PARAMS_VERSION, current_stream(), nullptr, &scratch.c);
 }
 
 int run_backward(fa_bwd_params& p, const Tensor& o, const Tensor& dout, const Tensor& lse, const Tensor& dq,
@@ -479,7 +500,8 @@ PyObject* py_attn_fwd(PyObject*, PyObject* const* argv, Py_ssize_t n) {
   ok = view4(b.defined() && b.numel() > 0 ? b : Tensor(), &p.B);
   p.Sm_scale = (float)a.real();
   ok &= view2(a.tensor(true), &p.L);
-  ok &= view4(a.tensor(false), &p.Out);
+  const Tensor o = a.tensor(false);
+  ok &= view4(o, &p.Out);
   p.dropout_p = (float)a.real();
   ok &= view0(a.tensor(false), &p.philox_seed_ptr);
   ok &= view0(a.tensor(false), &p.philox_offset1);
@@ -506,7 +528,10 @@ PyObject* py_attn_fwd(PyObject*, PyObject* const* argv, Py_ssize_t n) {
   int rc;
   {
     pybind11::gil_scoped_release no_gil;
-    rc = fa_attn_fwd(&p, FA_FWD_PARAMS_VERSION, stream == -1 ? current_stream() : reinterpret_cast<void*>(stream), &opt);
+    // torch's allocator orders its memory with torch's current stream only
+    Scratch scratch(o.device());
+    rc = stream == -1 ? fa_attn_fwd_alloc(&p, FA_FWD_PARAMS_VERSION, current_stream(), &opt, &scratch.c)
+                      : fa_attn_fwd(&p, FA_FWD_PARAMS_VERSION, reinterpret_cast<void*>(stream), &opt);
   }
   return PyLong_FromLong(rc);
   END_HANDLE_TH_ERRORS

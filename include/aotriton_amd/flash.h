@@ -232,6 +232,21 @@ FA_API int fa_check_gpu(void* hip_stream);
 FA_API int fa_attn_fwd(const fa_fwd_params* params, int32_t params_version,
                        void* hip_stream, const fa_options* options);
 
+/* As fa_attn_fwd, with the scratch memory of the call from the caller: `alloc` is asked at most
+ * once, for `bytes` of device memory that stay valid until the work of the call on the stream is
+ * done (a stream-ordered pool, a caching allocator; under stream capture, memory of the graph).
+ * It returns null when there is none.  The forward takes scratch when few query rows meet many
+ * keys (decode, short prompt chunks): the keys are split over workgroups and the parts' sums
+ * meet in memory.  fa_attn_fwd takes it from the library's workspace and, under stream capture or
+ * without memory, does not split; the results differ by fp32 summation order only.  No counterpart in
+ * the reference. */
+typedef struct fa_allocator {
+  void* cookie;
+  void* (*alloc)(struct fa_allocator* self, uint64_t bytes);
+} fa_allocator;
+FA_API int fa_attn_fwd_alloc(const fa_fwd_params* params, int32_t params_version, void* hip_stream,
+                             const fa_options* options, fa_allocator* alloc);
+
 /* v3::flash::attn_bwd -- include/aotriton/flash.h:176-180,
  * modules/flash/csrc/attn_bwd.cc:55-160.
  * Same tensors as the forward.  Single-launch kernels (backend 1) exist for fp16/bf16 up to head dim

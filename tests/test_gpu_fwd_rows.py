@@ -1,0 +1,139 @@
+"""The forward for few query rows per K/V head (fa_fwd_rows.h) against the oracle: blocks of 32 packed
+rows around their edges, keys around the 32-key steps, the four waves' shares and the splits, masks that
+leave splits, blocks or rows without a key.  Tolerances are the reference's model (tests/_util.py)."""
+import math
+
+import pytest
+import torch
+
+from _util import FUDGE, LSE_ATOL, check, make_inputs
+
+pytestmark = pytest.mark.gpu
+
+DEV = 'cuda'
+BR = 2      # flash.CausalType.BOTTOM_RIGHT
+
+CASES = [
+    # B, Hq, Hk, Sq, Sk, D, dtype, causal, bias
+    (1, 1, 1, 1, 1, 128, torch.bfloat16, False, False),
+    (2, 4, 4, 1, 31, 64, torch.float16, False, False),
+    (2, 8, 2, 1, 33, 128, torch.bfloat16, False, False),
+    (1, 32, 8, 1, 2051, 128, torch.bfloat16, False, False),
+    (3, 6, 2, 1, 127, 256, torch.float16, False, False),
+    (1, 8, 1, 1, 4096, 256, torch.bfloat16, True, False),
+    (1, 8, 2, 8, 129, 128, torch.float16, BR, False),           # one whole block of rows
+    (2, 8, 2, 9, 1000, 128, torch.bfloat16, BR, False),         # a second block with four rows
+    (1, 3, 1, 11, 513, 64, torch.bfloat16, BR, False),          # 33 rows
+    (2, 2, 2, 63, 640, 64, torch.float16, True, False),         # top left: most keys hidden
+    (1, 4, 2, 33, 300, 128, torch.float16, (20, 3), False),     # window: parts without a key
+    (1, 4, 4, 40, 16, 128, torch.bfloat16, (4, -6), False),     # rows without a key
+    (1, 4, 4, 64, 20, 128, torch.bfloat16, BR, False),          # bottom right with fewer keys than rows
+    (2, 4, 4, 1, 200, 72, torch.bfloat16, False, False),        # head dim rounded up
+    (1, 4, 2, 5, 777, 200, torch.float16, BR, False),
+    (2, 4, 2, 3, 257, 128, torch.float16, False, True),
+    (1, 8, 4, 7, 999, 64, torch.bfloat16, BR, True),
+    (1, 2, 2, 16, 70, 256, torch.float16, (30, 30), True),
+]
+
+
+def _forward(q, k, v, b, sm, causal, split):
+    """through the operator wrappers (scratch from torch's allocator) or, unsplit, without scratch"""
+    from aotriton_amd import flash
+    from aotriton_amd._lib import lib
+    ok = flash.hipError_t.hipSuccess
+    o = torch.full(q.shape[:3] + (v.shape[3],), float('nan'), device=DEV, dtype=q.dtype)
+    L = torch.full((q.shape[0] * q.shape[1], q.shape[2]), float('nan'), device=DEV)
+    null = torch.empty([0], device=DEV, dtype=torch.uint64)
+    args = (q, k, v, b, sm, L, o, 0.0, null, null, 0, null, null, None, causal, null)
+    if split == 'workspace':      # the C ABI without an allocator: the library's workspace
+        assert flash.attn_fwd(*args, stream=flash._stream()) == ok
+    elif split:
+        assert flash.attn_fwd(*args) == ok
+    else:
+        lib.fa_set_bwd_workspace_limit(0)
+        try:
+            assert flash.attn_fwd(*args, stream=flash._stream()) == ok
+        finally:
+            lib.fa_set_bwd_workspace_limit(-1)
+    torch.cuda.synchronize()
+    return o, L
+
+
+@pytest.mark.parametrize('case', CASES, ids=lambda c: '-'.join(str(x).replace('torch.', '') for x in c))
+def test_few_rows_meet_the_oracle(case):
+    from aotriton_amd import flash
+    from oracle import fa_ref
+    B, Hq, Hk, Sq, Sk, D, dtype, causal, bias = case
+    q, k, v, b, _ = make_inputs(B, Hq, Hk, Sq, Sk, D, dtype, DEV, seed=21, bias=bias, bshd=True)
+    if causal == BR:
+        causal = flash.CausalType.BOTTOM_RIGHT
+    sm = 1.0 / math.sqrt(D)
+    ct, wl, wr = flash.translate_causal(causal)
+    f = lambda t: None if t is None else t.float()
+    ro, rl, _ = fa_ref.attn_fwd_ref(f(q), f(k), f(v), f(b), sm, ct, wl, wr)
+    lo, _, _ = fa_ref.attn_fwd_ref(q, k, v, b, sm, ct, wl, wr)
+    for split in (True, 'workspace', False):
+        o, L = _forward(q, k, v, b, sm, causal, split)
+        check('out', o, ro, lo, FUDGE['out'])
+        L = L.view(B, Hq, Sq)
+        assert torch.equal(torch.isinf(L), torch.isinf(rl))
+        seen = torch.isfinite(rl)
+        assert (L[seen] - rl[seen]).abs().max().item() <= LSE_ATOL if seen.any() else True
+
+
+def test_scores_that_grow_and_huge_scores():
+    """the reference maximum moves in every step of every wave, and 16-bit scores of 1e4"""
+    from oracle import fa_ref
+    q, k, v, _, _ = make_inputs(1, 4, 2, 2, 900, 128, torch.bfloat16, DEV, seed=4)
+    k = k * torch.linspace(0.1, 60.0, 900, device=DEV, dtype=torch.float32).to(k.dtype).view(1, 1, -1, 1)
+    f = lambda t: t.float()
+    ro, rl, _ = fa_ref.attn_fwd_ref(f(q), f(k), f(v), None, 0.3, 0, 0, 0)
+    lo, _, _ = fa_ref.attn_fwd_ref(q, k, v, None, 0.3, 0, 0, 0)
+    o, L = _forward(q, k, v, None, 0.3, False, True)
+    check('out', o, ro, lo, FUDGE['out'])
+    assert ((L.view(1, 4, 2) - rl).abs() <= 1e-5 * rl.abs() + LSE_ATOL).all()
+
+
+def test_packed_decode_batch():
+    """one query per packed sequence, caches of different lengths (one of them empty)"""
+    from aotriton_amd.autograd import attention_varlen, AttentionExtraArgs
+    from oracle import fa_ref
+    lk = [700, 1, 0, 64, 333]
+    n, Hq, Hk, D = len(lk), 8, 2, 128
+    g = torch.Generator().manual_seed(2)
+    mk = lambda H, T: torch.randn(1, T, H, D, generator=g).to(torch.float16).to(DEV).transpose(1, 2)
+    q, k, v = mk(Hq, n), mk(Hk, sum(lk)), mk(Hk, sum(lk))
+    o, _, L = attention_varlen(q, k, v, [1] * n, lk, False, 0.1, 0.0, AttentionExtraArgs(return_logsumexp=True, fillnan=True))
+    at = 0
+    for i, len_k in enumerate(lk):
+        if len_k == 0:
+            assert (o[:, :, i] == 0).all() and torch.isinf(L[:, i]).all()
+            continue
+        ks, vs = k[:, :, at:at + len_k], v[:, :, at:at + len_k]
+        ro, rl, _ = fa_ref.attn_fwd_ref(q[:, :, i:i + 1].float(), ks.float(), vs.float(), None, 0.1, 0, 0, 0)
+        lo, _, _ = fa_ref.attn_fwd_ref(q[:, :, i:i + 1], ks, vs, None, 0.1, 0, 0, 0)
+        check('out', o[:, :, i:i + 1], ro, lo, FUDGE['out'])
+        assert (L[:, i] - rl.view(-1)).abs().max().item() <= LSE_ATOL
+        at += len_k
+
+
+def test_split_forward_replays_from_a_hip_graph():
+    """scratch under capture is the graph's own: replays, with eager calls between them, repeat the eager bits"""
+    from aotriton_amd.torch_ops import scaled_dot_product_attention as sdpa
+    q, k, v, _, _ = make_inputs(2, 8, 2, 1, 1500, 128, torch.bfloat16, DEV, seed=6)
+    run = lambda: sdpa(q, k, v, enable_gqa=True)
+    eager = run().clone()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        run()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = run()
+    for _ in range(3):
+        captured.fill_(float('nan'))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(captured, eager)
+        assert torch.equal(run(), eager)
