@@ -107,13 +107,17 @@ hipError_t scratch_of_device(int dev, float** out) {
 // allocation made the host wait for the GPU on every call).  Calls on one device share it: the
 // device's mutex covers the enqueue, and every call first waits (on the GPU) for the event recorded
 // behind the last use (no work when that was on the same stream; stream handles are not compared:
-// a destroyed stream's handle can come back).  fa_trim_workspace frees the buffers.
+// a destroyed stream's handle can come back).  The null stream is never destroyed, so uses on it
+// record nothing: the next call on it is ordered already, and a call on another stream records the
+// event then (recording and waiting in every call cost 4-5 us of a small backward).
+// fa_trim_workspace frees the buffers.
 std::atomic<int64_t> g_ws_limit{-1};        // bytes; -1: not set (environment, then default)
 struct Workspace {
   void* ptr = nullptr;
   size_t bytes = 0;
   hipEvent_t done = nullptr;
-  bool used = false;
+  bool used = false;           // `done` stands behind the last use
+  bool on_null = false;        // the last use was on the null stream and has no event yet
   std::mutex mutex;
 };
 Workspace g_ws[kMaxDevices];
@@ -142,7 +146,8 @@ hipError_t ws_acquire(int dev, size_t need, hipStream_t stream, void** out) {
   Workspace& w = g_ws[dev];
   w.mutex.lock();
   hipError_t e = hipSuccess;
-  if (w.bytes < need || w.done == nullptr) {
+  const bool order = w.on_null && stream != nullptr;
+  if (w.bytes < need || w.done == nullptr || order) {
     int cur = -1;
     e = hipGetDevice(&cur);
     if (e == hipSuccess && cur != dev) e = hipSetDevice(dev);
@@ -150,7 +155,7 @@ hipError_t ws_acquire(int dev, size_t need, hipStream_t stream, void** out) {
     if (e == hipSuccess && w.bytes < need) {
       // (hipFree waits for the device: nothing uses the old buffer any more)
       if (w.ptr != nullptr) (void)hipFree(w.ptr);
-      w.ptr = nullptr; w.bytes = 0; w.used = false;
+      w.ptr = nullptr; w.bytes = 0; w.used = w.on_null = false;
       size_t grow = need + need / 8;
       e = hipMalloc(&w.ptr, grow);
       if (e != hipSuccess) {      // no room for the margin: exactly what this call needs
@@ -159,6 +164,10 @@ hipError_t ws_acquire(int dev, size_t need, hipStream_t stream, void** out) {
         e = hipMalloc(&w.ptr, grow);
       }
       if (e == hipSuccess) w.bytes = grow; else w.ptr = nullptr;
+    }
+    if (e == hipSuccess && order && w.on_null) {
+      e = hipEventRecord(w.done, nullptr);      // behind everything on the device's null stream so far
+      if (e == hipSuccess) { w.used = true; w.on_null = false; }
     }
     if (cur >= 0 && cur != dev) (void)hipSetDevice(cur);
   }
@@ -174,7 +183,10 @@ hipError_t ws_acquire(int dev, size_t need, hipStream_t stream, void** out) {
 
 void ws_release(int dev, hipStream_t stream) {
   Workspace& w = g_ws[dev];
-  if (hipEventRecord(w.done, stream) == hipSuccess) {
+  w.on_null = stream == nullptr;
+  if (w.on_null) {
+    w.used = false;
+  } else if (hipEventRecord(w.done, stream) == hipSuccess) {
     w.used = true;
   } else {
     // without the event the next call cannot order itself behind this one
@@ -1330,7 +1342,7 @@ int fa_trim_workspace(void) {
     std::lock_guard<std::mutex> lock(g_ws[d].mutex);
     if (g_ws[d].ptr != nullptr) {
       const hipError_t e = hipFree(g_ws[d].ptr);      // waits for the device first
-      g_ws[d].ptr = nullptr; g_ws[d].bytes = 0; g_ws[d].used = false;
+      g_ws[d].ptr = nullptr; g_ws[d].bytes = 0; g_ws[d].used = g_ws[d].on_null = false;
       if (err == hipSuccess) err = e;
     }
   }
