@@ -630,6 +630,50 @@ int64_t ds_workspace_need(const fa_bwd_params* p, const Shape& s, int* ntq, int*
   return *ds_bytes + 2 * *stat_bytes;
 }
 
+// Parts of the dK/dV items (16-bit types, head dims up to 256).  An item is a 128-key tile of one kv-head
+// and runs through the query tiles of all q-heads of the group, one after the other: with few kv-heads
+// and short key ranges there are fewer items than CUs and each takes long.  Cut into parts (by
+// q-heads first, then by query tiles) they fill the chip; the parts' fp32 sums cost a round trip and a
+// launch.
+struct DkdvParts { int heads, tiles; int64_t bytes; };
+
+// The rule compares estimated times in microseconds: 1.9-2.3 per step (64 queries at D = 128, 128 at 64,
+// 32 at 256; more with a bias or dropout), 7 around an item, 4 for the second launch and 0.065 of the
+// chip's memory time per part (256 KB written and read at D = 128).
+DkdvParts dkdv_parts(const fa_bwd_params* p, const Shape& s, int num_cu) {
+  DkdvParts r{1, 1, 0};
+  if (s.elementwise || !is_16bit(p->Q.dtype) || s.d > 256 || s.max_sq <= 0 || s.max_sk <= 0 || s.batch <= 0) return r;
+  const int64_t nz = s.num_seqlens != 0 ? std::abs(s.num_seqlens) : s.batch;
+  const int n_tiles = (s.max_sk + 127) / 128, group = s.hq / s.hk;
+  const int64_t items = nz * s.hk * n_tiles;
+  if (items * 2 > num_cu) return r;
+  const int bm = s.d == 64 ? 128 : s.d == 128 ? 64 : 32;
+  int64_t most = 0;
+  for (int nt = 0; nt < n_tiles; ++nt) {
+    int64_t n = (s.max_sq + bm - 1) / bm;
+    if (s.windowed) {
+      const fa::Window w = fa::parse_window(p->causal_type, p->window_left, p->window_right, s.max_sq, s.max_sk);
+      const fa::BlockRanges b = fa::block_ranges(true, w.right, w.left, nt * 128, s.max_sk, s.max_sq, 128, bm);
+      n = b.hi - b.lo + 1;
+    }
+    most = n > most ? n : most;
+  }
+  const double t_step = (s.d == 64 ? 2.3 : s.d == 128 ? 1.9 : 2.1) * (s.dropout ? 1.7 : 1.0) * (s.bias ? 1.3 : 1.0);
+  double best = group * most * t_step + 7;
+  for (int heads = 1; heads <= group; ++heads) {
+    if (group % heads != 0) continue;
+    for (int tiles = 1; tiles <= 16 && tiles <= most; ++tiles) {
+      if (heads * tiles == 1 || (tiles > 1 && heads < group)) continue;
+      const int64_t wgs = items * heads * tiles, rounds = (wgs + num_cu - 1) / num_cu;
+      const double t = rounds * ((double)(group / heads) * ((most + tiles - 1) / tiles) * t_step + 7) + 4 +
+                       0.065 * s.d / 128 * wgs;
+      if (t < 0.95 * best) { best = t; r.heads = heads; r.tiles = tiles; }
+    }
+  }
+  if (r.heads * r.tiles > 1) r.bytes = items * r.heads * r.tiles * (2 * 128 * s.d * 4);
+  return r;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1013,7 +1057,7 @@ static int attn_bwd_impl(const fa_bwd_params* p_in, int32_t params_version, void
     if (validate_bwd(&p2, params_version, options, &s2, &be2) == FA_SUCCESS && be2 == 0) {
       int ntq = 0, ntk = 0;
       int64_t ds_bytes = 0, stat_bytes = 0;
-      inner = ds_workspace_need(&p2, s2, &ntq, &ntk, &ds_bytes, &stat_bytes);
+      inner = ds_workspace_need(&p2, s2, &ntq, &ntk, &ds_bytes, &stat_bytes) + dkdv_parts(&p2, s2, dev->num_cu).bytes;
       if ((int64_t)copies + inner > ws_limit_bytes(device_index(dev))) inner = 0;
     }
     const size_t need = copies + (size_t)inner;
@@ -1135,35 +1179,44 @@ static int attn_bwd_impl(const fa_bwd_params* p_in, int32_t params_version, void
     int64_t ds_bytes = 0, stat_bytes = 0;
     // (kernel_slot 4, 5, 6: one kernel of this backward only; the buffer keeps its content between calls)
     const int ds_slot = kernel_slot >= 4 ? kernel_slot - 4 : -1;
-    const int64_t need = (kernel_slot < 0 || ds_slot >= 0) && !own_delta
-                             ? ds_workspace_need(p, s, &ntq, &ntk, &ds_bytes, &stat_bytes) : 0;
+    int64_t need = (kernel_slot < 0 || ds_slot >= 0) && !own_delta
+                       ? ds_workspace_need(p, s, &ntq, &ntk, &ds_bytes, &stat_bytes) : 0;
+    if (need > ws_limit_bytes(device_index(dev)) && ds_slot < 0) need = 0;
+    // (single kernels, for timing, run uncut)
+    DkdvParts parts{1, 1, 0};
+    if (kernel_slot < 0 && !own_delta) parts = dkdv_parts(p, s, dev->num_cu);
     if (ds_slot >= 0 && (need == 0 || need > ws_limit_bytes(device_index(dev)))) {
       if (acquired && lazy->dispose != nullptr) lazy->dispose(lazy);
       return FA_ERROR_NOT_SUPPORTED;
     }
     const bool nested = t_ws_nested.active;
+    void* ws = nullptr;
+    bool held = false;
     if (nested) {
       // (the caller holds the buffer and has set a part of it aside)
-      if (need > 0 && (size_t)need <= t_ws_nested.bytes) {
-        ds_ws = t_ws_nested.ptr;
-        a.ds_ntq = ntq;
-        a.ds_ntk = ntk;
-        a.lse_scaled = reinterpret_cast<const float*>(static_cast<char*>(ds_ws) + ds_bytes);
-        a.delta_prep = reinterpret_cast<const float*>(static_cast<char*>(ds_ws) + ds_bytes + stat_bytes);
-      }
-    } else if (need > 0 && need <= ws_limit_bytes(device_index(dev))) {
-      if (!stream_is_capturing(stream)) {
-        if (ws_acquire(device_index(dev), (size_t)need, stream, &ds_ws) == hipSuccess) {
-          a.ds_ntq = ntq;
-          a.ds_ntk = ntk;
-          a.lse_scaled = reinterpret_cast<const float*>(static_cast<char*>(ds_ws) + ds_bytes);
-          a.delta_prep = reinterpret_cast<const float*>(static_cast<char*>(ds_ws) + ds_bytes + stat_bytes);
-        } else {
-          ds_ws = nullptr;
-          FA_LOG(2, "attn_bwd: no workspace of %lld bytes for dS, recomputing instead", (long long)need);
-        }
+      if ((size_t)(need + parts.bytes) <= t_ws_nested.bytes) ws = t_ws_nested.ptr;
+    } else if (need + parts.bytes > 0 && need + parts.bytes <= ws_limit_bytes(device_index(dev)) && !stream_is_capturing(stream)) {
+      held = ws_acquire(device_index(dev), (size_t)(need + parts.bytes), stream, &ws) == hipSuccess;
+      if (!held) {
+        ws = nullptr;
+        FA_LOG(2, "attn_bwd: no workspace of %lld bytes, recomputing instead", (long long)(need + parts.bytes));
       }
     }
+    if (ws != nullptr && need > 0) {
+      ds_ws = ws;
+      a.ds_ntq = ntq;
+      a.ds_ntk = ntk;
+      a.lse_scaled = reinterpret_cast<const float*>(static_cast<char*>(ds_ws) + ds_bytes);
+      a.delta_prep = reinterpret_cast<const float*>(static_cast<char*>(ds_ws) + ds_bytes + stat_bytes);
+    }
+    const bool cut = ws != nullptr && parts.bytes > 0;
+    if (cut) {
+      a.part_heads = parts.heads; a.part_tiles = parts.tiles;
+      a.part_ws = reinterpret_cast<float*>(static_cast<char*>(ws) + need);
+    }
+    auto run_dkdv = [&]() {
+      return (cut ? fa::run_bwd_dkdv_parts : fa::run_bwd_dkdv)(dt, s.d, a, s.windowed, s.bias, s.dropout, stream);
+    };
     if (ds_slot >= 0 && ds_ws == nullptr) {
       if (acquired && lazy->dispose != nullptr) lazy->dispose(lazy);
       return FA_ERROR_NOT_SUPPORTED;          // under stream capture, or no memory
@@ -1172,9 +1225,9 @@ static int attn_bwd_impl(const fa_bwd_params* p_in, int32_t params_version, void
       if (ds_slot < 0 || ds_slot == 0) err = fa::run_bwd_preprocess(dt, s.d, a, stream);
       a.ds_ws = ds_ws;
       if (err == hipSuccess && (ds_slot < 0 || ds_slot == 1))
-        err = fa::run_bwd_dkdv(dt, s.d, a, s.windowed, s.bias, s.dropout, stream);
+        err = run_dkdv();
       if (err == hipSuccess && (ds_slot < 0 || ds_slot == 2)) err = fa::run_bwd_dqs(dt, s.d, a, stream);
-      if (!nested) ws_release(device_index(dev), stream);
+      if (held) ws_release(device_index(dev), stream);
       if (acquired && lazy->dispose != nullptr) lazy->dispose(lazy);
       return (int)err;
     }
@@ -1191,9 +1244,10 @@ static int attn_bwd_impl(const fa_bwd_params* p_in, int32_t params_version, void
       else if (big)
         err = fa::run_bwd_d512(dt, slot, a, s.windowed, s.bias, s.dropout, stream);
       else
-        err = slot == 1 ? fa::run_bwd_dkdv(dt, s.d, a, s.windowed, s.bias, s.dropout, stream)
+        err = slot == 1 ? run_dkdv()
                         : fa::run_bwd_dq(dt, s.d, a, s.windowed, s.bias, s.dropout, stream);
     }
+    if (held) ws_release(device_index(dev), stream);
     if (acquired && lazy->dispose != nullptr) lazy->dispose(lazy);   // attn_bwd.cc:157
   } else {
     a.delta = nullptr;

@@ -94,6 +94,11 @@ struct BwdArgs {
   // with ds_ws: row statistics as that dK/dV kernel stages them, written by the delta kernel
   const float* lse_scaled;   // L / ln 2
   const float* delta_prep;   // -delta (delta with dropout)
+  // dK/dV items cut into parts (few keys, many queries or q-heads): part_heads parts of the GQA group's
+  // q-heads times part_tiles parts of the query tiles; each part's fp32 sums go to part_ws as
+  // (sequence and kv-head, key tile, part, dK then dV, key, column), where a second kernel adds them up
+  int32_t part_heads, part_tiles;
+  float* part_ws;            // null: not cut
 };
 
 // Copy between a rank-4 tensor of any strides and head dim (unit last stride) and its packed

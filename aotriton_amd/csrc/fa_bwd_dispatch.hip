@@ -23,6 +23,7 @@ namespace fa {
   }
 
 FA_DECL(run_bwd_dkdv)
+FA_DECL(run_bwd_dkdv_parts)
 FA_DECL(run_bwd_dq)
 FA_DECL(run_bwd_fused)
 #undef FA_DECL

@@ -14,7 +14,7 @@
 
 namespace fa {
 hipError_t FA_RUN(int dtype, const BwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s) {
-  if (dtype == kDtypeBF16) return launch_bwd_dkdv<bf16_t, 128, FA_PADDED != 0>(a, windowed, bias, dropout, s);
-  return launch_bwd_dkdv<f16_t, 128, FA_PADDED != 0>(a, windowed, bias, dropout, s);
+  if (dtype == kDtypeBF16) return launch_bwd_dkdv<bf16_t, 128, FA_PADDED != 0, false>(a, windowed, bias, dropout, s);
+  return launch_bwd_dkdv<f16_t, 128, FA_PADDED != 0, false>(a, windowed, bias, dropout, s);
 }
 }  // namespace fa

@@ -130,8 +130,8 @@ template <typename T, int D> struct DsTile {
 // kStoreDs: dS of every visited tile pair is also written to BwdArgs::ds_ws, and the row statistics
 // come prepared (BwdArgs::lse_scaled, delta_prep) so that they can travel straight into LDS.
 template <typename T, int D, int NW, int BM, bool kWindowed, bool kBias, bool kDropout, bool kInlineDelta, bool kPad,
-          bool kStoreDs = false>
-__device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const int nt, const int z,
+          bool kStoreDs = false, bool kParts = false>
+__device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const int nt, const int z, const int part,
                                           char* smem_raw) {
   using Tr = Traits<T>;
   using op_t = typename Tr::op_t;
@@ -161,7 +161,22 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
   w.right = w.right > (1 << 30) ? (1 << 30) : (w.right < -(1 << 30) ? -(1 << 30) : w.right);
   // Rows are keys here, columns are queries: key n sees query m iff n - right <= m <= n + left
   // (bwd_kernel_dk_dv.py:268-279 passes the window transposed in the same way).
-  const BlockRanges br = block_ranges(kWindowed, w.right, w.left, n0, si.seqlen_k, si.seqlen_q, BN, BM);
+  BlockRanges br = block_ranges(kWindowed, w.right, w.left, n0, si.seqlen_k, si.seqlen_q, BN, BM);
+
+  // this part's q-heads [g_lo, g_hi) and query tiles; all of them unless the item is cut (kParts)
+  const int group = a.hq / a.hk;
+  int g_lo = 0, g_hi = group;
+  float* part_ptr = nullptr;      // (a template flag: the extra state costs the uncut kernels 10 registers, and spills at D = 256)
+  if (kParts) {
+    const int ph = part / a.part_tiles, pt = part % a.part_tiles;
+    const int hs = group / a.part_heads;      // (part_heads divides the group)
+    g_lo = ph * hs;
+    g_hi = g_lo + hs;
+    const int per = (br.hi - br.lo + a.part_tiles) / a.part_tiles;
+    br.lo += pt * per;
+    if (br.lo + per - 1 < br.hi) br.hi = br.lo + per - 1;
+    part_ptr = a.part_ws + (((int64_t)(z * a.hk + hk) * a.num_n_tiles + nt) * (a.part_heads * a.part_tiles) + part) * (2 * BN * D);
+  }
 
   const int key = n0 + wave * 32 + c;
   const bool key_ok = key < si.seqlen_k;
@@ -171,6 +186,11 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
   T* dvptr = reinterpret_cast<T*>(a.dv) + (int64_t)si.batch_index * a.sdv.z + (int64_t)hk * a.sdv.h +
              (int64_t)(si.k_start + key_c) * a.sdv.s;
 
+  if (kParts && br.lo > br.hi) {      // nothing in this part
+    const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
+    for (int e = tid; e < 2 * BN * D / 4; e += NT) *reinterpret_cast<f32x4*>(part_ptr + 4 * e) = zero4;
+    return;
+  }
   if (br.lo > br.hi) {   // no query sees these keys
     if (key_ok) {
       q4_t zero4 = {0, 0, 0, 0};
@@ -217,9 +237,8 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
 #pragma unroll
     for (int i = 0; i < 16; ++i) { dk[db][i] = 0.f; dv[db][i] = 0.f; }
 
-  const int group = a.hq / a.hk;
   const int ntq = br.hi - br.lo + 1;
-  const int total = group * ntq;
+  const int total = (g_hi - g_lo) * ntq;
   const float qk_scale = a.sm_scale * kLog2e;
   // lane constants of the two LDS access patterns
   const int row_a = Swz<D>::row_base(lane), tr_a0 = Swz<D>::tr_base(lane, 0), tr_a1 = Swz<D>::tr_base(lane, 1);
@@ -798,7 +817,7 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
       *reinterpret_cast<op_t*>(smem_raw + SM::V_OFF + Swz<D>::addr(row, cc0)) = x;
     }
   }
-  fetch_begin(true, 0, 0);
+  fetch_begin(true, g_lo, 0);
 #pragma unroll
   for (int i = 0; i < FETCH_PIECES; ++i) fetch_piece(i);
 #pragma unroll
@@ -808,10 +827,11 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
   __syncthreads();
   // Per q-head the Q tiles come as [masked | full | masked]; each run has its own
   // loop so that the loop bodies are straight-line code.
-  const int n_lb = br.fb_lo <= br.fb_hi ? br.fb_lo - br.lo : ntq;
-  const int n_fb = br.fb_lo <= br.fb_hi ? br.fb_hi - br.fb_lo + 1 : 0;
+  const int fb_lo = kParts && br.fb_lo < br.lo ? br.lo : br.fb_lo, fb_hi = kParts && br.fb_hi > br.hi ? br.hi : br.fb_hi;
+  const int n_lb = fb_lo <= fb_hi ? fb_lo - br.lo : ntq;
+  const int n_fb = fb_lo <= fb_hi ? fb_hi - fb_lo + 1 : 0;
   int it = 0;
-  int g_cur = 0, e_cur = 0;
+  int g_cur = g_lo, e_cur = 0;
   auto step = [&](auto masked_tag) {
     const int stage = it & 1;
     int g_nxt = g_cur, e_nxt = e_cur + 1;
@@ -821,12 +841,24 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
     ++it;
     g_cur = g_nxt; e_cur = e_nxt;
   };
-  for (int g = 0; g < group; ++g) {
+  for (int g = g_lo; g < g_hi; ++g) {
     for (int e = 0; e < n_lb; ++e) step(std::true_type{});
     for (int e = 0; e < n_fb; ++e) step(std::false_type{});
     for (int e = n_lb + n_fb; e < ntq; ++e) step(std::true_type{});
   }
 
+  if (kParts) {
+    float* pk = part_ptr + (wave * 32 + c) * D + 4 * hi;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        *reinterpret_cast<f32x4*>(pk + 32 * db + 8 * g) = f32x4{dk[db][4 * g], dk[db][4 * g + 1], dk[db][4 * g + 2], dk[db][4 * g + 3]};
+        *reinterpret_cast<f32x4*>(pk + BN * D + 32 * db + 8 * g) =
+            f32x4{dv[db][4 * g], dv[db][4 * g + 1], dv[db][4 * g + 2], dv[db][4 * g + 3]};
+      }
+    return;
+  }
   if (key_ok) {
 #pragma unroll
     for (int db = 0; db < DB; ++db)
@@ -1387,7 +1419,8 @@ __host__ __device__ inline bool dkdv_level_list(const BwdArgs& a) {
   return D < 256 && a.seq.num_seqlens != 0 && a.bias == nullptr && a.zh_per_xcd <= kLevelCap && a.num_n_tiles <= 0xffff;
 }
 
-template <typename T, int D, int NW, int BM, bool kWindowed, bool kBias, bool kDropout, bool kPad, bool kStoreDs = false>
+template <typename T, int D, int NW, int BM, bool kWindowed, bool kBias, bool kDropout, bool kPad, bool kStoreDs = false,
+          bool kParts = false>
 __global__ __attribute__((amdgpu_flat_work_group_size(NW * 64, NW * 64)))
 void bwd_dkdv_kernel(const BwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
@@ -1409,15 +1442,17 @@ void bwd_dkdv_kernel(const BwdArgs a) {
                        zh_lo + a.zh_per_xcd < a.num_zh ? zh_lo + a.zh_per_xcd : a.num_zh, a.num_zh / a.hk, 1, NW * 32, true,
                        threadIdx.x);
   // (D = 256 is launched with one workgroup per item: the loop would cost registers there)
+  const int parts = kParts ? a.part_heads * a.part_tiles : 1;
   for (int r = 0; D >= 256 ? r < 1 : r * workers < a.items_per_xcd; ++r) {
-    const int li = r * workers + ((r & 1) ? workers - 1 - p : p);
+    const int lp = r * workers + ((r & 1) ? workers - 1 - p : p);
+    const int li = lp / parts;
     int zh, nt;
     if (ragged) {
       int e;
       if (!walk.at(li, e, nt)) break;
       zh = zh_lo + e;
     } else {
-      if (li >= a.items_per_xcd) continue;
+      if (lp >= a.items_per_xcd) continue;
       const int gi = li / per_group, gr = li % per_group;
       const int zl = gi * a.zh_group + gr % a.zh_group;
       zh = zh_lo + zl;
@@ -1426,7 +1461,7 @@ void bwd_dkdv_kernel(const BwdArgs a) {
     }
     int z, hk;
     split_zh(zh, a.num_zh / a.hk, 1, z, hk);
-    dkdv_item<T, D, NW, BM, kWindowed, kBias, kDropout, false, kPad, kStoreDs>(a, hk, nt, z, smem_raw);
+    dkdv_item<T, D, NW, BM, kWindowed, kBias, kDropout, false, kPad, kStoreDs, kParts>(a, hk, nt, z, kParts ? lp % parts : 0, smem_raw);
     __syncthreads();     // the next item reuses the LDS stages
   }
 }
@@ -1481,7 +1516,7 @@ void bwd_fused_kernel(const BwdArgs a) {
     split_zh(zh, a.num_zh / a.hk, 1, z, hk);
     const int item = gr / a.zh_group;
     if (item < a.num_n_tiles) {
-      dkdv_item<T, D, NW, BM, kWindowed, kBias, kDropout, true, kPad>(a, hk, item, z, smem_raw);
+      dkdv_item<T, D, NW, BM, kWindowed, kBias, kDropout, true, kPad>(a, hk, item, z, 0, smem_raw);
     } else {
       const int t = item - a.num_n_tiles;
       const int h = hk * group + t / a.num_m_tiles;
@@ -1549,7 +1584,36 @@ hipError_t launch_bwd_preprocess(const BwdArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
-template <typename T, int D, bool kPad, bool W, bool B, bool P>
+// dK, dV = the sums of the parts' fp32 dK (times the scale) and dV: one thread = four columns of one key
+// of one of the two.
+template <typename T, int D>
+static __global__ __launch_bounds__(256) void combine_dkdv_kernel(const BwdArgs a) {
+  using q4_t = typename Traits<T>::q4_t;
+  constexpr int BN = 128, QPR = D / 4;
+  const int gid = blockIdx.x * 256 + threadIdx.x;
+  const int col = gid % QPR * 4, key_l = gid / QPR % BN, which = gid / (QPR * BN) % 2, item = gid / (QPR * BN * 2);
+  const int nt = item % a.num_n_tiles, zh = item / a.num_n_tiles;
+  if (zh >= a.num_zh) return;
+  const int z = zh / a.hk, hk = zh % a.hk;
+  const SeqInfo si = get_seq(a.seq, z);
+  const int key = nt * BN + key_l;
+  if (key >= si.seqlen_k || col >= (which ? a.head_dim_v : a.head_dim)) return;
+  const int parts = a.part_heads * a.part_tiles;
+  const float* p = a.part_ws + ((int64_t)item * parts * 2 + which) * (BN * D) + key_l * D + col;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int i = 0; i < parts; ++i) acc += *reinterpret_cast<const f32x4*>(p + (int64_t)i * (2 * BN * D));
+  const Strides3& st = which ? a.sdv : a.sdk;
+  T* out = reinterpret_cast<T*>(which ? a.dv : a.dk) + (int64_t)si.batch_index * st.z + (int64_t)hk * st.h +
+           (int64_t)(si.k_start + key) * st.s + col;
+  const float f = which ? 1.0f : a.sm_scale;
+  q4_t t4;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) t4[r] = Traits<T>::cvt(acc[r] * f);
+  *reinterpret_cast<q4_t*>(out) = t4;
+}
+
+template <typename T, int D, bool kPad, bool W, bool B, bool P, bool kParts>
 hipError_t launch_dkdv_variant(const BwdArgs& a0, hipStream_t stream) {
   using Tile = BwdTile<T, D, W>;
   constexpr int NW = Tile::NW, BM = Tile::DKDV_BM, BN = NW * 32;
@@ -1558,23 +1622,28 @@ hipError_t launch_dkdv_variant(const BwdArgs& a0, hipStream_t stream) {
   a.num_zh = bwd_nseq(a) * a.hk;
   a.zh_per_xcd = (a.num_zh + kNumXcd - 1) / kNumXcd;
   a.zh_group = 2;
-  a.items_per_xcd = ((a.zh_per_xcd + a.zh_group - 1) / a.zh_group) * a.zh_group * a.num_n_tiles;
+  a.items_per_xcd = ((a.zh_per_xcd + a.zh_group - 1) / a.zh_group) * a.zh_group * a.num_n_tiles *
+                    (kParts ? a.part_heads * a.part_tiles : 1);
   dim3 grid((unsigned)(kNumXcd * persistent_workers<D>(a)));
   // (the level table's LDS is requested whether or not this launch uses it: the kernel's limit is set once)
   constexpr int smem = DkDvSmem<D, BM>::BYTES + (D < 256 ? kLevelBytes : 0);
-  if (a.ds_ws != nullptr) {
-    // (every build has the variant that stores dS; the host decides where it pays)
-    if constexpr (D == 64 || D == 128 || D == 256)
-      return launch_with_lds<bwd_dkdv_kernel<T, D, NW, BM, W, B, P, kPad, true>>(grid, NW * 64, smem, stream, a);
-    else
-      return hipErrorNotSupported;
+  // (every build has the variant that stores dS; the host decides where it pays)
+  hipError_t e = a.ds_ws != nullptr
+                     ? launch_with_lds<bwd_dkdv_kernel<T, D, NW, BM, W, B, P, kPad, true, kParts>>(grid, NW * 64, smem, stream, a)
+                     : launch_with_lds<bwd_dkdv_kernel<T, D, NW, BM, W, B, P, kPad, false, kParts>>(grid, NW * 64, smem, stream, a);
+  if constexpr (kParts) {
+    const int64_t threads = (int64_t)a.num_zh * a.num_n_tiles * 2 * BN * (D / 4);
+    if (e == hipSuccess && threads > 0) {
+      hipLaunchKernelGGL((combine_dkdv_kernel<T, D>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, a);
+      e = hipGetLastError();
+    }
   }
-  return launch_with_lds<bwd_dkdv_kernel<T, D, NW, BM, W, B, P, kPad>>(grid, NW * 64, smem, stream, a);
+  return e;
 }
 
-template <typename T, int D, bool kPad>
+template <typename T, int D, bool kPad, bool kParts>
 hipError_t launch_bwd_dkdv(const BwdArgs& a0, bool windowed, bool bias, bool dropout, hipStream_t stream) {
-#define FA_CALL(W, B, P) launch_dkdv_variant<T, D, kPad, W, B, P>(a0, stream)
+#define FA_CALL(W, B, P) launch_dkdv_variant<T, D, kPad, W, B, P, kParts>(a0, stream)
   FA_BWD_SWITCH(FA_CALL)
 #undef FA_CALL
 }

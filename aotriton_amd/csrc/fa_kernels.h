@@ -38,6 +38,8 @@ hipError_t run_mfma_rate(bool random_operands, int grid, int iters, float* out, 
 // backward: kernel_slot 0 = preprocess (delta), 1 = dK/dV, 2 = dQ, 3 = fused
 hipError_t run_bwd_preprocess(int dtype, int head_dim, const BwdArgs& a, hipStream_t s);
 hipError_t run_bwd_dkdv(int dtype, int head_dim, const BwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
+// the same with the items cut into parts and a kernel behind it that adds the parts up (BwdArgs::part_ws)
+hipError_t run_bwd_dkdv_parts(int dtype, int head_dim, const BwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
 hipError_t run_bwd_dq(int dtype, int head_dim, const BwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
 hipError_t run_bwd_fused(int dtype, int head_dim, const BwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
 TileShape bwd_tile_shape(int dtype, int head_dim, bool windowed, int kernel_slot);
