@@ -497,10 +497,23 @@ int validate_bwd(const fa_bwd_params* p, int32_t version, const fa_options* opt,
   return FA_SUCCESS;
 }
 
+// fp32: the kernels whose waves share 32 rows (fa_f32_rows.hip) or those that split the head dim over the
+// waves (fa_f32.hip)?  The first at 64 columns always (the second are compiled for 128).  At 128 columns the
+// forward is level on a full chip (2 % faster without a mask, 3 % slower under a causal mask with
+// grouped heads) and up to 1.8 x faster below that; the backward, whose dK/dV kernel lacks registers
+// there, gains up to 128 tiles of 64 rows (4-11 %) and loses from 168 on (15-50 %).
+bool f32_rows(const Shape& s, bool backward, int num_cu) {
+  const int64_t nz = s.num_seqlens != 0 ? std::abs(s.num_seqlens) : s.batch;
+  const int64_t tiles = nz * s.hq * ((s.max_sq + 63) / 64);
+  if (s.d == 64) return true;
+  if (s.d != 128) return false;
+  return backward ? tiles <= num_cu / 2 : !s.windowed || tiles < 4 * num_cu;
+}
+
 hipError_t run_fwd(int dtype, int d, const fa::FwdArgs& a, const Shape& s, hipStream_t stream) {
   if (s.elementwise) return fa::run_fwd_valu(dtype, d, a, stream);
   if (dtype == FA_DTYPE_FLOAT32)
-    return fa::run_fwd_f32(d, a, s.windowed, s.bias, s.dropout, stream);
+    return (f32_rows(s, false, a.num_cu) ? fa::run_fwd_f32_rows : fa::run_fwd_f32)(d, a, s.windowed, s.bias, s.dropout, stream);
   if (d > 256) return fa::run_fwd_d512(dtype, a, s.windowed, s.bias, s.dropout, stream);
   const bool padded = a.head_dim != d || a.head_dim_v != d;   // head dim rounded up: the copies that mask the excess columns
   switch (d) {
@@ -756,7 +769,9 @@ int fa_query_fwd_config(const fa_fwd_params* params, int32_t num_cu, fa_kernel_c
   if (e != FA_SUCCESS) return e;
   // the vector-ALU kernels (3-D grid), the fp32 kernels and the split-head-dim kernels (above 256)
   const bool valu = params->Q.dtype == FA_DTYPE_FLOAT32 || s.d > 256 || s.elementwise;
+  const bool rows32 = !s.elementwise && params->Q.dtype == FA_DTYPE_FLOAT32 && f32_rows(s, false, num_cu > 0 ? num_cu : 256);
   const fa::TileShape t = s.elementwise ? fa::TileShape{32, 1, 4, 0}
+                          : rows32 ? fa::f32_rows_tile_shape(s.d)
                           : params->Q.dtype == FA_DTYPE_FLOAT32 ? fa::f32_tile_shape(s.d, -1)
                           : s.d > 256 ? fa::d512_tile_shape(-1)
                                       : fa::fwd_tile_shape(params->Q.dtype, s.d, s.windowed);
@@ -767,6 +782,9 @@ int fa_query_fwd_config(const fa_fwd_params* params, int32_t num_cu, fa_kernel_c
     const int mt = (s.max_sq + t.block_m - 1) / t.block_m;
     if (s.elementwise) {      // vector-ALU kernels: 3-D grid
       out->grid[0] = mt; out->grid[1] = s.hq; out->grid[2] = nz;
+    } else if (rows32) {      // one workgroup per tile, the tiles of an XCD consecutive
+      out->grid[0] = fa::kNumXcd * ((nz * s.hq * mt + fa::kNumXcd - 1) / fa::kNumXcd);
+      out->grid[1] = 1; out->grid[2] = 1;
     } else {      // one workgroup per tile, the tiles of a kv-head's group back to back on one XCD
       out->grid[0] = fa::kNumXcd * ((nz * s.hk + fa::kNumXcd - 1) / fa::kNumXcd) * (s.hq / s.hk) * mt;
       out->grid[1] = 1; out->grid[2] = 1;
@@ -808,7 +826,9 @@ int fa_query_bwd_config(const fa_bwd_params* params, const fa_options* options, 
   if (valu && kernel_slot == 3) return FA_ERROR_PEER_ACCESS_UNSUPPORTED;
   const bool split_d = !s.elementwise && params->Q.dtype != FA_DTYPE_FLOAT32 && s.d > 256 && kernel_slot != 0;
   const bool f32_mfma = !s.elementwise && params->Q.dtype == FA_DTYPE_FLOAT32 && kernel_slot != 0;
-  const fa::TileShape t = f32_mfma ? fa::f32_tile_shape(s.d, kernel_slot)
+  const bool rows32 = f32_mfma && f32_rows(s, true, 256);
+  const fa::TileShape t = rows32 ? fa::f32_rows_tile_shape(s.d)
+                          : f32_mfma ? fa::f32_tile_shape(s.d, kernel_slot)
                           : split_d ? fa::d512_tile_shape(kernel_slot)
                           : valu  ? (kernel_slot == 1 ? fa::TileShape{1, 32, 4, 0} : fa::TileShape{32, 1, 4, 0})
                                   : fa::bwd_tile_shape(params->Q.dtype, s.d, s.windowed, kernel_slot);
@@ -831,7 +851,10 @@ int fa_query_bwd_config(const fa_bwd_params* params, const fa_options* options, 
   const int ratio = s.hq / s.hk;
   out->grid[1] = 1;
   out->grid[2] = 1;
-  if (f32_mfma || split_d) {      // one workgroup per tile, the tiles of a kv-head back to back on one XCD
+  if (rows32) {
+    const int items = kernel_slot == 1 ? nz * s.hk * nt : nz * s.hq * mt;
+    out->grid[0] = fa::kNumXcd * ((items + fa::kNumXcd - 1) / fa::kNumXcd);
+  } else if (f32_mfma || split_d) {      // one workgroup per tile, the tiles of a kv-head back to back on one XCD
     out->grid[0] = fa::kNumXcd * ((nz * s.hk + fa::kNumXcd - 1) / fa::kNumXcd) * (kernel_slot == 1 ? nt : ratio * mt);
   } else if (valu) {
     out->grid[0] = kernel_slot == 1 ? nt : mt;
@@ -1167,7 +1190,9 @@ static int attn_bwd_impl(const fa_bwd_params* p_in, int32_t params_version, void
     // 16-bit types up to head dim 256 computes delta from the O and dO rows it holds and writes it
     // out; the dK/dV kernel runs after it and reads it, so the whole backward is two launches
     // (kernel_slot 0 still launches the preprocess kernel on its own).
-    const bool delta_launch = f32 || big || slow;
+    // (fa_f32_rows.hip does the same)
+    const bool rows32 = f32 && f32_rows(s, true, dev->num_cu);
+    const bool delta_launch = (f32 && !rows32) || big || slow;
     // The 16-bit kernels up to head dim 256 can keep dS in HBM instead of recomputing S and dP in
     // the dQ kernel (5 GEMMs instead of 7): delta first, then dK/dV writing dS, then dQ = dS K.  It
     // takes 2 bytes per (query, key) pair of workspace; when that is above the limit, under stream
@@ -1232,7 +1257,7 @@ static int attn_bwd_impl(const fa_bwd_params* p_in, int32_t params_version, void
       return (int)err;
     }
     if (kernel_slot == 0 || (kernel_slot < 0 && delta_launch))
-      err = delta_launch ? fa::run_bwd_valu(dt, s.d, 0, a, stream) : fa::run_bwd_preprocess(dt, s.d, a, stream);
+      err = delta_launch || f32 ? fa::run_bwd_valu(dt, s.d, 0, a, stream) : fa::run_bwd_preprocess(dt, s.d, a, stream);
     const int order[2] = {delta_launch ? 1 : 2, delta_launch ? 2 : 1};
     for (int i = 0; i < 2 && err == hipSuccess; ++i) {
       const int slot = order[i];
@@ -1240,7 +1265,7 @@ static int attn_bwd_impl(const fa_bwd_params* p_in, int32_t params_version, void
       if (slow)
         err = fa::run_bwd_valu(dt, s.d, slot, a, stream);
       else if (f32)
-        err = fa::run_bwd_f32(s.d, slot, a, s.windowed, s.bias, s.dropout, stream);
+        err = (rows32 ? fa::run_bwd_f32_rows : fa::run_bwd_f32)(s.d, slot, a, s.windowed, s.bias, s.dropout, stream);
       else if (big)
         err = fa::run_bwd_d512(dt, slot, a, s.windowed, s.bias, s.dropout, stream);
       else

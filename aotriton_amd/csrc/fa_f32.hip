@@ -20,7 +20,7 @@
 // split over four waves that work on the same 32 rows, the GEMMs that contract over the head dim
 // exchange 32 x 32 partial blocks through LDS, and in the backward each wave does a quarter of the
 // element work and hands P and dS on.  Compiled for 128, 256 and 512 columns (smaller head dims
-// zero-filled).  At 512 columns two staged tiles fill 128 KB of the 160 KB of LDS: the forward and
+// zero-filled; up to 64 columns, and small batches at 128, run on fa_f32_rows.hip).  At 512 columns two staged tiles fill 128 KB of the 160 KB of LDS: the forward and
 // the dQ kernel then run one 32-row block per workgroup instead of two, and the partial blocks of
 // S and dP go through ONE area one after the other (two more barriers per tile, next to 256 MFMAs
 // of 64 cycles per wave).
@@ -856,7 +856,7 @@ hipError_t run_bwd_d(int kernel_slot, const BwdArgs& a, bool windowed, bool bias
 
 }  // namespace
 
-// head_dim: the compiled one that holds the tensors' head dims (64 runs on the 128-column kernels)
+// head_dim: the compiled one that holds the tensors' head dims
 hipError_t run_fwd_f32(int head_dim, const FwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s) {
   if (head_dim <= 128) return run_fwd_d<128>(a, windowed, bias, dropout, s);
   if (head_dim == 256) return run_fwd_d<256>(a, windowed, bias, dropout, s);

@@ -59,6 +59,12 @@ TileShape d512_tile_shape(int kernel_slot);
 hipError_t run_fwd_f32(int head_dim, const FwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
 hipError_t run_bwd_f32(int head_dim, int kernel_slot, const BwdArgs& a, bool windowed, bool bias, bool dropout,
                        hipStream_t s);
+// fp32, head dims up to 128 (compiled for 64 and 128 columns): four waves share 32 rows and split the other
+// side.  kernel_slot 2 also writes delta; kernel_slot 1 reads it.
+hipError_t run_fwd_f32_rows(int head_dim, const FwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
+hipError_t run_bwd_f32_rows(int head_dim, int kernel_slot, const BwdArgs& a, bool windowed, bool bias, bool dropout,
+                            hipStream_t s);
+TileShape f32_rows_tile_shape(int head_dim);
 TileShape f32_tile_shape(int head_dim, int kernel_slot);
 
 // Vector-ALU kernels (no MFMA): every type at every compiled head dim; they serve tensors whose

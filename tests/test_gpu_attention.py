@@ -696,3 +696,16 @@ def test_v2_positional_c_abi_matches_the_params_entry_points():
                                       True, s) == ok
     for a, b in zip(g1, g2):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize('shape', [
+    # B, Hq, Hk, Sq, Sk, D, causal, p, bias: blocks of 32 rows and 32 columns around their edges, shares of the
+    # four waves that are empty or ragged, both sides of the rule between the two families of fp32 kernels
+    (1, 1, 1, 1, 1, 64, False, 0.0, False), (1, 2, 1, 31, 33, 64, True, 0.0, False),
+    (2, 4, 2, 129, 97, 64, (40, 5), 0.0, False), (1, 2, 2, 65, 160, 40, False, 0.2, False),
+    (1, 2, 1, 70, 90, 56, True, 0.0, True), (1, 4, 2, 257, 130, 64, (10, -40), 0.1, True),
+    (2, 4, 4, 200, 75, 128, True, 0.0, False), (1, 2, 1, 33, 300, 96, False, 0.1, True),
+    (4, 16, 16, 270, 140, 128, False, 0.0, False)])
+def test_fp32_rows_kernels(shape):
+    B, Hq, Hk, Sq, Sk, D, causal, p, bias = shape
+    _run_case(B, Hq, Hk, Sq, Sk, D, torch.float32, causal, dropout_p=p, bias=bias, bshd=True, seed=17)
