@@ -34,13 +34,14 @@ struct FwdSmem {
   static constexpr int STAGES = 2;
   static constexpr int ROWS_OFF = STAGES * (K_ELEMS + V_ELEMS) * 2;   // the waves' row areas
   static constexpr int ROW_STR = D * 2 + 16;                          // bytes per staged Q / O row
-  static constexpr int BYTES = ROWS_OFF + NW * 32 * ROW_STR;
+  static constexpr int KEYB_OFF = ROWS_OFF + NW * 32 * ROW_STR;       // a bias that is the same for all rows: BN floats per stage
+  static constexpr int BYTES = KEYB_OFF + STAGES * BN * 4;
 };
 
 // One Q tile (BM rows of head h of sequence z) against all its visible K/V tiles, or with kSplit
 // against part `split` of a.splits of them: the fp32 sums and the row statistics of the part then go to
 // scratch memory, where combine_rows_kernel picks them up.
-template <typename T, int D, int NW, int BN, bool kWindowed, bool kBias, bool kDropout, bool kPad, bool kSplit>
+template <typename T, int D, int NW, int BN, bool kWindowed, bool kBias, bool kDropout, bool kPad, bool kSplit, bool kKeyBias>
 __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const int h, const int mt, const int split,
                                          char* smem_raw) {
   using Tr = Traits<T>;
@@ -147,6 +148,17 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
   const bool bias_vec = kBias && a.sb_n == 1 && ((a.sb_m | a.sb_h | a.sb_z) & 3) == 0 &&
                         (reinterpret_cast<uintptr_t>(a.bias) & 7) == 0;
 
+  // kKeyBias: a bias that does not depend on the query (row stride 0: a padding mask of keys) is staged
+  // with the K tile, one float per key in units of the exponent, and read back by broadcast.  As a general
+  // bias every wave would carry 32 copies of the row through its row area.  (A template flag: as one more
+  // run-time case it cost the general bias 5-15 % in spills.)
+  static_assert(kBias || !kKeyBias, "a bias of keys is a bias");
+  const T* kb_next = kKeyBias ? reinterpret_cast<const T*>(a.bias) + (int64_t)si.batch_index * a.sb_z + (int64_t)h * a.sb_h +
+                                 (int64_t)(br.lo * BN + tid) * a.sb_n
+                           : nullptr;
+  float kb_reg = 0.f;
+  float* const kb_lds = reinterpret_cast<float*>(smem_raw + SM::KEYB_OFF);
+
   DropoutState ds{};
   if (kDropout) ds = make_dropout(a.drop, z, h, a.hq, a.seq.max_seqlen_q, a.seq.max_seqlen_k);
 
@@ -183,6 +195,10 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
 #pragma unroll
     for (int i = 0; i < CH; ++i)
       vreg[i] = __builtin_bit_cast(op_t, __builtin_amdgcn_raw_buffer_load_b128(vrs, vvoff, i * vsoff, 0));
+    if (kKeyBias && tid < BN) {
+      kb_reg = tid < rows ? (float)*kb_next * kLog2e : 0.f;
+      kb_next += (int64_t)BN * a.sb_n;
+    }
     kt += k_step; vt += v_step; rows_left -= BN;
   };
 
@@ -216,6 +232,7 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
     for (int i = 0; i < CH; ++i) *reinterpret_cast<op_t*>(ks + i * RPI * KSTR) = kreg[i];
 #pragma unroll
     for (int i = 0; i < CH; ++i) *reinterpret_cast<op_t*>(vs + i * RPI * VSTR) = vreg[i];
+    if (kKeyBias && tid < BN) kb_lds[stage * BN + tid] = kb_reg;
   };
 
   // ---- online softmax state --------------------------------------------------
@@ -339,14 +356,23 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
   };
 
   // scale, bias and mask on the raw scores
-  auto prepare = [&](int j, bool masked) {
-    if (prescale) {
+  auto prepare = [&](int j, int stage, bool masked) {
+    if (kKeyBias) {
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const f32x4 b4 = *reinterpret_cast<const f32x4*>(kb_lds + stage * BN + mb * 32 + 8 * g + 4 * hi);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) s[mb][4 * g + r] = __builtin_fmaf(s[mb][4 * g + r], qk_scale, b4[r]);
+        }
+    } else if (prescale) {
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
         for (int i = 0; i < 16; ++i) s[mb][i] *= qk_scale;
     }
-    if (kBias) {
+    if (kBias && !kKeyBias) {
       if (bias_co && (j + 1) * BN <= si.seqlen_k) {
 #pragma unroll
         for (int ck = 0; ck < BN / BCK; ++ck) bias_chunk(j, ck);
@@ -441,7 +467,7 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
     const T* vs = Vs + stage * SM::V_ELEMS + v_lane;
 #pragma unroll
     for (int db = 0; db < DB; ++db) va[0][db] = lds_read_tr8<T>(vs + db * 32, VSTR);
-    prepare(j, masked);
+    prepare(j, stage, masked);
     float rs = 0.f;
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
@@ -463,7 +489,7 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
     // first V^T operands: in flight while the softmax runs
 #pragma unroll
     for (int db = 0; db < DB; ++db) va[0][db] = lds_read_tr8<T>(vs + db * 32, VSTR);
-    prepare(j, masked);
+    prepare(j, stage, masked);
     float mx = s[0][0];
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
@@ -588,7 +614,8 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
 // goes from one tile to the next without a relaunch.
 // QB = 0: fwd_item, NW waves of 32 rows.  QB > 0: fwd_item_pipe, 4 waves of 32 * QB rows, one wave
 // per SIMD.
-template <typename T, int D, int NW, int BN, int QB, bool kWindowed, bool kBias, bool kDropout, bool kPad, bool kSplit>
+template <typename T, int D, int NW, int BN, int QB, bool kWindowed, bool kBias, bool kDropout, bool kPad, bool kSplit,
+          bool kKeyBias>
 __global__ __attribute__((amdgpu_flat_work_group_size(NW * 64, NW * 64)))
 __attribute__((amdgpu_waves_per_eu(D <= 128 && QB == 0 ? 2 : 1, D <= 128 && QB == 0 ? 2 : 1)))
 void fwd_kernel(const FwdArgs a) {
@@ -648,7 +675,7 @@ void fwd_kernel(const FwdArgs a) {
       split_zh(zh, nseq, ratio, z, h);
     }
     if constexpr (QB > 0) fwd_item_pipe<T, D, QB, BN, kWindowed, kBias, kDropout, kPad>(a, z, h, mt, smem_raw);
-    else fwd_item<T, D, NW, BN, kWindowed, kBias, kDropout, kPad, kSplit>(a, z, h, mt, split, smem_raw);
+    else fwd_item<T, D, NW, BN, kWindowed, kBias, kDropout, kPad, kSplit, kKeyBias>(a, z, h, mt, split, smem_raw);
   }
 }
 
@@ -680,11 +707,12 @@ template <typename T, bool kWindowed> struct FwdTile<T, 128, kWindowed> : FwdTil
 // 629 vs 510; bias + dropout + window 1024: 361 vs 333).
 template <typename T, bool kWindowed> struct FwdTile<T, 256, kWindowed> : FwdTileOf<256, 4, 32, 1> {};
 
-template <typename T, int D, bool kWindowed, bool kBias, bool kDropout, bool kPad, bool kSplit = false>
+template <typename T, int D, bool kWindowed, bool kBias, bool kDropout, bool kPad, bool kSplit = false,
+          bool kKeyBias = false>
 hipError_t launch_fwd_variant(const FwdArgs& a, dim3 grid, hipStream_t stream) {
   using Tile = FwdTile<T, D, kWindowed>;
   constexpr int NW = Tile::NW;
-  auto kern = fwd_kernel<T, D, NW, Tile::BN, Tile::QB, kWindowed, kBias, kDropout, kPad, kSplit>;
+  auto kern = fwd_kernel<T, D, NW, Tile::BN, Tile::QB, kWindowed, kBias, kDropout, kPad, kSplit, kKeyBias>;
   constexpr int smem = Tile::LDS;
   if (grid.x == 0) return hipSuccess;      // no batch, no head or no query row: nothing to write
   if (smem > 64 * 1024) {
@@ -728,6 +756,12 @@ hipError_t launch_fwd(const FwdArgs& a, bool windowed, bool bias, bool dropout, 
         default: return launch_fwd_variant<T, D, true, true, false, kPad, true>(b, grid, stream);
       }
     }
+  }
+  // a bias that is the same for all rows (D <= 128, without dropout)
+  if constexpr (D <= 128) {
+    if (bias && !dropout && a.sb_m == 0)
+      return windowed ? launch_fwd_variant<T, D, true, true, false, kPad, false, true>(b, grid, stream)
+                      : launch_fwd_variant<T, D, false, true, false, kPad, false, true>(b, grid, stream);
   }
   const int key = (windowed ? 4 : 0) | (bias ? 2 : 0) | (dropout ? 1 : 0);
   switch (key) {

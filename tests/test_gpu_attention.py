@@ -709,3 +709,31 @@ def test_v2_positional_c_abi_matches_the_params_entry_points():
 def test_fp32_rows_kernels(shape):
     B, Hq, Hk, Sq, Sk, D, causal, p, bias = shape
     _run_case(B, Hq, Hk, Sq, Sk, D, torch.float32, causal, dropout_p=p, bias=bias, bshd=True, seed=17)
+
+
+@pytest.mark.parametrize('case', [
+    # B, H, Sq, Sk, D, dtype, causal: a mask of keys (one row for all queries), tiles whole and ragged, rows
+    # without a visible key
+    (2, 4, 300, 384, 64, torch.float16, False), (3, 2, 257, 933, 80, torch.bfloat16, False),
+    (2, 3, 513, 129, 64, torch.bfloat16, True), (1, 4, 700, 640, 128, torch.float16, (100, 30)),
+    (2, 2, 40, 70, 128, torch.bfloat16, False)])
+def test_bias_that_is_the_same_for_all_rows(case):
+    from aotriton_amd import flash
+    from aotriton_amd.autograd import attention, AttentionExtraArgs
+    from oracle import fa_ref
+    B, H, Sq, Sk, D, dtype, causal = case
+    q, k, v, _, _ = make_inputs(B, H, H, Sq, Sk, D, dtype, DEV, seed=41, bshd=True)
+    g = torch.Generator(device='cpu').manual_seed(3)
+    row = torch.randn(B, 1, 1, Sk, generator=g).to(dtype).to(DEV)
+    b = row.masked_fill(torch.arange(Sk, device=DEV) >= (2 * Sk) // 3, float('-inf')).expand(B, H, Sq, Sk)
+    sm = 1.0 / math.sqrt(D)
+    ct, wl, wr = flash.translate_causal(causal)
+    f = lambda t: t.float()
+    ro, rl, _ = fa_ref.attn_fwd_ref(f(q), f(k), f(v), f(b), sm, ct, wl, wr)
+    lo, _, _ = fa_ref.attn_fwd_ref(q, k, v, b, sm, ct, wl, wr)
+    o, _, L = attention(q, k, v, b, causal, sm, 0.0, AttentionExtraArgs(return_logsumexp=True, fillnan=True))
+    check('out', o, ro, lo, FUDGE['out'])
+    L = L.view(B, H, Sq)
+    assert torch.equal(torch.isinf(L), torch.isinf(rl))
+    seen = torch.isfinite(rl)
+    assert (L[seen] - rl[seen]).abs().max().item() <= LSE_ATOL
