@@ -29,19 +29,20 @@ COMMON = [
 
 
 # Per-file additions.  The dQ kernels post-process MFMA results with the vector ALU; letting
-# the register allocator keep those results in VGPRs saves the AGPR read per element.
+# the register allocator keep those results in VGPRs saves the AGPR read per element (kernels held to
+# 256 registers, two waves per SIMD, have their results there anyway).
 EXTRA = {
     # the ILP-first scheduling strategy: dK/dV kernel of the headline shape -1..2 % (same-box A/B,
     # no spills either way); level on the forward and the dQ-from-dS kernel, which keep the default
     'fa_bwd_dkdv_d128.hip': ['-mllvm', '-amdgpu-sched-strategy=max-ilp'],
     'fa_bwd_dkdv_parts_d128.hip': ['-mllvm', '-amdgpu-sched-strategy=max-ilp'],
-    'fa_bwd_dq_d64.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'],
+    'fa_bwd_dq_bias_d64.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'],
     'fa_bwd_dq_d128.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'],
 }
 
 # The per-head-dim kernel files are compiled a second time with FA_PADDED=1: the copies that
 # serve head dims rounded up to the compiled one.
-PADDED_RE = re.compile(r'fa_(fwd|fwd_rows|bwd_dkdv|bwd_dkdv_parts|bwd_dq|bwd_fused)_d\d+\.hip$')
+PADDED_RE = re.compile(r'fa_(fwd|fwd_rows|bwd_dkdv|bwd_dkdv_parts|bwd_dq|bwd_dq_bias|bwd_fused)_d\d+\.hip$')
 
 
 def sources():

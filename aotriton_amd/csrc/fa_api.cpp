@@ -637,7 +637,7 @@ int64_t ds_workspace_need(const fa_bwd_params* p, const Shape& s, int* ntq, int*
   // spared a bias or the Philox arithmetic (same box, stored / recomputing: 1.05-1.14 plain, 0.69-0.81 with either)
   if (s.d == 64 && !s.dropout && !s.bias) return 0;
   int64_t tile_bytes = 0;
-  fa::ds_tile_counts(p->Q.dtype, s.d, s.max_sq, s.max_sk, ntq, ntk, &tile_bytes);
+  fa::ds_tile_counts(p->Q.dtype, s.d, s.bias, s.dropout, s.max_sq, s.max_sk, ntq, ntk, &tile_bytes);
   *ds_bytes = (int64_t)s.batch * s.hq * *ntq * *ntk * tile_bytes;
   *stat_bytes = (s.row_stats * 4 + 255) & ~(int64_t)255;
   return *ds_bytes + 2 * *stat_bytes;

@@ -1,4 +1,4 @@
-// Backward dq kernel instantiations for head dim 64 (fp16 and bf16).
+// Backward dq kernel instantiations for head dim 64 without a bias (fp16 and bf16).
 #include "fa_bwd_impl.h"
 
 // Compiled twice: as is for tensors whose head dim is 64, and with FA_PADDED=1 for smaller
@@ -12,9 +12,17 @@
 #define FA_RUN run_bwd_dq_d64
 #endif
 
+#if FA_PADDED
+#define FA_RUN_BIAS run_bwd_dq_bias_d64_padded
+#else
+#define FA_RUN_BIAS run_bwd_dq_bias_d64
+#endif
+
 namespace fa {
+hipError_t FA_RUN_BIAS(int dtype, const BwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
 hipError_t FA_RUN(int dtype, const BwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s) {
-  if (dtype == kDtypeBF16) return launch_bwd_dq<bf16_t, 64, FA_PADDED != 0>(a, windowed, bias, dropout, s);
-  return launch_bwd_dq<f16_t, 64, FA_PADDED != 0>(a, windowed, bias, dropout, s);
+  if (bias) return FA_RUN_BIAS(dtype, a, windowed, bias, dropout, s);
+  if (dtype == kDtypeBF16) return launch_bwd_dq<bf16_t, 64, FA_PADDED != 0, 0>(a, windowed, bias, dropout, s);
+  return launch_bwd_dq<f16_t, 64, FA_PADDED != 0, 0>(a, windowed, bias, dropout, s);
 }
 }  // namespace fa

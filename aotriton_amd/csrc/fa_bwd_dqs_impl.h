@@ -32,13 +32,13 @@ struct DqsSmem {     // two stages of the K tile (swizzled), then one dS area pe
 };
 
 // One Q tile of 256 rows (8 waves x 32 queries) of head h against the key tiles that see it.
-template <typename T, int D, int BN, bool kPad>
+template <typename T, int D, int BN, bool kPad, bool kWideTile>
 __device__ __forceinline__ void dqs_item(const BwdArgs& a, const int h, const int mt, const int z, char* smem_raw) {
   using Tr = Traits<T>;
   using op_t = typename Tr::op_t;
   using q4_t = typename Tr::q4_t;
   using SM = DqsSmem<D, BN>;
-  using DT = DsTile<T, D>;
+  using DT = DsTile<T, D, kWideTile>;
   constexpr int NW = SM::NW, NT = NW * 64, BM = NW * 32;
   constexpr int DB = D / 32;
   constexpr int SPT = DT::BN / BN;          // steps per stored tile
@@ -200,7 +200,7 @@ __device__ __forceinline__ void dqs_item(const BwdArgs& a, const int h, const in
 
 // One workgroup per Q tile on a 1-D grid: consecutive ids go round the XCDs, an XCD takes its
 // (batch, q-head) pairs two at a time, the heaviest (last) tile of a causal mask first.
-template <typename T, int D, int BN, bool kPad>
+template <typename T, int D, int BN, bool kPad, bool kWideTile>
 __global__ __attribute__((amdgpu_flat_work_group_size(512, 512))) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void bwd_dqs_kernel(const BwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
@@ -213,7 +213,7 @@ void bwd_dqs_kernel(const BwdArgs a) {
   const int mt = a.num_m_tiles - 1 - gr / a.zh_group;
   int z, h;
   split_zh(zh, a.num_zh / a.hq, a.hq / a.hk, z, h);
-  dqs_item<T, D, BN, kPad>(a, h, mt, z, smem_raw);
+  dqs_item<T, D, BN, kPad, kWideTile>(a, h, mt, z, smem_raw);
 }
 
 template <typename T, int D, bool kPad>
@@ -226,7 +226,11 @@ hipError_t launch_bwd_dqs(const BwdArgs& a0, hipStream_t stream) {
   a.zh_group = a.hq / a.hk > 2 ? (a.hq / a.hk > 8 ? 8 : a.hq / a.hk) : 2;
   a.items_per_xcd = ((a.zh_per_xcd + a.zh_group - 1) / a.zh_group) * a.zh_group * a.num_m_tiles;
   dim3 grid((unsigned)(kNumXcd * a.items_per_xcd));
-  return launch_with_lds<bwd_dqs_kernel<T, D, BN, kPad>>(grid, 512, DqsSmem<D, BN>::BYTES, stream, a);
+  if constexpr (D == 64) {
+    if (a.bias != nullptr && !(a.drop.p > 0.f))      // kWide: how the dK/dV kernel of such a call stored it
+      return launch_with_lds<bwd_dqs_kernel<T, D, BN, kPad, true>>(grid, 512, DqsSmem<D, BN>::BYTES, stream, a);
+  }
+  return launch_with_lds<bwd_dqs_kernel<T, D, BN, kPad, false>>(grid, 512, DqsSmem<D, BN>::BYTES, stream, a);
 }
 
 }  // namespace fa

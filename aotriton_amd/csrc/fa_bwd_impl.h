@@ -95,16 +95,41 @@ struct DqSmem {     // per stage: K, V (swizzled); then one bias / dB tile per w
   static constexpr int BYTES = BIAS_OFF + 4 * 32 * BIAS_ROW;
 };
 
-// Tile table of the backward kernels, keyed on (element type, head dim, causal / windowed).  NW
-// waves; dK/dV: 32*NW keys per workgroup, DKDV_BM queries per step; dQ: 32*NW queries per
-// workgroup, DQ_BN keys per step.  The reference keeps separate tuned tiles for causal and
+// Tile table of the backward kernels, keyed on (element type, head dim, causal / windowed) and, at head dim
+// 64, on the options.  NW waves; dK/dV: 32*NW keys per workgroup, DKDV_BM queries per step; dQ: 32*NW
+// queries per workgroup, DQ_BN keys per step.  The reference keeps separate tuned tiles for causal and
 // non-causal shapes (its database has 64x16 / 64x32 for dK/dV and 64x64 / 64x32 for dQ at the
 // headline shape); here the same tile wins on both sides of every key (same-box A/B at D = 128,
 // bf16: 32-query / 32-key steps lose 6 % causal and 7-10 % non-causal on each kernel).
+// Head dim 64: with 64-query / 64-key steps the kernels without a bias fit 256 registers and run two
+// workgroups per CU, i.e. two waves per SIMD, which hide each other's prologues and phases (backward of
+// B4 H64 S4096: full 4.04 -> 3.65-3.8 ms, causal 2.25 -> 2.0-2.1; B8 H16 S512 47 -> 41.5 us, with dropout
+// B8 H12 S512 75.6 -> 63).  With a bias they do not (90-150 spilled registers): those keep one wave per SIMD
+// and 128-wide steps (64-wide ones lose 2-8 %), except that dK/dV with bias and dropout takes 64-query steps
+// (8 % faster).
 template <typename T, int D, bool kWindowed> struct BwdTile;
-template <typename T, bool kWindowed> struct BwdTile<T, 64, kWindowed>  { static constexpr int NW = 4, DKDV_BM = 128, DQ_BN = 128; };
+template <typename T, bool kWindowed> struct BwdTile<T, 64, kWindowed>  { static constexpr int NW = 4, DKDV_BM = 64, DQ_BN = 64; };
 template <typename T, bool kWindowed> struct BwdTile<T, 128, kWindowed> { static constexpr int NW = 4, DKDV_BM = 64, DQ_BN = 64; };
 template <typename T, bool kWindowed> struct BwdTile<T, 256, kWindowed> { static constexpr int NW = 4, DKDV_BM = 32, DQ_BN = 32; };
+// 128-query steps of the dK/dV kernel
+template <int D, bool kBias, bool kDropout> constexpr bool kWide = D == 64 && kBias && !kDropout;
+template <typename T, int D, bool kWindowed, bool kBias, bool kDropout>
+constexpr int kDkDvBM = kWide<D, kBias, kDropout> ? 128 : BwdTile<T, D, kWindowed>::DKDV_BM;
+template <typename T, int D, bool kWindowed, bool kBias>
+constexpr int kDqBN = D == 64 && kBias ? 128 : BwdTile<T, D, kWindowed>::DQ_BN;
+
+// Two workgroups per CU, two waves per SIMD (256 registers each)?
+template <int D, bool kBias> constexpr bool kTwoWaves = D == 64 && !kBias;
+// Position in the XCD's list of worker p in round r.  One workgroup per CU: serpentine, which pairs
+// heavy with light items.  Two per CU: the workgroups p and p + CUs of an XCD share a CU, so the second
+// half runs backwards through its part of the round, and every other round is turned round as a whole.
+template <bool kTwo>
+__device__ __forceinline__ int worker_pos(int r, int p, int workers, int num_cu) {
+  if (!kTwo) return r * workers + ((r & 1) ? workers - 1 - p : p);
+  const int c = num_cu / kNumXcd < workers ? num_cu / kNumXcd : workers;
+  const int pos = p < c ? p : c + workers - 1 - p;
+  return r * workers + ((r & 1) ? workers - 1 - pos : pos);
+}
 
 // Stored dS (BwdArgs::ds_ws): one tile per (batch element, q-head, key tile of 128, query tile of the
 // dK/dV step) holds 128 x BM values of the 16-bit type as [32-query block][32-key block][half of the
@@ -113,9 +138,9 @@ template <typename T, bool kWindowed> struct BwdTile<T, 256, kWindowed> { static
 // queries 16 t + 4 hi + {0..3} and 16 t + 8 + 4 hi + {0..3} (hi = lane / 32); it sits at piece position
 // (2 c + hi) ^ 8 (t & 1), where the transposing LDS reads of the kernel that consumes the tiles want
 // it.  A wave of that kernel owns one query block: what it needs of a tile is contiguous.
-template <typename T, int D> struct DsTile {
+template <typename T, int D, bool kWideTile> struct DsTile {
   static_assert(BwdTile<T, D, false>::DKDV_BM == BwdTile<T, D, true>::DKDV_BM, "one tile shape per head dim");
-  static constexpr int BM = BwdTile<T, D, false>::DKDV_BM;   // queries per stored tile
+  static constexpr int BM = kWideTile ? 128 : BwdTile<T, D, false>::DKDV_BM;   // queries per stored tile
   static constexpr int BN = 128;                             // keys per stored tile
   static constexpr int TS = BM / 16;                         // 1 KB pieces per 32-key block
   static constexpr int BYTES = BN * BM * 2;
@@ -253,7 +278,7 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
   // middle (where the compiler makes the first transposing read wait for the direct-to-LDS pieces
   // anyway), and the pieces leave in the half tile after it, as their operands get complete: the
   // youngest store is more than half a tile old at the next wait.
-  using DT = DsTile<T, D>;
+  using DT = DsTile<T, D, kWide<D, kBias, kDropout>>;
   static_assert(!kStoreDs || (!kInlineDelta && BM == DT::BM && BN == DT::BN), "stored tiles have the item's shape");
   const int ds_pos[2] = {((c << 1) | hi) << 4, (((c << 1) | hi) ^ 8) << 4};
   op_t sb[TS];                         // dS operands of the dK GEMM; with kStoreDs they outlive their tile
@@ -1025,7 +1050,7 @@ __device__ __forceinline__ void dq_item(const BwdArgs& a, const int h, const int
   // kernel needs more than 256 registers) but copies each one back before every use: 32-44
   // copies per key tile at D = 128, a quarter of the loop's vector instructions.  Not at
   // D = 256, where the allocation gets worse with the constraint.
-  if constexpr (D <= 128) {
+  if constexpr (D == 128 || (D == 64 && kBias)) {
 #pragma unroll
     for (int k = 0; k < KS; ++k) {
       asm volatile("" : "+a"(qreg[k]));
@@ -1421,7 +1446,7 @@ __host__ __device__ inline bool dkdv_level_list(const BwdArgs& a) {
 
 template <typename T, int D, int NW, int BM, bool kWindowed, bool kBias, bool kDropout, bool kPad, bool kStoreDs = false,
           bool kParts = false>
-__global__ __attribute__((amdgpu_flat_work_group_size(NW * 64, NW * 64)))
+__global__ __attribute__((amdgpu_flat_work_group_size(NW * 64, NW * 64))) __attribute__((amdgpu_waves_per_eu(kTwoWaves<D, kBias> ? 2 : 1, kTwoWaves<D, kBias> ? 2 : 1)))
 void bwd_dkdv_kernel(const BwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   // Persistent workgroups, one per CU (a relaunch per item costs a dispatch gap of several
@@ -1444,7 +1469,7 @@ void bwd_dkdv_kernel(const BwdArgs a) {
   // (D = 256 is launched with one workgroup per item: the loop would cost registers there)
   const int parts = kParts ? a.part_heads * a.part_tiles : 1;
   for (int r = 0; D >= 256 ? r < 1 : r * workers < a.items_per_xcd; ++r) {
-    const int lp = r * workers + ((r & 1) ? workers - 1 - p : p);
+    const int lp = worker_pos<kTwoWaves<D, kBias>>(r, p, workers, a.num_cu);
     const int li = lp / parts;
     int zh, nt;
     if (ragged) {
@@ -1467,7 +1492,7 @@ void bwd_dkdv_kernel(const BwdArgs a) {
 }
 
 template <typename T, int D, int NW, int BN, bool kWindowed, bool kBias, bool kDropout, bool kPad>
-__global__ __attribute__((amdgpu_flat_work_group_size(NW * 64, NW * 64)))
+__global__ __attribute__((amdgpu_flat_work_group_size(NW * 64, NW * 64))) __attribute__((amdgpu_waves_per_eu(kTwoWaves<D, kBias> ? 2 : 1, kTwoWaves<D, kBias> ? 2 : 1)))
 void bwd_dq_kernel(const BwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   // persistent workgroups with the same walk as the forward kernel: (batch, q-head) pairs
@@ -1476,7 +1501,7 @@ void bwd_dq_kernel(const BwdArgs a) {
   const int per_group = a.zh_group * a.num_m_tiles;
   // (D = 256 is launched with one workgroup per item: the loop would cost registers there)
   for (int r = 0; D >= 256 ? r < 1 : r * workers < a.items_per_xcd; ++r) {
-    const int li = r * workers + ((r & 1) ? workers - 1 - p : p);
+    const int li = worker_pos<kTwoWaves<D, kBias>>(r, p, workers, a.num_cu);
     if (li >= a.items_per_xcd) continue;
     const int gi = li / per_group, gr = li % per_group;
     const int zl = gi * a.zh_group + gr % a.zh_group;
@@ -1541,9 +1566,9 @@ inline int bwd_nseq(const BwdArgs& a) {
 // sequences of very different lengths.  D = 256 also gets one workgroup per item: its
 // dK/dV kernel has no register to spare for the loop.
 template <int D>
-inline int persistent_workers(const BwdArgs& a) {
+inline int persistent_workers(const BwdArgs& a, int per_cu) {
   if (a.bias != nullptr || D >= 256) return a.items_per_xcd;
-  int w = (a.num_cu > 0 ? a.num_cu : 256) / kNumXcd;
+  int w = (a.num_cu > 0 ? a.num_cu : 256) / kNumXcd * per_cu;
   if (w < 1) w = 1;
   return w > a.items_per_xcd ? a.items_per_xcd : w;
 }
@@ -1616,7 +1641,7 @@ static __global__ __launch_bounds__(256) void combine_dkdv_kernel(const BwdArgs 
 template <typename T, int D, bool kPad, bool W, bool B, bool P, bool kParts>
 hipError_t launch_dkdv_variant(const BwdArgs& a0, hipStream_t stream) {
   using Tile = BwdTile<T, D, W>;
-  constexpr int NW = Tile::NW, BM = Tile::DKDV_BM, BN = NW * 32;
+  constexpr int NW = Tile::NW, BM = kDkDvBM<T, D, W, B, P>, BN = NW * 32;
   BwdArgs a = a0;
   a.num_n_tiles = (a.seq.max_seqlen_k + BN - 1) / BN;
   a.num_zh = bwd_nseq(a) * a.hk;
@@ -1624,7 +1649,7 @@ hipError_t launch_dkdv_variant(const BwdArgs& a0, hipStream_t stream) {
   a.zh_group = 2;
   a.items_per_xcd = ((a.zh_per_xcd + a.zh_group - 1) / a.zh_group) * a.zh_group * a.num_n_tiles *
                     (kParts ? a.part_heads * a.part_tiles : 1);
-  dim3 grid((unsigned)(kNumXcd * persistent_workers<D>(a)));
+  dim3 grid((unsigned)(kNumXcd * persistent_workers<D>(a, kTwoWaves<D, B> ? 2 : 1)));
   // (the level table's LDS is requested whether or not this launch uses it: the kernel's limit is set once)
   constexpr int smem = DkDvSmem<D, BM>::BYTES + (D < 256 ? kLevelBytes : 0);
   // (every build has the variant that stores dS; the host decides where it pays)
@@ -1651,20 +1676,28 @@ hipError_t launch_bwd_dkdv(const BwdArgs& a0, bool windowed, bool bias, bool dro
 template <typename T, int D, bool kPad, bool W, bool B, bool P>
 hipError_t launch_dq_variant(const BwdArgs& a0, hipStream_t stream) {
   using Tile = BwdTile<T, D, W>;
-  constexpr int NW = Tile::NW, BN = Tile::DQ_BN, BM = NW * 32;
+  constexpr int NW = Tile::NW, BN = kDqBN<T, D, W, B>, BM = NW * 32;
   BwdArgs a = a0;
   a.num_m_tiles = (a.seq.max_seqlen_q + BM - 1) / BM;
   a.num_zh = bwd_nseq(a) * a.hq;
   a.zh_per_xcd = (a.num_zh + kNumXcd - 1) / kNumXcd;
   a.zh_group = a.hq / a.hk > 2 ? (a.hq / a.hk > 8 ? 8 : a.hq / a.hk) : 2;
   a.items_per_xcd = ((a.zh_per_xcd + a.zh_group - 1) / a.zh_group) * a.zh_group * a.num_m_tiles;
-  dim3 grid((unsigned)(kNumXcd * persistent_workers<D>(a)));
+  dim3 grid((unsigned)(kNumXcd * persistent_workers<D>(a, kTwoWaves<D, B> ? 2 : 1)));
   return launch_with_lds<bwd_dq_kernel<T, D, NW, BN, W, B, P, kPad>>(grid, NW * 64, DqSmem<D, BN>::BYTES, stream, a);
 }
 
-template <typename T, int D, bool kPad>
+template <typename T, int D, bool kPad, bool W, bool B, bool P, bool kBuilt>
+hipError_t launch_dq_if(const BwdArgs& a, hipStream_t stream) {
+  if constexpr (kBuilt) return launch_dq_variant<T, D, kPad, W, B, P>(a, stream);
+  else return hipErrorNotSupported;
+}
+
+// kOnly: -1 all kernels; 0 those without, 1 those with a bias (head dim 64, where the two are compiled
+// with different options)
+template <typename T, int D, bool kPad, int kOnly = -1>
 hipError_t launch_bwd_dq(const BwdArgs& a0, bool windowed, bool bias, bool dropout, hipStream_t stream) {
-#define FA_CALL(W, B, P) launch_dq_variant<T, D, kPad, W, B, P>(a0, stream)
+#define FA_CALL(W, B, P) launch_dq_if<T, D, kPad, W, B, P, kOnly == -1 || kOnly == (B ? 1 : 0)>(a0, stream)
   FA_BWD_SWITCH(FA_CALL)
 #undef FA_CALL
 }
@@ -1672,7 +1705,8 @@ hipError_t launch_bwd_dq(const BwdArgs& a0, bool windowed, bool bias, bool dropo
 template <typename T, int D, bool kPad, bool W, bool B, bool P>
 hipError_t launch_fused_variant(const BwdArgs& a0, hipStream_t stream) {
   using Tile = BwdTile<T, D, W>;
-  constexpr int NW = Tile::NW, BM = Tile::DKDV_BM, BN = Tile::DQ_BN;
+  // (one wave per SIMD, hence the wide steps at head dim 64)
+  constexpr int NW = Tile::NW, BM = D == 64 ? 128 : Tile::DKDV_BM, BN = D == 64 ? 128 : Tile::DQ_BN;
   constexpr int smem = DkDvSmem<D, BM>::BYTES > DqSmem<D, BN>::BYTES ? DkDvSmem<D, BM>::BYTES : DqSmem<D, BN>::BYTES;
   BwdArgs a = a0;
   a.num_n_tiles = (a.seq.max_seqlen_k + NW * 32 - 1) / (NW * 32);
@@ -1682,7 +1716,7 @@ hipError_t launch_fused_variant(const BwdArgs& a0, hipStream_t stream) {
   a.zh_group = 2;
   const int items = a.num_n_tiles + a.num_m_tiles * (a.hq / a.hk);
   a.items_per_xcd = ((a.zh_per_xcd + a.zh_group - 1) / a.zh_group) * a.zh_group * items;
-  dim3 grid((unsigned)(kNumXcd * persistent_workers<D>(a)));
+  dim3 grid((unsigned)(kNumXcd * persistent_workers<D>(a, 1)));
   return launch_with_lds<bwd_fused_kernel<T, D, NW, BM, BN, W, B, P, kPad>>(grid, NW * 64, smem, stream, a);
 }
 
