@@ -1059,9 +1059,9 @@ __device__ __forceinline__ void dq_item(const BwdArgs& a, const int h, const int
   }
 
   // Without dropout (the mask and the scale come between dP and the subtraction) dP starts at
-  // -delta.  Not in the dQ kernel at D = 64: with 128-key tiles its register allocation gets
-  // worse with the extra tuple (20-50 % slower); the single-launch kernel at D = 64 gains.
-  constexpr bool kFoldDelta = !kDropout && (D >= 128 || (kInlineDelta && !kStoreDelta));
+  // -delta.  Not at D = 64 with 128-key tiles (a bias), whose register allocation gets worse with the extra
+  // tuple (20-50 % slower); with 64-key tiles it gains 1-2 % there as well.
+  constexpr bool kFoldDelta = !kDropout && (D >= 128 || (kInlineDelta && !kStoreDelta) || !kBias);
   f32x16 negd16;      // -delta of this lane's query in every element: the initial value of dP
 #pragma unroll
   for (int i = 0; i < 16; ++i) negd16[i] = -d_row;
