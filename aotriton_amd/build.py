@@ -40,9 +40,11 @@ EXTRA = {
     'fa_bwd_dq_d128.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'],
 }
 
-# The per-head-dim kernel files are compiled a second time with FA_PADDED=1: the copies that
+# The per-head-dim kernel files are compiled a second time with FA_PADDED = the head dim: the copies that
 # serve head dims rounded up to the compiled one.
-PADDED_RE = re.compile(r'fa_(fwd|fwd_rows|bwd_dkdv|bwd_dkdv_parts|bwd_dq|bwd_dq_bias|bwd_fused)_d\d+\.hip$')
+PADDED_RE = re.compile(r'fa_(fwd|fwd_rows|bwd_dkdv|bwd_dkdv_parts|bwd_dq|bwd_dq_bias|bwd_fused)_d(\d+)\.hip$')
+# ... and these a third time with 96 columns, for head dims above 64 and up to 96
+COLS96_RE = re.compile(r'fa_(fwd|bwd_dkdv|bwd_dq)_d128\.hip$')
 
 
 def sources():
@@ -52,8 +54,10 @@ def sources():
         if not (f.endswith('.hip') or f.endswith('.cpp')):
             continue
         out.append((f, [], f + '.o'))
-        if PADDED_RE.match(f):
-            out.append((f, ['-DFA_PADDED=1'], f + '.padded.o'))
+        if m := PADDED_RE.match(f):
+            out.append((f, ['-DFA_PADDED=' + m.group(2)], f + '.padded.o'))
+        if COLS96_RE.match(f):
+            out.append((f, ['-DFA_PADDED=96'], f + '.cols96.o'))
     return out
 
 

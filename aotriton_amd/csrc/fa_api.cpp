@@ -518,7 +518,9 @@ hipError_t run_fwd(int dtype, int d, const fa::FwdArgs& a, const Shape& s, hipSt
   const bool padded = a.head_dim != d || a.head_dim_v != d;   // head dim rounded up: the copies that mask the excess columns
   switch (d) {
     case 64: return (padded ? fa::run_fwd_d64_padded : fa::run_fwd_d64)(dtype, a, s.windowed, s.bias, s.dropout, stream);
-    case 128: return (padded ? fa::run_fwd_d128_padded : fa::run_fwd_d128)(dtype, a, s.windowed, s.bias, s.dropout, stream);
+    case 128:
+      if (a.head_dim <= 96 && a.head_dim_v <= 96) return fa::run_fwd_d128_cols96(dtype, a, s.windowed, s.bias, s.dropout, stream);
+      return (padded ? fa::run_fwd_d128_padded : fa::run_fwd_d128)(dtype, a, s.windowed, s.bias, s.dropout, stream);
     case 256: return (padded ? fa::run_fwd_d256_padded : fa::run_fwd_d256)(dtype, a, s.windowed, s.bias, s.dropout, stream);
   }
   return hipErrorNotSupported;

@@ -1,7 +1,7 @@
 // Backward dkdv kernels whose items are cut into parts: instantiations for head dim 64 (fp16 and bf16).
 #include "fa_bwd_impl.h"
 
-// Compiled twice: as is for tensors whose head dim is 64, and with FA_PADDED=1 for smaller
+// Compiled twice: as is for tensors whose head dim is 64, and with FA_PADDED = the columns to compute for smaller
 // head dims (a multiple of 8), where the kernels mask the excess columns.
 #ifndef FA_PADDED
 #define FA_PADDED 0
@@ -14,7 +14,7 @@
 
 namespace fa {
 hipError_t FA_RUN(int dtype, const BwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s) {
-  if (dtype == kDtypeBF16) return launch_bwd_dkdv<bf16_t, 64, FA_PADDED != 0, true>(a, windowed, bias, dropout, s);
-  return launch_bwd_dkdv<f16_t, 64, FA_PADDED != 0, true>(a, windowed, bias, dropout, s);
+  if (dtype == kDtypeBF16) return launch_bwd_dkdv<bf16_t, 64, FA_PADDED, true>(a, windowed, bias, dropout, s);
+  return launch_bwd_dkdv<f16_t, 64, FA_PADDED, true>(a, windowed, bias, dropout, s);
 }
 }  // namespace fa

@@ -7,9 +7,10 @@ namespace fa {
 template <typename T>
 static hipError_t run_dqs_t(int head_dim, const BwdArgs& a, hipStream_t s) {
   const bool padded = a.head_dim != head_dim;
-  if (head_dim == 128) return padded ? launch_bwd_dqs<T, 128, true>(a, s) : launch_bwd_dqs<T, 128, false>(a, s);
-  if (head_dim == 64) return padded ? launch_bwd_dqs<T, 64, true>(a, s) : launch_bwd_dqs<T, 64, false>(a, s);
-  if (head_dim == 256) return padded ? launch_bwd_dqs<T, 256, true>(a, s) : launch_bwd_dqs<T, 256, false>(a, s);
+  if (head_dim == 128 && a.head_dim <= 96) return launch_bwd_dqs<T, 128, 96>(a, s);
+  if (head_dim == 128) return padded ? launch_bwd_dqs<T, 128, 128>(a, s) : launch_bwd_dqs<T, 128, 0>(a, s);
+  if (head_dim == 64) return padded ? launch_bwd_dqs<T, 64, 64>(a, s) : launch_bwd_dqs<T, 64, 0>(a, s);
+  if (head_dim == 256) return padded ? launch_bwd_dqs<T, 256, 256>(a, s) : launch_bwd_dqs<T, 256, 0>(a, s);
   return hipErrorNotSupported;
 }
 

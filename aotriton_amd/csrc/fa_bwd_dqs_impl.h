@@ -32,7 +32,7 @@ struct DqsSmem {     // two stages of the K tile (swizzled), then one dS area pe
 };
 
 // One Q tile of 256 rows (8 waves x 32 queries) of head h against the key tiles that see it.
-template <typename T, int D, int BN, bool kPad, bool kWideTile>
+template <typename T, int D, int BN, int kPad, bool kWideTile>
 __device__ __forceinline__ void dqs_item(const BwdArgs& a, const int h, const int mt, const int z, char* smem_raw) {
   using Tr = Traits<T>;
   using op_t = typename Tr::op_t;
@@ -40,7 +40,7 @@ __device__ __forceinline__ void dqs_item(const BwdArgs& a, const int h, const in
   using SM = DqsSmem<D, BN>;
   using DT = DsTile<T, D, kWideTile>;
   constexpr int NW = SM::NW, NT = NW * 64, BM = NW * 32;
-  constexpr int DB = D / 32;
+  constexpr int DB = (kPad ? kPad : D) / 32;
   constexpr int SPT = DT::BN / BN;          // steps per stored tile
   constexpr int KWS = BN / 32;              // 32-key blocks per step
   constexpr int NCK = KWS * 2;              // 1 KB pieces of dS per wave and step
@@ -200,7 +200,7 @@ __device__ __forceinline__ void dqs_item(const BwdArgs& a, const int h, const in
 
 // One workgroup per Q tile on a 1-D grid: consecutive ids go round the XCDs, an XCD takes its
 // (batch, q-head) pairs two at a time, the heaviest (last) tile of a causal mask first.
-template <typename T, int D, int BN, bool kPad, bool kWideTile>
+template <typename T, int D, int BN, int kPad, bool kWideTile>
 __global__ __attribute__((amdgpu_flat_work_group_size(512, 512))) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void bwd_dqs_kernel(const BwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
@@ -216,7 +216,7 @@ void bwd_dqs_kernel(const BwdArgs a) {
   dqs_item<T, D, BN, kPad, kWideTile>(a, h, mt, z, smem_raw);
 }
 
-template <typename T, int D, bool kPad>
+template <typename T, int D, int kPad>
 hipError_t launch_bwd_dqs(const BwdArgs& a0, hipStream_t stream) {
   constexpr int BN = D >= 256 ? 32 : 64;
   BwdArgs a = a0;

@@ -149,12 +149,15 @@ template <typename T, int D, bool kWideTile> struct DsTile {
   static constexpr int piece(int kw, int t) { return (t >> 1) * QBLOCK_BYTES + kw * 2048 + (t & 1) * 1024; }
 };
 
+// n elements of vector work spread evenly behind g MFMAs: the first one behind MFMA i
+constexpr int first_of(int i, int n, int g) { return (i * n + g - 1) / g; }
+
 // ---------------------------------------------------------------------------
 // dK / dV work item
 // ---------------------------------------------------------------------------
 // kStoreDs: dS of every visited tile pair is also written to BwdArgs::ds_ws, and the row statistics
 // come prepared (BwdArgs::lse_scaled, delta_prep) so that they can travel straight into LDS.
-template <typename T, int D, int NW, int BM, bool kWindowed, bool kBias, bool kDropout, bool kInlineDelta, bool kPad,
+template <typename T, int D, int NW, int BM, bool kWindowed, bool kBias, bool kDropout, bool kInlineDelta, int kPad,
           bool kStoreDs = false, bool kParts = false>
 __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const int nt, const int z, const int part,
                                           char* smem_raw) {
@@ -164,7 +167,8 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
   using SM = DkDvSmem<D, BM>;
   constexpr int NT = NW * 64;
   constexpr int BN = NW * 32;
-  constexpr int KS = D / 16, MB = BM / 32, DB = D / 32, TS = BM / 16;
+  constexpr int DC = kPad ? kPad : D;            // columns computed; those past a tensor's head dim are zero
+  constexpr int KS = DC / 16, MB = BM / 32, DB = DC / 32, TS = BM / 16;
   constexpr int NCH = BM * D / 8;                // 16-byte chunks per tile, per tensor
   constexpr int CH = (NCH + NT - 1) / NT;        // chunks per thread, per tensor
   constexpr int LPR = D / 8;                     // lanes that share one row
@@ -696,8 +700,6 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
     };
 
     // ---- dP = dO V^T, with p behind its MFMAs ------------------------------------
-    constexpr int EPG1 = 16 * MB / (KS * MB);    // elements per MFMA (D = 128: 2)
-    static_assert(16 * MB % (KS * MB) == 0 || KS * MB > 16 * MB, "element split");
 #pragma unroll
     for (int k = 0; k < KS; ++k) {
       if (k + kAhead < KS) {
@@ -711,21 +713,10 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
         dp[mb] = Tr::mfma(xa[(KS + k) % (kAhead + 1)][mb], kVLds ? vl[k % 3] : vreg[kVLds ? 0 : k],
                           k == 0 && kDropout ? zero16 : dp[mb]);
         const int gidx = k * MB + mb;
-        if constexpr (EPG1 >= 1) {
 #pragma unroll
-          for (int e = 0; e < (EPG1 >= 1 ? EPG1 : 1); ++e) {
-            const int E = gidx * EPG1 + e;
-            p_el(E);
-            if (E & 1) p_pair(E);
-          }
-        } else {
-          // more MFMAs than elements (D = 256): one element every other MFMA
-          constexpr int every = (KS * MB) / (16 * MB);
-          if (gidx % every == 0) {
-            const int E = gidx / every;
-            p_el(E);
-            if (E & 1) p_pair(E);
-          }
+        for (int E = first_of(gidx, 16 * MB, KS * MB); E < first_of(gidx + 1, 16 * MB, KS * MB); ++E) {
+          p_el(E);
+          if (E & 1) p_pair(E);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -753,8 +744,6 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
 
     // ---- dV^T += dO^T P, with ds behind its MFMAs --------------------------------
     constexpr int G3 = TS * DB;
-    constexpr int EPG3 = 16 * MB / G3;           // D = 128: 2
-    static_assert(16 * MB % G3 == 0 || G3 > 16 * MB, "element split");
 #pragma unroll
     for (int t = 0; t < TS; ++t) {
 #pragma unroll
@@ -769,20 +758,10 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
                                                                : swz_read_tr<T, D>(Qb, tr_a0, tr_a1, 0, db);
           dv[db] = Tr::mfma(ta[t & 1 & (kRingTa ? 0 : 1)][db], pb[t], dv[db]);
         }
-        if constexpr (EPG3 >= 1) {
 #pragma unroll
-          for (int e = 0; e < (EPG3 >= 1 ? EPG3 : 1); ++e) {
-            const int E = gidx * EPG3 + e;
-            ds_el(E);
-            if (E & 1) ds_pair(E);
-          }
-        } else {
-          constexpr int every = G3 / (16 * MB);
-          if (gidx % every == 0) {
-            const int E = gidx / every;
-            ds_el(E);
-            if (E & 1) ds_pair(E);
-          }
+        for (int E = first_of(gidx, 16 * MB, G3); E < first_of(gidx + 1, 16 * MB, G3); ++E) {
+          ds_el(E);
+          if (E & 1) ds_pair(E);
         }
         if (kStoreDs && TS >= kDsSlots && gidx == G3 / 2) store_ds_slot(ds_tile, 0);
         if (kStoreDs && gidx == 3 * G3 / 4) store_ds_slot(ds_tile, 1);
@@ -907,7 +886,7 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
 // kInlineDelta: delta = rowsum(O dO) of the item's rows is computed here, from the rows the lanes
 // load anyway (dO) and their O rows, instead of being read.  kStoreDelta: it is also written out:
 // the split backward has no preprocess launch, the dK/dV kernel runs after this one and reads it.
-template <typename T, int D, int NW, int BN, bool kWindowed, bool kBias, bool kDropout, bool kInlineDelta, bool kPad,
+template <typename T, int D, int NW, int BN, bool kWindowed, bool kBias, bool kDropout, bool kInlineDelta, int kPad,
           bool kStoreDelta = false>
 __device__ __forceinline__ void dq_item(const BwdArgs& a, const int h, const int mt, const int z,
                                         char* smem_raw) {
@@ -917,7 +896,8 @@ __device__ __forceinline__ void dq_item(const BwdArgs& a, const int h, const int
   using SM = DqSmem<D, BN>;
   constexpr int NT = NW * 64;
   constexpr int BM = NW * 32;
-  constexpr int KS = D / 16, MB = BN / 32, DB = D / 32, TS = BN / 16;
+  constexpr int DC = kPad ? kPad : D;            // columns computed; those past a tensor's head dim are zero
+  constexpr int KS = DC / 16, MB = BN / 32, DB = DC / 32, TS = BN / 16;
   constexpr int CH = (BN * D / 8) / NT;          // 16-byte chunks per thread, per tensor
   static_assert((BN * D / 8) % NT == 0, "tile must split evenly");
 
@@ -1325,8 +1305,6 @@ __device__ __forceinline__ void dq_item(const BwdArgs& a, const int h, const int
     };
 
     // ---- dP^T = V dO^T, with p behind its MFMAs -----------------------------------
-    constexpr int EPG1 = 16 / KS;          // elements per MFMA
-    static_assert(16 % KS == 0, "element split");
 #pragma unroll
     for (int k = 0; k < KS; ++k) {
       if (k + kAhead < KS) {
@@ -1338,7 +1316,7 @@ __device__ __forceinline__ void dq_item(const BwdArgs& a, const int h, const int
       for (int mb = 0; mb < MB; ++mb) {
         dp[mb] = Tr::mfma(xa[(KS + k) % (kAhead + 1)][mb], doreg[k], k == 0 ? (kFoldDelta ? negd16 : zero16) : dp[mb]);
 #pragma unroll
-        for (int e = 0; e < EPG1; ++e) p_el((k * MB + mb) * EPG1 + e);
+        for (int E = first_of(k * MB + mb, 16 * MB, KS * MB); E < first_of(k * MB + mb + 1, 16 * MB, KS * MB); ++E) p_el(E);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -1351,8 +1329,6 @@ __device__ __forceinline__ void dq_item(const BwdArgs& a, const int h, const int
     __builtin_amdgcn_sched_barrier(0);
 
     // ---- dQ^T += K^T dS^T, with the next step's ds and the LDS writes behind its MFMAs ----
-    constexpr int EPG3 = 8 / DB;
-    static_assert(8 % DB == 0, "element split");
 #pragma unroll
     for (int t = 0; t < TS; ++t) {
 #pragma unroll
@@ -1361,7 +1337,7 @@ __device__ __forceinline__ void dq_item(const BwdArgs& a, const int h, const int
         dq[db] = Tr::mfma(ta[t & 1][db], sb[t], dq[db]);
         if (t + 1 < TS) {
 #pragma unroll
-          for (int e = 0; e < EPG3; ++e) ds_el(8 * (t + 1) + db * EPG3 + e);
+          for (int e = first_of(db, 8, DB); e < first_of(db + 1, 8, DB); ++e) ds_el(8 * (t + 1) + e);
         }
         constexpr int per = (STORE_PIECES + G4 - 1) / G4;
 #pragma unroll
@@ -1444,7 +1420,7 @@ __host__ __device__ inline bool dkdv_level_list(const BwdArgs& a) {
   return D < 256 && a.seq.num_seqlens != 0 && a.bias == nullptr && a.zh_per_xcd <= kLevelCap && a.num_n_tiles <= 0xffff;
 }
 
-template <typename T, int D, int NW, int BM, bool kWindowed, bool kBias, bool kDropout, bool kPad, bool kStoreDs = false,
+template <typename T, int D, int NW, int BM, bool kWindowed, bool kBias, bool kDropout, int kPad, bool kStoreDs = false,
           bool kParts = false>
 __global__ __attribute__((amdgpu_flat_work_group_size(NW * 64, NW * 64))) __attribute__((amdgpu_waves_per_eu(kTwoWaves<D, kBias> ? 2 : 1, kTwoWaves<D, kBias> ? 2 : 1)))
 void bwd_dkdv_kernel(const BwdArgs a) {
@@ -1491,7 +1467,7 @@ void bwd_dkdv_kernel(const BwdArgs a) {
   }
 }
 
-template <typename T, int D, int NW, int BN, bool kWindowed, bool kBias, bool kDropout, bool kPad>
+template <typename T, int D, int NW, int BN, bool kWindowed, bool kBias, bool kDropout, int kPad>
 __global__ __attribute__((amdgpu_flat_work_group_size(NW * 64, NW * 64))) __attribute__((amdgpu_waves_per_eu(kTwoWaves<D, kBias> ? 2 : 1, kTwoWaves<D, kBias> ? 2 : 1)))
 void bwd_dq_kernel(const BwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
@@ -1520,7 +1496,7 @@ void bwd_dq_kernel(const BwdArgs a) {
 // the same 1-D grid as the split kernels: each XCD owns a contiguous range of (batch,
 // kv-head) pairs and walks them in pairs, so the tensors of the heads in flight stay in
 // that XCD's L2.
-template <typename T, int D, int NW, int BM, int BN, bool kWindowed, bool kBias, bool kDropout, bool kPad>
+template <typename T, int D, int NW, int BM, int BN, bool kWindowed, bool kBias, bool kDropout, int kPad>
 __global__ __attribute__((amdgpu_flat_work_group_size(NW * 64, NW * 64)))
 void bwd_fused_kernel(const BwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
@@ -1638,7 +1614,7 @@ static __global__ __launch_bounds__(256) void combine_dkdv_kernel(const BwdArgs 
   *reinterpret_cast<q4_t*>(out) = t4;
 }
 
-template <typename T, int D, bool kPad, bool W, bool B, bool P, bool kParts>
+template <typename T, int D, int kPad, bool W, bool B, bool P, bool kParts>
 hipError_t launch_dkdv_variant(const BwdArgs& a0, hipStream_t stream) {
   using Tile = BwdTile<T, D, W>;
   constexpr int NW = Tile::NW, BM = kDkDvBM<T, D, W, B, P>, BN = NW * 32;
@@ -1666,14 +1642,14 @@ hipError_t launch_dkdv_variant(const BwdArgs& a0, hipStream_t stream) {
   return e;
 }
 
-template <typename T, int D, bool kPad, bool kParts>
+template <typename T, int D, int kPad, bool kParts>
 hipError_t launch_bwd_dkdv(const BwdArgs& a0, bool windowed, bool bias, bool dropout, hipStream_t stream) {
 #define FA_CALL(W, B, P) launch_dkdv_variant<T, D, kPad, W, B, P, kParts>(a0, stream)
   FA_BWD_SWITCH(FA_CALL)
 #undef FA_CALL
 }
 
-template <typename T, int D, bool kPad, bool W, bool B, bool P>
+template <typename T, int D, int kPad, bool W, bool B, bool P>
 hipError_t launch_dq_variant(const BwdArgs& a0, hipStream_t stream) {
   using Tile = BwdTile<T, D, W>;
   constexpr int NW = Tile::NW, BN = kDqBN<T, D, W, B>, BM = NW * 32;
@@ -1687,7 +1663,7 @@ hipError_t launch_dq_variant(const BwdArgs& a0, hipStream_t stream) {
   return launch_with_lds<bwd_dq_kernel<T, D, NW, BN, W, B, P, kPad>>(grid, NW * 64, DqSmem<D, BN>::BYTES, stream, a);
 }
 
-template <typename T, int D, bool kPad, bool W, bool B, bool P, bool kBuilt>
+template <typename T, int D, int kPad, bool W, bool B, bool P, bool kBuilt>
 hipError_t launch_dq_if(const BwdArgs& a, hipStream_t stream) {
   if constexpr (kBuilt) return launch_dq_variant<T, D, kPad, W, B, P>(a, stream);
   else return hipErrorNotSupported;
@@ -1695,14 +1671,14 @@ hipError_t launch_dq_if(const BwdArgs& a, hipStream_t stream) {
 
 // kOnly: -1 all kernels; 0 those without, 1 those with a bias (head dim 64, where the two are compiled
 // with different options)
-template <typename T, int D, bool kPad, int kOnly = -1>
+template <typename T, int D, int kPad, int kOnly = -1>
 hipError_t launch_bwd_dq(const BwdArgs& a0, bool windowed, bool bias, bool dropout, hipStream_t stream) {
 #define FA_CALL(W, B, P) launch_dq_if<T, D, kPad, W, B, P, kOnly == -1 || kOnly == (B ? 1 : 0)>(a0, stream)
   FA_BWD_SWITCH(FA_CALL)
 #undef FA_CALL
 }
 
-template <typename T, int D, bool kPad, bool W, bool B, bool P>
+template <typename T, int D, int kPad, bool W, bool B, bool P>
 hipError_t launch_fused_variant(const BwdArgs& a0, hipStream_t stream) {
   using Tile = BwdTile<T, D, W>;
   // (one wave per SIMD, hence the wide steps at head dim 64)
@@ -1720,7 +1696,7 @@ hipError_t launch_fused_variant(const BwdArgs& a0, hipStream_t stream) {
   return launch_with_lds<bwd_fused_kernel<T, D, NW, BM, BN, W, B, P, kPad>>(grid, NW * 64, smem, stream, a);
 }
 
-template <typename T, int D, bool kPad>
+template <typename T, int D, int kPad>
 hipError_t launch_bwd_fused(const BwdArgs& a0, bool windowed, bool bias, bool dropout, hipStream_t stream) {
 #define FA_CALL(W, B, P) launch_fused_variant<T, D, kPad, W, B, P>(a0, stream)
   FA_BWD_SWITCH(FA_CALL)

@@ -2,12 +2,15 @@
 #include "fa_fwd_impl.h"
 #include "fa_kernels.h"
 
-// Compiled twice: as is for tensors whose head dim is 128, and with FA_PADDED=1 for smaller
-// head dims (a multiple of 8), where the kernels mask the excess columns.
+// Compiled three times: as is for tensors whose head dim is 128, and with FA_PADDED = the columns to compute
+// (128, or 96 for head dims up to that) for smaller head dims (a multiple of 8), where the kernels mask
+// the excess columns.
 #ifndef FA_PADDED
 #define FA_PADDED 0
 #endif
-#if FA_PADDED
+#if FA_PADDED == 96
+#define FA_RUN run_fwd_d128_cols96
+#elif FA_PADDED
 #define FA_RUN run_fwd_d128_padded
 #else
 #define FA_RUN run_fwd_d128
@@ -15,7 +18,7 @@
 
 namespace fa {
 hipError_t FA_RUN(int dtype, const FwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s) {
-  if (dtype == kDtypeBF16) return launch_fwd<bf16_t, 128, FA_PADDED != 0>(a, windowed, bias, dropout, s);
-  return launch_fwd<f16_t, 128, FA_PADDED != 0>(a, windowed, bias, dropout, s);
+  if (dtype == kDtypeBF16) return launch_fwd<bf16_t, 128, FA_PADDED>(a, windowed, bias, dropout, s);
+  return launch_fwd<f16_t, 128, FA_PADDED>(a, windowed, bias, dropout, s);
 }
 }  // namespace fa

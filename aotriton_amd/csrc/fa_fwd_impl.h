@@ -41,7 +41,7 @@ struct FwdSmem {
 // One Q tile (BM rows of head h of sequence z) against all its visible K/V tiles, or with kSplit
 // against part `split` of a.splits of them: the fp32 sums and the row statistics of the part then go to
 // scratch memory, where combine_rows_kernel picks them up.
-template <typename T, int D, int NW, int BN, bool kWindowed, bool kBias, bool kDropout, bool kPad, bool kSplit, bool kKeyBias>
+template <typename T, int D, int NW, int BN, bool kWindowed, bool kBias, bool kDropout, int kPad, bool kSplit, bool kKeyBias>
 __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const int h, const int mt, const int split,
                                          char* smem_raw) {
   using Tr = Traits<T>;
@@ -50,9 +50,10 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
   using SM = FwdSmem<D, BN, NW>;
   constexpr int NT = NW * 64;
   constexpr int BM = NW * 32;
-  constexpr int KS = D / 16;    // k-steps of S^T = K Q^T
+  constexpr int DC = kPad ? kPad : D;   // columns computed; those past a tensor's head dim are zero
+  constexpr int KS = DC / 16;   // k-steps of S^T = K Q^T
   constexpr int MB = BN / 32;   // 32-key blocks per tile
-  constexpr int DB = D / 32;    // 32-wide blocks of the head dim
+  constexpr int DB = DC / 32;   // 32-wide blocks of the head dim
   constexpr int TS = BN / 16;   // k-steps of O^T += V^T P^T
   constexpr int KSTR = SM::KSTR, VSTR = SM::VSTR;
   constexpr int CH = (BN * D / 8) / NT;                   // 16-byte chunks per thread, per tensor
@@ -614,7 +615,7 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
 // goes from one tile to the next without a relaunch.
 // QB = 0: fwd_item, NW waves of 32 rows.  QB > 0: fwd_item_pipe, 4 waves of 32 * QB rows, one wave
 // per SIMD.
-template <typename T, int D, int NW, int BN, int QB, bool kWindowed, bool kBias, bool kDropout, bool kPad, bool kSplit,
+template <typename T, int D, int NW, int BN, int QB, bool kWindowed, bool kBias, bool kDropout, int kPad, bool kSplit,
           bool kKeyBias>
 __global__ __attribute__((amdgpu_flat_work_group_size(NW * 64, NW * 64)))
 __attribute__((amdgpu_waves_per_eu(D <= 128 && QB == 0 ? 2 : 1, D <= 128 && QB == 0 ? 2 : 1)))
@@ -707,7 +708,7 @@ template <typename T, bool kWindowed> struct FwdTile<T, 128, kWindowed> : FwdTil
 // 629 vs 510; bias + dropout + window 1024: 361 vs 333).
 template <typename T, bool kWindowed> struct FwdTile<T, 256, kWindowed> : FwdTileOf<256, 4, 32, 1> {};
 
-template <typename T, int D, bool kWindowed, bool kBias, bool kDropout, bool kPad, bool kSplit = false,
+template <typename T, int D, bool kWindowed, bool kBias, bool kDropout, int kPad, bool kSplit = false,
           bool kKeyBias = false>
 hipError_t launch_fwd_variant(const FwdArgs& a, dim3 grid, hipStream_t stream) {
   using Tile = FwdTile<T, D, kWindowed>;
@@ -728,7 +729,7 @@ hipError_t launch_fwd_variant(const FwdArgs& a, dim3 grid, hipStream_t stream) {
 
 // kPad: a head dim of the tensors (FwdArgs::head_dim, head_dim_v) is smaller than D and the excess
 // columns are masked.
-template <typename T, int D, bool kPad>
+template <typename T, int D, int kPad>
 hipError_t launch_fwd(const FwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t stream) {
   const int BM = windowed ? FwdTile<T, D, true>::BM : FwdTile<T, D, false>::BM;
   const int nseq = a.seq.num_seqlens != 0 ? (a.seq.num_seqlens < 0 ? -a.seq.num_seqlens : a.seq.num_seqlens)

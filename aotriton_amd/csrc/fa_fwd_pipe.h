@@ -62,7 +62,7 @@ __device__ __forceinline__ void acc_scale(f32x16& t, float f) {
   FA_ACC_JOIN(t);
 }
 
-template <typename T, int D, int QB, int BN, bool kWindowed, bool kBias, bool kDropout, bool kPad>
+template <typename T, int D, int QB, int BN, bool kWindowed, bool kBias, bool kDropout, int kPad>
 __device__ __forceinline__ void fwd_item_pipe(const FwdArgs& a, const int z, const int h, const int mt, char* smem_raw) {
   using Tr = Traits<T>;
   using op_t = typename Tr::op_t;
