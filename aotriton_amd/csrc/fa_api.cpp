@@ -609,6 +609,20 @@ FwdPlan fwd_plan(int dtype, const Shape& s, int causal_type, int window_left, in
   return r;
 }
 
+// Tiles of 128 rows, two workgroups per CU, instead of 256 rows and one (FwdHalfTile)?  Where they save a part
+// of the rounds in which an XCD's CUs take its tiles; the line lies above what they cost per row.  Measured (bf16, us,
+// 256 -> 128 rows): B40 H16 S128 D64 19.2 -> 14.4 (3 rounds against 2), B16 H12 S640 D64 45 -> 34 and causal 44 -> 29,
+// D128 67 -> 52 and 62 -> 42 (3 : 2), B40 H16 S640 D64 113 -> 99 (8 : 7), S384 53 -> 47 (5 : 4); S800 271 -> 267 and causal
+// 210 -> 214 at D128 (10 : 9); at equal rounds 5-15 % slower.  With a bias the finer tiles cost more (10-15 %), so those keep the large ones.
+bool fwd_half_tiles(int dtype, const Shape& s, int num_cu) {
+  if (s.elementwise || !is_16bit(dtype) || s.d > 128 || s.bias || s.num_seqlens != 0) return false;
+  const int64_t heads = (s.batch * (int64_t)s.hq + fa::kNumXcd - 1) / fa::kNumXcd, cus = num_cu / fa::kNumXcd;
+  if (cus < 1) return false;
+  const int64_t whole = (heads * ((s.max_sq + 255) / 256) + cus - 1) / cus;
+  const int64_t half = (heads * ((s.max_sq + 127) / 128) + 2 * cus - 1) / (2 * cus);
+  return whole * 8 > half * 9;
+}
+
 hipError_t run_fwd_rows(int dtype, int d, const fa::FwdArgs& a, const Shape& s, hipStream_t stream) {
   const bool padded = a.head_dim != d || a.head_dim_v != d;
   switch (d) {
@@ -987,6 +1001,7 @@ static int attn_fwd_impl(const fa_fwd_params* p, int32_t params_version, void* h
     }
   }
   a.splits = scratch != nullptr ? plan.splits : 1;
+  if (a.splits <= 1 && !plan.rows) a.half_tiles = fwd_half_tiles(p->Q.dtype, s, dev->num_cu);
   if (plan.rows) {
     a.row_blocks = plan.row_blocks; a.part_rows = plan.part_rows;
     err = run_fwd_rows(p->Q.dtype, s.d, a, s, stream);

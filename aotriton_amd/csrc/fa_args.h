@@ -57,6 +57,7 @@ struct FwdArgs {
   int32_t items_per_xcd; // Q tiles (incl. padding of the last group) per XCD
   // keys split over workgroups (fa_fwd_rows.h, fwd_item's kSplit): parts, and their fp32 sums and row
   // statistics in scratch memory, laid out as combine_rows_kernel describes
+  int32_t half_tiles;    // tiles of 128 rows, two workgroups per CU (D <= 128, dense, no bias, not split)
   int32_t splits;        // <= 1: not split (kernels without kSplit do not look at it); at most 64
   int32_t row_blocks;    // blocks of rows per pair
   int32_t part_rows;     // rows stored per block

@@ -120,17 +120,6 @@ constexpr int kDqBN = D == 64 && kBias ? 128 : BwdTile<T, D, kWindowed>::DQ_BN;
 
 // Two workgroups per CU, two waves per SIMD (256 registers each)?
 template <int D, bool kBias> constexpr bool kTwoWaves = D == 64 && !kBias;
-// Position in the XCD's list of worker p in round r.  One workgroup per CU: serpentine, which pairs
-// heavy with light items.  Two per CU: the workgroups p and p + CUs of an XCD share a CU, so the second
-// half runs backwards through its part of the round, and every other round is turned round as a whole.
-template <bool kTwo>
-__device__ __forceinline__ int worker_pos(int r, int p, int workers, int num_cu) {
-  if (!kTwo) return r * workers + ((r & 1) ? workers - 1 - p : p);
-  const int c = num_cu / kNumXcd < workers ? num_cu / kNumXcd : workers;
-  const int pos = p < c ? p : c + workers - 1 - p;
-  return r * workers + ((r & 1) ? workers - 1 - pos : pos);
-}
-
 // Stored dS (BwdArgs::ds_ws): one tile per (batch element, q-head, key tile of 128, query tile of the
 // dK/dV step) holds 128 x BM values of the 16-bit type as [32-query block][32-key block][half of the
 // query block][64 pieces of 16 bytes].  A piece is what one lane of the dK/dV item holds as the MFMA

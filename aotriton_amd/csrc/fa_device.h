@@ -453,4 +453,15 @@ __device__ __forceinline__ int64_t lse_offset(const SeqInfo& si, int h, int hq) 
   return ((int64_t)si.batch_index * hq + h) * si.lse_stride + si.q_start;
 }
 
+// Position in the XCD's list of worker p in round r.  One workgroup per CU: serpentine, which pairs
+// heavy with light items.  Two per CU: the workgroups p and p + CUs of an XCD share a CU, so the second
+// half runs backwards through its part of the round, and every other round is turned round as a whole.
+template <bool kTwo>
+__device__ __forceinline__ int worker_pos(int r, int p, int workers, int num_cu) {
+  if (!kTwo) return r * workers + ((r & 1) ? workers - 1 - p : p);
+  const int c = num_cu / kNumXcd < workers ? num_cu / kNumXcd : workers;
+  const int pos = p < c ? p : c + workers - 1 - p;
+  return r * workers + ((r & 1) ? workers - 1 - pos : pos);
+}
+
 }  // namespace fa

@@ -641,6 +641,7 @@ void fwd_kernel(const FwdArgs a) {
   const bool ragged = a.seq.num_seqlens != 0;
   const int ratio = a.hq / a.hk, nseq = a.num_zh / a.hq;
   const bool levels = ragged && a.zh_per_xcd <= kLevelCap && a.num_m_tiles <= 0xffff;
+  constexpr bool kTwo = NW == 4 && QB == 0;      // (FwdHalfTile)
   constexpr int kRows = NW * 32 * (QB > 0 ? QB : 1);
   constexpr int kSmem = QB > 0 ? FwdPipeSmem<D, BN, (QB > 0 ? QB : 1)>::BYTES : FwdSmem<D, BN, NW>::BYTES;
   const int zh_lo = xcd * a.zh_per_xcd;
@@ -652,7 +653,7 @@ void fwd_kernel(const FwdArgs a) {
                         threadIdx.x);
   else if (ragged) walk.init(a.seq, xcd, a.zh_per_xcd, a.num_zh, ratio, nseq, kRows, false);
   for (int r = 0;; ++r) {
-    const int t = r * workers + ((r & 1) ? workers - 1 - p : p);
+    const int t = worker_pos<kTwo>(r, p, workers, a.num_cu);
     int z, h, mt, split = 0;
     if (levels) {
       int e;
@@ -708,10 +709,14 @@ template <typename T, bool kWindowed> struct FwdTile<T, 128, kWindowed> : FwdTil
 // 629 vs 510; bias + dropout + window 1024: 361 vs 333).
 template <typename T, bool kWindowed> struct FwdTile<T, 256, kWindowed> : FwdTileOf<256, 4, 32, 1> {};
 
+// Half the rows, two workgroups per CU (FwdArgs::half_tiles; dense calls without a bias at D <= 128).  A sequence
+// is cut finer, so that less of the last tile and of the last round is empty; per row it is 5-15 % slower (K and V
+// are staged once per 128 rows, narrower key tiles).  fwd_half_tiles in fa_api.cpp decides.
+template <int D> struct FwdHalfTile : FwdTileOf<D, 4, D == 64 ? 64 : 32, 0> {};
+
 template <typename T, int D, bool kWindowed, bool kBias, bool kDropout, int kPad, bool kSplit = false,
-          bool kKeyBias = false>
+          bool kKeyBias = false, typename Tile = FwdTile<T, D, kWindowed>>
 hipError_t launch_fwd_variant(const FwdArgs& a, dim3 grid, hipStream_t stream) {
-  using Tile = FwdTile<T, D, kWindowed>;
   constexpr int NW = Tile::NW;
   auto kern = fwd_kernel<T, D, NW, Tile::BN, Tile::QB, kWindowed, kBias, kDropout, kPad, kSplit, kKeyBias>;
   constexpr int smem = Tile::LDS;
@@ -731,7 +736,8 @@ hipError_t launch_fwd_variant(const FwdArgs& a, dim3 grid, hipStream_t stream) {
 // columns are masked.
 template <typename T, int D, int kPad>
 hipError_t launch_fwd(const FwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t stream) {
-  const int BM = windowed ? FwdTile<T, D, true>::BM : FwdTile<T, D, false>::BM;
+  const bool half = D <= 128 && a.half_tiles != 0;
+  const int BM = half ? 128 : windowed ? FwdTile<T, D, true>::BM : FwdTile<T, D, false>::BM;
   const int nseq = a.seq.num_seqlens != 0 ? (a.seq.num_seqlens < 0 ? -a.seq.num_seqlens : a.seq.num_seqlens)
                                           : a.batch;
   FwdArgs b = a;
@@ -743,7 +749,7 @@ hipError_t launch_fwd(const FwdArgs& a, bool windowed, bool bias, bool dropout, 
   // (with splits, an item is one part of the keys of a tile; only without dropout, at D <= 128)
   const bool split = a.splits > 1;
   b.items_per_xcd = groups * b.zh_group * b.num_m_tiles * (split ? a.splits : 1);
-  int workers = a.num_cu / kNumXcd;          // one workgroup per CU
+  int workers = a.num_cu / kNumXcd * (half ? 2 : 1);          // one workgroup per CU, or two
   if (workers < 1) workers = 1;
   if (workers > b.items_per_xcd) workers = b.items_per_xcd;
   dim3 grid((unsigned)(kNumXcd * workers));
@@ -763,6 +769,15 @@ hipError_t launch_fwd(const FwdArgs& a, bool windowed, bool bias, bool dropout, 
     if (bias && !dropout && a.sb_m == 0)
       return windowed ? launch_fwd_variant<T, D, true, true, false, kPad, false, true>(b, grid, stream)
                       : launch_fwd_variant<T, D, false, true, false, kPad, false, true>(b, grid, stream);
+  }
+  if constexpr (D <= 128) {
+    using Half = FwdHalfTile<D>;
+    switch (half ? (windowed ? 2 : 0) | (dropout ? 1 : 0) : -1) {
+      case 0: return launch_fwd_variant<T, D, false, false, false, kPad, false, false, Half>(b, grid, stream);
+      case 1: return launch_fwd_variant<T, D, false, false, true, kPad, false, false, Half>(b, grid, stream);
+      case 2: return launch_fwd_variant<T, D, true, false, false, kPad, false, false, Half>(b, grid, stream);
+      case 3: return launch_fwd_variant<T, D, true, false, true, kPad, false, false, Half>(b, grid, stream);
+    }
   }
   const int key = (windowed ? 4 : 0) | (bias ? 2 : 0) | (dropout ? 1 : 0);
   switch (key) {

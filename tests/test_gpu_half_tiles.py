@@ -1,0 +1,26 @@
+"""Forward tiles of 128 rows, two workgroups per CU, where 256-row tiles leave rounds empty: many heads with
+sequences a little over half a tile or a tile.  Against the oracle at ragged last tiles, masks and dropout."""
+import pytest
+import torch
+
+from test_gpu_attention import _run_case
+
+pytestmark = pytest.mark.gpu
+
+BF, HF = torch.bfloat16, torch.float16
+CASES = [
+    # B, Hq, Hk, Sq, Sk, D, dtype, causal, dropout
+    (40, 16, 16, 128, 128, 64, BF, False, 0.0),       # 3 rounds against 2
+    (40, 16, 4, 97, 130, 64, HF, True, 0.1),
+    (20, 32, 32, 1, 300, 64, BF, False, 0.1),         # (without dropout the rows kernel takes it)
+    (40, 16, 8, 113, 65, 128, BF, (40, 9), 0.0),
+    (16, 36, 36, 129, 33, 128, HF, False, 0.2),
+    (40, 16, 16, 128, 97, 96, HF, True, 0.0),
+    (40, 16, 16, 70, 128, 40, BF, False, 0.0),
+]
+
+
+@pytest.mark.parametrize('case', CASES, ids=lambda c: '-'.join(str(x).replace('torch.', '') for x in c))
+def test_half_tiles_meet_the_oracle(case):
+    B, Hq, Hk, Sq, Sk, D, dtype, causal, p = case
+    _run_case(B, Hq, Hk, Sq, Sk, D, dtype, causal, dropout_p=p, seed=23)
