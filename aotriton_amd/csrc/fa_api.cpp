@@ -646,8 +646,16 @@ fa::DropoutArgs dropout_args(float p, const fa_tensor0& seed, const fa_tensor0& 
 // packed sequences, dB wanted, an empty tensor).  *ds_bytes / *stat_bytes: the parts of the buffer.
 int64_t ds_workspace_need(const fa_bwd_params* p, const Shape& s, int* ntq, int* ntk, int64_t* ds_bytes,
                           int64_t* stat_bytes) {
-  if (s.elementwise || !is_16bit(p->Q.dtype) || (s.d != 64 && s.d != 128 && s.d != 256) || s.num_seqlens != 0 || p->DB.ptr != nullptr ||
+  if (s.elementwise || !is_16bit(p->Q.dtype) || (s.d != 64 && s.d != 128 && s.d != 256) || s.num_seqlens != 0 ||
       s.batch <= 0 || s.max_sq <= 0 || s.max_sk <= 0)
+    return 0;
+  // dB leaves the dQ-from-dS kernel as 16-byte pieces of its rows, or is left to the recomputing one; so are small
+  // calls, where the third launch costs what is saved (us forward + backward, recomputing -> stored: B2 H8 S256 D64
+  // 50 -> 53, B8 H12 S512 D64 118 -> 100, D128 148 -> 132, D256 468 -> 420, B16 H16 S1024 D64 842 -> 795, causal 670 -> 579)
+  if (p->DB.ptr != nullptr &&
+      ((int64_t)s.batch * s.hq * s.max_sq * s.max_sk < (int64_t)1 << 22 ||
+       p->DB.strides[3] != 1 || ((p->DB.strides[0] | p->DB.strides[1] | p->DB.strides[2]) & 7) != 0 ||
+       (reinterpret_cast<uintptr_t>(p->DB.ptr) & 15) != 0))
     return 0;
   // the 64-column build: 2 bytes per pair are too many for its little GEMM work unless the dQ kernel is
   // spared a bias or the Philox arithmetic (same box, stored / recomputing: 1.05-1.14 plain, 0.69-0.81 with either)

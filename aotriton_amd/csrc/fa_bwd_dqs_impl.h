@@ -32,7 +32,12 @@ struct DqsSmem {     // two stages of the K tile (swizzled), then one dS area pe
 };
 
 // One Q tile of 256 rows (8 waves x 32 queries) of head h against the key tiles that see it.
-template <typename T, int D, int BN, int kPad, bool kWideTile>
+// kDb: the stored dS is also what dB is, in another layout: the wave's operands of a step go through its LDS
+// area once more, into rows, and leave as 16-byte pieces (dB has unit column stride and rows of aligned
+// pieces); where no stored tile is, dB is zero.  The kernel stays bound by its streams, two written or
+// read once instead of one (B8 H12 S512 D64: 25 us for 50 MB in and 50 MB out, with 5 us for the statistics, where
+// the dQ kernel that recomputes S and dP and writes dB took 48).
+template <typename T, int D, int BN, int kPad, bool kWideTile, bool kDb>
 __device__ __forceinline__ void dqs_item(const BwdArgs& a, const int h, const int mt, const int z, char* smem_raw) {
   using Tr = Traits<T>;
   using op_t = typename Tr::op_t;
@@ -80,6 +85,23 @@ __device__ __forceinline__ void dqs_item(const BwdArgs& a, const int h, const in
   T* dqptr = reinterpret_cast<T*>(a.dq) + (int64_t)si.batch_index * a.sdq.z + (int64_t)h * a.sdq.h +
              (int64_t)(si.q_start + row_c) * a.sdq.s;
 
+  constexpr int BCR = BN / 8, BRI = 64 / BCR;      // dB: pieces per row of a step, rows per access
+  T* const db_head = kDb ? reinterpret_cast<T*>(a.db) + (int64_t)si.batch_index * a.sdb_z + (int64_t)h * a.sdb_h : nullptr;
+  auto db_piece = [&](int j, int i, const op_t x) {
+    const int m = q0 + wave_u * 32 + BRI * i + lane / BCR, n = j * BN + lane % BCR * 8;
+    if (m >= si.seqlen_q || n >= si.seqlen_k) return;
+    T* p = db_head + (int64_t)m * a.sdb_m + n;
+    if (n + 8 <= si.seqlen_k) {
+      *reinterpret_cast<op_t*>(p) = x;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (n + e < si.seqlen_k) p[e] = x[e];
+    }
+  };
+  const int j_steps = (si.seqlen_k + BN - 1) / BN;
+  int db_lo = 0, db_hi = -1;      // steps whose dB comes from stored tiles
+
   f32x16 dq[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db)
@@ -94,6 +116,8 @@ __device__ __forceinline__ void dqs_item(const BwdArgs& a, const int h, const in
     j1 = j1 < j_end ? j1 : j_end;
     const int jw0 = bw.lo * SPT, jw1 = bw.lo <= bw.hi ? bw.hi * SPT + SPT - 1 : -1;
     auto active = [&](int j) { return j >= jw0 && j <= jw1 && j <= j1; };
+    db_lo = jw0;
+    db_hi = jw1 < j1 ? jw1 : j1;
 
     // ---- K tiles: global -> registers -> LDS (swizzled), one step ahead ------------------------
     const T* kbase = reinterpret_cast<const T*>(a.k) + (int64_t)si.batch_index * a.sk.z + (int64_t)hk * a.sk.h +
@@ -155,14 +179,31 @@ __device__ __forceinline__ void dqs_item(const BwdArgs& a, const int h, const in
       load_ds(ring_tag, j + PD);
       if (act) {
         const char* Kb = smem_raw + (j & 1) * SM::K_BYTES;
+        op_t bs[kDb ? BN / 16 : 1];
 #pragma unroll
         for (int tk = 0; tk < BN / 16; ++tk) {
           const char* p = ds_area + ds_rd + (tk >> 1) * 2048 + (tk & 1) * 512;
           const q4_t lo = Tr::lds_read_tr(reinterpret_cast<const T*>(p));
           const q4_t up = Tr::lds_read_tr(reinterpret_cast<const T*>(p + 256));
           const op_t b = __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7);
+          if constexpr (kDb) bs[tk] = b;
 #pragma unroll
           for (int db = 0; db < DB; ++db) dq[db] = Tr::mfma(swz_read_tr<T, D>(Kb, tr_a0, tr_a1, tk, db), b, dq[db]);
+        }
+        if constexpr (kDb) {
+          // b holds the keys 16 tk + 4 hi + {0..3} and 16 tk + 8 + 4 hi + {0..3} of the lane's row; the pieces of a
+          // row of the area are exchanged by the row's number, so that rows do not share banks
+#pragma unroll
+          for (int tk = 0; tk < BN / 16; ++tk) {
+            char* r = ds_area + c * (BN * 2) + 8 * hi;
+            *reinterpret_cast<q4_t*>(r + (((2 * tk) ^ (c % BCR)) << 4)) = __builtin_shufflevector(bs[tk], bs[tk], 0, 1, 2, 3);
+            *reinterpret_cast<q4_t*>(r + (((2 * tk + 1) ^ (c % BCR)) << 4)) = __builtin_shufflevector(bs[tk], bs[tk], 4, 5, 6, 7);
+          }
+#pragma unroll
+          for (int i = 0; i < 32 / BRI; ++i) {
+            const int r = BRI * i + lane / BCR;
+            db_piece(j, i, *reinterpret_cast<const op_t*>(ds_area + r * (BN * 2) + (((lane % BCR) ^ (r % BCR)) << 4)));
+          }
         }
       }
       store_k((j + 1) & 1);
@@ -185,6 +226,12 @@ __device__ __forceinline__ void dqs_item(const BwdArgs& a, const int h, const in
     }
   }
 
+  if constexpr (kDb) {
+    for (int j = 0; j < j_steps; ++j)
+      if (j < db_lo || j > db_hi)
+#pragma unroll
+        for (int i = 0; i < 32 / BRI; ++i) db_piece(j, i, op_t{});
+  }
   if (row_ok) {
 #pragma unroll
     for (int db = 0; db < DB; ++db)
@@ -200,7 +247,7 @@ __device__ __forceinline__ void dqs_item(const BwdArgs& a, const int h, const in
 
 // One workgroup per Q tile on a 1-D grid: consecutive ids go round the XCDs, an XCD takes its
 // (batch, q-head) pairs two at a time, the heaviest (last) tile of a causal mask first.
-template <typename T, int D, int BN, int kPad, bool kWideTile>
+template <typename T, int D, int BN, int kPad, bool kWideTile, bool kDb>
 __global__ __attribute__((amdgpu_flat_work_group_size(512, 512))) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void bwd_dqs_kernel(const BwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
@@ -213,7 +260,7 @@ void bwd_dqs_kernel(const BwdArgs a) {
   const int mt = a.num_m_tiles - 1 - gr / a.zh_group;
   int z, h;
   split_zh(zh, a.num_zh / a.hq, a.hq / a.hk, z, h);
-  dqs_item<T, D, BN, kPad, kWideTile>(a, h, mt, z, smem_raw);
+  dqs_item<T, D, BN, kPad, kWideTile, kDb>(a, h, mt, z, smem_raw);
 }
 
 template <typename T, int D, int kPad>
@@ -226,11 +273,15 @@ hipError_t launch_bwd_dqs(const BwdArgs& a0, hipStream_t stream) {
   a.zh_group = a.hq / a.hk > 2 ? (a.hq / a.hk > 8 ? 8 : a.hq / a.hk) : 2;
   a.items_per_xcd = ((a.zh_per_xcd + a.zh_group - 1) / a.zh_group) * a.zh_group * a.num_m_tiles;
   dim3 grid((unsigned)(kNumXcd * a.items_per_xcd));
+  constexpr int lds = DqsSmem<D, BN>::BYTES;
+  const bool db = a.db != nullptr;
   if constexpr (D == 64) {
     if (a.bias != nullptr && !(a.drop.p > 0.f))      // kWide: how the dK/dV kernel of such a call stored it
-      return launch_with_lds<bwd_dqs_kernel<T, D, BN, kPad, true>>(grid, 512, DqsSmem<D, BN>::BYTES, stream, a);
+      return db ? launch_with_lds<bwd_dqs_kernel<T, D, BN, kPad, true, true>>(grid, 512, lds, stream, a)
+                : launch_with_lds<bwd_dqs_kernel<T, D, BN, kPad, true, false>>(grid, 512, lds, stream, a);
   }
-  return launch_with_lds<bwd_dqs_kernel<T, D, BN, kPad, false>>(grid, 512, DqsSmem<D, BN>::BYTES, stream, a);
+  return db ? launch_with_lds<bwd_dqs_kernel<T, D, BN, kPad, false, true>>(grid, 512, lds, stream, a)
+            : launch_with_lds<bwd_dqs_kernel<T, D, BN, kPad, false, false>>(grid, 512, lds, stream, a);
 }
 
 }  // namespace fa
