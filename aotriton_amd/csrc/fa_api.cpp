@@ -651,9 +651,10 @@ int64_t ds_workspace_need(const fa_bwd_params* p, const Shape& s, int* ntq, int*
     return 0;
   // dB leaves the dQ-from-dS kernel as 16-byte pieces of its rows, or is left to the recomputing one; so are small
   // calls, where the third launch costs what is saved (us forward + backward, recomputing -> stored: B2 H8 S256 D64
-  // 50 -> 53, B8 H12 S512 D64 118 -> 100, D128 148 -> 132, D256 468 -> 420, B16 H16 S1024 D64 842 -> 795, causal 670 -> 579)
+  // 50 -> 53, B8 H12 S512 D64 118 -> 100, D128 148 -> 132, D256 468 -> 420, B16 H16 S1024 D64 842 -> 795, causal 670 -> 579),
+  // and long rows at D = 64 (H8 S4096 causal 395 -> 370, H16 S8192 window 4000 1425 -> 1482)
   if (p->DB.ptr != nullptr &&
-      ((int64_t)s.batch * s.hq * s.max_sq * s.max_sk < (int64_t)1 << 22 ||
+      ((int64_t)s.batch * s.hq * s.max_sq * s.max_sk < (int64_t)1 << 22 || (s.d == 64 && s.max_sk > 4096) ||
        p->DB.strides[3] != 1 || ((p->DB.strides[0] | p->DB.strides[1] | p->DB.strides[2]) & 7) != 0 ||
        (reinterpret_cast<uintptr_t>(p->DB.ptr) & 15) != 0))
     return 0;
