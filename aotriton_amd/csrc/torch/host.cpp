@@ -439,6 +439,45 @@ std::tuple<Tensor, Tensor> forward_autograd(const Tensor& q, const Tensor& k, co
   return {r[0], r[1]};
 }
 
+// The backward op has no derivative of its own.  Its results say so when something asks for one; without
+// an Autograd kernel PyTorch would hand back undefined gradients with a warning, and a double backward
+// through flash_attention_forward would run this op on zeros.
+struct OpBackwardFunction : torch::autograd::Function<OpBackwardFunction> {
+  static variable_list forward(AutogradContext*, const Tensor& dout, const Tensor& q, const Tensor& k, const Tensor& v,
+                               const std::optional<Tensor>& bias, const Tensor& out, const Tensor& lse, double dropout_p,
+                               const c10::SymInt& causal_type, const c10::SymInt& window_left,
+                               const c10::SymInt& window_right, double sm_scale, const Tensor& seed,
+                               const Tensor& offset, bool need_dbias, const c10::SymInt& backend) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    auto [dq, dk, dv, db] = backward_op().call(dout, q, k, v, bias, out, lse, dropout_p, causal_type, window_left,
+                                               window_right, sm_scale, seed, offset, need_dbias, backend);
+    return {dq, dk, dv, db};
+  }
+  static variable_list backward(AutogradContext*, variable_list) {
+    TORCH_CHECK(false, "Trying to backward through aotriton_amd::flash_attention_backward, which has no autograd formula: "
+                       "second derivatives of the attention operators are not implemented");
+  }
+};
+
+std::tuple<Tensor, Tensor, Tensor, Tensor> backward_autograd(
+    const Tensor& dout, const Tensor& q, const Tensor& k, const Tensor& v, const std::optional<Tensor>& bias,
+    const Tensor& out, const Tensor& lse, double dropout_p, c10::SymInt causal_type, c10::SymInt window_left,
+    c10::SymInt window_right, double sm_scale, const Tensor& seed, const Tensor& offset, bool need_dbias,
+    c10::SymInt backend) {
+  const bool grad = at::GradMode::is_enabled() &&
+                    (dout.requires_grad() || q.requires_grad() || k.requires_grad() || v.requires_grad() ||
+                     (bias.has_value() && bias->defined() && bias->requires_grad()) || out.requires_grad() ||
+                     lse.requires_grad());
+  if (!grad) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    return backward_op().call(dout, q, k, v, bias, out, lse, dropout_p, causal_type, window_left, window_right, sm_scale,
+                              seed, offset, need_dbias, backend);
+  }
+  variable_list r = OpBackwardFunction::apply(dout, q, k, v, bias, out, lse, dropout_p, causal_type, window_left, window_right,
+                                              sm_scale, seed, offset, need_dbias, backend);
+  return {r[0], r[1], r[2], r[3]};
+}
+
 TORCH_LIBRARY(aotriton_amd, m) {
   m.def("philox_state(Tensor like, SymInt increment) -> (Tensor, Tensor)", {at::Tag::nondeterministic_seeded});
   m.def("flash_attention_forward(Tensor q, Tensor k, Tensor v, Tensor? bias, float dropout_p, SymInt causal_type, "
@@ -452,7 +491,10 @@ TORCH_LIBRARY_IMPL(aotriton_amd, CUDA, m) {
   m.impl("flash_attention_forward", &forward_kernel);
   m.impl("flash_attention_backward", &backward_kernel);
 }
-TORCH_LIBRARY_IMPL(aotriton_amd, Autograd, m) { m.impl("flash_attention_forward", &forward_autograd); }
+TORCH_LIBRARY_IMPL(aotriton_amd, Autograd, m) {
+  m.impl("flash_attention_forward", &forward_autograd);
+  m.impl("flash_attention_backward", &backward_autograd);
+}
 
 // ---- argument parsing of the Python functions ---------------------------------------------------------
 

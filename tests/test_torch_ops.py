@@ -27,6 +27,33 @@ def test_fake_implementations_give_the_operator_shapes():
     assert seed.shape == (1,) and seed.dtype == torch.uint64 and off.dtype == torch.uint64
 
 
+def _meta(Hk=4, grad=True):
+    mk = lambda *s: torch.empty(*s, dtype=torch.bfloat16, device='meta', requires_grad=grad)
+    return mk(2, 4, 16, 64), mk(2, Hk, 24, 64), mk(2, Hk, 24, 64)
+
+
+def test_second_derivatives_are_refused():
+    """neither a double backward through the forward op nor a backward through the backward op may
+    answer with zeros"""
+    from aotriton_amd.torch_ops import scaled_dot_product_attention as sdpa
+    q, k, v = _meta()
+    o = sdpa(q, k, v)
+    g, = torch.autograd.grad(o.sum(), [q], create_graph=True)
+    assert g.requires_grad
+    with pytest.raises(RuntimeError, match='Trying to backward through'):
+        torch.autograd.grad(g.sum(), [q, k, v])
+    s = torch.empty(1, dtype=torch.uint64, device='meta')
+    lse = torch.empty(8, 16, device='meta')
+    r = torch.ops.aotriton_amd.flash_attention_backward(o.detach(), q, k, v, None, o.detach(), lse, 0.0, 0, 0, 0, 0.1,
+                                                        s, s, False, -1)
+    assert r[0].requires_grad
+    with pytest.raises(RuntimeError, match='Trying to backward through'):
+        torch.autograd.grad(r[0].sum(), [q])
+    with torch.no_grad():
+        r = torch.ops.aotriton_amd.flash_attention_backward(o, q, k, v, None, o, lse, 0.0, 0, 0, 0, 0.1, s, s, False, -1)
+    assert not r[0].requires_grad
+
+
 def _inputs(B=2, Hq=4, Hk=2, Sq=150, Sk=170, D=64, dtype=torch.bfloat16, bias=False, seed=0):
     from tests._util import make_inputs
     return make_inputs(B, Hq, Hk, Sq, Sk, D, dtype, DEV, seed=seed, bias=bias)
