@@ -46,6 +46,7 @@ def attention(q, k, v, b, causal, sm_scale, dropout_p, ext=None):
 
 
 def attention_varlen(q, k, v, seqlens_q, seqlens_k, causal, sm_scale, dropout_p, ext=None):
-    """Compact varlen: q (1, Hq, total_q, D), k/v (1, Hk, total_k, D); the lengths are host arrays."""
+    """Compact varlen: q (1, Hq, total_q, D), k/v (1, Hk, total_k, D); the lengths are host arrays that add
+    up to total_q and total_k (ValueError otherwise)."""
     return _torch_host.attention_varlen(q, k, v, np.asarray(seqlens_q).tolist(), np.asarray(seqlens_k).tolist(),
                                         *translate_causal(causal), sm_scale, dropout_p, *_extra_args(ext or _DEFAULTS))

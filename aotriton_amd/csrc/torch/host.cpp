@@ -687,6 +687,27 @@ std::vector<int64_t> int_list(PyObject* o) {
   return v;
 }
 
+// Appends the offsets of sequences of these lengths in a packed (1, H, tokens, D) tensor and returns the
+// longest length.  The lengths have to add up to the tokens: rows past them would be left unwritten (Out, logsumexp,
+// gradients), and with more the kernels would run past the tensors.
+int64_t push_offsets(std::vector<uint32_t>* words, const std::vector<int64_t>& lens, const Tensor& packed, const char* side) {
+  TORCH_CHECK_VALUE(packed.dim() == 4, "packed sequences are (1, heads, tokens, head_dim) tensors");
+  TORCH_CHECK_VALUE(!lens.empty(), "no ", side, " sequence");
+  const int64_t tokens = packed.size(2);
+  TORCH_CHECK_VALUE(tokens <= std::numeric_limits<int32_t>::max(), "offsets of packed sequences are 32-bit");
+  int64_t sum = 0, longest = 0;
+  words->push_back(0);
+  for (const int64_t len : lens) {
+    TORCH_CHECK_VALUE(len >= 0 && len <= tokens - sum, side, " sequence lengths must not be negative and must add up to the ",
+                      tokens, " packed tokens");
+    sum += len;
+    longest = std::max(longest, len);
+    words->push_back((uint32_t)sum);
+  }
+  TORCH_CHECK_VALUE(sum == tokens, side, " sequence lengths add up to ", sum, ", the packed tensor holds ", tokens, " tokens");
+  return longest;
+}
+
 // attention_varlen(q, k, v, lens_q, lens_k, then as attention from `type` on): compact packed sequences
 PyObject* py_attention_varlen(PyObject*, PyObject* const* argv, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -698,19 +719,10 @@ PyObject* py_attention_varlen(PyObject*, PyObject* const* argv, Py_ssize_t n) {
   variable_list r;
   {
     pybind11::gil_scoped_release no_gil;
-    const c10::DeviceGuard guard(q.device());
     std::vector<uint32_t> w;
     w.reserve(lq.size() + lk.size() + 2);
-    int64_t longest[2] = {0, 0};
-    for (int side = 0; side < 2; ++side) {
-      int64_t sum = 0;
-      w.push_back(0);
-      for (int64_t len : side == 0 ? lq : lk) {
-        sum += len;
-        longest[side] = std::max(longest[side], len);
-        w.push_back((uint32_t)sum);
-      }
-    }
+    const int64_t longest[2] = {push_offsets(&w, lq, q, "query"), push_offsets(&w, lk, k, "key")};
+    const c10::DeviceGuard guard(q.device());
     at::AutoDispatchBelowADInplaceOrView below;
     const Tensor cu = words_on_device(w, at::kInt, (int64_t)w.size(), q.device());
     x.vl.cu_q = cu.narrow(0, 0, (int64_t)lq.size() + 1);
