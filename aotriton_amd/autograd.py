@@ -45,8 +45,13 @@ def attention(q, k, v, b, causal, sm_scale, dropout_p, ext=None):
     return _torch_host.attention(q, k, v, b, *translate_causal(causal), sm_scale, dropout_p, *_extra_args(ext or _DEFAULTS))
 
 
+def _lengths(seqlens):
+    """A host array of any shape and number type as the list of ints that the native function reads."""
+    return np.asarray(seqlens).reshape(-1).astype(np.int64).tolist()
+
+
 def attention_varlen(q, k, v, seqlens_q, seqlens_k, causal, sm_scale, dropout_p, ext=None):
     """Compact varlen: q (1, Hq, total_q, D), k/v (1, Hk, total_k, D); the lengths are host arrays that add
     up to total_q and total_k (ValueError otherwise)."""
-    return _torch_host.attention_varlen(q, k, v, np.asarray(seqlens_q).tolist(), np.asarray(seqlens_k).tolist(),
+    return _torch_host.attention_varlen(q, k, v, _lengths(seqlens_q), _lengths(seqlens_k),
                                         *translate_causal(causal), sm_scale, dropout_p, *_extra_args(ext or _DEFAULTS))
