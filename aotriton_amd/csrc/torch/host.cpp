@@ -306,8 +306,17 @@ struct AttentionFunction : torch::autograd::Function<AttentionFunction> {
   }
 };
 
+// There is no forward-mode formula.  A call without a gradient goes past the Function, whose own error would
+// come after the launch: without this check such a call would answer without the tangent.
+void refuse_tangents(std::initializer_list<const Tensor*> inputs) {
+  for (const Tensor* t : inputs)
+    TORCH_CHECK_NOT_IMPLEMENTED(!t->defined() || !t->_fw_grad(0).defined(),
+                                "forward-mode AD of the attention operators (jvp) is not implemented");
+}
+
 // (Out, encoded softmax, logsumexp); the last two undefined unless asked for
 variable_list attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& b, const AttentionOptions& x) {
+  refuse_tangents({&q, &k, &v, &b});
   const bool grad = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad() ||
                                                    (b.defined() && b.requires_grad()));
   if (grad) {
@@ -435,6 +444,8 @@ std::tuple<Tensor, Tensor> forward_autograd(const Tensor& q, const Tensor& k, co
     at::AutoDispatchBelowADInplaceOrView below;
     return forward_op().call(q, k, v, bias, dropout_p, causal_type, window_left, window_right, sm_scale, seed, offset);
   }
+  const Tensor b = bias.value_or(Tensor());
+  refuse_tangents({&q, &k, &v, &b});
   variable_list r = OpFunction::apply(q, k, v, bias, dropout_p, causal_type, window_left, window_right, sm_scale, seed, offset);
   return {r[0], r[1]};
 }
@@ -473,6 +484,8 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> backward_autograd(
     return backward_op().call(dout, q, k, v, bias, out, lse, dropout_p, causal_type, window_left, window_right, sm_scale,
                               seed, offset, need_dbias, backend);
   }
+  const Tensor b = bias.value_or(Tensor());
+  refuse_tangents({&dout, &q, &k, &v, &b, &out, &lse});
   variable_list r = OpBackwardFunction::apply(dout, q, k, v, bias, out, lse, dropout_p, causal_type, window_left, window_right,
                                               sm_scale, seed, offset, need_dbias, backend);
   return {r[0], r[1], r[2], r[3]};
@@ -717,6 +730,7 @@ PyObject* py_attention_varlen(PyObject*, PyObject* const* argv, Py_ssize_t n) {
   const std::vector<int64_t> lq = int_list(a.next()), lk = int_list(a.next());
   AttentionOptions x = read_options(a);
   variable_list r;
+  refuse_tangents({&q, &k, &v});
   {
     pybind11::gil_scoped_release no_gil;
     std::vector<uint32_t> w;

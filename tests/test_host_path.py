@@ -34,3 +34,38 @@ def test_packed_lengths_of_any_shape_and_number_type(lens):
     q, k = _meta(1, 4, 16, 64), _meta(1, 2, 24, 64)
     with pytest.raises(ValueError, match='key sequence lengths add up to 23'):
         attention_varlen(q, k, k, lens, [10, 13], False, 0.125, 0.0)
+
+
+@pytest.mark.parametrize('requires_grad', [False, True])
+@pytest.mark.parametrize('entry, dual', [(e, d) for e in ('attention', 'attention_varlen', 'sdpa') for d in 'qkvb'
+                                         if (e, d) != ('attention_varlen', 'b')])      # (that one takes no bias)
+def test_forward_mode_is_refused(entry, dual, requires_grad):
+    """a tangent must not be dropped, with or without a gradient to record"""
+    import torch.autograd.forward_ad as fwad
+    from aotriton_amd.autograd import attention, attention_varlen
+    from aotriton_amd.sdpa import scaled_dot_product_attention
+    t = {'q': _meta(1, 4, 16, 64), 'k': _meta(1, 4, 24, 64), 'v': _meta(1, 4, 24, 64), 'b': _meta(1, 4, 16, 24)}
+    for x in t.values():
+        x.requires_grad_(requires_grad)
+    with fwad.dual_level():
+        t[dual] = fwad.make_dual(t[dual], torch.empty_like(t[dual]))
+        with pytest.raises(NotImplementedError, match='forward-mode'):
+            if entry == 'attention':
+                attention(t['q'], t['k'], t['v'], t['b'], False, 0.125, 0.0)
+            elif entry == 'attention_varlen':
+                attention_varlen(t['q'], t['k'], t['v'], [16], [24], False, 0.125, 0.0)
+            else:
+                scaled_dot_product_attention(t['q'], t['k'], t['v'], t['b'])
+
+
+def test_forward_mode_of_the_ops_is_refused_with_a_gradient():
+    import torch.autograd.forward_ad as fwad
+    from aotriton_amd.torch_ops import flash_attention_backward, scaled_dot_product_attention
+    q, k = _meta(1, 4, 16, 64).requires_grad_(), _meta(1, 4, 24, 64)
+    s, lse = torch.empty(1, dtype=torch.uint64, device='meta'), torch.empty(4, 16, device='meta')
+    with fwad.dual_level():
+        d = fwad.make_dual(q, torch.empty_like(q))
+        with pytest.raises(NotImplementedError, match='forward-mode'):
+            scaled_dot_product_attention(d, k, k)
+        with pytest.raises(NotImplementedError, match='forward-mode'):
+            flash_attention_backward(q.detach(), d, k, k, None, q.detach(), lse, 0.0, 0, 0, 0, 0.1, s, s, False, -1)
