@@ -54,6 +54,44 @@ def test_second_derivatives_are_refused():
     assert not r[0].requires_grad
 
 
+class _Named(torch.Tensor):
+    """a subclass that notes the functions it is asked for"""
+    seen = []
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        cls.seen.append(func)
+        return super().__torch_function__(func, types, args, kwargs or {})
+
+
+@pytest.mark.parametrize('which', ['query', 'attn_mask'])
+def test_sdpa_of_a_tensor_subclass(which):
+    from aotriton_amd.torch_ops import scaled_dot_product_attention as sdpa
+    q, k, v = _meta(grad=False)
+    kw = dict(query=q, key=k, value=v, attn_mask=torch.empty(16, 24, dtype=torch.bool, device='meta'))
+    kw[which] = kw[which].as_subclass(_Named)
+    _Named.seen.clear()
+    assert type(sdpa(**kw)) is _Named
+    assert torch.ops.aotriton_amd.flash_attention_forward in _Named.seen
+
+
+@pytest.mark.parametrize('dropout_p', [0.0, 0.1])
+def test_function_modes_see_the_ops_of_sdpa(dropout_p):
+    from aotriton_amd.torch_ops import scaled_dot_product_attention as sdpa
+
+    class Seen(torch.overrides.TorchFunctionMode):
+        funcs = []
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            self.funcs.append(func)
+            return func(*args, **(kwargs or {}))
+
+    with Seen() as mode:
+        sdpa(*_meta(grad=False), dropout_p=dropout_p)
+    assert torch.ops.aotriton_amd.flash_attention_forward in mode.funcs
+    assert (torch.ops.aotriton_amd.philox_state in mode.funcs) == (dropout_p > 0)
+
+
 def _inputs(B=2, Hq=4, Hk=2, Sq=150, Sk=170, D=64, dtype=torch.bfloat16, bias=False, seed=0):
     from tests._util import make_inputs
     return make_inputs(B, Hq, Hk, Sq, Sk, D, dtype, DEV, seed=seed, bias=bias)
