@@ -17,6 +17,7 @@
 #include <ATen/ATen.h>
 #include <ATen/core/dispatch/Dispatcher.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
@@ -791,6 +792,17 @@ Sdpa prepare(const Tensor& query, const Tensor& key, const Tensor& value, const 
   return s;
 }
 
+// Tracers (make_fx, AOTAutograd) and other dispatch modes, tensors that dispatch to Python, functorch transforms: sizes
+// may be symbols there, and reading them here as integers would fix them in the trace.  The Python route keeps them.
+bool traced(std::initializer_list<const Tensor*> inputs) {
+  static constexpr c10::DispatchKeySet keys({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched,
+                                             c10::DispatchKey::FuncTorchGradWrapper});
+  if (c10::impl::TorchDispatchModeTLS::any_modes_set()) return true;
+  for (const Tensor* t : inputs)
+    if (t->defined() && t->key_set().has_any(keys)) return true;
+  return false;
+}
+
 struct SdpaArgs {
   Tensor q, k, v, mask;
   double dropout_p;
@@ -811,11 +823,12 @@ SdpaArgs read_sdpa(Args& a) {
 }
 
 // sdpa_ops(query, key, value, attn_mask, dropout_p, is_causal, scale, enable_gqa): on the custom ops,
-// Philox state from torch's generator
+// Philox state from torch's generator; None where the Python route has to take the call
 PyObject* py_sdpa_ops(PyObject*, PyObject* const* argv, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   Args a{argv, n};
   const SdpaArgs in = read_sdpa(a);
+  if (traced({&in.q, &in.k, &in.v, &in.mask})) Py_RETURN_NONE;
   Tensor out;
   {
     pybind11::gil_scoped_release no_gil;

@@ -74,7 +74,9 @@ def scaled_dot_product_attention(query, key, value, attn_mask=None, dropout_p=0.
     """
     # (subclasses and function modes that override torch's functions have to see the calls below)
     if not torch.compiler.is_compiling() and not torch.overrides.has_torch_function((query, key, value, attn_mask)):
-        return _torch_host.sdpa_ops(query, key, value, attn_mask, dropout_p, is_causal, scale, enable_gqa)
+        out = _torch_host.sdpa_ops(query, key, value, attn_mask, dropout_p, is_causal, scale, enable_gqa)
+        if out is not None:      # None: under a dispatch mode or a functorch transform
+            return out
     q, k, v, bias, sm_scale = prepare(query, key, value, attn_mask, is_causal, scale, enable_gqa)
     hq = q.shape[1]
     if dropout_p > 0.0:

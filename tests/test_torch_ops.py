@@ -54,6 +54,23 @@ def test_second_derivatives_are_refused():
     assert not r[0].requires_grad
 
 
+def test_symbolic_trace_of_sdpa_keeps_its_sizes():
+    """the Philox increment of a dropout call follows the traced sizes instead of being a constant"""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from aotriton_amd.torch_ops import scaled_dot_product_attention as sdpa
+    g = make_fx(lambda q, k, v: sdpa(q, k, v, dropout_p=0.1), tracing_mode='symbolic')(*_meta(grad=False))
+    calls = {n.target: n for n in g.graph.nodes if n.op == 'call_function'}
+    assert isinstance(calls[torch.ops.aotriton_amd.philox_state.default].args[1], torch.fx.Node)
+    assert torch.ops.aten.size.default not in calls
+
+
+def test_batched_tensors_reach_the_ops():
+    from aotriton_amd.torch_ops import scaled_dot_product_attention as sdpa
+    q = torch.empty(3, 2, 4, 16, 64, dtype=torch.bfloat16, device='meta')
+    mask = torch.empty(16, 16, dtype=torch.bool, device='meta')
+    assert torch.func.vmap(lambda q, k, v: sdpa(q, k, v, mask))(q, q, q).shape == q.shape
+
+
 class _Named(torch.Tensor):
     """a subclass that notes the functions it is asked for"""
     seen = []
