@@ -492,13 +492,19 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> backward_autograd(
   return {r[0], r[1], r[2], r[3]};
 }
 
+// (pt2_compliant_tag: fake implementations and Autograd kernels are there, so that torch.compile may keep the
+// ops in its graphs also where it is told to take compliant ops only)
 TORCH_LIBRARY(aotriton_amd, m) {
-  m.def("philox_state(Tensor like, SymInt increment) -> (Tensor, Tensor)", {at::Tag::nondeterministic_seeded});
+  const std::vector<at::Tag> compliant{at::Tag::pt2_compliant_tag};
+  m.def("philox_state(Tensor like, SymInt increment) -> (Tensor, Tensor)",
+        {at::Tag::pt2_compliant_tag, at::Tag::nondeterministic_seeded});
   m.def("flash_attention_forward(Tensor q, Tensor k, Tensor v, Tensor? bias, float dropout_p, SymInt causal_type, "
-        "SymInt window_left, SymInt window_right, float sm_scale, Tensor philox_seed, Tensor philox_offset) -> (Tensor, Tensor)");
+        "SymInt window_left, SymInt window_right, float sm_scale, Tensor philox_seed, Tensor philox_offset) -> (Tensor, Tensor)",
+        compliant);
   m.def("flash_attention_backward(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor? bias, Tensor out, Tensor lse, "
         "float dropout_p, SymInt causal_type, SymInt window_left, SymInt window_right, float sm_scale, "
-        "Tensor philox_seed, Tensor philox_offset, bool need_dbias, SymInt backend) -> (Tensor, Tensor, Tensor, Tensor)");
+        "Tensor philox_seed, Tensor philox_offset, bool need_dbias, SymInt backend) -> (Tensor, Tensor, Tensor, Tensor)",
+        compliant);
 }
 TORCH_LIBRARY_IMPL(aotriton_amd, CUDA, m) {
   m.impl("philox_state", &philox_kernel);

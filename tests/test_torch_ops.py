@@ -27,6 +27,14 @@ def test_fake_implementations_give_the_operator_shapes():
     assert seed.shape == (1,) and seed.dtype == torch.uint64 and off.dtype == torch.uint64
 
 
+@pytest.mark.parametrize('name', ['philox_state', 'flash_attention_forward', 'flash_attention_backward'])
+def test_ops_may_stay_in_compiled_graphs(name):
+    from aotriton_amd import torch_ops  # noqa: F401
+    tags = getattr(torch.ops.aotriton_amd, name).default.tags
+    assert torch.Tag.pt2_compliant_tag in tags
+    assert (torch.Tag.nondeterministic_seeded in tags) == (name == 'philox_state')
+
+
 def _meta(Hk=4, grad=True):
     mk = lambda *s: torch.empty(*s, dtype=torch.bfloat16, device='meta', requires_grad=grad)
     return mk(2, 4, 16, 64), mk(2, Hk, 24, 64), mk(2, Hk, 24, 64)
