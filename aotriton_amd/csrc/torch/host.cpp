@@ -546,7 +546,11 @@ struct Args {
     if (x == (unsigned long long)-1 && PyErr_Occurred()) throw python_error();
     return x;
   }
-  bool flag() { return PyObject_IsTrue(next()) == 1; }
+  bool flag() {
+    const int x = PyObject_IsTrue(next());
+    if (x < 0) throw python_error();
+    return x == 1;
+  }
 };
 
 // attn_fwd(q, k, v, b, sm_scale, M, o, dropout_p, seed, offset1, offset2, seed_out, offset_out, encoded, type, left,

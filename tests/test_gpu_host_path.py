@@ -54,3 +54,12 @@ def test_native_operators_equal_the_views(dropout_p):
         got.append((o, L, dq, dk, dv, db, so.view(torch.int64), oo.view(torch.int64)))
     for x, y in zip(*got):
         assert torch.equal(x, y)
+
+
+def test_a_flag_without_a_truth_value_is_reported():
+    """the error of the conversion, not a result returned with an error set"""
+    import numpy as np
+    from aotriton_amd.torch_ops import scaled_dot_product_attention as sdpa
+    q = torch.zeros(1, 2, 16, 64, device=DEV, dtype=torch.bfloat16)
+    with pytest.raises(ValueError, match='ambiguous'):
+        sdpa(q, q, q, enable_gqa=np.ones(2))
