@@ -18,6 +18,7 @@
 #include <ATen/core/dispatch/Dispatcher.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
@@ -141,19 +142,21 @@ struct LazyDelta {
   static void dispose(fa_lazy_tensor2* self) { static_cast<LazyDelta*>(self->cookie)->held.reset(); }
 };
 
-// scratch memory of a forward, from torch's allocator: ordered with the stream, and a graph's own under capture
+// Scratch memory of a forward, from torch's allocator: ordered with the stream, and a graph's own under capture.
+// It is taken on the current device, whose current stream the call runs on: on another device (where the
+// caller's tensors lie, say) the allocator could hand it on before the kernels are done with it.
 struct Scratch {
   fa_allocator c{};
   Tensor held;
-  at::Device device;
-  explicit Scratch(at::Device d) : device(d) {
+  Scratch() {
     c.cookie = this;
     c.alloc = &alloc;
   }
   static void* alloc(fa_allocator* self, uint64_t bytes) {
     auto* me = static_cast<Scratch*>(self->cookie);
     try {
-      me->held = at::empty({(int64_t)bytes}, at::TensorOptions(at::kByte).device(me->device));
+      const at::Device device(at::kCUDA, c10::hip::current_device());
+      me->held = at::empty({(int64_t)bytes}, at::TensorOptions(at::kByte).device(device));
       return me->held.data_ptr();
     } catch (...) {
       return nullptr;
@@ -191,7 +194,7 @@ void fill_common(P& p, const Tensor& q, const Tensor& k, const Tensor& v, const 
 
 int run_forward(fa_fwd_params& p, const Tensor& lse, const Tensor& o, const Tensor& encoded) {
   TORCH_CHECK(view2(lse, &p.L) && view4(o, &p.Out) && view4(encoded, &p.encoded_softmax), "outputs");
-  Scratch scratch(o.device());
+  Scratch scratch;
   return fa_attn_fwd_alloc(&p, FA_FWD_PARAMS_VERSION, current_stream(), nullptr, &scratch.c);
 }
 
@@ -595,7 +598,7 @@ PyObject* py_attn_fwd(PyObject*, PyObject* const* argv, Py_ssize_t n) {
   {
     pybind11::gil_scoped_release no_gil;
     // torch's allocator orders its memory with torch's current stream only
-    Scratch scratch(o.device());
+    Scratch scratch;
     rc = stream == -1 ? fa_attn_fwd_alloc(&p, FA_FWD_PARAMS_VERSION, current_stream(), &opt, &scratch.c)
                       : fa_attn_fwd(&p, FA_FWD_PARAMS_VERSION, reinterpret_cast<void*>(stream), &opt);
   }
