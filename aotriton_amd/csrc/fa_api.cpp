@@ -712,6 +712,14 @@ DkdvParts dkdv_parts(const fa_bwd_params* p, const Shape& s, int num_cu) {
   return r;
 }
 
+// What of the stored dS (`need` bytes) and the parts fits `room` bytes of workspace, and the bytes it takes.  The
+// parts give way first.
+int64_t fit_workspace(int64_t room, int64_t* need, DkdvParts* parts) {
+  if (*need > room) *need = 0;
+  if (*need + parts->bytes > room) *parts = DkdvParts{1, 1, 0};
+  return *need + parts->bytes;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1106,8 +1114,9 @@ static int attn_bwd_impl(const fa_bwd_params* p_in, int32_t params_version, void
     if (validate_bwd(&p2, params_version, options, &s2, &be2) == FA_SUCCESS && be2 == 0) {
       int ntq = 0, ntk = 0;
       int64_t ds_bytes = 0, stat_bytes = 0;
-      inner = ds_workspace_need(&p2, s2, &ntq, &ntk, &ds_bytes, &stat_bytes) + dkdv_parts(&p2, s2, dev->num_cu).bytes;
-      if ((int64_t)copies + inner > ws_limit_bytes(device_index(dev))) inner = 0;
+      int64_t ds_need = ds_workspace_need(&p2, s2, &ntq, &ntk, &ds_bytes, &stat_bytes);
+      DkdvParts parts = dkdv_parts(&p2, s2, dev->num_cu);
+      inner = fit_workspace(ws_limit_bytes(device_index(dev)) - (int64_t)copies, &ds_need, &parts);
     }
     const size_t need = copies + (size_t)inner;
     void* base = nullptr;
@@ -1232,25 +1241,28 @@ static int attn_bwd_impl(const fa_bwd_params* p_in, int32_t params_version, void
     const int ds_slot = kernel_slot >= 4 ? kernel_slot - 4 : -1;
     int64_t need = (kernel_slot < 0 || ds_slot >= 0) && !own_delta
                        ? ds_workspace_need(p, s, &ntq, &ntk, &ds_bytes, &stat_bytes) : 0;
-    if (need > ws_limit_bytes(device_index(dev)) && ds_slot < 0) need = 0;
-    // (single kernels, for timing, run uncut)
-    DkdvParts parts{1, 1, 0};
-    if (kernel_slot < 0 && !own_delta) parts = dkdv_parts(p, s, dev->num_cu);
-    if (ds_slot >= 0 && (need == 0 || need > ws_limit_bytes(device_index(dev)))) {
+    const int64_t limit = ws_limit_bytes(device_index(dev));
+    if (ds_slot >= 0 && (need == 0 || need > limit)) {
       if (acquired && lazy->dispose != nullptr) lazy->dispose(lazy);
       return FA_ERROR_NOT_SUPPORTED;
     }
+    // (single kernels, for timing, run uncut)
+    DkdvParts parts{1, 1, 0};
+    if (kernel_slot < 0 && !own_delta) parts = dkdv_parts(p, s, dev->num_cu);
+    // a nested call: the caller holds the buffer and has set a part of it aside
     const bool nested = t_ws_nested.active;
-    void* ws = nullptr;
+    int64_t bytes = fit_workspace(nested ? (int64_t)t_ws_nested.bytes : limit, &need, &parts);
+    void* ws = nested ? t_ws_nested.ptr : nullptr;
     bool held = false;
-    if (nested) {
-      // (the caller holds the buffer and has set a part of it aside)
-      if ((size_t)(need + parts.bytes) <= t_ws_nested.bytes) ws = t_ws_nested.ptr;
-    } else if (need + parts.bytes > 0 && need + parts.bytes <= ws_limit_bytes(device_index(dev)) && !stream_is_capturing(stream)) {
-      held = ws_acquire(device_index(dev), (size_t)(need + parts.bytes), stream, &ws) == hipSuccess;
+    if (!nested && bytes > 0 && !stream_is_capturing(stream)) {
+      held = ws_acquire(device_index(dev), (size_t)bytes, stream, &ws) == hipSuccess;
+      if (!held && need > 0 && need < bytes) {      // no memory for both
+        bytes = fit_workspace(need, &need, &parts);
+        held = ws_acquire(device_index(dev), (size_t)bytes, stream, &ws) == hipSuccess;
+      }
       if (!held) {
         ws = nullptr;
-        FA_LOG(2, "attn_bwd: no workspace of %lld bytes, recomputing instead", (long long)(need + parts.bytes));
+        FA_LOG(2, "attn_bwd: no workspace of %lld bytes, recomputing instead", (long long)bytes);
       }
     }
     if (ws != nullptr && need > 0) {
