@@ -10,10 +10,10 @@ from dataclasses import dataclass
 
 import numpy as np
 
-import torch  # noqa: F401  (its libraries come first: the extension links them)
-
-from . import _torch_host
+from . import _host
 from .flash import translate_causal
+
+_torch_host = _host.load()
 
 DEFAULT_PHILOX_SEED = 0x1BF52
 DEFAULT_PHILOX_OFFSET_1 = 0x1D4000

@@ -7,9 +7,7 @@ positional entry points (attn_fwd / attn_bwd / attn_bwd_fused /
 attn_fwd_compact_varlen / attn_bwd_compact_varlen) as thin wrappers that fill the
 v3 params.  Same names, argument meaning and error behaviour (hipError_t return).
 """
-import torch  # noqa: F401  (its libraries come first: the extension links them)
-
-from . import _torch_host
+from ._host import on_first_use as _torch_host
 from .pyaotriton import (T0, T1, T2, T4, DType, Stream, hipError_t, get_name_suffix,  # noqa: F401
                          hipGetLastError, hipDeviceSynchronize, lazy_tensor)
 from .pyaotriton.v2.flash import debug_simulate_encoded_softmax as fa_debug_simulate_encoded_softmax

@@ -9,8 +9,7 @@ import math
 
 import torch
 
-from . import _torch_host
-from .autograd import _DEFAULTS, _extra_args
+from .autograd import _DEFAULTS, _extra_args, _torch_host
 
 
 def prepare(query, key, value, attn_mask, is_causal, scale, enable_gqa):

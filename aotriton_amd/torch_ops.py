@@ -30,9 +30,11 @@ torch.nn.functional.scaled_dot_product_attention and runs on those ops.
 import torch
 from torch import Tensor
 
-from . import _torch_host      # registers the ops
+from . import _host
 from .flash import WindowValue
 from .sdpa import prepare
+
+_torch_host = _host.load()      # registers the ops
 
 __all__ = ['flash_attention_forward', 'flash_attention_backward', 'philox_state', 'scaled_dot_product_attention']
 

@@ -1,8 +1,14 @@
 """What the native host path (csrc/torch/host.cpp) checks before anything reaches a device; meta tensors
 stand in for GPU ones."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 import torch
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 def _meta(*shape):
@@ -69,3 +75,23 @@ def test_forward_mode_of_the_ops_is_refused_with_a_gradient():
             scaled_dot_product_attention(d, k, k)
         with pytest.raises(NotImplementedError, match='forward-mode'):
             flash_attention_backward(q.detach(), d, k, k, None, q.detach(), lse, 0.0, 0, 0, 0, 0.1, s, s, False, -1)
+
+
+def _in_a_new_interpreter(blocked, code):
+    code = f"import sys\nsys.modules[{blocked!r}] = None\n{code}"
+    return subprocess.run([sys.executable, '-c', code], cwd=ROOT, capture_output=True, text=True)
+
+
+@pytest.mark.parametrize('blocked', ['torch', 'aotriton_amd._torch_host'])
+def test_flash_imports_without_torch_or_the_extension(blocked):
+    """the constants, the params and the views are of use without either"""
+    r = _in_a_new_interpreter(blocked, 'from aotriton_amd import flash\nprint(flash.translate_causal((5, 7)), flash.get_name_suffix())')
+    assert r.returncode == 0, r.stderr
+    assert r.stdout.split() == ['(3,', '5,', '7)', '_amd_gfx950']
+
+
+@pytest.mark.parametrize('use', ['aotriton_amd.autograd', 'aotriton_amd.torch_ops',
+                                 'aotriton_amd.flash; aotriton_amd.flash.attn_fwd(*[None] * 14, False, None)'])
+def test_a_missing_extension_is_reported_with_the_way_to_build_it(use):
+    r = _in_a_new_interpreter('aotriton_amd._torch_host', f'import {use}')
+    assert r.returncode != 0 and 'ImportError' in r.stderr and 'python -m aotriton_amd.build' in r.stderr
