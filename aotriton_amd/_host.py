@@ -12,6 +12,8 @@ def load():
         from . import _torch_host
     except ImportError as e:
         raise ImportError(f'{PATH} is missing or does not load with torch {torch.__version__}: {hint}') from e
+    if _torch_host.torch_version != str(torch.__version__):      # its C++ ABI is another with every version
+        raise ImportError(f'{PATH} was built for torch {_torch_host.torch_version}, this is {torch.__version__}: {hint}')
     return _torch_host
 
 

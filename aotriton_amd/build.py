@@ -17,6 +17,7 @@ OBJ = os.path.join(CSRC, 'obj')
 LIB = os.path.join(HERE, 'libaotriton_amd.so')
 HOST_SRC = os.path.join(CSRC, 'torch', 'host.cpp')
 HOST_LIB = os.path.join(HERE, '_torch_host.so')
+HOST_STAMP = os.path.join(OBJ, '_torch_host.torch')      # the torch version it was built for
 HIPCC = os.environ.get('HIPCC', '/opt/rocm/bin/hipcc')
 
 COMMON = [
@@ -86,18 +87,28 @@ def _compile(unit, force):
     return obj, err, r.returncode
 
 
+def _host_is_current(torch_version):
+    """Whether the extension is there, newer than what it is built from, and built for this torch (its C++ ABI
+    is another with every version)."""
+    try:
+        built_for = open(HOST_STAMP).read()
+        newest = max(os.path.getmtime(p) for p in [HOST_SRC, os.path.join(ROOT, 'include', 'aotriton_amd', 'flash.h')])
+        return built_for == torch_version and os.path.getmtime(HOST_LIB) >= newest
+    except OSError:
+        return False
+
+
 def build_host(force=False):
     """The Python extension over torch's C++ API.  It links against the library next to it."""
-    newest = max(os.path.getmtime(p) for p in [HOST_SRC, os.path.join(ROOT, 'include', 'aotriton_amd', 'flash.h')])
-    if not force and os.path.exists(HOST_LIB) and os.path.getmtime(HOST_LIB) >= newest:
-        return HOST_LIB
     import sysconfig
     import torch
+    if not force and _host_is_current(str(torch.__version__)):
+        return HOST_LIB
     from torch.utils import cpp_extension
     includes = cpp_extension.include_paths('cuda') + [sysconfig.get_paths()['include'], os.path.join(ROOT, 'include')]
     torch_lib = os.path.join(os.path.dirname(torch.__file__), 'lib')
     cmd = ['g++', '-O2', '-std=c++17', '-fPIC', '-shared', '-fvisibility=hidden', '-D__HIP_PLATFORM_AMD__=1', '-DUSE_ROCM=1',
-           f'-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}', '-Wno-deprecated-declarations',
+           f'-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}', f'-DFA_TORCH_VERSION="{torch.__version__}"', '-Wno-deprecated-declarations',
            *[x for i in includes for x in ('-isystem', i)], HOST_SRC, '-o', HOST_LIB,
            '-L' + HERE, '-laotriton_amd', '-Wl,-rpath,$ORIGIN', '-L' + torch_lib, '-ltorch_python', '-ltorch', '-ltorch_cpu',
            '-ltorch_hip', '-lc10_hip', '-lc10']
@@ -105,6 +116,9 @@ def build_host(force=False):
     if r.returncode != 0:
         sys.stderr.write(r.stderr)
         raise RuntimeError('g++ failed on ' + HOST_SRC)
+    os.makedirs(OBJ, exist_ok=True)
+    with open(HOST_STAMP, 'w') as f:
+        f.write(torch.__version__)
     return HOST_LIB
 
 

@@ -905,4 +905,8 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_torch_host", nullptr, -1, kMetho
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__torch_host(void) { return PyModule_Create(&kModule); }
+PyMODINIT_FUNC PyInit__torch_host(void) {
+  PyObject* m = PyModule_Create(&kModule);
+  if (m != nullptr && PyModule_AddStringConstant(m, "torch_version", FA_TORCH_VERSION) != 0) Py_CLEAR(m);
+  return m;
+}

@@ -95,3 +95,28 @@ def test_flash_imports_without_torch_or_the_extension(blocked):
 def test_a_missing_extension_is_reported_with_the_way_to_build_it(use):
     r = _in_a_new_interpreter('aotriton_amd._torch_host', f'import {use}')
     assert r.returncode != 0 and 'ImportError' in r.stderr and 'python -m aotriton_amd.build' in r.stderr
+
+
+def test_the_extension_is_rebuilt_for_another_torch(tmp_path, monkeypatch):
+    from aotriton_amd import build
+    ran = []
+    monkeypatch.setattr(build, 'OBJ', str(tmp_path))
+    monkeypatch.setattr(build, 'HOST_LIB', str(tmp_path / 'ext.so'))
+    monkeypatch.setattr(build, 'HOST_STAMP', str(tmp_path / 'ext.torch'), raising=False)
+    monkeypatch.setattr(build.subprocess, 'run', lambda cmd, **kw: ran.append(cmd) or subprocess.CompletedProcess(cmd, 0))
+    (tmp_path / 'ext.so').touch()      # newer than the sources, built for nobody knows which torch
+    build.build_host()
+    assert len(ran) == 1
+    build.build_host()
+    assert len(ran) == 1
+    monkeypatch.setattr(torch, '__version__', '0.0.0')
+    build.build_host()
+    assert len(ran) == 2
+
+
+def test_an_extension_built_for_another_torch_is_refused(monkeypatch):
+    from aotriton_amd import _host
+    _host.load()
+    monkeypatch.setattr(torch, '__version__', '0.0.0')
+    with pytest.raises(ImportError, match='python -m aotriton_amd.build'):
+        _host.load()
