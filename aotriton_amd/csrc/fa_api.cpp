@@ -803,11 +803,15 @@ int fa_query_fwd_config(const fa_fwd_params* params, int32_t num_cu, fa_kernel_c
   // the vector-ALU kernels (3-D grid), the fp32 kernels and the split-head-dim kernels (above 256)
   const bool valu = params->Q.dtype == FA_DTYPE_FLOAT32 || s.d > 256 || s.elementwise;
   const bool rows32 = !s.elementwise && params->Q.dtype == FA_DTYPE_FLOAT32 && f32_rows(s, false, num_cu > 0 ? num_cu : 256);
+  const int cus = num_cu > 0 ? num_cu : 256;
+  const FwdPlan plan = fwd_plan(params->Q.dtype, s, params->causal_type, params->window_left, params->window_right, cus);
+  const bool split = !plan.rows && plan.splits > 1;
+  const bool half = !split && fwd_half_tiles(params->Q.dtype, s, cus);
   const fa::TileShape t = s.elementwise ? fa::TileShape{32, 1, 4, 0}
                           : rows32 ? fa::f32_rows_tile_shape(s.d)
                           : params->Q.dtype == FA_DTYPE_FLOAT32 ? fa::f32_tile_shape(s.d, -1)
                           : s.d > 256 ? fa::d512_tile_shape(-1)
-                                      : fa::fwd_tile_shape(params->Q.dtype, s.d, s.windowed);
+                                      : fa::fwd_tile_shape(params->Q.dtype, s.d, s.windowed, half);
   out->block_m = t.block_m; out->block_n = t.block_n; out->num_waves = t.num_waves;
   out->lds_bytes = t.lds_bytes;
   if (valu) {
@@ -824,21 +828,18 @@ int fa_query_fwd_config(const fa_fwd_params* params, int32_t num_cu, fa_kernel_c
     }
   } else {
     const int nz = s.num_seqlens != 0 ? std::abs(s.num_seqlens) : s.batch;
-    const int zh_per_xcd = (nz * s.hq + fa::kNumXcd - 1) / fa::kNumXcd;
-    const int ratio = s.hq / s.hk;
-    const int zg = ratio > 2 ? (ratio > 8 ? 8 : ratio) : 2;
-    const int groups = (zh_per_xcd + zg - 1) / zg;
-    // persistent workgroups: one per CU, at most one per Q tile
-    const int items = groups * zg * ((s.max_sq + t.block_m - 1) / t.block_m);
-    int workers = (num_cu > 0 ? num_cu : 256) / fa::kNumXcd;
-    workers = workers < 1 ? 1 : (workers > items ? items : workers);
-    out->grid[0] = fa::kNumXcd * workers;
+    const fa::TileWork w = fa::tile_work(nz * s.hq, fa::q_head_group(s.hq, s.hk),
+                                         (s.max_sq + t.block_m - 1) / t.block_m * (split ? plan.splits : 1));
+    out->grid[0] = fa::kNumXcd * fa::tile_workers(w.items_per_xcd, cus, t.per_cu);
     out->grid[1] = 1;
     out->grid[2] = 1;
   }
   out->backend_index = 0;
   out->head_dim = s.d;
   out->flags = (s.windowed ? 1 : 0) | (s.bias ? 2 : 0) | (s.dropout ? 4 : 0) | (s.num_seqlens != 0 ? 8 : 0);
+  // 64: the keys are split into parts, given scratch memory; 128: the packed-rows kernel takes the call (the tile and
+  // grid above are those of the tile kernel)
+  out->flags |= (plan.splits > 1 ? 64 : 0) | (plan.rows ? 128 : 0);
   // 32: fa_attn_fwd would run this call on packed copies in the workspace of the current device (the
   // tile and grid above are those of the element-wise kernels it runs on otherwise)
   int dev = 0;
@@ -864,24 +865,29 @@ int fa_query_bwd_config(const fa_bwd_params* params, const fa_options* options, 
                           : f32_mfma ? fa::f32_tile_shape(s.d, kernel_slot)
                           : split_d ? fa::d512_tile_shape(kernel_slot)
                           : valu  ? (kernel_slot == 1 ? fa::TileShape{1, 32, 4, 0} : fa::TileShape{32, 1, 4, 0})
-                                  : fa::bwd_tile_shape(params->Q.dtype, s.d, s.windowed, kernel_slot);
+                                  : fa::bwd_tile_shape(params->Q.dtype, s.d, s.windowed, s.bias, s.dropout, kernel_slot);
   const int nz = s.num_seqlens != 0 ? std::abs(s.num_seqlens) : s.batch;
   out->block_m = t.block_m; out->block_n = t.block_n; out->num_waves = t.num_waves;
   out->lds_bytes = t.lds_bytes;
   const int mt = (s.max_sq + t.block_m - 1) / t.block_m, nt = (s.max_sk + t.block_n - 1) / t.block_n;
-  // 1-D work lists of the main kernels: 8 XCDs x (heads per XCD, rounded up to whole groups) x
-  // items per head.  The fused kernel launches one workgroup per item, and so do dK/dV and dQ
-  // with a bias or at D = 256; otherwise they run persistent workgroups, one per CU (256 CUs assumed
-  // here) and at most one per item.
-  auto grid1d = [&](int heads, int zg, int items) {
-    const int per_xcd = (nz * heads + fa::kNumXcd - 1) / fa::kNumXcd;
-    return fa::kNumXcd * ((per_xcd + zg - 1) / zg) * zg * items;
-  };
-  auto persistent = [&](int items_total) {
-    const int per_xcd = items_total / fa::kNumXcd;
-    return s.bias || s.d >= 256 ? items_total : fa::kNumXcd * (per_xcd < 32 ? per_xcd : 32);
-  };
+  constexpr int kCus = 256;      // assumed here
   const int ratio = s.hq / s.hk;
+  // what of the workspace's uses the call gets (a host without a device: no limit unless one was set)
+  int ntq = 0, ntk = 0, dev = 0;
+  int64_t ds_bytes = 0, stat_bytes = 0, need = 0;
+  DkdvParts parts{1, 1, 0};
+  const bool have_dev = hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxDevices;
+  const int64_t set = g_ws_limit.load(std::memory_order_relaxed);
+  if (be == 0) {
+    need = ds_workspace_need(params, s, &ntq, &ntk, &ds_bytes, &stat_bytes);
+    parts = dkdv_parts(params, s, kCus);
+    fit_workspace(have_dev ? ws_limit_bytes(dev) : set >= 0 ? set : INT64_MAX, &need, &parts);
+  }
+  // 1-D work lists of the main kernels
+  auto workers = [&](int heads, int zg, int items) {
+    const fa::TileWork w = fa::tile_work(nz * heads, zg, items);
+    return fa::kNumXcd * fa::bwd_workers(s.d, s.bias, w.items_per_xcd, kCus, t.per_cu);
+  };
   out->grid[1] = 1;
   out->grid[2] = 1;
   if (rows32) {
@@ -895,27 +901,19 @@ int fa_query_bwd_config(const fa_bwd_params* params, const fa_options* options, 
     out->grid[2] = nz;
   } else switch (kernel_slot) {
     case 0: out->grid[0] = mt; out->grid[1] = s.hq; out->grid[2] = nz; break;
-    case 1: out->grid[0] = persistent(grid1d(s.hk, 2, nt)); break;
-    case 2: out->grid[0] = persistent(grid1d(s.hq, ratio > 2 ? (ratio > 8 ? 8 : ratio) : 2, mt)); break;
-    default: out->grid[0] = persistent(grid1d(s.hk, 2, nt + mt * ratio)); break;
+    case 1: out->grid[0] = workers(s.hk, 2, nt * parts.heads * parts.tiles); break;
+    case 2: out->grid[0] = workers(s.hq, fa::q_head_group(s.hq, s.hk), mt); break;
+    default: out->grid[0] = workers(s.hk, 2, nt + mt * ratio); break;
   }
   out->backend_index = be;
   out->head_dim = s.d;
   out->flags = (s.windowed ? 1 : 0) | (s.bias ? 2 : 0) | (s.dropout ? 4 : 0) | (s.num_seqlens != 0 ? 8 : 0);
   // 16: fa_attn_bwd would keep dS in HBM for this call on the current device (workspace within the
-  // limit; a call under stream capture recomputes all the same)
-  if (be == 0) {
-    int ntq = 0, ntk = 0, dev = 0;
-    int64_t ds_bytes = 0, stat_bytes = 0;
-    const int64_t need = ds_workspace_need(params, s, &ntq, &ntk, &ds_bytes, &stat_bytes);
-    if (need > 0 && hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxDevices && need <= ws_limit_bytes(dev))
-      out->flags |= 16;
-  }
+  // limit; a call under stream capture recomputes all the same); 64: it would cut the dK/dV items into parts
+  if (need > 0 && have_dev) out->flags |= 16;
+  if (parts.bytes > 0) out->flags |= 64;
   // 32: fa_attn_bwd would run this call on packed copies in the workspace
-  int dev = 0;
-  if (s.elementwise && hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxDevices &&
-      (int64_t)bwd_copies_bytes(params) <= ws_limit_bytes(dev))
-    out->flags |= 32;
+  if (s.elementwise && have_dev && (int64_t)bwd_copies_bytes(params) <= ws_limit_bytes(dev)) out->flags |= 32;
   return FA_SUCCESS;
 }
 
@@ -997,10 +995,6 @@ static int attn_fwd_impl(const fa_fwd_params* p, int32_t params_version, void* h
   a.atomic_counter = static_cast<int32_t*>(p->persistent_atomic_counter.ptr);
   a.num_cu = dev->num_cu;
 
-  const fa::TileShape t = (p->Q.dtype == FA_DTYPE_FLOAT32 || s.d > 256 || s.elementwise) ? fa::TileShape{32, 1, 4, 0} : fa::fwd_tile_shape(p->Q.dtype, s.d, s.windowed);
-  FA_LOG(4, "attn_fwd: D=%d BLOCK_M=%d BLOCK_N=%d waves=%d lds=%d windowed=%d bias=%d dropout=%d nseq=%d",
-         s.d, t.block_m, t.block_n, t.num_waves, t.lds_bytes, (int)s.windowed, (int)s.bias,
-         (int)s.dropout, s.num_seqlens);
   hipError_t err;
   const FwdPlan plan = fwd_plan(p->Q.dtype, s, p->causal_type, p->window_left, p->window_right, dev->num_cu);
   void* scratch = nullptr;
@@ -1019,6 +1013,8 @@ static int attn_fwd_impl(const fa_fwd_params* p, int32_t params_version, void* h
   }
   a.splits = scratch != nullptr ? plan.splits : 1;
   if (a.splits <= 1 && !plan.rows) a.half_tiles = fwd_half_tiles(p->Q.dtype, s, dev->num_cu);
+  FA_LOG(4, "attn_fwd: D=%d windowed=%d bias=%d dropout=%d nseq=%d rows=%d splits=%d half_tiles=%d", s.d, (int)s.windowed,
+         (int)s.bias, (int)s.dropout, s.num_seqlens, (int)plan.rows, a.splits, a.half_tiles);
   if (plan.rows) {
     a.row_blocks = plan.row_blocks; a.part_rows = plan.part_rows;
     err = run_fwd_rows(p->Q.dtype, s.d, a, s, stream);

@@ -7,6 +7,38 @@ namespace fa {
 
 constexpr int kNumXcd = 8;   // MI355X: 8 XCDs x 32 CUs, one L2 each
 
+// The 1-D work list of a kernel over the tiles of (batch element or sequence, head) pairs: each XCD owns a
+// contiguous range of pairs and walks them `zh_group` at a time.  Launchers and fa_query_*_config form it here.
+struct TileWork {
+  int32_t num_zh, zh_per_xcd, zh_group, items_per_xcd;   // items: incl. the padding of the last group
+};
+inline TileWork tile_work(int num_zh, int zh_group, int items_per_pair) {
+  TileWork w{num_zh, (num_zh + kNumXcd - 1) / kNumXcd, zh_group, 0};
+  w.items_per_xcd = (w.zh_per_xcd + zh_group - 1) / zh_group * zh_group * items_per_pair;
+  return w;
+}
+// pairs walked together by the kernels over q-heads (the q-heads of a GQA group share K and V)
+inline int q_head_group(int hq, int hk) {
+  const int ratio = hq / hk;
+  return ratio > 2 ? (ratio > 8 ? 8 : ratio) : 2;
+}
+// persistent workgroups per XCD: `per_cu` per CU, at most one per item
+inline int tile_workers(int items_per_xcd, int num_cu, int per_cu) {
+  int w = num_cu / kNumXcd * per_cu;
+  if (w < 1) w = 1;
+  return w > items_per_xcd ? items_per_xcd : w;
+}
+
+// Workgroups per XCD of the dK/dV and dQ kernels: one per CU (two: kTwoWaves), at most one per item.  With a
+// bias the kernels get one workgroup per item instead (the loop of a workgroup then runs
+// once): measured at B2 H16 S8192 D256 with window, bias, dB and dropout the persistent
+// grid was 10 % slower, while it gains 1 % at the headline shape and 12 % on packed
+// sequences of very different lengths.  D = 256 also gets one workgroup per item: its
+// dK/dV kernel has no register to spare for the loop.
+inline int bwd_workers(int head_dim, bool bias, int items_per_xcd, int num_cu, int per_cu) {
+  return bias || head_dim >= 256 ? items_per_xcd : tile_workers(items_per_xcd, num_cu > 0 ? num_cu : 256, per_cu);
+}
+
 struct Strides3 {   // batch, head, row
   int64_t z, h, s;
 };

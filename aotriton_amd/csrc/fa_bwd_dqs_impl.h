@@ -268,10 +268,7 @@ hipError_t launch_bwd_dqs(const BwdArgs& a0, hipStream_t stream) {
   constexpr int BN = D >= 256 ? 32 : 64;
   BwdArgs a = a0;
   a.num_m_tiles = (a.seq.max_seqlen_q + 255) / 256;
-  a.num_zh = bwd_nseq(a) * a.hq;
-  a.zh_per_xcd = (a.num_zh + kNumXcd - 1) / kNumXcd;
-  a.zh_group = a.hq / a.hk > 2 ? (a.hq / a.hk > 8 ? 8 : a.hq / a.hk) : 2;
-  a.items_per_xcd = ((a.zh_per_xcd + a.zh_group - 1) / a.zh_group) * a.zh_group * a.num_m_tiles;
+  set_work(a, tile_work(bwd_nseq(a) * a.hq, q_head_group(a.hq, a.hk), a.num_m_tiles));
   dim3 grid((unsigned)(kNumXcd * a.items_per_xcd));
   constexpr int lds = DqsSmem<D, BN>::BYTES;
   const bool db = a.db != nullptr;

@@ -117,6 +117,9 @@ template <typename T, int D, bool kWindowed, bool kBias, bool kDropout>
 constexpr int kDkDvBM = kWide<D, kBias, kDropout> ? 128 : BwdTile<T, D, kWindowed>::DKDV_BM;
 template <typename T, int D, bool kWindowed, bool kBias>
 constexpr int kDqBN = D == 64 && kBias ? 128 : BwdTile<T, D, kWindowed>::DQ_BN;
+// the single-launch kernel runs one wave per SIMD, hence the wide steps at head dim 64
+template <typename T, int D, bool W> constexpr int kFusedBM = D == 64 ? 128 : BwdTile<T, D, W>::DKDV_BM;
+template <typename T, int D, bool W> constexpr int kFusedBN = D == 64 ? 128 : BwdTile<T, D, W>::DQ_BN;
 
 // Two workgroups per CU, two waves per SIMD (256 registers each)?
 template <int D, bool kBias> constexpr bool kTwoWaves = D == 64 && !kBias;
@@ -1524,18 +1527,8 @@ inline int bwd_nseq(const BwdArgs& a) {
   return a.seq.num_seqlens != 0 ? (a.seq.num_seqlens < 0 ? -a.seq.num_seqlens : a.seq.num_seqlens) : a.batch;
 }
 
-// Workgroups per XCD of the dK/dV and dQ kernels: one per CU, at most one per item.  With a
-// bias the kernels get one workgroup per item instead (the loop of a workgroup then runs
-// once): measured at B2 H16 S8192 D256 with window, bias, dB and dropout the persistent
-// grid was 10 % slower, while it gains 1 % at the headline shape and 12 % on packed
-// sequences of very different lengths.  D = 256 also gets one workgroup per item: its
-// dK/dV kernel has no register to spare for the loop.
-template <int D>
-inline int persistent_workers(const BwdArgs& a, int per_cu) {
-  if (a.bias != nullptr || D >= 256) return a.items_per_xcd;
-  int w = (a.num_cu > 0 ? a.num_cu : 256) / kNumXcd * per_cu;
-  if (w < 1) w = 1;
-  return w > a.items_per_xcd ? a.items_per_xcd : w;
+inline void set_work(BwdArgs& a, const TileWork& w) {
+  a.num_zh = w.num_zh; a.zh_per_xcd = w.zh_per_xcd; a.zh_group = w.zh_group; a.items_per_xcd = w.items_per_xcd;
 }
 
 template <auto kern>
@@ -1609,12 +1602,8 @@ hipError_t launch_dkdv_variant(const BwdArgs& a0, hipStream_t stream) {
   constexpr int NW = Tile::NW, BM = kDkDvBM<T, D, W, B, P>, BN = NW * 32;
   BwdArgs a = a0;
   a.num_n_tiles = (a.seq.max_seqlen_k + BN - 1) / BN;
-  a.num_zh = bwd_nseq(a) * a.hk;
-  a.zh_per_xcd = (a.num_zh + kNumXcd - 1) / kNumXcd;
-  a.zh_group = 2;
-  a.items_per_xcd = ((a.zh_per_xcd + a.zh_group - 1) / a.zh_group) * a.zh_group * a.num_n_tiles *
-                    (kParts ? a.part_heads * a.part_tiles : 1);
-  dim3 grid((unsigned)(kNumXcd * persistent_workers<D>(a, kTwoWaves<D, B> ? 2 : 1)));
+  set_work(a, tile_work(bwd_nseq(a) * a.hk, 2, a.num_n_tiles * (kParts ? a.part_heads * a.part_tiles : 1)));
+  dim3 grid((unsigned)(kNumXcd * bwd_workers(D, B, a.items_per_xcd, a.num_cu, kTwoWaves<D, B> ? 2 : 1)));
   // (the level table's LDS is requested whether or not this launch uses it: the kernel's limit is set once)
   constexpr int smem = DkDvSmem<D, BM>::BYTES + (D < 256 ? kLevelBytes : 0);
   // (every build has the variant that stores dS; the host decides where it pays)
@@ -1644,11 +1633,8 @@ hipError_t launch_dq_variant(const BwdArgs& a0, hipStream_t stream) {
   constexpr int NW = Tile::NW, BN = kDqBN<T, D, W, B>, BM = NW * 32;
   BwdArgs a = a0;
   a.num_m_tiles = (a.seq.max_seqlen_q + BM - 1) / BM;
-  a.num_zh = bwd_nseq(a) * a.hq;
-  a.zh_per_xcd = (a.num_zh + kNumXcd - 1) / kNumXcd;
-  a.zh_group = a.hq / a.hk > 2 ? (a.hq / a.hk > 8 ? 8 : a.hq / a.hk) : 2;
-  a.items_per_xcd = ((a.zh_per_xcd + a.zh_group - 1) / a.zh_group) * a.zh_group * a.num_m_tiles;
-  dim3 grid((unsigned)(kNumXcd * persistent_workers<D>(a, kTwoWaves<D, B> ? 2 : 1)));
+  set_work(a, tile_work(bwd_nseq(a) * a.hq, q_head_group(a.hq, a.hk), a.num_m_tiles));
+  dim3 grid((unsigned)(kNumXcd * bwd_workers(D, B, a.items_per_xcd, a.num_cu, kTwoWaves<D, B> ? 2 : 1)));
   return launch_with_lds<bwd_dq_kernel<T, D, NW, BN, W, B, P, kPad>>(grid, NW * 64, DqSmem<D, BN>::BYTES, stream, a);
 }
 
@@ -1670,18 +1656,13 @@ hipError_t launch_bwd_dq(const BwdArgs& a0, bool windowed, bool bias, bool dropo
 template <typename T, int D, int kPad, bool W, bool B, bool P>
 hipError_t launch_fused_variant(const BwdArgs& a0, hipStream_t stream) {
   using Tile = BwdTile<T, D, W>;
-  // (one wave per SIMD, hence the wide steps at head dim 64)
-  constexpr int NW = Tile::NW, BM = D == 64 ? 128 : Tile::DKDV_BM, BN = D == 64 ? 128 : Tile::DQ_BN;
+  constexpr int NW = Tile::NW, BM = kFusedBM<T, D, W>, BN = kFusedBN<T, D, W>;
   constexpr int smem = DkDvSmem<D, BM>::BYTES > DqSmem<D, BN>::BYTES ? DkDvSmem<D, BM>::BYTES : DqSmem<D, BN>::BYTES;
   BwdArgs a = a0;
   a.num_n_tiles = (a.seq.max_seqlen_k + NW * 32 - 1) / (NW * 32);
   a.num_m_tiles = (a.seq.max_seqlen_q + NW * 32 - 1) / (NW * 32);
-  a.num_zh = bwd_nseq(a) * a.hk;
-  a.zh_per_xcd = (a.num_zh + kNumXcd - 1) / kNumXcd;
-  a.zh_group = 2;
-  const int items = a.num_n_tiles + a.num_m_tiles * (a.hq / a.hk);
-  a.items_per_xcd = ((a.zh_per_xcd + a.zh_group - 1) / a.zh_group) * a.zh_group * items;
-  dim3 grid((unsigned)(kNumXcd * persistent_workers<D>(a, 1)));
+  set_work(a, tile_work(bwd_nseq(a) * a.hk, 2, a.num_n_tiles + a.num_m_tiles * (a.hq / a.hk)));
+  dim3 grid((unsigned)(kNumXcd * bwd_workers(D, B, a.items_per_xcd, a.num_cu, 1)));
   return launch_with_lds<bwd_fused_kernel<T, D, NW, BM, BN, W, B, P, kPad>>(grid, NW * 64, smem, stream, a);
 }
 
@@ -1692,15 +1673,17 @@ hipError_t launch_bwd_fused(const BwdArgs& a0, bool windowed, bool bias, bool dr
 #undef FA_CALL
 }
 
-template <typename T, int D, bool kWindowed> TileShape bwd_shape(int slot) {
-  using Tile = BwdTile<T, D, kWindowed>;
-  constexpr int NW = Tile::NW, BM = Tile::DKDV_BM, BN = Tile::DQ_BN;
-  constexpr int s1 = DkDvSmem<D, BM>::BYTES, s2 = DqSmem<D, BN>::BYTES;
+// the tile of a kernel slot, as the launchers above choose it
+template <typename T, int D, bool W, bool B, bool P> TileShape bwd_shape(int slot) {
+  constexpr int NW = BwdTile<T, D, W>::NW, BM = kDkDvBM<T, D, W, B, P>, BN = kDqBN<T, D, W, B>;
+  constexpr int FM = kFusedBM<T, D, W>, FN = kFusedBN<T, D, W>, per_cu = kTwoWaves<D, B> ? 2 : 1;
   switch (slot) {
     case 0: return TileShape{256 / (D / 8), 0, 4, 0};
-    case 1: return TileShape{BM, NW * 32, NW, s1 + (D < 256 ? kLevelBytes : 0)};
-    case 2: return TileShape{NW * 32, BN, NW, s2};
-    default: return TileShape{NW * 32, NW * 32, NW, s1 > s2 ? s1 : s2};
+    case 1: return TileShape{BM, NW * 32, NW, DkDvSmem<D, BM>::BYTES + (D < 256 ? kLevelBytes : 0), per_cu};
+    case 2: return TileShape{NW * 32, BN, NW, DqSmem<D, BN>::BYTES, per_cu};
+    default:
+      return TileShape{NW * 32, NW * 32, NW,
+                       DkDvSmem<D, FM>::BYTES > DqSmem<D, FN>::BYTES ? DkDvSmem<D, FM>::BYTES : DqSmem<D, FN>::BYTES};
   }
 }
 

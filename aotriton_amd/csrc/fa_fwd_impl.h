@@ -742,17 +742,11 @@ hipError_t launch_fwd(const FwdArgs& a, bool windowed, bool bias, bool dropout, 
                                           : a.batch;
   FwdArgs b = a;
   b.num_m_tiles = (a.seq.max_seqlen_q + BM - 1) / BM;
-  b.num_zh = nseq * a.hq;
-  b.zh_per_xcd = (b.num_zh + kNumXcd - 1) / kNumXcd;
-  b.zh_group = a.hq / a.hk > 2 ? (a.hq / a.hk > 8 ? 8 : a.hq / a.hk) : 2;
-  const int groups = (b.zh_per_xcd + b.zh_group - 1) / b.zh_group;
   // (with splits, an item is one part of the keys of a tile; only without dropout, at D <= 128)
   const bool split = a.splits > 1;
-  b.items_per_xcd = groups * b.zh_group * b.num_m_tiles * (split ? a.splits : 1);
-  int workers = a.num_cu / kNumXcd * (half ? 2 : 1);          // one workgroup per CU, or two
-  if (workers < 1) workers = 1;
-  if (workers > b.items_per_xcd) workers = b.items_per_xcd;
-  dim3 grid((unsigned)(kNumXcd * workers));
+  const TileWork w = tile_work(nseq * a.hq, q_head_group(a.hq, a.hk), b.num_m_tiles * (split ? a.splits : 1));
+  b.num_zh = w.num_zh; b.zh_per_xcd = w.zh_per_xcd; b.zh_group = w.zh_group; b.items_per_xcd = w.items_per_xcd;
+  dim3 grid((unsigned)(kNumXcd * tile_workers(w.items_per_xcd, a.num_cu, half ? 2 : 1)));      // one workgroup per CU, or two
   if constexpr (D <= 128) {
     if (split) {
       b.part_group = 1; b.part_block = BM; b.part_rows = BM; b.row_blocks = b.num_m_tiles;

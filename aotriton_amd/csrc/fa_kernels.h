@@ -8,7 +8,7 @@ namespace fa {
 
 constexpr int kDtypeF32 = 1, kDtypeF16 = 2, kDtypeBF16 = 3;
 
-struct TileShape { int block_m, block_n, num_waves, lds_bytes; };
+struct TileShape { int block_m, block_n, num_waves, lds_bytes, per_cu = 1; };   // per_cu: persistent workgroups per CU
 
 hipError_t run_fwd_d64(int dtype, const FwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
 hipError_t run_fwd_d128(int dtype, const FwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
@@ -28,8 +28,8 @@ hipError_t run_fwd_rows_d256(int dtype, const FwdArgs& a, bool windowed, bool bi
 hipError_t run_fwd_rows_d64_padded(int dtype, const FwdArgs& a, bool windowed, bool bias, hipStream_t s);
 hipError_t run_fwd_rows_d128_padded(int dtype, const FwdArgs& a, bool windowed, bool bias, hipStream_t s);
 hipError_t run_fwd_rows_d256_padded(int dtype, const FwdArgs& a, bool windowed, bool bias, hipStream_t s);
-// tile table lookups: (element type, head dim, causal / windowed)
-TileShape fwd_tile_shape(int dtype, int head_dim, bool windowed);
+// tile table lookups: (element type, head dim, causal / windowed) and the variant
+TileShape fwd_tile_shape(int dtype, int head_dim, bool windowed, bool half_tiles);
 
 hipError_t run_encoded_softmax(const EncodedSoftmaxArgs& a, hipStream_t s);
 // strided -> packed (unpack false) or packed -> strided (unpack true); elem_bytes 2 or 4
@@ -46,7 +46,7 @@ hipError_t run_bwd_dkdv(int dtype, int head_dim, const BwdArgs& a, bool windowed
 hipError_t run_bwd_dkdv_parts(int dtype, int head_dim, const BwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
 hipError_t run_bwd_dq(int dtype, int head_dim, const BwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
 hipError_t run_bwd_fused(int dtype, int head_dim, const BwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
-TileShape bwd_tile_shape(int dtype, int head_dim, bool windowed, int kernel_slot);
+TileShape bwd_tile_shape(int dtype, int head_dim, bool windowed, bool bias, bool dropout, int kernel_slot);
 // dQ = dS K from the dS tiles that the dK/dV kernel stored (BwdArgs::ds_ws), and their geometry
 hipError_t run_bwd_dqs(int dtype, int head_dim, const BwdArgs& a, hipStream_t s);
 void ds_tile_counts(int dtype, int head_dim, bool bias, bool dropout, int max_sq, int max_sk, int* ntq, int* ntk, int64_t* tile_bytes);

@@ -1,39 +1,51 @@
-// Compile-time tile/occupancy table keyed on (element type, head dim, causal / windowed), reported
-// through fa_query_*_config.
+// Compile-time tile/occupancy table keyed on (element type, head dim, causal / windowed) and, where a kernel's
+// variants differ, on the options; reported through fa_query_*_config.
 #include "fa_fwd_impl.h"
 #include "fa_bwd_impl.h"
 #include "fa_kernels.h"
 
 namespace fa {
 
-template <typename T, int D, bool W> static TileShape fwd_shape() {
-  using Tile = FwdTile<T, D, W>;
-  return TileShape{Tile::BM, Tile::BN, Tile::NW, Tile::LDS};
+template <typename T, int D> static TileShape fwd_shape_of(bool windowed, bool half) {
+  auto shape = [](auto tile, int per_cu) {
+    using Tile = decltype(tile);
+    return TileShape{Tile::BM, Tile::BN, Tile::NW, Tile::LDS, per_cu};
+  };
+  if constexpr (D <= 128) {
+    if (half) return shape(FwdHalfTile<D>{}, 2);
+  }
+  return windowed ? shape(FwdTile<T, D, true>{}, 1) : shape(FwdTile<T, D, false>{}, 1);
 }
 
-template <typename T> static TileShape fwd_shape_of(int head_dim, bool windowed) {
-  switch (head_dim) {
-    case 64: return windowed ? fwd_shape<T, 64, true>() : fwd_shape<T, 64, false>();
-    case 128: return windowed ? fwd_shape<T, 128, true>() : fwd_shape<T, 128, false>();
-    default: return windowed ? fwd_shape<T, 256, true>() : fwd_shape<T, 256, false>();
+template <typename T, int D> static TileShape bwd_shape_of(bool windowed, bool bias, bool dropout, int slot) {
+  switch ((windowed ? 4 : 0) | (bias ? 2 : 0) | (dropout ? 1 : 0)) {
+    case 0: return bwd_shape<T, D, false, false, false>(slot);
+    case 1: return bwd_shape<T, D, false, false, true>(slot);
+    case 2: return bwd_shape<T, D, false, true, false>(slot);
+    case 3: return bwd_shape<T, D, false, true, true>(slot);
+    case 4: return bwd_shape<T, D, true, false, false>(slot);
+    case 5: return bwd_shape<T, D, true, false, true>(slot);
+    case 6: return bwd_shape<T, D, true, true, false>(slot);
+    default: return bwd_shape<T, D, true, true, true>(slot);
   }
 }
 
-TileShape fwd_tile_shape(int dtype, int head_dim, bool windowed) {
-  return dtype == kDtypeBF16 ? fwd_shape_of<bf16_t>(head_dim, windowed) : fwd_shape_of<f16_t>(head_dim, windowed);
-}
-
-template <typename T> static TileShape bwd_shape_of(int head_dim, bool windowed, int slot) {
+TileShape fwd_tile_shape(int dtype, int head_dim, bool windowed, bool half_tiles) {
+  const bool bf = dtype == kDtypeBF16;
   switch (head_dim) {
-    case 64: return windowed ? bwd_shape<T, 64, true>(slot) : bwd_shape<T, 64, false>(slot);
-    case 128: return windowed ? bwd_shape<T, 128, true>(slot) : bwd_shape<T, 128, false>(slot);
-    default: return windowed ? bwd_shape<T, 256, true>(slot) : bwd_shape<T, 256, false>(slot);
+    case 64: return bf ? fwd_shape_of<bf16_t, 64>(windowed, half_tiles) : fwd_shape_of<f16_t, 64>(windowed, half_tiles);
+    case 128: return bf ? fwd_shape_of<bf16_t, 128>(windowed, half_tiles) : fwd_shape_of<f16_t, 128>(windowed, half_tiles);
+    default: return bf ? fwd_shape_of<bf16_t, 256>(windowed, half_tiles) : fwd_shape_of<f16_t, 256>(windowed, half_tiles);
   }
 }
 
-TileShape bwd_tile_shape(int dtype, int head_dim, bool windowed, int kernel_slot) {
-  return dtype == kDtypeBF16 ? bwd_shape_of<bf16_t>(head_dim, windowed, kernel_slot)
-                             : bwd_shape_of<f16_t>(head_dim, windowed, kernel_slot);
+TileShape bwd_tile_shape(int dtype, int head_dim, bool windowed, bool bias, bool dropout, int slot) {
+  const bool bf = dtype == kDtypeBF16;
+  switch (head_dim) {
+    case 64: return bf ? bwd_shape_of<bf16_t, 64>(windowed, bias, dropout, slot) : bwd_shape_of<f16_t, 64>(windowed, bias, dropout, slot);
+    case 128: return bf ? bwd_shape_of<bf16_t, 128>(windowed, bias, dropout, slot) : bwd_shape_of<f16_t, 128>(windowed, bias, dropout, slot);
+    default: return bf ? bwd_shape_of<bf16_t, 256>(windowed, bias, dropout, slot) : bwd_shape_of<f16_t, 256>(windowed, bias, dropout, slot);
+  }
 }
 
 }  // namespace fa

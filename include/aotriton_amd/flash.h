@@ -205,7 +205,10 @@ typedef struct fa_kernel_config {
   int32_t grid[3];
   int32_t backend_index;
   int32_t head_dim;
-  int32_t flags; /* bit0 causal/windowed, bit1 bias, bit2 dropout, bit3 varlen, bit4 (backward) dS kept in HBM, bit5 runs on packed copies */
+  /* bit0 causal/windowed, bit1 bias, bit2 dropout, bit3 varlen, bit4 (backward) dS kept in HBM, bit5 runs on packed
+   * copies, bit6 work cut into parts whose fp32 sums a second kernel adds up (forward: the keys; backward: the dK/dV
+   * items), bit7 (forward) few query rows: the packed-rows kernel */
+  int32_t flags;
 } fa_kernel_config;
 
 /* The MFMA kernels read rows made of aligned 16-byte pieces; the test is the same for every element
@@ -370,7 +373,11 @@ FA_API int fa_validate_bwd(const fa_bwd_params* params, int32_t params_version,
                            const fa_options* options);
 
 /* Tile/grid the library would use (host only, num_cu = CU count to assume; the backward
- * query assumes 256 CUs). */
+ * query assumes 256 CUs).  The grid counts parts (bit 6), which the forward has when it gets scratch memory
+ * (fa_attn_fwd_alloc, or the workspace).  Where bit 5 or bit 7 of `flags` is set the call runs elsewhere, and tile
+ * and grid are those of the kernel that it would run on otherwise: element-wise or tile kernel.  Backward
+ * slots: 0 delta, 1 dK/dV, 2 dQ that recomputes S and dP (with bit 4 set fa_attn_bwd forms dQ from the
+ * stored dS instead), 3 fused. */
 FA_API int fa_query_fwd_config(const fa_fwd_params* params, int32_t num_cu,
                                fa_kernel_config* out);
 FA_API int fa_query_bwd_config(const fa_bwd_params* params, const fa_options* options,

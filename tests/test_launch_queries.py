@@ -1,0 +1,93 @@
+"""fa_query_*_config reports the tile and grid of the kernel variant that a call runs on.  Host only: the views
+point nowhere and nothing is launched."""
+import pytest
+
+CAUSAL = (3, -2147483647, -2147483647)
+
+
+def view(*sizes, name='kBFloat16'):
+    from aotriton_amd.pyaotriton import DType, T1, T2, T4
+    strides = [1]
+    for n in reversed(sizes[1:]):
+        strides.insert(0, strides[0] * n)
+    return {1: T1, 2: T2, 4: T4}[len(sizes)](4096, list(sizes), strides, getattr(DType, name))
+
+
+def fwd(B, Hq, Hk, Sq, Sk, D, causal=False, p=0.0, bias=False, num_cu=256):
+    from aotriton_amd.pyaotriton.v3.flash import attn_fwd_params, query_fwd_config
+    x = attn_fwd_params()
+    x.Q, x.K, x.V, x.Out = view(B, Hq, Sq, D), view(B, Hk, Sk, D), view(B, Hk, Sk, D), view(B, Hq, Sq, D)
+    _common(x, B, Hq, Sq, Sk, causal, p, bias)
+    err, c = query_fwd_config(x, num_cu)
+    assert int(err) == 0
+    return c
+
+
+def bwd(slot, B, Hq, Hk, Sq, Sk, D, causal=False, p=0.0, bias=False):
+    from aotriton_amd.pyaotriton.v3.flash import attn_bwd_params, query_bwd_config
+    from aotriton_amd.pyaotriton import lazy_tensor
+    x = attn_bwd_params()
+    x.Q = x.DQ = view(B, Hq, Sq, D)
+    x.Out = x.DO = view(B, Hq, Sq, D)
+    x.K = x.V = x.DK = x.DV = view(B, Hk, Sk, D)
+    x.L = view(B * Hq, Sq, name='kFloat32')
+    x.D = lazy_tensor.eager_delta(x.L)
+    _common(x, B, Hq, Sq, Sk, causal, p, bias)
+    err, c = query_bwd_config(x, slot)
+    assert int(err) == 0
+    return c
+
+
+def _common(x, B, Hq, Sq, Sk, causal, p, bias):
+    from aotriton_amd.pyaotriton import DType, T0
+    x.Sm_scale = 0.125
+    if bias:
+        x.B = view(B, Hq, Sq, Sk)
+    x.dropout_p = p
+    if p:
+        x.philox_seed_ptr = x.philox_offset1 = T0(4096, DType.kUInt64)
+    if causal:
+        x.causal_type, x.window_left, x.window_right = CAUSAL if causal is True else (3, *causal)
+
+
+def test_forward_variants():
+    full = fwd(4, 32, 32, 4096, 4096, 64)
+    assert (full.block_m, full.num_waves, full.grid[0], full.flags & 192) == (256, 8, 256, 0)
+    half = fwd(40, 16, 16, 128, 128, 64, p=0.1)                 # 128-row tiles, two workgroups per CU
+    assert (half.block_m, half.block_n, half.num_waves, half.grid[0]) == (128, 64, 4, 512)
+    assert half.lds_bytes < 80 * 1024
+    chunk = fwd(1, 32, 32, 1024, 16384, 128, causal=(-2147483646, -2147483646))      # tiles with their keys in parts
+    assert (chunk.block_m, chunk.grid[0], chunk.flags & 192) == (256, 256, 64)
+    few = fwd(1, 4, 4, 256, 8192, 128, p=0.0)
+    assert few.grid[0] > 8 * ((4 + 7) // 8) and few.flags & 64   # more workgroups than tiles
+    decode = fwd(1, 32, 8, 1, 4000, 128)
+    assert decode.flags & 192 == 192
+    assert fwd(1, 32, 8, 1, 4000, 128, p=0.1).flags & 192 == 0   # dropout stays on the tile kernel
+
+
+@pytest.mark.parametrize('slot, bias, p, tile, lds, grid', [
+    (1, False, 0.0, (64, 128), 72704, 512),
+    (1, False, 0.1, (64, 128), 72704, 512),
+    (1, True, 0.0, (128, 128), 141312, 2048),                    # one workgroup per item with a bias
+    (1, True, 0.1, (64, 128), 72704, 2048),
+    (2, False, 0.0, (128, 64), 51200, 512),
+    (2, True, 0.0, (128, 128), 100352, 2048),
+    (3, False, 0.0, (128, 128), 137216, 256),
+    (3, True, 0.1, (128, 128), 137216, 4096),
+])
+def test_backward_variants_at_head_dim_64(slot, bias, p, tile, lds, grid):
+    c = bwd(slot, 8, 16, 16, 2048, 2048, 64, bias=bias, p=p)
+    assert ((c.block_m, c.block_n), c.lds_bytes, c.grid[0]) == (tile, lds, grid)
+
+
+def test_backward_parts_are_counted():
+    whole, cut = bwd(1, 1, 8, 8, 64, 200, 128), bwd(1, 1, 8, 2, 1500, 200, 128)
+    assert whole.flags & 64 == 0 and whole.grid[0] == 8 * 4      # a pair of heads per XCD, two key tiles each
+    assert cut.flags & 64 and cut.grid[0] > 8 * 4
+    from aotriton_amd._lib import lib
+    lib.fa_set_bwd_workspace_limit(0)
+    try:
+        uncut = bwd(1, 1, 8, 2, 1500, 200, 128)
+        assert uncut.flags & 64 == 0 and uncut.grid[0] == 8 * 4
+    finally:
+        lib.fa_set_bwd_workspace_limit(-1)
