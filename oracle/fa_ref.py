@@ -46,7 +46,7 @@ def attn_fwd_ref(q, k, v, bias, sm_scale, causal_type=0, window_left=0,
     Sk = k.shape[2]
     kk = _expand_kv(k, Hq)
     vv = _expand_kv(v, Hq)
-    s = torch.matmul(q, kk.transpose(-1, -2)) * sm_scale
+    s = torch.matmul(q, kk.transpose(-1, -2).contiguous()) * sm_scale
     if bias is not None:
         s = s + bias
     vis = visible_mask(Sq, Sk, causal_type, window_left, window_right, q.device)
@@ -76,7 +76,7 @@ def attn_bwd_ref(q, k, v, bias, sm_scale, o, do, lse, causal_type=0,
     g = Hq // Hk
     kk = _expand_kv(k, Hq)
     vv = _expand_kv(v, Hq)
-    s = torch.matmul(q, kk.transpose(-1, -2)) * sm_scale
+    s = torch.matmul(q, kk.transpose(-1, -2).contiguous()) * sm_scale
     if bias is not None:
         s = s + bias
     vis = visible_mask(Sq, Sk, causal_type, window_left, window_right, q.device)
@@ -85,7 +85,7 @@ def attn_bwd_ref(q, k, v, bias, sm_scale, o, do, lse, causal_type=0,
     p = torch.where(vis, p, torch.zeros_like(p))
     p = torch.nan_to_num(p, nan=0.0)
     delta = (o * do).sum(dim=-1)                      # bwd_preprocess.py:28-133
-    dp = torch.matmul(do, vv.transpose(-1, -2))       # bwd_inner_dk_dv.py:231-236
+    dp = torch.matmul(do, vv.transpose(-1, -2).contiguous())     # bwd_inner_dk_dv.py:231-236
     if dropout_p > 0.0:
         scale = 1.0 / (1.0 - dropout_p)
         keepf = keep_mask.to(p.dtype)
@@ -128,7 +128,7 @@ def sdpa_math_ref(q, k, v, bias, sm_scale, causal_type=0, window_left=0,
 def lse_ref(q, k, bias, sm_scale, causal_type=0, window_left=0, window_right=0):
     """logsumexp of the masked scores (modules/flash/tune/sdpa_math.py:16-41)."""
     Hq = q.shape[1]
-    s = torch.matmul(q, _expand_kv(k, Hq).transpose(-1, -2)) * sm_scale
+    s = torch.matmul(q, _expand_kv(k, Hq).transpose(-1, -2).contiguous()) * sm_scale
     if bias is not None:
         s = s + bias
     vis = visible_mask(q.shape[2], k.shape[2], causal_type, window_left, window_right, q.device)
