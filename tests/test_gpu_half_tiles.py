@@ -17,6 +17,8 @@ CASES = [
     (16, 36, 36, 129, 33, 128, HF, False, 0.2),
     (40, 16, 16, 128, 97, 96, HF, True, 0.0),
     (40, 16, 16, 70, 128, 40, BF, False, 0.0),
+    (40, 16, 16, 70, 128, 40, BF, False, 0.1),        # (without dropout the rows kernel takes it)
+    (16, 36, 36, 290, 33, 128, HF, False, 0.2),       # 5 rounds against 4, a ragged third tile
 ]
 
 

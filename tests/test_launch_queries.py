@@ -91,3 +91,43 @@ def test_backward_parts_are_counted():
         assert uncut.flags & 64 == 0 and uncut.grid[0] == 8 * 4
     finally:
         lib.fa_set_bwd_workspace_limit(-1)
+
+
+def _name(case):
+    return '-'.join(str(x).replace('torch.', '') for x in case)
+
+
+# the cases of the GPU tests are cases of the kernels that those tests are about
+def test_cases_of_the_packed_rows_kernel():
+    from test_gpu_fwd_rows import BR, CASES
+    for B, Hq, Hk, Sq, Sk, D, _, causal, bias in CASES:
+        c = fwd(B, Hq, Hk, Sq, Sk, (D + 7) // 8 * 8, (-2147483646, -2147483646) if causal == BR else causal, 0.0, bias)
+        assert c.flags & 128, (B, Hq, Hk, Sq, Sk, D, causal)
+
+
+def test_cases_of_the_forward_tiles():
+    from test_gpu_fwd_tiles import SPLIT, TILES
+    seen = set()
+    for case in TILES + SPLIT:
+        B, Hq, Hk, Sq, Sk, D, _, causal, bias = case
+        c = fwd(B, Hq, Hk, Sq, Sk, D, causal, 0.0, bias is not None)
+        assert c.flags & 192 == (64 if case in SPLIT else 0), _name(case)
+        seen.add((c.head_dim, bool(causal), bias is not None, case in SPLIT, c.block_m if c.head_dim < 256 else 256))
+    for D in (64, 128):      # every variant without dropout, with whole and half tiles
+        for windowed in (False, True):
+            assert {(D, windowed, False, False, 256), (D, windowed, False, False, 128), (D, windowed, True, False, 256),
+                    (D, windowed, False, True, 256)} <= seen
+    assert {(256, False, False, False, 256), (256, True, False, False, 256)} <= seen
+
+
+def test_cases_of_the_half_tiles():
+    from test_gpu_half_tiles import CASES
+    half = [c for c in CASES if fwd(*c[:6], *c[7:]).flags & 192 == 0 and fwd(*c[:6], *c[7:]).block_m == 128]
+    assert len(half) == 7 and {(c[5] > 64, bool(c[7]), c[8] > 0) for c in half} >= {
+        (False, False, False), (False, True, True), (False, False, True), (True, True, False), (True, False, True)}
+
+
+def test_cases_of_the_backward_parts():
+    from test_gpu_bwd_parts import CASES
+    cut = [c for c in CASES if bwd(1, *c[:5], (c[5] + 7) // 8 * 8, *c[7:]).flags & 64]
+    assert len(cut) == len(CASES) - 1      # (the window of 60 and 30 leaves one step per key tile: uncut)
