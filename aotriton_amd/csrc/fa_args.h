@@ -95,7 +95,7 @@ struct FwdArgs {
   int32_t part_rows;     // rows stored per block
   int32_t part_group, part_block;
   float* part_o;         // columns: the compiled head dim
-  float* part_ml;        // reference maximum (log2) and row sum
+  float* part_ml;        // reference maximum (units of the scores) and row sum
 };
 
 struct BwdArgs {

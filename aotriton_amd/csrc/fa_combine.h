@@ -4,7 +4,7 @@
 
 namespace fa {
 
-// Sums the parts of a row: out = sum_i 2^(m_i - m) O_i / sum_i 2^(m_i - m) l_i, one wave per row.
+// Sums the parts of a row: out = sum_i 2^((m_i - m) sc) O_i / sum_i 2^((m_i - m) sc) l_i, one wave per row.
 // Parts lie as (pair, row block, part, row of the block): a pair is `part_group` q-heads of one
 // sequence, its rows are counted query * part_group + head and come in blocks of part_block.  What
 // bounds it is the latency of its loads: the statistics of all parts in one load, the sums eight parts
@@ -31,10 +31,11 @@ static __global__ __launch_bounds__(256) void combine_rows_kernel(const FwdArgs 
     const vec<float, 2> t = *reinterpret_cast<const vec<float, 2>*>(a.part_ml + (part + (int64_t)lane * a.part_rows) * 2);
     ms = t[0]; ls = t[1];
   }
+  const float sc = score_scale(a.sm_scale, a.bias != nullptr);
   float m = ms;
 #pragma unroll
   for (int d = 32; d >= 1; d /= 2) m = fmaxf(m, __shfl_xor(m, d));
-  const float f = ls != 0.f ? fast_exp2(ms - m) : 0.f;
+  const float f = ls != 0.f ? fast_exp2((ms - m) * sc) : 0.f;
   float lsum = f * ls;
 #pragma unroll
   for (int d = 32; d >= 1; d /= 2) lsum += __shfl_xor(lsum, d);
@@ -67,7 +68,7 @@ static __global__ __launch_bounds__(256) void combine_rows_kernel(const FwdArgs 
     for (int j = 0; j < PL; ++j) t[j] = Traits<T>::cvt(acc[j] * inv);
     *reinterpret_cast<vec<T, PL>*>(op) = t;
   }
-  if (a.lse && lane == 0) a.lse[lse_offset(si, ph, a.hq) + pq] = alive ? (m + fast_log2(lsum)) * kLn2 : __builtin_inff();
+  if (a.lse && lane == 0) a.lse[lse_offset(si, ph, a.hq) + pq] = lse_of(m, sc, lsum);
 }
 
 template <typename T, int D>

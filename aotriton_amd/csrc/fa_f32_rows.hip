@@ -316,7 +316,7 @@ __global__ __launch_bounds__(256) void fwd_f32_rows_kernel(const FwdArgs a) {
   const float l = cross_sum(l_i);
   put<D>(areas + wave * C::AREA, o, c, hi);
   if (hi == 0) {
-    ml[(wave * 32 + c) * 2] = m_i * sc;
+    ml[(wave * 32 + c) * 2] = m_i;
     ml[(wave * 32 + c) * 2 + 1] = l;
   }
   __syncthreads();
@@ -331,7 +331,7 @@ __global__ __launch_bounds__(256) void fwd_f32_rows_kernel(const FwdArgs a) {
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int v = 0; v < kWaves; ++v) {
-      const float f = fast_exp2(ml[(v * 32 + rr) * 2] - m);
+      const float f = fast_exp2((ml[(v * 32 + rr) * 2] - m) * sc);
       lsum += f * ml[(v * 32 + rr) * 2 + 1];
       acc += f * *reinterpret_cast<const f32x4*>(areas + v * C::AREA + rr * C::OSTR + col);
     }
@@ -340,7 +340,7 @@ __global__ __launch_bounds__(256) void fwd_f32_rows_kernel(const FwdArgs a) {
     if (kDropout) inv *= ds.scale;          // fwd_kernel.py:573-575
     if (col < a.head_dim_v) *reinterpret_cast<f32x4*>(out + (int64_t)rr * a.so.s + col) = acc * inv;
     if (a.lse && col == 0)
-      a.lse[lse_offset(si, h, a.hq) + q0 + rr] = alive ? (m + fast_log2(lsum)) * kLn2 : __builtin_inff();
+      a.lse[lse_offset(si, h, a.hq) + q0 + rr] = lse_of(m, sc, lsum);
   }
 }
 

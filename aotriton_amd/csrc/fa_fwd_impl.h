@@ -579,7 +579,7 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
           *reinterpret_cast<f32x4*>(a.part_o + part_row * D + 32 * db + 8 * g + 4 * hi) =
               f32x4{o[db][4 * g], o[db][4 * g + 1], o[db][4 * g + 2], o[db][4 * g + 3]};
       if (hi == 0) {
-        a.part_ml[part_row * 2] = m_i * sc;
+        a.part_ml[part_row * 2] = m_i;
         a.part_ml[part_row * 2 + 1] = l;
       }
     }

@@ -234,7 +234,7 @@ void fwd_rows_kernel(const FwdArgs a) {
         *reinterpret_cast<f32x4*>(ow + c * OSTR + 32 * db + 8 * g + 4 * hi) =
             f32x4{o[db][4 * g], o[db][4 * g + 1], o[db][4 * g + 2], o[db][4 * g + 3]};
     if (hi == 0) {
-      ml[(wave * 32 + c) * 2] = m_i * sc;      // (kNegBig where the wave saw no key of the row; l is 0 then)
+      ml[(wave * 32 + c) * 2] = m_i;      // (kNegBig where the wave saw no key of the row; l is 0 then)
       ml[(wave * 32 + c) * 2 + 1] = l;
     }
   }
@@ -249,7 +249,7 @@ void fwd_rows_kernel(const FwdArgs a) {
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int v = 0; v < kRowsWaves; ++v) {
-      const float f = fast_exp2(ml[(v * 32 + r) * 2] - m);
+      const float f = fast_exp2((ml[(v * 32 + r) * 2] - m) * sc);
       lsum += f * ml[(v * 32 + r) * 2 + 1];
       acc += f * *reinterpret_cast<const f32x4*>(smem_raw + v * SM::O_BYTES + (r * OSTR + col) * 4);
     }
@@ -270,7 +270,7 @@ void fwd_rows_kernel(const FwdArgs a) {
       *reinterpret_cast<q4_t*>(reinterpret_cast<T*>(a.out) + (int64_t)si.batch_index * a.so.z + (int64_t)ph * a.so.h +
                                (int64_t)(si.q_start + pq) * a.so.s + col) = t4;
       if (a.lse && col == 0)
-        a.lse[lse_offset(si, ph, a.hq) + pq] = alive ? (m + fast_log2(lsum)) * kLn2 : __builtin_inff();
+        a.lse[lse_offset(si, ph, a.hq) + pq] = lse_of(m, sc, lsum);
     }
   }
 }

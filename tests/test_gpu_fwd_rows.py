@@ -137,3 +137,21 @@ def test_split_forward_replays_from_a_hip_graph():
         torch.cuda.synchronize()
         assert torch.equal(captured, eager)
         assert torch.equal(run(), eager)
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float32])
+def test_logsumexp_where_waves_meet(dtype):
+    """L = (m sc + log2 l) ln 2 with m sc never rounded by itself.  For these rows m sc lies around 4.6 and the sum in
+    [8, 16): its rounding (2^-20 wide, rms 2.8e-7) times ln 2, that of the product (2^-21, 1.4e-7) and half as much
+    from the scores and the logarithm make 4.1e-8 of L; a rounded m sc (2^-21) makes it 4.5e-8."""
+    from aotriton_amd.autograd import attention, AttentionExtraArgs
+    B, Hq, Hk, Sk, D = 8, 32, 8, 700, 128
+    err, n = 0.0, 10
+    for seed in range(n):
+        g = torch.Generator(device=DEV).manual_seed(seed)
+        q, k = (torch.randn(B, h, s, D, device=DEV, generator=g).to(dtype) for h, s in ((Hq, 1), (Hk, Sk)))
+        _, _, L = attention(q, k, k, None, False, D ** -0.5, 0.0, AttentionExtraArgs(return_logsumexp=True))
+        kt = k.double().repeat_interleave(Hq // Hk, 1).transpose(-1, -2).contiguous()
+        want = torch.logsumexp(torch.matmul(q.double(), kt) * D ** -0.5, -1).reshape(L.shape)
+        err += ((L.double() - want).norm() / want.norm()).item() / n
+    assert err < 4.3e-8
