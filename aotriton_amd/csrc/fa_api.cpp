@@ -540,10 +540,14 @@ struct FwdPlan {
 // 256) with all CUs busy (a quarter less on an idle chip, whose clock is higher), one workgroup per
 // CU, and 6 us around that; the rows kernel takes four waves of 32 rows through 4 x 32 keys in
 // 0.9 / 1.2 / 2.6 us, two workgroups of a CU (one at D = 256) taking turns, and 4 us around that; a part's sums of 256 rows cost
-// 0.07 us of the whole chip's memory time at D = 128, the second launch 5 us.  Within 10-20 % of the
-// measured times at 24 shapes of 1-2048 queries and 64-30000 keys; the gains it decides on are larger
-// (one query, 2051 keys, Hq 32 / Hk 8: 56 -> 11 us; 32 sequences of 8190 keys: 833 -> 189; 80 queries,
-// 3216 keys: 85 -> 34; 1024 queries, 16384 keys: 398 -> 274).
+// 0.07 us of the whole chip's memory time at D = 128, the second launch 5 us.  Against 665 measured shapes of 1-2048
+// queries and 64-10000 keys (profiles/forward_routes.txt holds a third of them) the estimate of whole tiles is within
+// 25 % for 84 %, that of the rows kernel, which knows no HBM rate, for 63 %; the route taken is the best of
+// the three, or within a tenth of it, for 95 %.  One measured shape is more than 10 % slower than whole tiles on its
+// route (Hq 8, Hk 2, 512 causal, D = 256: 28 -> 33).  The gains it decides on are larger
+// (one query, 2051 keys, Hq 32 / Hk 8: 55 -> 11 us; 32 sequences of 8190 keys: 833 -> 189; 80 queries,
+// 3216 keys: 88 -> 35; 1024 queries, 16384 keys: 402 -> 266).  Tiles of 128 rows (fwd_half_tiles below) are not among
+// what is compared: they are asked about where this rule leaves the tiles whole.
 FwdPlan fwd_plan(int dtype, const Shape& s, int causal_type, int window_left, int window_right, int num_cu) {
   FwdPlan r{};
   r.splits = 1;
@@ -578,7 +582,8 @@ FwdPlan fwd_plan(int dtype, const Shape& s, int causal_type, int window_left, in
     return (even > longest ? even : longest) * t64 * (0.75 + 0.25 * busy) + 6 * rounds +
            (parts > 1 ? 5 + 0.07 * wide * tiles * parts : 0.0);
   };
-  double best = tile_time(1);
+  const double whole = tile_time(1);
+  double best = whole;
   if (s.d <= 128 && s.num_seqlens == 0)
     for (int64_t parts = 2; parts <= 16 && parts * 2 <= most; ++parts)
       if (const double t = tile_time(parts); t < 0.9 * best) { best = t; r.splits = (int)parts; }
@@ -594,11 +599,24 @@ FwdPlan fwd_plan(int dtype, const Shape& s, int causal_type, int window_left, in
   const double per_cu = s.d > 128 ? (double)row_rounds : (double)(items * splits) / num_cu;
   const double t128 = s.d == 64 ? 0.9 : s.d == 128 ? 1.2 : 2.6;
   const double rows_time = (per_cu > 1 ? per_cu : 1) * steps * t128 + 4 * (double)row_rounds + 1 + (splits > 1 ? 4 : 0);
-  r.rows = rows_time < best;
+  // The row blocks of a (pair, part) run on one XCD (fwd_rows_kernel), so with fewer than eight of those, or a few more
+  // than a multiple of eight, the busiest XCD has more than its share; with many row blocks that decides.  There the
+  // blocks take the average tile's keys, and the rows kernel is refused where that is slower than whole tiles (us, whole tiles
+  // / rows kernel, Hq 8 and Hk 2 unless said: 2048 queries and keys D128 57 / 157, causal 57 / 97; 1024 D256
+  // 44 / 112; 1024 D64 22 / 27; 600 x 900 D256 41 / 79, Hq = Hk = 12 41 / 55; kept: 1024 D64 causal 23 / 20, Hq = Hk = 2
+  // 2048 D128 55 / 32).
+  const int64_t cus = num_cu >= fa::kNumXcd ? num_cu / fa::kNumXcd : 1, row_blocks = (rows + 31) / 32;
+  const int64_t busiest = (nz * s.hk * splits + fa::kNumXcd - 1) / fa::kNumXcd * row_blocks;
+  const int64_t busy_rounds = (busiest + slots / num_cu * cus - 1) / (slots / num_cu * cus);
+  const double average = most > 0 ? (double)sum / ((double)most * m_tiles) : 1.0;
+  const double load = average * (s.d > 128 ? (double)busy_rounds : (double)busiest / cus);
+  const double busy_time = (load > 1 ? load : 1) * steps * t128 + 4 * (double)busy_rounds + 1 + (splits > 1 ? 4 : 0);
+  // (the lines: D = 128 and 256 level at 1.1 of these figures, D = 64, whose steps take 0.55 us on two XCDs, at 1.7)
+  r.rows = rows_time < best && busy_time <= (s.d == 64 ? 1.75 : 1.08) * whole;
   int64_t stored;
   if (r.rows) {
     r.splits = (int)splits;
-    r.row_blocks = (int)((rows + 31) / 32);
+    r.row_blocks = (int)row_blocks;
     r.part_rows = (int)(rows < 32 ? rows : 32);
     stored = items * splits * r.part_rows;
   } else {

@@ -70,20 +70,23 @@ def test_parts_give_way_to_the_stored_ds(D):
     from aotriton_amd.autograd import attention
     from aotriton_amd._lib import lib
     B, Hq, Hk, Sq, Sk = 1, 8, 2, 1500, 200
-    q, k, v, _, do = make_inputs(B, Hq, Hk, Sq, Sk, D, BF, 'cuda', seed=9)
     up = lambda n: (n + 255) // 256 * 256
     tiles_q, tiles_k = (Sq + 63) // 64 | 1, (Sk + 127) // 128      # of 64 queries (an odd number of them) and 128 keys
     ds = B * Hq * tiles_q * tiles_k * 64 * 128 * 2 + 2 * up(B * Hq * Sq * 4)
-    copies = 0 if D % 8 == 0 else sum(up(t.numel() // D * 104 * 2) for t in (q, q, q, q, k, k, v, v))
-    dq = {}
-    for limit in (-1, copies + ds, copies + ds - 256):
-        lib.fa_set_bwd_workspace_limit(limit)
-        x = [t.clone().requires_grad_() for t in (q, k, v)]
-        attention(*x, None, False, 1 / math.sqrt(D), 0.0)[0].backward(do)
-        torch.cuda.synchronize()
-        dq[limit] = x[0].grad
-    lib.fa_set_bwd_workspace_limit(-1)
-    # one rounding to bf16 of P and dS on either path, sums over 200 keys: the recomputing kernel's dQ is close, not equal
-    assert torch.equal(dq[copies + ds], dq[-1])
-    assert not torch.equal(dq[copies + ds - 256], dq[-1])
-    assert (dq[copies + ds - 256].float() - dq[-1].float()).abs().max() <= 2 ** -6 * dq[-1].float().abs().max()
+    copies = 0 if D % 8 == 0 else 2 * (2 * up(B * Hq * Sq * 104 * 2) + 2 * up(B * Hk * Sk * 104 * 2))
+    recomputed_differs = False
+    for seed in range(9, 15):
+        q, k, v, _, do = make_inputs(B, Hq, Hk, Sq, Sk, D, BF, 'cuda', seed=seed)
+        dq = {}
+        for limit in (-1, copies + ds, copies + ds - 256):
+            lib.fa_set_bwd_workspace_limit(limit)
+            x = [t.clone().requires_grad_() for t in (q, k, v)]
+            attention(*x, None, False, 1 / math.sqrt(D), 0.0)[0].backward(do)
+            torch.cuda.synchronize()
+            dq[limit] = x[0].grad
+        lib.fa_set_bwd_workspace_limit(-1)
+        assert torch.equal(dq[copies + ds], dq[-1])
+        # the recomputing kernel forms delta in another order: a few of the 1.5 million elements round the other way
+        recomputed_differs |= not torch.equal(dq[copies + ds - 256], dq[-1])
+        assert (dq[copies + ds - 256].float() - dq[-1].float()).abs().max() <= 2 ** -6 * dq[-1].float().abs().max()
+    assert recomputed_differs

@@ -131,3 +131,13 @@ def test_cases_of_the_backward_parts():
     from test_gpu_bwd_parts import CASES
     cut = [c for c in CASES if bwd(1, *c[:5], (c[5] + 7) // 8 * 8, *c[7:]).flags & 64]
     assert len(cut) == len(CASES) - 1      # (the window of 60 and 30 leaves one step per key tile: uncut)
+
+
+@pytest.mark.parametrize('call, rows', [
+    ((1, 8, 2, 2048, 2048, 128), False), ((1, 8, 2, 2048, 2048, 128, True), False), ((1, 8, 2, 1024, 1024, 256), False),
+    ((1, 8, 2, 1024, 1024, 64), False), ((1, 12, 12, 600, 900, 256), False), ((1, 4, 4, 2048, 2048, 256), False),
+    ((1, 8, 2, 1024, 1024, 64, True), True), ((1, 2, 2, 2048, 2048, 128), True), ((1, 32, 8, 512, 512, 128, True), True),
+])
+def test_packed_rows_only_where_their_xcds_are_not_the_bottleneck(call, rows):
+    """two K/V heads put all row blocks on two of the eight XCDs: 157 us where whole tiles take 57"""
+    assert bool(fwd(*call).flags & 128) == rows
