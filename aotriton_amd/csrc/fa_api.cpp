@@ -704,7 +704,7 @@ DkdvParts dkdv_parts(const fa_bwd_params* p, const Shape& s, int num_cu) {
   const int64_t items = nz * s.hk * n_tiles;
   if (items * 2 > num_cu) return r;
   const int bm = s.d == 64 ? 128 : s.d == 128 ? 64 : 32;
-  int64_t most = 0;
+  int64_t most = 0, sum = 0;
   for (int nt = 0; nt < n_tiles; ++nt) {
     int64_t n = (s.max_sq + bm - 1) / bm;
     if (s.windowed) {
@@ -713,6 +713,7 @@ DkdvParts dkdv_parts(const fa_bwd_params* p, const Shape& s, int num_cu) {
       n = b.hi - b.lo + 1;
     }
     most = n > most ? n : most;
+    sum += n;
   }
   const double t_step = (s.d == 64 ? 2.3 : s.d == 128 ? 1.9 : 2.1) * (s.dropout ? 1.7 : 1.0) * (s.bias ? 1.3 : 1.0);
   double best = group * most * t_step + 7;
@@ -726,6 +727,19 @@ DkdvParts dkdv_parts(const fa_bwd_params* p, const Shape& s, int num_cu) {
       if (t < 0.95 * best) { best = t; r.heads = heads; r.tiles = tiles; }
     }
   }
+  // An XCD owns the items of its kv-heads: with fewer kv-heads than XCDs the parts may just make more rounds there.
+  // Under a narrow window, whose items are alike, nothing is gained then (us of the whole backward, uncut / cut, B1 H2
+  // S1536, window 200: dropout D128 49 / 67, D256 68 / 78, bias 56 / 65); items of uneven weight fill each other's gaps
+  // (three packed sequences of 1500-2500 tokens, Hq 8, Hk 2, D128 causal 265 / 184).
+  const int64_t cus = num_cu >= fa::kNumXcd ? num_cu / fa::kNumXcd : 1;
+  const int64_t busiest = (nz * s.hk + fa::kNumXcd - 1) / fa::kNumXcd * n_tiles;
+  auto xcd_time = [&](int heads, int tiles) {
+    return (double)((busiest * heads * tiles + cus - 1) / cus) *
+           ((double)(group / heads) * ((most + tiles - 1) / tiles) * t_step + 7);
+  };
+  if (s.windowed && s.num_seqlens == 0 && sum * 5 > most * n_tiles * 4 && r.heads * r.tiles > 1 &&
+      xcd_time(r.heads, r.tiles) + 4 + 0.065 * s.d / 128 * items * r.heads * r.tiles > 1.05 * xcd_time(1, 1))
+    r.heads = r.tiles = 1;
   if (r.heads * r.tiles > 1) r.bytes = items * r.heads * r.tiles * (2 * 128 * s.d * 4);
   return r;
 }

@@ -27,7 +27,7 @@ CASES = [
     (1, 4, 2, 800, 100, 72, HF, False, 0.1, False),          # head dim rounded up
     (1, 4, 2, 500, 100, 113, BF, True, 0.0, False),          # through packed copies
     (1, 2, 2, 1500, 1400, 128, BF, True, 0.0, False),        # the last key tiles have fewer query tiles than parts
-    (1, 2, 2, 1500, 1400, 64, HF, (700, 10), 0.0, False),
+    (1, 2, 1, 1500, 1400, 64, HF, (700, 10), 0.0, False),
     (1, 2, 1, 1500, 700, 128, BF, (-200, 900), 0.1, False),  # keys that no row sees
 ]
 

@@ -141,3 +141,9 @@ def test_cases_of_the_backward_parts():
 def test_packed_rows_only_where_their_xcds_are_not_the_bottleneck(call, rows):
     """two K/V heads put all row blocks on two of the eight XCDs: 157 us where whole tiles take 57"""
     assert bool(fwd(*call).flags & 128) == rows
+
+
+def test_narrow_windows_leave_items_whole_where_parts_only_make_rounds():
+    assert bwd(1, 1, 2, 2, 1536, 1536, 128, (200, 0), 0.1).flags & 64 == 0
+    assert bwd(1, 1, 2, 2, 1536, 1536, 128, True, 0.1).flags & 64
+    assert bwd(1, 1, 8, 2, 1536, 1536, 128, (200, 0), 0.1).flags & 64
