@@ -497,23 +497,48 @@ int validate_bwd(const fa_bwd_params* p, int32_t version, const fa_options* opt,
   return FA_SUCCESS;
 }
 
+// fp32 forward at 128 columns: does it take fewer rounds of the CUs' time with 32 rows per workgroup (fa_f32_rows.hip) than
+// with 64 (fa_f32.hip)?  Estimated in microseconds from measurements on one box: a workgroup takes 7 us and 0.036 per key
+// against 5 and 0.075, 256 of them at a time, the heaviest first, and 2 us against 0.018 per key once.  Measured, rows kernel / 64-row tiles (B H S, us): 1 16 512
+// 28.5 / 50.8, 4 8 512 53.5 / 54.6, 8 8 512 105 / 98, 16 8 512 207 / 184; 4 8 1024 179 / 182, causal 116 / 167; 16 8 128
+// 25.9 / 20.2, 128 8 128 182 / 112; 8 8 256 35.3 / 31.7; 64 rows of 64 keys 12.4 / 11.8, 2048 of those 158 / 74.
+bool f32_fwd_rows128(const Shape& s, int64_t heads, int causal_type, int window_left, int window_right, int num_cu) {
+  const int64_t tiles = heads * ((s.max_sq + 63) / 64);
+  if (tiles <= 0 || s.max_sk <= 0) return true;
+  if (tiles > 16 * num_cu) return false;
+  auto time = [&](int rows, double once, double around, double per_key) {
+    const int64_t n = (s.max_sq + rows - 1) / rows;
+    double t = once;
+    for (int64_t at = 0; at < heads * n; at += num_cu) {
+      int64_t keys = s.max_sk;
+      if (s.windowed) {
+        const fa::Window w = fa::parse_window(causal_type, window_left, window_right, s.max_sq, s.max_sk);
+        const fa::BlockRanges b = fa::block_ranges(true, w.left, w.right, (int)(n - 1 - at / heads) * rows, s.max_sq, s.max_sk, rows, 32);
+        keys = b.hi < b.lo ? 0 : (b.hi - b.lo + 1) * 32;
+      }
+      t += around + per_key * (double)keys;
+    }
+    return t;
+  };
+  return time(32, 2, 7, 0.0363) < time(64, 0.018 * s.max_sk, 5, 0.075);
+}
+
 // fp32: the kernels whose waves share 32 rows (fa_f32_rows.hip) or those that split the head dim over the
 // waves (fa_f32.hip)?  The first at 64 columns always (the second are compiled for 128).  At 128 columns the
-// forward is level on a full chip (2 % faster without a mask, 3 % slower under a causal mask with
-// grouped heads) and up to 1.8 x faster below that; the backward, whose dK/dV kernel lacks registers
+// forward goes by the estimate above; the backward, whose dK/dV kernel lacks registers
 // there, gains up to 128 tiles of 64 rows (4-11 %) and loses from 168 on (15-50 %).
-bool f32_rows(const Shape& s, bool backward, int num_cu) {
+bool f32_rows(const Shape& s, bool backward, int causal_type, int window_left, int window_right, int num_cu) {
   const int64_t nz = s.num_seqlens != 0 ? std::abs(s.num_seqlens) : s.batch;
-  const int64_t tiles = nz * s.hq * ((s.max_sq + 63) / 64);
   if (s.d == 64) return true;
   if (s.d != 128) return false;
-  return backward ? tiles <= num_cu / 2 : !s.windowed || tiles < 4 * num_cu;
+  return backward ? nz * s.hq * ((s.max_sq + 63) / 64) <= num_cu / 2
+                  : f32_fwd_rows128(s, nz * s.hq, causal_type, window_left, window_right, num_cu);
 }
 
 hipError_t run_fwd(int dtype, int d, const fa::FwdArgs& a, const Shape& s, hipStream_t stream) {
   if (s.elementwise) return fa::run_fwd_valu(dtype, d, a, stream);
   if (dtype == FA_DTYPE_FLOAT32)
-    return (f32_rows(s, false, a.num_cu) ? fa::run_fwd_f32_rows : fa::run_fwd_f32)(d, a, s.windowed, s.bias, s.dropout, stream);
+    return (f32_rows(s, false, a.mask.causal_type, a.mask.window_left, a.mask.window_right, a.num_cu) ? fa::run_fwd_f32_rows : fa::run_fwd_f32)(d, a, s.windowed, s.bias, s.dropout, stream);
   if (d > 256) return fa::run_fwd_d512(dtype, a, s.windowed, s.bias, s.dropout, stream);
   const bool padded = a.head_dim != d || a.head_dim_v != d;   // head dim rounded up: the copies that mask the excess columns
   switch (d) {
@@ -834,7 +859,7 @@ int fa_query_fwd_config(const fa_fwd_params* params, int32_t num_cu, fa_kernel_c
   if (e != FA_SUCCESS) return e;
   // the vector-ALU kernels (3-D grid), the fp32 kernels and the split-head-dim kernels (above 256)
   const bool valu = params->Q.dtype == FA_DTYPE_FLOAT32 || s.d > 256 || s.elementwise;
-  const bool rows32 = !s.elementwise && params->Q.dtype == FA_DTYPE_FLOAT32 && f32_rows(s, false, num_cu > 0 ? num_cu : 256);
+  const bool rows32 = !s.elementwise && params->Q.dtype == FA_DTYPE_FLOAT32 && f32_rows(s, false, params->causal_type, params->window_left, params->window_right, num_cu > 0 ? num_cu : 256);
   const int cus = num_cu > 0 ? num_cu : 256;
   const FwdPlan plan = fwd_plan(params->Q.dtype, s, params->causal_type, params->window_left, params->window_right, cus);
   const bool split = !plan.rows && plan.splits > 1;
@@ -892,7 +917,7 @@ int fa_query_bwd_config(const fa_bwd_params* params, const fa_options* options, 
   if (valu && kernel_slot == 3) return FA_ERROR_PEER_ACCESS_UNSUPPORTED;
   const bool split_d = !s.elementwise && params->Q.dtype != FA_DTYPE_FLOAT32 && s.d > 256 && kernel_slot != 0;
   const bool f32_mfma = !s.elementwise && params->Q.dtype == FA_DTYPE_FLOAT32 && kernel_slot != 0;
-  const bool rows32 = f32_mfma && f32_rows(s, true, 256);
+  const bool rows32 = f32_mfma && f32_rows(s, true, params->causal_type, params->window_left, params->window_right, 256);
   const fa::TileShape t = rows32 ? fa::f32_rows_tile_shape(s.d)
                           : f32_mfma ? fa::f32_tile_shape(s.d, kernel_slot)
                           : split_d ? fa::d512_tile_shape(kernel_slot)
@@ -1254,7 +1279,7 @@ static int attn_bwd_impl(const fa_bwd_params* p_in, int32_t params_version, void
     // out; the dK/dV kernel runs after it and reads it, so the whole backward is two launches
     // (kernel_slot 0 still launches the preprocess kernel on its own).
     // (fa_f32_rows.hip does the same)
-    const bool rows32 = f32 && f32_rows(s, true, dev->num_cu);
+    const bool rows32 = f32 && f32_rows(s, true, p->causal_type, p->window_left, p->window_right, dev->num_cu);
     const bool delta_launch = (f32 && !rows32) || big || slow;
     // The 16-bit kernels up to head dim 256 can keep dS in HBM instead of recomputing S and dP in
     // the dQ kernel (5 GEMMs instead of 7): delta first, then dK/dV writing dS, then dQ = dS K.  It

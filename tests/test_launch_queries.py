@@ -143,6 +143,27 @@ def test_packed_rows_only_where_their_xcds_are_not_the_bottleneck(call, rows):
     assert bool(fwd(*call).flags & 128) == rows
 
 
+def fwd32(B, H, Sq, Sk, D, causal=False):
+    from aotriton_amd.pyaotriton.v3.flash import attn_fwd_params, query_fwd_config
+    x = attn_fwd_params()
+    f32 = lambda *s: view(*s, name='kFloat32')
+    x.Q, x.K, x.V, x.Out = f32(B, H, Sq, D), f32(B, H, Sk, D), f32(B, H, Sk, D), f32(B, H, Sq, D)
+    _common(x, B, H, Sq, Sk, causal, 0.0, False)
+    err, c = query_fwd_config(x, 256)
+    assert int(err) == 0
+    return c
+
+
+@pytest.mark.parametrize('call, rows', [
+    ((1, 16, 512, 512, 128), 32), ((8, 8, 512, 512, 128), 64), ((16, 8, 512, 512, 128), 64), ((8, 8, 128, 128, 128), 32),
+    ((16, 8, 192, 192, 128), 64), ((24, 8, 128, 128, 128), 64), ((128, 8, 128, 128, 128), 64), ((4, 8, 1024, 1024, 128, True), 32),
+    ((16, 8, 1024, 1024, 128), 64), ((16, 16, 1, 1000, 128), 32), ((128, 8, 128, 128, 64), 32), ((600, 16, 256, 256, 128), 64),
+])
+def test_fp32_rows_of_a_workgroup(call, rows):
+    """at 128 columns the kernel that needs less of the CUs' time; always 32 rows at 64"""
+    assert fwd32(*call).block_m == rows
+
+
 def test_narrow_windows_leave_items_whole_where_parts_only_make_rounds():
     assert bwd(1, 1, 2, 2, 1536, 1536, 128, (200, 0), 0.1).flags & 64 == 0
     assert bwd(1, 1, 2, 2, 1536, 1536, 128, True, 0.1).flags & 64
