@@ -15,6 +15,7 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/core/dispatch/Dispatcher.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
@@ -22,6 +23,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/forward_grad.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/pybind.h>
 #include <torch/library.h>
@@ -313,6 +315,7 @@ struct AttentionFunction : torch::autograd::Function<AttentionFunction> {
 // There is no forward-mode formula.  A call without a gradient goes past the Function, whose own error would
 // come after the launch: without this check such a call would answer without the tangent.
 void refuse_tangents(std::initializer_list<const Tensor*> inputs) {
+  if (torch::autograd::ForwardADLevel::try_get_by_idx(0) == nullptr) return;      // (the tensors' own look takes locks)
   for (const Tensor* t : inputs)
     TORCH_CHECK_NOT_IMPLEMENTED(!t->defined() || !t->_fw_grad(0).defined(),
                                 "forward-mode AD of the attention operators (jvp) is not implemented");
@@ -839,6 +842,11 @@ SdpaArgs read_sdpa(Args& a) {
 // Philox state from torch's generator; None where the Python route has to take the call
 PyObject* py_sdpa_ops(PyObject*, PyObject* const* argv, Py_ssize_t n) {
   HANDLE_TH_ERRORS
+  // subclasses (all but Parameter) and function modes may override torch's functions: they have to see the calls of the
+  // Python route
+  if (at::impl::torch_function_mode_enabled()) Py_RETURN_NONE;
+  for (Py_ssize_t i = 0; i < n && i < 4; ++i)
+    if (THPVariable_Check(argv[i]) && !THPVariable_CheckTypeExact(Py_TYPE(argv[i]))) Py_RETURN_NONE;
   Args a{argv, n};
   const SdpaArgs in = read_sdpa(a);
   if (traced({&in.q, &in.k, &in.v, &in.mask})) Py_RETURN_NONE;

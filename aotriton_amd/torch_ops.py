@@ -74,10 +74,9 @@ def scaled_dot_product_attention(query, key, value, attn_mask=None, dropout_p=0.
     governs it) but uses the operators' Philox stream, not the one of torch's own kernels.
     As in torch, is_causal means the top-left aligned lower triangle.
     """
-    # (subclasses and function modes that override torch's functions have to see the calls below)
-    if not torch.compiler.is_compiling() and not torch.overrides.has_torch_function((query, key, value, attn_mask)):
+    if not torch.compiler.is_compiling():
         out = _torch_host.sdpa_ops(query, key, value, attn_mask, dropout_p, is_causal, scale, enable_gqa)
-        if out is not None:      # None: under a dispatch mode or a functorch transform
+        if out is not None:      # None: subclasses, function and dispatch modes, functorch transforms
             return out
     q, k, v, bias, sm_scale = prepare(query, key, value, attn_mask, is_causal, scale, enable_gqa)
     hq = q.shape[1]
