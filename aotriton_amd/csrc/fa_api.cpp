@@ -102,7 +102,8 @@ hipError_t scratch_of_device(int dev, float** out) {
   return hipSuccess;
 }
 
-// Workspace of the backward that keeps dS in HBM between its two kernels: one buffer per device
+// Workspace (dS of the backward that keeps it in HBM between its kernels, parts of dK/dV items, the parts of a split forward
+// without an allocator, packed copies): one buffer per device
 // that belongs to the library and only grows (hipMalloc once, then reused: a stream-ordered pool
 // allocation made the host wait for the GPU on every call).  Calls on one device share it: the
 // device's mutex covers the enqueue, and every call first waits (on the GPU) for the event recorded
@@ -654,9 +655,10 @@ FwdPlan fwd_plan(int dtype, const Shape& s, int causal_type, int window_left, in
 
 // Tiles of 128 rows, two workgroups per CU, instead of 256 rows and one (FwdHalfTile)?  Where they save a part
 // of the rounds in which an XCD's CUs take its tiles; the line lies above what they cost per row.  Measured (bf16, us,
-// 256 -> 128 rows): B40 H16 S128 D64 19.2 -> 14.4 (3 rounds against 2), B16 H12 S640 D64 45 -> 34 and causal 44 -> 29,
-// D128 67 -> 52 and 62 -> 42 (3 : 2), B40 H16 S640 D64 113 -> 99 (8 : 7), S384 53 -> 47 (5 : 4); S800 271 -> 267 and causal
-// 210 -> 214 at D128 (10 : 9); at equal rounds 5-15 % slower.  With a bias the finer tiles cost more (10-15 %), so those keep the large ones.
+// 256 -> 128 rows): B40 H16 S128 D64 19.1 -> 14.6 (3 rounds against 2), B16 H12 S640 D64 46.6 -> 39.2 and causal 43.4 -> 31.0,
+// D128 68 -> 59 and 63 -> 45 (3 : 2), B40 H16 S640 D64 116 -> 108 (8 : 7), S384 54 -> 48 (5 : 4); B32 H16 S800 D128 227 -> 224
+// (10 : 9); at equal rounds 5-15 % slower.  With a bias the finer tiles cost more (10-15 %), so those keep the large ones.
+// Rounds are all that is compared: what a causal mask does to the tiles of one round is not.
 bool fwd_half_tiles(int dtype, const Shape& s, int num_cu) {
   if (s.elementwise || !is_16bit(dtype) || s.d > 128 || s.bias || s.num_seqlens != 0) return false;
   const int64_t heads = (s.batch * (int64_t)s.hq + fa::kNumXcd - 1) / fa::kNumXcd, cus = num_cu / fa::kNumXcd;
@@ -685,8 +687,9 @@ fa::DropoutArgs dropout_args(float p, const fa_tensor0& seed, const fa_tensor0& 
 }
 
 // Bytes of workspace with which the split backward keeps dS in HBM, 0 when this call recomputes S
-// and dP in its dQ kernel instead (anything but the 16-bit MFMA kernels of the 128-column build,
-// packed sequences, dB wanted, an empty tensor).  *ds_bytes / *stat_bytes: the parts of the buffer.
+// and dP in its dQ kernel instead (anything but the 16-bit MFMA kernels up to 256 columns, packed sequences, an
+// empty tensor, plain calls at 64 columns, and with dB what the first test below names).  *ds_bytes / *stat_bytes: the
+// parts of the buffer.
 int64_t ds_workspace_need(const fa_bwd_params* p, const Shape& s, int* ntq, int* ntk, int64_t* ds_bytes,
                           int64_t* stat_bytes) {
   if (s.elementwise || !is_16bit(p->Q.dtype) || (s.d != 64 && s.d != 128 && s.d != 256) || s.num_seqlens != 0 ||
@@ -695,7 +698,10 @@ int64_t ds_workspace_need(const fa_bwd_params* p, const Shape& s, int* ntq, int*
   // dB leaves the dQ-from-dS kernel as 16-byte pieces of its rows, or is left to the recomputing one; so are small
   // calls, where the third launch costs what is saved (us forward + backward, recomputing -> stored: B2 H8 S256 D64
   // 50 -> 53, B8 H12 S512 D64 118 -> 100, D128 148 -> 132, D256 468 -> 420, B16 H16 S1024 D64 842 -> 795, causal 670 -> 579),
-  // and long rows at D = 64 (H8 S4096 causal 395 -> 370, H16 S8192 window 4000 1425 -> 1482)
+  // and long rows at D = 64.  There (us of the backward alone, recomputing -> stored, B1): H8 S4096 causal 312 -> 300, H16
+  // S4096 610 -> 560, window 1000 283 -> 254, S6144 causal 793 -> 744, S8192 2195 -> 2050, window 1000 713 -> 710, but causal
+  // 1272 -> 1298 and window 4000 1076 -> 1138: the line gives up 6 % of some calls for 2-6 % of others (stored tiles
+  // against visible pairs would tell them apart)
   if (p->DB.ptr != nullptr &&
       ((int64_t)s.batch * s.hq * s.max_sq * s.max_sk < (int64_t)1 << 22 || (s.d == 64 && s.max_sk > 4096) ||
        p->DB.strides[3] != 1 || ((p->DB.strides[0] | p->DB.strides[1] | p->DB.strides[2]) & 7) != 0 ||
@@ -720,7 +726,11 @@ struct DkdvParts { int heads, tiles; int64_t bytes; };
 
 // The rule compares estimated times in microseconds: 1.9-2.3 per step (64 queries at D = 128, 128 at 64,
 // 32 at 256; more with a bias or dropout), 7 around an item, 4 for the second launch and 0.065 of the
-// chip's memory time per part (256 KB written and read at D = 128).
+// chip's memory time per part (256 KB written and read at D = 128).  Head dim 64 without a bias is older than the kernel
+// there, which takes 64-query steps, two workgroups per CU: the figures stand for 128 queries and one, and calls
+// with more than num_cu / 2 items stay whole although there are twice as many places.  What it chooses there holds (us of
+// the backward, whole / cut, B1: Hq 8 Hk 2 2048 x 256 143 / 35, Hq 16 Hk 4 1024 causal 90 / 46, H8 4096 x 512 82 / 41, H4 4096 x
+// 1024 causal 88 / 50, Hq 16 Hk 8 512 x 1024 causal 36 / 34; H8 1024 x 1000 39 / 40), finer cuts have not been measured.
 DkdvParts dkdv_parts(const fa_bwd_params* p, const Shape& s, int num_cu) {
   DkdvParts r{1, 1, 0};
   if (s.elementwise || !is_16bit(p->Q.dtype) || s.d > 256 || s.max_sq <= 0 || s.max_sk <= 0 || s.batch <= 0) return r;
@@ -1284,7 +1294,7 @@ static int attn_bwd_impl(const fa_bwd_params* p_in, int32_t params_version, void
     // The 16-bit kernels up to head dim 256 can keep dS in HBM instead of recomputing S and dP in
     // the dQ kernel (5 GEMMs instead of 7): delta first, then dK/dV writing dS, then dQ = dS K.  It
     // takes 2 bytes per (query, key) pair of workspace; when that is above the limit, under stream
-    // capture, for packed sequences or with dB the kernels recompute.  (Measured at S4096, 16384 tokens:
+    // capture, for packed sequences and where ds_workspace_need says so the kernels recompute.  (Measured at S4096, 16384 tokens:
     // head dim 128 gains 5 %, 256 gains 16 %; head dim 64, where a pair costs half the arithmetic and
     // the same bytes, loses 12 % unless the dQ kernel is spared dropout or a bias: then it gains 20-30 %.)
     void* ds_ws = nullptr;

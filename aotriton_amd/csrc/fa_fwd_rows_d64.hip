@@ -2,7 +2,7 @@
 #include "fa_fwd_rows.h"
 #include "fa_kernels.h"
 
-// Compiled twice, as the other per-head-dim files: FA_PADDED=1 for smaller head dims (a multiple of 8).
+// Compiled twice, as the other per-head-dim files: FA_PADDED=64 for smaller head dims (a multiple of 8).
 #ifndef FA_PADDED
 #define FA_PADDED 0
 #endif

@@ -240,9 +240,14 @@ FA_API int fa_attn_fwd(const fa_fwd_params* params, int32_t params_version,
  * done (a stream-ordered pool, a caching allocator; under stream capture, memory of the graph).
  * It returns null when there is none.  The forward takes scratch when few query rows meet many
  * keys (decode, short prompt chunks): the keys are split over workgroups and the parts' sums
- * meet in memory.  fa_attn_fwd takes it from the library's workspace and, under stream capture or
- * without memory, does not split; the results differ by fp32 summation order only.  No counterpart in
- * the reference. */
+ * meet in memory.  fa_attn_fwd (which the Python wrappers call when they are given a stream) takes it from
+ * the library's workspace: forwards that split share that one buffer per device with each other and with the
+ * backward, so two of them on two streams take turns on the GPU, and one that needs more than the buffer
+ * holds allocates (hipFree of the old buffer, which waits for the device, and hipMalloc).  Under stream capture or
+ * without memory it does not split.  Results of the two ways are not the same bits: the fp32 sums are added in
+ * another order, and P is rounded to 16 bits against the reference maximum of each part, or of each wave of
+ * the packed-rows kernel, instead of one per row block.  Nothing is held in fewer bits either way.  No
+ * counterpart in the reference. */
 typedef struct fa_allocator {
   void* cookie;
   void* (*alloc)(struct fa_allocator* self, uint64_t bytes);
@@ -323,14 +328,17 @@ FA_API int fa_v2_attn_bwd_compact_varlen(
 FA_API int fa_attn_bwd_noalloc(const fa_bwd_params* params, int32_t params_version,
                                void* hip_stream);
 
-/* Workspace of the split backward.  For 16-bit tensors at head dims up to 256 (dense batches, no dB,
- * not under stream capture; up to head dim 64 only with dropout or a bias, where it pays) fa_attn_bwd keeps dS in HBM between its dK/dV and dQ kernels instead of
- * recomputing S and dP in the dQ kernel (5 GEMMs instead of 7; delta kernel, dK/dV kernel writing dS,
- * dQ = dS K kernel): 2 bytes per (batch, q-head, query, key) plus 8 bytes per (batch, q-head, query),
- * in a buffer per device that belongs to the library, is allocated on first use, only grows and is
+/* Workspace: a buffer per device that belongs to the library, is allocated on first use, only grows and is
  * reused by every later call (calls on one device take turns: a call on another stream than the last
- * one waits on the GPU for the last one's kernels).  A call that would need more than the limit
- * recomputes instead, with the same results up to fp32 summation order.  The limit is, in this
+ * one waits on the GPU for the last one's kernels).  Its main user is the split backward.  For 16-bit tensors at head
+ * dims up to 256 (dense batches, not under stream capture; up to head dim 64 only with dropout or a bias, where it
+ * pays; with dB when its rows are made of aligned 16-byte pieces and the call is neither small nor, at head dim 64,
+ * longer than 4096 keys) fa_attn_bwd keeps dS in HBM between its dK/dV and dQ kernels instead of
+ * recomputing S and dP in the dQ kernel (5 GEMMs instead of 7; delta kernel, dK/dV kernel writing dS,
+ * dQ = dS K kernel): 2 bytes per (batch, q-head, query, key) plus 8 bytes per (batch, q-head, query).
+ * The others: parts of dK/dV items where these do not fill the chip (fp32 sums), split forwards
+ * (fa_attn_fwd_alloc above), packed copies.  A backward that would need more than the limit goes without the
+ * parts first and then without dS, and recomputes, with the same results up to fp32 summation order.  The limit is, in this
  * order: the last fa_set_bwd_workspace_limit(bytes >= 0); AOTRITON_AMD_BWD_WORKSPACE_MB of the
  * environment; an eighth of the device's memory.  0 switches the workspace off, a negative value
  * forgets the last call.  fa_query_bwd_config sets bit 4 of `flags` when a call would use it.  fa_trim_workspace
