@@ -499,7 +499,7 @@ int validate_bwd(const fa_bwd_params* p, int32_t version, const fa_options* opt,
 }
 
 // fp32 forward at 128 columns: does it take fewer rounds of the CUs' time with 32 rows per workgroup (fa_f32_rows.hip) than
-// with 64 (fa_f32.hip)?  Estimated in microseconds from measurements on one box: a workgroup takes 7 us and 0.036 per key
+// with 64 (fa_f32.hip)?  Estimated in microseconds from measurements on an MI355X: a workgroup takes 7 us and 0.036 per key
 // against 5 and 0.075, 256 of them at a time, the heaviest first, and 2 us against 0.018 per key once.  Measured, rows kernel / 64-row tiles (B H S, us): 1 16 512
 // 28.5 / 50.8, 4 8 512 53.5 / 54.6, 8 8 512 105 / 98, 16 8 512 207 / 184; 4 8 1024 179 / 182, causal 116 / 167; 16 8 128
 // 25.9 / 20.2, 128 8 128 182 / 112; 8 8 256 35.3 / 31.7; 64 rows of 64 keys 12.4 / 11.8, 2048 of those 158 / 74.
