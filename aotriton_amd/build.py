@@ -38,14 +38,16 @@ EXTRA = {
     'fa_bwd_dkdv_d128.hip': ['-mllvm', '-amdgpu-sched-strategy=max-ilp'],
     'fa_bwd_dkdv_parts_d128.hip': ['-mllvm', '-amdgpu-sched-strategy=max-ilp'],
     'fa_bwd_dq_bias_d64.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'],
+    # (S and dP in vector registers; the accumulators are asm operands and stay in accumulation registers)
+    'fa_bwd_wide_d128.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'],
     'fa_bwd_dq_d128.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'],
 }
 
 # The per-head-dim kernel files are compiled a second time with FA_PADDED = the head dim: the copies that
 # serve head dims rounded up to the compiled one.
-PADDED_RE = re.compile(r'fa_(fwd|fwd_rows|bwd_dkdv|bwd_dkdv_parts|bwd_dq|bwd_dq_bias|bwd_fused)_d(\d+)\.hip$')
+PADDED_RE = re.compile(r'fa_(fwd|fwd_rows|bwd_dkdv|bwd_dkdv_parts|bwd_dq|bwd_dq_bias|bwd_wide|bwd_fused)_d(\d+)\.hip$')
 # ... and these a third time with 96 columns, for head dims above 64 and up to 96
-COLS96_RE = re.compile(r'fa_(fwd|bwd_dkdv|bwd_dq)_d128\.hip$')
+COLS96_RE = re.compile(r'fa_(fwd|bwd_dkdv|bwd_dq|bwd_wide)_d128\.hip$')
 
 
 def sources():
@@ -149,6 +151,32 @@ _WATERFALL = re.compile(r'v_readfirstlane_b32[^\n]*\n(?:[^\n]*\n){0,24}?[^\n]*s_
                         r'[^\n]*s_xor_b64 exec, exec[^\n]*\n[^\n]*s_cbranch_execnz')
 
 
+def asm_mfma_hazards(text):
+    """MFMAs written as asm whose operands a vector instruction writes less than two instructions before: the compiler keeps
+    that distance for its own MFMAs and does not look into asm.  Returns the lines."""
+    def registers(operand):
+        m = re.match(r'v\[(\d+):(\d+)\]$', operand) or re.match(r'v(\d+)()$', operand)
+        return set(range(int(m.group(1)), int(m.group(2) or m.group(1)) + 1)) if m else set()
+    found, before, in_asm = [], [], False
+    for line in text.splitlines():
+        if '#ASM' in line:
+            in_asm = 'START' in line
+        line = line.split(';')[0].strip()
+        if not line or line.startswith('.') or line.endswith(':'):
+            continue
+        op, _, rest = line.partition(' ')
+        args = [a.strip() for a in rest.split(',')]
+        if in_asm and op.startswith('v_mfma'):
+            sources, distance = registers(args[1]) | registers(args[2]), 0
+            for written, states in reversed(before):
+                if distance < 2 and written & sources:
+                    found.append(line)
+                distance += states
+        vector = op.startswith('v_') and not op.startswith('v_mfma')
+        before = (before + [(registers(args[0]) if vector else set(), int(args[0], 0) + 1 if op == 's_nop' else 1)])[-4:]
+    return found
+
+
 def scan(jobs=8):
     """Compiles every kernel file to assembly and reports per-descriptor loops around buffer
     accesses ("waterfall" loops: readfirstlane, compare, masked issue, repeat while lanes are left).
@@ -156,7 +184,7 @@ def scan(jobs=8):
     threadIdx.x >> 6.  They cost time, and hipcc 7.2 has placed a register spill in the block such
     a loop exits to, before exec is restored: the store runs with no lane enabled and the reload
     later returns whatever the slot held.  The kernels here are written so that none is emitted;
-    returns the list of (file, loops, functions left out of line) that have some of either."""
+    returns the list of (file, loops, functions left out of line, asm_mfma_hazards) that have some of any."""
     import tempfile
     tmpdir = tempfile.TemporaryDirectory(prefix='fa_scan_')
     tmp = tmpdir.name
@@ -164,7 +192,7 @@ def scan(jobs=8):
     def one(unit):
         src, defines, objname = unit
         if not src.endswith('.hip'):
-            return src, 0, 0
+            return src, 0, 0, []
         out = os.path.join(tmp, objname + '.s')
         cmd = [HIPCC] + COMMON + EXTRA.get(src, []) + defines + ['-x', 'hip', '--cuda-device-only', '-S',
                                                                  os.path.join(CSRC, src), '-o', out]
@@ -175,10 +203,10 @@ def scan(jobs=8):
         # a device function left out of line (a lambda the inliner gave up on) keeps its captures in
         # memory and reads them back with flat loads; every kernel here is meant to be one function
         outlined = len(re.findall(r'^\s*\.type\s+\S+,@function', text, re.M)) - text.count('.amdhsa_kernel ')
-        return objname, len(_WATERFALL.findall(text)), outlined
+        return objname, len(_WATERFALL.findall(text)), outlined, asm_mfma_hazards(text)
 
     with tmpdir, concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as ex:
-        return [(n, c, o) for n, c, o in ex.map(one, sources()) if c or o]
+        return [r for r in ex.map(one, sources()) if any(r[1:])]
 
 
 if __name__ == '__main__':
@@ -189,6 +217,6 @@ if __name__ == '__main__':
     a = ap.parse_args()
     if a.scan:
         found = scan(a.j)
-        print('per-descriptor loops / functions left out of line:', found if found else 'none')
+        print('per-descriptor loops / functions left out of line / asm MFMAs too close behind their operands:', found if found else 'none')
         sys.exit(1 if found else 0)
     print(build(a.j, a.force))

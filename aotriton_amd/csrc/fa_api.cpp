@@ -11,6 +11,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <vector>
 
 #include "aotriton_amd/flash.h"
 #include "aotriton_amd/probe.h"
@@ -779,6 +780,75 @@ DkdvParts dkdv_parts(const fa_bwd_params* p, const Shape& s, int num_cu) {
   return r;
 }
 
+// The kernels with 64 rows per wave (fa_bwd_wide.h; 16-bit types, head dims above 64 and up to 128, no bias, no dropout) take
+// the matrix work of a pair in 8-25 % less time, in workgroups of 256 rows instead of 128: they are chosen where that does
+// not leave more of the chip idle.  The rule compares the walks of both over the busiest XCD, in microseconds: an item
+// takes what its steps take (128 x 64 or 256 x 32 pairs) and what it costs to begin and to end.  Fitted to 128 calls (bf16,
+// D128; heads 8-512, 64-4096 tokens, causal or not, GQA, windows; us of the whole backward, 128 -> 256 rows): B16 H16 S512
+// causal 136 -> 124, B8 H16 S1024 173 -> 157, B4 H16 S4096 912 -> 825, full 1584 -> 1493; left alone B8 H16 S512 causal 72 / 74,
+// B1 H8 S1024 60 / 91, Hq 32 Hk 8 S2048 183 / 405.  It is off the better choice by 4 % in one of them.
+// Packed sequences stand for as many of their average length, but no walk is shorter than the longest one's heaviest item.
+struct BwdRoute {
+  bool wide_dkdv, wide_dq;
+  bool recompute;               // both, and faster than the kernels that keep dS
+  int group_dkdv, group_dq;     // heads walked together by the wide kernels
+};
+struct WalkCost { double item, step; };
+// rows: the side the items are tiles of; cols: the side they step over
+double tile_walk_time(const fa_bwd_params* p, const Shape& s, bool keys, int num_heads, int zh_group, int tile, int step,
+                      int heads_per_item, WalkCost c, int num_cu, int max_rows, int max_cols, int nz) {
+  const int n_tiles = (max_rows + tile - 1) / tile;
+  std::vector<float> cost((size_t)n_tiles);
+  fa::Window w{0, 0};
+  if (s.windowed)
+    w = fa::parse_window(p->causal_type, p->window_left, p->window_right, keys ? max_cols : max_rows, keys ? max_rows : max_cols);
+  for (int t = 0; t < n_tiles; ++t) {
+    const fa::BlockRanges b = fa::block_ranges(s.windowed, keys ? w.right : w.left, keys ? w.left : w.right, t * tile, max_rows,
+                                               max_cols, tile, step);
+    cost[keys ? t : n_tiles - 1 - t] = (float)(c.item + c.step * heads_per_item * (b.hi - b.lo + 1));
+  }
+  return fa::walk_time(fa::tile_work(nz * num_heads, zh_group, n_tiles), cost.data(), n_tiles, num_cu);
+}
+bool wide_bwd_built(const fa_bwd_params* p, const Shape& s) {
+  return !s.elementwise && is_16bit(p->Q.dtype) && s.d == 128 && !s.bias && !s.dropout && s.max_sq > 0 && s.max_sk > 0 && s.batch > 0;
+}
+BwdRoute bwd_route(const fa_bwd_params* p, const Shape& s, int num_cu) {
+  BwdRoute r{false, false, false, 2, fa::q_head_group(s.hq, s.hk)};
+  if (!wide_bwd_built(p, s)) return r;
+  const int nz = s.num_seqlens != 0 ? std::abs(s.num_seqlens) : s.batch, group = s.hq / s.hk;
+  int sq = s.max_sq, sk = s.max_sk;
+  if (s.num_seqlens > 0) {
+    sq = std::max(1, std::min(sq, (int)(p->Q.sizes[2] / nz)));
+    sk = std::max(1, std::min(sk, (int)(p->K.sizes[2] / nz)));
+  }
+  struct Best { double t; int group; };
+  auto walk = [&](bool keys, int tile, int step, WalkCost c) {
+    const int heads = keys ? s.hk : s.hq, zg = keys ? 2 : fa::q_head_group(s.hq, s.hk), per_item = keys ? group : 1;
+    const int rows = keys ? sk : sq, cols = keys ? sq : sk;
+    Best b{tile_walk_time(p, s, keys, heads, zg, tile, step, per_item, c, num_cu, rows, cols, nz), zg};
+    if (s.num_seqlens != 0) {
+      const double longest = tile_walk_time(p, s, keys, 1, 1, tile, step, per_item, c, 1 << 20, keys ? s.max_sk : s.max_sq, keys ? s.max_sq : s.max_sk, 1);
+      b.t = std::max(b.t, longest);
+    } else if (tile == 256) {
+      // all heads of an XCD side by side, the heavy tiles of all of them first: better balanced, more streams in flight
+      const int all = (nz * heads + fa::kNumXcd - 1) / fa::kNumXcd;
+      const double t = 1.04 * tile_walk_time(p, s, keys, heads, all, tile, step, per_item, c, num_cu, rows, cols, nz);
+      if (t < b.t) b = Best{t, all};
+    }
+    return b;
+  };
+  const Best k_old = walk(true, 128, 64, {9, 1.95}), k_wide = walk(true, 256, 32, {7, 1.8});
+  const Best q_old = walk(false, 128, 64, {5, 1.7}), q_wide = walk(false, 256, 32, {5, 1.42});
+  // (with 128 rows half of every tile would be empty)
+  r.wide_dkdv = sk > 128 && k_wide.t < k_old.t;
+  r.wide_dq = sq > 128 && q_wide.t < q_old.t;
+  r.group_dkdv = k_wide.group;
+  r.group_dq = q_wide.group;
+  // (keeping dS takes 0.9-1.1 of what the 128-row kernels take for recomputing)
+  r.recompute = r.wide_dkdv && r.wide_dq && p->DB.ptr == nullptr && k_wide.t + q_wide.t < 0.97 * (k_old.t + q_old.t);
+  return r;
+}
+
 // What of the stored dS (`need` bytes) and the parts fits `room` bytes of workspace, and the bytes it takes.  The
 // parts give way first.
 int64_t fit_workspace(int64_t room, int64_t* need, DkdvParts* parts) {
@@ -928,17 +998,8 @@ int fa_query_bwd_config(const fa_bwd_params* params, const fa_options* options, 
   const bool split_d = !s.elementwise && params->Q.dtype != FA_DTYPE_FLOAT32 && s.d > 256 && kernel_slot != 0;
   const bool f32_mfma = !s.elementwise && params->Q.dtype == FA_DTYPE_FLOAT32 && kernel_slot != 0;
   const bool rows32 = f32_mfma && f32_rows(s, true, params->causal_type, params->window_left, params->window_right, 256);
-  const fa::TileShape t = rows32 ? fa::f32_rows_tile_shape(s.d)
-                          : f32_mfma ? fa::f32_tile_shape(s.d, kernel_slot)
-                          : split_d ? fa::d512_tile_shape(kernel_slot)
-                          : valu  ? (kernel_slot == 1 ? fa::TileShape{1, 32, 4, 0} : fa::TileShape{32, 1, 4, 0})
-                                  : fa::bwd_tile_shape(params->Q.dtype, s.d, s.windowed, s.bias, s.dropout, kernel_slot);
-  const int nz = s.num_seqlens != 0 ? std::abs(s.num_seqlens) : s.batch;
-  out->block_m = t.block_m; out->block_n = t.block_n; out->num_waves = t.num_waves;
-  out->lds_bytes = t.lds_bytes;
-  const int mt = (s.max_sq + t.block_m - 1) / t.block_m, nt = (s.max_sk + t.block_n - 1) / t.block_n;
   constexpr int kCus = 256;      // assumed here
-  const int ratio = s.hq / s.hk;
+  const BwdRoute route = bwd_route(params, s, kCus);
   // what of the workspace's uses the call gets (a host without a device: no limit unless one was set)
   int ntq = 0, ntk = 0, dev = 0;
   int64_t ds_bytes = 0, stat_bytes = 0, need = 0;
@@ -948,8 +1009,25 @@ int fa_query_bwd_config(const fa_bwd_params* params, const fa_options* options, 
   if (be == 0) {
     need = ds_workspace_need(params, s, &ntq, &ntk, &ds_bytes, &stat_bytes);
     parts = dkdv_parts(params, s, kCus);
+    if (route.recompute) {
+      need = 0;
+      parts = DkdvParts{1, 1, 0};
+    }
     fit_workspace(have_dev ? ws_limit_bytes(dev) : set >= 0 ? set : INT64_MAX, &need, &parts);
   }
+  const bool wide_dkdv = route.wide_dkdv && need == 0 && parts.bytes == 0;
+  const fa::TileShape t = rows32 ? fa::f32_rows_tile_shape(s.d)
+                          : f32_mfma ? fa::f32_tile_shape(s.d, kernel_slot)
+                          : split_d ? fa::d512_tile_shape(kernel_slot)
+                          : valu  ? (kernel_slot == 1 ? fa::TileShape{1, 32, 4, 0} : fa::TileShape{32, 1, 4, 0})
+                          : kernel_slot == 1 && wide_dkdv ? fa::bwd_wide_shape(true)
+                          : kernel_slot == 2 && route.wide_dq ? fa::bwd_wide_shape(false)
+                                  : fa::bwd_tile_shape(params->Q.dtype, s.d, s.windowed, s.bias, s.dropout, kernel_slot);
+  const int nz = s.num_seqlens != 0 ? std::abs(s.num_seqlens) : s.batch;
+  out->block_m = t.block_m; out->block_n = t.block_n; out->num_waves = t.num_waves;
+  out->lds_bytes = t.lds_bytes;
+  const int mt = (s.max_sq + t.block_m - 1) / t.block_m, nt = (s.max_sk + t.block_n - 1) / t.block_n;
+  const int ratio = s.hq / s.hk;
   // 1-D work lists of the main kernels
   auto workers = [&](int heads, int zg, int items) {
     const fa::TileWork w = fa::tile_work(nz * heads, zg, items);
@@ -968,8 +1046,8 @@ int fa_query_bwd_config(const fa_bwd_params* params, const fa_options* options, 
     out->grid[2] = nz;
   } else switch (kernel_slot) {
     case 0: out->grid[0] = mt; out->grid[1] = s.hq; out->grid[2] = nz; break;
-    case 1: out->grid[0] = workers(s.hk, 2, nt * parts.heads * parts.tiles); break;
-    case 2: out->grid[0] = workers(s.hq, fa::q_head_group(s.hq, s.hk), mt); break;
+    case 1: out->grid[0] = workers(s.hk, wide_dkdv ? route.group_dkdv : 2, nt * parts.heads * parts.tiles); break;
+    case 2: out->grid[0] = workers(s.hq, route.wide_dq ? route.group_dq : fa::q_head_group(s.hq, s.hk), mt); break;
     default: out->grid[0] = workers(s.hk, 2, nt + mt * ratio); break;
   }
   out->backend_index = be;
@@ -1312,6 +1390,11 @@ static int attn_bwd_impl(const fa_bwd_params* p_in, int32_t params_version, void
     // (single kernels, for timing, run uncut)
     DkdvParts parts{1, 1, 0};
     if (kernel_slot < 0 && !own_delta) parts = dkdv_parts(p, s, dev->num_cu);
+    const BwdRoute route = bwd_route(p, s, dev->num_cu);
+    if (route.recompute && kernel_slot < 0) {
+      need = 0;
+      parts = DkdvParts{1, 1, 0};
+    }
     // a nested call: the caller holds the buffer and has set a part of it aside
     const bool nested = t_ws_nested.active;
     int64_t bytes = fit_workspace(nested ? (int64_t)t_ws_nested.bytes : limit, &need, &parts);
@@ -1341,6 +1424,10 @@ static int attn_bwd_impl(const fa_bwd_params* p_in, int32_t params_version, void
       a.part_ws = reinterpret_cast<float*>(static_cast<char*>(ws) + need);
     }
     auto run_dkdv = [&]() {
+      if (route.wide_dkdv && !cut && a.ds_ws == nullptr) {
+        a.walk_group = route.group_dkdv;
+        return fa::run_bwd_dkdv_wide(dt, a, s.windowed, stream);
+      }
       return (cut ? fa::run_bwd_dkdv_parts : fa::run_bwd_dkdv)(dt, s.d, a, s.windowed, s.bias, s.dropout, stream);
     };
     if (ds_slot >= 0 && ds_ws == nullptr) {
@@ -1369,9 +1456,13 @@ static int attn_bwd_impl(const fa_bwd_params* p_in, int32_t params_version, void
         err = (rows32 ? fa::run_bwd_f32_rows : fa::run_bwd_f32)(s.d, slot, a, s.windowed, s.bias, s.dropout, stream);
       else if (big)
         err = fa::run_bwd_d512(dt, slot, a, s.windowed, s.bias, s.dropout, stream);
-      else
-        err = slot == 1 ? run_dkdv()
-                        : fa::run_bwd_dq(dt, s.d, a, s.windowed, s.bias, s.dropout, stream);
+      else if (slot == 1)
+        err = run_dkdv();
+      else if (route.wide_dq) {
+        a.walk_group = route.group_dq;
+        err = fa::run_bwd_dq_wide(dt, a, s.windowed, stream);
+      } else
+        err = fa::run_bwd_dq(dt, s.d, a, s.windowed, s.bias, s.dropout, stream);
     }
     if (held) ws_release(device_index(dev), stream);
     if (acquired && lazy->dispose != nullptr) lazy->dispose(lazy);   // attn_bwd.cc:157

@@ -29,6 +29,27 @@ inline int tile_workers(int items_per_xcd, int num_cu, int per_cu) {
   return w > items_per_xcd ? items_per_xcd : w;
 }
 
+// What the busiest worker of an XCD with the full number of pairs has to do in the persistent walk (worker_pos, one
+// workgroup per CU): cost[t] is that of the t-th tile of a pair in the walk's order.
+inline double walk_time(const TileWork& w, const float* cost, int tiles, int num_cu) {
+  const int workers = tile_workers(w.items_per_xcd, num_cu, 1);
+  double sum = 0, most = 0;
+  if (workers > 64 || w.items_per_xcd > 8192) {      // one item per worker, or so many that they balance
+    for (int t = 0; t < tiles; ++t) { sum += cost[t]; most = cost[t] > most ? cost[t] : most; }
+    sum = sum * w.zh_per_xcd / (workers > 0 ? workers : 1);
+    return sum > most ? sum : most;
+  }
+  double load[64] = {};
+  int pos = 0;
+  for (int first = 0; first < w.zh_per_xcd; first += w.zh_group)
+    for (int t = 0; t < tiles; ++t)
+      for (int i = 0; i < w.zh_group; ++i, ++pos)
+        if (first + i < w.zh_per_xcd && first + i < w.num_zh)
+          load[pos / workers & 1 ? workers - 1 - pos % workers : pos % workers] += cost[t];
+  for (int p = 0; p < workers; ++p) most = load[p] > most ? load[p] : most;
+  return most;
+}
+
 // Workgroups per XCD of the dK/dV and dQ kernels: one per CU (two: kTwoWaves), at most one per item.  With a
 // bias the kernels get one workgroup per item instead (the loop of a workgroup then runs
 // once): measured at B2 H16 S8192 D256 with window, bias, dB and dropout the persistent
@@ -120,6 +141,7 @@ struct BwdArgs {
   int32_t zh_group;      // heads walked together on one XCD
   int32_t num_cu;        // CUs of the device (host fills it in)
   int32_t items_per_xcd; // work items (incl. padding of the last group) per XCD
+  int32_t walk_group;    // the wide kernels' zh_group, chosen by the host (bwd_route)
   // dS kept in HBM between the dK/dV kernel (writes it) and the dQ kernel that only does dQ = dS K:
   // tiles of 128 keys x (the dK/dV step's queries), ds_ntk x ds_ntq of them per (batch element, q-head)
   void* ds_ws;           // null: dS is not stored

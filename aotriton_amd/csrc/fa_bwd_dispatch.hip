@@ -32,6 +32,19 @@ FA_DECL(run_bwd_dq, cols96)
 FA_DECL(run_bwd_fused, padded)
 #undef FA_DECL
 
+#define FA_DECL_WIDE(name)                                                                    \
+  hipError_t name##_d128(int, const BwdArgs&, bool, hipStream_t);                             \
+  hipError_t name##_d128_padded(int, const BwdArgs&, bool, hipStream_t);                      \
+  hipError_t name##_d128_cols96(int, const BwdArgs&, bool, hipStream_t);                      \
+  hipError_t name(int dtype, const BwdArgs& a, bool w, hipStream_t s) {                       \
+    if (a.head_dim == 128 && a.head_dim_v == 128) return name##_d128(dtype, a, w, s);         \
+    const bool upto96 = a.head_dim <= 96 && a.head_dim_v <= 96;                               \
+    return upto96 ? name##_d128_cols96(dtype, a, w, s) : name##_d128_padded(dtype, a, w, s);  \
+  }
+FA_DECL_WIDE(run_bwd_dkdv_wide)
+FA_DECL_WIDE(run_bwd_dq_wide)
+#undef FA_DECL_WIDE
+
 hipError_t run_bwd_preprocess(int dtype, int head_dim, const BwdArgs& a, hipStream_t s) {
   const bool bf = dtype == kDtypeBF16;
   switch (head_dim) {

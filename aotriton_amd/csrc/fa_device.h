@@ -178,6 +178,15 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t wave_rsrc(P* base, int bytes) 
                                            __builtin_amdgcn_readfirstlane(bytes), 0x00020000);
 }
 
+// The same descriptor as four words, for buffer instructions written as asm.
+template <typename P>
+__device__ __forceinline__ u32x4_t wave_rsrc_words(P* base, int bytes) {
+  const uint64_t a = reinterpret_cast<uint64_t>(base);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a), hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+  const uint32_t n = __builtin_amdgcn_readfirstlane(bytes);
+  return u32x4_t{lo, hi, n, 0x00020000u};
+}
+
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float fast_log2(float x) { return __builtin_amdgcn_logf(x); }
 

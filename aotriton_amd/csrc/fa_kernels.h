@@ -45,6 +45,10 @@ hipError_t run_bwd_dkdv(int dtype, int head_dim, const BwdArgs& a, bool windowed
 // the same with the items cut into parts and a kernel behind it that adds the parts up (BwdArgs::part_ws)
 hipError_t run_bwd_dkdv_parts(int dtype, int head_dim, const BwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
 hipError_t run_bwd_dq(int dtype, int head_dim, const BwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
+// head dims above 64 and up to 128 without bias and dropout: 64 rows per wave (fa_bwd_wide.h)
+hipError_t run_bwd_dkdv_wide(int dtype, const BwdArgs& a, bool windowed, hipStream_t s);
+hipError_t run_bwd_dq_wide(int dtype, const BwdArgs& a, bool windowed, hipStream_t s);
+TileShape bwd_wide_shape(bool dkdv);
 hipError_t run_bwd_fused(int dtype, int head_dim, const BwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
 TileShape bwd_tile_shape(int dtype, int head_dim, bool windowed, bool bias, bool dropout, int kernel_slot);
 // dQ = dS K from the dS tiles that the dK/dV kernel stored (BwdArgs::ds_ws), and their geometry

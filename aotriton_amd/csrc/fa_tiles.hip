@@ -1,7 +1,7 @@
 // Compile-time tile/occupancy table keyed on (element type, head dim, causal / windowed) and, where a kernel's
 // variants differ, on the options; reported through fa_query_*_config.
 #include "fa_fwd_impl.h"
-#include "fa_bwd_impl.h"
+#include "fa_bwd_wide.h"
 #include "fa_kernels.h"
 
 namespace fa {
@@ -46,6 +46,10 @@ TileShape bwd_tile_shape(int dtype, int head_dim, bool windowed, bool bias, bool
     case 128: return bf ? bwd_shape_of<bf16_t, 128>(windowed, bias, dropout, slot) : bwd_shape_of<f16_t, 128>(windowed, bias, dropout, slot);
     default: return bf ? bwd_shape_of<bf16_t, 256>(windowed, bias, dropout, slot) : bwd_shape_of<f16_t, 256>(windowed, bias, dropout, slot);
   }
+}
+
+TileShape bwd_wide_shape(bool dkdv) {
+  return dkdv ? TileShape{kWideBM, kWideBN, 4, WideDkDvSmem::BYTES + kLevelBytes, 1} : TileShape{kWideBN, kWideBM, 4, WideDqSmem::BYTES + kLevelBytes, 1};
 }
 
 }  // namespace fa
