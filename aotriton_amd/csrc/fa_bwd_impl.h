@@ -141,9 +141,6 @@ template <typename T, int D, bool kWideTile> struct DsTile {
   static constexpr int piece(int kw, int t) { return (t >> 1) * QBLOCK_BYTES + kw * 2048 + (t & 1) * 1024; }
 };
 
-// n elements of vector work spread evenly behind g MFMAs: the first one behind MFMA i
-constexpr int first_of(int i, int n, int g) { return (i * n + g - 1) / g; }
-
 // ---------------------------------------------------------------------------
 // dK / dV work item
 // ---------------------------------------------------------------------------

@@ -19,34 +19,9 @@
 // product of the library reaches 1220-1270 on this card.  Spreading the vector work differently over the MFMAs is level.
 #pragma once
 #include "fa_bwd_impl.h"
+#include "fa_wide.h"
 
 namespace fa {
-
-// One MFMA onto an accumulator that stays in accumulation registers.  What the compiler sees to for its own MFMAs (its hazard
-// recognizer does not look into an asm statement) is arranged by the callers: the conversions that make a B operand are at
-// least two instructions back (s_nop where a phase begins; `build --scan` checks the compiler's output for it), and the
-// accumulators are touched by nothing else inside the loops and read behind acc_settle only.
-template <typename T> __device__ __forceinline__ void mfma_acc(f32x16& c, typename Traits<T>::op_t a, typename Traits<T>::op_t b);
-template <> __device__ __forceinline__ void mfma_acc<bf16_t>(f32x16& c, Traits<bf16_t>::op_t a, Traits<bf16_t>::op_t b) {
-  asm("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
-}
-template <> __device__ __forceinline__ void mfma_acc<f16_t>(f32x16& c, Traits<f16_t>::op_t a, Traits<f16_t>::op_t b) {
-  asm("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
-}
-
-// An accumulator of zeros, made by the matrix pipe as well (through vector registers it would take as many of those).
-template <typename T> __device__ __forceinline__ void acc_zero(f32x16& c) {
-  const u32x4_t z = {0, 0, 0, 0};
-  if constexpr (std::is_same<T, bf16_t>::value) asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %1, 0" : "=a"(c) : "v"(z));
-  else asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_f16 %0, %1, %1, 0" : "=a"(c) : "v"(z));
-}
-// Waits until the MFMAs have written the accumulators (16 passes and what the register file takes).
-template <int N> __device__ __forceinline__ void acc_settle(f32x16 (&x)[N], f32x16 (&y)[N]) {
-  if constexpr (N == 4)
-    asm volatile("s_nop 15\n\ts_nop 15" : "+a"(x[0]), "+a"(x[1]), "+a"(x[2]), "+a"(x[3]), "+a"(y[0]), "+a"(y[1]), "+a"(y[2]), "+a"(y[3]));
-  else
-    asm volatile("s_nop 15\n\ts_nop 15" : "+a"(x[0]), "+a"(x[1]), "+a"(x[2]), "+a"(y[0]), "+a"(y[1]), "+a"(y[2]));
-}
 
 constexpr int kWideBM = 32, kWideBN = 256;
 
@@ -59,20 +34,6 @@ struct WideDkDvSmem {
   static constexpr int BYTES = V_OFF + kWideBN * 256;
   static_assert(3 * STAGE_BYTES <= V_OFF, "three stages");
 };
-
-// A wave's 1 KB of a tile straight into LDS (64 lanes x 16 bytes at voff + soff, to lds + 16 lane).  The compiler's builtin
-// does the same but makes the first transposing LDS read behind it wait for it; here the tile's one wait is placed by hand.
-__device__ __forceinline__ void load_to_lds(u32x4_t rsrc, int voff, int soff, int lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               :: "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "m0");
-}
-template <typename V> __device__ __forceinline__ V lds_read(int at) {
-  return *reinterpret_cast<__attribute__((address_space(3))) const V*>(at);
-}
-__device__ __forceinline__ tr_raw_t lds_read_tr_at(int at) {
-  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<__attribute__((address_space(3))) tr_raw_t*>(at));
-}
-__device__ __forceinline__ int lds_offset(const void* p) { return (int)(uintptr_t)(__attribute__((address_space(3))) const void*)p; }
 
 template <typename T, bool kWindowed, int kPad>
 __device__ __forceinline__ void dkdv_wide_item(const BwdArgs& a, const int hk, const int nt, const int z, char* smem_raw) {
@@ -90,7 +51,7 @@ __device__ __forceinline__ void dkdv_wide_item(const BwdArgs& a, const int hk, c
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int d_qk = kPad ? a.head_dim : D, d_v = kPad ? a.head_dim_v : D;
 
-  const SeqInfo si = get_seq(a.seq, z);
+  const SeqInfo si = uniform(get_seq(a.seq, z));
   const int n0 = nt * BN;
   if (n0 >= si.seqlen_k) return;
 
@@ -151,8 +112,8 @@ __device__ __forceinline__ void dkdv_wide_item(const BwdArgs& a, const int hk, c
   }
 
   // ---- staging ----------------------------------------------------------------------------
-  // Tiles of 32 queries, from the last one down: under a causal mask the items of a head that run side by side then read the
-  // same tiles at the same time (from the first one up each starts at its own diagonal).  Three stages: while a tile is worked on, the next one lands and the one after it is requested
+  // Tiles of 32 queries.  (From the last one down, which would let the items of a head that run side by side under a causal
+  // mask read the same tiles at the same time, 0-1 % faster; up, sums and results are those of the 128-row kernel.)  Three stages: while a tile is worked on, the next one lands and the one after it is requested
   // (behind the barrier in the middle of the tile, where every wave has left the tile before).
   const int smem0 = lds_offset(smem_raw);
   const int r0 = tid / 16, gch = ch ^ Swz<D>::f(r0);      // row of a tile and 16-byte chunk this lane fetches; rows r0 + 16 too
@@ -167,12 +128,12 @@ __device__ __forceinline__ void dkdv_wide_item(const BwdArgs& a, const int hk, c
   float st_val = 0.f;
   auto set_head = [&]() __attribute__((always_inline)) {
     const int hq = hk * group + f_g;
-    const int64_t row0 = (int64_t)si.q_start + (int64_t)br.hi * BM;
+    const int64_t row0 = (int64_t)si.q_start + (int64_t)br.lo * BM;
     qb = reinterpret_cast<const T*>(a.q) + (int64_t)si.batch_index * a.sq.z + (int64_t)hq * a.sq.h + row0 * a.sq.s;
     dob = reinterpret_cast<const T*>(a.dout) + (int64_t)si.batch_index * a.sdo.z + (int64_t)hq * a.sdo.h + row0 * a.sdo.s;
     st_b = (hi ? a.delta : a.lse) + lse_offset(si, hq, a.hq);
     f_e = ntq;
-    f_m = br.hi * BM;
+    f_m = br.lo * BM;
   };
   u32x4_t q_rs, do_rs;
   auto fetch_begin = [&]() __attribute__((always_inline)) {
@@ -182,7 +143,7 @@ __device__ __forceinline__ void dkdv_wide_item(const BwdArgs& a, const int hk, c
     do_rs = wave_rsrc_words(dob, max(rows * do_row - do_gap, 0));
     // (every wave reads and stores the row statistics: a branch for one of them would split the tile's code into blocks,
     // between which the compiler moves the work that is placed behind the MFMAs)
-    st_val = st_b[max(min(f_m + c, si.seqlen_q - 1), 0)];      // (below the first tile once nothing is left to fetch)
+    st_val = st_b[min(f_m + c, si.seqlen_q - 1)];
   };
   auto fetch_piece = [&](int stage, int i) __attribute__((always_inline)) {
     const int lds = smem0 + stage + wave * 4 * ROWB + (i & 1) * 16 * ROWB;
@@ -190,8 +151,8 @@ __device__ __forceinline__ void dkdv_wide_item(const BwdArgs& a, const int hk, c
     else load_to_lds(do_rs, do_voff, (i & 1) * 16 * do_row, lds + SM::TILE_BYTES);
   };
   auto fetch_end = [&]() __attribute__((always_inline)) {
-    qb -= (int64_t)BM * a.sq.s; dob -= (int64_t)BM * a.sdo.s;
-    f_m -= BM;
+    qb += (int64_t)BM * a.sq.s; dob += (int64_t)BM * a.sdo.s;
+    f_m += BM;
     if (--f_e == 0 && ++f_g < group) set_head();
   };
   auto fetch_all = [&](int stage) __attribute__((always_inline)) {
@@ -308,7 +269,7 @@ __device__ __forceinline__ void dkdv_wide_item(const BwdArgs& a, const int hk, c
 #pragma unroll
     for (int b = 0; b < KB; ++b) q_d[b] = q_none[b] ? 0x40000000u : (unsigned)(m0 + 4 * hi - q_lo[b]);
     // elements in the order rows 4 q .. 4 q + 3 of key block 0, then of block 1 (the statistics serve both)
-    auto p_el = [&](int E) __attribute__((always_inline)) {
+    auto exponent = [&](int E) __attribute__((always_inline)) {
       const int q = E / 8, b = (E / 4) % 2, r = E % 4, i = 4 * q + r;
       if (E % 8 == 0 && q < 3) l4[(q + 1) & 1] = l_read(q + 1);
       float x = __builtin_fmaf(s[b][i], qk_scale, l4[q & 1][r]);
@@ -316,7 +277,11 @@ __device__ __forceinline__ void dkdv_wide_item(const BwdArgs& a, const int hk, c
         const bool vis = q_d[b] + (unsigned)(8 * q + r) <= q_rng[b];
         x = vis ? x : -__builtin_inff();
       }
-      s[b][i] = fast_exp2(x);
+      s[b][i] = x;
+    };
+    auto power = [&](int E) __attribute__((always_inline)) {
+      const int b = (E / 4) % 2, i = 4 * (E / 8) + E % 4;
+      s[b][i] = fast_exp2(s[b][i]);
     };
     auto p_pair = [&](int E) __attribute__((always_inline)) {      // E odd
       const int q = E / 8, b = (E / 4) % 2, r = E % 4, i = 4 * q + r;
@@ -325,13 +290,14 @@ __device__ __forceinline__ void dkdv_wide_item(const BwdArgs& a, const int hk, c
       pb[b][i / 8][i % 8] = p2[1];
     };
     auto ds_el = [&](int E) __attribute__((always_inline)) {
-      const int q = E / 8, b = (E / 4) % 2, r = E % 4, i = 4 * q + r;
+      const int b = (E / 4) % 2, i = 4 * (E / 8) + E % 4;
       dp[b][i] = s[b][i] * dp[b][i];      // (dP started at -delta)
-      if (E & 1) {
-        const typename Tr::p2_t s2 = Tr::cvt2(dp[b][i - 1], dp[b][i]);
-        sb[b][i / 8][i % 8 - 1] = s2[0];
-        sb[b][i / 8][i % 8] = s2[1];
-      }
+    };
+    auto ds_pair = [&](int E) __attribute__((always_inline)) {      // E odd
+      const int b = (E / 4) % 2, i = 4 * (E / 8) + E % 4;
+      const typename Tr::p2_t s2 = Tr::cvt2(dp[b][i - 1], dp[b][i]);
+      sb[b][i / 8][i % 8 - 1] = s2[0];
+      sb[b][i / 8][i % 8] = s2[1];
     };
     // one ring of transposed operands runs through dV and dK
     constexpr int G3 = TS * DB, kRing = 4;
@@ -343,7 +309,7 @@ __device__ __forceinline__ void dkdv_wide_item(const BwdArgs& a, const int hk, c
       return __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7);
     };
 
-    // ---- dP = dO V^T, with p behind its MFMAs (the conversions one step behind the exponentials)
+    // ---- dP = dO V^T, with p behind its MFMAs
     op_t vl[2];
     vl[0] = swz_read_row<T, D>(Vt, row_a, 0, 1);
 #pragma unroll
@@ -358,16 +324,17 @@ __device__ __forceinline__ void dkdv_wide_item(const BwdArgs& a, const int hk, c
       for (int b = 0; b < KB; ++b) {
         dp[b] = Tr::mfma(xa[(KS + k) % 3], b == 0 ? vreg[k] : vl[k % 2], k == 0 ? nd : dp[b]);
         const int gi = k * KB + b;
-        const int E0 = first_of(gi, 32, KS * KB), E1 = first_of(gi + 1, 32, KS * KB);
+        // (the three parts of an element one after the other behind different MFMAs: none waits for the one before)
+        const int E0 = first_of(gi, 34, KS * KB), E1 = first_of(gi + 1, 34, KS * KB);
 #pragma unroll
         for (int E = E0; E < E1; ++E) {
-          p_el(E);
+          if (E < 32) exponent(E);
+          if (E >= 1 && E <= 32) power(E - 1);
           if (E >= 2 && (E & 1)) p_pair(E - 2);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
     }
-    p_pair(31);
 #pragma unroll
     for (int b = 0; b < KB; ++b)
 #pragma unroll
@@ -387,7 +354,10 @@ __device__ __forceinline__ void dkdv_wide_item(const BwdArgs& a, const int hk, c
         if (gi == 0) fetch_begin();
         if (gi >= 1 && gi <= 4) fetch_piece(st_fetch, gi - 1);
 #pragma unroll
-        for (int E = first_of(gi, 32, G3 * KB); E < first_of(gi + 1, 32, G3 * KB); ++E) ds_el(E);
+        for (int E = first_of(gi, 34, G3 * KB); E < first_of(gi + 1, 34, G3 * KB); ++E) {
+          if (E < 32) ds_el(E);
+          if (E >= 2 && (E & 1)) ds_pair(E - 2);
+        }
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -419,12 +389,12 @@ __device__ __forceinline__ void dkdv_wide_item(const BwdArgs& a, const int hk, c
     prefetch();
   };
   for (int g = 0; g < group; ++g) {
-    int e = ntq;
-    for (; e > e_end; --e) skip();
-    for (; e > f_end; --e) { compute(std::true_type{}, e - 1); fetch_end(); }
-    for (; e > f_lo; --e) { compute(std::false_type{}, e - 1); fetch_end(); }
-    for (; e > e_lo; --e) { compute(std::true_type{}, e - 1); fetch_end(); }
-    for (; e > 0; --e) skip();
+    int e = 0;
+    for (; e < e_lo; ++e) skip();
+    for (; e < f_lo; ++e) { compute(std::true_type{}, e); fetch_end(); }
+    for (; e < f_end; ++e) { compute(std::false_type{}, e); fetch_end(); }
+    for (; e < e_end; ++e) { compute(std::true_type{}, e); fetch_end(); }
+    for (; e < ntq; ++e) skip();
   }
   // (fetches past the last tile write zeros into stages nobody reads, but before the next item's stages are filled)
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -511,7 +481,7 @@ __device__ __forceinline__ void dq_wide_item(const BwdArgs& a, const int h, cons
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int d_qk = kPad ? a.head_dim : D, d_v = kPad ? a.head_dim_v : D;
 
-  const SeqInfo si = get_seq(a.seq, z);
+  const SeqInfo si = uniform(get_seq(a.seq, z));
   const int q0 = mt * BM;
   if (q0 >= si.seqlen_q) return;
 

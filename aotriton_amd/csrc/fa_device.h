@@ -187,6 +187,9 @@ __device__ __forceinline__ u32x4_t wave_rsrc_words(P* base, int bytes) {
   return u32x4_t{lo, hi, n, 0x00020000u};
 }
 
+// n elements of vector work spread evenly behind g MFMAs: the first one behind MFMA i
+constexpr int first_of(int i, int n, int g) { return (i * n + g - 1) / g; }
+
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float fast_log2(float x) { return __builtin_amdgcn_logf(x); }
 
