@@ -669,6 +669,36 @@ bool fwd_half_tiles(int dtype, const Shape& s, int num_cu) {
   return whole * 8 > half * 9;
 }
 
+// The kernel with 64 rows per wave (fa_fwd_wide.h; 16-bit types, head dims above 64 and up to 128, no bias, no dropout, a
+// positive scale) for these 256-row tiles?  It takes a tile of 64 keys in 5-7 % less time and an item costs it 1.5-2.5 us
+// more at its ends, where the two waves per SIMD of the other kernel cover for each other.  Measured (bf16, D128, us, other
+// -> this kernel): B4 H16 S4096 causal 270 -> 255, full 485 -> 456, 1024 queries of 16384 keys Hq 32 Hk 8 262 -> 248, B4 H16 S1536
+// causal 81 -> 79; left alone B16 H16 S2048 causal 291 / 299 (17 tiles an item, four rounds), S1024 full 277 / 280, B4 H16 S2048
+// window 256 46 / 48.  The lines: 20 key tiles per item on average, or 10 where the items go in at most two rounds.
+// Packed sequences stand for as many of their average length.
+bool fwd_wide(const fa_fwd_params* p, const Shape& s, int splits, int num_cu) {
+  if (s.elementwise || !is_16bit(p->Q.dtype) || s.d != 128 || s.bias || s.dropout || !(p->Sm_scale > 0.f) || s.max_sq <= 0 ||
+      s.max_sk <= 0 || s.batch <= 0)
+    return false;
+  const int64_t nz = s.num_seqlens != 0 ? std::abs(s.num_seqlens) : s.batch;
+  int sq = s.max_sq, sk = s.max_sk;
+  if (s.num_seqlens > 0) {
+    sq = std::max(1, std::min(sq, (int)(p->Q.sizes[2] / nz)));
+    sk = std::max(1, std::min(sk, (int)(p->K.sizes[2] / nz)));
+  }
+  const int m_tiles = (sq + 255) / 256;
+  int64_t sum = 0;
+  fa::Window w{0, 0};
+  if (s.windowed) w = fa::parse_window(p->causal_type, p->window_left, p->window_right, sq, sk);
+  for (int mt = 0; mt < m_tiles; ++mt) {
+    const fa::BlockRanges b = fa::block_ranges(s.windowed, w.left, w.right, mt * 256, sq, sk, 256, 64);
+    sum += b.hi - b.lo + 1;
+  }
+  const int64_t cus = num_cu >= fa::kNumXcd ? num_cu / fa::kNumXcd : 1;
+  const int64_t rounds = ((nz * s.hq + fa::kNumXcd - 1) / fa::kNumXcd * m_tiles * splits + cus - 1) / cus;
+  return sum >= (rounds <= 2 ? 10 : 20) * (int64_t)m_tiles * splits;
+}
+
 hipError_t run_fwd_rows(int dtype, int d, const fa::FwdArgs& a, const Shape& s, hipStream_t stream) {
   const bool padded = a.head_dim != d || a.head_dim_v != d;
   switch (d) {
@@ -944,10 +974,12 @@ int fa_query_fwd_config(const fa_fwd_params* params, int32_t num_cu, fa_kernel_c
   const FwdPlan plan = fwd_plan(params->Q.dtype, s, params->causal_type, params->window_left, params->window_right, cus);
   const bool split = !plan.rows && plan.splits > 1;
   const bool half = !split && fwd_half_tiles(params->Q.dtype, s, cus);
+  const bool wide = !plan.rows && !half && fwd_wide(params, s, split ? plan.splits : 1, cus);
   const fa::TileShape t = s.elementwise ? fa::TileShape{32, 1, 4, 0}
                           : rows32 ? fa::f32_rows_tile_shape(s.d)
                           : params->Q.dtype == FA_DTYPE_FLOAT32 ? fa::f32_tile_shape(s.d, -1)
                           : s.d > 256 ? fa::d512_tile_shape(-1)
+                          : wide ? fa::fwd_wide_shape()
                                       : fa::fwd_tile_shape(params->Q.dtype, s.d, s.windowed, half);
   out->block_m = t.block_m; out->block_n = t.block_n; out->num_waves = t.num_waves;
   out->lds_bytes = t.lds_bytes;
@@ -1158,11 +1190,14 @@ static int attn_fwd_impl(const fa_fwd_params* p, int32_t params_version, void* h
   }
   a.splits = scratch != nullptr ? plan.splits : 1;
   if (a.splits <= 1 && !plan.rows) a.half_tiles = fwd_half_tiles(p->Q.dtype, s, dev->num_cu);
-  FA_LOG(4, "attn_fwd: D=%d windowed=%d bias=%d dropout=%d nseq=%d rows=%d splits=%d half_tiles=%d", s.d, (int)s.windowed,
-         (int)s.bias, (int)s.dropout, s.num_seqlens, (int)plan.rows, a.splits, a.half_tiles);
+  const bool wide = !plan.rows && !a.half_tiles && fwd_wide(p, s, a.splits, dev->num_cu);
+  FA_LOG(4, "attn_fwd: D=%d windowed=%d bias=%d dropout=%d nseq=%d rows=%d splits=%d half_tiles=%d wide=%d", s.d, (int)s.windowed,
+         (int)s.bias, (int)s.dropout, s.num_seqlens, (int)plan.rows, a.splits, a.half_tiles, (int)wide);
   if (plan.rows) {
     a.row_blocks = plan.row_blocks; a.part_rows = plan.part_rows;
     err = run_fwd_rows(p->Q.dtype, s.d, a, s, stream);
+  } else if (wide) {
+    err = fa::run_fwd_wide(p->Q.dtype, a, s.windowed, stream);
   } else {
     err = run_fwd(p->Q.dtype, s.d, a, s, stream);
   }

@@ -21,6 +21,15 @@ hipError_t run_fwd_d128_padded(int dtype, const FwdArgs& a, bool windowed, bool 
 // full, backward 1726 -> 1572 causal; with dropout, bound by the vector ALU, 2 %).  Same sums: what is left out is zero.
 hipError_t run_fwd_d128_cols96(int dtype, const FwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
 hipError_t run_fwd_d256_padded(int dtype, const FwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
+// head dims above 64 and up to 128 without bias and dropout, a positive scale: 64 rows per wave (fa_fwd_wide.h)
+hipError_t run_fwd_wide_d128(int dtype, const FwdArgs& a, bool windowed, hipStream_t s);
+hipError_t run_fwd_wide_d128_padded(int dtype, const FwdArgs& a, bool windowed, hipStream_t s);
+hipError_t run_fwd_wide_d128_cols96(int dtype, const FwdArgs& a, bool windowed, hipStream_t s);
+inline hipError_t run_fwd_wide(int dtype, const FwdArgs& a, bool windowed, hipStream_t s) {
+  if (a.head_dim == 128 && a.head_dim_v == 128) return run_fwd_wide_d128(dtype, a, windowed, s);
+  return (a.head_dim <= 96 && a.head_dim_v <= 96 ? run_fwd_wide_d128_cols96 : run_fwd_wide_d128_padded)(dtype, a, windowed, s);
+}
+TileShape fwd_wide_shape();
 // few query rows per K/V head: packed rows of a GQA group, keys split over workgroups (fa_fwd_rows.h)
 hipError_t run_fwd_rows_d64(int dtype, const FwdArgs& a, bool windowed, bool bias, hipStream_t s);
 hipError_t run_fwd_rows_d128(int dtype, const FwdArgs& a, bool windowed, bool bias, hipStream_t s);

@@ -2,6 +2,7 @@
 // variants differ, on the options; reported through fa_query_*_config.
 #include "fa_fwd_impl.h"
 #include "fa_bwd_wide.h"
+#include "fa_fwd_wide.h"
 #include "fa_kernels.h"
 
 namespace fa {
@@ -47,6 +48,8 @@ TileShape bwd_tile_shape(int dtype, int head_dim, bool windowed, bool bias, bool
     default: return bf ? bwd_shape_of<bf16_t, 256>(windowed, bias, dropout, slot) : bwd_shape_of<f16_t, 256>(windowed, bias, dropout, slot);
   }
 }
+
+TileShape fwd_wide_shape() { return TileShape{256, 64, 4, WideFwdSmem::BYTES + kLevelBytes, 1}; }
 
 TileShape bwd_wide_shape(bool dkdv) {
   return dkdv ? TileShape{kWideBM, kWideBN, 4, WideDkDvSmem::BYTES + kLevelBytes, 1} : TileShape{kWideBN, kWideBM, 4, WideDqSmem::BYTES + kLevelBytes, 1};
