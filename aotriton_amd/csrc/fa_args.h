@@ -147,8 +147,8 @@ struct BwdArgs {
   void* ds_ws;           // null: dS is not stored
   int32_t ds_ntq, ds_ntk;
   // with ds_ws: row statistics as that dK/dV kernel stages them, written by the delta kernel
-  const float* lse_scaled;   // L / ln 2
-  const float* delta_prep;   // -delta (delta with dropout)
+  const float* lse_scaled;   // L / ln 2 (with dropout: minus log2 of its scale)
+  const float* delta_prep;   // -delta (with dropout: times 1 - p)
   // dK/dV items cut into parts (few keys, many queries or q-heads): part_heads parts of the GQA group's
   // q-heads times part_tiles parts of the query tiles; each part's fp32 sums go to part_ws as
   // (sequence and kv-head, key tile, part, dK then dV, key, column), where a second kernel adds them up

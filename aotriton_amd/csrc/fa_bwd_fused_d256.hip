@@ -1,5 +1,5 @@
 // Backward fused kernel instantiations for head dim 256 (fp16 and bf16).
-#include "fa_bwd_impl.h"
+#include "fa_bwd_fused_impl.h"
 
 // Compiled twice: as is for tensors whose head dim is 256, and with FA_PADDED = the columns to compute for smaller
 // head dims (a multiple of 8), where the kernels mask the excess columns.

@@ -30,8 +30,7 @@ namespace fa {
 // delta = rowsum(O * dO) in fp32, same layout as LSE.
 // ---------------------------------------------------------------------------
 // kPrep: also writes what the dK/dV kernel that stores dS stages without touching it: L in base 2
-// (BwdArgs::lse_scaled) and the initial value of its dP accumulators (delta_prep: -delta, or delta
-// itself when dropout comes between dP and the subtraction).
+// (BwdArgs::lse_scaled) and -delta (delta_prep), with dropout in the form that DropoutFold describes.
 template <typename T, int D, bool kPrep = false>
 __global__ void bwd_preprocess_kernel(const BwdArgs a) {
   using op_t = typename Traits<T>::op_t;
@@ -58,8 +57,9 @@ __global__ void bwd_preprocess_kernel(const BwdArgs a) {
     const int64_t at = lse_offset(si, h, a.hq) + row;
     a.delta[at] = acc;
     if constexpr (kPrep) {
-      const_cast<float*>(a.lse_scaled)[at] = a.lse[at] * kRcpLn2;          // bwd_inner_dk_dv.py:185-186
-      const_cast<float*>(a.delta_prep)[at] = a.drop.p > 0.f ? acc : -acc;
+      const DropoutFold f = dropout_fold(a.drop.p);
+      const_cast<float*>(a.lse_scaled)[at] = __builtin_fmaf(a.lse[at], kRcpLn2, -f.log2_scale);     // bwd_inner_dk_dv.py:185-186
+      const_cast<float*>(a.delta_prep)[at] = -acc * f.keep;
     }
   }
 }
@@ -146,8 +146,14 @@ template <typename T, int D, bool kWideTile> struct DsTile {
 // ---------------------------------------------------------------------------
 // kStoreDs: dS of every visited tile pair is also written to BwdArgs::ds_ws, and the row statistics
 // come prepared (BwdArgs::lse_scaled, delta_prep) so that they can travel straight into LDS.
-template <typename T, int D, int NW, int BM, bool kWindowed, bool kBias, bool kDropout, bool kInlineDelta, int kPad,
-          bool kStoreDs = false, bool kParts = false>
+// kBiasPlain: every row of the bias is whole aligned 16-byte pieces (plain_bias); the branches for other layouts, which sit
+// in the tile loop, and the registers that they hold go.  One wave per SIMD issues every instruction of its tile one after the
+// other, so what these kernels with bias or dropout take is counted in instructions: at B2 H16 S8192 D256 fp16, window 1024,
+// bias and dropout, a full tile's went from 1750 to 1090 (that flag; DropoutFold; no struct members in the loop, see
+// own_scalar; 16 spilled vector registers gone) and the kernel from 1.15 to 1.05 ms; B8 H12 S512 D64 bf16 with bias 50 -> 44 us,
+// B4 H16 1000 x 1531 D80 fp16 with dropout 195 -> 190 us.
+template <typename T, int D, int NW, int BM, bool kWindowed, bool kBias, bool kDropout, int kPad, bool kStoreDs = false,
+          bool kParts = false, bool kBiasPlain = false>
 __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const int nt, const int z, const int part,
                                           char* smem_raw) {
   using Tr = Traits<T>;
@@ -272,10 +278,9 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
   // anyway), and the pieces leave in the half tile after it, as their operands get complete: the
   // youngest store is more than half a tile old at the next wait.
   using DT = DsTile<T, D, kWide<D, kBias, kDropout>>;
-  static_assert(!kStoreDs || (!kInlineDelta && BM == DT::BM && BN == DT::BN), "stored tiles have the item's shape");
+  static_assert(!kStoreDs || (BM == DT::BM && BN == DT::BN), "stored tiles have the item's shape");
   const int ds_pos[2] = {((c << 1) | hi) << 4, (((c << 1) | hi) ^ 8) << 4};
   op_t sb[TS];                         // dS operands of the dK GEMM; with kStoreDs they outlive their tile
-  char* ds_tile = nullptr;             // stored tile of the running (q-head, Q tile) step
   constexpr int kDsSlots = 4;
   // cache policy bits of the stores: non-temporal (the tile is read once, by another kernel) at agent scope;
   // measured against the other combinations of sc0 / sc1 / nt on one box: 1-2 % of the kernel
@@ -309,67 +314,62 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
   // global side: the lane at chunk position p of row r fetches chunk p ^ f(r).  Lanes outside the
   // descriptor's range deliver zeros.  The pieces count in vmcnt like any load; the compiler makes
   // the first transposing LDS read after them wait for all of them (mid-tile: they have landed).
-  // The fused kernel computes delta from the staged O and dO registers and keeps them.
-  constexpr bool kDirect = !kInlineDelta;
   constexpr int RWI = 64 / LPR;                  // rows one wave instruction covers
-  op_t qch[kDirect ? 1 : CH], doch[kDirect ? 1 : CH], och[kInlineDelta ? CH : 1];
   float l_stage = 0.f, d_stage = 0.f;
   const int r0 = tid / LPR, cc0 = tid % LPR;
   int f_stage = 0;                               // stage the running fetch fills
   // f(r0 + k RPI) takes at most two values, for even and odd k (RPI is a multiple of 8, f has period 16)
   int q_voff_d[2] = {0, 0}, do_voff_d[2] = {0, 0};
-  if (kDirect) {
-    static_assert(!kDirect || RPI % 8 == 0, "the swizzle must repeat every two pieces");
+  static_assert(RPI % 8 == 0, "the swizzle must repeat every two pieces");
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const int gch = cc0 ^ Swz<D>::f(r0 + k * RPI);
-      q_voff_d[k] = gch * 8 < d_qk ? r0 * (int)a.sq.s * 2 + gch * 16 : kVoffOutOfRange;
-      do_voff_d[k] = gch * 8 < d_v ? r0 * (int)a.sdo.s * 2 + gch * 16 : kVoffOutOfRange;
-    }
+  for (int k = 0; k < 2; ++k) {
+    const int gch = cc0 ^ Swz<D>::f(r0 + k * RPI);
+    q_voff_d[k] = gch * 8 < d_qk ? r0 * (int)a.sq.s * 2 + gch * 16 : kVoffOutOfRange;
+    do_voff_d[k] = gch * 8 < d_v ? r0 * (int)a.sdo.s * 2 + gch * 16 : kVoffOutOfRange;
   }
   using lds_ptr_t = __attribute__((address_space(3))) void*;
-  const int q_voff = cc0 * 8 < d_qk ? r0 * (int)a.sq.s * 2 + cc0 * 16 : kVoffOutOfRange,       // bytes inside a tile
-            do_voff = cc0 * 8 < d_v ? r0 * (int)a.sdo.s * 2 + cc0 * 16 : kVoffOutOfRange,
-            o_voff = cc0 * 8 < d_v ? r0 * (int)a.so.s * 2 + cc0 * 16 : kVoffOutOfRange;
-  const int q_soff = RPI * (int)a.sq.s * 2, do_soff = RPI * (int)a.sdo.s * 2, o_soff = RPI * (int)a.so.s * 2;
-  int lds_off[CH];                                                        // bytes inside a tile
-#pragma unroll
-  for (int k = 0; k < CH; ++k) lds_off[k] = Swz<D>::addr(r0 + k * RPI, cc0);
+  // What a tile needs of the arguments sits in registers of its own: as members of the struct they are spilled and
+  // reloaded sixteen at a time, and one wave per SIMD issues those v_readlanes between its MFMAs.
+  const int q_row = own_scalar((int)a.sq.s * 2), do_row = own_scalar((int)a.sdo.s * 2), bias_row = kBias ? own_scalar((int)a.sb_m * 2) : 0;
+  const int q_soff = RPI * q_row, do_soff = RPI * do_row;
 
   // Tile base pointers advance incrementally (one 64-bit add per tensor and tile);
   // with one wave per SIMD a chain of scalar multiplies per tile is not hidden.
-  const int64_t q_tile_step = (int64_t)BM * a.sq.s, do_tile_step = (int64_t)BM * a.sdo.s,
-                o_tile_step = (int64_t)BM * a.so.s;
-  const T* qb = nullptr; const T* dob = nullptr; const T* ob = nullptr;
+  // A new q-head reads its arguments from the kernel's argument segment, through a pointer that the compiler
+  // cannot see through, so that they do not stay in registers over the tiles.
+  const char* qb = nullptr; const char* dob = nullptr; const char* bb = nullptr;
   const float* lse_b = nullptr; const float* delta_b = nullptr;
+  DropoutState dst{};      // of the running q-head (the fetches are a tile ahead)
+  char* ds_tile = nullptr;             // stored tile of the running (q-head, Q tile) step
   auto set_head = [&](int g) {
+    const KernelArgs<BwdArgs> k = kernel_args<BwdArgs>();
     const int hq = hk * group + g;
     const int64_t row0 = (int64_t)si.q_start + (int64_t)br.lo * BM;
-    qb = reinterpret_cast<const T*>(a.q) + (int64_t)si.batch_index * a.sq.z + (int64_t)hq * a.sq.h + row0 * a.sq.s;
-    dob = reinterpret_cast<const T*>(a.dout) + (int64_t)si.batch_index * a.sdo.z + (int64_t)hq * a.sdo.h +
-          row0 * a.sdo.s;
-    if (kInlineDelta)
-      ob = reinterpret_cast<const T*>(a.out) + (int64_t)si.batch_index * a.so.z + (int64_t)hq * a.so.h +
-           row0 * a.so.s;
-    lse_b = (kStoreDs ? a.lse_scaled : a.lse) + lse_offset(si, hq, a.hq) + (int64_t)br.lo * BM;
-    if (!kInlineDelta) delta_b = (kStoreDs ? a.delta_prep : a.delta) + lse_offset(si, hq, a.hq) + (int64_t)br.lo * BM;
+    qb = reinterpret_cast<const char*>(k->q) + ((int64_t)si.batch_index * k->sq.z + (int64_t)hq * k->sq.h + row0 * k->sq.s) * 2;
+    dob = reinterpret_cast<const char*>(k->dout) +
+          ((int64_t)si.batch_index * k->sdo.z + (int64_t)hq * k->sdo.h + row0 * k->sdo.s) * 2;
+    const int64_t stat0 = lse_offset(si, hq, k->hq) + (int64_t)br.lo * BM;
+    lse_b = (kStoreDs ? k->lse_scaled : k->lse) + stat0;
+    delta_b = (kStoreDs ? k->delta_prep : k->delta) + stat0;
+    if (kBias)
+      bb = reinterpret_cast<const char*>(k->bias) +
+           ((int64_t)si.batch_index * k->sb_z + (int64_t)hq * k->sb_h + (int64_t)br.lo * BM * k->sb_m + (int64_t)n0 * k->sb_n) * 2;
   };
-  __amdgpu_buffer_rsrc_t q_rs, do_rs, o_rs, b_rs;
+  __amdgpu_buffer_rsrc_t q_rs, do_rs, b_rs;
   // The bias tile (BM queries x the workgroup's 128 keys) is staged through LDS like Q
   // and dO when its layout allows 16-byte loads; otherwise elements are loaded directly.
   static_assert(BN == 128, "bias staging assumes 128 keys per workgroup");
   constexpr int CHB = kBias ? (BM * 16) / NT : 0;        // 16-byte bias pieces per thread
-  const bool bias_lds = kBias && a.sb_n == 1 && ((a.sb_m | a.sb_h | a.sb_z) & 7) == 0 &&
-                        (reinterpret_cast<uintptr_t>(a.bias) & 15) == 0;
+  const bool bias_lds = kBiasPlain || (kBias && a.sb_n == 1 && ((a.sb_m | a.sb_h | a.sb_z) & 7) == 0 &&
+                                       (reinterpret_cast<uintptr_t>(a.bias) & 15) == 0);
   op_t bch[CHB > 0 ? CHB : 1];
-  const int b_voff = (tid / 16) * (int)a.sb_m * 2 + (tid % 16) * 16;   // bytes inside a bias tile
-  const int b_soff = (NT / 16) * (int)a.sb_m * 2;
+  const int b_voff = (tid / 16) * bias_row + (tid % 16) * 16;   // bytes inside a bias tile
+  const int b_soff = (NT / 16) * bias_row;
   const int b_lds = (tid / 16) * SM::BIAS_STR + (tid % 16) * 16;
-  const T* bb = nullptr;
   const T* bb_tile = nullptr;     // bias tile being fetched, its valid rows
   int b_rows = 0;
   const int b_cols = si.seqlen_k - n0 < BN ? si.seqlen_k - n0 : BN;      // valid keys of this item
-  const bool bias_plain = bias_lds && (b_cols & 7) == 0;                 // no piece straddles the end of a row
+  const bool bias_plain = kBiasPlain || (bias_lds && (b_cols & 7) == 0);   // no piece straddles the end of a row
   // (g, e) = (q-head inside the GQA group, Q tile inside the range) of the tile to fetch;
   // called for consecutive tiles only; `live` false: nothing is fetched
   auto fetch_begin = [&](bool live, int g, int e) {
@@ -379,18 +379,13 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
     rows = live ? rows : 0;
     const bool any = rows > 0;
     if (kBias) {
-      if (live && e == 0)
-        bb = reinterpret_cast<const T*>(a.bias) + (int64_t)si.batch_index * a.sb_z +
-             (int64_t)(hk * group + g) * a.sb_h + (int64_t)br.lo * BM * a.sb_m + (int64_t)n0 * a.sb_n;
-      bb_tile = bb;
+      bb_tile = reinterpret_cast<const T*>(bb);
       b_rows = rows;
-      b_rs = wave_rsrc(bb, any && bias_lds ? ((rows - 1) * (int)a.sb_m + b_cols) * 2 : 0);
-      if (live) bb += (int64_t)BM * a.sb_m;
+      b_rs = wave_rsrc(bb, any && bias_lds ? (rows - 1) * bias_row + b_cols * 2 : 0);
+      if (live) bb += kBiasPlain ? BM * bias_row : (int64_t)BM * 2 * a.sb_m;
     }
-    q_rs = wave_rsrc(qb, any ? ((rows - 1) * (int)a.sq.s + d_qk) * 2 : 0);
-    do_rs = wave_rsrc(dob, any ? ((rows - 1) * (int)a.sdo.s + d_v) * 2 : 0);
-    if (kInlineDelta)
-      o_rs = wave_rsrc(ob, any ? ((rows - 1) * (int)a.so.s + d_v) * 2 : 0);
+    q_rs = wave_rsrc(qb, any ? (rows - 1) * q_row + d_qk * 2 : 0);
+    do_rs = wave_rsrc(dob, any ? (rows - 1) * do_row + d_v * 2 : 0);
     if constexpr (kStoreDs) {
       // the prepared statistics (L log2e; -delta, or delta with dropout) go straight into the stage:
       // no register load in the loop, hence no wait of the compiler's for one at the end of a tile
@@ -405,15 +400,14 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
     } else if (tid < BM) {
       const bool ok = tid < rows;
       l_stage = ok ? lse_b[tid] : 0.f;
-      if (!kInlineDelta) d_stage = ok ? delta_b[tid] : 0.f;
+      d_stage = ok ? delta_b[tid] : 0.f;
     }
     if (live) {
-      qb += q_tile_step; dob += do_tile_step; lse_b += BM;
-      if (kInlineDelta) ob += o_tile_step; else delta_b += BM;
+      qb += BM * q_row; dob += BM * do_row; lse_b += BM; delta_b += BM;
     }
   };
   constexpr int FETCH_PIECES = 2 * CH + CHB;
-  auto fetch_piece = [&](int i) {        // Q pieces first, then dO (and O), then bias
+  auto fetch_piece = [&](int i) {        // Q pieces first, then dO, then bias
     if (i >= 2 * CH) {
       const int k = i - 2 * CH;
       if (bias_plain) {
@@ -445,61 +439,31 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
         bch[k] = x;
       }
     } else if (i < CH) {
-      if constexpr (kDirect) {
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            q_rs, (lds_ptr_t)(stage_ptr(f_stage) + (i * RPI + RWI * wave_u) * Swz<D>::ROWB), 16, q_voff_d[i & 1],
-            i * q_soff, 0, 0);
-      } else {
-        qch[i] = __builtin_bit_cast(op_t, __builtin_amdgcn_raw_buffer_load_b128(q_rs, q_voff, i * q_soff, 0));
-      }
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          q_rs, (lds_ptr_t)(stage_ptr(f_stage) + (i * RPI + RWI * wave_u) * Swz<D>::ROWB), 16, q_voff_d[i & 1],
+          i * q_soff, 0, 0);
     } else {
       const int k = i - CH;
-      if constexpr (kDirect) {
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            do_rs, (lds_ptr_t)(stage_ptr(f_stage) + SM::TILE_BYTES + (k * RPI + RWI * wave_u) * Swz<D>::ROWB), 16,
-            do_voff_d[k & 1], k * do_soff, 0, 0);
-      } else {
-        doch[k] = __builtin_bit_cast(op_t, __builtin_amdgcn_raw_buffer_load_b128(do_rs, do_voff, k * do_soff, 0));
-      }
-      if (kInlineDelta)
-        och[k] = __builtin_bit_cast(op_t, __builtin_amdgcn_raw_buffer_load_b128(o_rs, o_voff, k * o_soff, 0));
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          do_rs, (lds_ptr_t)(stage_ptr(f_stage) + SM::TILE_BYTES + (k * RPI + RWI * wave_u) * Swz<D>::ROWB), 16,
+          do_voff_d[k & 1], k * do_soff, 0, 0);
     }
   };
   // all of this wave's direct pieces have landed (vmcnt 0; the other counters stay as they are)
-  auto direct_landed = [&]() {
-    if constexpr (kDirect) __builtin_amdgcn_s_waitcnt(0x0F70);
+  auto direct_landed = [&]() { __builtin_amdgcn_s_waitcnt(0x0F70); };
+  auto bias_store = [&](int k, int stage) {
+    *reinterpret_cast<op_t*>(stage_ptr(stage) + 2 * SM::TILE_BYTES + 2 * BM * 4 + b_lds + k * (NT / 16) * SM::BIAS_STR) = bch[k];
   };
-  constexpr int STORE_PIECES = 2 * CH + CHB;
-  auto store_piece = [&](int i, int stage) {   // same order as the fetches
-    char* sp = stage_ptr(stage);
-    if (i >= 2 * CH)
-      *reinterpret_cast<op_t*>(sp + 2 * SM::TILE_BYTES + 2 * BM * 4 + b_lds + (i - 2 * CH) * (NT / 16) * SM::BIAS_STR) =
-          bch[i - 2 * CH];
-    else if (kDirect) return;
-    else if (i < CH) *reinterpret_cast<op_t*>(sp + lds_off[i]) = qch[i];
-    else *reinterpret_cast<op_t*>(sp + SM::TILE_BYTES + lds_off[i - CH]) = doch[i - CH];
-  };
+  DropoutFold fold{};
+  if (kDropout) fold = dropout_fold(a.drop.p);
   auto store_stats = [&](int stage) {
     char* sp = stage_ptr(stage);
     float* Ls = reinterpret_cast<float*>(sp + 2 * SM::TILE_BYTES);
     float* Ds = Ls + BM;
-    if (kInlineDelta) {
-      // delta recomputed from O and dO (bwd_kernel_fuse.py:307-310); the LPR threads
-      // that share a row are consecutive lanes
-#pragma unroll
-      for (int k = 0; k < CH; ++k) {
-        float acc = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc += (float)och[k][e] * (float)doch[k][e];
-#pragma unroll
-        for (int off = LPR / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
-        if (cc0 == 0) Ds[r0 + k * RPI] = kDropout ? acc : -acc;
-      }
-    }
     if (!kStoreDs && tid < BM) {
-      Ls[tid] = l_stage * kRcpLn2;                          // bwd_inner_dk_dv.py:185-186
-      // without dropout -delta is staged: it is the initial value of the dP accumulators
-      if (!kInlineDelta) Ds[tid] = kDropout ? d_stage : -d_stage;
+      Ls[tid] = kDropout ? __builtin_fmaf(l_stage, kRcpLn2, -fold.log2_scale) : l_stage * kRcpLn2;     // bwd_inner_dk_dv.py:185-186
+      // (without dropout -delta is the initial value of the dP accumulators)
+      Ds[tid] = kDropout ? -d_stage * fold.keep : -d_stage;
     }
   };
 
@@ -508,10 +472,9 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
   if (kDropout) drop0 = make_dropout_base(a.drop, a.seq.max_seqlen_k);
 
   // ---- one (q-head, Q tile) step -----------------------------------------------
-  auto compute = [&](auto masked_tag, int g, int e, int stage, bool live, int g_nxt, int e_nxt) {
+  auto compute = [&](auto masked_tag, int e, int stage, bool live, int g_nxt, int e_nxt) {
     constexpr bool masked = decltype(masked_tag)::value;
     constexpr int G1 = KS * MB, G4 = TS * DB;
-    const int hq = hk * group + g;
     const int m0 = (br.lo + e) * BM;
     char* sp = stage_ptr(stage);
     const char* Qb = sp;
@@ -527,19 +490,10 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
     f32x16 s[MB], dp[MB];
     const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 
-    DropoutState dst{};
-    if (kDropout) dst = dropout_for_head(drop0, z, hq, a.hq, a.seq.max_seqlen_q);
-    if constexpr (kStoreDs) {
-      // (the tiles of a q-head follow each other)
-      ds_tile = e == 0 ? reinterpret_cast<char*>(a.ds_ws) +
-                             ((((int64_t)z * a.hq + hq) * a.ds_ntk + nt) * a.ds_ntq + br.lo) * DT::BYTES
-                       : ds_tile + DT::BYTES;
-    }
-
     // The vector ALU work is spread over the MFMAs of the GEMMs that do not depend on
     // it: p = exp2(...) of S runs behind the MFMAs of dP, ds = p (dP - delta) behind
     // those of dV.  Fences keep the hand-made order.
-    constexpr int kAhead = D >= 256 ? 1 : 2;
+    constexpr int kAhead = 2;      // (one at D = 256 left each read's latency behind a single MFMA: 2-5 % of the kernel)
     op_t xa[kAhead + 1][MB];
     op_t pb[TS];
     uint32_t kw[kDropout ? MB : 1][4];
@@ -618,23 +572,24 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
       }
     }
     const char* Vt = smem_raw + SM::V_OFF;
-    op_t vl[3];          // ring of V operands when they come from LDS
+    op_t vl[4];          // ring of V operands when they come from LDS
     if (kVLds) {
       vl[0] = swz_read_row<T, D>(Vt, row_a, 0, wave);
       vl[1] = swz_read_row<T, D>(Vt, row_a, 1, wave);
+      vl[2] = swz_read_row<T, D>(Vt, row_a, 2, wave);
     }
 
-    // element E = 16*mb + i of the tile: p (kept in s, undropped) and its operand form
+    // element E = 16*mb + i of the tile: p (kept in s, undropped, times the dropout scale) and its operand form
     const unsigned q_d = q_none ? 0x40000000u : (unsigned)(m0 + 4 * hi - q_lo);
     auto p_el = [&](int E) {
       const int mb = E / 16, i = E % 16, g = i / 4, r = i % 4;
       if (E % 4 == 0 && E + 4 < 16 * MB) l4[(E / 4 + 1) & 1] = *reinterpret_cast<const f32x4*>(stat_ptr(Ls, E / 4 + 1));
-      // p = exp2(s*c + bias*log2e - L*log2e), one fma per element (bwd_inner_dk_dv.py:187-188)
+      // p = exp2(s*c + (bias*log2e - L*log2e)) (bwd_inner_dk_dv.py:187-188)
       float x;
       if (kBias) {
         if (kBiasRing && E % 4 == 0 && E + 4 < 16 * MB) bias4[(E / 4 + 1) & 1] = bias_read(E / 4 + 1);
         const float bv = (float)bias4[kBiasRing ? (E / 4) & 1 : E / 4][r];
-        x = __builtin_fmaf(s[mb][i], qk_scale, bv * kLog2e) - l4[(E / 4) & 1][r];
+        x = __builtin_fmaf(s[mb][i], qk_scale, __builtin_fmaf(bv, kLog2e, -l4[(E / 4) & 1][r]));
       } else {
         x = __builtin_fmaf(s[mb][i], qk_scale, -l4[(E / 4) & 1][r]);
       }
@@ -664,8 +619,8 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
       if (kDropout) {
         keep_bit[E - 1] = keep_of(E - 1);
         keep_bit[E] = keep_of(E);
-        p0 = keep_bit[E - 1] ? p0 * dst.scale : 0.f;              // :200-201
-        p1 = keep_bit[E] ? p1 * dst.scale : 0.f;
+        p0 = keep_bit[E - 1] ? p0 : 0.f;              // :200-201 (the scale is in p)
+        p1 = keep_bit[E] ? p1 : 0.f;
       }
       const typename Tr::p2_t p2 = Tr::cvt2(p0, p1);     // p cast to dO's dtype (composed_tensors.py:191-193)
       pb[E / 8][E % 8 - 1] = p2[0];
@@ -678,9 +633,8 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
         return;
       }
       if (E % 4 == 0 && E + 4 < 16 * MB) d4[(E / 4 + 1) & 1] = *reinterpret_cast<const f32x4*>(stat_ptr(Ds, E / 4 + 1));
-      float dpv = dp[mb][i];
-      dpv = keep_bit[E] ? dpv * dst.scale : 0.f;                  // :239-240
-      dp[mb][i] = s[mb][i] * (dpv - d4[(E / 4) & 1][r]);          // ds uses the undropped p (:242)
+      const float dpv = keep_bit[E] ? dp[mb][i] : 0.f;            // :239-240
+      dp[mb][i] = s[mb][i] * (dpv + d4[(E / 4) & 1][r]);          // ds uses the undropped p (:242)
     };
     auto ds_pair = [&](int E) {  // E odd: ds cast to Q's dtype
       const typename Tr::p2_t s2 = Tr::cvt2(dp[E / 16][E % 16 - 1], dp[E / 16][E % 16]);
@@ -696,10 +650,10 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
         for (int mb = 0; mb < MB; ++mb)
           xa[(KS + k + kAhead) % (kAhead + 1)][mb] = swz_read_row<T, D>(dOb, row_a, k + kAhead, mb);
       }
-      if (kVLds && k + 2 < KS) vl[(k + 2) % 3] = swz_read_row<T, D>(Vt, row_a, k + 2, wave);
+      if (kVLds && k + 3 < KS) vl[(k + 3) % 4] = swz_read_row<T, D>(Vt, row_a, k + 3, wave);
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) {
-        dp[mb] = Tr::mfma(xa[(KS + k) % (kAhead + 1)][mb], kVLds ? vl[k % 3] : vreg[kVLds ? 0 : k],
+        dp[mb] = Tr::mfma(xa[(KS + k) % (kAhead + 1)][mb], kVLds ? vl[k % 4] : vreg[kVLds ? 0 : k],
                           k == 0 && kDropout ? zero16 : dp[mb]);
         const int gidx = k * MB + mb;
 #pragma unroll
@@ -718,9 +672,10 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
     // delta of the tile's queries, first transposed dO operands
     if (kDropout) d4[0] = *reinterpret_cast<const f32x4*>(stat_ptr(Ds, 0));
     // Transposed operands are read ahead of their MFMAs: a whole 16-query step ahead, or,
-    // where that would take too many registers (D = 256), through a ring of kRing operands.
+    // where that would take too many registers (D = 256), through a ring of kRing operands
+    // (4 instead of 6 cost 1-2 %; 8, with a V ring of 5, spills).
     constexpr bool kRingTa = DB >= 8;
-    constexpr int kRing = 4;
+    constexpr int kRing = 6;
     op_t ta[kRingTa ? 1 : 2][kRingTa ? kRing : DB];
     auto ta_read = [&](const char* tile, int gidx) { return swz_read_tr<T, D>(tile, tr_a0, tr_a1, gidx / DB, gidx % DB); };
     if (kRingTa) {
@@ -781,13 +736,9 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
           dk[db] = Tr::mfma(ta[t & 1 & (kRingTa ? 0 : 1)][db], sb[t], dk[db]);
         }
         if (kStoreDs && t * DB + db == 2) store_ds_slot(ds_tile, 3);
-        // the next tile's LDS writes ride behind these MFMAs
-        constexpr int per = (STORE_PIECES + G4 - 1) / G4;
-#pragma unroll
-        for (int q = 0; q < per; ++q) {
-          const int piece = (t * DB + db) * per + q;
-          if (piece < STORE_PIECES) store_piece(piece, stage ^ 1);
-        }
+        static_assert(CHB <= G4, "one piece per MFMA");
+        // the next tile's bias is written behind the last of these MFMAs
+        if (t * DB + db >= G4 - CHB) bias_store(t * DB + db - (G4 - CHB), stage ^ 1);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -814,7 +765,7 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
 #pragma unroll
   for (int i = 0; i < FETCH_PIECES; ++i) fetch_piece(i);
 #pragma unroll
-  for (int i = 0; i < STORE_PIECES; ++i) store_piece(i, 0);
+  for (int k = 0; k < CHB; ++k) bias_store(k, 0);
   store_stats(0);
   direct_landed();
   __syncthreads();
@@ -829,12 +780,20 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
     const int stage = it & 1;
     int g_nxt = g_cur, e_nxt = e_cur + 1;
     if (e_nxt == ntq) { e_nxt = 0; ++g_nxt; }
-    compute(masked_tag, g_cur, e_cur, stage, it + 1 < total, g_nxt, e_nxt);
+    compute(masked_tag, e_cur, stage, it + 1 < total, g_nxt, e_nxt);
     __syncthreads();
     ++it;
     g_cur = g_nxt; e_cur = e_nxt;
+    if constexpr (kStoreDs) ds_tile += DT::BYTES;      // (the tiles of a q-head follow each other)
   };
   for (int g = g_lo; g < g_hi; ++g) {
+    if (kDropout || kStoreDs) {
+      const KernelArgs<BwdArgs> k = kernel_args<BwdArgs>();
+      const int hq = hk * group + g;
+      if (kDropout) dst = dropout_for_head(drop0, z, hq, k->hq, k->seq.max_seqlen_q);
+      if constexpr (kStoreDs)
+        ds_tile = reinterpret_cast<char*>(k->ds_ws) + ((((int64_t)z * k->hq + hq) * k->ds_ntk + nt) * k->ds_ntq + br.lo) * DT::BYTES;
+    }
     for (int e = 0; e < n_lb; ++e) step(std::true_type{});
     for (int e = 0; e < n_fb; ++e) step(std::false_type{});
     for (int e = n_lb + n_fb; e < ntq; ++e) step(std::true_type{});
@@ -1410,7 +1369,7 @@ __host__ __device__ inline bool dkdv_level_list(const BwdArgs& a) {
 }
 
 template <typename T, int D, int NW, int BM, bool kWindowed, bool kBias, bool kDropout, int kPad, bool kStoreDs = false,
-          bool kParts = false>
+          bool kParts = false, bool kBiasPlain = false>
 __global__ __attribute__((amdgpu_flat_work_group_size(NW * 64, NW * 64))) __attribute__((amdgpu_waves_per_eu(kTwoWaves<D, kBias> ? 2 : 1, kTwoWaves<D, kBias> ? 2 : 1)))
 void bwd_dkdv_kernel(const BwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
@@ -1451,7 +1410,7 @@ void bwd_dkdv_kernel(const BwdArgs a) {
     }
     int z, hk;
     split_zh(zh, a.num_zh / a.hk, 1, z, hk);
-    dkdv_item<T, D, NW, BM, kWindowed, kBias, kDropout, false, kPad, kStoreDs, kParts>(a, hk, nt, z, kParts ? lp % parts : 0, smem_raw);
+    dkdv_item<T, D, NW, BM, kWindowed, kBias, kDropout, kPad, kStoreDs, kParts, kBiasPlain>(a, hk, nt, z, kParts ? lp % parts : 0, smem_raw);
     __syncthreads();     // the next item reuses the LDS stages
   }
 }
@@ -1476,43 +1435,6 @@ void bwd_dq_kernel(const BwdArgs a) {
     int z, h;
     split_zh(zh, a.num_zh / a.hq, a.hq / a.hk, z, h);
     dq_item<T, D, NW, BN, kWindowed, kBias, kDropout, true, kPad, true>(a, h, mt, z, smem_raw);
-    __syncthreads();     // the next item reuses the LDS stages
-  }
-}
-
-// Per (batch, kv-head): num_n_tiles dK/dV items followed by num_m_tiles*(Hq/Hk) dQ items
-// (modules/flash/csrc/attn_bwd_fused.cc:13-22, bwd_kernel_fuse.py:107-118), laid out on
-// the same 1-D grid as the split kernels: each XCD owns a contiguous range of (batch,
-// kv-head) pairs and walks them in pairs, so the tensors of the heads in flight stay in
-// that XCD's L2.
-template <typename T, int D, int NW, int BM, int BN, bool kWindowed, bool kBias, bool kDropout, int kPad>
-__global__ __attribute__((amdgpu_flat_work_group_size(NW * 64, NW * 64)))
-void bwd_fused_kernel(const BwdArgs a) {
-  extern __shared__ __attribute__((aligned(16))) char smem_raw[];
-  const int group = a.hq / a.hk;
-  const int items = a.num_n_tiles + a.num_m_tiles * group;
-  // persistent workgroups with the walk of the split kernels (one workgroup per item with a bias
-  // or at D = 256, where the loop runs once)
-  const int xcd = blockIdx.x % kNumXcd, p = blockIdx.x / kNumXcd, workers = gridDim.x / kNumXcd;
-  const int per_group = a.zh_group * items;
-  for (int r = 0; D >= 256 ? r < 1 : r * workers < a.items_per_xcd; ++r) {
-    const int li = r * workers + ((r & 1) ? workers - 1 - p : p);
-    if (li >= a.items_per_xcd) continue;
-    const int gi = li / per_group, gr = li % per_group;
-    const int zl = gi * a.zh_group + gr % a.zh_group;
-    const int zh = xcd * a.zh_per_xcd + zl;
-    if (zl >= a.zh_per_xcd || zh >= a.num_zh) continue;
-    int z, hk;
-    split_zh(zh, a.num_zh / a.hk, 1, z, hk);
-    const int item = gr / a.zh_group;
-    if (item < a.num_n_tiles) {
-      dkdv_item<T, D, NW, BM, kWindowed, kBias, kDropout, true, kPad>(a, hk, item, z, 0, smem_raw);
-    } else {
-      const int t = item - a.num_n_tiles;
-      const int h = hk * group + t / a.num_m_tiles;
-      const int mt = a.num_m_tiles - 1 - t % a.num_m_tiles;
-      dq_item<T, D, NW, BN, kWindowed, kBias, kDropout, true, kPad>(a, h, mt, z, smem_raw);
-    }
     __syncthreads();     // the next item reuses the LDS stages
   }
 }
@@ -1593,6 +1515,12 @@ static __global__ __launch_bounds__(256) void combine_dkdv_kernel(const BwdArgs 
   *reinterpret_cast<q4_t*>(out) = t4;
 }
 
+// Every row of the bias is whole 16-byte pieces at 16-byte boundaries, in every item.
+template <typename T> inline bool plain_bias(const BwdArgs& a) {
+  return a.seq.num_seqlens == 0 && a.seq.max_seqlen_k % 8 == 0 && a.sb_n == 1 && ((a.sb_m | a.sb_h | a.sb_z) & 7) == 0 &&
+         (reinterpret_cast<uintptr_t>(a.bias) & 15) == 0;
+}
+
 template <typename T, int D, int kPad, bool W, bool B, bool P, bool kParts>
 hipError_t launch_dkdv_variant(const BwdArgs& a0, hipStream_t stream) {
   using Tile = BwdTile<T, D, W>;
@@ -1603,6 +1531,9 @@ hipError_t launch_dkdv_variant(const BwdArgs& a0, hipStream_t stream) {
   dim3 grid((unsigned)(kNumXcd * bwd_workers(D, B, a.items_per_xcd, a.num_cu, kTwoWaves<D, B> ? 2 : 1)));
   // (the level table's LDS is requested whether or not this launch uses it: the kernel's limit is set once)
   constexpr int smem = DkDvSmem<D, BM>::BYTES + (D < 256 ? kLevelBytes : 0);
+  if constexpr (B && !kParts)
+    if (a.ds_ws != nullptr && plain_bias<T>(a))
+      return launch_with_lds<bwd_dkdv_kernel<T, D, NW, BM, W, B, P, kPad, true, false, true>>(grid, NW * 64, smem, stream, a);
   // (every build has the variant that stores dS; the host decides where it pays)
   hipError_t e = a.ds_ws != nullptr
                      ? launch_with_lds<bwd_dkdv_kernel<T, D, NW, BM, W, B, P, kPad, true, kParts>>(grid, NW * 64, smem, stream, a)
@@ -1646,26 +1577,6 @@ hipError_t launch_dq_if(const BwdArgs& a, hipStream_t stream) {
 template <typename T, int D, int kPad, int kOnly = -1>
 hipError_t launch_bwd_dq(const BwdArgs& a0, bool windowed, bool bias, bool dropout, hipStream_t stream) {
 #define FA_CALL(W, B, P) launch_dq_if<T, D, kPad, W, B, P, kOnly == -1 || kOnly == (B ? 1 : 0)>(a0, stream)
-  FA_BWD_SWITCH(FA_CALL)
-#undef FA_CALL
-}
-
-template <typename T, int D, int kPad, bool W, bool B, bool P>
-hipError_t launch_fused_variant(const BwdArgs& a0, hipStream_t stream) {
-  using Tile = BwdTile<T, D, W>;
-  constexpr int NW = Tile::NW, BM = kFusedBM<T, D, W>, BN = kFusedBN<T, D, W>;
-  constexpr int smem = DkDvSmem<D, BM>::BYTES > DqSmem<D, BN>::BYTES ? DkDvSmem<D, BM>::BYTES : DqSmem<D, BN>::BYTES;
-  BwdArgs a = a0;
-  a.num_n_tiles = (a.seq.max_seqlen_k + NW * 32 - 1) / (NW * 32);
-  a.num_m_tiles = (a.seq.max_seqlen_q + NW * 32 - 1) / (NW * 32);
-  set_work(a, tile_work(bwd_nseq(a) * a.hk, 2, a.num_n_tiles + a.num_m_tiles * (a.hq / a.hk)));
-  dim3 grid((unsigned)(kNumXcd * bwd_workers(D, B, a.items_per_xcd, a.num_cu, 1)));
-  return launch_with_lds<bwd_fused_kernel<T, D, NW, BM, BN, W, B, P, kPad>>(grid, NW * 64, smem, stream, a);
-}
-
-template <typename T, int D, int kPad>
-hipError_t launch_bwd_fused(const BwdArgs& a0, bool windowed, bool bias, bool dropout, hipStream_t stream) {
-#define FA_CALL(W, B, P) launch_fused_variant<T, D, kPad, W, B, P>(a0, stream)
   FA_BWD_SWITCH(FA_CALL)
 #undef FA_CALL
 }

@@ -187,6 +187,22 @@ __device__ __forceinline__ u32x4_t wave_rsrc_words(P* base, int bytes) {
   return u32x4_t{lo, hi, n, 0x00020000u};
 }
 
+// The value in a scalar register of its own, of which the compiler does not know where it came from.
+__device__ __forceinline__ int own_scalar(int x) {
+  x = __builtin_amdgcn_readfirstlane(x);
+  asm("" : "+s"(x));
+  return x;
+}
+
+// The kernel's one argument, read where it is used: the pointer is opaque, so nothing read through it is kept from
+// an earlier place.
+template <typename A> using KernelArgs = const __attribute__((address_space(4))) A*;
+template <typename A> __device__ __forceinline__ KernelArgs<A> kernel_args() {
+  KernelArgs<A> k = (KernelArgs<A>)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(k));
+  return k;
+}
+
 // n elements of vector work spread evenly behind g MFMAs: the first one behind MFMA i
 constexpr int first_of(int i, int n, int g) { return (i * n + g - 1) / g; }
 
@@ -241,6 +257,18 @@ struct DropoutState {
   int32_t thr;
   float scale;       // 1/(1-p)
 };
+
+// The dropout scale c = 1 / (1 - p) folded into the row statistics, for kernels that have p from L:
+//   dV += (keep ? c p : 0) dO,   ds = p ((keep ? c dp : 0) - delta) = c p ((keep ? dp : 0) - delta (1 - p))
+// so with c p = exp2(x - (L log2e - log2 c)) neither product costs an instruction per element.
+// (Nothing is kept at p = 1: any scale will do.)
+struct DropoutFold {
+  float log2_scale, keep;      // log2 c, 1 - p
+};
+__device__ __forceinline__ DropoutFold dropout_fold(float p) {
+  const float keep = p < 1.0f ? 1.0f - p : 1.0f;
+  return {-fast_log2(keep), keep};
+}
 
 // The part that reads memory (seed and offset are device scalars): once per work item.  A kernel
 // that walks several heads keeps this and calls dropout_for_head per head; reading the two scalars

@@ -1,0 +1,46 @@
+"""dK/dV with a bias whose rows are whole aligned 16-byte pieces take a kernel of their own: to the bit the results of the
+kernel for any layout, given the same bias with an odd row stride; and dropout whose scale lies in the row statistics,
+against the oracle at probabilities near both ends."""
+import math
+
+import pytest
+import torch
+
+from test_gpu_attention import _run_case
+from _util import make_inputs
+
+pytestmark = pytest.mark.gpu
+
+BF, HF = torch.bfloat16, torch.float16
+
+
+@pytest.mark.parametrize('D', [64, 80, 128, 256])
+@pytest.mark.parametrize('Sq,Sk,causal,p', [(70, 72, False, 0.0), (300, 136, True, 0.1), (257, 520, (60, 90), 0.3), (129, 264, (40, -5), 0.0)])
+def test_aligned_rows_give_the_bits_of_the_general_kernel(D, Sq, Sk, causal, p):
+    from aotriton_amd import flash
+    Hq, Hk, dt = 6, 2, HF
+    B = 2 ** 23 // (Hq * Sq * Sk) + 1      # large enough for the stored dS
+    q, k, v, _, do = make_inputs(B, Hq, Hk, Sq, Sk, D, dt, 'cuda', seed=9)
+    b = torch.randn(B, Hq, Sq, Sk, device='cuda', dtype=dt)
+    odd = torch.empty(B, Hq, Sq, Sk + 3, device='cuda', dtype=dt)[..., 1:Sk + 1].copy_(b)
+    seed = torch.tensor([77], device='cuda', dtype=torch.uint64)
+    off = torch.tensor([5], device='cuda', dtype=torch.uint64)
+    null = torch.empty([0], device='cuda', dtype=torch.uint64)
+    rng = (seed, off) if p else (null, null)
+    sm, out = 1 / math.sqrt(D), []
+    o, L = torch.empty_like(q), torch.empty(B * Hq, Sq, device='cuda')
+    assert flash.attn_fwd(q, k, v, b, sm, L, o, p, *rng, 0, null, null, None, causal, null) == flash.hipError_t.hipSuccess
+    for bias in (b, odd):
+        dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+        err = flash.attn_bwd(q, k, v, bias, sm, o, do, dq, dk, dv, None, flash.lazy_dq_acc(q), L, flash.lazy_delta(L), p, *rng,
+                             0, causal)
+        assert err == flash.hipError_t.hipSuccess
+        out.append((dq, dk, dv))
+    for x, y in zip(*out):
+        assert torch.isfinite(x).all() and torch.equal(x, y)
+
+
+@pytest.mark.parametrize('p', [0.003, 0.5, 0.97])
+@pytest.mark.parametrize('D,bias', [(64, True), (80, False), (128, True), (256, False)])
+def test_dropout_scale_in_the_row_statistics(D, bias, p):
+    _run_case(4, 6, 3, 260, 200, D, BF, True, dropout_p=p, bias=bias, seed=31)
