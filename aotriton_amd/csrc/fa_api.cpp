@@ -6,10 +6,12 @@
 // kernels linked into this library.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <initializer_list>
 #include <mutex>
 #include <vector>
 
@@ -573,7 +575,7 @@ struct FwdPlan {
 // the three, or within a tenth of it, for 95 %.  One measured shape is more than 10 % slower than whole tiles on its
 // route (Hq 8, Hk 2, 512 causal, D = 256: 28 -> 33).  The gains it decides on are larger
 // (one query, 2051 keys, Hq 32 / Hk 8: 55 -> 11 us; 32 sequences of 8190 keys: 833 -> 189; 80 queries,
-// 3216 keys: 88 -> 35; 1024 queries, 16384 keys: 402 -> 266).  Tiles of 128 rows (fwd_half_tiles below) are not among
+// 3216 keys: 88 -> 35; 1024 queries, 16384 keys: 402 -> 266).  Tiles of 128 rows (fwd_small_tiles below) are not among
 // what is compared: they are asked about where this rule leaves the tiles whole.
 FwdPlan fwd_plan(int dtype, const Shape& s, int causal_type, int window_left, int window_right, int num_cu) {
   FwdPlan r{};
@@ -654,21 +656,6 @@ FwdPlan fwd_plan(int dtype, const Shape& s, int causal_type, int window_left, in
   return r;
 }
 
-// Tiles of 128 rows, two workgroups per CU, instead of 256 rows and one (FwdHalfTile)?  Where they save a part
-// of the rounds in which an XCD's CUs take its tiles; the line lies above what they cost per row.  Measured (bf16, us,
-// 256 -> 128 rows): B40 H16 S128 D64 19.1 -> 14.6 (3 rounds against 2), B16 H12 S640 D64 46.6 -> 39.2 and causal 43.4 -> 31.0,
-// D128 68 -> 59 and 63 -> 45 (3 : 2), B40 H16 S640 D64 116 -> 108 (8 : 7), S384 54 -> 48 (5 : 4); B32 H16 S800 D128 227 -> 224
-// (10 : 9); at equal rounds 5-15 % slower.  With a bias the finer tiles cost more (10-15 %), so those keep the large ones.
-// Rounds are all that is compared: what a causal mask does to the tiles of one round is not.
-bool fwd_half_tiles(int dtype, const Shape& s, int num_cu) {
-  if (s.elementwise || !is_16bit(dtype) || s.d > 128 || s.bias || s.num_seqlens != 0) return false;
-  const int64_t heads = (s.batch * (int64_t)s.hq + fa::kNumXcd - 1) / fa::kNumXcd, cus = num_cu / fa::kNumXcd;
-  if (cus < 1) return false;
-  const int64_t whole = (heads * ((s.max_sq + 255) / 256) + cus - 1) / cus;
-  const int64_t half = (heads * ((s.max_sq + 127) / 128) + 2 * cus - 1) / (2 * cus);
-  return whole * 8 > half * 9;
-}
-
 // The kernel with 64 rows per wave (fa_fwd_wide.h; 16-bit types, head dims above 64 and up to 128, no bias, no dropout, a
 // positive scale) for these 256-row tiles?  It takes a tile of 64 keys in 5-7 % less time and an item costs it 1.5-2.5 us
 // more at its ends, where the two waves per SIMD of the other kernel cover for each other.  Measured (bf16, D128, us, other
@@ -697,6 +684,54 @@ bool fwd_wide(const fa_fwd_params* p, const Shape& s, int splits, int num_cu) {
   const int64_t cus = num_cu >= fa::kNumXcd ? num_cu / fa::kNumXcd : 1;
   const int64_t rounds = ((nz * s.hq + fa::kNumXcd - 1) / fa::kNumXcd * m_tiles * splits + cus - 1) / cus;
   return sum >= (rounds <= 2 ? 10 : 20) * (int64_t)m_tiles * splits;
+}
+
+// Tiles of 128 rows, two workgroups per CU (FwdHalfTile) or at D = 64 three (FwdThirdTile), instead of 256 rows and one?
+// Returns their number per CU, 0 for whole tiles (`wide`: those of the kernel with 64 rows per wave).  Per row the smaller
+// tiles cost 5-20 % more; what they save is the part of the last round that whole tiles leave empty and, with a causal mask,
+// the wait for the CU that got the heaviest ones.  So the walk of each is gone through, an item costing a + b * (its 64-key
+// tiles), and a CU whose other workgroups are done being faster (constants fitted to 63 shapes at D = 64, each timed in all
+// three ways, and 43 above: B1-32 H8-32, 64-2500 queries and keys, with and without a causal mask; us).  Against the best of
+// the three the choices lose 0.9 % in the geometric mean at D = 64 (counting rounds only: 9 %, a third of the shapes more
+// than 10 %) and 0.1 % above (1.7 %).  B16 H32 S325 D64 causal 40 / 33 / 29 us (256 rows / 128 twice / 128 three times), B4 H16
+// S2136 D64 causal 86 / 67 / 78, B8 H32 S1369 D64 causal 114 / 152 / 134, B8 H12 S553 D128 causal 40 / 25.  Beyond eight rounds the
+// whole tiles are even enough.  A bias that differs between rows keeps the whole tiles (10-15 % dearer in the smaller ones).
+int fwd_small_tiles(const fa_fwd_params* p, const Shape& s, bool wide, int num_cu) {
+  const bool key_bias = s.bias && !s.dropout && p->B.strides[2] == 0;
+  const int cus = num_cu / fa::kNumXcd;
+  if (s.elementwise || !is_16bit(p->Q.dtype) || s.d > 128 || (s.bias && !key_bias) || s.num_seqlens != 0 || s.max_sq <= 0 ||
+      s.max_sk <= 0 || s.batch <= 0 || cus < 1 || cus > 64)
+    return 0;
+  const int m_tiles = (s.max_sq + 255) / 256, group = fa::q_head_group(s.hq, s.hk);
+  if (fa::tile_work(s.batch * s.hq, group, m_tiles).items_per_xcd > std::min(8 * cus, 448)) return 0;
+  fa::Window w{0, 0};
+  if (s.windowed) w = fa::parse_window(p->causal_type, p->window_left, p->window_right, s.max_sq, s.max_sk);
+  if (s.windowed && w.left < s.max_sq - 1) {      // bounded on the left as well: not among the fitted shapes, rounds are counted
+    const int64_t heads = (s.batch * (int64_t)s.hq + fa::kNumXcd - 1) / fa::kNumXcd;
+    return (heads * m_tiles + cus - 1) / cus * 8 > (heads * ((s.max_sq + 127) / 128) + 2 * cus - 1) / (2 * cus) * 9 ? 2 : 0;
+  }
+  const float cols = s.d > 64 && std::max(s.d_qk, s.d_v) <= 96 ? 0.84f : 1.0f;
+  const int halves = (s.max_sq + 127) / 128;
+  int seen[2][1024];      // 64-key tiles of each tile of 256 and of 128 rows, in the walk's order: from the end of the sequence
+  for (int i = 0; i < 2; ++i)
+    for (int t = 0, bm = 256 >> i, n = i ? halves : m_tiles; t < n; ++t) {
+      const fa::BlockRanges br = fa::block_ranges(s.windowed, w.left, w.right, (n - 1 - t) * bm, s.max_sq, s.max_sk, bm, 64);
+      seen[i][t] = std::max(0, br.hi - br.lo + 1);
+    }
+  auto time = [&](int per_cu, float a, float b, std::initializer_list<float> alone) {
+    float cost[1024];
+    const int tiles = per_cu > 1 ? halves : m_tiles;
+    for (int t = 0; t < tiles; ++t) cost[t] = a + b * cols * seen[per_cu > 1][t];
+    return fa::walk_time_shared(fa::tile_work(s.batch * s.hq, group, tiles), cost, tiles, num_cu, per_cu, alone.begin());
+  };
+  if (s.d > 64) {
+    const float whole = wide ? time(1, 6.9f, 1.51f, {1}) : time(1, 6.3f, 1.74f, {1});
+    return time(2, 7.3f, 1.99f, {0.78f, 1}) < 0.97f * whole ? 2 : 0;
+  }
+  const float whole = time(1, 4.35f, 1.12f, {1}), two = time(2, 4.54f, 1.27f, {0.74f, 1});
+  // (with dropout three waves per SIMD have no idle vector ALU to use)
+  const float three = s.dropout ? 2 * two : time(3, 5.16f, 1.93f, {0.62f, 0.78f, 1});
+  return std::min(two, three) >= 0.98f * whole ? 0 : three < two ? 3 : 2;
 }
 
 hipError_t run_fwd_rows(int dtype, int d, const fa::FwdArgs& a, const Shape& s, hipStream_t stream) {
@@ -973,8 +1008,9 @@ int fa_query_fwd_config(const fa_fwd_params* params, int32_t num_cu, fa_kernel_c
   const int cus = num_cu > 0 ? num_cu : 256;
   const FwdPlan plan = fwd_plan(params->Q.dtype, s, params->causal_type, params->window_left, params->window_right, cus);
   const bool split = !plan.rows && plan.splits > 1;
-  const bool half = !split && fwd_half_tiles(params->Q.dtype, s, cus);
-  const bool wide = !plan.rows && !half && fwd_wide(params, s, split ? plan.splits : 1, cus);
+  const bool may_wide = !plan.rows && fwd_wide(params, s, split ? plan.splits : 1, cus);
+  const int half = split || plan.rows ? 0 : fwd_small_tiles(params, s, may_wide, cus);
+  const bool wide = may_wide && !half;
   const fa::TileShape t = s.elementwise ? fa::TileShape{32, 1, 4, 0}
                           : rows32 ? fa::f32_rows_tile_shape(s.d)
                           : params->Q.dtype == FA_DTYPE_FLOAT32 ? fa::f32_tile_shape(s.d, -1)
@@ -1189,8 +1225,9 @@ static int attn_fwd_impl(const fa_fwd_params* p, int32_t params_version, void* h
     }
   }
   a.splits = scratch != nullptr ? plan.splits : 1;
-  if (a.splits <= 1 && !plan.rows) a.half_tiles = fwd_half_tiles(p->Q.dtype, s, dev->num_cu);
-  const bool wide = !plan.rows && !a.half_tiles && fwd_wide(p, s, a.splits, dev->num_cu);
+  const bool may_wide = !plan.rows && fwd_wide(p, s, a.splits, dev->num_cu);
+  if (a.splits <= 1 && !plan.rows) a.half_tiles = fwd_small_tiles(p, s, may_wide, dev->num_cu);
+  const bool wide = may_wide && !a.half_tiles;
   FA_LOG(4, "attn_fwd: D=%d windowed=%d bias=%d dropout=%d nseq=%d rows=%d splits=%d half_tiles=%d wide=%d", s.d, (int)s.windowed,
          (int)s.bias, (int)s.dropout, s.num_seqlens, (int)plan.rows, a.splits, a.half_tiles, (int)wide);
   if (plan.rows) {

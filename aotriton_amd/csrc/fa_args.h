@@ -40,13 +40,53 @@ inline double walk_time(const TileWork& w, const float* cost, int tiles, int num
     return sum > most ? sum : most;
   }
   double load[64] = {};
-  int pos = 0;
+  int at = 0, step = 1;      // the worker of the next item (counted along: a division per item would show in the host's time)
   for (int first = 0; first < w.zh_per_xcd; first += w.zh_group)
     for (int t = 0; t < tiles; ++t)
-      for (int i = 0; i < w.zh_group; ++i, ++pos)
-        if (first + i < w.zh_per_xcd && first + i < w.num_zh)
-          load[pos / workers & 1 ? workers - 1 - pos % workers : pos % workers] += cost[t];
+      for (int i = 0; i < w.zh_group; ++i) {
+        if (first + i < w.zh_per_xcd && first + i < w.num_zh) load[at] += cost[t];
+        if (at + step < 0 || at + step == workers) step = -step;
+        else at += step;
+      }
   for (int p = 0; p < workers; ++p) most = load[p] > most ? load[p] : most;
+  return most;
+}
+
+// The same with per_cu workgroups on a CU: the time of the busiest CU.  The workgroups of a CU run side by side; with l + 1 of
+// them left, what remains of each takes alone[l] of what its cost says (alone[per_cu - 1] = 1: costs are those of a full CU).
+// For walks of at most 64 CUs and 1024 items per XCD.
+inline float walk_time_shared(const TileWork& w, const float* cost, int tiles, int num_cu, int per_cu, const float* alone) {
+  const int workers = tile_workers(w.items_per_xcd, num_cu, per_cu), cus = num_cu / kNumXcd < workers ? num_cu / kNumXcd : workers;
+  float of[256];      // by position in the walk's rows
+  for (int q = 0; q < workers; ++q) of[q] = 0;
+  int at = 0, step = 1;
+  for (int first = 0; first < w.zh_per_xcd; first += w.zh_group) {
+    const int heads = w.zh_per_xcd - first < w.zh_group ? w.zh_per_xcd - first : w.zh_group;
+    for (int t = 0; t < tiles; ++t)
+      for (int i = 0; i < w.zh_group; ++i) {
+        if (i < heads) of[at] += cost[t];
+        if (at + step < 0 || at + step == workers) step = -step;
+        else at += step;
+      }
+  }
+  float most = 0;
+  for (int c = 0; c < cus; ++c) {
+    // (worker_pos: the workgroups past the first cus sit in the row back to front)
+    float l[4];
+    int n = 0;
+    for (int p = c; p < workers; p += cus) {
+      const float x = of[p < cus ? p : cus + workers - 1 - p];
+      int k = n++;
+      for (; k > 0 && l[k - 1] > x; --k) l[k] = l[k - 1];
+      l[k] = x;
+    }
+    float time = 0, before = 0;
+    for (int i = 0; i < n; ++i) {
+      time += (l[i] - before) * alone[n - 1 - i];
+      before = l[i];
+    }
+    most = time > most ? time : most;
+  }
   return most;
 }
 
@@ -110,7 +150,7 @@ struct FwdArgs {
   int32_t items_per_xcd; // Q tiles (incl. padding of the last group) per XCD
   // keys split over workgroups (fa_fwd_rows.h, fwd_item's kSplit): parts, and their fp32 sums and row
   // statistics in scratch memory, laid out as combine_rows_kernel describes
-  int32_t half_tiles;    // tiles of 128 rows, two workgroups per CU (D <= 128, dense, no bias, not split)
+  int32_t half_tiles;    // tiles of 128 rows: their workgroups per CU, 2 or (D = 64) 3; 0: whole tiles (fwd_small_tiles)
   int32_t splits;        // <= 1: not split (kernels without kSplit do not look at it); at most 64
   int32_t row_blocks;    // blocks of rows per pair
   int32_t part_rows;     // rows stored per block

@@ -464,10 +464,10 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
   // takes the full step.
   bool have_ref = false;     // every row of the wave has a usable reference maximum
   // The reference is settled on the first kRefTiles tiles, in full steps that adopt every larger maximum: as many keys
-  // as the 256-row tile sees in its first step.  P is rounded to 16 bits against the reference, and the largest
+  // as the 256-row tile sees in its first step (128 at D = 64, 64 above).  P is rounded to 16 bits against the reference, and the largest
   // probability of those keys is then exactly 1: settled on one narrow tile, the results of FwdHalfTile were
   // 0.4-3.2 % further from a computation in 64 bits (B40 H16 S128 D64 bf16: 2.16e-3 -> 2.23e-3).
-  constexpr int kRefTiles = NW == 4 ? 2 : 1;
+  constexpr int kRefTiles = NW == 4 ? (D == 64 ? 128 : 64) / BN : 1;
   int ref_tiles = 0;
   float msc_ref = 0.f;       // m_i * sc
   auto sv_fast = [&](int j, int stage, bool masked) -> bool {
@@ -620,12 +620,13 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
 // interleaved, and the workgroups of the XCD take them in serpentine order (worker p
 // takes p, 2P-1-p, 2P+p, ...), which pairs heavy with light tiles.  A workgroup
 // goes from one tile to the next without a relaunch.
-// QB = 0: fwd_item, NW waves of 32 rows.  QB > 0: fwd_item_pipe, 4 waves of 32 * QB rows, one wave
+// QB = 0: fwd_item, NW waves of 32 rows, two waves per SIMD or (FwdThirdTile) three.  QB > 0: fwd_item_pipe, 4 waves of 32 * QB rows, one wave
 // per SIMD.
+template <int D, int NW, int BN, int QB> constexpr int kFwdWaves = D > 128 || QB > 0 ? 1 : D == 64 && NW == 4 && BN == 32 ? 3 : 2;
 template <typename T, int D, int NW, int BN, int QB, bool kWindowed, bool kBias, bool kDropout, int kPad, bool kSplit,
           bool kKeyBias>
 __global__ __attribute__((amdgpu_flat_work_group_size(NW * 64, NW * 64)))
-__attribute__((amdgpu_waves_per_eu(D <= 128 && QB == 0 ? 2 : 1, D <= 128 && QB == 0 ? 2 : 1)))
+__attribute__((amdgpu_waves_per_eu(kFwdWaves<D, NW, BN, QB>, kFwdWaves<D, NW, BN, QB>)))
 void fwd_kernel(const FwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   if (kDropout && blockIdx.x == 0 && threadIdx.x == 0) {
@@ -716,10 +717,14 @@ template <typename T, bool kWindowed> struct FwdTile<T, 128, kWindowed> : FwdTil
 // 629 vs 510; bias + dropout + window 1024: 361 vs 333).
 template <typename T, bool kWindowed> struct FwdTile<T, 256, kWindowed> : FwdTileOf<256, 4, 32, 1> {};
 
-// Half the rows, two workgroups per CU (FwdArgs::half_tiles; dense calls without a bias at D <= 128).  A sequence
+// Half the rows, two workgroups per CU (FwdArgs::half_tiles; dense calls at D <= 128, without a bias or with one of the keys).  A sequence
 // is cut finer, so that less of the last tile and of the last round is empty; per row it is 5-15 % slower (K and V
-// are staged once per 128 rows, narrower key tiles).  fwd_half_tiles in fa_api.cpp decides.
+// are staged once per 128 rows, narrower key tiles).  fwd_small_tiles in fa_api.cpp decides.
 template <int D> struct FwdHalfTile : FwdTileOf<D, 4, D == 64 ? 64 : 32, 0> {};
+// Three of them per CU, on 32-key tiles: 150 registers per wave and 40 KB of LDS.  A barrier every 32 keys makes a full CU 5-10 %
+// slower than with two, but an XCD takes 96 tiles at once instead of 64 (B16 H12 S384 22.2 -> 18.6 us, B16 H32 S325 causal
+// 32.9 -> 28.6, B4 H12 S1544 causal 46.8 -> 41.5).
+struct FwdThirdTile : FwdTileOf<64, 4, 32, 0> {};
 
 template <typename T, int D, bool kWindowed, bool kBias, bool kDropout, int kPad, bool kSplit = false,
           bool kKeyBias = false, typename Tile = FwdTile<T, D, kWindowed>>
@@ -743,7 +748,7 @@ hipError_t launch_fwd_variant(const FwdArgs& a, dim3 grid, hipStream_t stream) {
 // columns are masked.
 template <typename T, int D, int kPad>
 hipError_t launch_fwd(const FwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t stream) {
-  const bool half = D <= 128 && a.half_tiles != 0;
+  const int half = D <= 128 ? a.half_tiles : 0;      // workgroups per CU of 128-row tiles
   const int BM = half ? 128 : windowed ? FwdTile<T, D, true>::BM : FwdTile<T, D, false>::BM;
   const int nseq = a.seq.num_seqlens != 0 ? (a.seq.num_seqlens < 0 ? -a.seq.num_seqlens : a.seq.num_seqlens)
                                           : a.batch;
@@ -753,7 +758,7 @@ hipError_t launch_fwd(const FwdArgs& a, bool windowed, bool bias, bool dropout, 
   const bool split = a.splits > 1;
   const TileWork w = tile_work(nseq * a.hq, q_head_group(a.hq, a.hk), b.num_m_tiles * (split ? a.splits : 1));
   b.num_zh = w.num_zh; b.zh_per_xcd = w.zh_per_xcd; b.zh_group = w.zh_group; b.items_per_xcd = w.items_per_xcd;
-  dim3 grid((unsigned)(kNumXcd * tile_workers(w.items_per_xcd, a.num_cu, half ? 2 : 1)));      // one workgroup per CU, or two
+  dim3 grid((unsigned)(kNumXcd * tile_workers(w.items_per_xcd, a.num_cu, half ? half : 1)));      // one workgroup per CU, or two or three
   if constexpr (D <= 128) {
     if (split) {
       b.part_group = 1; b.part_block = BM; b.part_rows = BM; b.row_blocks = b.num_m_tiles;
@@ -767,11 +772,23 @@ hipError_t launch_fwd(const FwdArgs& a, bool windowed, bool bias, bool dropout, 
   }
   // a bias that is the same for all rows (D <= 128, without dropout)
   if constexpr (D <= 128) {
+    if (bias && !dropout && a.sb_m == 0 && half) {
+      if constexpr (D == 64)
+        if (half == 3)
+          return windowed ? launch_fwd_variant<T, D, true, true, false, kPad, false, true, FwdThirdTile>(b, grid, stream)
+                          : launch_fwd_variant<T, D, false, true, false, kPad, false, true, FwdThirdTile>(b, grid, stream);
+      return windowed ? launch_fwd_variant<T, D, true, true, false, kPad, false, true, FwdHalfTile<D>>(b, grid, stream)
+                      : launch_fwd_variant<T, D, false, true, false, kPad, false, true, FwdHalfTile<D>>(b, grid, stream);
+    }
     if (bias && !dropout && a.sb_m == 0)
       return windowed ? launch_fwd_variant<T, D, true, true, false, kPad, false, true>(b, grid, stream)
                       : launch_fwd_variant<T, D, false, true, false, kPad, false, true>(b, grid, stream);
   }
   if constexpr (D <= 128) {
+    if constexpr (D == 64)
+      if (half == 3)      // (without dropout)
+        return windowed ? launch_fwd_variant<T, D, true, false, false, kPad, false, false, FwdThirdTile>(b, grid, stream)
+                        : launch_fwd_variant<T, D, false, false, false, kPad, false, false, FwdThirdTile>(b, grid, stream);
     using Half = FwdHalfTile<D>;
     switch (half ? (windowed ? 2 : 0) | (dropout ? 1 : 0) : -1) {
       case 0: return launch_fwd_variant<T, D, false, false, false, kPad, false, false, Half>(b, grid, stream);

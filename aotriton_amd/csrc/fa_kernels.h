@@ -38,7 +38,7 @@ hipError_t run_fwd_rows_d64_padded(int dtype, const FwdArgs& a, bool windowed, b
 hipError_t run_fwd_rows_d128_padded(int dtype, const FwdArgs& a, bool windowed, bool bias, hipStream_t s);
 hipError_t run_fwd_rows_d256_padded(int dtype, const FwdArgs& a, bool windowed, bool bias, hipStream_t s);
 // tile table lookups: (element type, head dim, causal / windowed) and the variant
-TileShape fwd_tile_shape(int dtype, int head_dim, bool windowed, bool half_tiles);
+TileShape fwd_tile_shape(int dtype, int head_dim, bool windowed, int half_tiles);
 
 hipError_t run_encoded_softmax(const EncodedSoftmaxArgs& a, hipStream_t s);
 // strided -> packed (unpack false) or packed -> strided (unpack true); elem_bytes 2 or 4

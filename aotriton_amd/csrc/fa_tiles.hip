@@ -7,12 +7,13 @@
 
 namespace fa {
 
-template <typename T, int D> static TileShape fwd_shape_of(bool windowed, bool half) {
+template <typename T, int D> static TileShape fwd_shape_of(bool windowed, int half) {
   auto shape = [](auto tile, int per_cu) {
     using Tile = decltype(tile);
     return TileShape{Tile::BM, Tile::BN, Tile::NW, Tile::LDS, per_cu};
   };
   if constexpr (D <= 128) {
+    if (D == 64 && half == 3) return shape(FwdThirdTile{}, 3);
     if (half) return shape(FwdHalfTile<D>{}, 2);
   }
   return windowed ? shape(FwdTile<T, D, true>{}, 1) : shape(FwdTile<T, D, false>{}, 1);
@@ -31,7 +32,7 @@ template <typename T, int D> static TileShape bwd_shape_of(bool windowed, bool b
   }
 }
 
-TileShape fwd_tile_shape(int dtype, int head_dim, bool windowed, bool half_tiles) {
+TileShape fwd_tile_shape(int dtype, int head_dim, bool windowed, int half_tiles) {
   const bool bf = dtype == kDtypeBF16;
   switch (head_dim) {
     case 64: return bf ? fwd_shape_of<bf16_t, 64>(windowed, half_tiles) : fwd_shape_of<f16_t, 64>(windowed, half_tiles);

@@ -1,0 +1,59 @@
+"""Forward tiles of 128 rows with three workgroups per CU (head dims up to 64), and those and two per CU under a bias of the
+keys: at ragged last tiles and the fewest keys, against a computation in 64 bits."""
+import pytest
+import torch
+
+from test_gpu_attention import _run_case
+from test_launch_queries import fwd
+
+BF, HF = torch.bfloat16, torch.float16
+THREE = [
+    # B, Hq, Hk, Sq, Sk, D, dtype, causal
+    (40, 16, 16, 128, 1, 64, BF, False),
+    (16, 32, 8, 325, 325, 64, HF, True),
+    (16, 12, 12, 384, 33, 64, BF, False),
+    (16, 32, 32, 257, 129, 64, HF, True),
+    (16, 32, 32, 257, 161, 48, BF, (-2147483646, -2147483646)),
+    (16, 12, 12, 383, 300, 40, HF, False),
+]
+# a boolean mask of the keys, as the SDPA entry point passes it on
+KEYS = [
+    (16, 12, 384, 384, 64, HF),
+    (16, 32, 130, 65, 64, BF),
+    (40, 16, 128, 97, 40, HF),
+    (16, 36, 290, 131, 128, BF),
+    (16, 36, 290, 31, 80, HF),
+]
+
+
+def _id(c):
+    return '-'.join(str(x).replace('torch.', '') for x in c)
+
+
+def test_cases_are_of_these_tiles():
+    for c in THREE:
+        assert (lambda x: (x.block_m, x.block_n, x.num_waves))(fwd(*c[:6], c[7])) == (128, 32, 4), _id(c)
+    assert fwd(8, 32, 32, 1369, 1369, 64, True).block_m == 256 and fwd(64, 32, 32, 300, 300, 64).block_m == 256
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('case', THREE, ids=_id)
+def test_three_per_cu_meet_the_oracle(case):
+    _run_case(*case, seed=29)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('case', KEYS, ids=_id)
+def test_key_masks(case):
+    from aotriton_amd import sdpa
+    B, H, Sq, Sk, D, dt = case
+    g = torch.Generator(device='cuda').manual_seed(3)
+    q, k, v = (torch.randn(B, H, s, D, device='cuda', generator=g).to(dt) for s in (Sq, Sk, Sk))
+    mask = torch.rand(B, 1, 1, Sk, device='cuda', generator=g) < 0.7
+    mask[..., 0] = True
+    o = sdpa.scaled_dot_product_attention(q, k, v, attn_mask=mask)
+    s = torch.matmul(q.double(), k.double().transpose(-1, -2).contiguous()) * D ** -0.5
+    p = torch.softmax(s.masked_fill(~mask, float('-inf')), -1)
+    want = torch.matmul(p, v.double())
+    # P rounded to the 16-bit type, the fp32 sums, the result rounded: 3 roundings of the type in the norm
+    assert ((o.double() - want).norm() / want.norm()).item() < 3 * torch.finfo(dt).eps / 2
