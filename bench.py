@@ -38,8 +38,7 @@ def hbm_bytes_from_profile(kernel):
     """HBM bytes per launch of `kernel` at the headline shape: the 'total ... B' figure of the
     committed rocprofv3 summary of that kernel (FETCH_SIZE / WRITE_SIZE runs, scaled by a
     256 MiB elementwise probe).  Counters cannot be read from inside this process."""
-    names = {'fwd_kernel': 'attn_fwd', 'bwd_dkdv_kernel': 'bwd_dkdv', 'bwd_dq_kernel': 'bwd_dq',
-             'bwd_dkdv_kernel (storing dS)': 'bwd_dkdv_storing_ds', 'bwd_dqs_kernel': 'bwd_dqs'}
+    names = {'fwd_wide_kernel': 'attn_fwd', 'bwd_dkdv_wide_kernel': 'bwd_dkdv', 'bwd_dq_wide_kernel': 'bwd_dq'}
     path = os.path.join(ROOT, 'profiles', f'{names.get(kernel, kernel)}_b4_h32_s4096_d128_bf16_causal.txt')
     try:
         m = re.search(r'total ([0-9.e+]+) B', open(path).read())
@@ -357,9 +356,8 @@ def main():
     r_pre = do_bench(lambda: bwd_slot(0))
     r_dkdv = do_bench(lambda: bwd_slot(1))
     r_dq = do_bench(lambda: bwd_slot(2))
-    bwd(0)                                        # the workspace holds this shape's dS for slot 6
     r_prep = do_bench(lambda: bwd_slot(4))
-    r_dkdv_s = do_bench(lambda: bwd_slot(5))
+    r_dkdv_s = do_bench(lambda: bwd_slot(5))      # (leaves this shape's dS in the workspace for slot 6)
     r_dqs = do_bench(lambda: bwd_slot(6))
     torch.cuda.synchronize()
 
@@ -375,32 +373,29 @@ def main():
         return d
 
     # Dominant kernel of the step (the kernels the default step launches) and the GEMM work it is
-    # required to do: forward 2 GEMMs, dK/dV 4 GEMMs (S, dP, dV, dK), dQ from stored dS 1 GEMM; one
+    # required to do: forward 2 GEMMs, dQ with S and dP recomputed 3, dK/dV 4 (S, dP, dV, dK); one
     # causal GEMM = 2*B*H*S^2*D*0.5 FLOP.
     gemm = 2.0 * B * H * S * S * D * (0.5 if causal else 1.0)
-    kernels = {'fwd_kernel': (r_fwd, 2 * gemm), 'bwd_dkdv_kernel (storing dS)': (r_dkdv_s, 4 * gemm),
-               'bwd_dqs_kernel': (r_dqs, 1 * gemm)}
+    kernels = {'fwd_wide_kernel': (r_fwd, 2 * gemm), 'bwd_dq_wide_kernel': (r_dq, 3 * gemm),
+               'bwd_dkdv_wide_kernel': (r_dkdv, 4 * gemm)}
     dom = max(kernels, key=lambda kname: kernels[kname][0]['mean'])
     dom_r, dom_fl = kernels[dom]
     dom_ms = dom_r['mean']
-    # the backward as a whole in the reference's convention (5 GEMMs of algorithmic work; 5 executed
-    # when dS is kept, 7 when the dQ kernel recomputes)
-    bwd_kernels_ms = r_prep['mean'] + r_dkdv_s['mean'] + r_dqs['mean']
+    # the backward as a whole in the reference's convention (5 GEMMs of algorithmic work; 7 executed)
+    bwd_kernels_ms = r_dq['mean'] + r_dkdv['mean']
     elem = 2 * B * H * S * D                                   # bytes of one bf16 activation tensor
     ds_bytes = 2.0 * B * H * S * S * (0.5 if causal else 1.0)  # one 16-bit dS value per visible (query, key) pair
-    algorithmic_bytes = {'fwd_kernel': 4 * elem + 4 * B * H * S,            # Q, K, V in, O out, LSE out
-                         # Q, K, V, dO in, dK, dV out, the two row statistics in, dS out
-                         'bwd_dkdv_kernel (storing dS)': 6 * elem + 8 * B * H * S + ds_bytes,
-                         'bwd_dqs_kernel': 2 * elem + ds_bytes}             # K in, dQ out, dS in
+    algorithmic_bytes = {'fwd_wide_kernel': 4 * elem + 4 * B * H * S,           # Q, K, V in, O out, LSE out
+                         'bwd_dq_wide_kernel': 6 * elem + 8 * B * H * S,        # Q, K, V, O, dO, LSE in, dQ, delta out
+                         'bwd_dkdv_wide_kernel': 6 * elem + 8 * B * H * S}      # Q, K, V, dO, LSE, delta in, dK, dV out
     roofline = {'bound': 'mfma', 'kernel': dom, 'achieved': tf(dom_fl, dom_ms), 'peak': PEAK_BF16_TFLOPS,
                 'unit': 'TFLOP/s', 'frac': tf(dom_fl, dom_ms) / PEAK_BF16_TFLOPS,
                 'traffic': hbm_bytes_from_profile(dom), 'algorithmic_bytes': algorithmic_bytes[dom],
                 'avg_ms': dom_ms, 'median_ms': dom_r['median'], 'flop_per_launch': dom_fl,
                 'frac_ref_convention': tf(f_bwd, bwd_kernels_ms) / PEAK_BF16_TFLOPS,
                 'frac_ref_convention_note': 'whole split backward: 2.5 x forward FLOP (5 GEMMs) over the summed '
-                                            'mean durations of its three kernels (delta and row statistics, '
-                                            'dK/dV writing dS, dQ from dS); frac counts the GEMMs the dominant '
-                                            'kernel executes'}
+                                            'mean durations of its two kernels (dQ with delta, dK/dV); frac counts '
+                                            'the GEMMs the dominant kernel executes'}
 
     out = {
         'metric': 'attn fwd/bwd TFLOPS and % bf16 MFMA peak, B4 H32 S4096 D128 causal, 1 GPU',
@@ -414,14 +409,13 @@ def main():
         'timing': 'per launch: 512 MiB zeroed before it, warm-up >= 25 ms, >= 100 ms of launches, HIP events, '
                   'median (p20, p80); value/ms_per_step: K back-to-back steps between synchronisations',
         'fwd': row(f_fwd, r_fwd),
-        'bwd_split': row(f_bwd, r_split, {'kernels_ms': {'delta_and_row_statistics': r_prep['median'],
-                                                         'bwd_dkdv_storing_ds': r_dkdv_s['median'],
-                                                         'bwd_dq_from_ds': r_dqs['median']},
-                                          'workspace_bytes': ds_bytes * 2 if causal else ds_bytes}),
-        'bwd_split_recompute': row(f_bwd, r_recomp, {'kernels_ms': {'bwd_dq_with_delta': r_dq['median'],
-                                                                    'bwd_dkdv': r_dkdv['median'],
-                                                                    'bwd_preprocess_standalone_not_launched': r_pre['median']},
-                                                     'note': 'workspace limit 0: the dQ kernel recomputes S and dP (7 GEMMs)'}),
+        'bwd_split': row(f_bwd, r_split, {'kernels_ms': {'bwd_dq_with_delta': r_dq['median'],
+                                                         'bwd_dkdv': r_dkdv['median']},
+                                          'note': 'S and dP are recomputed in the dQ kernel (7 GEMMs)'}),
+        'bwd_split_no_workspace': row(f_bwd, r_recomp, {'note': 'workspace limit 0: the same kernels'}),
+        'bwd_kernels_not_launched_ms': {'preprocess': r_pre['median'], 'delta_and_row_statistics': r_prep['median'],
+                                        'dkdv_storing_ds': r_dkdv_s['median'], 'dq_from_ds': r_dqs['median'],
+                                        'stored_ds_bytes': ds_bytes},
         'bwd_fused': row(f_bwd, r_fused),
         'roofline': roofline,
     }
