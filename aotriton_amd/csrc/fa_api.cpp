@@ -695,19 +695,26 @@ bool fwd_wide(const fa_fwd_params* p, const Shape& s, int splits, int num_cu) {
 // the three the choices lose 0.9 % in the geometric mean at D = 64 (counting rounds only: 9 %, a third of the shapes more
 // than 10 %) and 0.1 % above (1.7 %).  B16 H32 S325 D64 causal 40 / 33 / 29 us (256 rows / 128 twice / 128 three times), B4 H16
 // S2136 D64 causal 86 / 67 / 78, B8 H32 S1369 D64 causal 114 / 152 / 134, B8 H12 S553 D128 causal 40 / 25.  Beyond eight rounds the
-// whole tiles are even enough.  A bias that differs between rows keeps the whole tiles (10-15 % dearer in the smaller ones).
+// whole tiles are even enough.
+// A bias that differs between rows, at D = 64 without dropout: its 128-row tiles take rows at any alignment and the last,
+// partial key tile in 16-byte pieces (kAnyRow), the whole tile the aligned rows of whole key tiles only, the rest element by
+// element.  So the partial tile has a cost of its own per item (26 shapes, B1-16 H8-16, 64-1000 queries and keys: 0.3 % from the
+// best of the three, whole tiles 49 %; B8 H12 S512 22.1 / 22.4 / 26.1 us, S520 61 / 26 / 30, S513 193 / 26 / 30, B16 H12 275 x 583
+// 62 / 51 / 38), and unaligned rows never take whole tiles.  Up to three rounds; beyond, the launch queries promise whole ones.
 int fwd_small_tiles(const fa_fwd_params* p, const Shape& s, bool wide, int num_cu) {
   const bool key_bias = s.bias && !s.dropout && p->B.strides[2] == 0;
+  const bool row_bias = s.bias && !key_bias && !s.dropout && s.d == 64 && p->B.strides[3] == 1;
   const int cus = num_cu / fa::kNumXcd;
-  if (s.elementwise || !is_16bit(p->Q.dtype) || s.d > 128 || (s.bias && !key_bias) || s.num_seqlens != 0 || s.max_sq <= 0 ||
+  if (s.elementwise || !is_16bit(p->Q.dtype) || s.d > 128 || (s.bias && !key_bias && !row_bias) || s.num_seqlens != 0 || s.max_sq <= 0 ||
       s.max_sk <= 0 || s.batch <= 0 || cus < 1 || cus > 64)
     return 0;
   const int m_tiles = (s.max_sq + 255) / 256, group = fa::q_head_group(s.hq, s.hk);
-  if (fa::tile_work(s.batch * s.hq, group, m_tiles).items_per_xcd > std::min(8 * cus, 448)) return 0;
+  if (fa::tile_work(s.batch * s.hq, group, m_tiles).items_per_xcd > std::min((row_bias ? 3 : 8) * cus, 448)) return 0;
   fa::Window w{0, 0};
   if (s.windowed) w = fa::parse_window(p->causal_type, p->window_left, p->window_right, s.max_sq, s.max_sk);
   if (s.windowed && w.left < s.max_sq - 1) {      // bounded on the left as well: not among the fitted shapes, rounds are counted
     const int64_t heads = (s.batch * (int64_t)s.hq + fa::kNumXcd - 1) / fa::kNumXcd;
+    if (row_bias) return 0;
     return (heads * m_tiles + cus - 1) / cus * 8 > (heads * ((s.max_sq + 127) / 128) + 2 * cus - 1) / (2 * cus) * 9 ? 2 : 0;
   }
   const float cols = s.d > 64 && std::max(s.d_qk, s.d_v) <= 96 ? 0.84f : 1.0f;
@@ -718,15 +725,26 @@ int fwd_small_tiles(const fa_fwd_params* p, const Shape& s, bool wide, int num_c
       const fa::BlockRanges br = fa::block_ranges(s.windowed, w.left, w.right, (n - 1 - t) * bm, s.max_sq, s.max_sk, bm, 64);
       seen[i][t] = std::max(0, br.hi - br.lo + 1);
     }
-  auto time = [&](int per_cu, float a, float b, std::initializer_list<float> alone) {
+  // `end`: what a key tile of `bn` keys that reaches past the last key costs on top
+  auto time = [&](int per_cu, float a, float b, std::initializer_list<float> alone, float end = 0, int bn = 1) {
     float cost[1024];
     const int tiles = per_cu > 1 ? halves : m_tiles;
-    for (int t = 0; t < tiles; ++t) cost[t] = a + b * cols * seen[per_cu > 1][t];
+    const bool partial = s.max_sk % bn != 0;
+    for (int t = 0; t < tiles; ++t) {
+      const int n = seen[per_cu > 1][t];
+      cost[t] = a + b * cols * n + (partial && n * 64 > s.max_sk / bn * bn ? end : 0.0f);
+    }
     return fa::walk_time_shared(fa::tile_work(s.batch * s.hq, group, tiles), cost, tiles, num_cu, per_cu, alone.begin());
   };
   if (s.d > 64) {
     const float whole = wide ? time(1, 6.9f, 1.51f, {1}) : time(1, 6.3f, 1.74f, {1});
     return time(2, 7.3f, 1.99f, {0.78f, 1}) < 0.97f * whole ? 2 : 0;
+  }
+  if (row_bias) {
+    const bool aligned = fa::bias_aligned(p->B.ptr, p->B.strides[0], p->B.strides[1], p->B.strides[2], p->B.strides[3]);
+    const float two = time(2, 3.85f, 2.32f, {0.83f, 1}, 2.1f, 64), three = time(3, 4.54f, 3.43f, {0.72f, 0.83f, 1}, 0.85f, 32);
+    if (aligned && std::min(two, three) >= 0.98f * time(1, 4.65f, 2.18f, {1}, 8.3f, 128)) return 0;
+    return three < two ? 3 : 2;
   }
   const float whole = time(1, 4.35f, 1.12f, {1}), two = time(2, 4.54f, 1.27f, {0.74f, 1});
   // (with dropout three waves per SIMD have no idle vector ALU to use)

@@ -90,6 +90,11 @@ inline float walk_time_shared(const TileWork& w, const float* cost, int tiles, i
   return most;
 }
 
+// Do the rows of a bias start at 16-byte boundaries, with unit column stride?
+inline bool bias_aligned(const void* bias, int64_t sz, int64_t sh, int64_t sm, int64_t sn) {
+  return sn == 1 && ((sz | sh | sm) & 7) == 0 && ((uintptr_t)bias & 15) == 0;
+}
+
 // Workgroups per XCD of the dK/dV and dQ kernels: one per CU (two: kTwoWaves), at most one per item.  With a
 // bias the kernels get one workgroup per item instead (the loop of a workgroup then runs
 // once): measured at B2 H16 S8192 D256 with window, bias, dB and dropout the persistent

@@ -203,6 +203,23 @@ template <typename A> __device__ __forceinline__ KernelArgs<A> kernel_args() {
   return k;
 }
 
+// Eight elements from column `col` on of a row of `cols` >= 8 elements (unit stride, any alignment: the machine's vector loads
+// take any).  kEnd: the piece may reach past the row; nothing past the row is read then, and what stands for it is
+// unspecified.  (The load is moved back to the row's last eight elements and shifted.)
+template <typename T, bool kEnd>
+__device__ __forceinline__ typename Traits<T>::op_t load_row_piece(const T* row, int col, int cols) {
+  const int at = kEnd && col + 8 > cols ? cols - 8 : col;
+  uint64_t x[2];
+  __builtin_memcpy(x, row + at, 16);
+  if (kEnd) {
+    const int n = 16 * (col - at < 7 ? col - at : 7);
+    const uint64_t up = n < 64 ? (x[1] << 1) << (63 - n) : x[1] >> (n - 64);
+    x[0] = n < 64 ? (x[0] >> n) | up : up;
+    x[1] = n < 64 ? x[1] >> n : 0;
+  }
+  return __builtin_bit_cast(typename Traits<T>::op_t, x);
+}
+
 // n elements of vector work spread evenly behind g MFMAs: the first one behind MFMA i
 constexpr int first_of(int i, int n, int g) { return (i * n + g - 1) / g; }
 

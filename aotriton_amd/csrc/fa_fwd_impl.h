@@ -41,7 +41,8 @@ struct FwdSmem {
 // One Q tile (BM rows of head h of sequence z) against all its visible K/V tiles, or with kSplit
 // against part `split` of a.splits of them: the fp32 sums and the row statistics of the part then go to
 // scratch memory, where combine_rows_kernel picks them up.
-template <typename T, int D, int NW, int BN, bool kWindowed, bool kBias, bool kDropout, int kPad, bool kSplit, bool kKeyBias>
+template <typename T, int D, int NW, int BN, bool kWindowed, bool kBias, bool kDropout, int kPad, bool kSplit, bool kKeyBias,
+          bool kAnyRow>
 __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const int h, const int mt, const int split,
                                          char* smem_raw) {
   using Tr = Traits<T>;
@@ -145,10 +146,16 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
   if (kBias)
     bptr = reinterpret_cast<const T*>(a.bias) + (int64_t)si.batch_index * a.sb_z + (int64_t)h * a.sb_h +
            (int64_t)row_c * a.sb_m;
+
   // 8-byte bias loads need unit column stride and 8-byte aligned rows
-  const bool bias_vec = kBias && a.sb_n == 1 && ((a.sb_m | a.sb_h | a.sb_z) & 3) == 0 &&
+  const bool bias_vec = kBias && !kAnyRow && a.sb_n == 1 && ((a.sb_m | a.sb_h | a.sb_z) & 3) == 0 &&
                         (reinterpret_cast<uintptr_t>(a.bias) & 7) == 0;
 
+  // kAnyRow: bias rows at any alignment, and the tile that reaches past the last key, travel as 16-byte pieces too
+  // (load_row_piece).  A kernel of its own: in the one for aligned rows it cost 9 % (D = 128), 20 % (with dropout) and 30 %
+  // (D = 64) in spills, and element by element unaligned rows took twice to five times as long (B1 H16 S2047 fp16, us, old -> this:
+  // D128 209 -> 96, with dropout 415 -> 174, D64 with dropout 400 -> 169; on 128-row tiles B8 H12 S513 D64 bf16 193 -> 26).
+  static_assert(!kAnyRow || (kBias && !kKeyBias), "rows of a bias");
   // kKeyBias: a bias that does not depend on the query (row stride 0: a padding mask of keys) is staged
   // with the K tile, one float per key in units of the exponent, and read back by broadcast.  As a general
   // bias every wave would carry 32 copies of the row through its row area.  (A template flag: as one more
@@ -302,21 +309,32 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
   constexpr int BRPI = 64 / BLPR;         // rows per wave-wide access
   constexpr int BNI = 32 / BRPI;          // accesses per chunk
   const int brow = lane / BLPR, bch = lane % BLPR;
-  const bool bias_co = kBias && a.sb_n == 1 && ((a.sb_m | a.sb_h | a.sb_z) & 7) == 0 &&
-                       (reinterpret_cast<uintptr_t>(a.bias) & 15) == 0;
-  // adds chunk `ck` of tile j's bias to s (the tile lies inside the key range)
-  auto bias_chunk = [&](int j, int ck) {
+  const bool bias_co = kBias && a.sb_n == 1 &&
+                       (kAnyRow ? si.seqlen_k >= 8
+                                : ((a.sb_m | a.sb_h | a.sb_z) & 7) == 0 && (reinterpret_cast<uintptr_t>(a.bias) & 15) == 0);
+  // adds chunk `ck` of tile j's bias to s (end_tag: the tile may reach past the last key)
+  auto bias_chunk = [&](auto end_tag, int j, int ck) {
     const T* bh = reinterpret_cast<const T*>(a.bias) + (int64_t)si.batch_index * a.sb_z + (int64_t)h * a.sb_h;
-    op_t bco[BNI];
-#pragma unroll
-    for (int i = 0; i < BNI; ++i) {
+    constexpr bool kEnd = decltype(end_tag)::value;
+    auto piece = [&](int i) {
       int m = q0 + wave * 32 + brow + BRPI * i;
       m = m < si.seqlen_q ? m : si.seqlen_q - 1;
-      bco[i] = *reinterpret_cast<const op_t*>(bh + (int64_t)m * a.sb_m + j * BN + ck * BCK + bch * 8);
-    }
+      return load_row_piece<T, kEnd>(bh + (int64_t)m * a.sb_m, j * BN + ck * BCK + bch * 8, si.seqlen_k);
+    };
+    auto put = [&](int i, op_t x) { *reinterpret_cast<op_t*>(rowbuf + (brow + BRPI * i) * SM::ROW_STR + bch * 16) = x; };
+    if constexpr (kEnd) {      // (one after the other: once per item, and all at once spills)
 #pragma unroll
-    for (int i = 0; i < BNI; ++i)
-      *reinterpret_cast<op_t*>(rowbuf + (brow + BRPI * i) * SM::ROW_STR + bch * 16) = bco[i];
+      for (int i = 0; i < BNI; ++i) {
+        put(i, piece(i));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      op_t bco[BNI];
+#pragma unroll
+      for (int i = 0; i < BNI; ++i) bco[i] = piece(i);
+#pragma unroll
+      for (int i = 0; i < BNI; ++i) put(i, bco[i]);
+    }
 #pragma unroll
     for (int mbl = 0; mbl < BCK / 32; ++mbl)
 #pragma unroll
@@ -376,7 +394,11 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
     if (kBias && !kKeyBias) {
       if (bias_co && (j + 1) * BN <= si.seqlen_k) {
 #pragma unroll
-        for (int ck = 0; ck < BN / BCK; ++ck) bias_chunk(j, ck);
+        for (int ck = 0; ck < BN / BCK; ++ck) bias_chunk(std::false_type{}, j, ck);
+      } else if (kAnyRow && bias_co) {
+        if constexpr (kAnyRow)
+#pragma unroll
+          for (int ck = 0; ck < BN / BCK; ++ck) bias_chunk(std::true_type{}, j, ck);
       } else if (bias_vec && (j + 1) * BN <= si.seqlen_k) {
         // a lane's four consecutive keys of every 8-key group in one 8-byte load
 #pragma unroll
@@ -624,7 +646,7 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
 // per SIMD.
 template <int D, int NW, int BN, int QB> constexpr int kFwdWaves = D > 128 || QB > 0 ? 1 : D == 64 && NW == 4 && BN == 32 ? 3 : 2;
 template <typename T, int D, int NW, int BN, int QB, bool kWindowed, bool kBias, bool kDropout, int kPad, bool kSplit,
-          bool kKeyBias>
+          bool kKeyBias, bool kAnyRow = false>
 __global__ __attribute__((amdgpu_flat_work_group_size(NW * 64, NW * 64)))
 __attribute__((amdgpu_waves_per_eu(kFwdWaves<D, NW, BN, QB>, kFwdWaves<D, NW, BN, QB>)))
 void fwd_kernel(const FwdArgs a) {
@@ -685,7 +707,7 @@ void fwd_kernel(const FwdArgs a) {
       split_zh(zh, nseq, ratio, z, h);
     }
     if constexpr (QB > 0) fwd_item_pipe<T, D, QB, BN, kWindowed, kBias, kDropout, kPad>(a, z, h, mt, smem_raw);
-    else fwd_item<T, D, NW, BN, kWindowed, kBias, kDropout, kPad, kSplit, kKeyBias>(a, z, h, mt, split, smem_raw);
+    else fwd_item<T, D, NW, BN, kWindowed, kBias, kDropout, kPad, kSplit, kKeyBias, kAnyRow>(a, z, h, mt, split, smem_raw);
   }
 }
 
@@ -727,10 +749,10 @@ template <int D> struct FwdHalfTile : FwdTileOf<D, 4, D == 64 ? 64 : 32, 0> {};
 struct FwdThirdTile : FwdTileOf<64, 4, 32, 0> {};
 
 template <typename T, int D, bool kWindowed, bool kBias, bool kDropout, int kPad, bool kSplit = false,
-          bool kKeyBias = false, typename Tile = FwdTile<T, D, kWindowed>>
+          bool kKeyBias = false, typename Tile = FwdTile<T, D, kWindowed>, bool kAnyRow = false>
 hipError_t launch_fwd_variant(const FwdArgs& a, dim3 grid, hipStream_t stream) {
   constexpr int NW = Tile::NW;
-  auto kern = fwd_kernel<T, D, NW, Tile::BN, Tile::QB, kWindowed, kBias, kDropout, kPad, kSplit, kKeyBias>;
+  auto kern = fwd_kernel<T, D, NW, Tile::BN, Tile::QB, kWindowed, kBias, kDropout, kPad, kSplit, kKeyBias, kAnyRow>;
   constexpr int smem = Tile::LDS;
   if (grid.x == 0) return hipSuccess;      // no batch, no head or no query row: nothing to write
   if (smem > 64 * 1024) {
@@ -772,6 +794,14 @@ hipError_t launch_fwd(const FwdArgs& a, bool windowed, bool bias, bool dropout, 
   }
   // a bias that is the same for all rows (D <= 128, without dropout)
   if constexpr (D <= 128) {
+    if constexpr (D == 64)
+      if (bias && !dropout && a.sb_m != 0 && half) {      // a bias that differs between rows
+        if (half == 3)
+          return windowed ? launch_fwd_variant<T, D, true, true, false, kPad, false, false, FwdThirdTile, true>(b, grid, stream)
+                          : launch_fwd_variant<T, D, false, true, false, kPad, false, false, FwdThirdTile, true>(b, grid, stream);
+        return windowed ? launch_fwd_variant<T, D, true, true, false, kPad, false, false, FwdHalfTile<D>, true>(b, grid, stream)
+                        : launch_fwd_variant<T, D, false, true, false, kPad, false, false, FwdHalfTile<D>, true>(b, grid, stream);
+      }
     if (bias && !dropout && a.sb_m == 0 && half) {
       if constexpr (D == 64)
         if (half == 3)
@@ -798,6 +828,16 @@ hipError_t launch_fwd(const FwdArgs& a, bool windowed, bool bias, bool dropout, 
     }
   }
   const int key = (windowed ? 4 : 0) | (bias ? 2 : 0) | (dropout ? 1 : 0);
+  if constexpr (D <= 128) {
+    using Whole = FwdTile<T, D, true>;
+    static_assert(std::is_base_of_v<FwdTileOf<D, Whole::NW, Whole::BN, 0>, FwdTile<T, D, false>>, "one tile with and without a mask");
+    switch (bias && a.sb_n == 1 && !bias_aligned(a.bias, a.sb_z, a.sb_h, a.sb_m, a.sb_n) ? key : 0) {
+      case 2: return launch_fwd_variant<T, D, false, true, false, kPad, false, false, Whole, true>(b, grid, stream);
+      case 3: return launch_fwd_variant<T, D, false, true, true, kPad, false, false, Whole, true>(b, grid, stream);
+      case 6: return launch_fwd_variant<T, D, true, true, false, kPad, false, false, Whole, true>(b, grid, stream);
+      case 7: return launch_fwd_variant<T, D, true, true, true, kPad, false, false, Whole, true>(b, grid, stream);
+    }
+  }
   switch (key) {
     case 0: return launch_fwd_variant<T, D, false, false, false, kPad>(b, grid, stream);
     case 1: return launch_fwd_variant<T, D, false, false, true, kPad>(b, grid, stream);
