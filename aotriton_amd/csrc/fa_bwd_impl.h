@@ -356,12 +356,12 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
            ((int64_t)si.batch_index * k->sb_z + (int64_t)hq * k->sb_h + (int64_t)br.lo * BM * k->sb_m + (int64_t)n0 * k->sb_n) * 2;
   };
   __amdgpu_buffer_rsrc_t q_rs, do_rs, b_rs;
-  // The bias tile (BM queries x the workgroup's 128 keys) is staged through LDS like Q
-  // and dO when its layout allows 16-byte loads; otherwise elements are loaded directly.
+  // The bias tile (BM queries x the workgroup's 128 keys) is staged through LDS like Q and dO, in 16-byte pieces of its rows
+  // wherever they start (load_row_piece; element by element it took, us, old -> this: B8 H12 S513 D64 bf16 101 -> 71, B1 H16 S2047
+  // fp16 window 512 with dropout D128 88 -> 68, D256 146 -> 99); a bias whose columns lie apart is gathered.
   static_assert(BN == 128, "bias staging assumes 128 keys per workgroup");
   constexpr int CHB = kBias ? (BM * 16) / NT : 0;        // 16-byte bias pieces per thread
-  const bool bias_lds = kBiasPlain || (kBias && a.sb_n == 1 && ((a.sb_m | a.sb_h | a.sb_z) & 7) == 0 &&
-                                       (reinterpret_cast<uintptr_t>(a.bias) & 15) == 0);
+  const bool bias_rows = kBias && a.sb_n == 1 && si.seqlen_k >= 8;       // 16-byte pieces at any alignment
   op_t bch[CHB > 0 ? CHB : 1];
   const int b_voff = (tid / 16) * bias_row + (tid % 16) * 16;   // bytes inside a bias tile
   const int b_soff = (NT / 16) * bias_row;
@@ -369,7 +369,6 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
   const T* bb_tile = nullptr;     // bias tile being fetched, its valid rows
   int b_rows = 0;
   const int b_cols = si.seqlen_k - n0 < BN ? si.seqlen_k - n0 : BN;      // valid keys of this item
-  const bool bias_plain = kBiasPlain || (bias_lds && (b_cols & 7) == 0);   // no piece straddles the end of a row
   // (g, e) = (q-head inside the GQA group, Q tile inside the range) of the tile to fetch;
   // called for consecutive tiles only; `live` false: nothing is fetched
   auto fetch_begin = [&](bool live, int g, int e) {
@@ -381,7 +380,7 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
     if (kBias) {
       bb_tile = reinterpret_cast<const T*>(bb);
       b_rows = rows;
-      b_rs = wave_rsrc(bb, any && bias_lds ? (rows - 1) * bias_row + b_cols * 2 : 0);
+      b_rs = wave_rsrc(bb, any && kBiasPlain ? (rows - 1) * bias_row + b_cols * 2 : 0);
       if (live) bb += kBiasPlain ? BM * bias_row : (int64_t)BM * 2 * a.sb_m;
     }
     q_rs = wave_rsrc(qb, any ? (rows - 1) * q_row + d_qk * 2 : 0);
@@ -410,23 +409,14 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
   auto fetch_piece = [&](int i) {        // Q pieces first, then dO, then bias
     if (i >= 2 * CH) {
       const int k = i - 2 * CH;
-      if (bias_plain) {
-        // (the usual case behind one scalar branch: the two below test per lane)
+      if (kBiasPlain) {
         bch[k] = __builtin_bit_cast(op_t, __builtin_amdgcn_raw_buffer_load_b128(b_rs, b_voff, k * b_soff, 0));
-      } else if (bias_lds) {
-        bch[k] = __builtin_bit_cast(op_t, __builtin_amdgcn_raw_buffer_load_b128(b_rs, b_voff, k * b_soff, 0));
-        // The descriptor ends at the last valid element of the tile's last row.  When that is
-        // not at a 16-byte boundary the piece that straddles the end loses its valid elements
-        // to the range check too (a dword that holds the last of an odd number of columns reads
-        // as zero): that one piece is gathered element by element.
+      } else if (bias_rows) {
         const int row = tid / 16 + k * (NT / 16), col = (tid % 16) * 8;
-        if ((b_cols & 7) != 0 && row == b_rows - 1 && col < b_cols && col + 8 > b_cols) {
-          op_t x;
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-            x[e] = col + e < b_cols ? bb_tile[(int64_t)row * a.sb_m + col + e] : Tr::cvt(0.f);
-          bch[k] = x;
-        }
+        op_t x = {0, 0, 0, 0, 0, 0, 0, 0};
+        if (row < b_rows && col < b_cols)
+          x = load_row_piece<T, true>(bb_tile - n0 + (int64_t)row * a.sb_m, n0 + col, si.seqlen_k);
+        bch[k] = x;
       } else {
         // any other layout: the piece is gathered element by element
         const int row = tid / 16 + k * (NT / 16), col = (tid % 16) * 8;
@@ -493,7 +483,10 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
     // The vector ALU work is spread over the MFMAs of the GEMMs that do not depend on
     // it: p = exp2(...) of S runs behind the MFMAs of dP, ds = p (dP - delta) behind
     // those of dV.  Fences keep the hand-made order.
-    constexpr int kAhead = 2;      // (one at D = 256 left each read's latency behind a single MFMA: 2-5 % of the kernel)
+    // (one read ahead at D = 256 left each read's latency behind a single MFMA: 2-5 % of the kernel; the bias of any layout has
+    // no registers for more)
+    constexpr bool kDeep = D < 256 || !kBias || kBiasPlain;
+    constexpr int kAhead = kDeep ? 2 : 1;
     op_t xa[kAhead + 1][MB];
     op_t pb[TS];
     uint32_t kw[kDropout ? MB : 1][4];
@@ -572,11 +565,11 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
       }
     }
     const char* Vt = smem_raw + SM::V_OFF;
-    op_t vl[4];          // ring of V operands when they come from LDS
+    constexpr int kVRing = kDeep ? 4 : 3;
+    op_t vl[kVRing];          // ring of V operands when they come from LDS
     if (kVLds) {
-      vl[0] = swz_read_row<T, D>(Vt, row_a, 0, wave);
-      vl[1] = swz_read_row<T, D>(Vt, row_a, 1, wave);
-      vl[2] = swz_read_row<T, D>(Vt, row_a, 2, wave);
+#pragma unroll
+      for (int k = 0; k < kVRing - 1; ++k) vl[k] = swz_read_row<T, D>(Vt, row_a, k, wave);
     }
 
     // element E = 16*mb + i of the tile: p (kept in s, undropped, times the dropout scale) and its operand form
@@ -650,10 +643,10 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
         for (int mb = 0; mb < MB; ++mb)
           xa[(KS + k + kAhead) % (kAhead + 1)][mb] = swz_read_row<T, D>(dOb, row_a, k + kAhead, mb);
       }
-      if (kVLds && k + 3 < KS) vl[(k + 3) % 4] = swz_read_row<T, D>(Vt, row_a, k + 3, wave);
+      if (kVLds && k + kVRing - 1 < KS) vl[(k + kVRing - 1) % kVRing] = swz_read_row<T, D>(Vt, row_a, k + kVRing - 1, wave);
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) {
-        dp[mb] = Tr::mfma(xa[(KS + k) % (kAhead + 1)][mb], kVLds ? vl[k % 4] : vreg[kVLds ? 0 : k],
+        dp[mb] = Tr::mfma(xa[(KS + k) % (kAhead + 1)][mb], kVLds ? vl[k % kVRing] : vreg[kVLds ? 0 : k],
                           k == 0 && kDropout ? zero16 : dp[mb]);
         const int gidx = k * MB + mb;
 #pragma unroll
@@ -675,7 +668,7 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
     // where that would take too many registers (D = 256), through a ring of kRing operands
     // (4 instead of 6 cost 1-2 %; 8, with a V ring of 5, spills).
     constexpr bool kRingTa = DB >= 8;
-    constexpr int kRing = 6;
+    constexpr int kRing = kDeep ? 6 : 4;
     op_t ta[kRingTa ? 1 : 2][kRingTa ? kRing : DB];
     auto ta_read = [&](const char* tile, int gidx) { return swz_read_tr<T, D>(tile, tr_a0, tr_a1, gidx / DB, gidx % DB); };
     if (kRingTa) {

@@ -44,3 +44,16 @@ def test_aligned_rows_give_the_bits_of_the_general_kernel(D, Sq, Sk, causal, p):
 @pytest.mark.parametrize('D,bias', [(64, True), (80, False), (128, True), (256, False)])
 def test_dropout_scale_in_the_row_statistics(D, bias, p):
     _run_case(4, 6, 3, 260, 200, D, BF, True, dropout_p=p, bias=bias, seed=31)
+
+
+@pytest.mark.parametrize('D,dt', [(64, BF), (128, HF), (256, HF)])
+@pytest.mark.parametrize('Sq,Sk,causal,p', [(40, 7, False, 0.0), (70, 9, False, 0.1), (200, 131, True, 0.0), (129, 257, (60, 90), 0.2)])
+@pytest.mark.parametrize('keep', [True, False])
+def test_rows_at_any_alignment(D, dt, Sq, Sk, causal, p, keep):
+    """rows that start anywhere and end inside a piece, against the oracle, with and without a workspace"""
+    from aotriton_amd._lib import lib
+    lib.fa_set_bwd_workspace_limit(-1 if keep else 0)
+    try:
+        _run_case(3, 4, 2, Sq, Sk, D, dt, causal, dropout_p=p, bias=True, bias_layout='odd', seed=12)
+    finally:
+        lib.fa_set_bwd_workspace_limit(-1)
