@@ -1014,10 +1014,11 @@ __device__ __forceinline__ void dq_item(const BwdArgs& a, const int h, const int
                        (reinterpret_cast<uintptr_t>(a.bias) & 15) == 0;
   const bool db_co = kBias && a.db != nullptr && a.sdb_n == 1 && ((a.sdb_m | a.sdb_h | a.sdb_z) & 7) == 0 &&
                      (reinterpret_cast<uintptr_t>(a.db) & 15) == 0;
-  // an item's tiles take the vector code when the bias can be read as vectors and dB (if wanted)
-  // written through the LDS area
+  // An item's tiles take the vector code when the bias can be read as vectors and dB (if wanted)
+  // written through the LDS area; in the split kernel at any alignment of the rows (element by element
+  // B8 H12 S513 D64 bf16 with dB took 139 us, this 69).
   const bool want_db = kBias && a.db != nullptr;
-  const bool item_fast = !kBias || (bias_vec && (!want_db || (db_co && db_vec)));
+  const bool item_fast = !kBias || (kStoreDelta ? a.sb_n == 1 && (!want_db || a.sdb_n == 1) : bias_vec && (!want_db || (db_co && db_vec)));
   const T* bias_head = kBias ? reinterpret_cast<const T*>(a.bias) + (int64_t)si.batch_index * a.sb_z +
                                    (int64_t)h * a.sb_h : nullptr;
   T* db_head = kBias && a.db != nullptr ? reinterpret_cast<T*>(a.db) + (int64_t)si.batch_index * a.sdb_z +
@@ -1136,7 +1137,7 @@ __device__ __forceinline__ void dq_item(const BwdArgs& a, const int h, const int
     // the tile's bias, requested before the S MFMAs and used behind the dP MFMAs: with one wave per
     // SIMD a load that is used where it is issued costs its whole latency
     q4_t bias4[kBias ? 4 * MB : 1];
-    const bool tile_co = kFast && bias_co;                     // bias through the wave's LDS area
+    const bool tile_co = kFast && (kStoreDelta || bias_co);                     // bias through the wave's LDS area
     const bool tile_dbco = kFast && want_db;                   // dB through it
     op_t bco[kBias ? BNI : 1];
     if (kBias && tile_co) {
@@ -1144,7 +1145,8 @@ __device__ __forceinline__ void dq_item(const BwdArgs& a, const int h, const int
       for (int i = 0; i < BNI; ++i) {
         int m = q0 + wave * 32 + brow + BRPI * i;
         m = m < si.seqlen_q ? m : si.seqlen_q - 1;
-        bco[i] = *reinterpret_cast<const op_t*>(bias_head + (int64_t)m * a.sb_m + j * BN + bch * 8);
+        if constexpr (kStoreDelta) bco[i] = load_row_piece<T, false>(bias_head + (int64_t)m * a.sb_m, j * BN + bch * 8, 0);
+        else bco[i] = *reinterpret_cast<const op_t*>(bias_head + (int64_t)m * a.sb_m + j * BN + bch * 8);
       }
     } else if (kBias && tile_vec) {
 #pragma unroll
@@ -1295,7 +1297,9 @@ __device__ __forceinline__ void dq_item(const BwdArgs& a, const int h, const int
       for (int i = 0; i < BNI; ++i) {
         const int m = q0 + wave * 32 + brow + BRPI * i;
         const op_t x = *reinterpret_cast<const op_t*>(bw + (brow + BRPI * i) * SM::BIAS_ROW + bch * 16);
-        if (m < si.seqlen_q) *reinterpret_cast<op_t*>(db_head + (int64_t)m * a.sdb_m + j * BN + bch * 8) = x;
+        if constexpr (kStoreDelta) {
+          if (m < si.seqlen_q) __builtin_memcpy(db_head + (int64_t)m * a.sdb_m + j * BN + bch * 8, &x, 16);
+        } else if (m < si.seqlen_q) *reinterpret_cast<op_t*>(db_head + (int64_t)m * a.sdb_m + j * BN + bch * 8) = x;
       }
     }
     direct_landed();

@@ -57,3 +57,37 @@ def test_rows_at_any_alignment(D, dt, Sq, Sk, causal, p, keep):
         _run_case(3, 4, 2, Sq, Sk, D, dt, causal, dropout_p=p, bias=True, bias_layout='odd', seed=12)
     finally:
         lib.fa_set_bwd_workspace_limit(-1)
+
+
+@pytest.mark.parametrize('D', [64, 128, 256])
+@pytest.mark.parametrize('Sq,Sk,causal,p', [(70, 299, False, 0.0), (161, 128, True, 0.1), (33, 257, (20, 100), 0.0)])
+def test_db_rows_at_any_alignment(D, Sq, Sk, causal, p):
+    """odd bias and dB rows against rows that start at 16-byte boundaries: the same bits, nothing written beside them"""
+    from aotriton_amd import flash
+    from aotriton_amd._lib import lib
+    B, H, dt = 2, 3, BF
+    q, k, v, _, do = make_inputs(B, H, H, Sq, Sk, D, dt, 'cuda', seed=14)
+    seed, off = (torch.tensor([x], device='cuda', dtype=torch.uint64) for x in (7, 8))
+    null, sm, out = torch.empty([0], device='cuda', dtype=torch.uint64), 1 / math.sqrt(D), []
+    values = torch.randn(B, H, Sq, Sk, device='cuda', dtype=dt)
+    lib.fa_set_bwd_workspace_limit(0)
+    try:
+        for width in ((Sk + 7) // 8 * 8, Sk + (1 - Sk % 2) + 2):
+            b, db = (torch.full((B * H * Sq * width + 8,), x, device='cuda', dtype=dt) for x in (float('nan'), 7.0))
+            at = 0 if width % 8 == 0 else 1
+            view = lambda t: t[at:at + B * H * Sq * width].view(B, H, Sq, width)[..., :Sk]
+            view(b).copy_(values)
+            o, L = torch.empty_like(q), torch.empty(B * H, Sq, device='cuda')
+            assert flash.attn_fwd(q, k, v, values, sm, L, o, p, seed, off, 0, null, null, None, causal, null) == flash.hipError_t.hipSuccess
+            dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+            err = flash.attn_bwd(q, k, v, view(b), sm, o, do, dq, dk, dv, view(db), flash.lazy_dq_acc(q), L, flash.lazy_delta(L), p,
+                                 seed, off, 0, causal)
+            assert err == flash.hipError_t.hipSuccess
+            got = view(db).clone()
+            view(db).fill_(7.0)
+            assert (db == 7.0).all()
+            out.append((dq, dk, dv, got))
+    finally:
+        lib.fa_set_bwd_workspace_limit(-1)
+    for x, y in zip(*out):
+        assert torch.isfinite(x).all() and torch.equal(x, y)
