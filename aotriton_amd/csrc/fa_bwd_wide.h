@@ -120,7 +120,6 @@ __device__ __forceinline__ void dkdv_wide_item(const BwdArgs& a, const int hk, c
   const int q_voff = gch * 8 < d_qk ? r0 * (int)a.sq.s * 2 + gch * 16 : kVoffOutOfRange;
   const int do_voff = gch * 8 < d_v ? r0 * (int)a.sdo.s * 2 + gch * 16 : kVoffOutOfRange;
   const int q_row = (int)a.sq.s * 2, do_row = (int)a.sdo.s * 2;
-  const int q_gap = q_row - d_qk * 2, do_gap = do_row - d_v * 2;      // a row's bytes that are not the head's (>= 0)
   const int ntq = br.hi - br.lo + 1;
   const T* qb = nullptr; const T* dob = nullptr;
   const float* st_b = nullptr;      // lower half of the lanes: L of the head, upper half: delta
@@ -139,8 +138,8 @@ __device__ __forceinline__ void dkdv_wide_item(const BwdArgs& a, const int hk, c
   auto fetch_begin = [&]() __attribute__((always_inline)) {
     // (arithmetic instead of choices, for which the compiler makes branches)
     const int rows = min(f_e > 0 ? si.seqlen_q - f_m : 0, BM);
-    q_rs = wave_rsrc_words(qb, max(rows * q_row - q_gap, 0));
-    do_rs = wave_rsrc_words(dob, max(rows * do_row - do_gap, 0));
+    q_rs = wave_rsrc_words(qb, rows_extent(rows, q_row, d_qk * 2));
+    do_rs = wave_rsrc_words(dob, rows_extent(rows, do_row, d_v * 2));
     // (every wave reads and stores the row statistics: a branch for one of them would split the tile's code into blocks,
     // between which the compiler moves the work that is placed behind the MFMAs)
     st_val = st_b[min(f_m + c, si.seqlen_q - 1)];
@@ -537,15 +536,14 @@ __device__ __forceinline__ void dq_wide_item(const BwdArgs& a, const int h, cons
   const int k_voff = gch * 8 < d_qk ? r0 * (int)a.sk.s * 2 + gch * 16 : kVoffOutOfRange;
   const int v_voff = gch * 8 < d_v ? r0 * (int)a.sv.s * 2 + gch * 16 : kVoffOutOfRange;
   const int k_row = (int)a.sk.s * 2, v_row = (int)a.sv.s * 2;
-  const int k_gap = k_row - d_qk * 2, v_gap = v_row - d_v * 2;
   const T* kb = reinterpret_cast<const T*>(a.k) + (int64_t)si.batch_index * a.sk.z + (int64_t)hk * a.sk.h + ((int64_t)si.k_start + (int64_t)br.lo * BN) * a.sk.s;
   const T* vb = reinterpret_cast<const T*>(a.v) + (int64_t)si.batch_index * a.sv.z + (int64_t)hk * a.sv.h + ((int64_t)si.k_start + (int64_t)br.lo * BN) * a.sv.s;
   int f_tiles = ntk, f_rows = si.seqlen_k - br.lo * BN;
   u32x4_t k_rs, v_rs;
   auto fetch_begin = [&]() __attribute__((always_inline)) {
-    const int rows = f_tiles > 0 ? min(max(f_rows, 0), BN) : 0;
-    k_rs = wave_rsrc_words(kb, max(rows * k_row - k_gap, 0));
-    v_rs = wave_rsrc_words(vb, max(rows * v_row - v_gap, 0));
+    const int rows = f_tiles > 0 ? min(f_rows, BN) : 0;
+    k_rs = wave_rsrc_words(kb, rows_extent(rows, k_row, d_qk * 2));
+    v_rs = wave_rsrc_words(vb, rows_extent(rows, v_row, d_v * 2));
     kb += (int64_t)BN * a.sk.s; vb += (int64_t)BN * a.sv.s;
     f_rows -= BN; --f_tiles;
   };

@@ -111,15 +111,14 @@ __device__ __forceinline__ void fwd_wide_item(const FwdArgs& a, const int z, con
   const int k_voff = gch * 8 < d_qk ? r0 * (int)a.sk.s * 2 + gch * 16 : kVoffOutOfRange;
   const int v_voff = gch * 8 < d_v ? r0 * (int)a.sv.s * 2 + gch * 16 : kVoffOutOfRange;
   const int k_row = (int)a.sk.s * 2, v_row = (int)a.sv.s * 2;
-  const int k_gap = k_row - d_qk * 2, v_gap = v_row - d_v * 2;
   const T* kb = reinterpret_cast<const T*>(a.k) + (int64_t)si.batch_index * a.sk.z + (int64_t)hk * a.sk.h + ((int64_t)si.k_start + (int64_t)br.lo * BN) * a.sk.s;
   const T* vb = reinterpret_cast<const T*>(a.v) + (int64_t)si.batch_index * a.sv.z + (int64_t)hk * a.sv.h + ((int64_t)si.k_start + (int64_t)br.lo * BN) * a.sv.s;
   int f_tiles = br.hi - br.lo + 1, f_rows = si.seqlen_k - br.lo * BN;
   u32x4_t k_rs, v_rs;
   auto fetch_begin = [&]() __attribute__((always_inline)) {
-    const int rows = f_tiles > 0 ? min(max(f_rows, 0), BN) : 0;
-    k_rs = wave_rsrc_words(kb, max(rows * k_row - k_gap, 0));
-    v_rs = wave_rsrc_words(vb, max(rows * v_row - v_gap, 0));
+    const int rows = f_tiles > 0 ? min(f_rows, BN) : 0;
+    k_rs = wave_rsrc_words(kb, rows_extent(rows, k_row, d_qk * 2));
+    v_rs = wave_rsrc_words(vb, rows_extent(rows, v_row, d_v * 2));
     kb += (int64_t)BN * a.sk.s; vb += (int64_t)BN * a.sv.s;
     f_rows -= BN; --f_tiles;
   };

@@ -1,4 +1,4 @@
-// Window parsing and K-block ranges for one tile of rows; compiled for host and
+// Window parsing, K-block ranges and the extent of a tile's rows; compiled for host and
 // device.  Semantics of the element predicate and of the sentinels follow
 // modules/flash/kernel/masked_load_store.py:43-63 and
 // modules/flash/kernel/fwd_kernel_inner.py:137-148 of the reference; the range
@@ -87,6 +87,13 @@ FA_HD BlockRanges block_ranges(bool windowed, int32_t left, int32_t right, int32
   r.fb_lo = f_lo; r.fb_hi = f_hi;
   r.rb_lo = f_hi + 1; r.rb_hi = j_hi;
   return r;
+}
+
+// Bytes from the first of `rows` rows to the end of the last one; `row` from one to the next, `head` of each belong to the tensor.
+// 0 without a row, also where rows overlap (row < head): the pointer of a request behind the last tile is past the tensor.
+// (A mask, because a choice becomes a branch in the middle of a tile.)
+FA_HD int32_t rows_extent(int32_t rows, int32_t row, int32_t head) {
+  return (int32_t)((uint32_t)(rows - 1) * (uint32_t)row + (uint32_t)head) & (-rows >> 31);
 }
 
 // int32 keep threshold: fptosi(fp32(fp32(p) - 0.5f) * 2^32), as the reference
