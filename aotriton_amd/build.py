@@ -178,6 +178,34 @@ def asm_mfma_hazards(text):
     return found
 
 
+def asm_memory_hazards(text):
+    """Memory instructions that read a scalar register less than five wait states after a vector instruction wrote it: the
+    compiler keeps that distance for its own and does not look into asm.  Returns the lines.  (Followed from line to line, so
+    that what stands in front of a jump counts for the label behind it only.)"""
+    def scalars(operand):
+        m = re.match(r's\[(\d+):(\d+)\]$', operand) or re.match(r's(\d+)()$', operand)
+        return range(int(m.group(1)), int(m.group(2) or m.group(1)) + 1) if m else ()
+    found, written, now = [], {}, 0
+    for line in text.splitlines():
+        line = line.split(';')[0].strip()
+        if not line or line.startswith('.') or line.endswith(':'):
+            continue
+        op, _, rest = line.partition(' ')
+        args = [a.split()[0] for a in rest.split(',')] if rest else []
+        if op.startswith(('buffer_', 'global_', 'flat_', 'scratch_')):
+            if any(now - written.get(r, -5) < 5 for a in args for r in scalars(a)):
+                found.append(line)
+        now += int(args[0], 0) + 1 if op == 's_nop' else 1
+        for a in args[:2] if op.startswith('v_') else args[:1] if op.startswith('s_') and not op.startswith('s_cmp') else ():
+            for r in scalars(a):
+                # (of the vector instructions that write a scalar register some have it in the second place)
+                if op.startswith(('v_readlane', 'v_readfirstlane', 'v_cmp')) and a is args[0] or '_co_u32' in op or op.startswith(('v_mad_u64', 'v_mad_i64', 'v_div_scale')):
+                    written[r] = now
+                elif op.startswith('s_'):
+                    written.pop(r, None)
+    return found
+
+
 def scan(jobs=8):
     """Compiles every kernel file to assembly and reports per-descriptor loops around buffer
     accesses ("waterfall" loops: readfirstlane, compare, masked issue, repeat while lanes are left).
@@ -185,7 +213,7 @@ def scan(jobs=8):
     threadIdx.x >> 6.  They cost time, and hipcc 7.2 has placed a register spill in the block such
     a loop exits to, before exec is restored: the store runs with no lane enabled and the reload
     later returns whatever the slot held.  The kernels here are written so that none is emitted;
-    returns the list of (file, loops, functions left out of line, asm_mfma_hazards) that have some of any."""
+    returns the list of (file, loops, functions left out of line, asm_mfma_hazards, asm_memory_hazards) that have some of any."""
     import tempfile
     tmpdir = tempfile.TemporaryDirectory(prefix='fa_scan_')
     tmp = tmpdir.name
@@ -193,7 +221,7 @@ def scan(jobs=8):
     def one(unit):
         src, defines, objname = unit
         if not src.endswith('.hip'):
-            return src, 0, 0, []
+            return src, 0, 0, [], []
         out = os.path.join(tmp, objname + '.s')
         cmd = [HIPCC] + COMMON + EXTRA.get(src, []) + defines + ['-x', 'hip', '--cuda-device-only', '-S',
                                                                  os.path.join(CSRC, src), '-o', out]
@@ -204,7 +232,7 @@ def scan(jobs=8):
         # a device function left out of line (a lambda the inliner gave up on) keeps its captures in
         # memory and reads them back with flat loads; every kernel here is meant to be one function
         outlined = len(re.findall(r'^\s*\.type\s+\S+,@function', text, re.M)) - text.count('.amdhsa_kernel ')
-        return objname, len(_WATERFALL.findall(text)), outlined, asm_mfma_hazards(text)
+        return objname, len(_WATERFALL.findall(text)), outlined, asm_mfma_hazards(text), asm_memory_hazards(text)
 
     with tmpdir, concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as ex:
         return [r for r in ex.map(one, sources()) if any(r[1:])]
@@ -218,6 +246,6 @@ if __name__ == '__main__':
     a = ap.parse_args()
     if a.scan:
         found = scan(a.j)
-        print('per-descriptor loops / functions left out of line / asm MFMAs too close behind their operands:', found if found else 'none')
+        print('per-descriptor loops / functions left out of line / asm MFMAs and memory accesses too close behind their operands:', found if found else 'none')
         sys.exit(1 if found else 0)
     print(build(a.j, a.force))

@@ -145,9 +145,9 @@ __device__ __forceinline__ void dkdv_wide_item(const BwdArgs& a, const int hk, c
     st_val = st_b[min(f_m + c, si.seqlen_q - 1)];
   };
   auto fetch_piece = [&](int stage, int i) __attribute__((always_inline)) {
-    const int lds = smem0 + stage + wave * 4 * ROWB + (i & 1) * 16 * ROWB;
-    if (i < 2) load_to_lds(q_rs, q_voff, (i & 1) * 16 * q_row, lds);
-    else load_to_lds(do_rs, do_voff, (i & 1) * 16 * do_row, lds + SM::TILE_BYTES);
+    const int lds = smem0 + stage + i * SM::TILE_BYTES + wave * 4 * ROWB;
+    if (i == 0) load_to_lds(q_rs, q_voff, 0, lds, q_voff, 16 * q_row, lds + 16 * ROWB);
+    else load_to_lds(do_rs, do_voff, 0, lds, do_voff, 16 * do_row, lds + 16 * ROWB);
   };
   auto fetch_end = [&]() __attribute__((always_inline)) {
     qb += (int64_t)BM * a.sq.s; dob += (int64_t)BM * a.sdo.s;
@@ -157,7 +157,7 @@ __device__ __forceinline__ void dkdv_wide_item(const BwdArgs& a, const int hk, c
   auto fetch_all = [&](int stage) __attribute__((always_inline)) {
     fetch_begin();
 #pragma unroll
-    for (int i = 0; i < 4; ++i) fetch_piece(stage, i);
+    for (int i = 0; i < 2; ++i) fetch_piece(stage, i);
     fetch_end();
   };
   const float st_mul = hi ? -1.0f : -kRcpLn2;
@@ -172,12 +172,9 @@ __device__ __forceinline__ void dkdv_wide_item(const BwdArgs& a, const int hk, c
     const auto k_rs = wave_rsrc_words(kb, rows_k > 0 ? ((rows_k - 1) * (int)a.sk.s + d_qk) * 2 : 0);
     const auto v_rs = wave_rsrc_words(vb, rows_k > 0 ? ((rows_k - 1) * (int)a.sv.s + d_v) * 2 : 0);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int gc = ch ^ Swz<D>::f(row4 + 4 * i);
-      load_to_lds(k_rs, gc * 8 < d_qk ? row4 * (int)a.sk.s * 2 + gc * 16 : kVoffOutOfRange, 4 * i * (int)a.sk.s * 2,
-                  smem0 + SM::K_OFF + wave * 64 * ROWB + i * 1024);
-      load_to_lds(v_rs, gc * 8 < d_v ? row4 * (int)a.sv.s * 2 + gc * 16 : kVoffOutOfRange, 4 * i * (int)a.sv.s * 2,
-                  smem0 + SM::V_OFF + wave * 64 * ROWB + i * 1024);
+    for (int i = 0; i < 16; i += 2) {
+      rows_to_lds(k_rs, row4 * (int)a.sk.s * 2, 4 * (int)a.sk.s * 2, d_qk, smem0 + SM::K_OFF + wave * 64 * ROWB, i);
+      rows_to_lds(v_rs, row4 * (int)a.sv.s * 2, 4 * (int)a.sv.s * 2, d_v, smem0 + SM::V_OFF + wave * 64 * ROWB, i);
     }
   }
   set_head();
@@ -351,7 +348,7 @@ __device__ __forceinline__ void dkdv_wide_item(const BwdArgs& a, const int hk, c
         mfma_acc<T>(dv[b][i % DB], ta[i % kRing], pb[b][i / DB]);
         const int gi = i * KB + b;
         if (gi == 0) fetch_begin();
-        if (gi >= 1 && gi <= 4) fetch_piece(st_fetch, gi - 1);
+        if (gi == 1 || gi == 3) fetch_piece(st_fetch, gi / 2);
 #pragma unroll
         for (int E = first_of(gi, 34, G3 * KB); E < first_of(gi + 1, 34, G3 * KB); ++E) {
           if (E < 32) ds_el(E);
@@ -518,12 +515,9 @@ __device__ __forceinline__ void dq_wide_item(const BwdArgs& a, const int h, cons
     const auto q_rs = wave_rsrc_words(qp, rows_q > 0 ? ((rows_q - 1) * (int)a.sq.s + d_qk) * 2 : 0);
     const auto do_rs = wave_rsrc_words(dop, rows_q > 0 ? ((rows_q - 1) * (int)a.sdo.s + d_v) * 2 : 0);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int gc = ch ^ Swz<D>::f(row4 + 4 * i);
-      load_to_lds(q_rs, gc * 8 < d_qk ? row4 * (int)a.sq.s * 2 + gc * 16 : kVoffOutOfRange, 4 * i * (int)a.sq.s * 2,
-                  smem0 + SM::Q_OFF + wave * 64 * ROWB + i * 1024);
-      load_to_lds(do_rs, gc * 8 < d_v ? row4 * (int)a.sdo.s * 2 + gc * 16 : kVoffOutOfRange, 4 * i * (int)a.sdo.s * 2,
-                  smem0 + SM::DO_OFF + wave * 64 * ROWB + i * 1024);
+    for (int i = 0; i < 16; i += 2) {
+      rows_to_lds(q_rs, row4 * (int)a.sq.s * 2, 4 * (int)a.sq.s * 2, d_qk, smem0 + SM::Q_OFF + wave * 64 * ROWB, i);
+      rows_to_lds(do_rs, row4 * (int)a.sdo.s * 2, 4 * (int)a.sdo.s * 2, d_v, smem0 + SM::DO_OFF + wave * 64 * ROWB, i);
     }
   }
   int row_c[QB];
@@ -548,14 +542,14 @@ __device__ __forceinline__ void dq_wide_item(const BwdArgs& a, const int h, cons
     f_rows -= BN; --f_tiles;
   };
   auto fetch_piece = [&](int stage, int i) __attribute__((always_inline)) {
-    const int lds = smem0 + stage + wave * 4 * ROWB + (i & 1) * 16 * ROWB;
-    if (i < 2) load_to_lds(k_rs, k_voff, (i & 1) * 16 * k_row, lds);
-    else load_to_lds(v_rs, v_voff, (i & 1) * 16 * v_row, lds + SM::TILE_BYTES);
+    const int lds = smem0 + stage + i * SM::TILE_BYTES + wave * 4 * ROWB;
+    if (i == 0) load_to_lds(k_rs, k_voff, 0, lds, k_voff, 16 * k_row, lds + 16 * ROWB);
+    else load_to_lds(v_rs, v_voff, 0, lds, v_voff, 16 * v_row, lds + 16 * ROWB);
   };
   auto fetch_all = [&](int stage) __attribute__((always_inline)) {
     fetch_begin();
 #pragma unroll
-    for (int i = 0; i < 4; ++i) fetch_piece(stage, i);
+    for (int i = 0; i < 2; ++i) fetch_piece(stage, i);
   };
   fetch_all(0);
 
@@ -752,7 +746,7 @@ __device__ __forceinline__ void dq_wide_item(const BwdArgs& a, const int h, cons
     for (int i = 0; i < P; ++i) {
       mfma_acc<T>(dq[1][i % DB], x[i], sb[1][i / DB]);
       x[i] = k_row_read(i);
-      if (i < 4) fetch_piece(st_nxt, i);
+      if (i == 0 || i == 2) fetch_piece(st_nxt, i / 2);
       work(5 * P + i);
     }
   };

@@ -123,14 +123,14 @@ __device__ __forceinline__ void fwd_wide_item(const FwdArgs& a, const int z, con
     f_rows -= BN; --f_tiles;
   };
   auto fetch_piece = [&](int stage, int i) __attribute__((always_inline)) {
-    const int lds = smem0 + stage + wave * 4 * ROWB + (i & 3) * 16 * ROWB;
-    if (i < 4) load_to_lds(k_rs, k_voff, (i & 3) * 16 * k_row, lds);
-    else load_to_lds(v_rs, v_voff, (i & 3) * 16 * v_row, lds + SM::TILE_BYTES);
+    const int half = i & 1, lds = smem0 + stage + i / 2 * SM::TILE_BYTES + wave * 4 * ROWB + half * 32 * ROWB;
+    if (i < 2) load_to_lds(k_rs, k_voff, half * 32 * k_row, lds, k_voff, half * 32 * k_row + 16 * k_row, lds + 16 * ROWB);
+    else load_to_lds(v_rs, v_voff, half * 32 * v_row, lds, v_voff, half * 32 * v_row + 16 * v_row, lds + 16 * ROWB);
   };
   auto fetch_all = [&](int stage) __attribute__((always_inline)) {
     fetch_begin();
 #pragma unroll
-    for (int i = 0; i < 8; ++i) fetch_piece(stage, i);
+    for (int i = 0; i < 4; ++i) fetch_piece(stage, i);
   };
 
   // ---- the item's Q rows: memory -> LDS -> registers ---------------------------------------------------------
@@ -140,11 +140,8 @@ __device__ __forceinline__ void fwd_wide_item(const FwdArgs& a, const int z, con
     const T* qp = reinterpret_cast<const T*>(a.q) + (int64_t)si.batch_index * a.sq.z + (int64_t)h * a.sq.h + (int64_t)(si.q_start + qw) * a.sq.s;
     const auto q_rs = wave_rsrc_words(qp, rows_q > 0 ? ((rows_q - 1) * (int)a.sq.s + d_qk) * 2 : 0);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int gc = ch ^ Swz<D>::f(row4 + 4 * i);
-      load_to_lds(q_rs, gc * 8 < d_qk ? row4 * (int)a.sq.s * 2 + gc * 16 : kVoffOutOfRange, 4 * i * (int)a.sq.s * 2,
-                  smem0 + SM::Q_OFF + wave * 64 * ROWB + i * 1024);
-    }
+    for (int i = 0; i < 16; i += 2)
+      rows_to_lds(q_rs, row4 * (int)a.sq.s * 2, 4 * (int)a.sq.s * 2, d_qk, smem0 + SM::Q_OFF + wave * 64 * ROWB, i);
     fetch_all(0);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     const char* Qt = smem_raw + SM::Q_OFF + wave * 64 * ROWB;
@@ -349,7 +346,7 @@ __device__ __forceinline__ void fwd_wide_item(const FwdArgs& a, const int z, con
       }
     };
     mfmas(u_tag, [&](int slot) __attribute__((always_inline)) {
-      if (U == 1 && slot >= 1 && slot <= 8) fetch_piece(st_nxt, slot - 1);
+      if (U == 1 && slot < 8 && slot % 2 == 1) fetch_piece(st_nxt, slot / 2);
 #pragma unroll
       for (int E = first_of(slot, 32 + kLag, 4 * P); E < first_of(slot + 1, 32 + kLag, 4 * P); ++E) {
         if (E < 32) exponent(E);

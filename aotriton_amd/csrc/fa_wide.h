@@ -32,11 +32,23 @@ template <int N> __device__ __forceinline__ void acc_settle(f32x16 (&x)[N], f32x
     asm volatile("s_nop 15\n\ts_nop 15" : "+a"(x[0]), "+a"(x[1]), "+a"(x[2]), "+a"(y[0]), "+a"(y[1]), "+a"(y[2]));
 }
 
-// A wave's 1 KB of a tile straight into LDS (64 lanes x 16 bytes at voff + soff, to lds + 16 lane).  The compiler's builtin
+// Twice a wave's 1 KB of a tile straight into LDS (64 lanes x 16 bytes at voff + soff, to lds + 16 lane).  The compiler's builtin
 // does the same but makes the first transposing LDS read behind it wait for it; here the tile's one wait is placed by hand.
-__device__ __forceinline__ void load_to_lds(u32x4_t rsrc, int voff, int soff, int lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               :: "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "m0");
+// A scalar register that a vector instruction has written (v_readfirstlane, the v_readlane that brings a spilled one back) may be
+// read by a memory instruction five wait states later.  The compiler sees to it for its own and does not look into asm: the
+// move and s_nop 3 are the five, whatever stands in front; two loads share them.
+__device__ __forceinline__ void load_to_lds(u32x4_t rsrc, int voff0, int soff0, int lds0, int voff1, int soff1, int lds1) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %2, %4, %5 offen lds\n\t"
+               "s_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %3, %4, %6 offen lds"
+               :: "s"(lds0), "s"(lds1), "v"(voff0), "v"(voff1), "s"(rsrc), "s"(soff0), "s"(soff1) : "m0");
+}
+// Accesses i and i + 1 of the 16 that bring a wave's 64 rows of 128 columns into LDS (swizzled; a lane's row of access 0 is `voff`
+// bytes from the first, the rows of two accesses `step` apart; chunks past column d are zero).
+__device__ __forceinline__ void rows_to_lds(u32x4_t rsrc, int voff, int step, int d, int lds, int i) {
+  const int lane = threadIdx.x & 63, row4 = lane / 16, ch = lane % 16;
+  const int c0 = ch ^ Swz<128>::f(row4 + 4 * i), c1 = ch ^ Swz<128>::f(row4 + 4 * i + 4);
+  load_to_lds(rsrc, c0 * 8 < d ? voff + c0 * 16 : kVoffOutOfRange, i * step, lds + i * 1024,
+              c1 * 8 < d ? voff + c1 * 16 : kVoffOutOfRange, (i + 1) * step, lds + (i + 1) * 1024);
 }
 // (lengths that were loaded arrive in vector registers, and the arithmetic on them stays there unless told otherwise)
 __device__ __forceinline__ SeqInfo uniform(SeqInfo s) {

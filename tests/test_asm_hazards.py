@@ -1,0 +1,43 @@
+"""Wait states that the compiler does not see to because the reading instruction stands in asm: the checks of `build --scan` on
+listings with a known answer, and on the loads into LDS (fa_wide.h) compiled behind the instructions that precede them."""
+import os
+import subprocess
+
+import pytest
+
+from aotriton_amd import build
+
+LOAD = 'buffer_load_dwordx4 v5, s[4:7], s39 offen lds'
+
+
+@pytest.mark.parametrize('between, found', [
+    (['v_readlane_b32 s39, v254, 2', 's_mov_b32 m0, s50', 's_nop 0'], 1),
+    (['v_readfirstlane_b32 s7, v1', 's_mov_b32 m0, s50', 's_nop 2'], 1),
+    (['v_cmp_gt_u32_e64 s[6:7], v0, v1', 's_mov_b32 m0, s50', 's_nop 0'], 1),
+    (['v_readlane_b32 s39, v254, 2', 's_mov_b32 m0, s50', 's_nop 3'], 0),
+    (['v_readlane_b32 s39, v254, 2', 's_mov_b32 s39, s3', 's_nop 0'], 0),      # written again by a scalar instruction
+    (['v_readlane_b32 s8, v254, 2', 's_nop 0'], 0),                           # another register
+    (['v_add_u32_e32 v5, s39, v5', 's_nop 0'], 0),                            # read, not written
+])
+def test_memory_hazards_of_a_listing(between, found):
+    assert len(build.asm_memory_hazards('\n'.join(f'\t{x}' for x in between + [LOAD]))) == found
+
+
+def test_loads_into_lds_wait_for_their_scalars(tmp_path):
+    """descriptor and offset come out of vector registers right in front of the load"""
+    (tmp_path / 'x.hip').write_text('''#include "fa_wide.h"
+__global__ void k(const char* p, const int* n) {
+  extern __shared__ char smem[];
+  const int t = threadIdx.x, o = n[t];
+  fa::load_to_lds(fa::wave_rsrc_words(p + o, o), t * 16, __builtin_amdgcn_readfirstlane(o + 1), fa::lds_offset(smem),
+                  t * 16, __builtin_amdgcn_readfirstlane(o + 2), fa::lds_offset(smem) + 1024);
+}
+''')
+    if not os.path.exists(build.HIPCC):
+        pytest.skip('no hipcc')
+    out = tmp_path / 'x.s'
+    subprocess.run([build.HIPCC] + build.COMMON + ['-x', 'hip', '--cuda-device-only', '-S', str(tmp_path / 'x.hip'), '-o', str(out)],
+                   check=True, capture_output=True)
+    text = out.read_text()
+    assert text.count('offen lds') == 2 and 'v_readfirstlane' in text
+    assert build.asm_memory_hazards(text) == []
