@@ -5,10 +5,13 @@ Usage: python -m aotriton_amd.build [-j N] [--force]
 """
 import argparse
 import concurrent.futures
+import glob
 import os
 import re
+import shutil
 import subprocess
 import sys
+import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, 'csrc')
@@ -83,10 +86,20 @@ def _compile(unit, force):
     if (not force and inputs and os.path.exists(obj) and all(os.path.exists(p) for p in inputs) and
             os.path.getmtime(obj) >= max(os.path.getmtime(p) for p in inputs)):
         return obj, '', 0
-    cmd = [HIPCC] + COMMON + EXTRA.get(src, []) + defines + ['-MD', '-MF', obj + '.d', '-x', 'hip', '-c', path, '-o', obj]
-    r = subprocess.run(cmd, capture_output=True, text=True)
-    # the host pass does not know the packed-fp32 feature name; that note is noise
-    err = '\n'.join(l for l in r.stderr.splitlines() if 'packed-fp32-ops' not in l)
+    # the compiler's listing of the kernels (on its way to the object) is looked at before the object is taken
+    with tempfile.TemporaryDirectory(prefix='fa_build_') as tmp:
+        made = os.path.join(tmp, objname)
+        cmd = [HIPCC] + COMMON + EXTRA.get(src, []) + defines + ['-save-temps=obj', '-MD', '-MF', obj + '.d', '-x', 'hip', '-c',
+                                                                 path, '-o', made]
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        # the host pass does not know the packed-fp32 feature name; that note is noise
+        err = '\n'.join(l for l in r.stderr.splitlines() if 'packed-fp32-ops' not in l)
+        if r.returncode == 0:
+            for listing in glob.glob(os.path.join(tmp, '*gfx950.s')):
+                lost = masked_spills(open(listing).read())
+                if lost:
+                    return obj, err + f'\n{objname}: values moved while lanes are off: {lost}', 1
+            shutil.move(made, obj)
     return obj, err, r.returncode
 
 
@@ -152,6 +165,39 @@ _WATERFALL = re.compile(r'v_readfirstlane_b32[^\n]*\n(?:[^\n]*\n){0,24}?[^\n]*s_
                         r'[^\n]*s_xor_b64 exec, exec[^\n]*\n[^\n]*s_cbranch_execnz')
 
 
+def masked_spills(text):
+    """Vector instructions between the label where the lanes of a branch meet again and the instruction that turns them on:
+    values the register allocator moved or spilled there.  hipcc 7.2 does so when a scalar move or reload stands in front of that
+    instruction (it takes the block's prologue to end there); the lanes that are off keep what the new place held before, and a
+    pointer among such values faults.  Found in the dQ kernel for padded head dims above 128 with a window and a bias, whose lanes
+    32-63 stored dQ through such a pointer.  Returns (kernel, instruction) pairs."""
+    joins = set(re.findall(r'^\s*s_cbranch_execz (\.LBB\w+)', text, re.M))
+    found, head, before, kernel = [], None, '', ''
+    for line in text.splitlines():
+        block = re.match(r'(\.LBB\w+):|; (%bb\.\d+):', line.strip())
+        if block:
+            # (a block without a label and behind no jump is a meeting place whose jump was removed)
+            falls_in = block.group(1) is None and not before.startswith(('s_cbranch', 's_branch', 's_endpgm', 's_setpc'))
+            head = [] if block.group(1) in joins or falls_in else None
+            continue
+        if re.match(r'\w+:', line):
+            kernel = line.split(':')[0]
+        line = line.split(';')[0].strip()
+        if not line or line.startswith('.') or line.endswith(':'):
+            continue
+        if head is not None:
+            op = line.split()[0]
+            if op.startswith(('s_cbranch', 's_branch', 's_endpgm')) or re.match(r's_\w+ exec,|s_\w+saveexec', line):
+                if line.startswith('s_or_b64 exec, exec,'):
+                    found += [(kernel, x) for x in head]
+                head = None
+            elif (op.startswith(('v_', 'scratch_', 'global_', 'buffer_', 'flat_', 'ds_')) and
+                  not op.startswith(('v_readlane', 'v_writelane', 'v_readfirstlane', 'v_cmp'))):
+                head.append(line)
+        before = line
+    return found
+
+
 def asm_mfma_hazards(text):
     """MFMAs written as asm whose operands a vector instruction writes less than two instructions before: the compiler keeps
     that distance for its own MFMAs and does not look into asm.  Returns the lines."""
@@ -213,15 +259,15 @@ def scan(jobs=8):
     threadIdx.x >> 6.  They cost time, and hipcc 7.2 has placed a register spill in the block such
     a loop exits to, before exec is restored: the store runs with no lane enabled and the reload
     later returns whatever the slot held.  The kernels here are written so that none is emitted;
-    returns the list of (file, loops, functions left out of line, asm_mfma_hazards, asm_memory_hazards) that have some of any."""
-    import tempfile
+    returns the list of (file, loops, functions left out of line, asm_mfma_hazards, asm_memory_hazards, masked_spills) that
+    have some of any."""
     tmpdir = tempfile.TemporaryDirectory(prefix='fa_scan_')
     tmp = tmpdir.name
 
     def one(unit):
         src, defines, objname = unit
         if not src.endswith('.hip'):
-            return src, 0, 0, [], []
+            return src, 0, 0, [], [], []
         out = os.path.join(tmp, objname + '.s')
         cmd = [HIPCC] + COMMON + EXTRA.get(src, []) + defines + ['-x', 'hip', '--cuda-device-only', '-S',
                                                                  os.path.join(CSRC, src), '-o', out]
@@ -232,7 +278,7 @@ def scan(jobs=8):
         # a device function left out of line (a lambda the inliner gave up on) keeps its captures in
         # memory and reads them back with flat loads; every kernel here is meant to be one function
         outlined = len(re.findall(r'^\s*\.type\s+\S+,@function', text, re.M)) - text.count('.amdhsa_kernel ')
-        return objname, len(_WATERFALL.findall(text)), outlined, asm_mfma_hazards(text), asm_memory_hazards(text)
+        return objname, len(_WATERFALL.findall(text)), outlined, asm_mfma_hazards(text), asm_memory_hazards(text), masked_spills(text)
 
     with tmpdir, concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as ex:
         return [r for r in ex.map(one, sources()) if any(r[1:])]
@@ -246,6 +292,6 @@ if __name__ == '__main__':
     a = ap.parse_args()
     if a.scan:
         found = scan(a.j)
-        print('per-descriptor loops / functions left out of line / asm MFMAs and memory accesses too close behind their operands:', found if found else 'none')
+        print('per-descriptor loops / functions left out of line / asm MFMAs and memory accesses too close behind their operands / values moved while lanes are off:', found if found else 'none')
         sys.exit(1 if found else 0)
     print(build(a.j, a.force))

@@ -962,7 +962,12 @@ __device__ __forceinline__ void dq_item(const BwdArgs& a, const int h, const int
       for (int e = 0; e < 8; ++e) acc += (float)o8[e] * (float)doreg[k][e];
     }
     d_row = cross_sum(acc);
-    if (kStoreDelta && row_ok && hi == 0) a.delta[lo] = d_row;
+    if (kStoreDelta) {
+      // (through a descriptor instead of a branch: lanes with hi set and rows past the sequence write nothing)
+      const int first = q0 + wave * 32, rows = si.seqlen_q - first;
+      const auto rs = wave_rsrc(a.delta + lse_offset(si, h, a.hq) + first, rows < 0 ? 0 : rows < 32 ? rows * 4 : 128);
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, d_row), rs, hi ? kVoffOutOfRange : c * 4, 0, 0);
+    }
   } else {
     d_row = a.delta[lo];
   }

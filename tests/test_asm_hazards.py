@@ -1,5 +1,6 @@
-"""Wait states that the compiler does not see to because the reading instruction stands in asm: the checks of `build --scan` on
-listings with a known answer, and on the loads into LDS (fa_wide.h) compiled behind the instructions that precede them."""
+"""The checks of the compiler's listings (build.py) on listings with a known answer: wait states that the compiler does not see to
+because the reading instruction stands in asm, also on the loads into LDS (fa_wide.h) compiled behind the instructions that
+precede them; values that the register allocator moves while lanes are off."""
 import os
 import subprocess
 
@@ -41,3 +42,23 @@ __global__ void k(const char* p, const int* n) {
     text = out.read_text()
     assert text.count('offen lds') == 2 and 'v_readfirstlane' in text
     assert build.asm_memory_hazards(text) == []
+
+
+def listing(*between, meeting='.LBB6_108:'):
+    return '\n'.join(['_ZN2fa6kernelEv:', '\ts_and_saveexec_b64 s[4:5], s[8:9]', '\ts_cbranch_execz .LBB6_108', '; %bb.107:',
+                      '\tglobal_store_dword v[4:5], v2, off', meeting] + [f'\t{x}' for x in between] + ['\ts_or_b64 exec, exec, s[4:5]',
+                                                                                                    '\tv_mov_b32_e32 v1, v3'])
+
+
+@pytest.mark.parametrize('text, found', [
+    (listing('v_accvgpr_write_b32 a205, v31', 'v_accvgpr_write_b32 a204, v30', 's_mov_b32 s93, s87'), 2),
+    (listing('s_mov_b64 s[98:99], s[64:65]', 'scratch_store_dwordx2 off, v[250:251], off offset:72 ; 8-byte Folded Spill'), 1),
+    (listing('v_mov_b32_e32 v7, v8', meeting='; %bb.108:'), 1),
+    (listing('s_mov_b32 s93, s87', 'v_readlane_b32 s5, v254, 25', 'v_writelane_b32 v253, s97, 2', 's_waitcnt vmcnt(0)'), 0),      # scalars
+    (listing(), 0),
+    # the lanes' own work, with the meeting point's instruction at its end
+    ('_ZN2fa6kernelEv:\n\ts_cbranch_execz .LBB2_50\n.LBB2_53:\n\tv_add_u32_e32 v2, v2, v252\n\ts_or_b64 exec, exec, s[16:17]', 0),
+])
+def test_values_moved_while_lanes_are_off(text, found):
+    got = build.masked_spills(text)
+    assert len(got) == found and all(k == '_ZN2fa6kernelEv' for k, _ in got)

@@ -91,3 +91,18 @@ def test_db_rows_at_any_alignment(D, Sq, Sk, causal, p):
         lib.fa_set_bwd_workspace_limit(-1)
     for x, y in zip(*out):
         assert torch.isfinite(x).all() and torch.equal(x, y)
+
+
+@pytest.mark.parametrize('D', [136, 200, 248])
+@pytest.mark.parametrize('dt', [BF, HF])
+@pytest.mark.parametrize('Sq,Sk,causal,p', [(40, 136, (60, 90), 0.0), (300, 136, True, 0.0), (70, 72, (40, -5), 0.0), (129, 264, False, 0.0),
+                                            (129, 264, True, 0.2)])
+@pytest.mark.parametrize('layout', ['padded', 'odd'])
+def test_recomputed_dq_at_padded_head_dims(D, dt, Sq, Sk, causal, p, layout):
+    """dQ and dB without a workspace, head dims rounded up to 256 columns: every lane stores through its own pointer"""
+    from aotriton_amd._lib import lib
+    lib.fa_set_bwd_workspace_limit(0)
+    try:
+        _run_case(2, 4, 2, Sq, Sk, D, dt, causal, dropout_p=p, bias=True, bias_layout=layout, seed=23)
+    finally:
+        lib.fa_set_bwd_workspace_limit(-1)
