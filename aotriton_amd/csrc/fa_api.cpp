@@ -13,7 +13,6 @@
 #include <cstring>
 #include <initializer_list>
 #include <mutex>
-#include <vector>
 
 #include "aotriton_amd/flash.h"
 #include "aotriton_amd/probe.h"
@@ -669,9 +668,10 @@ bool fwd_wide(const fa_fwd_params* p, const Shape& s, int splits, int num_cu) {
     return false;
   const int64_t nz = s.num_seqlens != 0 ? std::abs(s.num_seqlens) : s.batch;
   int sq = s.max_sq, sk = s.max_sk;
-  if (s.num_seqlens > 0) {
-    sq = std::max(1, std::min(sq, (int)(p->Q.sizes[2] / nz)));
-    sk = std::max(1, std::min(sk, (int)(p->K.sizes[2] / nz)));
+  if (s.num_seqlens != 0) {      // (the maximal lengths are the caller's word, the tensors are there)
+    const int share = s.num_seqlens > 0 ? (int)nz : 1;
+    sq = std::max(1, std::min(sq, (int)(p->Q.sizes[2] / share)));
+    sk = std::max(1, std::min(sk, (int)(p->K.sizes[2] / share)));
   }
   const int m_tiles = (sq + 255) / 256;
   int64_t sum = 0;
@@ -880,17 +880,29 @@ struct WalkCost { double item, step; };
 // rows: the side the items are tiles of; cols: the side they step over
 double tile_walk_time(const fa_bwd_params* p, const Shape& s, bool keys, int num_heads, int zh_group, int tile, int step,
                       int heads_per_item, WalkCost c, int num_cu, int max_rows, int max_cols, int nz) {
-  const int n_tiles = (max_rows + tile - 1) / tile;
-  std::vector<float> cost((size_t)n_tiles);
+  // Beyond kMost tiles, which any walk balances, evenly spaced ones stand for all.  (The maximal length of packed sequences is
+  // the caller's word: nothing here may grow with it, neither memory nor time.)
+  constexpr int kMost = 1024;
+  float cost[kMost];
+  const int n_tiles = (int)(((int64_t)max_rows + tile - 1) / tile), n = std::min(n_tiles, kMost);
   fa::Window w{0, 0};
   if (s.windowed)
     w = fa::parse_window(p->causal_type, p->window_left, p->window_right, keys ? max_cols : max_rows, keys ? max_rows : max_cols);
-  for (int t = 0; t < n_tiles; ++t) {
-    const fa::BlockRanges b = fa::block_ranges(s.windowed, keys ? w.right : w.left, keys ? w.left : w.right, t * tile, max_rows,
+  double sum = 0, most = 0;
+  for (int t = 0; t < n; ++t) {
+    const int at = n == n_tiles ? t : (int)((int64_t)t * n_tiles / n);
+    const fa::BlockRanges b = fa::block_ranges(s.windowed, keys ? w.right : w.left, keys ? w.left : w.right, at * tile, max_rows,
                                                max_cols, tile, step);
-    cost[keys ? t : n_tiles - 1 - t] = (float)(c.item + c.step * heads_per_item * (b.hi - b.lo + 1));
+    const float x = (float)(c.item + c.step * heads_per_item * (b.hi - b.lo + 1));
+    cost[keys ? t : n - 1 - t] = x;
+    sum += x;
+    most = std::max(most, (double)x);
   }
-  return fa::walk_time(fa::tile_work(nz * num_heads, zh_group, n_tiles), cost.data(), n_tiles, num_cu);
+  if (n < n_tiles) {
+    const double per_xcd = (nz * (double)num_heads + fa::kNumXcd - 1) / fa::kNumXcd, workers = std::max(1, num_cu / fa::kNumXcd);
+    return std::max(sum / n * n_tiles * per_xcd / std::min(workers, n_tiles * per_xcd), most);
+  }
+  return fa::walk_time(fa::tile_work(nz * num_heads, zh_group, n_tiles), cost, n_tiles, num_cu);
 }
 bool wide_bwd_built(const fa_bwd_params* p, const Shape& s) {
   return !s.elementwise && is_16bit(p->Q.dtype) && s.d == 128 && !s.bias && !s.dropout && s.max_sq > 0 && s.max_sk > 0 && s.batch > 0;
@@ -899,10 +911,13 @@ BwdRoute bwd_route(const fa_bwd_params* p, const Shape& s, int num_cu) {
   BwdRoute r{false, false, false, 2, fa::q_head_group(s.hq, s.hk)};
   if (!wide_bwd_built(p, s)) return r;
   const int nz = s.num_seqlens != 0 ? std::abs(s.num_seqlens) : s.batch, group = s.hq / s.hk;
-  int sq = s.max_sq, sk = s.max_sk;
-  if (s.num_seqlens > 0) {
-    sq = std::max(1, std::min(sq, (int)(p->Q.sizes[2] / nz)));
-    sk = std::max(1, std::min(sk, (int)(p->K.sizes[2] / nz)));
+  constexpr int kLongest = 1 << 30;      // (the arithmetic on tiles goes a little past the end)
+  const int max_sq = std::min(s.max_sq, kLongest), max_sk = std::min(s.max_sk, kLongest);
+  int sq = max_sq, sk = max_sk;
+  if (s.num_seqlens != 0) {
+    const int share = s.num_seqlens > 0 ? nz : 1;
+    sq = std::max(1, std::min(sq, (int)(p->Q.sizes[2] / share)));
+    sk = std::max(1, std::min(sk, (int)(p->K.sizes[2] / share)));
   }
   struct Best { double t; int group; };
   auto walk = [&](bool keys, int tile, int step, WalkCost c) {
@@ -910,7 +925,7 @@ BwdRoute bwd_route(const fa_bwd_params* p, const Shape& s, int num_cu) {
     const int rows = keys ? sk : sq, cols = keys ? sq : sk;
     Best b{tile_walk_time(p, s, keys, heads, zg, tile, step, per_item, c, num_cu, rows, cols, nz), zg};
     if (s.num_seqlens != 0) {
-      const double longest = tile_walk_time(p, s, keys, 1, 1, tile, step, per_item, c, 1 << 20, keys ? s.max_sk : s.max_sq, keys ? s.max_sq : s.max_sk, 1);
+      const double longest = tile_walk_time(p, s, keys, 1, 1, tile, step, per_item, c, 1 << 20, keys ? max_sk : max_sq, keys ? max_sq : max_sk, 1);
       b.t = std::max(b.t, longest);
     } else if (tile == 256) {
       // all heads of an XCD side by side, the heavy tiles of all of them first: better balanced, more streams in flight

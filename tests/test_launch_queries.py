@@ -38,6 +38,26 @@ def bwd(slot, B, Hq, Hk, Sq, Sk, D, causal=False, p=0.0, bias=False):
     return c
 
 
+def packed(slot, lens_q, lens_k, Hq, Hk, D, causal=False, longest=None, num_cu=256):
+    """the configuration of packed sequences (compact), forward with slot None"""
+    from aotriton_amd.pyaotriton.v3.flash import attn_bwd_params, attn_fwd_params, query_bwd_config, query_fwd_config
+    from aotriton_amd.pyaotriton import lazy_tensor
+    Sq, Sk = int(sum(lens_q)), int(sum(lens_k))
+    x = attn_fwd_params() if slot is None else attn_bwd_params()
+    x.Q = x.Out = view(1, Hq, Sq, D)
+    x.K = x.V = view(1, Hk, Sk, D)
+    if slot is not None:
+        x.DQ, x.DO, x.DK, x.DV, x.L = x.Q, x.Q, x.K, x.K, view(Hq, Sq, name='kFloat32')
+        x.D = lazy_tensor.eager_delta(x.L)
+    _common(x, 1, Hq, Sq, Sk, causal, 0.0, False)
+    x.cu_seqlens_q = x.cu_seqlens_k = view(len(lens_q) + 1, name='kInt32')
+    x.varlen_type = 1
+    x.Max_seqlen_q, x.Max_seqlen_k = longest or int(max(lens_q)), longest or int(max(lens_k))
+    err, c = query_fwd_config(x, num_cu) if slot is None else query_bwd_config(x, slot)
+    assert int(err) == 0
+    return c
+
+
 def _common(x, B, Hq, Sq, Sk, causal, p, bias):
     from aotriton_amd.pyaotriton import DType, T0
     x.Sm_scale = 0.125
@@ -168,3 +188,14 @@ def test_narrow_windows_leave_items_whole_where_parts_only_make_rounds():
     assert bwd(1, 1, 2, 2, 1536, 1536, 128, (200, 0), 0.1).flags & 64 == 0
     assert bwd(1, 1, 2, 2, 1536, 1536, 128, True, 0.1).flags & 64
     assert bwd(1, 1, 8, 2, 1536, 1536, 128, (200, 0), 0.1).flags & 64
+
+
+@pytest.mark.parametrize('causal', [False, True, (200, 100)])
+def test_a_caller_may_name_any_longest_sequence(causal):
+    """the maximal lengths of packed sequences need not be those of the tensors; the choice of kernels neither grows with them nor
+    fails on them"""
+    lens = [5000, 3000, 9000, 3000]
+    for slot, m, n in [(None, 256, 64), (1, 32, 256), (2, 256, 32)]:
+        for longest in (1 << 24, 1 << 30, (1 << 31) - 200, (1 << 31) - 1):
+            c = packed(slot, lens, lens, 16, 8, 128, causal, longest)
+            assert (c.block_m, c.block_n) in ((m, n), (64, 128) if slot == 1 else (128, 64))
