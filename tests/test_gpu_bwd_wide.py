@@ -9,7 +9,7 @@ import torch
 
 from test_gpu_attention import _run_case
 from test_gpu_varlen_dropout import _run_varlen_case
-from test_launch_queries import bwd
+from test_launch_queries import bwd, packed
 from _util import make_inputs
 
 BF, HF = torch.bfloat16, torch.float16
@@ -89,3 +89,20 @@ def test_wide_items_of_packed_sequences(D, causal):
     lens = np.random.default_rng(3).integers(100, 500, size=24)
     lens[5], lens[11] = 0, 257
     _run_varlen_case(lens, lens[::-1].copy() if D == 96 else lens, 16, 16, D, BF, causal, 0, seed=6)
+
+
+PACKED = np.random.default_rng(3).integers(100, 500, size=24) * 2 + 1
+PACKED[5], PACKED[11], PACKED[17] = 0, 257, 1
+PACKED_CASES = [(128, True, 16, 16), (128, (50, 30), 16, 16), (96, False, 16, 16), (72, True, 64, 32), (128, (-40, 200), 32, 32)]
+
+
+def test_packed_cases_are_of_these_kernels():
+    for D, causal, Hq, Hk in PACKED_CASES:
+        c1, c2 = (packed(slot, PACKED, PACKED[::-1] if D == 96 else PACKED, Hq, Hk, D, causal) for slot in (1, 2))
+        assert (c1.block_m, c1.block_n, c2.block_m, c2.block_n) == (32, 256, 256, 32), (D, causal, Hq, Hk)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('D, causal, Hq, Hk', PACKED_CASES)
+def test_packed_sequences_on_both_kernels_meet_the_oracle(D, causal, Hq, Hk):
+    _run_varlen_case(PACKED, PACKED[::-1].copy() if D == 96 else PACKED, Hq, Hk, D, HF if D == 72 else BF, causal, 0, seed=16)

@@ -9,7 +9,7 @@ import torch
 
 import test_gpu_fwd_tiles
 from test_gpu_varlen_dropout import _run_varlen_case
-from test_launch_queries import fwd
+from test_launch_queries import fwd, packed
 from _util import make_inputs
 
 BF, HF = torch.bfloat16, torch.float16
@@ -74,3 +74,21 @@ def test_maximum_grows_from_unit_to_unit(dtype, top):
 def test_wide_forward_of_packed_sequences(D, causal):
     lens = np.array([1411, 900, 0, 1800, 1290, 257, 2048, 1024])
     _run_varlen_case(lens, lens, 16, 8, D, BF, causal, 0, seed=8)
+
+
+# lengths whose average brings the rule to these kernels: an empty sequence, ones that end with a row or a key in a tile of their own
+PACKED = [np.array([1411, 900, 0, 1800, 1290, 257, 2048, 1024]), np.array([3001, 1, 2304, 0, 1345])]
+PACKED_CASES = [(i, D, c, Hq, Hk) for D, c in [(128, True), (80, False), (128, (1200, 40)), (96, BR)] for i, Hq, Hk in [(0, 8, 4), (1, 8, 8)]]
+
+
+def test_packed_cases_are_of_this_kernel():
+    for i, D, causal, Hq, Hk in PACKED_CASES:
+        c = packed(None, PACKED[i], PACKED[i][::-1] if causal == BR else PACKED[i], Hq, Hk, D, causal)
+        assert (c.block_m, c.num_waves, c.flags & 192) == (256, 4, 0), (i, D, causal)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('i, D, causal, Hq, Hk', PACKED_CASES)
+def test_packed_sequences_on_this_kernel_meet_the_oracle(i, D, causal, Hq, Hk):
+    lens = PACKED[i]
+    _run_varlen_case(lens, lens[::-1].copy() if causal == BR else lens, Hq, Hk, D, BF if i else HF, causal, 0, seed=18)
