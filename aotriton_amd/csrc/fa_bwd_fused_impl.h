@@ -1,9 +1,9 @@
 // The backward in one launch (gfx950): dK/dV items and dQ items of a head on one grid, delta recomputed in both.
 // The dQ item is the split kernel's (fa_bwd_impl.h).  The dK/dV item here computes the same as the split one, whose comments
 // describe it, but its tiles pass through registers on their way into LDS, because delta comes from the O and dO pieces there.
-// The split item's scalars (own_scalar, kernel_args) and DropoutFold are not in it: built with them the D = 256 kernel with a
-// bias accessed memory outside its tensors.  The source shows no such access; these builds spill 85 vector and 400 scalar
-// registers, and what went wrong there was not found, so the code that the compiler is known to get right stays as it was.
+// The split item's scalars (own_scalar, kernel_args) and DropoutFold are not in it: a build with them (85 vector and 400 scalar
+// registers spilled at D = 256) accessed memory outside its tensors.  Its listing has what masked_spills in build.py looks for,
+// registers that the compiler moved while lanes were off; the kernel as it stands has none.
 #pragma once
 #include "fa_bwd_impl.h"
 
@@ -11,7 +11,6 @@ namespace fa {
 
 template <typename T, int D, int NW, int BM, bool kWindowed, bool kBias, bool kDropout, int kPad>
 __device__ __forceinline__ void fused_dkdv_item(const BwdArgs& a, const int hk, const int nt, const int z, char* smem_raw) {
-  constexpr bool kInlineDelta = true;
   using Tr = Traits<T>;
   using op_t = typename Tr::op_t;
   using q4_t = typename Tr::q4_t;
@@ -26,7 +25,6 @@ __device__ __forceinline__ void fused_dkdv_item(const BwdArgs& a, const int hk, 
 
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63, c = lane & 31, hi = lane >> 5;
-  const int wave_u = __builtin_amdgcn_readfirstlane(tid >> 6);
   // columns of Q/K/dQ/dK and of V/Out/dOut/dV: <= D, multiples of 8; constants unless a head dim is rounded up
   const int d_qk = kPad ? a.head_dim : D, d_v = kPad ? a.head_dim_v : D;
 
@@ -118,33 +116,10 @@ __device__ __forceinline__ void fused_dkdv_item(const BwdArgs& a, const int hk, 
   // the last tile into a no-op.
   static_assert(NCH % NT == 0, "threads must cover the tile evenly");
   constexpr int RPI = NT / LPR;                  // rows between two pieces of one thread
-  // The Q and dO pieces go from global memory straight into the LDS stage (no staging registers
-  // and no LDS write instructions: 3-5 % at D = 64 and 128; at D = 256 the staging registers,
-  // next to 256 accumulators, the K operands and the softmax state, were what pushed the K
-  // operands out to scratch, and a scratch reload waits for every load in flight).  A wave
-  // instruction fills 1 KB of consecutive LDS, 64 / LPR rows; the swizzle is applied on the
-  // global side: the lane at chunk position p of row r fetches chunk p ^ f(r).  Lanes outside the
-  // descriptor's range deliver zeros.  The pieces count in vmcnt like any load; the compiler makes
-  // the first transposing LDS read after them wait for all of them (mid-tile: they have landed).
-  // The fused kernel computes delta from the staged O and dO registers and keeps them.
-  constexpr bool kDirect = !kInlineDelta;
-  constexpr int RWI = 64 / LPR;                  // rows one wave instruction covers
-  op_t qch[kDirect ? 1 : CH], doch[kDirect ? 1 : CH], och[kInlineDelta ? CH : 1];
-  float l_stage = 0.f, d_stage = 0.f;
+  // (The split kernel's pieces go straight into LDS; here delta is computed from the O and dO registers.)
+  op_t qch[CH], doch[CH], och[CH];
+  float l_stage = 0.f;
   const int r0 = tid / LPR, cc0 = tid % LPR;
-  int f_stage = 0;                               // stage the running fetch fills
-  // f(r0 + k RPI) takes at most two values, for even and odd k (RPI is a multiple of 8, f has period 16)
-  int q_voff_d[2] = {0, 0}, do_voff_d[2] = {0, 0};
-  if (kDirect) {
-    static_assert(!kDirect || RPI % 8 == 0, "the swizzle must repeat every two pieces");
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const int gch = cc0 ^ Swz<D>::f(r0 + k * RPI);
-      q_voff_d[k] = gch * 8 < d_qk ? r0 * (int)a.sq.s * 2 + gch * 16 : kVoffOutOfRange;
-      do_voff_d[k] = gch * 8 < d_v ? r0 * (int)a.sdo.s * 2 + gch * 16 : kVoffOutOfRange;
-    }
-  }
-  using lds_ptr_t = __attribute__((address_space(3))) void*;
   const int q_voff = cc0 * 8 < d_qk ? r0 * (int)a.sq.s * 2 + cc0 * 16 : kVoffOutOfRange,       // bytes inside a tile
             do_voff = cc0 * 8 < d_v ? r0 * (int)a.sdo.s * 2 + cc0 * 16 : kVoffOutOfRange,
             o_voff = cc0 * 8 < d_v ? r0 * (int)a.so.s * 2 + cc0 * 16 : kVoffOutOfRange;
@@ -158,18 +133,16 @@ __device__ __forceinline__ void fused_dkdv_item(const BwdArgs& a, const int hk, 
   const int64_t q_tile_step = (int64_t)BM * a.sq.s, do_tile_step = (int64_t)BM * a.sdo.s,
                 o_tile_step = (int64_t)BM * a.so.s;
   const T* qb = nullptr; const T* dob = nullptr; const T* ob = nullptr;
-  const float* lse_b = nullptr; const float* delta_b = nullptr;
+  const float* lse_b = nullptr;
   auto set_head = [&](int g) {
     const int hq = hk * group + g;
     const int64_t row0 = (int64_t)si.q_start + (int64_t)br.lo * BM;
     qb = reinterpret_cast<const T*>(a.q) + (int64_t)si.batch_index * a.sq.z + (int64_t)hq * a.sq.h + row0 * a.sq.s;
     dob = reinterpret_cast<const T*>(a.dout) + (int64_t)si.batch_index * a.sdo.z + (int64_t)hq * a.sdo.h +
           row0 * a.sdo.s;
-    if (kInlineDelta)
-      ob = reinterpret_cast<const T*>(a.out) + (int64_t)si.batch_index * a.so.z + (int64_t)hq * a.so.h +
-           row0 * a.so.s;
+    ob = reinterpret_cast<const T*>(a.out) + (int64_t)si.batch_index * a.so.z + (int64_t)hq * a.so.h +
+         row0 * a.so.s;
     lse_b = a.lse + lse_offset(si, hq, a.hq) + (int64_t)br.lo * BM;
-    if (!kInlineDelta) delta_b = a.delta + lse_offset(si, hq, a.hq) + (int64_t)br.lo * BM;
   };
   __amdgpu_buffer_rsrc_t q_rs, do_rs, o_rs, b_rs;
   // The bias tile (BM queries x the workgroup's 128 keys) is staged through LDS like Q
@@ -206,16 +179,14 @@ __device__ __forceinline__ void fused_dkdv_item(const BwdArgs& a, const int hk, 
     }
     q_rs = wave_rsrc(qb, any ? ((rows - 1) * (int)a.sq.s + d_qk) * 2 : 0);
     do_rs = wave_rsrc(dob, any ? ((rows - 1) * (int)a.sdo.s + d_v) * 2 : 0);
-    if (kInlineDelta)
-      o_rs = wave_rsrc(ob, any ? ((rows - 1) * (int)a.so.s + d_v) * 2 : 0);
+    o_rs = wave_rsrc(ob, any ? ((rows - 1) * (int)a.so.s + d_v) * 2 : 0);
     if (tid < BM) {
       const bool ok = tid < rows;
       l_stage = ok ? lse_b[tid] : 0.f;
-      if (!kInlineDelta) d_stage = ok ? delta_b[tid] : 0.f;
     }
     if (live) {
       qb += q_tile_step; dob += do_tile_step; lse_b += BM;
-      if (kInlineDelta) ob += o_tile_step; else delta_b += BM;
+      ob += o_tile_step;
     }
   };
   constexpr int FETCH_PIECES = 2 * CH + CHB;
@@ -251,29 +222,12 @@ __device__ __forceinline__ void fused_dkdv_item(const BwdArgs& a, const int hk, 
         bch[k] = x;
       }
     } else if (i < CH) {
-      if constexpr (kDirect) {
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            q_rs, (lds_ptr_t)(stage_ptr(f_stage) + (i * RPI + RWI * wave_u) * Swz<D>::ROWB), 16, q_voff_d[i & 1],
-            i * q_soff, 0, 0);
-      } else {
-        qch[i] = __builtin_bit_cast(op_t, __builtin_amdgcn_raw_buffer_load_b128(q_rs, q_voff, i * q_soff, 0));
-      }
+      qch[i] = __builtin_bit_cast(op_t, __builtin_amdgcn_raw_buffer_load_b128(q_rs, q_voff, i * q_soff, 0));
     } else {
       const int k = i - CH;
-      if constexpr (kDirect) {
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            do_rs, (lds_ptr_t)(stage_ptr(f_stage) + SM::TILE_BYTES + (k * RPI + RWI * wave_u) * Swz<D>::ROWB), 16,
-            do_voff_d[k & 1], k * do_soff, 0, 0);
-      } else {
-        doch[k] = __builtin_bit_cast(op_t, __builtin_amdgcn_raw_buffer_load_b128(do_rs, do_voff, k * do_soff, 0));
-      }
-      if (kInlineDelta)
-        och[k] = __builtin_bit_cast(op_t, __builtin_amdgcn_raw_buffer_load_b128(o_rs, o_voff, k * o_soff, 0));
+      doch[k] = __builtin_bit_cast(op_t, __builtin_amdgcn_raw_buffer_load_b128(do_rs, do_voff, k * do_soff, 0));
+      och[k] = __builtin_bit_cast(op_t, __builtin_amdgcn_raw_buffer_load_b128(o_rs, o_voff, k * o_soff, 0));
     }
-  };
-  // all of this wave's direct pieces have landed (vmcnt 0; the other counters stay as they are)
-  auto direct_landed = [&]() {
-    if constexpr (kDirect) __builtin_amdgcn_s_waitcnt(0x0F70);
   };
   constexpr int STORE_PIECES = 2 * CH + CHB;
   auto store_piece = [&](int i, int stage) {   // same order as the fetches
@@ -281,7 +235,6 @@ __device__ __forceinline__ void fused_dkdv_item(const BwdArgs& a, const int hk, 
     if (i >= 2 * CH)
       *reinterpret_cast<op_t*>(sp + 2 * SM::TILE_BYTES + 2 * BM * 4 + b_lds + (i - 2 * CH) * (NT / 16) * SM::BIAS_STR) =
           bch[i - 2 * CH];
-    else if (kDirect) return;
     else if (i < CH) *reinterpret_cast<op_t*>(sp + lds_off[i]) = qch[i];
     else *reinterpret_cast<op_t*>(sp + SM::TILE_BYTES + lds_off[i - CH]) = doch[i - CH];
   };
@@ -289,24 +242,18 @@ __device__ __forceinline__ void fused_dkdv_item(const BwdArgs& a, const int hk, 
     char* sp = stage_ptr(stage);
     float* Ls = reinterpret_cast<float*>(sp + 2 * SM::TILE_BYTES);
     float* Ds = Ls + BM;
-    if (kInlineDelta) {
-      // delta recomputed from O and dO (bwd_kernel_fuse.py:307-310); the LPR threads
-      // that share a row are consecutive lanes
+    // delta recomputed from O and dO (bwd_kernel_fuse.py:307-310); the LPR threads that share a row are consecutive
+    // lanes.  Without dropout -delta is staged: it is the initial value of the dP accumulators.
 #pragma unroll
-      for (int k = 0; k < CH; ++k) {
-        float acc = 0.f;
+    for (int k = 0; k < CH; ++k) {
+      float acc = 0.f;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc += (float)och[k][e] * (float)doch[k][e];
+      for (int e = 0; e < 8; ++e) acc += (float)och[k][e] * (float)doch[k][e];
 #pragma unroll
-        for (int off = LPR / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
-        if (cc0 == 0) Ds[r0 + k * RPI] = kDropout ? acc : -acc;
-      }
+      for (int off = LPR / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+      if (cc0 == 0) Ds[r0 + k * RPI] = kDropout ? acc : -acc;
     }
-    if (tid < BM) {
-      Ls[tid] = l_stage * kRcpLn2;                          // bwd_inner_dk_dv.py:185-186
-      // without dropout -delta is staged: it is the initial value of the dP accumulators
-      if (!kInlineDelta) Ds[tid] = kDropout ? d_stage : -d_stage;
-    }
+    if (tid < BM) Ls[tid] = l_stage * kRcpLn2;                          // bwd_inner_dk_dv.py:185-186
   };
 
   // seed and offset of the dropout mask: read once per item, not once per tile
@@ -377,7 +324,7 @@ __device__ __forceinline__ void fused_dkdv_item(const BwdArgs& a, const int hk, 
         // the next tile's descriptors and global loads ride behind these MFMAs
         constexpr int every = G1 / FETCH_PIECES > 0 ? G1 / FETCH_PIECES : 1;
         const int gidx = k * MB + mb;
-        if (gidx == 0) { f_stage = stage ^ 1; fetch_begin(live, g_nxt, e_nxt); }
+        if (gidx == 0) fetch_begin(live, g_nxt, e_nxt);
         if (kDropout) {
           // One Philox call yields the keep bits of 4 consecutive keys, i.e. of the 4
           // lanes of a quad, for one row: quad lane q runs the calls of the rows with
@@ -582,7 +529,6 @@ __device__ __forceinline__ void fused_dkdv_item(const BwdArgs& a, const int hk, 
       __builtin_amdgcn_sched_barrier(0);
     }
     store_stats(stage ^ 1);
-    direct_landed();
   };
 
   if (kVLds) {
@@ -606,7 +552,6 @@ __device__ __forceinline__ void fused_dkdv_item(const BwdArgs& a, const int hk, 
 #pragma unroll
   for (int i = 0; i < STORE_PIECES; ++i) store_piece(i, 0);
   store_stats(0);
-  direct_landed();
   __syncthreads();
   // Per q-head the Q tiles come as [masked | full | masked]; each run has its own
   // loop so that the loop bodies are straight-line code.
