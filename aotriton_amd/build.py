@@ -41,9 +41,10 @@ EXTRA = {
     'fa_bwd_dkdv_d128.hip': ['-mllvm', '-amdgpu-sched-strategy=max-ilp'],
     'fa_bwd_dkdv_parts_d128.hip': ['-mllvm', '-amdgpu-sched-strategy=max-ilp'],
     'fa_bwd_dq_bias_d64.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'],
-    # (scores in vector registers; the accumulators are asm operands and stay in accumulation registers)
-    'fa_fwd_wide_d128.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'],
-    'fa_bwd_wide_d128.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'],
+    # (scores in vector registers; the accumulators are asm operands and stay in accumulation registers.  The loads into LDS
+    # written as asm name m0 among what they change, and the compiler notes at each that it reserves that register.)
+    'fa_fwd_wide_d128.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form', '-Wno-inline-asm'],
+    'fa_bwd_wide_d128.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form', '-Wno-inline-asm'],
     'fa_bwd_dq_d128.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'],
 }
 
@@ -224,6 +225,55 @@ def asm_mfma_hazards(text):
     return found
 
 
+def asm_accumulator_hazards(text):
+    """Instructions that read or write an accumulation register less than 20 wait states after an asm MFMA wrote it (16 passes and
+    what the register file takes), on any path, except the next MFMA onto the same accumulator: the compiler keeps that
+    distance behind its own MFMAs and does not look into asm.  Returns the lines.  (An MFMA counts as one state.)"""
+    def accumulators(operand):
+        m = re.match(r'a\[(\d+):(\d+)\]$', operand) or re.match(r'a(\d+)()$', operand)
+        return frozenset(range(int(m.group(1)), int(m.group(2) or m.group(1)) + 1)) if m else frozenset()
+
+    # blocks: [instructions (line, states, accumulators per operand, asm MFMA?), blocks that follow by label, falls through?]
+    blocks, at, in_asm = [[[], [], True]], {}, False
+    for line in text.splitlines():
+        if '#ASM' in line:
+            in_asm = 'START' in line
+        line = line.split(';')[0].strip()
+        if line.endswith(':') and (line.startswith('.LBB') or not line.startswith('.')):
+            blocks.append([[], [], True])
+            at[line[:-1]] = len(blocks) - 1
+            blocks[-2][2] &= line.startswith('.')      # (not into the next kernel)
+        if not line or line.startswith('.') or line.endswith(':'):
+            continue
+        op, _, rest = line.partition(' ')
+        args = [a.split()[0] for a in rest.split(',')] if rest else []
+        blocks[-1][0].append((line, int(args[0], 0) + 1 if op == 's_nop' else 1, [accumulators(a) for a in args],
+                              in_asm and op.startswith('v_mfma')))
+        if op.startswith(('s_cbranch', 's_branch', 's_endpgm', 's_setpc')):
+            blocks[-1][1:] = [[args[0]] if 'branch' in op else [], op.startswith('s_cbranch')]
+            blocks.append([[], [], True])
+
+    # wait states since the last write of each accumulator, the fewest over all paths into a block
+    found, entry, todo = {}, [{} for _ in blocks], set(range(len(blocks)))
+    while todo:
+        i = todo.pop()
+        instructions, labels, falls = blocks[i]
+        ages = dict(entry[i])
+        for n, (line, states, used, asm_mfma) in enumerate(instructions):
+            onto = used[0] if line.startswith('v_mfma') and used[3] in (used[0], frozenset()) else None
+            if any(u & group and not u == onto == group for u in used for group in ages):
+                found[i, n] = line
+            ages = {group: age + states for group, age in ages.items() if age + states < 20}
+            if asm_mfma and used[0]:
+                ages[used[0]] = 0
+        for j in [at[x] for x in labels if x in at] + ([i + 1] if falls and i + 1 < len(blocks) else []):
+            merged = {g: min(ages.get(g, 20), entry[j].get(g, 20)) for g in {*ages, *entry[j]}}
+            if merged != entry[j]:
+                entry[j] = merged
+                todo.add(j)
+    return list(found.values())
+
+
 def asm_memory_hazards(text):
     """Memory instructions that read a scalar register less than five wait states after a vector instruction wrote it: the
     compiler keeps that distance for its own and does not look into asm.  Returns the lines.  (Followed from line to line, so
@@ -259,15 +309,15 @@ def scan(jobs=8):
     threadIdx.x >> 6.  They cost time, and hipcc 7.2 has placed a register spill in the block such
     a loop exits to, before exec is restored: the store runs with no lane enabled and the reload
     later returns whatever the slot held.  The kernels here are written so that none is emitted;
-    returns the list of (file, loops, functions left out of line, asm_mfma_hazards, asm_memory_hazards, masked_spills) that
-    have some of any."""
+    returns the list of (file, loops, functions left out of line, asm_mfma_hazards, asm_accumulator_hazards, asm_memory_hazards,
+    masked_spills) that have some of any."""
     tmpdir = tempfile.TemporaryDirectory(prefix='fa_scan_')
     tmp = tmpdir.name
 
     def one(unit):
         src, defines, objname = unit
         if not src.endswith('.hip'):
-            return src, 0, 0, [], [], []
+            return src, 0, 0, [], [], [], []
         out = os.path.join(tmp, objname + '.s')
         cmd = [HIPCC] + COMMON + EXTRA.get(src, []) + defines + ['-x', 'hip', '--cuda-device-only', '-S',
                                                                  os.path.join(CSRC, src), '-o', out]
@@ -278,7 +328,8 @@ def scan(jobs=8):
         # a device function left out of line (a lambda the inliner gave up on) keeps its captures in
         # memory and reads them back with flat loads; every kernel here is meant to be one function
         outlined = len(re.findall(r'^\s*\.type\s+\S+,@function', text, re.M)) - text.count('.amdhsa_kernel ')
-        return objname, len(_WATERFALL.findall(text)), outlined, asm_mfma_hazards(text), asm_memory_hazards(text), masked_spills(text)
+        return (objname, len(_WATERFALL.findall(text)), outlined, asm_mfma_hazards(text), asm_accumulator_hazards(text),
+                asm_memory_hazards(text), masked_spills(text))
 
     with tmpdir, concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as ex:
         return [r for r in ex.map(one, sources()) if any(r[1:])]
@@ -292,6 +343,6 @@ if __name__ == '__main__':
     a = ap.parse_args()
     if a.scan:
         found = scan(a.j)
-        print('per-descriptor loops / functions left out of line / asm MFMAs and memory accesses too close behind their operands / values moved while lanes are off:', found if found else 'none')
+        print('per-descriptor loops / functions left out of line / asm MFMAs and memory accesses too close behind their operands or in front of what follows / values moved while lanes are off:', found if found else 'none')
         sys.exit(1 if found else 0)
     print(build(a.j, a.force))

@@ -1,5 +1,5 @@
 """The checks of the compiler's listings (build.py) on listings with a known answer: wait states that the compiler does not see to
-because the reading instruction stands in asm, also on the loads into LDS (fa_wide.h) compiled behind the instructions that
+because one of the two instructions stands in asm, also on the loads into LDS (fa_wide.h) compiled behind the instructions that
 precede them; values that the register allocator moves while lanes are off."""
 import os
 import subprocess
@@ -22,6 +22,27 @@ LOAD = 'buffer_load_dwordx4 v5, s[4:7], s39 offen lds'
 ])
 def test_memory_hazards_of_a_listing(between, found):
     assert len(build.asm_memory_hazards('\n'.join(f'\t{x}' for x in between + [LOAD]))) == found
+
+
+MFMA = [';;#ASMSTART', 'v_mfma_f32_32x32x16_bf16 a[0:15], v[2:5], v[6:9], a[0:15]', ';;#ASMEND']
+
+
+@pytest.mark.parametrize('behind, found', [
+    (['s_nop 15', 's_nop 2', 'v_accvgpr_read_b32 v1, a3'], 1),
+    (['s_nop 15', 's_nop 3', 'v_accvgpr_read_b32 v1, a3'], 0),
+    (['v_accvgpr_write_b32 a15, v1'], 1),
+    (['v_accvgpr_write_b32 a16, v1', 'global_store_dword v[2:3], a40, off'], 0),      # other registers
+    (['global_store_dword v[2:3], a4, off'], 1),
+    (['v_mfma_f32_32x32x16_bf16 a[0:15], v[2:5], v[6:9], a[0:15]'], 0),               # onto the same accumulator
+    (['v_mfma_f32_32x32x16_bf16 v[20:35], a[12:15], v[6:9], 0'], 1),                  # as an operand
+    (['v_mfma_f32_32x32x16_bf16 a[8:23], v[2:5], v[6:9], a[8:23]'], 1),               # a part of it
+    # out of a loop to where its results are read, with and without a wait there
+    (['s_cbranch_scc1 .LBB0_2', 's_nop 15', 's_nop 15', '.LBB0_2:', 'v_accvgpr_read_b32 v1, a3'], 1),
+    (['s_cbranch_scc1 .LBB0_2', 's_branch .LBB0_3', '.LBB0_2:', 's_nop 15', 's_nop 3', '.LBB0_3:', 'v_mov_b32 v1, v2'], 0),
+    (['s_branch .LBB0_3', '.LBB0_2:', 'v_accvgpr_read_b32 v1, a3', 's_endpgm', '.LBB0_3:', 's_nop 15', 's_nop 3', 's_branch .LBB0_2'], 0),
+])
+def test_accumulator_hazards_of_a_listing(behind, found):
+    assert len(build.asm_accumulator_hazards('\n'.join(f'\t{x}' for x in MFMA + behind))) == found
 
 
 def test_loads_into_lds_wait_for_their_scalars(tmp_path):
