@@ -700,7 +700,8 @@ bool fwd_wide(const fa_fwd_params* p, const Shape& s, int splits, int num_cu) {
 // partial key tile in 16-byte pieces (kAnyRow), the whole tile the aligned rows of whole key tiles only, the rest element by
 // element.  So the partial tile has a cost of its own per item (26 shapes, B1-16 H8-16, 64-1000 queries and keys: 0.3 % from the
 // best of the three, whole tiles 49 %; B8 H12 S512 22.1 / 22.4 / 26.1 us, S520 61 / 26 / 30, S513 193 / 26 / 30, B16 H12 275 x 583
-// 62 / 51 / 38), and unaligned rows never take whole tiles.  Up to three rounds; beyond, the launch queries promise whole ones.
+// 62 / 51 / 38); within the three rounds that this rule covers unaligned rows take no whole tiles, unless a window is bounded on the
+// left.  Beyond, and with such a window, the tiles are whole (fa_query_fwd_config reports them).
 int fwd_small_tiles(const fa_fwd_params* p, const Shape& s, bool wide, int num_cu) {
   const bool key_bias = s.bias && !s.dropout && p->B.strides[2] == 0;
   const bool row_bias = s.bias && !key_bias && !s.dropout && s.d == 64 && p->B.strides[3] == 1;

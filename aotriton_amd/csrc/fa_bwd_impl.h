@@ -298,9 +298,9 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
   };
 
   // ---- staging -----------------------------------------------------------------
-  // Q and dO tiles travel global -> registers -> LDS in 16-byte pieces.  The pieces
-  // are issued between the MFMAs of the running tile (loads behind S = Q K^T, LDS
-  // writes behind dK^T += Q^T dS), so staging costs no issue time of its own.
+  // Q and dO tiles travel in 16-byte pieces that are issued between the MFMAs of the running tile
+  // (behind S = Q K^T), so staging costs little issue time of its own; a bias passes through registers,
+  // its LDS writes behind dK^T += Q^T dS.
   // Buffer loads with a descriptor rebased on every tile: rows past the end of the
   // sequence read as zero, and a descriptor of zero records turns the fetch after
   // the last tile into a no-op.
@@ -386,7 +386,7 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
     q_rs = wave_rsrc(qb, any ? (rows - 1) * q_row + d_qk * 2 : 0);
     do_rs = wave_rsrc(dob, any ? (rows - 1) * do_row + d_v * 2 : 0);
     if constexpr (kStoreDs) {
-      // the prepared statistics (L log2e; -delta, or delta with dropout) go straight into the stage:
+      // the prepared statistics (L log2e and -delta, with dropout as DropoutFold has them) go straight into the stage:
       // no register load in the loop, hence no wait of the compiler's for one at the end of a tile
       // (16 bytes per lane: BM / 4 lanes of wave 0 fetch each array)
       if (tid < BM / 4) {
