@@ -2,8 +2,8 @@
 // The dQ item is the split kernel's (fa_bwd_impl.h).  The dK/dV item here computes the same as the split one, whose comments
 // describe it, but its tiles pass through registers on their way into LDS, because delta comes from the O and dO pieces there.
 // The split item's scalars (own_scalar, kernel_args) and DropoutFold are not in it: a build with them (85 vector and 400 scalar
-// registers spilled at D = 256) accessed memory outside its tensors.  Its listing has what masked_spills in build.py looks for,
-// registers that the compiler moved while lanes were off; the kernel as it stands has none.
+// registers spilled at D = 256) accessed memory outside its tensors.  The same sources built with a window show what masked_spills
+// in build.py looks for, registers that the compiler moved while lanes were off; the kernel as it stands has none.
 #pragma once
 #include "fa_bwd_impl.h"
 

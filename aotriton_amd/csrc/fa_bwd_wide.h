@@ -14,9 +14,9 @@
 // through LDS (an item of the 32-row kernels spends 9 us on that and its other ends, one of these 6).
 //
 // Measured (bf16, D128, us, 32-row kernel -> this; one box): dK/dV B4 H32 S4096 causal 1125 -> 1000, full 1956 -> 1740, B1 H32
-// S16384 causal 3840 -> 3380; dQ 840 -> 735, 1435 -> 1280, 2770 -> 2495.  Both run into the power limit: the matrix pipe is
-// busy for 63 % / 68 % of the time (53 % / 56 % before) at 1.77 / 1.69 GHz (1.90 / 1.89 before), 1250 / 1290 TFLOP/s, a bf16
-// product of the library reaches 1220-1270 on this card.  Spreading the vector work differently over the MFMAs is level.
+// S16384 causal 3840 -> 3380; dQ 840 -> 735, 1435 -> 1280, 2770 -> 2495.  The clock falls with the load: at length the matrix
+// pipe is busy for 63 % / 68 % of the time (53 % / 56 % before) at 1.77 / 1.69 GHz (1.90 / 1.89 before), 1250 / 1290 TFLOP/s; a
+// few launches of B4 H32 S4096 causal 57 % / 59 % at about 1.85.  A bf16 product of the library reaches 1220-1270 on this card.  Spreading the vector work differently over the MFMAs is level.
 #pragma once
 #include "fa_bwd_impl.h"
 #include "fa_wide.h"

@@ -11,7 +11,8 @@
 //
 // Measured (bf16, D128, us, 32-row kernel -> this; one box): B8 H16 S4096 full 968 -> 908, causal 535 -> 522, B1 H32 S16384 causal
 // 1930 -> 1830, 1024 queries of 16384 keys Hq 32 Hk 8 262 -> 248.  What bounds it is what the wave issues: per unit 32 MFMAs (512
-// cycles of its port), 112 vector instructions (610), 24 LDS reads; 1570 cycles, of which the matrix pipe is busy 65 %.
+// cycles of its port), 112 vector instructions (610), 24 LDS reads; 1570 cycles, of which the matrix pipe is busy 65 % (52-54 % of
+// the wave time of whole launches, with masked tiles and the ends of items).
 // The parts of an element behind one MFMA: 2 % slower; the rows and the first tile of the next item requested before the results
 // go out: level (full, 512 keys: 4 % faster; long items 1 % slower).
 #pragma once
