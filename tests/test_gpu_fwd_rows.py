@@ -81,6 +81,22 @@ def test_few_rows_meet_the_oracle(case):
         assert (L[seen] - rl[seen]).abs().max().item() <= LSE_ATOL if seen.any() else True
 
 
+@pytest.mark.parametrize('D', [64, 128, 256])
+@pytest.mark.parametrize('parts', [2, 3, 4, 5, 8, 9, 17, 63, 64])
+def test_sums_of_few_and_many_parts(parts, D):
+    """One row block and 128 keys a part (four waves of 32): up to eight parts each thread has all of its columns' (two, or two
+    groups of four), beyond that the threads of a workgroup share them."""
+    from oracle import fa_ref
+    q, k, v, _, _ = make_inputs(1, 5, 1, 1, 128 * parts, D, torch.bfloat16, DEV, seed=parts)
+    f = lambda t: t.float()
+    sm = D ** -0.5
+    ro, rl, _ = fa_ref.attn_fwd_ref(f(q), f(k), f(v), None, sm, 0, 0, 0)
+    lo, _, _ = fa_ref.attn_fwd_ref(q, k, v, None, sm, 0, 0, 0)
+    o, L = _forward(q, k, v, None, sm, False, True)
+    check('out', o, ro, lo, FUDGE['out'])
+    assert (L.view(1, 5, 1) - rl).abs().max().item() <= LSE_ATOL
+
+
 def test_scores_that_grow_and_huge_scores():
     """the reference maximum moves in every step of every wave, and 16-bit scores of 1e4"""
     from oracle import fa_ref
