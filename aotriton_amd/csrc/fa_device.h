@@ -249,22 +249,27 @@ __device__ __forceinline__ float cross_sum(float x) {
 
 // Philox-4x32-10 with counter (c0, c1, 0, 0); Salmon et al. SC'11.  The
 // reference reaches it through Triton's tl.randint4x
-// (modules/flash/kernel/dropout.py:19).
-__device__ __forceinline__ void philox4x32_10(uint32_t c0, uint32_t c1, uint32_t k0, uint32_t k1,
-                                              uint32_t (&w)[4]) {
-  uint32_t c2 = 0, c3 = 0;
-#pragma unroll
-  for (int i = 0; i < 10; ++i) {
+// (modules/flash/kernel/dropout.py:19).  Round by round, so that a kernel can put them behind its MFMAs.
+struct Philox {
+  uint32_t c0, c1, c2, c3;
+  __device__ __forceinline__ void start(uint32_t lo, uint32_t up) { c0 = lo; c1 = up; c2 = 0; c3 = 0; }
+  __device__ __forceinline__ void round(int i, uint32_t k0, uint32_t k1) {
+    k0 += (uint32_t)i * 0x9E3779B9u; k1 += (uint32_t)i * 0xBB67AE85u;
     // one 32x32->64 multiply per product (v_mad_u64_u32) instead of a high and a low half
     const uint64_t p0 = (uint64_t)0xD2511F53u * c0, p1 = (uint64_t)0xCD9E8D57u * c2;
-    const uint32_t hi0 = (uint32_t)(p0 >> 32), lo0 = (uint32_t)p0;
-    const uint32_t hi1 = (uint32_t)(p1 >> 32), lo1 = (uint32_t)p1;
     // (three-input xor: one v_bitop3_b32 with truth table 0x96 instead of two v_xor_b32)
-    const uint32_t n0 = __builtin_amdgcn_bitop3_b32(hi1, c1, k0, 0x96), n2 = __builtin_amdgcn_bitop3_b32(hi0, c3, k1, 0x96);
-    c0 = n0; c1 = lo1; c2 = n2; c3 = lo0;
-    k0 += 0x9E3779B9u; k1 += 0xBB67AE85u;
+    const uint32_t n0 = __builtin_amdgcn_bitop3_b32((uint32_t)(p1 >> 32), c1, k0, 0x96);
+    const uint32_t n2 = __builtin_amdgcn_bitop3_b32((uint32_t)(p0 >> 32), c3, k1, 0x96);
+    c0 = n0; c1 = (uint32_t)p1; c2 = n2; c3 = (uint32_t)p0;
   }
-  w[0] = c0; w[1] = c1; w[2] = c2; w[3] = c3;
+};
+__device__ __forceinline__ void philox4x32_10(uint32_t c0, uint32_t c1, uint32_t k0, uint32_t k1,
+                                              uint32_t (&w)[4]) {
+  Philox p;
+  p.start(c0, c1);
+#pragma unroll
+  for (int i = 0; i < 10; ++i) p.round(i, k0, k1);
+  w[0] = p.c0; w[1] = p.c1; w[2] = p.c2; w[3] = p.c3;
 }
 
 struct DropoutState {

@@ -19,6 +19,11 @@
 // need a mask, the units at the ends of a wave's range and every unit while some row has no
 // reference yet take the plain path: the three stages one after the other, full softmax step.
 //
+// With dropout the rounds of the Philox counters (one per four keys) ride behind the PV MFMAs of the speculative step, a quarter
+// of them per element.  As one block the compiler moved them behind the branch to the full step, where nothing ran next to
+// their 190 instructions (B2 H16 S8192 D256 fp16, us, before -> now: window 1024 568 -> 530, with a bias 647 -> 628; S4096
+// causal 443 -> 408).
+//
 // LDS: two stages of K tiles and two of V tiles (BN keys each); V is staged LV tiles behind K since
 // its consumer runs two units behind.  One barrier per tile.
 #pragma once
@@ -296,7 +301,12 @@ __device__ __forceinline__ void fwd_item_pipe(const FwdArgs& a, const int z, con
                        (reinterpret_cast<uintptr_t>(a.bias) & 15) == 0;
 
   DropoutState ds{};
-  if (kDropout) ds = make_dropout(a.drop, z, h, a.hq, a.seq.max_seqlen_q, a.seq.max_seqlen_k);
+  if (kDropout) {
+    ds = make_dropout(a.drop, z, h, a.hq, a.seq.max_seqlen_q, a.seq.max_seqlen_k);
+    // (the round keys in scalar registers: as vector registers they push the Q operands out)
+    ds.k0 = __builtin_amdgcn_readfirstlane(ds.k0);
+    ds.k1 = __builtin_amdgcn_readfirstlane(ds.k1);
+  }
 
   const int k_lane = c * KSTR + hi * 8;
   // lane-constant part of the V^T operand address (see lds_read_tr8)
@@ -304,14 +314,27 @@ __device__ __forceinline__ void fwd_item_pipe(const FwdArgs& a, const int z, con
   const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 
   // dropout and conversion of one pair of p's into its slot of the P operand
-  auto put_pair = [&](op_t (&pout)[2], int e, float p0, float p1, uint32_t keep) {
+  auto put_pair = [&](op_t (&pout)[2], int e, float p0, float p1, bool keep0, bool keep1) {
     if (kDropout) {
-      p0 = ((keep >> ((e - 1) & 3)) & 1u) ? p0 : 0.f;
-      p1 = ((keep >> (e & 3)) & 1u) ? p1 : 0.f;
+      p0 = keep0 ? p0 : 0.f;
+      p1 = keep1 ? p1 : 0.f;
     }
-    pout[e / 8][e % 8 - 1] = Tr::cvt(p0);      // P is cast to V's dtype for the second GEMM (:274)
-    pout[e / 8][e % 8] = Tr::cvt(p1);
+    // P is cast to V's dtype for the second GEMM (:274)
+    const typename Tr::p2_t p2 = kDropout ? Tr::cvt2(p0, p1) : typename Tr::p2_t{Tr::cvt(p0), Tr::cvt(p1)};
+    pout[e / 8][e % 8 - 1] = p2[0];
+    pout[e / 8][e % 8] = p2[1];
   };
+  // Philox counters of this lane's rows at key 0.  The speculative step takes the upper word for the same along the row (the
+  // second round's first product is then the same for all keys): where the lower word wraps within the row, the whole item
+  // takes the plain path.
+  uint64_t ctr[QB];
+  bool ctr_wraps = false;
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    ctr[qb] = kDropout ? ds.base + (uint64_t)(w_rmin + 32 * qb + c) * ds.stride : 0;
+    ctr_wraps |= kDropout && (uint32_t)ctr[qb] > 0xffffffffu - ds.stride;
+  }
+  const bool no_spec = kDropout && __builtin_amdgcn_ballot_w64(ctr_wraps) != 0;
 
   // Full online-softmax step on the raw scores x of unit u (modified in place): scale, bias,
   // mask, row maximum, lazy move of the reference, exponentials, row sum; O and l follow the
@@ -407,8 +430,8 @@ __device__ __forceinline__ void fwd_item_pipe(const FwdArgs& a, const int z, con
       for (int g = 0; g < 4; ++g) {
         uint32_t keep = 0;
         if (kDropout) keep = dropout_keep4(ds, row, u * 32 + 8 * g + 4 * hi);
-        put_pair(pout[qb], 4 * g + 1, p[4 * g], p[4 * g + 1], keep);
-        put_pair(pout[qb], 4 * g + 3, p[4 * g + 2], p[4 * g + 3], keep);
+        put_pair(pout[qb], 4 * g + 1, p[4 * g], p[4 * g + 1], keep & 1u, keep & 2u);
+        put_pair(pout[qb], 4 * g + 3, p[4 * g + 2], p[4 * g + 3], keep & 4u, keep & 8u);
       }
     }
     have_ref = !any_big;
@@ -499,10 +522,10 @@ __device__ __forceinline__ void fwd_item_pipe(const FwdArgs& a, const int z, con
     ka[1] = *reinterpret_cast<const op_t*>(ks + 16);
     va[0] = lds_read_tr8<T>(vs, VSTR);
     va[1] = lds_read_tr8<T>(vs + (1 / DB) * 16 * VSTR + (1 % DB) * 32, VSTR);
-    float rs[QB], plast[QB];
-    uint32_t keep[QB];
+    float rs[QB], p4[QB][4];      // p of the running four keys, whose keep bits come from one Philox counter
+    Philox rng[QB];
 #pragma unroll
-    for (int qb = 0; qb < QB; ++qb) { rs[qb] = 0.f; plast[qb] = 0.f; keep[qb] = 0; }
+    for (int qb = 0; qb < QB; ++qb) rs[qb] = 0.f;
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < NM; ++i) {
@@ -518,21 +541,44 @@ __device__ __forceinline__ void fwd_item_pipe(const FwdArgs& a, const int z, con
 #pragma unroll
         for (int q = 0; q < EPS; ++q) {
           const int e = EPS * k + q;
-          if (kDropout && e % 4 == 0)
-            keep[qb] = dropout_keep4(ds, w_rmin + 32 * qb + c, (g - 1) * 32 + 8 * (e / 4) + 4 * hi);
-          float xv = x[qb][e];
           // (without a bias the speculative step is only taken with a positive scale: sc = qk_scale)
           float p;
-          if (kBias) p = fast_exp2(__builtin_fmaf(xv, qk_scale, (float)bin[qb][e / 4][e % 4] * kLog2e) - msc_ref[qb]);
-          else p = fast_exp2(__builtin_fmaf(xv, qk_scale, -msc_ref[qb]));
+          if (kBias && kDropout)      // (one multiply-add instead of two operations; without dropout nothing waits for them)
+            p = fast_exp2(__builtin_fmaf(x[qb][e], qk_scale, __builtin_fmaf((float)bin[qb][e / 4][e % 4], kLog2e, -msc_ref[qb])));
+          else if (kBias)
+            p = fast_exp2(__builtin_fmaf(x[qb][e], qk_scale, (float)bin[qb][e / 4][e % 4] * kLog2e) - msc_ref[qb]);
+          else
+            p = fast_exp2(__builtin_fmaf(x[qb][e], qk_scale, -msc_ref[qb]));
           rs[qb] += p;      // the row sum is over the fp32, undropped p (fwd_kernel_inner.py:213-214)
-          if (e & 1) put_pair(pout[qb], e, plast[qb], p, keep[qb]);
-          else plast[qb] = p;
+          p4[qb][e % 4] = p;
+          if (!kDropout && (e & 1)) put_pair(pout[qb], e, p4[qb][e % 4 - 1], p, true, true);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
       o[qb][k % DB] = Tr::mfma(va[k % 3], pin[qb][k / DB], o[qb][k % DB]);
       __builtin_amdgcn_sched_barrier(0);
+      if (kSpec && kDropout) {
+        // behind the other MFMA, a quarter of the Philox rounds of each element's four
+#pragma unroll
+        for (int q = 0; q < EPS; ++q) {
+          const int e = EPS * k + q;
+          constexpr int kRound[5] = {0, 3, 5, 8, 10};
+          if (e % 4 == 0) rng[qb].start((uint32_t)ctr[qb] + (uint32_t)((g - 1) * 8 + 2 * (e / 4) + hi), (uint32_t)(ctr[qb] >> 32));
+#pragma unroll
+          for (int r = kRound[e % 4]; r < kRound[e % 4 + 1]; ++r) rng[qb].round(r, ds.k0, ds.k1);
+          if (e % 4 == 3) {      // word order along the row: dropout_keep4
+            put_pair(pout[qb], e - 2, p4[qb][0], p4[qb][1], (int32_t)rng[qb].c0 > ds.thr, (int32_t)rng[qb].c2 > ds.thr);
+            put_pair(pout[qb], e, p4[qb][2], p4[qb][3], (int32_t)rng[qb].c1 > ds.thr, (int32_t)rng[qb].c3 > ds.thr);
+          }
+        }
+      }
+      // (P and its dropout are not needed where some row takes the full step, and the compiler moves what they are made of
+      // out of the MFMAs' shadow to behind that branch unless it is pinned here)
+      if (kSpec && kDropout) {
+        asm volatile("" : "+v"(rng[qb].c0), "+v"(rng[qb].c1), "+v"(rng[qb].c2), "+v"(rng[qb].c3));
+        if ((EPS * (k + 1)) % 4 == 0) asm volatile("" : "+v"(pout[qb][(EPS * (k + 1) - 1) / 8]));
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
     if (!kSpec) return false;
     // a row whose p grew too far (also inf and NaN) takes the full step on the untouched scores
@@ -544,9 +590,11 @@ __device__ __forceinline__ void fwd_item_pipe(const FwdArgs& a, const int z, con
     for (int qb = 0; qb < QB; ++qb) l_i[qb] += rs[qb];
     return false;
   };
-  // unit g-1 may take the speculative step (given a reference in every row)
+  // unit g-1 may take the speculative step (given a reference in every row).  (With dropout what holds for the whole item is
+  // part of the bound: as conditions of their own the compiler makes a copy of the loops for each, and 500 registers spill.)
+  const int spec_last = kDropout && ((kBias ? !bias_co : prescale) || no_spec) ? -1 : u1;
   auto spec_ok = [&](int g) -> bool {
-    return g <= u1 && unit_sees_all(g - 1) && (kBias ? bias_co : !prescale);
+    return g <= spec_last && unit_sees_all(g - 1) && (kDropout || (kBias ? bias_co : !prescale));
   };
 
   // ---- main loop ---------------------------------------------------------------------------------------------

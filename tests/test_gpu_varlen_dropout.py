@@ -297,6 +297,28 @@ def test_per_head_counter_term_wraps_in_int32():
     torch.cuda.empty_cache()
 
 
+@pytest.mark.parametrize('bias', [False, True])
+@pytest.mark.parametrize('causal', [False, True])
+def test_counter_word_wraps_within_rows(causal, bias):
+    """Head dim 256: the forward's speculative step keeps the upper counter word along a row, and items in which the
+    lower word wraps within one take the other step.  The wrap lies inside row 37 of head 1: head 0 and the later items
+    are away from it."""
+    from _util import keep_mask_from_oracle, ref_fwd
+    from aotriton_amd import flash
+    from aotriton_amd.autograd import AttentionExtraArgs, attention
+    B, H, S, D, p = 1, 2, 256, 256, 0.25
+    q, k, v, b, _ = make_inputs(B, H, H, S, S, D, torch.float16, DEV, seed=9, bias=bias)
+    at = S * (S // 4) + 37 * (S // 4) + 21
+    ext = AttentionExtraArgs(return_logsumexp=True, philox_seed=0x9e3779b97f4a7c15, philox_offset1=(1 << 32) - at, philox_offset2=0)
+    sm = 1.0 / math.sqrt(D)
+    o, _, L = attention(q, k, v, b, causal, sm, p, ext)
+    ct, wl, wr = flash.translate_causal(causal)
+    keep = keep_mask_from_oracle(B, H, S, S, p, ext.philox_seed, ext.philox_offset1, DEV)
+    rh = ref_fwd(q, k, v, b, sm, ct, wl, wr, p, keep, torch.float32)
+    rl = ref_fwd(q, k, v, b, sm, ct, wl, wr, p, keep, torch.float16)
+    check('out', o, rh[0], rl[0], FUDGE['out'])
+
+
 def test_config5_mask_first_words_and_popcount():
     """Mask of the benchmark configuration with dropout (seed 0x1234, offset 0, p=0.1, 8192x8192) on sampled
     (b, h) slices: bit-exact rows against the oracle and a keep-rate check."""
