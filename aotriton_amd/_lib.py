@@ -99,6 +99,8 @@ SYMBOLS = {
     'fa_attn_fwd': (ctypes.c_int, [P(fa_fwd_params), ctypes.c_int32, ctypes.c_void_p, P(fa_options)]),
     'fa_attn_fwd_alloc': (ctypes.c_int, [P(fa_fwd_params), ctypes.c_int32, ctypes.c_void_p, P(fa_options),
                                          ctypes.c_void_p]),
+    'fa_attn_fwd_key_mask': (ctypes.c_int, [P(fa_fwd_params), ctypes.c_int32, ctypes.c_void_p, P(fa_options),
+                                            ctypes.c_void_p]),
     'fa_attn_bwd': (ctypes.c_int, [P(fa_bwd_params), ctypes.c_int32, ctypes.c_void_p, P(fa_options)]),
     'fa_v2_attn_fwd': (ctypes.c_int, [P(fa_tensor4)] * 4 + [ctypes.c_float, P(fa_tensor2), P(fa_tensor4), ctypes.c_float,
                                       P(fa_tensor0), P(fa_tensor0), ctypes.c_int64, P(fa_tensor0), P(fa_tensor0),

@@ -1186,10 +1186,11 @@ int fa_debug_simulate_encoded_softmax(const fa_tensor4* r, float dropout_p, cons
 }
 
 static int attn_fwd_impl(const fa_fwd_params* p, int32_t params_version, void* hip_stream,
-                         const fa_options* options, fa_allocator* alloc) {
+                         const fa_options* options, fa_allocator* alloc, bool key_mask = false) {
   Shape s{};
   int e = validate_fwd(p, params_version, options, &s);
   if (e != FA_SUCCESS) return e;
+  if (key_mask && (s.elementwise || !is_16bit(p->Q.dtype) || s.d > 128 || s.dropout || s.num_seqlens != 0)) return FA_ERROR_NOT_SUPPORTED;
   hipStream_t stream = static_cast<hipStream_t>(hip_stream);
   const DeviceInfo* dev = device_of_stream(stream);
   if (dev == nullptr || !dev->is_gfx950) return FA_ERROR_NO_BINARY_FOR_GPU;
@@ -1244,6 +1245,8 @@ static int attn_fwd_impl(const fa_fwd_params* p, int32_t params_version, void* h
 
   hipError_t err;
   const FwdPlan plan = fwd_plan(p->Q.dtype, s, p->causal_type, p->window_left, p->window_right, dev->num_cu);
+  if (key_mask && !plan.rows && plan.splits > 1) return FA_ERROR_NOT_SUPPORTED;      // (split tiles take any bias as one of rows)
+  a.key_mask = key_mask ? 1 : 0;
   void* scratch = nullptr;
   bool held = false;
   if (plan.splits > 1) {
@@ -1290,6 +1293,16 @@ int fa_attn_fwd(const fa_fwd_params* p, int32_t params_version, void* hip_stream
 int fa_attn_fwd_alloc(const fa_fwd_params* p, int32_t params_version, void* hip_stream, const fa_options* options,
                       fa_allocator* alloc) {
   return attn_fwd_impl(p, params_version, hip_stream, options, alloc);
+}
+
+int fa_attn_fwd_key_mask(const fa_fwd_params* p, int32_t params_version, void* hip_stream, const fa_options* options,
+                         fa_allocator* alloc) {
+  if (p == nullptr || p->B.ptr == nullptr || p->B.dtype != FA_DTYPE_UINT8) return FA_ERROR_INVALID_VALUE;
+  if (p->B.sizes[2] > 1 && p->B.strides[2] != 0) return FA_ERROR_NOT_SUPPORTED;
+  fa_fwd_params q = *p;
+  q.B.dtype = p->Q.dtype;
+  q.B.strides[2] = 0;
+  return attn_fwd_impl(&q, params_version, hip_stream, options, alloc, true);
 }
 
 // kernel_slot < 0: the whole backward of the chosen backend; otherwise only that

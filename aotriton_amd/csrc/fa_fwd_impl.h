@@ -161,10 +161,13 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
   // bias every wave would carry 32 copies of the row through its row area.  (A template flag: as one more
   // run-time case it cost the general bias 5-15 % in spills.)
   static_assert(kBias || !kKeyBias, "a bias of keys is a bias");
-  const T* kb_next = kKeyBias ? reinterpret_cast<const T*>(a.bias) + (int64_t)si.batch_index * a.sb_z + (int64_t)h * a.sb_h +
-                                 (int64_t)(br.lo * BN + tid) * a.sb_n
-                           : nullptr;
-  float kb_reg = 0.f;
+  // FwdArgs::key_mask: it is a boolean mask of keys and becomes 0 or -inf here (as a launch of its own that took 4 of the 24 us
+  // of B16 H12 S384 D64).
+  const int kb_size = kKeyBias && a.key_mask ? 1 : 2;
+  const char* kb_next = kKeyBias ? reinterpret_cast<const char*>(a.bias) + ((int64_t)si.batch_index * a.sb_z + (int64_t)h * a.sb_h +
+                                                                            (int64_t)(br.lo * BN + tid) * a.sb_n) * kb_size
+                                 : nullptr;
+  uint32_t kb_raw = 0;      // as it lies; what it stands for is formed a tile later, when it has arrived
   float* const kb_lds = reinterpret_cast<float*>(smem_raw + SM::KEYB_OFF);
 
   DropoutState ds{};
@@ -204,8 +207,9 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
     for (int i = 0; i < CH; ++i)
       vreg[i] = __builtin_bit_cast(op_t, __builtin_amdgcn_raw_buffer_load_b128(vrs, vvoff, i * vsoff, 0));
     if (kKeyBias && tid < BN) {
-      kb_reg = tid < rows ? (float)*kb_next * kLog2e : 0.f;
-      kb_next += (int64_t)BN * a.sb_n;
+      kb_raw = a.key_mask ? 1 : 0;
+      if (tid < rows) kb_raw = a.key_mask ? *reinterpret_cast<const uint8_t*>(kb_next) : *reinterpret_cast<const uint16_t*>(kb_next);
+      kb_next += (int64_t)BN * a.sb_n * kb_size;
     }
     kt += k_step; vt += v_step; rows_left -= BN;
   };
@@ -240,7 +244,9 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
     for (int i = 0; i < CH; ++i) *reinterpret_cast<op_t*>(ks + i * RPI * KSTR) = kreg[i];
 #pragma unroll
     for (int i = 0; i < CH; ++i) *reinterpret_cast<op_t*>(vs + i * RPI * VSTR) = vreg[i];
-    if (kKeyBias && tid < BN) kb_lds[stage * BN + tid] = kb_reg;
+    if (kKeyBias && tid < BN)
+      kb_lds[stage * BN + tid] = a.key_mask ? (kb_raw != 0 ? 0.f : -__builtin_inff())
+                                            : (float)__builtin_bit_cast(T, (uint16_t)kb_raw) * kLog2e;
   };
 
   // ---- online softmax state --------------------------------------------------

@@ -111,8 +111,12 @@ void fwd_rows_kernel(const FwdArgs a) {
   const T* vbase = reinterpret_cast<const T*>(a.v) + (int64_t)si.batch_index * a.sv.z + (int64_t)hk * a.sv.h +
                    (int64_t)si.k_start * a.sv.s;
   const T* bptr = nullptr;
-  if (kBias)
-    bptr = reinterpret_cast<const T*>(a.bias) + (int64_t)si.batch_index * a.sb_z + (int64_t)h * a.sb_h + (int64_t)row * a.sb_m;
+  const uint8_t* mptr = nullptr;      // FwdArgs::key_mask
+  if (kBias) {
+    const int64_t at = (int64_t)si.batch_index * a.sb_z + (int64_t)h * a.sb_h + (int64_t)row * a.sb_m;
+    bptr = reinterpret_cast<const T*>(a.bias) + at;
+    mptr = reinterpret_cast<const uint8_t*>(a.bias) + at;
+  }
   const bool bias_vec = kBias && a.sb_n == 1 && ((a.sb_m | a.sb_h | a.sb_z) & 3) == 0 &&
                         (reinterpret_cast<uintptr_t>(a.bias) & 7) == 0;
 
@@ -167,7 +171,14 @@ void fwd_rows_kernel(const FwdArgs a) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) s[i] *= qk_scale;
     const int n0 = b * 32;
-    if (kBias) {
+    if (kBias && a.key_mask) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        int n = n0 + 8 * (i / 4) + 4 * hi + (i % 4);
+        n = n < si.seqlen_k ? n : si.seqlen_k - 1;
+        s[i] = mptr[(int64_t)n * a.sb_n] != 0 ? s[i] : -__builtin_inff();
+      }
+    } else if (kBias) {
       if (bias_vec && n0 + 32 <= si.seqlen_k) {
 #pragma unroll
         for (int g = 0; g < 4; ++g) {

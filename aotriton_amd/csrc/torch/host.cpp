@@ -350,6 +350,14 @@ const c10::TypedOperatorHandle<FwdSig>& forward_op() {
                              .findSchemaOrThrow("aotriton_amd::flash_attention_forward", "").typed<FwdSig>();
   return op;
 }
+// flash_attention_forward_key_mask(q, k, v, mask, sm_scale): a boolean mask that is the same for all query rows, 4-D and
+// broadcast here
+using MaskSig = std::tuple<Tensor, Tensor>(const Tensor&, const Tensor&, const Tensor&, const Tensor&, double);
+const c10::TypedOperatorHandle<MaskSig>& key_mask_op() {
+  static const auto op = c10::Dispatcher::singleton()
+                             .findSchemaOrThrow("aotriton_amd::flash_attention_forward_key_mask", "").typed<MaskSig>();
+  return op;
+}
 const c10::TypedOperatorHandle<BwdSig>& backward_op() {
   static const auto op = c10::Dispatcher::singleton()
                              .findSchemaOrThrow("aotriton_amd::flash_attention_backward", "").typed<BwdSig>();
@@ -372,6 +380,46 @@ std::tuple<Tensor, Tensor> forward_kernel(const Tensor& q, const Tensor& k, cons
   Tensor o = at::empty({q.size(0), q.size(1), q.size(2), v.size(3)}, q.options());
   Tensor lse = at::empty({q.size(0) * q.size(1), q.size(2)}, q.options().dtype(at::kFloat));
   check_rc(run_forward(p, lse, o, Tensor()), false);
+  return {std::move(o), std::move(lse)};
+}
+
+// log(1) = 0 where the key is visible, log(0) = -inf where it is not: the additive mask in one kernel
+Tensor additive_mask(const Tensor& mask, const at::TensorOptions& like) {
+  Tensor additive = at::empty_like(mask, like);
+  at::log_out(additive, mask);
+  return additive;
+}
+Tensor unit_stride(const Tensor& t) { return t.stride(-1) == 1 ? t : t.contiguous(); }
+Tensor broadcast_bias(const Tensor& m, const Tensor& q, const Tensor& k) {
+  return unit_stride(m.expand({q.size(0), q.size(1), q.size(2), k.size(2)}));
+}
+std::tuple<Tensor, Tensor> forward_additive(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& mask, double sm_scale) {
+  const Tensor none = at::empty({0}, q.options().dtype(at::kUInt64));      // not read
+  return forward_op().call(q, k, v, std::optional<Tensor>(broadcast_bias(additive_mask(mask, q.options()), q, k)), 0.0, FA_CAUSAL_NONE, 0, 0,
+                           sm_scale, none, none);
+}
+
+std::tuple<Tensor, Tensor> key_mask_kernel(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& mask, double sm_scale) {
+  TORCH_CHECK(mask.scalar_type() == at::kBool && mask.dim() == 4 && mask.size(2) == 1 && mask.device() == q.device(),
+              "a boolean (.., .., 1, keys) mask on the device of the queries");
+  const c10::DeviceGuard guard(q.device());
+  fa_fwd_params p{};
+  fill_common(p, q, k, v, Tensor(), sm_scale, 0.0, Mask{}, Varlen{});
+  const Tensor m = mask.expand({q.size(0), q.size(1), 1, k.size(2)});
+  Tensor o = at::empty({q.size(0), q.size(1), q.size(2), v.size(3)}, q.options());
+  Tensor lse = at::empty({q.size(0) * q.size(1), q.size(2)}, q.options().dtype(at::kFloat));
+  p.B.ptr = m.numel() > 0 ? m.data_ptr() : nullptr;
+  for (int i = 0; i < 4; ++i) {
+    p.B.sizes[i] = (uint64_t)(i == 2 ? q.size(2) : m.size(i));
+    p.B.strides[i] = (uint64_t)(i == 2 ? 0 : m.stride(i));
+  }
+  p.B.dtype = FA_DTYPE_UINT8;
+  TORCH_CHECK(view2(lse, &p.L) && view4(o, &p.Out), "outputs");
+  Scratch scratch;
+  const int rc = p.B.ptr == nullptr ? (int)FA_ERROR_NOT_SUPPORTED
+                                    : fa_attn_fwd_key_mask(&p, FA_FWD_PARAMS_VERSION, current_stream(), nullptr, &scratch.c);
+  if (rc == FA_ERROR_NOT_SUPPORTED) return forward_additive(q, k, v, mask, sm_scale);
+  check_rc(rc, false);
   return {std::move(o), std::move(lse)};
 }
 
@@ -457,6 +505,13 @@ std::tuple<Tensor, Tensor> forward_autograd(const Tensor& q, const Tensor& k, co
   return {r[0], r[1]};
 }
 
+std::tuple<Tensor, Tensor> key_mask_autograd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& mask, double sm_scale) {
+  if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad()))
+    return forward_additive(q, k, v, mask, sm_scale);      // (the backward takes an additive mask)
+  at::AutoDispatchBelowADInplaceOrView below;
+  return key_mask_op().call(q, k, v, mask, sm_scale);
+}
+
 // The backward op has no derivative of its own.  Its results say so when something asks for one; without
 // an Autograd kernel PyTorch would hand back undefined gradients with a warning, and a double backward
 // through flash_attention_forward would run this op on zeros.
@@ -507,6 +562,7 @@ TORCH_LIBRARY(aotriton_amd, m) {
   m.def("flash_attention_forward(Tensor q, Tensor k, Tensor v, Tensor? bias, float dropout_p, SymInt causal_type, "
         "SymInt window_left, SymInt window_right, float sm_scale, Tensor philox_seed, Tensor philox_offset) -> (Tensor, Tensor)",
         compliant);
+  m.def("flash_attention_forward_key_mask(Tensor q, Tensor k, Tensor v, Tensor mask, float sm_scale) -> (Tensor, Tensor)", compliant);
   m.def("flash_attention_backward(Tensor dout, Tensor q, Tensor k, Tensor v, Tensor? bias, Tensor out, Tensor lse, "
         "float dropout_p, SymInt causal_type, SymInt window_left, SymInt window_right, float sm_scale, "
         "Tensor philox_seed, Tensor philox_offset, bool need_dbias, SymInt backend) -> (Tensor, Tensor, Tensor, Tensor)",
@@ -515,10 +571,12 @@ TORCH_LIBRARY(aotriton_amd, m) {
 TORCH_LIBRARY_IMPL(aotriton_amd, CUDA, m) {
   m.impl("philox_state", &philox_kernel);
   m.impl("flash_attention_forward", &forward_kernel);
+  m.impl("flash_attention_forward_key_mask", &key_mask_kernel);
   m.impl("flash_attention_backward", &backward_kernel);
 }
 TORCH_LIBRARY_IMPL(aotriton_amd, Autograd, m) {
   m.impl("flash_attention_forward", &forward_autograd);
+  m.impl("flash_attention_forward_key_mask", &key_mask_autograd);
   m.impl("flash_attention_backward", &backward_autograd);
 }
 
@@ -774,14 +832,13 @@ PyObject* py_attention_varlen(PyObject*, PyObject* const* argv, Py_ssize_t n) {
 
 struct Sdpa {
   Tensor q, k, v, bias;
+  Tensor key_mask;      // instead of the bias: a boolean mask of one row, 4-D, not broadcast yet
   double scale = 0;
 };
 
-Tensor unit_stride(const Tensor& t) { return t.stride(-1) == 1 ? t : t.contiguous(); }
-
 // sdpa.py's prepare(): argument checks, unit last strides, the mask as an additive (B, H, L, S) bias
 Sdpa prepare(const Tensor& query, const Tensor& key, const Tensor& value, const Tensor& mask, bool is_causal,
-             std::optional<double> scale, bool gqa) {
+             std::optional<double> scale, bool gqa, bool take_key_mask = false) {
   TORCH_CHECK_VALUE(query.dim() == 4 && key.dim() == 4 && value.dim() == 4, "expected (batch, heads, seq, head_dim) tensors");
   TORCH_CHECK_VALUE(!(is_causal && mask.defined()), "attn_mask and is_causal cannot both be set");
   const int64_t hq = query.size(1), hk = key.size(1);
@@ -795,15 +852,18 @@ Sdpa prepare(const Tensor& query, const Tensor& key, const Tensor& value, const 
   if (mask.defined()) {
     Tensor m = mask;
     if (m.scalar_type() == at::kBool) {
-      // log(1) = 0 where the key is visible, log(0) = -inf where it is not: the additive mask in one kernel
-      Tensor additive = at::empty_like(m, s.q.options());
-      at::log_out(additive, m);
-      m = additive;
+      if (take_key_mask && m.dim() > 0 && m.dim() <= 4 && (m.dim() == 1 || m.size(-2) == 1) && m.size(-1) == s.k.size(2) &&
+          m.device() == s.q.device()) {
+        while (m.dim() < 4) m = m.unsqueeze(0);
+        s.key_mask = m;
+        return s;
+      }
+      m = additive_mask(m, s.q.options());
     } else if (m.scalar_type() != s.q.scalar_type()) {
       m = m.to(s.q.scalar_type());
     }
     while (m.dim() < 4) m = m.unsqueeze(0);
-    s.bias = unit_stride(m.expand({s.q.size(0), hq, s.q.size(2), s.k.size(2)}));
+    s.bias = broadcast_bias(m, s.q, s.k);
   }
   return s;
 }
@@ -853,20 +913,24 @@ PyObject* py_sdpa_ops(PyObject*, PyObject* const* argv, Py_ssize_t n) {
   Tensor out;
   {
     pybind11::gil_scoped_release no_gil;
-    const Sdpa s = prepare(in.q, in.k, in.v, in.mask, in.causal, in.scale, in.gqa);
-    Tensor seed, offset;
-    if (in.dropout_p > 0) {
-      static const auto op = c10::Dispatcher::singleton().findSchemaOrThrow("aotriton_amd::philox_state", "")
-                                 .typed<std::tuple<Tensor, Tensor>(const Tensor&, c10::SymInt)>();
-      const int64_t per_row = (s.k.size(2) + 3) / 4;      // Philox counters per query row
-      std::tie(seed, offset) = op.call(s.q, s.q.size(0) * s.q.size(1) * s.q.size(2) * per_row);
+    const Sdpa s = prepare(in.q, in.k, in.v, in.mask, in.causal, in.scale, in.gqa, in.dropout_p == 0);
+    if (s.key_mask.defined()) {
+      out = std::get<0>(key_mask_op().call(s.q, s.k, s.v, s.key_mask, s.scale));
     } else {
-      seed = offset = at::empty({0}, s.q.options().dtype(at::kUInt64));      // not read
+      Tensor seed, offset;
+      if (in.dropout_p > 0) {
+        static const auto op = c10::Dispatcher::singleton().findSchemaOrThrow("aotriton_amd::philox_state", "")
+                                   .typed<std::tuple<Tensor, Tensor>(const Tensor&, c10::SymInt)>();
+        const int64_t per_row = (s.k.size(2) + 3) / 4;      // Philox counters per query row
+        std::tie(seed, offset) = op.call(s.q, s.q.size(0) * s.q.size(1) * s.q.size(2) * per_row);
+      } else {
+        seed = offset = at::empty({0}, s.q.options().dtype(at::kUInt64));      // not read
+      }
+      const int64_t edge = in.causal ? (int64_t)FA_WINDOW_TOP_LEFT : 0;
+      out = std::get<0>(forward_op().call(s.q, s.k, s.v, s.bias.defined() ? std::optional<Tensor>(s.bias) : std::nullopt,
+                                          in.dropout_p, in.causal ? FA_CAUSAL_WINDOWED : FA_CAUSAL_NONE, edge, edge, s.scale,
+                                          seed, offset));
     }
-    const int64_t edge = in.causal ? (int64_t)FA_WINDOW_TOP_LEFT : 0;
-    out = std::get<0>(forward_op().call(s.q, s.k, s.v, s.bias.defined() ? std::optional<Tensor>(s.bias) : std::nullopt,
-                                        in.dropout_p, in.causal ? FA_CAUSAL_WINDOWED : FA_CAUSAL_NONE, edge, edge, s.scale,
-                                        seed, offset));
   }
   return wrap(out);
   END_HANDLE_TH_ERRORS

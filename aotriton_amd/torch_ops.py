@@ -6,6 +6,8 @@ so that code using them can be traced by torch.compile / AOTAutograd.
 
     flash_attention_forward(q, k, v, bias, dropout_p, causal_type, window_left, window_right, sm_scale, seed, offset)
         -> Out (B, Hq, Sq, Dv), logsumexp (B*Hq, Sq) fp32
+    flash_attention_forward_key_mask(q, k, v, mask, sm_scale)
+        -> the same, under a boolean (B or 1, Hq or 1, 1, Sk) mask that the kernels read as it is
     flash_attention_backward(dout, q, k, v, bias, out, lse, dropout_p, causal_type, window_left, window_right,
                              sm_scale, seed, offset, need_dbias, backend)
         -> dQ, dK, dV, dB (empty unless need_dbias); backend: -1 the library's choice, 0 split, 1 fused
@@ -52,6 +54,13 @@ def _(like, increment):
 
 @torch.library.register_fake('aotriton_amd::flash_attention_forward')
 def _(q, k, v, bias, dropout_p, causal_type, window_left, window_right, sm_scale, philox_seed, philox_offset):
+    o = torch.empty((q.shape[0], q.shape[1], q.shape[2], v.shape[3]), device=q.device, dtype=q.dtype)
+    lse = torch.empty((q.shape[0] * q.shape[1], q.shape[2]), device=q.device, dtype=torch.float32)
+    return o, lse
+
+
+@torch.library.register_fake('aotriton_amd::flash_attention_forward_key_mask')
+def _(q, k, v, mask, sm_scale):
     o = torch.empty((q.shape[0], q.shape[1], q.shape[2], v.shape[3]), device=q.device, dtype=q.dtype)
     lse = torch.empty((q.shape[0] * q.shape[1], q.shape[2]), device=q.device, dtype=torch.float32)
     return o, lse

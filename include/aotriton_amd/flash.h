@@ -254,6 +254,12 @@ typedef struct fa_allocator {
 } fa_allocator;
 FA_API int fa_attn_fwd_alloc(const fa_fwd_params* params, int32_t params_version, void* hip_stream,
                              const fa_options* options, fa_allocator* alloc);
+/* The same with a boolean mask of keys as the bias: B of dtype FA_DTYPE_UINT8 and of one row (row stride 0, or one query), 0
+ * where a key is hidden.  Takes dense 16-bit calls of aligned rows, head dims up to 128, without dropout, and of those not the
+ * ones whose tiles it would split along the keys (fa_query_fwd_config); for any other it returns FA_ERROR_NOT_SUPPORTED, with
+ * nothing launched. */
+FA_API int fa_attn_fwd_key_mask(const fa_fwd_params* params, int32_t params_version, void* hip_stream,
+                                const fa_options* options, fa_allocator* allocator);
 
 /* v3::flash::attn_bwd -- include/aotriton/flash.h:176-180,
  * modules/flash/csrc/attn_bwd.cc:55-160.

@@ -57,3 +57,47 @@ def test_key_masks(case):
     want = torch.matmul(p, v.double())
     # P rounded to the 16-bit type, the fp32 sums, the result rounded: 3 roundings of the type in the norm
     assert ((o.double() - want).norm() / want.norm()).item() < 3 * torch.finfo(dt).eps / 2
+
+
+BOOL = KEYS + [
+    (1, 16, 1, 3000, 64, BF),              # packed rows, split keys
+    (4, 16, 142, 142, 80, HF),             # packed rows
+    (2, 16, 7, 70, 128, BF),
+    (16, 32, 300, 300, 128, HF),           # whole tiles
+    (40, 32, 520, 200, 64, BF),
+    (1, 4, 1030, 4099, 128, BF),           # split tiles, other head dims and types: the mask is made additive first
+    (2, 8, 200, 96, 256, BF),
+    (2, 4, 60, 50, 64, torch.float32),
+    (2, 4, 60, 50, 36, HF),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('form', ['batch', 'head', 'one', 'vector', 'strided', 'one key', 'hidden'])
+@pytest.mark.parametrize('case', BOOL, ids=_id)
+def test_boolean_key_masks_are_the_additive_ones(case, form):
+    """To the bit: the forward reads the boolean mask as 0 and -inf."""
+    from aotriton_amd.torch_ops import scaled_dot_product_attention as sdpa
+    B, H, Sq, Sk, D, dt = case
+    g = torch.Generator(device='cuda').manual_seed(5)
+    q, k, v = (torch.randn(B, H, s, D, device='cuda', generator=g).to(dt) for s in (Sq, Sk, Sk))
+    shape = {'batch': (B, 1, 1, Sk), 'head': (B, H, 1, Sk), 'one': (1, 1, 1, Sk), 'vector': (Sk,), 'strided': (B, 1, 1, 3 * Sk),
+             'one key': (B, 1, 1, 1), 'hidden': (B, 1, 1, Sk)}[form]
+    mask = torch.rand(shape, device='cuda', generator=g) < 0.7
+    if form == 'strided':
+        mask = mask[..., 1::3]
+    if form == 'hidden':      # (an element of the batch without a key: zeros)
+        mask[B - 1] = False
+    additive = torch.zeros(mask.shape, device='cuda', dtype=dt).masked_fill(~mask, float('-inf'))
+    assert torch.equal(sdpa(q, k, v, attn_mask=mask), sdpa(q, k, v, attn_mask=additive))
+    # the route that keeps what the backward needs takes the additive mask
+    qg = q.clone().requires_grad_()
+    og = sdpa(qg, k, v, attn_mask=mask)
+    assert og.requires_grad and torch.equal(og, sdpa(q, k, v, attn_mask=additive))
+
+
+def test_fake_key_mask_op():
+    import aotriton_amd.torch_ops  # noqa: F401
+    q = torch.empty(2, 4, 8, 64, device='meta', dtype=HF)
+    o, lse = torch.ops.aotriton_amd.flash_attention_forward_key_mask(q, q, q, torch.empty(2, 1, 1, 8, device='meta', dtype=torch.bool), 1.0)
+    assert o.shape == q.shape and lse.shape == (8, 8)
