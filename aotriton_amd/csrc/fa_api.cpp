@@ -780,7 +780,8 @@ int64_t ds_workspace_need(const fa_bwd_params* p, const Shape& s, int* ntq, int*
   if (s.elementwise || !is_16bit(p->Q.dtype) || (s.d != 64 && s.d != 128 && s.d != 256) || s.num_seqlens != 0 ||
       s.batch <= 0 || s.max_sq <= 0 || s.max_sk <= 0)
     return 0;
-  // dB leaves the dQ-from-dS kernel as 16-byte pieces of its rows, or is left to the recomputing one; so are small
+  // dB leaves the dQ-from-dS kernel as 16-byte pieces of its rows, wherever they start (rows at odd places left to the recomputing
+  // one: B9 H16 S1007 D64 bf16 forward + backward 732 us, stored 576; B16 H12 S700 fp16 520 -> 383); columns that lie apart are left to the recomputing one; so are small
   // calls, where the third launch costs what is saved (us forward + backward, recomputing -> stored: B2 H8 S256 D64
   // 50 -> 53, B8 H12 S512 D64 118 -> 100, D128 148 -> 132, D256 468 -> 420, B16 H16 S1024 D64 842 -> 795, causal 670 -> 579),
   // and long rows at D = 64.  There (us of the backward alone, recomputing -> stored, B1): H8 S4096 causal 312 -> 300, H16
@@ -789,14 +790,13 @@ int64_t ds_workspace_need(const fa_bwd_params* p, const Shape& s, int* ntq, int*
   // against visible pairs would tell them apart)
   if (p->DB.ptr != nullptr &&
       ((int64_t)s.batch * s.hq * s.max_sq * s.max_sk < (int64_t)1 << 22 || (s.d == 64 && s.max_sk > 4096) ||
-       p->DB.strides[3] != 1 || ((p->DB.strides[0] | p->DB.strides[1] | p->DB.strides[2]) & 7) != 0 ||
-       (reinterpret_cast<uintptr_t>(p->DB.ptr) & 15) != 0))
+       p->DB.strides[3] != 1))
     return 0;
   // the 64-column build: 2 bytes per pair are too many for its little GEMM work unless the dQ kernel is
   // spared a bias or the Philox arithmetic (same box, stored / recomputing: 1.05-1.14 plain, 0.69-0.81 with either)
   if (s.d == 64 && !s.dropout && !s.bias) return 0;
   int64_t tile_bytes = 0;
-  fa::ds_tile_counts(p->Q.dtype, s.d, s.bias, s.dropout, s.max_sq, s.max_sk, ntq, ntk, &tile_bytes);
+  fa::ds_tile_counts(s.d, s.max_sq, s.max_sk, ntq, ntk, &tile_bytes);
   *ds_bytes = (int64_t)s.batch * s.hq * *ntq * *ntk * tile_bytes;
   *stat_bytes = (s.row_stats * 4 + 255) & ~(int64_t)255;
   return *ds_bytes + 2 * *stat_bytes;
@@ -837,6 +837,9 @@ DkdvParts dkdv_parts(const fa_bwd_params* p, const Shape& s, int num_cu) {
   }
   const double t_step = (s.d == 64 ? 2.3 : s.d == 128 ? 1.9 : 2.1) * (s.dropout ? 1.7 : 1.0) * (s.bias ? 1.3 : 1.0);
   double best = group * most * t_step + 7;
+  // (at D = 64 with a bias and no dropout parts share CUs, kTwoDkDv, and level estimates are worth taking: us of the backward
+  // with 1 / 2 / 3 / 4 parts, S1024: B1 H8 52.9 / 48.5 / 46.1 / 44.1, B2 H8 55.8 / 53.2 / 56.3 / 55.1, B1 H16 55 / 52.3 / 55 / 54)
+  const double gain = s.d == 64 && s.bias && !s.dropout ? 1.02 : 0.95;
   for (int heads = 1; heads <= group; ++heads) {
     if (group % heads != 0) continue;
     for (int tiles = 1; tiles <= 16 && tiles <= most; ++tiles) {
@@ -844,7 +847,7 @@ DkdvParts dkdv_parts(const fa_bwd_params* p, const Shape& s, int num_cu) {
       const int64_t wgs = items * heads * tiles, rounds = (wgs + num_cu - 1) / num_cu;
       const double t = rounds * ((double)(group / heads) * ((most + tiles - 1) / tiles) * t_step + 7) + 4 +
                        0.065 * s.d / 128 * wgs;
-      if (t < 0.95 * best) { best = t; r.heads = heads; r.tiles = tiles; }
+      if (t < gain * best) { best = t; r.heads = heads; r.tiles = tiles; }
     }
   }
   // An XCD owns the items of its kv-heads: with fewer kv-heads than XCDs the parts may just make more rounds there.

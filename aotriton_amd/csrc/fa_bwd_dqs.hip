@@ -19,12 +19,8 @@ hipError_t run_bwd_dqs(int dtype, int head_dim, const BwdArgs& a, hipStream_t s)
 }
 
 // tiles of stored dS per (batch element, q-head): key tiles of 128 x query tiles of the dK/dV step
-void ds_tile_counts(int dtype, int head_dim, bool bias, bool dropout, int max_sq, int max_sk, int* ntq, int* ntk,
-                    int64_t* tile_bytes) {
-  const int bm = head_dim >= 256 ? DsTile<bf16_t, 256, false>::BM
-                 : head_dim > 64 ? DsTile<bf16_t, 128, false>::BM
-                 : bias && !dropout ? DsTile<bf16_t, 64, true>::BM : DsTile<bf16_t, 64, false>::BM;
-  (void)dtype;
+void ds_tile_counts(int head_dim, int max_sq, int max_sk, int* ntq, int* ntk, int64_t* tile_bytes) {
+  const int bm = head_dim >= 256 ? DsTile<bf16_t, 256>::BM : head_dim > 64 ? DsTile<bf16_t, 128>::BM : DsTile<bf16_t, 64>::BM;
   *ntq = ((max_sq + bm - 1) / bm) | 1;     // odd: the rows of tiles of different key tiles and heads do not start a power of two apart
   *ntk = (max_sk + 127) / 128;
   *tile_bytes = (int64_t)128 * bm * 2;

@@ -33,17 +33,17 @@ struct DqsSmem {     // two stages of the K tile (swizzled), then one dS area pe
 
 // One Q tile of 256 rows (8 waves x 32 queries) of head h against the key tiles that see it.
 // kDb: the stored dS is also what dB is, in another layout: the wave's operands of a step go through its LDS
-// area once more, into rows, and leave as 16-byte pieces (dB has unit column stride and rows of aligned
-// pieces); where no stored tile is, dB is zero.  The kernel stays bound by its streams, two written or
+// area once more, into rows, and leave as 16-byte pieces (dB has unit column stride; its rows may start anywhere);
+// where no stored tile is, dB is zero.  The kernel stays bound by its streams, two written or
 // read once instead of one (B8 H12 S512 D64: 25 us for 50 MB in and 50 MB out, with 5 us for the statistics, where
 // the dQ kernel that recomputes S and dP and writes dB took 48).
-template <typename T, int D, int BN, int kPad, bool kWideTile, bool kDb>
+template <typename T, int D, int BN, int kPad, bool kDb>
 __device__ __forceinline__ void dqs_item(const BwdArgs& a, const int h, const int mt, const int z, char* smem_raw) {
   using Tr = Traits<T>;
   using op_t = typename Tr::op_t;
   using q4_t = typename Tr::q4_t;
   using SM = DqsSmem<D, BN>;
-  using DT = DsTile<T, D, kWideTile>;
+  using DT = DsTile<T, D>;
   constexpr int NW = SM::NW, NT = NW * 64, BM = NW * 32;
   constexpr int DB = (kPad ? kPad : D) / 32;
   constexpr int SPT = DT::BN / BN;          // steps per stored tile
@@ -92,7 +92,7 @@ __device__ __forceinline__ void dqs_item(const BwdArgs& a, const int h, const in
     if (m >= si.seqlen_q || n >= si.seqlen_k) return;
     T* p = db_head + (int64_t)m * a.sdb_m + n;
     if (n + 8 <= si.seqlen_k) {
-      *reinterpret_cast<op_t*>(p) = x;
+      __builtin_memcpy(p, &x, 16);      // (rows may start anywhere)
     } else {
 #pragma unroll
       for (int e = 0; e < 8; ++e)
@@ -247,7 +247,7 @@ __device__ __forceinline__ void dqs_item(const BwdArgs& a, const int h, const in
 
 // One workgroup per Q tile on a 1-D grid: consecutive ids go round the XCDs, an XCD takes its
 // (batch, q-head) pairs two at a time, the heaviest (last) tile of a causal mask first.
-template <typename T, int D, int BN, int kPad, bool kWideTile, bool kDb>
+template <typename T, int D, int BN, int kPad, bool kDb>
 __global__ __attribute__((amdgpu_flat_work_group_size(512, 512))) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void bwd_dqs_kernel(const BwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
@@ -260,7 +260,7 @@ void bwd_dqs_kernel(const BwdArgs a) {
   const int mt = a.num_m_tiles - 1 - gr / a.zh_group;
   int z, h;
   split_zh(zh, a.num_zh / a.hq, a.hq / a.hk, z, h);
-  dqs_item<T, D, BN, kPad, kWideTile, kDb>(a, h, mt, z, smem_raw);
+  dqs_item<T, D, BN, kPad, kDb>(a, h, mt, z, smem_raw);
 }
 
 template <typename T, int D, int kPad>
@@ -272,13 +272,8 @@ hipError_t launch_bwd_dqs(const BwdArgs& a0, hipStream_t stream) {
   dim3 grid((unsigned)(kNumXcd * a.items_per_xcd));
   constexpr int lds = DqsSmem<D, BN>::BYTES;
   const bool db = a.db != nullptr;
-  if constexpr (D == 64) {
-    if (a.bias != nullptr && !(a.drop.p > 0.f))      // kWide: how the dK/dV kernel of such a call stored it
-      return db ? launch_with_lds<bwd_dqs_kernel<T, D, BN, kPad, true, true>>(grid, 512, lds, stream, a)
-                : launch_with_lds<bwd_dqs_kernel<T, D, BN, kPad, true, false>>(grid, 512, lds, stream, a);
-  }
-  return db ? launch_with_lds<bwd_dqs_kernel<T, D, BN, kPad, false, true>>(grid, 512, lds, stream, a)
-            : launch_with_lds<bwd_dqs_kernel<T, D, BN, kPad, false, false>>(grid, 512, lds, stream, a);
+  return db ? launch_with_lds<bwd_dqs_kernel<T, D, BN, kPad, true>>(grid, 512, lds, stream, a)
+            : launch_with_lds<bwd_dqs_kernel<T, D, BN, kPad, false>>(grid, 512, lds, stream, a);
 }
 
 }  // namespace fa

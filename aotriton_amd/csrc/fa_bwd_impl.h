@@ -105,16 +105,17 @@ struct DqSmem {     // per stage: K, V (swizzled); then one bias / dB tile per w
 // workgroups per CU, i.e. two waves per SIMD, which hide each other's prologues and phases (backward of
 // B4 H64 S4096: full 4.04 -> 3.65-3.8 ms, causal 2.25 -> 2.0-2.1; B8 H16 S512 47 -> 41.5 us, with dropout
 // B8 H12 S512 75.6 -> 63).  With a bias they do not (90-150 spilled registers): those keep one wave per SIMD
-// and 128-wide steps (64-wide ones lose 2-8 %), except that dK/dV with bias and dropout takes 64-query steps
-// (8 % faster).
+// and 128-wide steps (64-wide ones lose 2-8 %), except that dK/dV takes 64-query steps with bias and dropout
+// (8 % faster) and where it stores dS; there, without dropout and with a bias of a known form, it fits two workgroups per CU
+// (kTwoDkDv: B8 H12 S512 bf16 with a trained bias, forward + backward, 98-104 -> 94 us).
 template <typename T, int D, bool kWindowed> struct BwdTile;
 template <typename T, bool kWindowed> struct BwdTile<T, 64, kWindowed>  { static constexpr int NW = 4, DKDV_BM = 64, DQ_BN = 64; };
 template <typename T, bool kWindowed> struct BwdTile<T, 128, kWindowed> { static constexpr int NW = 4, DKDV_BM = 64, DQ_BN = 64; };
 template <typename T, bool kWindowed> struct BwdTile<T, 256, kWindowed> { static constexpr int NW = 4, DKDV_BM = 32, DQ_BN = 32; };
 // 128-query steps of the dK/dV kernel
 template <int D, bool kBias, bool kDropout> constexpr bool kWide = D == 64 && kBias && !kDropout;
-template <typename T, int D, bool kWindowed, bool kBias, bool kDropout>
-constexpr int kDkDvBM = kWide<D, kBias, kDropout> ? 128 : BwdTile<T, D, kWindowed>::DKDV_BM;
+template <typename T, int D, bool kWindowed, bool kBias, bool kDropout, bool kStoreDs = false>
+constexpr int kDkDvBM = kWide<D, kBias, kDropout> && !kStoreDs ? 128 : BwdTile<T, D, kWindowed>::DKDV_BM;
 template <typename T, int D, bool kWindowed, bool kBias>
 constexpr int kDqBN = D == 64 && kBias ? 128 : BwdTile<T, D, kWindowed>::DQ_BN;
 // the single-launch kernel runs one wave per SIMD, hence the wide steps at head dim 64
@@ -123,6 +124,11 @@ template <typename T, int D, bool W> constexpr int kFusedBN = D == 64 ? 128 : Bw
 
 // Two workgroups per CU, two waves per SIMD (256 registers each)?
 template <int D, bool kBias> constexpr bool kTwoWaves = D == 64 && !kBias;
+// What the dK/dV kernel knows of its bias: nothing, that its rows are whole aligned 16-byte pieces (plain_bias), or that they have
+// unit column stride and at least eight columns.
+enum BiasForm { kBiasAny, kBiasPlain, kBiasRows };
+template <int D, bool kBias, bool kDropout, bool kStoreDs, int kForm>
+constexpr bool kTwoDkDv = kTwoWaves<D, kBias> || (D == 64 && kStoreDs && !kDropout && kForm != kBiasAny);
 // Stored dS (BwdArgs::ds_ws): one tile per (batch element, q-head, key tile of 128, query tile of the
 // dK/dV step) holds 128 x BM values of the 16-bit type as [32-query block][32-key block][half of the
 // query block][64 pieces of 16 bytes].  A piece is what one lane of the dK/dV item holds as the MFMA
@@ -130,9 +136,9 @@ template <int D, bool kBias> constexpr bool kTwoWaves = D == 64 && !kBias;
 // queries 16 t + 4 hi + {0..3} and 16 t + 8 + 4 hi + {0..3} (hi = lane / 32); it sits at piece position
 // (2 c + hi) ^ 8 (t & 1), where the transposing LDS reads of the kernel that consumes the tiles want
 // it.  A wave of that kernel owns one query block: what it needs of a tile is contiguous.
-template <typename T, int D, bool kWideTile> struct DsTile {
+template <typename T, int D> struct DsTile {
   static_assert(BwdTile<T, D, false>::DKDV_BM == BwdTile<T, D, true>::DKDV_BM, "one tile shape per head dim");
-  static constexpr int BM = kWideTile ? 128 : BwdTile<T, D, false>::DKDV_BM;   // queries per stored tile
+  static constexpr int BM = BwdTile<T, D, false>::DKDV_BM;   // queries per stored tile
   static constexpr int BN = 128;                             // keys per stored tile
   static constexpr int TS = BM / 16;                         // 1 KB pieces per 32-key block
   static constexpr int BYTES = BN * BM * 2;
@@ -141,19 +147,37 @@ template <typename T, int D, bool kWideTile> struct DsTile {
   static constexpr int piece(int kw, int t) { return (t >> 1) * QBLOCK_BYTES + kw * 2048 + (t & 1) * 1024; }
 };
 
+// The keep bits that dropout_keep4 gives, appended to `bits`: two instructions each and no condition (the sign of a saturated
+// difference, shifted in).
+__device__ __forceinline__ uint32_t dropout_append4(const DropoutState& s, int m, int n0, uint32_t bits) {
+  const uint64_t ctr = s.base + (uint64_t)m * s.stride + (uint64_t)(n0 >> 2);
+  uint32_t w[4];
+  philox4x32_10((uint32_t)ctr, (uint32_t)(ctr >> 32), s.k0, s.k1, w);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int i = r == 1 ? 2 : r == 2 ? 1 : r;      // (the word order of a row)
+    bits = __builtin_amdgcn_alignbit(bits, (uint32_t)__builtin_elementwise_sub_sat(s.thr, (int32_t)w[i]), 31);
+  }
+  return bits;
+}
+
 // ---------------------------------------------------------------------------
 // dK / dV work item
 // ---------------------------------------------------------------------------
 // kStoreDs: dS of every visited tile pair is also written to BwdArgs::ds_ws, and the row statistics
 // come prepared (BwdArgs::lse_scaled, delta_prep) so that they can travel straight into LDS.
-// kBiasPlain: every row of the bias is whole aligned 16-byte pieces (plain_bias); the branches for other layouts, which sit
-// in the tile loop, and the registers that they hold go.  One wave per SIMD issues every instruction of its tile one after the
+// kForm: with kBiasPlain and kBiasRows the branches for other layouts, which sit in the tile loop, and the registers that they
+// hold go.  One wave per SIMD issues every instruction of its tile one after the
 // other, so what these kernels with bias or dropout take is counted in instructions: at B2 H16 S8192 D256 fp16, window 1024,
 // bias and dropout, a full tile's went from 1750 to 1090 (that flag; DropoutFold; no struct members in the loop, see
 // own_scalar; 16 spilled vector registers gone) and the kernel from 1.15 to 1.05 ms; B8 H12 S512 D64 bf16 with bias 50 -> 44 us,
 // B4 H16 1000 x 1531 D80 fp16 with dropout 195 -> 190 us.
+// kBiasRows: a tile that lies inside the sequences is fetched as it is, without a condition per lane (window, bias and dropout,
+// odd lengths, forward + backward: B1 H16 S3001 D64 fp16 259 -> 211 us, B2 H8 S1801 D128 168 -> 150, B1 H16 S2711 D256 465 -> 438,
+// 15 of which are the forward's).  Keep bits in one word: 78 of 1031 instructions a tile less at D = 96, cross attention 1000 x 1531
+// D80 315 -> 303 us.
 template <typename T, int D, int NW, int BM, bool kWindowed, bool kBias, bool kDropout, int kPad, bool kStoreDs = false,
-          bool kParts = false, bool kBiasPlain = false>
+          bool kParts = false, int kForm = kBiasAny>
 __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const int nt, const int z, const int part,
                                           char* smem_raw) {
   using Tr = Traits<T>;
@@ -277,7 +301,7 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
   // middle (where the compiler makes the first transposing read wait for the direct-to-LDS pieces
   // anyway), and the pieces leave in the half tile after it, as their operands get complete: the
   // youngest store is more than half a tile old at the next wait.
-  using DT = DsTile<T, D, kWide<D, kBias, kDropout>>;
+  using DT = DsTile<T, D>;
   static_assert(!kStoreDs || (BM == DT::BM && BN == DT::BN), "stored tiles have the item's shape");
   const int ds_pos[2] = {((c << 1) | hi) << 4, (((c << 1) | hi) ^ 8) << 4};
   op_t sb[TS];                         // dS operands of the dK GEMM; with kStoreDs they outlive their tile
@@ -368,6 +392,7 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
   const int b_lds = (tid / 16) * SM::BIAS_STR + (tid % 16) * 16;
   const T* bb_tile = nullptr;     // bias tile being fetched, its valid rows
   int b_rows = 0;
+  bool b_whole = false;           // kBiasRows: no row and no piece of a row of it is past the sequence
   const int b_cols = si.seqlen_k - n0 < BN ? si.seqlen_k - n0 : BN;      // valid keys of this item
   // (g, e) = (q-head inside the GQA group, Q tile inside the range) of the tile to fetch;
   // called for consecutive tiles only; `live` false: nothing is fetched
@@ -380,8 +405,9 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
     if (kBias) {
       bb_tile = reinterpret_cast<const T*>(bb);
       b_rows = rows;
-      b_rs = wave_rsrc(bb, any && kBiasPlain ? (rows - 1) * bias_row + b_cols * 2 : 0);
-      if (live) bb += kBiasPlain ? BM * bias_row : (int64_t)BM * 2 * a.sb_m;
+      b_whole = rows == BM && b_cols == BN;
+      b_rs = wave_rsrc(bb, any && kForm == kBiasPlain ? (rows - 1) * bias_row + b_cols * 2 : 0);
+      if (live) bb += kForm != kBiasAny ? BM * bias_row : (int64_t)BM * 2 * a.sb_m;
     }
     q_rs = wave_rsrc(qb, any ? (rows - 1) * q_row + d_qk * 2 : 0);
     do_rs = wave_rsrc(dob, any ? (rows - 1) * do_row + d_v * 2 : 0);
@@ -409,9 +435,11 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
   auto fetch_piece = [&](int i) {        // Q pieces first, then dO, then bias
     if (i >= 2 * CH) {
       const int k = i - 2 * CH;
-      if (kBiasPlain) {
+      if (kForm == kBiasPlain) {
         bch[k] = __builtin_bit_cast(op_t, __builtin_amdgcn_raw_buffer_load_b128(b_rs, b_voff, k * b_soff, 0));
-      } else if (bias_rows) {
+      } else if (kForm == kBiasRows && b_whole) {
+        __builtin_memcpy(&bch[k], reinterpret_cast<const char*>(bb_tile) + k * b_soff + (uint32_t)b_voff, 16);
+      } else if (kForm == kBiasRows || bias_rows) {
         const int row = tid / 16 + k * (NT / 16), col = (tid % 16) * 8;
         op_t x = {0, 0, 0, 0, 0, 0, 0, 0};
         if (row < b_rows && col < b_cols)
@@ -446,6 +474,8 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
   };
   DropoutFold fold{};
   if (kDropout) fold = dropout_fold(a.drop.p);
+  uint32_t key_bit = 1u << (lane & 3);      // of this lane's key in the four bits of a Philox call
+  asm("" : "+v"(key_bit));                  // (as a value of its own: a test of it is one instruction with the quad's exchange)
   auto store_stats = [&](int stage) {
     char* sp = stage_ptr(stage);
     float* Ls = reinterpret_cast<float*>(sp + 2 * SM::TILE_BYTES);
@@ -485,11 +515,18 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
     // those of dV.  Fences keep the hand-made order.
     // (one read ahead at D = 256 left each read's latency behind a single MFMA: 2-5 % of the kernel; the bias of any layout has
     // no registers for more)
-    constexpr bool kDeep = D < 256 || !kBias || kBiasPlain;
+    constexpr bool kDeep = D < 256 || !kBias || kForm == kBiasPlain;
     constexpr int kAhead = kDeep ? 2 : 1;
     op_t xa[kAhead + 1][MB];
     op_t pb[TS];
-    uint32_t kw[kDropout ? MB : 1][4];
+    // Keep bits.  kWord: all of a lane's in one word, the first call's uppermost; then, in kw[r], those of its quad's row r,
+    // shifted so that the bit of this lane's key is the first of each call's four.  Else the four bits of call i in kw[i] (D = 256,
+    // whose K operands are moved about for the word: 2 % slower with it).
+    constexpr bool kWord = D < 256;
+    constexpr int kCalls = 4 * MB;
+    static_assert(!kDropout || kCalls * 4 <= 32, "a word holds a tile's bits");
+    uint32_t kw[kWord ? 4 : kCalls];
+    if (kDropout && kWord) kw[0] = 0;
     // row statistics are read four rows at a time, one read ahead of their use
     f32x4 l4[2], d4[2];
     auto stat_ptr = [&](const float* base, int q) { return base + 32 * (q / 4) + 8 * (q % 4) + 4 * hi; };
@@ -531,11 +568,12 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
           // lanes of a quad, for one row: quad lane q runs the calls of the rows with
           // m % 4 == q (8 per tile of 64 rows instead of 32) and the bits are exchanged
           // with quad broadcasts when they are used.
-          constexpr int calls = 4 * MB, stride = G1 / calls > 0 ? G1 / calls : 1;
-          if (gidx % stride == 0 && gidx / stride < calls) {
+          constexpr int stride = G1 / kCalls > 0 ? G1 / kCalls : 1;
+          if (gidx % stride == 0 && gidx / stride < kCalls) {
             const int cidx = gidx / stride;
-            kw[cidx / 4][cidx % 4] =
-                dropout_keep4(dst, m0 + 32 * (cidx / 4) + 8 * (cidx % 4) + 4 * hi + (lane & 3), key & ~3);
+            const int m = m0 + 32 * (cidx / 4) + 8 * (cidx % 4) + 4 * hi + (lane & 3);
+            if (kWord) kw[0] = dropout_append4(dst, m, key & ~3, kw[0]);
+            else kw[cidx] = dropout_keep4(dst, m, key & ~3);
           }
         }
         if (gidx % every == every - 1) {
@@ -547,6 +585,19 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
         }
       }
       __builtin_amdgcn_sched_barrier(0);
+    }
+    auto of_row = [&](uint32_t w, int r) -> uint32_t {      // what the quad's lane r has (quad_perm: [r, r, r, r])
+      switch (r) {
+        case 0: return (uint32_t)__builtin_amdgcn_mov_dpp((int)w, 0x00, 0xf, 0xf, true);
+        case 1: return (uint32_t)__builtin_amdgcn_mov_dpp((int)w, 0x55, 0xf, 0xf, true);
+        case 2: return (uint32_t)__builtin_amdgcn_mov_dpp((int)w, 0xaa, 0xf, 0xf, true);
+        default: return (uint32_t)__builtin_amdgcn_mov_dpp((int)w, 0xff, 0xf, 0xf, true);
+      }
+    };
+    if (kDropout && kWord) {
+      const uint32_t w = kw[0];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) kw[r] = of_row(w, r) << (lane & 3);
     }
     // row statistics of the tile's queries and the first dO operands
     l4[0] = *reinterpret_cast<const f32x4*>(stat_ptr(Ls, 0));
@@ -593,27 +644,35 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
       }
       s[mb][i] = fast_exp2(x);
     };
-    // keep bit of element E: held by the quad lane that ran the Philox call of its row
-    auto keep_of = [&](int E) -> bool {
-      const int mb = E / 16, g = (E % 16) / 4, r = E % 4;
-      const int w = (int)kw[mb][g];
-      int w4;
-      switch (r) {       // quad_perm: [r, r, r, r]
-        case 0: w4 = __builtin_amdgcn_mov_dpp(w, 0x00, 0xf, 0xf, true); break;
-        case 1: w4 = __builtin_amdgcn_mov_dpp(w, 0x55, 0xf, 0xf, true); break;
-        case 2: w4 = __builtin_amdgcn_mov_dpp(w, 0xaa, 0xf, 0xf, true); break;
-        default: w4 = __builtin_amdgcn_mov_dpp(w, 0xff, 0xf, 0xf, true); break;
+    // The keep bit of an element spread over a register (one instruction), and x where it is set, else zero.  (As a condition per
+    // element, with the four bits of a call in a register of their own, that was three instructions and waits for the scalar
+    // register.  The asm keeps the compiler from making a comparison and a selection of it again.)
+    constexpr bool kKeepMasks = D == 128;      // registers to hold them from P to dS; else the bit is spread a second time
+    int keep_mask[kDropout && kWord ? 16 * MB : 1];
+    bool keep_bit[kDropout && !kWord ? 16 * MB : 1];
+    auto spread = [&](int E) {
+      if constexpr (!kWord) {
+        keep_bit[E] = (of_row(kw[E / 4], E % 4) & key_bit) != 0;
+        return;
       }
-      return ((uint32_t)w4 >> (lane & 3)) & 1u;
+#define FA_KEEP_BIT(n) \
+  case n: asm volatile("v_bfe_i32 %0, %1, %2, 1" : "=v"(keep_mask[E]) : "v"(kw[E % 4]), "n"((4 * kCalls - 1 - 4 * (n)) & 31)); break;
+      switch (E / 4) {
+        FA_KEEP_BIT(0) FA_KEEP_BIT(1) FA_KEEP_BIT(2) FA_KEEP_BIT(3) FA_KEEP_BIT(4) FA_KEEP_BIT(5) FA_KEEP_BIT(6) FA_KEEP_BIT(7)
+      }
+#undef FA_KEEP_BIT
     };
-    bool keep_bit[kDropout ? 16 * MB : 1];
+    auto kept = [&](int E, float x) -> float {
+      if constexpr (!kWord) return keep_bit[E] ? x : 0.f;
+      else return __builtin_bit_cast(float, __builtin_bit_cast(int, x) & keep_mask[E]);
+    };
     auto p_pair = [&](int E) {   // E odd: operand form of (E-1, E); dropout applies to the operand only
       float p0 = s[E / 16][E % 16 - 1], p1 = s[E / 16][E % 16];
       if (kDropout) {
-        keep_bit[E - 1] = keep_of(E - 1);
-        keep_bit[E] = keep_of(E);
-        p0 = keep_bit[E - 1] ? p0 : 0.f;              // :200-201 (the scale is in p)
-        p1 = keep_bit[E] ? p1 : 0.f;
+        spread(E - 1);
+        spread(E);
+        p0 = kept(E - 1, p0);              // :200-201 (the scale is in p)
+        p1 = kept(E, p1);
       }
       const typename Tr::p2_t p2 = Tr::cvt2(p0, p1);     // p cast to dO's dtype (composed_tensors.py:191-193)
       pb[E / 8][E % 8 - 1] = p2[0];
@@ -626,7 +685,8 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
         return;
       }
       if (E % 4 == 0 && E + 4 < 16 * MB) d4[(E / 4 + 1) & 1] = *reinterpret_cast<const f32x4*>(stat_ptr(Ds, E / 4 + 1));
-      const float dpv = keep_bit[E] ? dp[mb][i] : 0.f;            // :239-240
+      if (kWord && !kKeepMasks) spread(E);
+      const float dpv = kept(E, dp[mb][i]);                       // :239-240
       dp[mb][i] = s[mb][i] * (dpv + d4[(E / 4) & 1][r]);          // ds uses the undropped p (:242)
     };
     auto ds_pair = [&](int E) {  // E odd: ds cast to Q's dtype
@@ -1371,8 +1431,9 @@ __host__ __device__ inline bool dkdv_level_list(const BwdArgs& a) {
 }
 
 template <typename T, int D, int NW, int BM, bool kWindowed, bool kBias, bool kDropout, int kPad, bool kStoreDs = false,
-          bool kParts = false, bool kBiasPlain = false>
-__global__ __attribute__((amdgpu_flat_work_group_size(NW * 64, NW * 64))) __attribute__((amdgpu_waves_per_eu(kTwoWaves<D, kBias> ? 2 : 1, kTwoWaves<D, kBias> ? 2 : 1)))
+          bool kParts = false, int kForm = kBiasAny>
+__global__ __attribute__((amdgpu_flat_work_group_size(NW * 64, NW * 64)))
+__attribute__((amdgpu_waves_per_eu(kTwoDkDv<D, kBias, kDropout, kStoreDs, kForm> ? 2 : 1, kTwoDkDv<D, kBias, kDropout, kStoreDs, kForm> ? 2 : 1)))
 void bwd_dkdv_kernel(const BwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   // Persistent workgroups, one per CU (a relaunch per item costs a dispatch gap of several
@@ -1395,7 +1456,7 @@ void bwd_dkdv_kernel(const BwdArgs a) {
   // (D = 256 is launched with one workgroup per item: the loop would cost registers there)
   const int parts = kParts ? a.part_heads * a.part_tiles : 1;
   for (int r = 0; D >= 256 ? r < 1 : r * workers < a.items_per_xcd; ++r) {
-    const int lp = worker_pos<kTwoWaves<D, kBias>>(r, p, workers, a.num_cu);
+    const int lp = worker_pos<kTwoDkDv<D, kBias, kDropout, kStoreDs, kForm>>(r, p, workers, a.num_cu);
     const int li = lp / parts;
     int zh, nt;
     if (ragged) {
@@ -1412,7 +1473,7 @@ void bwd_dkdv_kernel(const BwdArgs a) {
     }
     int z, hk;
     split_zh(zh, a.num_zh / a.hk, 1, z, hk);
-    dkdv_item<T, D, NW, BM, kWindowed, kBias, kDropout, kPad, kStoreDs, kParts, kBiasPlain>(a, hk, nt, z, kParts ? lp % parts : 0, smem_raw);
+    dkdv_item<T, D, NW, BM, kWindowed, kBias, kDropout, kPad, kStoreDs, kParts, kForm>(a, hk, nt, z, kParts ? lp % parts : 0, smem_raw);
     __syncthreads();     // the next item reuses the LDS stages
   }
 }
@@ -1523,23 +1584,16 @@ template <typename T> inline bool plain_bias(const BwdArgs& a) {
          (reinterpret_cast<uintptr_t>(a.bias) & 15) == 0;
 }
 
-template <typename T, int D, int kPad, bool W, bool B, bool P, bool kParts>
-hipError_t launch_dkdv_variant(const BwdArgs& a0, hipStream_t stream) {
-  using Tile = BwdTile<T, D, W>;
-  constexpr int NW = Tile::NW, BM = kDkDvBM<T, D, W, B, P>, BN = NW * 32;
+template <typename T, int D, int kPad, bool W, bool B, bool P, bool kParts, bool kStoreDs, int kForm>
+hipError_t launch_dkdv_form(const BwdArgs& a0, hipStream_t stream) {
+  constexpr int NW = BwdTile<T, D, W>::NW, BM = kDkDvBM<T, D, W, B, P, kStoreDs>, BN = NW * 32;
   BwdArgs a = a0;
   a.num_n_tiles = (a.seq.max_seqlen_k + BN - 1) / BN;
   set_work(a, tile_work(bwd_nseq(a) * a.hk, 2, a.num_n_tiles * (kParts ? a.part_heads * a.part_tiles : 1)));
   dim3 grid((unsigned)(kNumXcd * bwd_workers(D, B, a.items_per_xcd, a.num_cu, kTwoWaves<D, B> ? 2 : 1)));
   // (the level table's LDS is requested whether or not this launch uses it: the kernel's limit is set once)
   constexpr int smem = DkDvSmem<D, BM>::BYTES + (D < 256 ? kLevelBytes : 0);
-  if constexpr (B && !kParts)
-    if (a.ds_ws != nullptr && plain_bias<T>(a))
-      return launch_with_lds<bwd_dkdv_kernel<T, D, NW, BM, W, B, P, kPad, true, false, true>>(grid, NW * 64, smem, stream, a);
-  // (every build has the variant that stores dS; the host decides where it pays)
-  hipError_t e = a.ds_ws != nullptr
-                     ? launch_with_lds<bwd_dkdv_kernel<T, D, NW, BM, W, B, P, kPad, true, kParts>>(grid, NW * 64, smem, stream, a)
-                     : launch_with_lds<bwd_dkdv_kernel<T, D, NW, BM, W, B, P, kPad, false, kParts>>(grid, NW * 64, smem, stream, a);
+  hipError_t e = launch_with_lds<bwd_dkdv_kernel<T, D, NW, BM, W, B, P, kPad, kStoreDs, kParts, kForm>>(grid, NW * 64, smem, stream, a);
   if constexpr (kParts) {
     const int64_t threads = (int64_t)a.num_zh * a.num_n_tiles * 2 * BN * (D / 4);
     if (e == hipSuccess && threads > 0) {
@@ -1548,6 +1602,18 @@ hipError_t launch_dkdv_variant(const BwdArgs& a0, hipStream_t stream) {
     }
   }
   return e;
+}
+
+template <typename T, int D, int kPad, bool W, bool B, bool P, bool kParts>
+hipError_t launch_dkdv_variant(const BwdArgs& a, hipStream_t stream) {
+  // (every build has the variant that stores dS; the host decides where it pays)
+  if (a.ds_ws == nullptr) return launch_dkdv_form<T, D, kPad, W, B, P, kParts, false, kBiasAny>(a, stream);
+  if constexpr (B && (!kParts || kTwoDkDv<D, B, P, true, kBiasPlain>)) {
+    if (plain_bias<T>(a)) return launch_dkdv_form<T, D, kPad, W, B, P, kParts, true, kBiasPlain>(a, stream);
+    if (a.seq.num_seqlens == 0 && a.seq.max_seqlen_k >= 8 && a.sb_n == 1)
+      return launch_dkdv_form<T, D, kPad, W, B, P, kParts, true, kBiasRows>(a, stream);
+  }
+  return launch_dkdv_form<T, D, kPad, W, B, P, kParts, true, kBiasAny>(a, stream);
 }
 
 template <typename T, int D, int kPad, bool kParts>

@@ -106,3 +106,42 @@ def test_recomputed_dq_at_padded_head_dims(D, dt, Sq, Sk, causal, p, layout):
         _run_case(2, 4, 2, Sq, Sk, D, dt, causal, dropout_p=p, bias=True, bias_layout=layout, seed=23)
     finally:
         lib.fa_set_bwd_workspace_limit(-1)
+
+
+@pytest.mark.parametrize('D', [40, 64, 128, 256])
+@pytest.mark.parametrize('Sq,Sk,causal,p', [(70, 136, False, 0.0), (300, 131, True, 0.0), (257, 520, (60, 90), 0.0), (129, 261, False, 0.1),
+                                            (65, 9, False, 0.0)])
+def test_stored_ds_under_rows_at_any_alignment(D, Sq, Sk, causal, p):
+    """The backward that keeps dS and writes dB from it, given the same bias and the same dB in rows that start at 16-byte
+    boundaries and in odd ones: the same bits, nothing written beside dB's rows."""
+    from aotriton_amd import flash
+    H, dt = 6, BF
+    B = 2 ** 22 // (H * Sq * Sk) + 1      # large enough for the stored dS
+    q, k, v, _, do = make_inputs(B, H, H, Sq, Sk, D, dt, 'cuda', seed=15)
+    seed, off = (torch.tensor([x], device='cuda', dtype=torch.uint64) for x in (7, 8))
+    null, sm, out = torch.empty([0], device='cuda', dtype=torch.uint64), 1 / math.sqrt(D), []
+    values = torch.randn(B, H, Sq, Sk, device='cuda', dtype=dt)
+    o, L = torch.empty_like(q), torch.empty(B * H, Sq, device='cuda')
+    assert flash.attn_fwd(q, k, v, values, sm, L, o, p, seed, off, 0, null, null, None, causal, null) == flash.hipError_t.hipSuccess
+    odd = Sk + (1 - Sk % 2) + 2
+    for width, at in (((Sk + 7) // 8 * 8, 0), (odd, 1)):
+        b = torch.full((B * H * Sq * width + 8,), float('nan'), device='cuda', dtype=dt)
+        view = lambda t: t[at:at + B * H * Sq * width].view(B, H, Sq, width)[..., :Sk]
+        view(b).copy_(values)
+        db = torch.full_like(b, 7.0)
+        dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+        err = flash.attn_bwd(q, k, v, view(b), sm, o, do, dq, dk, dv, view(db), flash.lazy_dq_acc(q), L,
+                             flash.lazy_delta(L), p, seed, off, 0, causal)
+        assert err == flash.hipError_t.hipSuccess
+        out.append((dq, dk, dv, view(db).clone()))
+        view(db).fill_(7.0)
+        assert (db == 7.0).all()
+    for x, y in zip(*out):
+        assert torch.isfinite(x).all() and torch.equal(x, y)
+
+
+@pytest.mark.parametrize('B,H,Sq,Sk,causal,layout', [(1, 8, 1024, 1024, False, 'padded'), (1, 4, 1000, 1023, True, 'odd'),
+                                                     (2, 8, 1024, 1000, (300, 100), 'odd')])
+def test_parts_with_a_bias(B, H, Sq, Sk, causal, layout):
+    """dK/dV items cut into parts, several to a CU, at D = 64 with a bias: against the oracle"""
+    _run_case(B, H, H, Sq, Sk, 64, BF, causal, bias=True, bias_layout=layout, seed=33)
