@@ -307,9 +307,12 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
   // which is idle between the Q rows at the start and the O rows at the end of an item.  (One
   // 8-byte load per lane and 4 keys touches 32 cache lines for 16 bytes each; the vector memory
   // pipe's line rate then costs more than the bias bytes.)  A row of the area holds D keys, so a
-  // tile passes in BN / BCK chunks of BCK keys.  The pieces are requested behind the QK MFMAs, not
-  // before them: 16 more live registers across that phase cost the causal kernel more in spills
-  // than the exposed latency costs with two waves per SIMD.
+  // tile passes in BN / BCK chunks of BCK keys.  kBiasAhead, the 128-row tiles: a tile's pieces are requested a tile ahead, next
+  // to its K and V, and lie in the area while the tile is worked on (us, D64, before -> after: B3 H16 S357 16.4 -> 15.5, B16 H12
+  // S700 80 -> 75, B8 H16 S256 13.3 -> 12.5; B9 H16 S1007 with 292 MB of bias 131 -> 129).
+  // The tiles of 256 rows have no registers for that (75 more spilled at D = 64, 45 at D = 128): the pieces are requested behind
+  // the QK MFMAs.
+  constexpr bool kBiasAhead = kBias && !kKeyBias && NW == 4;
   constexpr int BCK = BN < D ? BN : D;    // keys per chunk
   constexpr int BLPR = BCK / 8;           // 16-byte pieces per chunk row
   constexpr int BRPI = 64 / BLPR;         // rows per wave-wide access
@@ -318,28 +321,61 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
   const bool bias_co = kBias && a.sb_n == 1 &&
                        (kAnyRow ? si.seqlen_k >= 8
                                 : ((a.sb_m | a.sb_h | a.sb_z) & 7) == 0 && (reinterpret_cast<uintptr_t>(a.bias) & 15) == 0);
+  static_assert(!kBiasAhead || BCK == BN, "the area holds a tile");
+  op_t bias_next[kBiasAhead ? BNI : 1];
+  auto bias_put = [&](int i, op_t x) { *reinterpret_cast<op_t*>(rowbuf + (brow + BRPI * i) * SM::ROW_STR + bch * 16) = x; };
+  auto bias_piece = [&](auto end_tag, int j, int i) {
+    const T* bh = reinterpret_cast<const T*>(a.bias) + (int64_t)si.batch_index * a.sb_z + (int64_t)h * a.sb_h;
+    int m = q0 + wave * 32 + brow + BRPI * i;
+    m = m < si.seqlen_q ? m : si.seqlen_q - 1;
+    return load_row_piece<T, decltype(end_tag)::value>(bh + (int64_t)m * a.sb_m, j * BN + bch * 8, si.seqlen_k);
+  };
+  auto request_bias = [&](int j) {
+    if constexpr (kBiasAhead)
+      if (bias_co && (j + 1) * BN <= si.seqlen_k)
+#pragma unroll
+        for (int i = 0; i < BNI; ++i) bias_next[i] = bias_piece(std::false_type{}, j, i);
+  };
+  auto store_bias = [&](int j) {      // tile j's pieces into the area
+    if constexpr (kBiasAhead) {
+      if (bias_co && (j + 1) * BN <= si.seqlen_k) {
+#pragma unroll
+        for (int i = 0; i < BNI; ++i) bias_put(i, bias_next[i]);
+      } else if (kAnyRow && bias_co) {      // (one after the other: once per item)
+#pragma unroll
+        for (int i = 0; i < BNI; ++i) {
+          bias_put(i, bias_piece(std::true_type{}, j, i));
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+  };
   // adds chunk `ck` of tile j's bias to s (end_tag: the tile may reach past the last key)
   auto bias_chunk = [&](auto end_tag, int j, int ck) {
-    const T* bh = reinterpret_cast<const T*>(a.bias) + (int64_t)si.batch_index * a.sb_z + (int64_t)h * a.sb_h;
     constexpr bool kEnd = decltype(end_tag)::value;
-    auto piece = [&](int i) {
-      int m = q0 + wave * 32 + brow + BRPI * i;
-      m = m < si.seqlen_q ? m : si.seqlen_q - 1;
-      return load_row_piece<T, kEnd>(bh + (int64_t)m * a.sb_m, j * BN + ck * BCK + bch * 8, si.seqlen_k);
-    };
-    auto put = [&](int i, op_t x) { *reinterpret_cast<op_t*>(rowbuf + (brow + BRPI * i) * SM::ROW_STR + bch * 16) = x; };
-    if constexpr (kEnd) {      // (one after the other: once per item, and all at once spills)
+    if constexpr (!kBiasAhead) {
+      // (pointer and closures of its own: with those above 73 registers spill at D = 128 instead of 63, and a window with bias and
+      // dropout at odd lengths takes 5 % more time)
+      const T* bh = reinterpret_cast<const T*>(a.bias) + (int64_t)si.batch_index * a.sb_z + (int64_t)h * a.sb_h;
+      auto piece = [&](int i) {
+        int m = q0 + wave * 32 + brow + BRPI * i;
+        m = m < si.seqlen_q ? m : si.seqlen_q - 1;
+        return load_row_piece<T, kEnd>(bh + (int64_t)m * a.sb_m, j * BN + ck * BCK + bch * 8, si.seqlen_k);
+      };
+      auto put = [&](int i, op_t x) { *reinterpret_cast<op_t*>(rowbuf + (brow + BRPI * i) * SM::ROW_STR + bch * 16) = x; };
+      if constexpr (kEnd) {      // (one after the other: once per item, and all at once spills)
 #pragma unroll
-      for (int i = 0; i < BNI; ++i) {
-        put(i, piece(i));
-        __builtin_amdgcn_sched_barrier(0);
+        for (int i = 0; i < BNI; ++i) {
+          put(i, piece(i));
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      } else {
+        op_t bco[BNI];
+#pragma unroll
+        for (int i = 0; i < BNI; ++i) bco[i] = piece(i);
+#pragma unroll
+        for (int i = 0; i < BNI; ++i) put(i, bco[i]);
       }
-    } else {
-      op_t bco[BNI];
-#pragma unroll
-      for (int i = 0; i < BNI; ++i) bco[i] = piece(i);
-#pragma unroll
-      for (int i = 0; i < BNI; ++i) put(i, bco[i]);
     }
 #pragma unroll
     for (int mbl = 0; mbl < BCK / 32; ++mbl)
@@ -578,11 +614,16 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
   };
 
   // ---- main loop: LDS double buffer, one barrier per tile ---------------------
+  request_bias(br.lo);
   store_tile(0);
   __syncthreads();
   for (int j = br.lo; j <= br.hi; ++j) {
     const int stage = (j - br.lo) & 1;
-    if (j < br.hi) load_next_tile();
+    store_bias(j);
+    if (j < br.hi) {
+      load_next_tile();
+      request_bias(j + 1);
+    }
     if (j <= wave_hi) {
       qk(stage);
       // per-element masks only where some row of this wave has a hidden key in the tile

@@ -19,6 +19,11 @@ CASES = [
     (4, 8, 260, 383, 128, HF, True),
     (1, 2, 200, 65, 80, BF, False),
     (2, 4, 300, 191, 128, BF, (-20, 90)),
+    (2, 4, 300, 261, 256, BF, (100, 0)),
+    (1, 3, 260, 389, 256, HF, True),
+    (1, 2, 140, 97, 200, BF, False),
+    (1, 2, 129, 32, 256, HF, False),
+    (1, 2, 40, 7, 256, BF, False),
 ]
 
 
