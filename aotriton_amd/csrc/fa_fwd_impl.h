@@ -318,6 +318,10 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
   constexpr int BRPI = 64 / BLPR;         // rows per wave-wide access
   constexpr int BNI = 32 / BRPI;          // accesses per chunk
   const int brow = lane / BLPR, bch = lane % BLPR;
+  const int b_row = kBias ? (int)a.sb_m * 2 : 0;
+  const int b_first = q0 + wave_u * 32 < si.seqlen_q ? q0 + wave_u * 32 : si.seqlen_q - 1;
+  const char* bias_tile = reinterpret_cast<const char*>(a.bias) +
+                          2 * ((int64_t)si.batch_index * a.sb_z + (int64_t)h * a.sb_h + (int64_t)b_first * a.sb_m);
   const bool bias_co = kBias && a.sb_n == 1 &&
                        (kAnyRow ? si.seqlen_k >= 8
                                 : ((a.sb_m | a.sb_h | a.sb_z) & 7) == 0 && (reinterpret_cast<uintptr_t>(a.bias) & 15) == 0);
@@ -354,13 +358,20 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
   auto bias_chunk = [&](auto end_tag, int j, int ck) {
     constexpr bool kEnd = decltype(end_tag)::value;
     if constexpr (!kBiasAhead) {
-      // (pointer and closures of its own: with those above 73 registers spill at D = 128 instead of 63, and a window with bias and
-      // dropout at odd lengths takes 5 % more time)
-      const T* bh = reinterpret_cast<const T*>(a.bias) + (int64_t)si.batch_index * a.sb_z + (int64_t)h * a.sb_h;
+      const char* base = bias_tile + (int64_t)(j * BN + ck * BCK) * 2;
       auto piece = [&](int i) {
-        int m = q0 + wave * 32 + brow + BRPI * i;
-        m = m < si.seqlen_q ? m : si.seqlen_q - 1;
-        return load_row_piece<T, kEnd>(bh + (int64_t)m * a.sb_m, j * BN + ck * BCK + bch * 8, si.seqlen_k);
+        // The row inside the wave, as a 32-bit offset from a scalar base (rows are at most 2^21 elements apart); rows past the
+        // sequence repeat the last one.  (As a 64-bit pointer per row the offsets were spilled, and their reloads waited for the
+        // tile's K and V.  Window, bias and dropout, us, B2 H16 S4096 D128 282 -> 259, B1 H16 S3000 187 -> 157, B2 H16 S2048 D64
+        // 67.7 -> 63.)
+        const int m = brow + BRPI * i < wrows - 1 ? brow + BRPI * i : (wrows > 0 ? wrows - 1 : 0);
+        if constexpr (kEnd) {
+          return load_row_piece<T, true>(reinterpret_cast<const T*>(bias_tile + (uint32_t)(m * b_row)), j * BN + ck * BCK + bch * 8, si.seqlen_k);
+        } else {
+          op_t x;
+          __builtin_memcpy(&x, base + (uint32_t)(m * b_row + bch * 16), 16);
+          return x;
+        }
       };
       auto put = [&](int i, op_t x) { *reinterpret_cast<op_t*>(rowbuf + (brow + BRPI * i) * SM::ROW_STR + bch * 16) = x; };
       if constexpr (kEnd) {      // (one after the other: once per item, and all at once spills)

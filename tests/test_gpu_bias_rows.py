@@ -73,3 +73,27 @@ def test_bias_rows_at_any_alignment(case, p):
         want = torch.matmul(torch.softmax(s, -1).nan_to_num(0.0), v.double())
         for o, _ in out:      # P rounded, the result rounded
             assert ((o.double() - want).norm() / want.norm()).item() < 3 * torch.finfo(dt).eps / 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('p', [0.0, 0.2])
+@pytest.mark.parametrize('step', [(1 << 21) - 1, 1 << 21])
+def test_rows_far_apart(step, p):
+    """Rows of the bias as far apart as they may be (their offsets are kept in 32 bits), next to the same rows close together."""
+    from aotriton_amd import flash
+    B, H, Sq, Sk, D, dt = 8, 16, 262, 136, 128, HF
+    assert fwd(B, H, H, Sq, Sk, D, False, p, True).block_m == 256
+    g = torch.Generator(device='cuda').manual_seed(5)
+    rn = lambda *s: torch.randn(*s, device='cuda', generator=g).to(dt)
+    q, k, v, near = rn(B, H, Sq, D), rn(B, H, Sk, D), rn(B, H, Sk, D), rn(Sq, Sk)
+    far = torch.empty((Sq - 1) * step + Sk, device='cuda', dtype=dt).as_strided((Sq, Sk), (step, 1)).copy_(near)
+    seed, off = (torch.tensor([x], device='cuda', dtype=torch.uint64) for x in (3, 4))
+    null, out = torch.empty([0], device='cuda', dtype=torch.uint64), []
+    for b in (near, far):
+        o, L = torch.empty_like(q), torch.empty(B * H, Sq, device='cuda')
+        b = b.expand(B, H, Sq, Sk)
+        assert flash.attn_fwd(q, k, v, b, D ** -0.5, L, o, p, seed, off, 0, null, null, None, False, null) == flash.hipError_t.hipSuccess
+        out.append((o, L))
+    assert (out[0][1] - out[1][1]).abs().max().item() < 1e-5 * (1 + out[0][1].abs().max().item())
+    d = (out[0][0].double() - out[1][0].double()).norm() / out[0][0].double().norm()
+    assert d.item() < 2 * torch.finfo(dt).eps
