@@ -147,8 +147,8 @@ template <typename T, int D> struct DsTile {
   static constexpr int piece(int kw, int t) { return (t >> 1) * QBLOCK_BYTES + kw * 2048 + (t & 1) * 1024; }
 };
 
-// The keep bits that dropout_keep4 gives, appended to `bits`: two instructions each and no condition (the sign of a saturated
-// difference, shifted in).
+// The keep bits that dropout_keep4 gives, appended to `bits` with the first uppermost: two instructions each and no condition (the
+// sign of a saturated difference, shifted in; as a condition each is three and a wait of two states for the condition).
 __device__ __forceinline__ uint32_t dropout_append4(const DropoutState& s, int m, int n0, uint32_t bits) {
   const uint64_t ctr = s.base + (uint64_t)m * s.stride + (uint64_t)(n0 >> 2);
   uint32_t w[4];
@@ -474,7 +474,7 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
   };
   DropoutFold fold{};
   if (kDropout) fold = dropout_fold(a.drop.p);
-  uint32_t key_bit = 1u << (lane & 3);      // of this lane's key in the four bits of a Philox call
+  uint32_t key_bit = 8u >> (lane & 3);      // of this lane's key in the four bits of a Philox call
   asm("" : "+v"(key_bit));                  // (as a value of its own: a test of it is one instruction with the quad's exchange)
   auto store_stats = [&](int stage) {
     char* sp = stage_ptr(stage);
@@ -573,7 +573,7 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
             const int cidx = gidx / stride;
             const int m = m0 + 32 * (cidx / 4) + 8 * (cidx % 4) + 4 * hi + (lane & 3);
             if (kWord) kw[0] = dropout_append4(dst, m, key & ~3, kw[0]);
-            else kw[cidx] = dropout_keep4(dst, m, key & ~3);
+            else kw[cidx] = dropout_append4(dst, m, key & ~3, 0);
           }
         }
         if (gidx % every == every - 1) {
@@ -625,6 +625,14 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
 
     // element E = 16*mb + i of the tile: p (kept in s, undropped, times the dropout scale) and its operand form
     const unsigned q_d = q_none ? 0x40000000u : (unsigned)(m0 + 4 * hi - q_lo);
+    // An element's bias*log2e - L*log2e.  At D = 256, with one element behind each MFMA, it is formed an element ahead: the mixed
+    // multiply-add's result is not ready for the next instruction, and nothing else stands there to be issued.  (With the keep bits
+    // of dropout_append4, B2 H16 S8192 fp16, window, bias and dropout: 767 instead of 817 instructions a plain tile, 9 of 51 s_nop.)
+    float bias_next = 0.f;
+    auto bias_part = [&](int E) {
+      const float bv = (float)bias4[kBiasRing ? (E / 4) & 1 : E / 4][E % 4];
+      return __builtin_fmaf(bv, kLog2e, -l4[(E / 4) & 1][E % 4]);
+    };
     auto p_el = [&](int E) {
       const int mb = E / 16, i = E % 16, g = i / 4, r = i % 4;
       if (E % 4 == 0 && E + 4 < 16 * MB) l4[(E / 4 + 1) & 1] = *reinterpret_cast<const f32x4*>(stat_ptr(Ls, E / 4 + 1));
@@ -632,8 +640,9 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
       float x;
       if (kBias) {
         if (kBiasRing && E % 4 == 0 && E + 4 < 16 * MB) bias4[(E / 4 + 1) & 1] = bias_read(E / 4 + 1);
-        const float bv = (float)bias4[kBiasRing ? (E / 4) & 1 : E / 4][r];
-        x = __builtin_fmaf(s[mb][i], qk_scale, __builtin_fmaf(bv, kLog2e, -l4[(E / 4) & 1][r]));
+        const float here = kBiasRing && E % 4 != 0 ? bias_next : bias_part(E);
+        if (kBiasRing && E % 4 != 3) bias_next = bias_part(E + 1);
+        x = __builtin_fmaf(s[mb][i], qk_scale, here);
       } else {
         x = __builtin_fmaf(s[mb][i], qk_scale, -l4[(E / 4) & 1][r]);
       }
