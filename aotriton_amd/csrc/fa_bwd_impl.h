@@ -627,7 +627,8 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
     const unsigned q_d = q_none ? 0x40000000u : (unsigned)(m0 + 4 * hi - q_lo);
     // An element's bias*log2e - L*log2e.  At D = 256, with one element behind each MFMA, it is formed an element ahead: the mixed
     // multiply-add's result is not ready for the next instruction, and nothing else stands there to be issued.  (With the keep bits
-    // of dropout_append4, B2 H16 S8192 fp16, window, bias and dropout: 767 instead of 817 instructions a plain tile, 9 of 51 s_nop.)
+    // of dropout_append4, B2 H16 S8192 fp16, window, bias and dropout: 767 instead of 817 instructions a plain tile, 9 of them s_nop instead
+    // of 51, and 1 % less time: an s_nop costs little.)
     float bias_next = 0.f;
     auto bias_part = [&](int E) {
       const float bv = (float)bias4[kBiasRing ? (E / 4) & 1 : E / 4][E % 4];
