@@ -816,7 +816,8 @@ struct DkdvParts { int heads, tiles; int64_t bytes; };
 // with more than num_cu / 2 items stay whole although there are twice as many places.  What it chooses there holds (us of
 // the backward, whole / cut, B1: Hq 8 Hk 2 2048 x 256 143 / 35, Hq 16 Hk 4 1024 causal 90 / 46, H8 4096 x 512 82 / 41, H4 4096 x
 // 1024 causal 88 / 50, Hq 16 Hk 8 512 x 1024 causal 36 / 34; H8 1024 x 1000 39 / 40), finer cuts have not been measured.
-DkdvParts dkdv_parts(const fa_bwd_params* p, const Shape& s, int num_cu) {
+// `stored`: the items keep dS in HBM.
+DkdvParts dkdv_parts(const fa_bwd_params* p, const Shape& s, bool stored, int num_cu) {
   DkdvParts r{1, 1, 0};
   if (s.elementwise || !is_16bit(p->Q.dtype) || s.d > 256 || s.max_sq <= 0 || s.max_sk <= 0 || s.batch <= 0) return r;
   const int64_t nz = s.num_seqlens != 0 ? std::abs(s.num_seqlens) : s.batch;
@@ -836,19 +837,42 @@ DkdvParts dkdv_parts(const fa_bwd_params* p, const Shape& s, int num_cu) {
     sum += n;
   }
   const double t_step = (s.d == 64 ? 2.3 : s.d == 128 ? 1.9 : 2.1) * (s.dropout ? 1.7 : 1.0) * (s.bias ? 1.3 : 1.0);
-  double best = group * most * t_step + 7;
-  // (at D = 64 with a bias and no dropout parts share CUs, kTwoDkDv, and level estimates are worth taking: us of the backward
-  // with 1 / 2 / 3 / 4 parts, S1024: B1 H8 52.9 / 48.5 / 46.1 / 44.1, B2 H8 55.8 / 53.2 / 56.3 / 55.1, B1 H16 55 / 52.3 / 55 / 54)
-  const double gain = s.d == 64 && s.bias && !s.dropout ? 1.02 : 0.95;
-  for (int heads = 1; heads <= group; ++heads) {
-    if (group % heads != 0) continue;
-    for (int tiles = 1; tiles <= 16 && tiles <= most; ++tiles) {
-      if (heads * tiles == 1 || (tiles > 1 && heads < group)) continue;
-      const int64_t wgs = items * heads * tiles, rounds = (wgs + num_cu - 1) / num_cu;
-      const double t = rounds * ((double)(group / heads) * ((most + tiles - 1) / tiles) * t_step + 7) + 4 +
-                       0.065 * s.d / 128 * wgs;
-      if (t < gain * best) { best = t; r.heads = heads; r.tiles = tiles; }
+  // Head dim 64 with a bias and no dropout, of the cuts within some of the lowest estimate:
+  // - items that store dS (kTwoDkDv): 64-query steps, two parts share a CU, and what the estimate calls level is a gain.  The lowest
+  //   may be 2 % above whole items, and the finest cut within 2 % of it is taken: 16 shapes (B1-8 H1-16, 256-4096 x 128-2048), each
+  //   in eight cuts, come out 1.9 % above their best in the geometric mean (the general rule: 3.6 %).  us of the backward, whole /
+  //   this / the general rule: B2 H8 S1024 54.6 / 51.6 / 54.6, B1 H8 S512 34.2 / 32.8 / 34.2, B3 H2 2247 x 151 113 / 36 / 39.
+  // - items that do not, as with dB in small calls: a part has a CU to itself and more of them make more rounds on the XCDs of
+  //   few heads.  The coarsest cut within 8 % is taken where the lowest is below whole items: 30 shapes (B1-4 H1-24, 250-2250 x
+  //   128-2000) come out 1.9 % above their best (the general rule: 3.3 %, the rule above: 3.6 %).  us, whole / this / the general rule /
+  //   the rule above: B1 H2 S1400 122 / 114 / 124 / 124, S1024 82 / 66 / 66 / 76, B1 H8 S512 44.8 / 43.2 / 44.8 / 41.7.
+  const bool bias64 = s.d == 64 && s.bias && !s.dropout && s.num_seqlens == 0 && p->B.strides[3] == 1;
+  const bool shared = bias64 && stored && s.max_sk >= 8;
+  const double whole = group * most * t_step + 7;
+  double best = whole;
+  auto for_cuts = [&](auto&& take) {      // from the coarsest to the finest
+    for (int heads = 1; heads <= group; ++heads) {
+      if (group % heads != 0) continue;
+      for (int tiles = 1; tiles <= 16 && tiles <= most; ++tiles) {
+        if (heads * tiles == 1 || (tiles > 1 && heads < group)) continue;
+        const int64_t wgs = items * heads * tiles, rounds = (wgs + num_cu - 1) / num_cu;
+        const double t = rounds * ((double)(group / heads) * ((most + tiles - 1) / tiles) * t_step + 7) + 4 +
+                         0.065 * s.d / 128 * wgs;
+        take(heads, tiles, t);
+      }
     }
+  };
+  if (bias64) {
+    const double level = (shared ? 1.02 : 1.0) * whole;
+    best = level;
+    for_cuts([&](int, int, double t) { best = std::min(best, t); });
+    const double most_t = (shared ? 1.02 : 1.08) * best;
+    if (best < level)
+      for_cuts([&](int heads, int tiles, double t) {
+        if (t <= most_t && (shared || r.heads * r.tiles == 1)) { r.heads = heads; r.tiles = tiles; }
+      });
+  } else {
+    for_cuts([&](int heads, int tiles, double t) { if (t < 0.95 * best) { best = t; r.heads = heads; r.tiles = tiles; } });
   }
   // An XCD owns the items of its kv-heads: with fewer kv-heads than XCDs the parts may just make more rounds there.
   // Under a narrow window, whose items are alike, nothing is gained then (us of the whole backward, uncut / cut, B1 H2
@@ -1113,12 +1137,13 @@ int fa_query_bwd_config(const fa_bwd_params* params, const fa_options* options, 
   const int64_t set = g_ws_limit.load(std::memory_order_relaxed);
   if (be == 0) {
     need = ds_workspace_need(params, s, &ntq, &ntk, &ds_bytes, &stat_bytes);
-    parts = dkdv_parts(params, s, kCus);
+    const int64_t room = have_dev ? ws_limit_bytes(dev) : set >= 0 ? set : INT64_MAX;
+    parts = dkdv_parts(params, s, need > 0 && need <= room, kCus);
     if (route.recompute) {
       need = 0;
       parts = DkdvParts{1, 1, 0};
     }
-    fit_workspace(have_dev ? ws_limit_bytes(dev) : set >= 0 ? set : INT64_MAX, &need, &parts);
+    fit_workspace(room, &need, &parts);
   }
   const bool wide_dkdv = route.wide_dkdv && need == 0 && parts.bytes == 0;
   const fa::TileShape t = rows32 ? fa::f32_rows_tile_shape(s.d)
@@ -1378,8 +1403,9 @@ static int attn_bwd_impl(const fa_bwd_params* p_in, int32_t params_version, void
       int ntq = 0, ntk = 0;
       int64_t ds_bytes = 0, stat_bytes = 0;
       int64_t ds_need = ds_workspace_need(&p2, s2, &ntq, &ntk, &ds_bytes, &stat_bytes);
-      DkdvParts parts = dkdv_parts(&p2, s2, dev->num_cu);
-      inner = fit_workspace(ws_limit_bytes(device_index(dev)) - (int64_t)copies, &ds_need, &parts);
+      const int64_t room = ws_limit_bytes(device_index(dev)) - (int64_t)copies;
+      DkdvParts parts = dkdv_parts(&p2, s2, ds_need > 0 && ds_need <= room, dev->num_cu);
+      inner = fit_workspace(room, &ds_need, &parts);
     }
     const size_t need = copies + (size_t)inner;
     void* base = nullptr;
@@ -1509,17 +1535,18 @@ static int attn_bwd_impl(const fa_bwd_params* p_in, int32_t params_version, void
       if (acquired && lazy->dispose != nullptr) lazy->dispose(lazy);
       return FA_ERROR_NOT_SUPPORTED;
     }
+    // a nested call: the caller holds the buffer and has set a part of it aside
+    const bool nested = t_ws_nested.active;
+    const int64_t room = nested ? (int64_t)t_ws_nested.bytes : limit;
     // (single kernels, for timing, run uncut)
     DkdvParts parts{1, 1, 0};
-    if (kernel_slot < 0 && !own_delta) parts = dkdv_parts(p, s, dev->num_cu);
+    if (kernel_slot < 0 && !own_delta) parts = dkdv_parts(p, s, need > 0 && need <= room, dev->num_cu);
     const BwdRoute route = bwd_route(p, s, dev->num_cu);
     if (route.recompute && kernel_slot < 0) {
       need = 0;
       parts = DkdvParts{1, 1, 0};
     }
-    // a nested call: the caller holds the buffer and has set a part of it aside
-    const bool nested = t_ws_nested.active;
-    int64_t bytes = fit_workspace(nested ? (int64_t)t_ws_nested.bytes : limit, &need, &parts);
+    int64_t bytes = fit_workspace(room, &need, &parts);
     void* ws = nested ? t_ws_nested.ptr : nullptr;
     bool held = false;
     if (!nested && bytes > 0 && !stream_is_capturing(stream)) {

@@ -23,7 +23,7 @@ def fwd(B, Hq, Hk, Sq, Sk, D, causal=False, p=0.0, bias=False, num_cu=256):
     return c
 
 
-def bwd(slot, B, Hq, Hk, Sq, Sk, D, causal=False, p=0.0, bias=False):
+def bwd(slot, B, Hq, Hk, Sq, Sk, D, causal=False, p=0.0, bias=False, db=False):
     from aotriton_amd.pyaotriton.v3.flash import attn_bwd_params, query_bwd_config
     from aotriton_amd.pyaotriton import lazy_tensor
     x = attn_bwd_params()
@@ -33,6 +33,8 @@ def bwd(slot, B, Hq, Hk, Sq, Sk, D, causal=False, p=0.0, bias=False):
     x.L = view(B * Hq, Sq, name='kFloat32')
     x.D = lazy_tensor.eager_delta(x.L)
     _common(x, B, Hq, Sq, Sk, causal, p, bias)
+    if db:
+        x.DB = x.B
     err, c = query_bwd_config(x, slot)
     assert int(err) == 0
     return c
@@ -109,6 +111,25 @@ def test_backward_parts_are_counted():
     try:
         uncut = bwd(1, 1, 8, 2, 1500, 200, 128)
         assert uncut.flags & 64 == 0 and uncut.grid[0] == 8 * 4
+    finally:
+        lib.fa_set_bwd_workspace_limit(-1)
+
+
+@pytest.mark.parametrize('call, db, parts', [
+    ((2, 8, 1024, 1024), False, 2), ((1, 8, 1024, 1024), False, 4), ((1, 8, 512, 512), False, 4), ((4, 16, 256, 256), False, 1),
+    ((3, 2, 2247, 151), False, 10), ((1, 12, 2304, 128), False, 10),      # the finest cut within 2 % of the lowest estimate: 9 parts, not of another cut
+    # dB of a small call: dS is not stored
+    ((1, 2, 1024, 1024), True, 4), ((1, 8, 512, 512), True, 2), ((3, 2, 2247, 151), True, 9), ((1, 2, 1400, 1400), True, 4),
+    ((1, 3, 900, 900), True, 4), ((1, 8, 256, 256), True, 1),
+])
+def test_parts_share_cus_only_where_ds_is_stored(call, db, parts):
+    """head dim 64 with a bias: level estimates are a gain for the kernels with two workgroups per CU, and cost the others up to 16 %"""
+    from aotriton_amd._lib import lib
+    B, H, Sq, Sk = call
+    cut = bwd(1, B, H, H, Sq, Sk, 64, bias=True, db=db).grid[0]
+    lib.fa_set_bwd_workspace_limit(0)
+    try:
+        assert cut == parts * bwd(1, B, H, H, Sq, Sk, 64, bias=True, db=db).grid[0]
     finally:
         lib.fa_set_bwd_workspace_limit(-1)
 
