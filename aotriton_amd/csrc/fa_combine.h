@@ -7,10 +7,10 @@ namespace fa {
 // Sums the parts of a row: out = sum_i 2^((m_i - m) sc) O_i / sum_i 2^((m_i - m) sc) l_i.
 // Parts lie as (pair, row block, part, row of the block): a pair is `part_group` q-heads of one
 // sequence, its rows are counted query * part_group + head and come in blocks of part_block.
-// A thread takes four columns.  With many parts the calls are small (a few hundred rows at most) and what bounds them is the
+// A thread takes four columns.  With many parts of few rows (packed rows: 896 at most) what bounds the sum is the
 // latency of the loads, which miss L2 (other XCDs wrote them): a workgroup per row, whose threads hold all its parts between
-// them and request sums and statistics together, so that one latency is left of several.  Few parts are summed over many rows
-// and bound by HBM: a thread has all parts of its columns, 256 / (D / 4) rows per workgroup, registers for eight waves a SIMD.
+// them and request sums and statistics together, so that one latency is left of several.  Few parts, or many rows, are bound by
+// HBM: a thread has all parts of its columns, 256 / (D / 4) rows per workgroup, registers for eight waves a SIMD.
 // One wave per row, statistics first, then eight parts at a time, took (us, old -> this): 17 parts of 32 rows D128 5.8 -> 4.6,
 // 64 of 64 rows D64 6.5 -> 4.1; 2 parts of 32768 rows D128 21.2 -> 9.8 (42 MB), 8 of 18432 rows D64 10.0 -> 5.9.
 struct CombineRow {
@@ -44,8 +44,11 @@ __device__ __forceinline__ void combine_store(const FwdArgs& a, const CombineRow
   if (a.lse && col == 0) a.lse[lse_offset(c.si, c.h, a.hq) + c.pq] = lse_of(m, sc, l);
 }
 
-// More than this: a workgroup per row (its reduction through LDS costs what one more round of loads does).
-constexpr int kManyParts = 8;
+// A workgroup per row: more parts than kManyParts (its reduction through LDS costs what one more round of loads does) and no
+// more rows than kManyRows, beyond which most of its threads have nothing to load and the rows come to thousands of workgroups (us,
+// a workgroup per row / all parts in one thread: D64 11 parts of 768 rows 4.3 / 4.8, 10 of 6144 12.4 / 6.4, D128 10 of 96 4.2 / 4.5, of 768
+// 5.1 / 5.1, of 4096 12.4 / 7.2).  Split tiles have at most kMostTileParts parts, packed rows with more never that many rows.
+constexpr int kManyParts = 8, kMostTileParts = 16, kManyRows = 1024;
 
 template <typename T, int D, int kParts>      // at most kParts parts, four of them in flight
 static __global__ __launch_bounds__(256, 8) void combine_rows_kernel(const FwdArgs a) {
@@ -143,10 +146,11 @@ hipError_t launch_combine_rows(const FwdArgs& a, int pairs, hipStream_t stream) 
   const int64_t blocks = (int64_t)pairs * a.row_blocks;
   if (blocks * a.part_rows == 0) return hipSuccess;
   constexpr int ROWS = 256 / (D / 4);
-  if (a.splits > kManyParts)
+  if (a.splits > kMostTileParts || (a.splits > kManyParts && blocks * a.part_rows <= kManyRows))
     hipLaunchKernelGGL((combine_many_kernel<T, D>), dim3((unsigned)(blocks * a.part_rows)), dim3(256), 0, stream, a);
   else
-    hipLaunchKernelGGL((a.splits > 2 ? combine_rows_kernel<T, D, kManyParts> : combine_rows_kernel<T, D, 2>),
+    hipLaunchKernelGGL((a.splits > kManyParts ? combine_rows_kernel<T, D, kMostTileParts>
+                        : a.splits > 2 ? combine_rows_kernel<T, D, kManyParts> : combine_rows_kernel<T, D, 2>),
                        dim3((unsigned)(blocks * ((a.part_rows + ROWS - 1) / ROWS))), dim3(256), 0, stream, a);
   return hipGetLastError();
 }

@@ -81,20 +81,53 @@ def test_few_rows_meet_the_oracle(case):
         assert (L[seen] - rl[seen]).abs().max().item() <= LSE_ATOL if seen.any() else True
 
 
+def _scratch_bytes(rows, D):      # the parts' fp32 sums and statistics
+    return rows * (4 * D + 8)
+
+
+def _scratch_of(call):
+    """its result, and the memory that it held beside its result: the scratch of a split forward (_forward's outputs excluded)"""
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    out = call()
+    stats = torch.cuda.memory_stats()
+    return out, stats['requested_bytes.all.peak'] - stats['requested_bytes.all.current']
+
+
 @pytest.mark.parametrize('D', [64, 128, 256])
 @pytest.mark.parametrize('parts', [2, 3, 4, 5, 8, 9, 17, 63, 64])
 def test_sums_of_few_and_many_parts(parts, D):
     """One row block and 128 keys a part (four waves of 32): up to eight parts each thread has all of its columns' (two, or two
-    groups of four), beyond that the threads of a workgroup share them."""
+    groups of four), beyond that the threads of a workgroup share them.  (Two parts of that many keys do not pay; of 1024 and for
+    100 K/V heads they do.)"""
     from oracle import fa_ref
-    q, k, v, _, _ = make_inputs(1, 5, 1, 1, 128 * parts, D, torch.bfloat16, DEV, seed=parts)
+    Hk, Sk = (100, 1024) if parts == 2 else (1, 128 * parts)
+    q, k, v, _, _ = make_inputs(1, 5 * Hk, Hk, 1, Sk, D, torch.bfloat16, DEV, seed=parts)
     f = lambda t: t.float()
     sm = D ** -0.5
     ro, rl, _ = fa_ref.attn_fwd_ref(f(q), f(k), f(v), None, sm, 0, 0, 0)
     lo, _, _ = fa_ref.attn_fwd_ref(q, k, v, None, sm, 0, 0, 0)
-    o, L = _forward(q, k, v, None, sm, False, True)
+    (o, L), scratch = _scratch_of(lambda: _forward(q, k, v, None, sm, False, True))
+    assert scratch == _scratch_bytes(parts * 5 * Hk, D)      # as many parts of five rows
     check('out', o, ro, lo, FUDGE['out'])
-    assert (L.view(1, 5, 1) - rl).abs().max().item() <= LSE_ATOL
+    assert (L.view(1, 5 * Hk, 1) - rl).abs().max().item() <= LSE_ATOL
+
+
+@pytest.mark.parametrize('D, H, Sq, Sk, parts', [
+    (64, 8, 767, 3000, 5), (64, 5, 1000, 3000, 8), (64, 4, 767, 4100, 9), (64, 2, 1030, 8192, 10), (64, 4, 1000, 11825, 16),
+    (128, 5, 1000, 4100, 5), (128, 5, 1000, 6000, 8), (128, 4, 1000, 11825, 9), (128, 4, 767, 6000, 12), (128, 2, 1030, 11825, 15)])
+def test_sums_of_many_parts_of_many_rows(D, H, Sq, Sk, parts):
+    """split tiles have more rows than packed rows ever do: all parts of a column in one thread, in two to four groups of four"""
+    from oracle import fa_ref
+    q, k, v, _, _ = make_inputs(1, H, H, Sq, Sk, D, torch.bfloat16, DEV, seed=parts)
+    f = lambda t: t.float()
+    sm = D ** -0.5
+    ro, rl, _ = fa_ref.attn_fwd_ref(f(q), f(k), f(v), None, sm, 0, 0, 0)
+    lo, _, _ = fa_ref.attn_fwd_ref(q, k, v, None, sm, 0, 0, 0)
+    (o, L), scratch = _scratch_of(lambda: _forward(q, k, v, None, sm, False, True))
+    assert scratch == _scratch_bytes(parts * H * ((Sq + 255) // 256) * 256, D)
+    check('out', o, ro, lo, FUDGE['out'])
+    assert (L.view(1, H, Sq) - rl).abs().max().item() <= LSE_ATOL
 
 
 def test_scores_that_grow_and_huge_scores():
