@@ -408,17 +408,24 @@ std::tuple<Tensor, Tensor> key_mask_kernel(const Tensor& q, const Tensor& k, con
   const Tensor m = mask.expand({q.size(0), q.size(1), 1, k.size(2)});
   Tensor o = at::empty({q.size(0), q.size(1), q.size(2), v.size(3)}, q.options());
   Tensor lse = at::empty({q.size(0) * q.size(1), q.size(2)}, q.options().dtype(at::kFloat));
-  p.B.ptr = m.numel() > 0 ? m.data_ptr() : nullptr;
-  for (int i = 0; i < 4; ++i) {
-    p.B.sizes[i] = (uint64_t)(i == 2 ? q.size(2) : m.size(i));
-    p.B.strides[i] = (uint64_t)(i == 2 ? 0 : m.stride(i));
+  int rc = FA_ERROR_NOT_SUPPORTED;
+  // (what is known here to be refused is not asked for)
+  if (m.numel() > 0 && q.element_size() == 2 && q.size(3) <= 128 && v.size(3) <= 128) {
+    p.B.ptr = m.data_ptr();
+    for (int i = 0; i < 4; ++i) {
+      p.B.sizes[i] = (uint64_t)(i == 2 ? q.size(2) : m.size(i));
+      p.B.strides[i] = (uint64_t)(i == 2 ? 0 : m.stride(i));
+    }
+    p.B.dtype = FA_DTYPE_UINT8;
+    TORCH_CHECK(view2(lse, &p.L) && view4(o, &p.Out), "outputs");
+    Scratch scratch;
+    rc = fa_attn_fwd_key_mask(&p, FA_FWD_PARAMS_VERSION, current_stream(), nullptr, &scratch.c);
   }
-  p.B.dtype = FA_DTYPE_UINT8;
-  TORCH_CHECK(view2(lse, &p.L) && view4(o, &p.Out), "outputs");
-  Scratch scratch;
-  const int rc = p.B.ptr == nullptr ? (int)FA_ERROR_NOT_SUPPORTED
-                                    : fa_attn_fwd_key_mask(&p, FA_FWD_PARAMS_VERSION, current_stream(), nullptr, &scratch.c);
-  if (rc == FA_ERROR_NOT_SUPPORTED) return forward_additive(q, k, v, mask, sm_scale);
+  if (rc == FA_ERROR_NOT_SUPPORTED) {      // nothing was launched: the additive mask instead, into the same outputs
+    const Tensor b = broadcast_bias(additive_mask(mask, q.options()), q, k);
+    TORCH_CHECK(view4(b.numel() > 0 ? b : Tensor(), &p.B), "the last stride of tensors must be 1");
+    rc = run_forward(p, lse, o, Tensor());
+  }
   check_rc(rc, false);
   return {std::move(o), std::move(lse)};
 }

@@ -96,6 +96,25 @@ def test_boolean_key_masks_are_the_additive_ones(case, form):
     assert og.requires_grad and torch.equal(og, sdpa(q, k, v, attn_mask=additive))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize('case', BOOL[-4:], ids=_id)
+def test_masks_made_additive_cost_one_allocation(case):
+    """a boolean mask that the kernels do not read: its additive copy, the outputs, and nothing twice"""
+    from aotriton_amd.torch_ops import scaled_dot_product_attention as sdpa
+    B, H, Sq, Sk, D, dt = case
+    q, k, v = (torch.randn(B, H, s, D, device='cuda').to(dt) for s in (Sq, Sk, Sk))
+    mask = torch.rand(B, 1, 1, Sk, device='cuda') < 0.7
+    additive = torch.zeros(mask.shape, device='cuda', dtype=dt).masked_fill(~mask, float('-inf'))
+    count = lambda: torch.cuda.memory_stats()['allocation.all.allocated']
+    taken = []
+    for m in (mask, additive):
+        sdpa(q, k, v, attn_mask=m)
+        before = count()
+        sdpa(q, k, v, attn_mask=m)
+        taken.append(count() - before)
+    assert taken[0] == taken[1] + 1
+
+
 def test_fake_key_mask_op():
     import aotriton_amd.torch_ops  # noqa: F401
     q = torch.empty(2, 4, 8, 64, device='meta', dtype=HF)
