@@ -172,11 +172,22 @@ void fwd_rows_kernel(const FwdArgs a) {
       for (int i = 0; i < 16; ++i) s[i] *= qk_scale;
     const int n0 = b * 32;
     if (kBias && a.key_mask) {
+      // (0 or -inf is added, not selected: what an additive mask makes of inf and NaN)
+      if (a.sb_n == 1 && n0 + 32 <= si.seqlen_k) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        int n = n0 + 8 * (i / 4) + 4 * hi + (i % 4);
-        n = n < si.seqlen_k ? n : si.seqlen_k - 1;
-        s[i] = mptr[(int64_t)n * a.sb_n] != 0 ? s[i] : -__builtin_inff();
+        for (int g = 0; g < 4; ++g) {
+          uint32_t m4;
+          __builtin_memcpy(&m4, mptr + n0 + 8 * g + 4 * hi, 4);      // (masks may start anywhere)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) s[4 * g + r] += (m4 & 0xffu << 8 * r) != 0 ? 0.f : -__builtin_inff();
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          int n = n0 + 8 * (i / 4) + 4 * hi + (i % 4);
+          n = n < si.seqlen_k ? n : si.seqlen_k - 1;
+          s[i] += mptr[(int64_t)n * a.sb_n] != 0 ? 0.f : -__builtin_inff();
+        }
       }
     } else if (kBias) {
       if (bias_vec && n0 + 32 <= si.seqlen_k) {

@@ -97,6 +97,26 @@ def test_boolean_key_masks_are_the_additive_ones(case, form):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('score', ['inf', '-inf', 'nan'])
+@pytest.mark.parametrize('case', [(1, 16, 1, 3000, 64, BF), (2, 16, 7, 70, 128, HF), (16, 12, 384, 384, 64, HF)], ids=_id)
+def test_hidden_keys_of_any_score(case, score):
+    """a hidden key whose score is infinite or NaN: in the packed-rows kernel as in the tiles what the additive mask gives"""
+    from aotriton_amd.torch_ops import scaled_dot_product_attention as sdpa
+    B, H, Sq, Sk, D, dt = case
+    g = torch.Generator(device='cuda').manual_seed(5)
+    q, k, v = (torch.randn(B, H, s, D, device='cuda', generator=g).to(dt) for s in (Sq, Sk, Sk))
+    q[..., 0] = 1.0
+    k[0, 3, 17] = 0.0
+    k[0, 3, 17, 0] = float(score)      # one key of one head
+    mask = torch.ones(B, 1, 1, Sk, device='cuda', dtype=torch.bool)
+    mask[..., 17] = False
+    additive = torch.zeros(mask.shape, device='cuda', dtype=dt).masked_fill(~mask, float('-inf'))
+    o, want = sdpa(q, k, v, attn_mask=mask), sdpa(q, k, v, attn_mask=additive)
+    assert torch.equal(o.isnan(), want.isnan()) and torch.equal(o.nan_to_num(), want.nan_to_num())
+    assert want[0, 3].isnan().any().item() == (score != '-inf')
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize('case', BOOL[-4:], ids=_id)
 def test_masks_made_additive_cost_one_allocation(case):
     """a boolean mask that the kernels do not read: its additive copy, the outputs, and nothing twice"""
