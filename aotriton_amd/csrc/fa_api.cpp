@@ -1152,7 +1152,7 @@ int fa_query_bwd_config(const fa_bwd_params* params, const fa_options* options, 
                           : valu  ? (kernel_slot == 1 ? fa::TileShape{1, 32, 4, 0} : fa::TileShape{32, 1, 4, 0})
                           : kernel_slot == 1 && wide_dkdv ? fa::bwd_wide_shape(true)
                           : kernel_slot == 2 && route.wide_dq ? fa::bwd_wide_shape(false)
-                                  : fa::bwd_tile_shape(params->Q.dtype, s.d, s.windowed, s.bias, s.dropout, kernel_slot);
+                                  : fa::bwd_tile_shape(params->Q.dtype, s.d, s.windowed, s.bias, s.dropout, kernel_slot, need > 0);
   const int nz = s.num_seqlens != 0 ? std::abs(s.num_seqlens) : s.batch;
   out->block_m = t.block_m; out->block_n = t.block_n; out->num_waves = t.num_waves;
   out->lds_bytes = t.lds_bytes;

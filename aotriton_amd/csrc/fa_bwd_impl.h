@@ -1659,13 +1659,15 @@ hipError_t launch_bwd_dq(const BwdArgs& a0, bool windowed, bool bias, bool dropo
 #undef FA_CALL
 }
 
-// the tile of a kernel slot, as the launchers above choose it
-template <typename T, int D, bool W, bool B, bool P> TileShape bwd_shape(int slot) {
-  constexpr int NW = BwdTile<T, D, W>::NW, BM = kDkDvBM<T, D, W, B, P>, BN = kDqBN<T, D, W, B>;
+// the tile of a kernel slot, as the launchers above choose it (`stored`: the dK/dV kernel that stores dS)
+template <typename T, int D, bool W, bool B, bool P> TileShape bwd_shape(int slot, bool stored) {
+  constexpr int NW = BwdTile<T, D, W>::NW, BM = kDkDvBM<T, D, W, B, P>, SM = kDkDvBM<T, D, W, B, P, true>, BN = kDqBN<T, D, W, B>;
   constexpr int FM = kFusedBM<T, D, W>, FN = kFusedBN<T, D, W>, per_cu = kTwoWaves<D, B> ? 2 : 1;
   switch (slot) {
     case 0: return TileShape{256 / (D / 8), 0, 4, 0};
-    case 1: return TileShape{BM, NW * 32, NW, DkDvSmem<D, BM>::BYTES + (D < 256 ? kLevelBytes : 0), per_cu};
+    case 1:
+      return TileShape{stored ? SM : BM, NW * 32, NW,
+                       (stored ? DkDvSmem<D, SM>::BYTES : DkDvSmem<D, BM>::BYTES) + (D < 256 ? kLevelBytes : 0), per_cu};
     case 2: return TileShape{NW * 32, BN, NW, DqSmem<D, BN>::BYTES, per_cu};
     default:
       return TileShape{NW * 32, NW * 32, NW,

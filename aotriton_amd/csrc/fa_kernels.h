@@ -59,7 +59,7 @@ hipError_t run_bwd_dkdv_wide(int dtype, const BwdArgs& a, bool windowed, hipStre
 hipError_t run_bwd_dq_wide(int dtype, const BwdArgs& a, bool windowed, hipStream_t s);
 TileShape bwd_wide_shape(bool dkdv);
 hipError_t run_bwd_fused(int dtype, int head_dim, const BwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
-TileShape bwd_tile_shape(int dtype, int head_dim, bool windowed, bool bias, bool dropout, int kernel_slot);
+TileShape bwd_tile_shape(int dtype, int head_dim, bool windowed, bool bias, bool dropout, int kernel_slot, bool stored_ds);
 // dQ = dS K from the dS tiles that the dK/dV kernel stored (BwdArgs::ds_ws), and their geometry
 hipError_t run_bwd_dqs(int dtype, int head_dim, const BwdArgs& a, hipStream_t s);
 void ds_tile_counts(int head_dim, int max_sq, int max_sk, int* ntq, int* ntk, int64_t* tile_bytes);

@@ -19,16 +19,16 @@ template <typename T, int D> static TileShape fwd_shape_of(bool windowed, int ha
   return windowed ? shape(FwdTile<T, D, true>{}, 1) : shape(FwdTile<T, D, false>{}, 1);
 }
 
-template <typename T, int D> static TileShape bwd_shape_of(bool windowed, bool bias, bool dropout, int slot) {
+template <typename T, int D> static TileShape bwd_shape_of(bool windowed, bool bias, bool dropout, int slot, bool stored) {
   switch ((windowed ? 4 : 0) | (bias ? 2 : 0) | (dropout ? 1 : 0)) {
-    case 0: return bwd_shape<T, D, false, false, false>(slot);
-    case 1: return bwd_shape<T, D, false, false, true>(slot);
-    case 2: return bwd_shape<T, D, false, true, false>(slot);
-    case 3: return bwd_shape<T, D, false, true, true>(slot);
-    case 4: return bwd_shape<T, D, true, false, false>(slot);
-    case 5: return bwd_shape<T, D, true, false, true>(slot);
-    case 6: return bwd_shape<T, D, true, true, false>(slot);
-    default: return bwd_shape<T, D, true, true, true>(slot);
+    case 0: return bwd_shape<T, D, false, false, false>(slot, stored);
+    case 1: return bwd_shape<T, D, false, false, true>(slot, stored);
+    case 2: return bwd_shape<T, D, false, true, false>(slot, stored);
+    case 3: return bwd_shape<T, D, false, true, true>(slot, stored);
+    case 4: return bwd_shape<T, D, true, false, false>(slot, stored);
+    case 5: return bwd_shape<T, D, true, false, true>(slot, stored);
+    case 6: return bwd_shape<T, D, true, true, false>(slot, stored);
+    default: return bwd_shape<T, D, true, true, true>(slot, stored);
   }
 }
 
@@ -41,12 +41,12 @@ TileShape fwd_tile_shape(int dtype, int head_dim, bool windowed, int half_tiles)
   }
 }
 
-TileShape bwd_tile_shape(int dtype, int head_dim, bool windowed, bool bias, bool dropout, int slot) {
+TileShape bwd_tile_shape(int dtype, int head_dim, bool windowed, bool bias, bool dropout, int slot, bool stored) {
   const bool bf = dtype == kDtypeBF16;
   switch (head_dim) {
-    case 64: return bf ? bwd_shape_of<bf16_t, 64>(windowed, bias, dropout, slot) : bwd_shape_of<f16_t, 64>(windowed, bias, dropout, slot);
-    case 128: return bf ? bwd_shape_of<bf16_t, 128>(windowed, bias, dropout, slot) : bwd_shape_of<f16_t, 128>(windowed, bias, dropout, slot);
-    default: return bf ? bwd_shape_of<bf16_t, 256>(windowed, bias, dropout, slot) : bwd_shape_of<f16_t, 256>(windowed, bias, dropout, slot);
+    case 64: return bf ? bwd_shape_of<bf16_t, 64>(windowed, bias, dropout, slot, stored) : bwd_shape_of<f16_t, 64>(windowed, bias, dropout, slot, stored);
+    case 128: return bf ? bwd_shape_of<bf16_t, 128>(windowed, bias, dropout, slot, stored) : bwd_shape_of<f16_t, 128>(windowed, bias, dropout, slot, stored);
+    default: return bf ? bwd_shape_of<bf16_t, 256>(windowed, bias, dropout, slot, stored) : bwd_shape_of<f16_t, 256>(windowed, bias, dropout, slot, stored);
   }
 }
 

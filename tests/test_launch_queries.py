@@ -87,18 +87,25 @@ def test_forward_variants():
     assert fwd(1, 32, 8, 1, 4000, 128, p=0.1).flags & 192 == 0   # dropout stays on the tile kernel
 
 
-@pytest.mark.parametrize('slot, bias, p, tile, lds, grid', [
-    (1, False, 0.0, (64, 128), 72704, 512),
-    (1, False, 0.1, (64, 128), 72704, 512),
-    (1, True, 0.0, (128, 128), 141312, 2048),                    # one workgroup per item with a bias
-    (1, True, 0.1, (64, 128), 72704, 2048),
-    (2, False, 0.0, (128, 64), 51200, 512),
-    (2, True, 0.0, (128, 128), 100352, 2048),
-    (3, False, 0.0, (128, 128), 137216, 256),
-    (3, True, 0.1, (128, 128), 137216, 4096),
+@pytest.mark.parametrize('slot, bias, p, stored, tile, lds, grid', [
+    (1, False, 0.0, False, (64, 128), 72704, 512),
+    (1, False, 0.1, True, (64, 128), 72704, 512),
+    (1, True, 0.0, True, (64, 128), 72704, 2048),                # one workgroup per item with a bias; 64-query steps storing dS,
+    (1, True, 0.0, False, (128, 128), 141312, 2048),             # 128 recomputing it
+    (1, True, 0.1, True, (64, 128), 72704, 2048),
+    (1, True, 0.1, False, (64, 128), 72704, 2048),
+    (2, False, 0.0, False, (128, 64), 51200, 512),
+    (2, True, 0.0, True, (128, 128), 100352, 2048),
+    (3, False, 0.0, False, (128, 128), 137216, 256),
+    (3, True, 0.1, False, (128, 128), 137216, 4096),
 ])
-def test_backward_variants_at_head_dim_64(slot, bias, p, tile, lds, grid):
-    c = bwd(slot, 8, 16, 16, 2048, 2048, 64, bias=bias, p=p)
+def test_backward_variants_at_head_dim_64(slot, bias, p, stored, tile, lds, grid):
+    from aotriton_amd._lib import lib
+    lib.fa_set_bwd_workspace_limit(-1 if stored else 0)
+    try:
+        c = bwd(slot, 8, 16, 16, 2048, 2048, 64, bias=bias, p=p)
+    finally:
+        lib.fa_set_bwd_workspace_limit(-1)
     assert ((c.block_m, c.block_n), c.lds_bytes, c.grid[0]) == (tile, lds, grid)
 
 
