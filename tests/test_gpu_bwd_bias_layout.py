@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from test_gpu_attention import _run_case
+from test_launch_queries import bwd
 from _util import make_inputs
 
 pytestmark = pytest.mark.gpu
@@ -130,6 +131,8 @@ def test_stored_ds_under_rows_at_any_alignment(D, Sq, Sk, causal, p):
         view(b).copy_(values)
         db = torch.full_like(b, 7.0)
         dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+        strides = view(db).stride()
+        assert bwd(1, B, H, H, Sq, Sk, D, causal, p, bias=strides, db=True, at=2 * at).flags & 16
         err = flash.attn_bwd(q, k, v, view(b), sm, o, do, dq, dk, dv, view(db), flash.lazy_dq_acc(q), L,
                              flash.lazy_delta(L), p, seed, off, 0, causal)
         assert err == flash.hipError_t.hipSuccess
@@ -140,8 +143,9 @@ def test_stored_ds_under_rows_at_any_alignment(D, Sq, Sk, causal, p):
         assert torch.isfinite(x).all() and torch.equal(x, y)
 
 
-@pytest.mark.parametrize('B,H,Sq,Sk,causal,layout', [(1, 8, 1024, 1024, False, 'padded'), (1, 4, 1000, 1023, True, 'odd'),
-                                                     (2, 8, 1024, 1000, (300, 100), 'odd')])
+@pytest.mark.parametrize('B,H,Sq,Sk,causal,layout', [(1, 8, 1024, 1024, False, 'padded'), (1, 5, 1000, 1023, True, 'odd'),
+                                                     (1, 5, 1024, 1000, (600, 400), 'odd')])
 def test_parts_with_a_bias(B, H, Sq, Sk, causal, layout):
-    """dK/dV items cut into parts, several to a CU, at D = 64 with a bias: against the oracle"""
+    """dK/dV items that store dS cut into parts, several to a CU, at D = 64 with a bias: against the oracle"""
+    assert bwd(1, B, H, H, Sq, Sk, 64, causal, bias=True, db=True).flags & 80 == 80
     _run_case(B, H, H, Sq, Sk, 64, BF, causal, bias=True, bias_layout=layout, seed=33)

@@ -96,6 +96,66 @@ def test_boolean_key_masks_are_the_additive_ones(case, form):
     assert og.requires_grad and torch.equal(og, sdpa(q, k, v, attn_mask=additive))
 
 
+GROUPED = [      # B, Hq, Hk, Sq, Sk, D, dtype, packed rows?
+    (1, 32, 8, 1, 3000, 128, BF, True),
+    (2, 12, 4, 7, 501, 64, HF, True),
+    (3, 6, 2, 11, 401, 40, BF, True),
+    (16, 16, 4, 300, 301, 64, HF, False),
+    (8, 32, 8, 290, 131, 128, BF, False),
+]
+TL, BOTTOM_RIGHT = -2147483647, -2147483646
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('case', GROUPED, ids=_id)
+def test_boolean_key_masks_per_head_with_fewer_kv_heads(case):
+    """a mask of its own for every query head, whose rows are packed by K/V head in one of the kernels: the additive one's bits"""
+    from aotriton_amd.torch_ops import scaled_dot_product_attention as sdpa
+    B, Hq, Hk, Sq, Sk, D, dt, rows = case
+    assert bool(fwd(B, Hq, Hk, Sq, Sk, D, bias=True).flags & 128) == rows
+    g = torch.Generator(device='cuda').manual_seed(5)
+    q, k, v = (torch.randn(B, h, s, D, device='cuda', generator=g).to(dt) for h, s in ((Hq, Sq), (Hk, Sk), (Hk, Sk)))
+    for shape in ((B, Hq, 1, Sk), (1, Hq, 1, Sk), (B, 1, 1, Sk)):
+        mask = torch.rand(shape, device='cuda', generator=g) < 0.7
+        additive = torch.zeros(shape, device='cuda', dtype=dt).masked_fill(~mask, float('-inf'))
+        assert torch.equal(sdpa(q, k, v, attn_mask=mask, enable_gqa=True), sdpa(q, k, v, attn_mask=additive, enable_gqa=True))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('window', [(0, 0, 0), (3, TL, TL), (3, BOTTOM_RIGHT, BOTTOM_RIGHT), (3, 40, 25), (3, 100, -3)])
+@pytest.mark.parametrize('case', GROUPED, ids=_id)
+def test_key_mask_entry_point_takes_windows(case, window):
+    """fa_attn_fwd_key_mask against fa_attn_fwd with the additive mask, under every kind of window: the same bits; rows of a mask
+    and other element types are refused"""
+    import ctypes
+    from aotriton_amd._lib import lib
+    from aotriton_amd.flash import mk_aotensor
+    from aotriton_amd.pyaotriton.v3.flash import attn_fwd_params
+    B, Hq, Hk, Sq, Sk, D, dt, _ = case
+    g = torch.Generator(device='cuda').manual_seed(5)
+    q, k, v = (torch.randn(B, h, s, D, device='cuda', generator=g).to(dt) for h, s in ((Hq, Sq), (Hk, Sk), (Hk, Sk)))
+    mask = torch.rand(B, Hq, 1, Sk, device='cuda', generator=g) < 0.7
+    additive = torch.zeros(mask.shape, device='cuda', dtype=dt).masked_fill(~mask, float('-inf'))
+    stream, out = torch.cuda.current_stream().cuda_stream, []
+    for b in (mask.view(torch.uint8), additive):
+        o, L = torch.full_like(q, 7.0), torch.full((B * Hq, Sq), 7.0, device='cuda')
+        x = attn_fwd_params()
+        x.Q, x.K, x.V, x.Out, x.L, x.B = (mk_aotensor(t) for t in (q, k, v, o, L, b.expand(B, Hq, Sq, Sk)))
+        x.Sm_scale, x.causal_type, x.window_left, x.window_right = D ** -0.5, *window
+        c = x.to_c()
+        if b is additive:
+            rc = lib.fa_attn_fwd(ctypes.byref(c), x.kVersion, stream, None)
+            assert lib.fa_attn_fwd_key_mask(ctypes.byref(c), x.kVersion, stream, None, None) == 1      # not a mask of bytes
+        else:
+            rc = lib.fa_attn_fwd_key_mask(ctypes.byref(c), x.kVersion, stream, None, None)
+            if Sq > 1:
+                c.B.strides[2] = Sk
+                assert lib.fa_attn_fwd_key_mask(ctypes.byref(c), x.kVersion, stream, None, None) == 801
+        assert rc == 0
+        out.append((o, L))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize('score', ['inf', '-inf', 'nan'])
 @pytest.mark.parametrize('case', [(1, 16, 1, 3000, 64, BF), (2, 16, 7, 70, 128, HF), (16, 12, 384, 384, 64, HF)], ids=_id)

@@ -23,9 +23,10 @@ def fwd(B, Hq, Hk, Sq, Sk, D, causal=False, p=0.0, bias=False, num_cu=256):
     return c
 
 
-def bwd(slot, B, Hq, Hk, Sq, Sk, D, causal=False, p=0.0, bias=False, db=False):
+def bwd(slot, B, Hq, Hk, Sq, Sk, D, causal=False, p=0.0, bias=False, db=False, at=0):
+    """bias: whether there is one, or its strides (`at` bytes behind a 16-byte boundary); db: the gradient is laid out as it is"""
     from aotriton_amd.pyaotriton.v3.flash import attn_bwd_params, query_bwd_config
-    from aotriton_amd.pyaotriton import lazy_tensor
+    from aotriton_amd.pyaotriton import DType, T4, lazy_tensor
     x = attn_bwd_params()
     x.Q = x.DQ = view(B, Hq, Sq, D)
     x.Out = x.DO = view(B, Hq, Sq, D)
@@ -33,6 +34,8 @@ def bwd(slot, B, Hq, Hk, Sq, Sk, D, causal=False, p=0.0, bias=False, db=False):
     x.L = view(B * Hq, Sq, name='kFloat32')
     x.D = lazy_tensor.eager_delta(x.L)
     _common(x, B, Hq, Sq, Sk, causal, p, bias)
+    if isinstance(bias, tuple):
+        x.B = T4(4096 + at, [B, Hq, Sq, Sk], list(bias), DType.kBFloat16)
     if db:
         x.DB = x.B
     err, c = query_bwd_config(x, slot)
