@@ -780,9 +780,10 @@ int64_t ds_workspace_need(const fa_bwd_params* p, const Shape& s, int* ntq, int*
   if (s.elementwise || !is_16bit(p->Q.dtype) || (s.d != 64 && s.d != 128 && s.d != 256) || s.num_seqlens != 0 ||
       s.batch <= 0 || s.max_sq <= 0 || s.max_sk <= 0)
     return 0;
-  // dB leaves the dQ-from-dS kernel as 16-byte pieces of its rows, wherever they start (rows at odd places left to the recomputing
-  // one: B9 H16 S1007 D64 bf16 forward + backward 732 us, stored 576; B16 H12 S700 fp16 520 -> 383); columns that lie apart are left to the recomputing one; so are small
-  // calls, where the third launch costs what is saved (us forward + backward, recomputing -> stored: B2 H8 S256 D64
+  // dB leaves the dQ-from-dS kernel as 16-byte pieces of its rows, wherever they start (rows at odd places left to the
+  // recomputing one: B9 H16 S1007 D64 bf16 forward + backward 732 us, stored 576; B16 H12 S700 fp16 520 -> 383).  Columns that
+  // lie apart are left to the recomputing one; so are small calls,
+  // where the third launch costs what is saved (us forward + backward, recomputing -> stored: B2 H8 S256 D64
   // 50 -> 53, B8 H12 S512 D64 118 -> 100, D128 148 -> 132, D256 468 -> 420, B16 H16 S1024 D64 842 -> 795, causal 670 -> 579),
   // and long rows at D = 64.  There (us of the backward alone, recomputing -> stored, B1): H8 S4096 causal 312 -> 300, H16
   // S4096 610 -> 560, window 1000 283 -> 254, S6144 causal 793 -> 744, S8192 2195 -> 2050, window 1000 713 -> 710, but causal

@@ -625,6 +625,8 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
   };
 
   // ---- main loop: LDS double buffer, one barrier per tile ---------------------
+  // (Of the tiles past wave_hi, which a wave does not work on, it fetches the bias all the same.  Left out, causal at D = 64, us, B8
+  // H16 S256 12.8 -> 12.4, B4 H16 S357 and B8 H12 S512 level, B9 H16 S400 25.3 -> 25.9.)
   request_bias(br.lo);
   store_tile(0);
   __syncthreads();

@@ -338,8 +338,8 @@ FA_API int fa_attn_bwd_noalloc(const fa_bwd_params* params, int32_t params_versi
  * reused by every later call (calls on one device take turns: a call on another stream than the last
  * one waits on the GPU for the last one's kernels).  Its main user is the split backward.  For 16-bit tensors at head
  * dims up to 256 (dense batches, not under stream capture; up to head dim 128 only where it pays: with dropout or a
- * bias, and at 65-128 also for calls too small for the kernels with 64 rows per wave; with dB when its rows are made of aligned 16-byte pieces and the call is neither small nor, at head dim 64,
- * longer than 4096 keys) fa_attn_bwd keeps dS in HBM between its dK/dV and dQ kernels instead of
+ * bias, and at 65-128 also for calls too small for the kernels with 64 rows per wave; with dB when its columns are adjacent (its rows may start anywhere) and the call is neither small nor, at head
+ * dim 64, longer than 4096 keys) fa_attn_bwd keeps dS in HBM between its dK/dV and dQ kernels instead of
  * recomputing S and dP in the dQ kernel (5 GEMMs instead of 7; delta kernel, dK/dV kernel writing dS,
  * dQ = dS K kernel): 2 bytes per (batch, q-head, query, key) plus 8 bytes per (batch, q-head, query).
  * The others: parts of dK/dV items where these do not fill the chip (fp32 sums), split forwards
