@@ -142,8 +142,13 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
                    (int64_t)hk * a.sk.h + (int64_t)si.k_start * a.sk.s;
   const T* vbase = reinterpret_cast<const T*>(a.v) + (int64_t)si.batch_index * a.sv.z +
                    (int64_t)hk * a.sv.h + (int64_t)si.k_start * a.sv.s;
+  // This lane's bias row, for the layouts that are read without the wave's area.  In the windowed 256-row tiles of aligned rows,
+  // which take them only at an item's end, it is formed where it is read (causal, bias and dropout, us, held -> formed: D128 B4 H16
+  // S1024 bf16 86 -> 74, fp16 74 -> 72, D64 bf16 72 -> 59).  Not without dropout at 96 columns (2 % slower) and at D = 64 in bf16
+  // (window, S1024 29.5 -> 27.5, but S1000, whose last tile reads elements, 32 -> 36.5).
+  constexpr bool kHoldRow = kAnyRow || NW == 4 || !kWindowed || (!kDropout && (kPad == 96 || (D == 64 && __is_same(T, bf16_t))));
   const T* bptr = nullptr;
-  if (kBias)
+  if (kBias && kHoldRow)
     bptr = reinterpret_cast<const T*>(a.bias) + (int64_t)si.batch_index * a.sb_z + (int64_t)h * a.sb_h +
            (int64_t)row_c * a.sb_m;
 
@@ -313,6 +318,11 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
   // The tiles of 256 rows have no registers for that (75 more spilled at D = 64, 45 at D = 128): the pieces are requested behind
   // the QK MFMAs.
   constexpr bool kBiasAhead = kBias && !kKeyBias && NW == 4;
+  // kBufferBias: aligned rows of a whole tile come through a descriptor of the wave's rows, which reads rows past the sequence as
+  // zero: one address register instead of a clamped offset per row (us, offsets -> this, with the rows below formed where they are
+  // read: D128 causal with dropout B4 H16 S1024 bf16 91 -> 74, fp16 91 -> 72, without dropout bf16 52 -> 46; D64 causal with dropout
+  // bf16 72 -> 59, fp16 74 -> 63).  At 96 columns without dropout, where nothing spills, it is 4 % slower.
+  constexpr bool kBufferBias = !kAnyRow && (kDropout || kPad != 96);
   constexpr int BCK = BN < D ? BN : D;    // keys per chunk
   constexpr int BLPR = BCK / 8;           // 16-byte pieces per chunk row
   constexpr int BRPI = 64 / BLPR;         // rows per wave-wide access
@@ -382,8 +392,15 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
         }
       } else {
         op_t bco[BNI];
+        if constexpr (!kBufferBias) {
 #pragma unroll
-        for (int i = 0; i < BNI; ++i) bco[i] = piece(i);
+          for (int i = 0; i < BNI; ++i) bco[i] = piece(i);
+        } else {
+          const auto brs = wave_rsrc(base, wrows > 0 ? (wrows - 1) * b_row + BCK * 2 : 0);
+#pragma unroll
+          for (int i = 0; i < BNI; ++i)
+            bco[i] = __builtin_bit_cast(op_t, __builtin_amdgcn_raw_buffer_load_b128(brs, brow * b_row + bch * 16, i * BRPI * b_row, 0));
+        }
 #pragma unroll
         for (int i = 0; i < BNI; ++i) put(i, bco[i]);
       }
@@ -427,6 +444,12 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
     __builtin_amdgcn_s_setprio(0);
   };
 
+  [[maybe_unused]] auto row_pointer = [&]() {
+    int r = row_c - b_first;
+    asm volatile("" : "+v"(r));
+    return reinterpret_cast<const T*>(bias_tile + (uint32_t)(r * b_row));
+  };
+
   // scale, bias and mask on the raw scores
   auto prepare = [&](int j, int stage, bool masked) {
     if (kKeyBias) {
@@ -454,6 +477,7 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
           for (int ck = 0; ck < BN / BCK; ++ck) bias_chunk(std::true_type{}, j, ck);
       } else if (bias_vec && (j + 1) * BN <= si.seqlen_k) {
         // a lane's four consecutive keys of every 8-key group in one 8-byte load
+        if constexpr (!kHoldRow) bptr = row_pointer();
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
@@ -463,6 +487,7 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
             for (int r = 0; r < 4; ++r) s[mb][4 * g + r] += (float)b4[r] * kLog2e;   // fwd_kernel_inner.py:187
           }
       } else {
+        if constexpr (!kHoldRow) bptr = row_pointer();
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
 #pragma unroll

@@ -24,6 +24,10 @@ CASES = [
     (1, 2, 140, 97, 200, BF, False),
     (1, 2, 129, 32, 256, HF, False),
     (1, 2, 40, 7, 256, BF, False),
+    (4, 16, 290, 300, 64, HF, (100, 3)),     # whole tiles, waves with few rows or none
+    (4, 16, 270, 392, 64, BF, (200, 10)),
+    (4, 16, 270, 392, 96, BF, True),
+    (4, 16, 257, 256, 128, HF, True),
 ]
 
 
