@@ -603,6 +603,7 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
     l4[0] = *reinterpret_cast<const f32x4*>(stat_ptr(Ls, 0));
     // D = 256 has no registers for the whole column: there the reads run one ahead of their use
     constexpr bool kBiasRing = D >= 256;
+    constexpr bool kBiasNext = kBiasRing && (kWindowed || kPad || !kDropout || __is_same(T, bf16_t));
     typename Tr::q4_t bias4[kBias ? (kBiasRing ? 2 : 4 * MB) : 1];
     auto bias_read = [&](int q) {
       return Tr::lds_read_tr(reinterpret_cast<const T*>(Bt + (32 * (q / 4) + 8 * (q % 4)) * SM::BIAS_STR));
@@ -628,7 +629,8 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
     // An element's bias*log2e - L*log2e.  At D = 256, with one element behind each MFMA, it is formed an element ahead: the mixed
     // multiply-add's result is not ready for the next instruction, and nothing else stands there to be issued.  (With the keep bits
     // of dropout_append4, B2 H16 S8192 fp16, window, bias and dropout: 767 instead of 817 instructions a plain tile, 9 of them s_nop instead
-    // of 51, and 1 % less time: an s_nop costs little.)
+    // of 51, and 1 % less time: an s_nop costs little.)  Not in kBiasNext's one exception, where the compiler spills 16 registers
+    // for it inside the loop (B1 H16 S4096 fp16, bias and dropout, no window, us of the backward: 1066-1093, formed in place 934).
     float bias_next = 0.f;
     auto bias_part = [&](int E) {
       const float bv = (float)bias4[kBiasRing ? (E / 4) & 1 : E / 4][E % 4];
@@ -641,8 +643,8 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
       float x;
       if (kBias) {
         if (kBiasRing && E % 4 == 0 && E + 4 < 16 * MB) bias4[(E / 4 + 1) & 1] = bias_read(E / 4 + 1);
-        const float here = kBiasRing && E % 4 != 0 ? bias_next : bias_part(E);
-        if (kBiasRing && E % 4 != 3) bias_next = bias_part(E + 1);
+        const float here = kBiasNext && E % 4 != 0 ? bias_next : bias_part(E);
+        if (kBiasNext && E % 4 != 3) bias_next = bias_part(E + 1);
         x = __builtin_fmaf(s[mb][i], qk_scale, here);
       } else {
         x = __builtin_fmaf(s[mb][i], qk_scale, -l4[(E / 4) & 1][r]);
@@ -1617,12 +1619,21 @@ hipError_t launch_dkdv_form(const BwdArgs& a0, hipStream_t stream) {
 template <typename T, int D, int kPad, bool W, bool B, bool P, bool kParts>
 hipError_t launch_dkdv_variant(const BwdArgs& a, hipStream_t stream) {
   // (every build has the variant that stores dS; the host decides where it pays)
-  if (a.ds_ws == nullptr) return launch_dkdv_form<T, D, kPad, W, B, P, kParts, false, kBiasAny>(a, stream);
-  if constexpr (B && (!kParts || kTwoDkDv<D, B, P, true, kBiasPlain>)) {
-    if (plain_bias<T>(a)) return launch_dkdv_form<T, D, kPad, W, B, P, kParts, true, kBiasPlain>(a, stream);
-    if (a.seq.num_seqlens == 0 && a.seq.max_seqlen_k >= 8 && a.sb_n == 1)
-      return launch_dkdv_form<T, D, kPad, W, B, P, kParts, true, kBiasRows>(a, stream);
+  const bool rows = a.seq.num_seqlens == 0 && a.seq.max_seqlen_k >= 8 && a.sb_n == 1;      // kBiasRows
+  // D = 256 with dropout: items that recompute, and parts, know a bias of rows, too.  In the form for any layout they spill 14-36
+  // registers inside the loop (us of the backward, fp16, any layout -> rows: without a workspace B2 H8 S1801 causal 374 -> 300, window
+  // 129 -> 107; in parts B2 H8 S1024 causal D256 139 -> 115, D200 134 -> 112).
+  constexpr bool kRows256 = B && P && D == 256;
+  if (a.ds_ws == nullptr) {
+    if constexpr (kRows256)
+      if (rows) return launch_dkdv_form<T, D, kPad, W, B, P, kParts, false, kBiasRows>(a, stream);
+    return launch_dkdv_form<T, D, kPad, W, B, P, kParts, false, kBiasAny>(a, stream);
   }
+  constexpr bool kForms = B && (!kParts || kTwoDkDv<D, B, P, true, kBiasPlain>);
+  if constexpr (kForms)
+    if (plain_bias<T>(a)) return launch_dkdv_form<T, D, kPad, W, B, P, kParts, true, kBiasPlain>(a, stream);
+  if constexpr (kForms || kRows256)
+    if (rows) return launch_dkdv_form<T, D, kPad, W, B, P, kParts, true, kBiasRows>(a, stream);
   return launch_dkdv_form<T, D, kPad, W, B, P, kParts, true, kBiasAny>(a, stream);
 }
 

@@ -149,3 +149,51 @@ def test_parts_with_a_bias(B, H, Sq, Sk, causal, layout):
     """dK/dV items that store dS cut into parts, several to a CU, at D = 64 with a bias: against the oracle"""
     assert bwd(1, B, H, H, Sq, Sk, 64, causal, bias=True, db=True).flags & 80 == 80
     _run_case(B, H, H, Sq, Sk, 64, BF, causal, bias=True, bias_layout=layout, seed=33)
+
+
+@pytest.mark.parametrize('stored', [True, False])
+@pytest.mark.parametrize('D,dt,B,H,Sq,Sk,causal', [(256, HF, 1, 4, 520, 261, False), (256, BF, 1, 4, 300, 261, True),
+                                                   (256, HF, 1, 3, 300, 9, False), (200, BF, 2, 3, 520, 136, True),
+                                                   (200, HF, 1, 4, 300, 389, (100, 30)), (256, BF, 1, 2, 260, 7, False)])
+@pytest.mark.parametrize('layout', ['padded', 'odd'])
+def test_rows_of_a_bias_with_dropout(D, dt, B, H, Sq, Sk, causal, layout, stored):
+    """256 columns, bias and dropout: dK/dV items cut into parts, and items that recompute dS without a workspace, whose bias has
+    rows of unit stride (fewer than eight keys: one of any layout)"""
+    from aotriton_amd._lib import lib
+    lib.fa_set_bwd_workspace_limit(-1 if stored else 0)
+    try:
+        assert bwd(1, B, H, H, Sq, Sk, D, causal, 0.2, bias=True).flags & 80 == (80 if stored else 0)
+        _run_case(B, H, H, Sq, Sk, D, dt, causal, dropout_p=0.2, bias=True, bias_layout=layout, seed=35)
+    finally:
+        lib.fa_set_bwd_workspace_limit(-1)
+
+
+@pytest.mark.parametrize('D', [200, 256])
+@pytest.mark.parametrize('stored', [True, False])
+def test_columns_of_a_bias_apart_with_dropout(D, stored):
+    """the same with the columns of the bias apart, which the views of the bindings take: the bits of adjacent columns"""
+    from aotriton_amd import flash
+    from aotriton_amd._lib import lib
+    from aotriton_amd.pyaotriton import T4
+    B, H, Sq, Sk, causal = 1, 4, 300, 261, True
+    q, k, v, _, do = make_inputs(B, H, H, Sq, Sk, D, BF, 'cuda', seed=16)
+    b = torch.randn(B, H, Sq, Sk, device='cuda').to(BF)
+    seed, off = (torch.tensor([x], device='cuda', dtype=torch.uint64) for x in (7, 8))
+    null, sm, out = torch.empty([0], device='cuda', dtype=torch.uint64), 1 / math.sqrt(D), []
+    o, L = torch.empty_like(q), torch.empty(B * H, Sq, device='cuda')
+    assert flash.attn_fwd(q, k, v, b, sm, L, o, 0.2, seed, off, 0, null, null, None, causal, null) == flash.hipError_t.hipSuccess
+    lib.fa_set_bwd_workspace_limit(-1 if stored else 0)
+    try:
+        for x in (b, b.transpose(2, 3).contiguous().transpose(2, 3)):
+            grads = [torch.empty_like(t) for t in (q, k, v)]
+            params = flash.fa_backward_op_params()
+            flash._fill_bwd(params, q, k, v, None, sm, o, do, *grads, None, flash.lazy_dq_acc(q), L, flash.lazy_delta(L), 0.2,
+                            seed, off, 0, causal)
+            params.B = T4(x.data_ptr(), tuple(x.size()), x.stride(), flash.cast_dtype(BF))
+            params.varlen_type = 0
+            assert flash.fa_backward_op(params, params.kVersion, flash._stream(), None) == flash.hipError_t.hipSuccess
+            out.append(grads)
+    finally:
+        lib.fa_set_bwd_workspace_limit(-1)
+    for x, y in zip(*out):
+        assert torch.isfinite(x).all() and torch.equal(x, y)
