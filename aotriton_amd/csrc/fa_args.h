@@ -137,7 +137,6 @@ struct FwdArgs {
   void* out; float* lse;
   Strides3 sq, sk, sv, so;
   int64_t sb_z, sb_h, sb_m, sb_n;
-  int32_t key_mask;      // the bias is one byte per key, the same for all rows (sb_m = 0): 0 hides the key
   int32_t batch, hq, hk;
   int32_t head_dim;      // columns of Q and K (<= the compiled head dim; a multiple of 8 unless `elementwise`)
   int32_t head_dim_v;    // columns of V, Out and dOut (same bounds)
@@ -163,6 +162,7 @@ struct FwdArgs {
   int32_t part_group, part_block;
   float* part_o;         // columns: the compiled head dim
   float* part_ml;        // reference maximum (units of the scores) and row sum
+  int32_t key_mask;      // the bias is one byte per key, the same for all rows (sb_m = 0): 0 hides the key
 };
 
 struct BwdArgs {
