@@ -142,11 +142,12 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
                    (int64_t)hk * a.sk.h + (int64_t)si.k_start * a.sk.s;
   const T* vbase = reinterpret_cast<const T*>(a.v) + (int64_t)si.batch_index * a.sv.z +
                    (int64_t)hk * a.sv.h + (int64_t)si.k_start * a.sv.s;
-  // This lane's bias row, for the layouts that are read without the wave's area.  In the windowed 256-row tiles of aligned rows,
-  // which take them only at an item's end, it is formed where it is read (causal, bias and dropout, us, held -> formed: D128 B4 H16
-  // S1024 bf16 86 -> 74, fp16 74 -> 72, D64 bf16 72 -> 59).  Not without dropout at 96 columns (2 % slower) and at D = 64 in bf16
-  // (window, S1024 29.5 -> 27.5, but S1000, whose last tile reads elements, 32 -> 36.5).
-  constexpr bool kHoldRow = kAnyRow || NW == 4 || !kWindowed || (!kDropout && (kPad == 96 || (D == 64 && __is_same(T, bf16_t))));
+  // This lane's bias row, for the layouts that are read without the wave's area.  The 256-row tiles of aligned rows, which take
+  // them only at an item's end, form it where it is read (us, held -> formed: causal with dropout, B4 H16 S1024, D128 bf16 86 -> 74,
+  // fp16 74 -> 72, D64 bf16 72 -> 59; neither, D64 fp16, B16 H12 S256 15.4 -> 13.9, B16 H16 S512 43.5 -> 42.2).  Held: without a window
+  // at D = 128 (bf16 with dropout 8 % slower formed), without dropout at 96 columns (2 %) and at D = 64 in bf16 (B16 H16 S512 38.4 ->
+  // 40.1; window, S1024 29.5 -> 27.5, but S1000, whose last tile reads elements, 32 -> 36.5).
+  constexpr bool kHoldRow = kAnyRow || NW == 4 || (D == 64 ? !kDropout && __is_same(T, bf16_t) : !kWindowed || (kPad == 96 && !kDropout));
   const T* bptr = nullptr;
   if (kBias && kHoldRow)
     bptr = reinterpret_cast<const T*>(a.bias) + (int64_t)si.batch_index * a.sb_z + (int64_t)h * a.sb_h +
