@@ -373,8 +373,7 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
       auto piece = [&](int i) {
         // The row inside the wave, as a 32-bit offset from a scalar base (rows are at most 2^21 elements apart); rows past the
         // sequence repeat the last one.  (As a 64-bit pointer per row the offsets were spilled, and their reloads waited for the
-        // tile's K and V.  Window, bias and dropout, us, B2 H16 S4096 D128 282 -> 259, B1 H16 S3000 187 -> 157, B2 H16 S2048 D64
-        // 67.7 -> 63.)
+        // tile's K and V.  Window, bias and dropout, us, B1 H16 S3001 D64 93 -> 88, B2 H8 S1801 D128 75.8 -> 73.5.)
         const int m = brow + BRPI * i < wrows - 1 ? brow + BRPI * i : (wrows > 0 ? wrows - 1 : 0);
         if constexpr (kEnd) {
           return load_row_piece<T, true>(reinterpret_cast<const T*>(bias_tile + (uint32_t)(m * b_row)), j * BN + ck * BCK + bch * 8, si.seqlen_k);
