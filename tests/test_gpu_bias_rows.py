@@ -101,3 +101,29 @@ def test_rows_far_apart(step, p):
     assert (out[0][1] - out[1][1]).abs().max().item() < 1e-5 * (1 + out[0][1].abs().max().item())
     d = (out[0][0].double() - out[1][0].double()).norm() / out[0][0].double().norm()
     assert d.item() < 2 * torch.finfo(dt).eps
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('p', [0.0, 0.2])
+@pytest.mark.parametrize('D,dt,causal', [(64, HF, True), (64, BF, False), (96, BF, True), (128, BF, True), (128, HF, (90, 20))])
+def test_rows_that_overlap(D, dt, causal, p):
+    """Rows that start 16 bytes apart in one vector of memory (a bias by distance), the last of them ending where the memory does, and
+    the same rows apart: the same bits."""
+    from aotriton_amd import flash
+    B, H, Sq, Sk = 4, 16, 291, 384
+    assert fwd(B, H, H, Sq, Sk, D, causal, 0.2, True).block_m == 256
+    g = torch.Generator(device='cuda').manual_seed(6)
+    rn = lambda *s: torch.randn(*s, device='cuda', generator=g).to(dt)
+    q, k, v = rn(B, H, Sq, D), rn(B, H, Sk, D), rn(B, H, Sk, D)
+    n = 8 * (Sq - 1) + Sk
+    memory = torch.full((H * n + 64,), float('nan'), device='cuda', dtype=dt)
+    memory[:H * n] = rn(H * n)
+    near = memory.as_strided((B, H, Sq, Sk), (0, n, 8, 1))
+    seed, off = (torch.tensor([x], device='cuda', dtype=torch.uint64) for x in (3, 4))
+    null, out = torch.empty([0], device='cuda', dtype=torch.uint64), []
+    for b in (near, near.contiguous()):
+        o, L = torch.empty_like(q), torch.empty(B * H, Sq, device='cuda')
+        assert flash.attn_fwd(q, k, v, b, D ** -0.5, L, o, p, seed, off, 0, null, null, None, causal, null) == flash.hipError_t.hipSuccess
+        out.append((o, L))
+    assert torch.isfinite(out[0][0]).all()
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
