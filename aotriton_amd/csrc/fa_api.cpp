@@ -1147,11 +1147,15 @@ int fa_query_bwd_config(const fa_bwd_params* params, const fa_options* options, 
     fit_workspace(room, &need, &parts);
   }
   const bool wide_dkdv = route.wide_dkdv && need == 0 && parts.bytes == 0;
+  const bool pair_dkdv = s.d == 256 && need > 0 &&
+                         (!s.bias || (s.max_sk % 8 == 0 && fa::bias_aligned(params->B.ptr, params->B.strides[0], params->B.strides[1],
+                                                                            params->B.strides[2], params->B.strides[3])));
   const fa::TileShape t = rows32 ? fa::f32_rows_tile_shape(s.d)
                           : f32_mfma ? fa::f32_tile_shape(s.d, kernel_slot)
                           : split_d ? fa::d512_tile_shape(kernel_slot)
                           : valu  ? (kernel_slot == 1 ? fa::TileShape{1, 32, 4, 0} : fa::TileShape{32, 1, 4, 0})
                           : kernel_slot == 1 && wide_dkdv ? fa::bwd_wide_shape(true)
+                          : kernel_slot == 1 && pair_dkdv ? fa::bwd_pair_shape(s.bias)
                           : kernel_slot == 2 && route.wide_dq ? fa::bwd_wide_shape(false)
                                   : fa::bwd_tile_shape(params->Q.dtype, s.d, s.windowed, s.bias, s.dropout, kernel_slot, need > 0);
   const int nz = s.num_seqlens != 0 ? std::abs(s.num_seqlens) : s.batch;
@@ -1578,6 +1582,8 @@ static int attn_bwd_impl(const fa_bwd_params* p_in, int32_t params_version, void
         a.walk_group = route.group_dkdv;
         return fa::run_bwd_dkdv_wide(dt, a, s.windowed, stream);
       }
+      if (a.ds_ws != nullptr && s.d == 256 && (!s.bias || fa::plain_bias(a)))
+        return fa::run_bwd_dkdv_pair(dt, a, s.windowed, s.bias, s.dropout, stream);
       return (cut ? fa::run_bwd_dkdv_parts : fa::run_bwd_dkdv)(dt, s.d, a, s.windowed, s.bias, s.dropout, stream);
     };
     if (ds_slot >= 0 && ds_ws == nullptr) {

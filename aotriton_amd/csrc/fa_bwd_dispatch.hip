@@ -32,6 +32,13 @@ FA_DECL(run_bwd_dq, cols96)
 FA_DECL(run_bwd_fused, padded)
 #undef FA_DECL
 
+hipError_t run_bwd_dkdv_pair_d256(int, const BwdArgs&, bool, bool, bool, hipStream_t);
+hipError_t run_bwd_dkdv_pair_d256_padded(int, const BwdArgs&, bool, bool, bool, hipStream_t);
+hipError_t run_bwd_dkdv_pair(int dtype, const BwdArgs& a, bool w, bool b, bool p, hipStream_t s) {
+  const bool padded = a.head_dim != 256 || a.head_dim_v != 256;
+  return (padded ? run_bwd_dkdv_pair_d256_padded : run_bwd_dkdv_pair_d256)(dtype, a, w, b, p, s);
+}
+
 #define FA_DECL_WIDE(name)                                                                    \
   hipError_t name##_d128(int, const BwdArgs&, bool, hipStream_t);                             \
   hipError_t name##_d128_padded(int, const BwdArgs&, bool, hipStream_t);                      \

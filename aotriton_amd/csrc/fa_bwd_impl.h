@@ -149,16 +149,19 @@ template <typename T, int D> struct DsTile {
 
 // The keep bits that dropout_keep4 gives, appended to `bits` with the first uppermost: two instructions each and no condition (the
 // sign of a saturated difference, shifted in; as a condition each is three and a wait of two states for the condition).
+__device__ __forceinline__ uint32_t dropout_append(const Philox& p, int32_t thr, uint32_t bits) {
+  const uint32_t w[4] = {p.c0, p.c2, p.c1, p.c3};      // (the word order of a row)
+#pragma unroll
+  for (int r = 0; r < 4; ++r) bits = __builtin_amdgcn_alignbit(bits, (uint32_t)__builtin_elementwise_sub_sat(thr, (int32_t)w[r]), 31);
+  return bits;
+}
 __device__ __forceinline__ uint32_t dropout_append4(const DropoutState& s, int m, int n0, uint32_t bits) {
   const uint64_t ctr = s.base + (uint64_t)m * s.stride + (uint64_t)(n0 >> 2);
-  uint32_t w[4];
-  philox4x32_10((uint32_t)ctr, (uint32_t)(ctr >> 32), s.k0, s.k1, w);
+  Philox p;
+  p.start((uint32_t)ctr, (uint32_t)(ctr >> 32));
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int i = r == 1 ? 2 : r == 2 ? 1 : r;      // (the word order of a row)
-    bits = __builtin_amdgcn_alignbit(bits, (uint32_t)__builtin_elementwise_sub_sat(s.thr, (int32_t)w[i]), 31);
-  }
-  return bits;
+  for (int i = 0; i < 10; ++i) p.round(i, s.k0, s.k1);
+  return dropout_append(p, s.thr, bits);
 }
 
 // ---------------------------------------------------------------------------
@@ -1590,10 +1593,12 @@ static __global__ __launch_bounds__(256) void combine_dkdv_kernel(const BwdArgs 
   *reinterpret_cast<q4_t*>(out) = t4;
 }
 
-// Every row of the bias is whole 16-byte pieces at 16-byte boundaries, in every item.
-template <typename T> inline bool plain_bias(const BwdArgs& a) {
-  return a.seq.num_seqlens == 0 && a.seq.max_seqlen_k % 8 == 0 && a.sb_n == 1 && ((a.sb_m | a.sb_h | a.sb_z) & 7) == 0 &&
-         (reinterpret_cast<uintptr_t>(a.bias) & 15) == 0;
+template <typename T, int D>
+hipError_t launch_combine_dkdv(const BwdArgs& a, hipStream_t stream) {
+  const int64_t threads = (int64_t)a.num_zh * a.num_n_tiles * 2 * 128 * (D / 4);
+  if (threads == 0) return hipSuccess;
+  hipLaunchKernelGGL((combine_dkdv_kernel<T, D>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, a);
+  return hipGetLastError();
 }
 
 template <typename T, int D, int kPad, bool W, bool B, bool P, bool kParts, bool kStoreDs, int kForm>
@@ -1607,11 +1612,7 @@ hipError_t launch_dkdv_form(const BwdArgs& a0, hipStream_t stream) {
   constexpr int smem = DkDvSmem<D, BM>::BYTES + (D < 256 ? kLevelBytes : 0);
   hipError_t e = launch_with_lds<bwd_dkdv_kernel<T, D, NW, BM, W, B, P, kPad, kStoreDs, kParts, kForm>>(grid, NW * 64, smem, stream, a);
   if constexpr (kParts) {
-    const int64_t threads = (int64_t)a.num_zh * a.num_n_tiles * 2 * BN * (D / 4);
-    if (e == hipSuccess && threads > 0) {
-      hipLaunchKernelGGL((combine_dkdv_kernel<T, D>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, a);
-      e = hipGetLastError();
-    }
+    if (e == hipSuccess) e = launch_combine_dkdv<T, D>(a, stream);
   }
   return e;
 }
@@ -1629,12 +1630,17 @@ hipError_t launch_dkdv_variant(const BwdArgs& a, hipStream_t stream) {
       if (rows) return launch_dkdv_form<T, D, kPad, W, B, P, kParts, false, kBiasRows>(a, stream);
     return launch_dkdv_form<T, D, kPad, W, B, P, kParts, false, kBiasAny>(a, stream);
   }
-  constexpr bool kForms = B && (!kParts || kTwoDkDv<D, B, P, true, kBiasPlain>);
-  if constexpr (kForms)
-    if (plain_bias<T>(a)) return launch_dkdv_form<T, D, kPad, W, B, P, kParts, true, kBiasPlain>(a, stream);
-  if constexpr (kForms || kRows256)
-    if (rows) return launch_dkdv_form<T, D, kPad, W, B, P, kParts, true, kBiasRows>(a, stream);
-  return launch_dkdv_form<T, D, kPad, W, B, P, kParts, true, kBiasAny>(a, stream);
+  // (head dims above 128 that store dS, without a bias or with a plain one: fa_bwd_pair.h)
+  if constexpr (D == 256 && !B) {
+    return hipErrorNotSupported;
+  } else {
+    constexpr bool kForms = B && (!kParts || kTwoDkDv<D, B, P, true, kBiasPlain>);
+    if constexpr (kForms && D < 256)
+      if (plain_bias(a)) return launch_dkdv_form<T, D, kPad, W, B, P, kParts, true, kBiasPlain>(a, stream);
+    if constexpr (kForms || kRows256)
+      if (rows) return launch_dkdv_form<T, D, kPad, W, B, P, kParts, true, kBiasRows>(a, stream);
+    return launch_dkdv_form<T, D, kPad, W, B, P, kParts, true, kBiasAny>(a, stream);
+  }
 }
 
 template <typename T, int D, int kPad, bool kParts>

@@ -53,6 +53,14 @@ hipError_t run_bwd_preprocess(int dtype, int head_dim, const BwdArgs& a, hipStre
 hipError_t run_bwd_dkdv(int dtype, int head_dim, const BwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
 // the same with the items cut into parts and a kernel behind it that adds the parts up (BwdArgs::part_ws)
 hipError_t run_bwd_dkdv_parts(int dtype, int head_dim, const BwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
+// Every row of the bias is whole 16-byte pieces at 16-byte boundaries, in every item.
+inline bool plain_bias(const BwdArgs& a) {
+  return a.seq.num_seqlens == 0 && a.seq.max_seqlen_k % 8 == 0 && bias_aligned(a.bias, a.sb_z, a.sb_h, a.sb_m, a.sb_n);
+}
+// The same for items that store dS at head dims above 128, whole or in parts, without a bias or with a plain one: pairs of waves
+// (fa_bwd_pair.h).
+hipError_t run_bwd_dkdv_pair(int dtype, const BwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
+TileShape bwd_pair_shape(bool bias);
 hipError_t run_bwd_dq(int dtype, int head_dim, const BwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
 // head dims above 64 and up to 128 without bias and dropout: 64 rows per wave (fa_bwd_wide.h)
 hipError_t run_bwd_dkdv_wide(int dtype, const BwdArgs& a, bool windowed, hipStream_t s);

@@ -1,6 +1,7 @@
 // Compile-time tile/occupancy table keyed on (element type, head dim, causal / windowed) and, where a kernel's
 // variants differ, on the options; reported through fa_query_*_config.
 #include "fa_fwd_impl.h"
+#include "fa_bwd_pair.h"
 #include "fa_bwd_wide.h"
 #include "fa_fwd_wide.h"
 #include "fa_kernels.h"
@@ -51,6 +52,8 @@ TileShape bwd_tile_shape(int dtype, int head_dim, bool windowed, bool bias, bool
 }
 
 TileShape fwd_wide_shape() { return TileShape{256, 64, 4, WideFwdSmem::BYTES + kLevelBytes, 1}; }
+
+TileShape bwd_pair_shape(bool bias) { return TileShape{32, 128, 8, bias ? PairSmem<true>::BYTES : PairSmem<false>::BYTES, 1}; }
 
 TileShape bwd_wide_shape(bool dkdv) {
   return dkdv ? TileShape{kWideBM, kWideBN, 4, WideDkDvSmem::BYTES + kLevelBytes, 1} : TileShape{kWideBN, kWideBM, 4, WideDqSmem::BYTES + kLevelBytes, 1};
