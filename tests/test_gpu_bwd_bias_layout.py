@@ -197,3 +197,16 @@ def test_columns_of_a_bias_apart_with_dropout(D, stored):
         lib.fa_set_bwd_workspace_limit(-1)
     for x, y in zip(*out):
         assert torch.isfinite(x).all() and torch.equal(x, y)
+
+
+@pytest.mark.parametrize('D', [64, 128, 256])
+@pytest.mark.parametrize('Sk', [136, 131])
+def test_rows_that_a_bias_hides(D, Sk):
+    """a finite bias that hides all keys of every other row: what stands for keys past the sequence must not reach dQ"""
+    from aotriton_amd.autograd import attention
+    q, k, v, b, do = make_inputs(4, 16, 16, 512, Sk, D, BF, 'cuda', seed=4, bias=True)
+    b = b.contiguous()
+    b[:, :, ::2] = -30000
+    x = [t.clone().requires_grad_() for t in (q, k, v)]
+    attention(*x, b, False, 1 / math.sqrt(D), 0.0)[0].backward(do)
+    assert all(torch.isfinite(t.grad).all() for t in x)
