@@ -46,13 +46,13 @@ EXTRA = {
     'fa_fwd_wide_d128.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form', '-Wno-inline-asm'],
     'fa_bwd_wide_d128.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form', '-Wno-inline-asm'],
     'fa_bwd_pair_d256.hip': ['-Wno-inline-asm'],
-    'fa_fwd_drop_d256.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'],
+    'fa_fwd_d256.hip': ['-Wno-inline-asm'],
     'fa_bwd_dq_d128.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'],
 }
 
 # The per-head-dim kernel files are compiled a second time with FA_PADDED = the head dim: the copies that
 # serve head dims rounded up to the compiled one.
-PADDED_RE = re.compile(r'fa_(fwd|fwd_drop|fwd_rows|fwd_wide|bwd_dkdv|bwd_dkdv_parts|bwd_dq|bwd_dq_bias|bwd_wide|bwd_pair|bwd_fused)_d(\d+)\.hip$')
+PADDED_RE = re.compile(r'fa_(fwd|fwd_rows|fwd_wide|bwd_dkdv|bwd_dkdv_parts|bwd_dq|bwd_dq_bias|bwd_wide|bwd_pair|bwd_fused)_d(\d+)\.hip$')
 # ... and these a third time with 96 columns, for head dims above 64 and up to 96
 COLS96_RE = re.compile(r'fa_(fwd|fwd_wide|bwd_dkdv|bwd_dq|bwd_wide)_d128\.hip$')
 

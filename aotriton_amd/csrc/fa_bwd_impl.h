@@ -147,14 +147,6 @@ template <typename T, int D> struct DsTile {
   static constexpr int piece(int kw, int t) { return (t >> 1) * QBLOCK_BYTES + kw * 2048 + (t & 1) * 1024; }
 };
 
-// The keep bits that dropout_keep4 gives, appended to `bits` with the first uppermost: two instructions each and no condition (the
-// sign of a saturated difference, shifted in; as a condition each is three and a wait of two states for the condition).
-__device__ __forceinline__ uint32_t dropout_append(const Philox& p, int32_t thr, uint32_t bits) {
-  const uint32_t w[4] = {p.c0, p.c2, p.c1, p.c3};      // (the word order of a row)
-#pragma unroll
-  for (int r = 0; r < 4; ++r) bits = __builtin_amdgcn_alignbit(bits, (uint32_t)__builtin_elementwise_sub_sat(thr, (int32_t)w[r]), 31);
-  return bits;
-}
 __device__ __forceinline__ uint32_t dropout_append4(const DropoutState& s, int m, int n0, uint32_t bits) {
   const uint64_t ctr = s.base + (uint64_t)m * s.stride + (uint64_t)(n0 >> 2);
   Philox p;

@@ -56,9 +56,6 @@ __device__ __forceinline__ int lane_here() {
   asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(x));
   return x;
 }
-template <typename V> __device__ __forceinline__ void lds_write(int at, V x) {
-  *reinterpret_cast<__attribute__((address_space(3))) V*>(at) = x;
-}
 
 template <typename T, bool kWindowed, bool kBias, bool kDropout, int kPad>
 __device__ __forceinline__ void dkdv_pair_item(const BwdArgs& a, const int hk, const int nt, const int z, const int part,

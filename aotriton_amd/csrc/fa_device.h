@@ -333,6 +333,15 @@ __device__ __forceinline__ uint32_t dropout_keep4(const DropoutState& s, int m, 
          ((int32_t)w[1] > s.thr ? 4u : 0u) | ((int32_t)w[3] > s.thr ? 8u : 0u);
 }
 
+// The keep bits that dropout_keep4 gives, appended to `bits` with the first uppermost: two instructions each and no condition (the
+// sign of a saturated difference, shifted in; as a condition each is three and a wait of two states for the condition).
+__device__ __forceinline__ uint32_t dropout_append(const Philox& p, int32_t thr, uint32_t bits) {
+  const uint32_t w[4] = {p.c0, p.c2, p.c1, p.c3};      // (the word order of a row)
+#pragma unroll
+  for (int r = 0; r < 4; ++r) bits = __builtin_amdgcn_alignbit(bits, (uint32_t)__builtin_elementwise_sub_sat(thr, (int32_t)w[r]), 31);
+  return bits;
+}
+
 // Keep bit of a single element.
 __device__ __forceinline__ bool dropout_keep1(const DropoutState& s, int m, int n) {
   return (dropout_keep4(s, m, n & ~3) >> (n & 3)) & 1u;

@@ -14,15 +14,6 @@
 #endif
 
 namespace fa {
-// (the kernels with dropout: fa_fwd_drop_d256.hip)
-#define FA_DROPOUT(T)                                                                                               \
-  extern template hipError_t launch_fwd_variant<T, 256, false, false, true, FA_PADDED>(const FwdArgs&, dim3, hipStream_t); \
-  extern template hipError_t launch_fwd_variant<T, 256, false, true, true, FA_PADDED>(const FwdArgs&, dim3, hipStream_t);  \
-  extern template hipError_t launch_fwd_variant<T, 256, true, false, true, FA_PADDED>(const FwdArgs&, dim3, hipStream_t);  \
-  extern template hipError_t launch_fwd_variant<T, 256, true, true, true, FA_PADDED>(const FwdArgs&, dim3, hipStream_t);
-FA_DROPOUT(f16_t)
-FA_DROPOUT(bf16_t)
-
 hipError_t FA_RUN(int dtype, const FwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s) {
   if (dtype == kDtypeBF16) return launch_fwd<bf16_t, 256, FA_PADDED>(a, windowed, bias, dropout, s);
   return launch_fwd<f16_t, 256, FA_PADDED>(a, windowed, bias, dropout, s);

@@ -21,7 +21,7 @@
 
 #include "fa_combine.h"
 #include "fa_device.h"
-#include "fa_fwd_pipe.h"
+#include "fa_fwd_pair.h"
 
 namespace fa {
 
@@ -64,12 +64,7 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
   T* Vs = Ks + SM::STAGES * SM::K_ELEMS;
 
   const int tid = threadIdx.x;
-  // At D = 256 (one wave per SIMD, accumulators in AGPRs) the wave index is taken as a scalar:
-  // the branches on it are then uniform for the compiler too, and it keeps the copies of the 128
-  // accumulator registers that the rarely taken full softmax step needs out of the common path
-  // (they doubled the vector instructions per tile of the causal kernel: 737 -> 895 TFLOP/s at
-  // S = 16384).  At D <= 128 there are no AGPRs and the plain form measures 0-4 % faster.
-  const int wave = D >= 256 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
+  const int wave = tid >> 6;
   const int lane = tid & 63, c = lane & 31, hi = lane >> 5;
   // columns of Q/K and of V/Out: <= D, multiples of 8; constants unless a head dim is rounded up
   const int d_qk = kPad ? a.head_dim : D, d_v = kPad ? a.head_dim_v : D;
@@ -727,13 +722,12 @@ __device__ __forceinline__ void fwd_item(const FwdArgs& a, const int z, const in
 // interleaved, and the workgroups of the XCD take them in serpentine order (worker p
 // takes p, 2P-1-p, 2P+p, ...), which pairs heavy with light tiles.  A workgroup
 // goes from one tile to the next without a relaunch.
-// QB = 0: fwd_item, NW waves of 32 rows, two waves per SIMD or (FwdThirdTile) three.  QB > 0: fwd_item_pipe, 4 waves of 32 * QB rows, one wave
-// per SIMD.
-template <int D, int NW, int BN, int QB> constexpr int kFwdWaves = D > 128 || QB > 0 ? 1 : D == 64 && NW == 4 && BN == 32 ? 3 : 2;
-template <typename T, int D, int NW, int BN, int QB, bool kWindowed, bool kBias, bool kDropout, int kPad, bool kSplit,
+// fwd_item with NW waves of 32 rows, two waves per SIMD or (FwdThirdTile) three; or, kPairs, fwd_item_pair with two waves for 32 rows.
+template <int D, int NW, int BN> constexpr int kFwdWaves = D == 64 && NW == 4 && BN == 32 ? 3 : 2;
+template <typename T, int D, int NW, int BN, bool kPairs, bool kWindowed, bool kBias, bool kDropout, int kPad, bool kSplit,
           bool kKeyBias, bool kAnyRow = false>
 __global__ __attribute__((amdgpu_flat_work_group_size(NW * 64, NW * 64)))
-__attribute__((amdgpu_waves_per_eu(kFwdWaves<D, NW, BN, QB>, kFwdWaves<D, NW, BN, QB>)))
+__attribute__((amdgpu_waves_per_eu(kFwdWaves<D, NW, BN>, kFwdWaves<D, NW, BN>)))
 void fwd_kernel(const FwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   if (kDropout && blockIdx.x == 0 && threadIdx.x == 0) {
@@ -756,9 +750,9 @@ void fwd_kernel(const FwdArgs a) {
   const bool ragged = a.seq.num_seqlens != 0;
   const int ratio = a.hq / a.hk, nseq = a.num_zh / a.hq;
   const bool levels = ragged && a.zh_per_xcd <= kLevelCap && a.num_m_tiles <= 0xffff;
-  constexpr bool kTwo = NW == 4 && QB == 0;      // (FwdHalfTile)
-  constexpr int kRows = NW * 32 * (QB > 0 ? QB : 1);
-  constexpr int kSmem = QB > 0 ? FwdPipeSmem<D, BN, (QB > 0 ? QB : 1)>::BYTES : FwdSmem<D, BN, NW>::BYTES;
+  constexpr bool kTwo = NW == 4;      // (FwdHalfTile)
+  constexpr int kRows = kPairs ? NW * 16 : NW * 32;
+  constexpr int kSmem = kPairs ? FwdPairSmem::BYTES : FwdSmem<D, BN, NW>::BYTES;
   const int zh_lo = xcd * a.zh_per_xcd;
   RaggedWalk walk;
   LevelWalk lwalk;
@@ -791,7 +785,7 @@ void fwd_kernel(const FwdArgs a) {
       mt = a.num_m_tiles - 1 - gr / a.zh_group;
       split_zh(zh, nseq, ratio, z, h);
     }
-    if constexpr (QB > 0) fwd_item_pipe<T, D, QB, BN, kWindowed, kBias, kDropout, kPad>(a, z, h, mt, smem_raw);
+    if constexpr (kPairs) fwd_item_pair<T, kWindowed, kBias, kDropout, kPad>(a, z, h, mt, smem_raw);
     else fwd_item<T, D, NW, BN, kWindowed, kBias, kDropout, kPad, kSplit, kKeyBias, kAnyRow>(a, z, h, mt, split, smem_raw);
   }
 }
@@ -802,42 +796,37 @@ void fwd_kernel(const FwdArgs a) {
 // differ between causal and non-causal).  Here the measured best tile is the same on both sides
 // of every key; the alternatives that lost are noted per entry (same-box A/B, bf16, B*H*D = 16384,
 // S = 4096 and 16384).
-template <int D_, int NW_, int BN_, int QB_> struct FwdTileOf {
-  static constexpr int NW = NW_, BN = BN_, QB = QB_;
-  static constexpr int BM = NW * 32 * (QB > 0 ? QB : 1);
+template <int D_, int NW_, int BN_, bool kPairs_ = false> struct FwdTileOf {
+  static constexpr int NW = NW_, BN = BN_;
+  static constexpr bool kPairs = kPairs_;
+  static constexpr int BM = kPairs ? NW * 16 : NW * 32;
   // (the level table of packed sequences sits behind the item's LDS)
-  static constexpr int ITEM_LDS = QB > 0 ? FwdPipeSmem<D_, BN, (QB > 0 ? QB : 1)>::BYTES : FwdSmem<D_, BN, NW>::BYTES;
+  static constexpr int ITEM_LDS = kPairs ? FwdPairSmem::BYTES : FwdSmem<D_, BN, NW>::BYTES;
   static constexpr int LDS = ITEM_LDS + kLevelBytes;
 };
 template <typename T, int D, bool kWindowed> struct FwdTile;
 // D = 64: 128-key tiles; 64-key tiles lose 2 % causal and 6 % non-causal at S = 4096.
-template <typename T, bool kWindowed> struct FwdTile<T, 64, kWindowed> : FwdTileOf<64, 8, 128, 0> {};
+template <typename T, bool kWindowed> struct FwdTile<T, 64, kWindowed> : FwdTileOf<64, 8, 128> {};
 // D = 128: 64-key tiles; 32-key tiles (finer skipping on the causal diagonal, twice the barriers)
 // lose 6-7 % causal and 5 % non-causal.  128-key tiles do not fit the LDS next to the row areas.
-template <typename T, bool kWindowed> struct FwdTile<T, 128, kWindowed> : FwdTileOf<128, 8, 64, 0> {};
-// (The pipelined item with 64 rows per wave, FwdTileOf<128, 4, 64, 2>, halves the LDS operand traffic
-// per MFMA but measures 20 % slower than this one at S = 4096 and 16384: one wave per SIMD issues
-// its MFMAs, vector and LDS instructions one after the other, and two waves overlap better.)
-// D = 256: one wave per SIMD (the accumulators of 32 rows take 128 registers), 32-key tiles, the
-// software-pipelined item: level with fwd_item without bias and dropout (B2 H16 S8192 fp16: 903 vs
-// 875 TFLOP/s non-causal, 827 vs 835 causal), 15-25 % faster with them (bias: 644 vs 553, causal
-// 629 vs 510; bias + dropout + window 1024: 361 vs 333).
-template <typename T, bool kWindowed> struct FwdTile<T, 256, kWindowed> : FwdTileOf<256, 4, 32, 1> {};
+template <typename T, bool kWindowed> struct FwdTile<T, 128, kWindowed> : FwdTileOf<128, 8, 64> {};
+// D = 256: 128 rows on eight waves, two for 32 rows (fa_fwd_pair.h, with what it was measured against).
+template <typename T, bool kWindowed> struct FwdTile<T, 256, kWindowed> : FwdTileOf<256, 8, 32, true> {};
 
 // Half the rows, two workgroups per CU (FwdArgs::half_tiles; dense calls at D <= 128, without a bias or with one of the keys).  A sequence
 // is cut finer, so that less of the last tile and of the last round is empty; per row it is 5-15 % slower (K and V
 // are staged once per 128 rows, narrower key tiles).  fwd_small_tiles in fa_api.cpp decides.
-template <int D> struct FwdHalfTile : FwdTileOf<D, 4, D == 64 ? 64 : 32, 0> {};
+template <int D> struct FwdHalfTile : FwdTileOf<D, 4, D == 64 ? 64 : 32> {};
 // Three of them per CU, on 32-key tiles: 150 registers per wave and 40 KB of LDS.  A barrier every 32 keys makes a full CU 5-10 %
 // slower than with two, but an XCD takes 96 tiles at once instead of 64 (B16 H12 S384 22.2 -> 18.6 us, B16 H32 S325 causal
 // 32.9 -> 28.6, B4 H12 S1544 causal 46.8 -> 41.5).
-struct FwdThirdTile : FwdTileOf<64, 4, 32, 0> {};
+struct FwdThirdTile : FwdTileOf<64, 4, 32> {};
 
 template <typename T, int D, bool kWindowed, bool kBias, bool kDropout, int kPad, bool kSplit = false,
           bool kKeyBias = false, typename Tile = FwdTile<T, D, kWindowed>, bool kAnyRow = false>
 hipError_t launch_fwd_variant(const FwdArgs& a, dim3 grid, hipStream_t stream) {
   constexpr int NW = Tile::NW;
-  auto kern = fwd_kernel<T, D, NW, Tile::BN, Tile::QB, kWindowed, kBias, kDropout, kPad, kSplit, kKeyBias, kAnyRow>;
+  auto kern = fwd_kernel<T, D, NW, Tile::BN, Tile::kPairs, kWindowed, kBias, kDropout, kPad, kSplit, kKeyBias, kAnyRow>;
   constexpr int smem = Tile::LDS;
   if (grid.x == 0) return hipSuccess;      // no batch, no head or no query row: nothing to write
   if (smem > 64 * 1024) {
@@ -915,7 +904,7 @@ hipError_t launch_fwd(const FwdArgs& a, bool windowed, bool bias, bool dropout, 
   const int key = (windowed ? 4 : 0) | (bias ? 2 : 0) | (dropout ? 1 : 0);
   if constexpr (D <= 128) {
     using Whole = FwdTile<T, D, true>;
-    static_assert(std::is_base_of_v<FwdTileOf<D, Whole::NW, Whole::BN, 0>, FwdTile<T, D, false>>, "one tile with and without a mask");
+    static_assert(std::is_base_of_v<FwdTileOf<D, Whole::NW, Whole::BN>, FwdTile<T, D, false>>, "one tile with and without a mask");
     switch (bias && a.sb_n == 1 && !bias_aligned(a.bias, a.sb_z, a.sb_h, a.sb_m, a.sb_n) ? key : 0) {
       case 2: return launch_fwd_variant<T, D, false, true, false, kPad, false, false, Whole, true>(b, grid, stream);
       case 3: return launch_fwd_variant<T, D, false, true, true, kPad, false, false, Whole, true>(b, grid, stream);

@@ -1,4 +1,4 @@
-// What the kernels with 64 rows per wave share (fa_bwd_wide.h, fa_fwd_wide.h).
+// What the kernels with 64 rows per wave (fa_bwd_wide.h, fa_fwd_wide.h) and those of pairs of waves (fa_bwd_pair.h, fa_fwd_pair.h) share.
 #pragma once
 #include <type_traits>
 
@@ -32,6 +32,28 @@ template <int N> __device__ __forceinline__ void acc_settle(f32x16 (&x)[N], f32x
     asm volatile("s_nop 15\n\ts_nop 15" : "+a"(x[0]), "+a"(x[1]), "+a"(x[2]), "+a"(y[0]), "+a"(y[1]), "+a"(y[2]));
 }
 
+// The rescaling of an O^T accumulator tuple (a lane's 16 values times its row's factor) in place in
+// the accumulation registers: the tuple never shows up in VGPRs.  The waits cover the hazards that
+// nobody checks inside an asm block: an MFMA result read by the vector ALU (up to 19 wait states)
+// and a vector write read by an MFMA as its C operand.
+#define FA_ACC_OPS(m) m(0) m(1) m(2) m(3) m(4) m(5) m(6) m(7) m(8) m(9) m(10) m(11) m(12) m(13) m(14) m(15)
+#define FA_ACC_SCALE1(i) "v_accvgpr_read_b32 %16, %" #i "\n v_mul_f32 %16, %16, %17\n v_accvgpr_write_b32 %" #i ", %16\n"
+#define FA_ACC_SPLIT(t) \
+  float e0 = t[0], e1 = t[1], e2 = t[2], e3 = t[3], e4 = t[4], e5 = t[5], e6 = t[6], e7 = t[7], e8 = t[8], e9 = t[9], \
+        e10 = t[10], e11 = t[11], e12 = t[12], e13 = t[13], e14 = t[14], e15 = t[15]
+#define FA_ACC_JOIN(t) \
+  t[0] = e0; t[1] = e1; t[2] = e2; t[3] = e3; t[4] = e4; t[5] = e5; t[6] = e6; t[7] = e7; t[8] = e8; t[9] = e9; \
+  t[10] = e10; t[11] = e11; t[12] = e12; t[13] = e13; t[14] = e14; t[15] = e15
+__device__ __forceinline__ void acc_scale(f32x16& t, float f) {
+  float tmp;
+  FA_ACC_SPLIT(t);
+  asm volatile("s_nop 15\n s_nop 7\n" FA_ACC_OPS(FA_ACC_SCALE1) "s_nop 3\n"
+               : "+a"(e0), "+a"(e1), "+a"(e2), "+a"(e3), "+a"(e4), "+a"(e5), "+a"(e6), "+a"(e7), "+a"(e8), "+a"(e9),
+                 "+a"(e10), "+a"(e11), "+a"(e12), "+a"(e13), "+a"(e14), "+a"(e15), "=&v"(tmp)
+               : "v"(f));
+  FA_ACC_JOIN(t);
+}
+
 // Twice a wave's 1 KB of a tile straight into LDS (64 lanes x 16 bytes at voff + soff, to lds + 16 lane).  The compiler's builtin
 // does the same but makes the first transposing LDS read behind it wait for it; here the tile's one wait is placed by hand.
 // A scalar register that a vector instruction has written (v_readfirstlane, the v_readlane that brings a spilled one back) may be
@@ -58,6 +80,9 @@ __device__ __forceinline__ SeqInfo uniform(SeqInfo s) {
 }
 template <typename V> __device__ __forceinline__ V lds_read(int at) {
   return *reinterpret_cast<__attribute__((address_space(3))) const V*>(at);
+}
+template <typename V> __device__ __forceinline__ void lds_write(int at, V x) {
+  *reinterpret_cast<__attribute__((address_space(3))) V*>(at) = x;
 }
 __device__ __forceinline__ tr_raw_t lds_read_tr_at(int at) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<__attribute__((address_space(3))) tr_raw_t*>(at));

@@ -1,0 +1,86 @@
+"""Forward at head dims above 128 by pairs of waves (fa_fwd_pair.h), against the oracle where its steps and stages can go wrong: fewer units
+than stages, row blocks without rows or without visible keys, masked units at both ends, moved references, bias rows anywhere."""
+import math
+
+import pytest
+import torch
+
+from test_gpu_attention import _run_case
+from test_launch_queries import fwd
+from oracle import fa_ref
+from _util import FUDGE, check, make_inputs
+
+pytestmark = pytest.mark.gpu
+
+BF, HF = torch.bfloat16, torch.float16
+CASES = [
+    # B, Hq, Hk, Sq, Sk, D, Dv, dtype, causal, dropout, bias
+    (2, 2, 2, 17, 1, 256, 256, BF, False, 0.0, False),             # one key, three row blocks without rows
+    (2, 4, 2, 33, 32, 256, 256, HF, False, 0.3, True),             # one whole unit
+    (1, 4, 4, 128, 33, 256, 256, BF, False, 0.1, False),           # two units
+    (2, 2, 1, 129, 96, 256, 256, HF, False, 0.0, True),            # as many units as stages
+    (2, 2, 1, 160, 97, 256, 256, BF, False, 0.2, True),
+    (1, 4, 2, 300, 300, 256, 256, HF, True, 0.0, False),
+    (1, 4, 2, 257, 390, 256, 256, BF, True, 0.25, True),
+    (1, 2, 2, 390, 257, 256, 256, HF, (-140, 200), 0.0, True),     # rows that see nothing
+    (1, 2, 1, 515, 520, 256, 256, BF, (60, 90), 0.3, True),        # masked units on both sides, skipped ones on the left
+    (1, 2, 1, 515, 520, 256, 256, HF, (40, -8), 0.0, False),
+    (2, 4, 2, 260, 392, 136, 136, BF, True, 0.1, True),            # head dims rounded up
+    (1, 4, 2, 129, 200, 200, 248, HF, False, 0.0, False),
+    (1, 2, 2, 270, 264, 248, 160, BF, (40, 20), 0.2, True),
+]
+
+
+@pytest.mark.parametrize('case', CASES, ids=lambda c: '-'.join(str(x).replace('torch.', '') for x in c))
+def test_pairs_meet_the_oracle(case):
+    B, Hq, Hk, Sq, Sk, D, Dv, dtype, causal, p, bias = case
+    x = fwd(B, Hq, Hk, Sq, Sk, max(D, Dv), causal, p, bias)
+    assert (x.block_m, x.block_n, x.num_waves) == (128, 32, 8)
+    _run_case(B, Hq, Hk, Sq, Sk, D, dtype, causal, dropout_p=p, bias=bias, seed=23, Dv=Dv)
+
+
+def _forward(q, k, v, b, causal, sm):
+    from aotriton_amd import flash
+    o = torch.full((*q.shape[:-1], v.shape[-1]), float('nan'), device='cuda', dtype=q.dtype)
+    lse = torch.full((q.shape[0] * q.shape[1], q.shape[2]), float('nan'), device='cuda')
+    null = torch.empty(0, device='cuda', dtype=torch.int64)
+    err = flash.attn_fwd(q, k, v, b, sm, lse, o, 0.0, null, null, 0, null, null, None, causal, torch.zeros(1, device='cuda', dtype=torch.int32))
+    assert err == flash.hipError_t.hipSuccess
+    torch.cuda.synchronize()
+    return o, lse.view(q.shape[0], q.shape[1], -1)
+
+
+@pytest.mark.parametrize('dtype,causal,sm,bias', [(BF, False, 1 / 16, False), (HF, True, 1 / 16, True), (BF, False, -1 / 16, False), (HF, False, 1.0, False)])
+def test_references_that_move(dtype, causal, sm, bias):
+    """Scores that grow along the keys (every few units the exponentials leave their range and a unit is done in full), for some rows
+    only; a negative scale; scores past the range in which the scale is folded into the exponent."""
+    q, k, v, b, _ = make_inputs(1, 2, 2, 200, 700, 256, dtype, 'cuda', seed=5, bias=bias)
+    k *= (torch.arange(700, device='cuda') / 100)[None, None, :, None].to(dtype)
+    q[:, :, ::3] *= 0.05
+    o, lse = _forward(q, k, v, b if bias else torch.empty(0, 0, 0, 0, device='cuda', dtype=dtype), causal, sm)
+    from aotriton_amd import flash
+    ct, wl, wr = flash.translate_causal(causal)
+    f = lambda t: t.float()
+    ro, rl, _ = fa_ref.attn_fwd_ref(f(q), f(k), f(v), f(b) if bias else None, sm, ct, wl, wr, 0.0, None)
+    lo, _, _ = fa_ref.attn_fwd_ref(q, k, v, b if bias else None, sm, ct, wl, wr, 0.0, None)
+    check('out', o, ro, lo, FUDGE['out'])
+    # fp32 sums of 256 products, each term rounded to 2^-24 of it
+    assert ((lse - rl.view_as(lse)).abs() <= 1e-5 * (1 + rl.view_as(lse).abs()) + 2e-4).all()
+
+
+@pytest.mark.parametrize('kind', ['offset', 'odd rows', 'broadcast rows'])
+def test_bias_layouts_agree(kind):
+    """A bias gives the same bits wherever its rows lie."""
+    B, H, Sq, Sk = 1, 2, 190, 230
+    q, k, v, b, _ = make_inputs(B, H, H, Sq, Sk, 256, BF, 'cuda', seed=6, bias=True)
+    if kind == 'broadcast rows':
+        b = b[:, :, :1].expand(B, H, Sq, Sk)
+    want, wl = _forward(q, k, v, b.contiguous(), (100, 30), 1 / 16)
+    if kind == 'offset':
+        x = torch.empty(B * H * Sq * Sk + 1, device='cuda', dtype=BF)[1:].view(B, H, Sq, Sk).copy_(b)
+    elif kind == 'odd rows':
+        x = torch.empty(B, H, Sq, Sk + 3, device='cuda', dtype=BF)[..., :Sk].copy_(b)
+    else:
+        x = b
+    got, gl = _forward(q, k, v, x, (100, 30), 1 / 16)
+    assert torch.equal(got, want) and torch.equal(gl, wl)

@@ -1,7 +1,7 @@
 """The kernels test an element's visibility with one unsigned comparison: the visible keys of a
 query row (or the queries that see a key) form one range [lo, lo + rng], and `n` is inside iff
 uint32(n - lo) <= rng, with an empty range mapped to an offset no element reaches
-(fa_fwd_impl.h: prepare, fa_fwd_pipe.h: softmax_full).  This checks that form against the
+(fa_fwd_impl.h: prepare, fa_fwd_pair.h: softmax_full).  This checks that form against the
 element predicate of the reference (modules/flash/kernel/fwd_kernel_inner.py:140-160:
 row - left <= key <= row + right, and key < seqlen_k) on the CPU, over window values of both
 signs, the clamped sentinels and ragged sequence ends."""
