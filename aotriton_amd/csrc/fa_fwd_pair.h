@@ -3,7 +3,7 @@
 // Same arithmetic as fwd_item (fa_fwd_impl.h; modules/flash/kernel/fwd_kernel.py:83-644, fwd_kernel_inner.py:46-287 of the
 // reference), other division of the work:
 //   wave w      S^T(u) = K(u) Q^T, the online softmax of unit u - 1 (bias, mask, row maximum, row sum) behind it    holds Q
-//   wave w + 4  O^T += V(u - 2)^T P(u - 2)^T; requests K and V, draws the keep bits                                 holds O
+//   wave w + 4  O^T += V(u - 2)^T P(u - 2)^T; requests K and V                                                      holds O
 // P goes from one to the other through LDS as the operand it becomes, with the factor that takes O to the rows' new reference
 // where it has moved.
 //
@@ -15,7 +15,9 @@
 // load into LDS, so the eight of a wave stand between its MFMAs: in front of them they held it up for 650 cycles of a step's 2300.
 //
 // Bound: the two waves' 32 MFMAs take 1024 cycles of a step's 1950 (at 1.9 GHz); what is left is that after the barrier both wait for their first
-// operands and before it for the last exponentials and P, with the matrix pipe idle.  With dropout the Philox rounds (900 cycles) fill part of it.
+// operands and before it for the last exponentials and P, with the matrix pipe idle.  With dropout the rounds of a unit's Philox calls (300 cycles
+// each next to the other wave) are longer than that: with all four in the second wave its step takes 2800 and the first one's 2000; two each, us, window
+// S1801 38.5 -> 37.4, S8192 571 -> 562 (one card; long calls run at the clock that the power leaves, and moving work between the waves gives them less).
 // Level or slower: more operands in flight, wave priorities, the first operands of the next unit read in front of the barrier (a stage
 // more of K), the second waves over 64 columns of all rows (less LDS traffic, 5-8 % slower).
 //
@@ -36,8 +38,8 @@ struct FwdPairSmem {
   static constexpr int P_OFF = 2 * V_OFF, P_BYTES = 4 * 2048;            // per step: two operands per lane of the four first waves
   static constexpr int FACTOR_OFF = P_OFF + 2 * P_BYTES;                 // and a float
   static constexpr int KEEP_OFF = FACTOR_OFF + 2 * 1024;                 // keep bits, a word per lane of the four first waves
-  static constexpr int BIAS_OFF = KEEP_OFF + 2 * 1024, BIAS_ROW = 64 + 16, BIAS_BYTES = 32 * BIAS_ROW;      // per first wave
-  static constexpr int BYTES = BIAS_OFF + 4 * BIAS_BYTES;
+  static constexpr int BIAS_OFF = KEEP_OFF + 2 * 1024, BIAS_ROW = 64 + 16, BIAS_BYTES = 32 * BIAS_ROW;      // per first wave, for units in turn
+  static constexpr int BYTES = BIAS_OFF + 2 * 4 * BIAS_BYTES;
   static constexpr int ROW_STR = D * 2 + 16;                             // O rows on their way out, where K and V were
   static_assert(4 * 32 * ROW_STR <= P_OFF, "four waves' rows");
 };
@@ -118,6 +120,33 @@ __device__ __forceinline__ void fwd_item_pair(const FwdArgs& a, const int z, con
   const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 
   constexpr int kRing = 5;      // operands in flight
+
+  // ---- keep bits of the lane's row: four calls per unit, for the columns 8 g + 4 hi .. + 3.  The first wave runs kOwn of them, the second
+  // wave the others, of unit u behind its MFMAs in step u
+  constexpr int kOwn = 2;
+  uint64_t ctr = 0;                              // of the wave's first call of the unit
+  uint32_t x_k0 = 0, x_k1 = 0;
+  int32_t x_thr = 0;
+  Philox px;
+  uint32_t word = 0;
+  auto keep_begin = [&]() __attribute__((always_inline)) {      // (behind the item's first requests: it waits for the seed)
+    if (!kDropout) return;
+    const DropoutState ds = make_dropout(a.drop, z, h, a.hq, a.seq.max_seqlen_q, a.seq.max_seqlen_k);
+    x_k0 = __builtin_amdgcn_readfirstlane(ds.k0);
+    x_k1 = __builtin_amdgcn_readfirstlane(ds.k1);
+    x_thr = __builtin_amdgcn_readfirstlane(ds.thr);
+    ctr = ds.base + (uint64_t)row * ds.stride + (uint64_t)(G0 * 8 + hi + (first ? 0 : 2 * kOwn));
+  };
+  auto keep_round = [&](int i, int n) __attribute__((always_inline)) {      // round i % 10 of call i / 10, of n calls
+    if (i == 0) word = 0;
+    if (i % 10 == 0) {
+      const uint64_t at = ctr + (uint64_t)(2 * (i / 10));
+      px.start((uint32_t)at, (uint32_t)(at >> 32));
+    }
+    px.round(i % 10, x_k0, x_k1);
+    if (i % 10 == 9) word = dropout_append(px, x_thr, word);
+    if (i == 10 * n - 1) ctr += 8;
+  };
   if (first) {
     // this lane's Q row, the B operand of S^T = K Q^T
     op_t qreg[KS];
@@ -161,9 +190,9 @@ __device__ __forceinline__ void fwd_item_pair(const FwdArgs& a, const int z, con
     auto put_bias = [&](auto set) {
       if constexpr (kBias)
 #pragma unroll
-        for (int i = 0; i < 2; ++i) lds_write(area + (lane / 4 + 16 * i) * SM::BIAS_ROW + (lane % 4) * 16, bco[set][i]);
+        for (int i = 0; i < 2; ++i) lds_write(area + set * 4 * SM::BIAS_BYTES + (lane / 4 + 16 * i) * SM::BIAS_ROW + (lane % 4) * 16, bco[set][i]);
     };
-    auto bias_read = [&](int q) { return lds_read<q4_t>(area + c * SM::BIAS_ROW + (8 * q + 4 * hi) * 2); };
+    auto bias_read = [&](int set, int q) { return lds_read<q4_t>(area + set * 4 * SM::BIAS_BYTES + c * SM::BIAS_ROW + (8 * q + 4 * hi) * 2); };
 
     // every key of the unit is visible to every valid row of the wave
     auto sees_all = [&](int u) -> bool {
@@ -202,7 +231,7 @@ __device__ __forceinline__ void fwd_item_pair(const FwdArgs& a, const int z, con
       if (e % 8 == 6) lds_write(p_place(u) + e / 8 * 1024, pb);
     };
     // Full online-softmax step on the raw scores: scale, bias, mask, row maximum, lazy move of the reference, exponentials, row sum.
-    auto softmax_full = [&](int u, f32x16 x) {
+    auto softmax_full = [&](int set, int u, f32x16 x) {
       if (prescale) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) x[i] *= qk_scale;
@@ -211,7 +240,7 @@ __device__ __forceinline__ void fwd_item_pair(const FwdArgs& a, const int z, con
         if (bias_fits(u)) {
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            const q4_t b4 = bias_read(q);
+            const q4_t b4 = bias_read(set, q);
 #pragma unroll
             for (int r = 0; r < 4; ++r) x[4 * q + r] += (float)b4[r] * kLog2e;   // fwd_kernel_inner.py:187
           }
@@ -269,6 +298,7 @@ __device__ __forceinline__ void fwd_item_pair(const FwdArgs& a, const int z, con
     using odd = std::integral_constant<int, 1>;
     request_bias(even{}, G0);
     request_bias(odd{}, G0 + 1);
+    keep_begin();
     __builtin_amdgcn_s_waitcnt(0x0F70);      // (before the steps: the compiler otherwise waits in each of them for Q to have arrived)
     meet();                                  // the first two units of K are there
     f32x16 x = zero16;                       // raw scores of the unit before the running one
@@ -277,7 +307,18 @@ __device__ __forceinline__ void fwd_item_pair(const FwdArgs& a, const int z, con
       bool full = u > u0 && u - 1 <= u1;      // there is a unit whose softmax is still to be done in full
       f32x16 acc = zero16;
       op_t ka[kRing];
-      if (kDropout) keep = lds_read<uint32_t>(keep_place(u - 1));
+      if (kDropout) keep = word << (16 - 4 * kOwn) | lds_read<uint32_t>(keep_place(u - 1));      // (of the unit before)
+      // behind MFMA k: the unit's bias into its area, the one after the next requested; the first calls of its keep bits
+      auto behind = [&](int k) __attribute__((always_inline)) {
+        if (k == 8) {
+          put_bias(set);
+          request_bias(set, u + 2);
+        }
+        if (kDropout)
+#pragma unroll
+          for (int i = first_of(k, 10 * kOwn, KS); i < first_of(k + 1, 10 * kOwn, KS); ++i) keep_round(i, kOwn);
+        __builtin_amdgcn_sched_barrier(0);
+      };
       if (act) {
 #pragma unroll
         for (int k = 0; k < kRing - 1; ++k) ka[k] = k_read(k);
@@ -289,7 +330,7 @@ __device__ __forceinline__ void fwd_item_pair(const FwdArgs& a, const int z, con
         q4_t b4[4];
         if (kBias)
 #pragma unroll
-          for (int q = 0; q < 4; ++q) b4[q] = bias_read(q);
+          for (int q = 0; q < 4; ++q) b4[q] = bias_read(1 - set, q);
 #pragma unroll
         for (int k = 0; k < KS; ++k) {
           if (k + kRing - 1 < KS) ka[(k + kRing - 1) % kRing] = k_read(k + kRing - 1);
@@ -299,7 +340,7 @@ __device__ __forceinline__ void fwd_item_pair(const FwdArgs& a, const int z, con
           rs += p;
           if (k % 2 == 0) p_even = p;
           else put_pair(u - 1, k - 1, p_even, p);
-          __builtin_amdgcn_sched_barrier(0);
+          behind(k);
         }
         full = __builtin_amdgcn_ballot_w64(!(rs < 4096.f)) != 0;
         if (!full) {
@@ -311,13 +352,15 @@ __device__ __forceinline__ void fwd_item_pair(const FwdArgs& a, const int z, con
         for (int k = 0; k < KS; ++k) {
           if (k + kRing - 1 < KS) ka[(k + kRing - 1) % kRing] = k_read(k + kRing - 1);
           acc = Tr::mfma(ka[k % kRing], qreg[k], k == 0 ? zero16 : acc);
-          __builtin_amdgcn_sched_barrier(0);
+          behind(k);
         }
+      } else {
+        put_bias(set);
+        request_bias(set, u + 2);
+        if (kDropout) ctr += 8;
       }
-      if (full) softmax_full(u - 1, x);
+      if (full) softmax_full(1 - set, u - 1, x);
       x = acc;
-      put_bias(set);
-      request_bias(set, u + 2);
       k_stage = k_stage == SM::STAGES - 1 ? 0 : k_stage + 1;
       k_at += k_stage == 0 ? (1 - SM::STAGES) * SM::TILE_BYTES : SM::TILE_BYTES;
       meet();
@@ -384,32 +427,6 @@ __device__ __forceinline__ void fwd_item_pair(const FwdArgs& a, const int z, con
       v_st = v_st == SM::STAGES - 1 ? 0 : v_st + 1;
     };
 
-    // ---- keep bits of the lane's row: four calls per unit, for the columns 8 g + 4 hi .. + 3
-    uint64_t ctr = 0;
-    uint32_t x_k0 = 0, x_k1 = 0;
-    int32_t x_thr = 0;
-    Philox px;
-    uint32_t word = 0;
-    if (kDropout) {
-      const DropoutState ds = make_dropout(a.drop, z, h, a.hq, a.seq.max_seqlen_q, a.seq.max_seqlen_k);
-      x_k0 = __builtin_amdgcn_readfirstlane(ds.k0);
-      x_k1 = __builtin_amdgcn_readfirstlane(ds.k1);
-      x_thr = __builtin_amdgcn_readfirstlane(ds.thr);
-      ctr = ds.base + (uint64_t)row * ds.stride + (uint64_t)(G0 * 8 + hi);
-    }
-    auto keep_round = [&](int i) __attribute__((always_inline)) {      // round i % 10 of call i / 10
-      if (i == 0) word = 0;
-      if (i % 10 == 0) {
-        const uint64_t at = ctr + (uint64_t)(2 * (i / 10));
-        px.start((uint32_t)at, (uint32_t)(at >> 32));
-      }
-      px.round(i % 10, x_k0, x_k1);
-      if (i % 10 == 9) {
-        word = dropout_append(px, x_thr, word);
-      }
-      if (i == 39) ctr += 8;
-    };
-
     f32x16 o[DB];
 #pragma unroll
     for (int db = 0; db < DB; ++db)
@@ -423,6 +440,7 @@ __device__ __forceinline__ void fwd_item_pair(const FwdArgs& a, const int z, con
       for (int i = 0; i < CH; i += 2) request_k(i);
       request_end(false);
     }
+    keep_begin();
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     meet();
     int v_at = smem0 + SM::V_OFF + Swz<D>::tr_base(lane, 0), v_stage = 0;
@@ -452,16 +470,15 @@ __device__ __forceinline__ void fwd_item_pair(const FwdArgs& a, const int z, con
       if (kDropout) {
         if (u >= u0 && u <= u1) {
 #pragma nounroll
-          for (int n = 0; n < 4; ++n) {
-            px.start((uint32_t)ctr, (uint32_t)(ctr >> 32));
+          for (int n = 0; n < 4 - kOwn; ++n) {
+            const uint64_t at = ctr + (uint64_t)(2 * n);
+            px.start((uint32_t)at, (uint32_t)(at >> 32));
 #pragma unroll
             for (int i = 0; i < 10; ++i) px.round(i, x_k0, x_k1);
-            word = dropout_append(px, x_thr, word);
-            ctr += 2;
+            word = dropout_append(px, x_thr, n == 0 ? 0u : word);
           }
-        } else {
-          ctr += 8;
         }
+        ctr += 8;
       }
       end(u);
     };
@@ -495,7 +512,7 @@ __device__ __forceinline__ void fwd_item_pair(const FwdArgs& a, const int z, con
         }
         if (kDropout)
 #pragma unroll
-          for (int j = first_of(i, 40, 2 * DB); j < first_of(i + 1, 40, 2 * DB); ++j) keep_round(j);
+          for (int j = first_of(i, 10 * (4 - kOwn), 2 * DB); j < first_of(i + 1, 10 * (4 - kOwn), 2 * DB); ++j) keep_round(j, 4 - kOwn);
         __builtin_amdgcn_sched_barrier(0);
       }
       end(u);
