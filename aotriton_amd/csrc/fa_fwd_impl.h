@@ -813,7 +813,7 @@ template <typename T, bool kWindowed> struct FwdTile<T, 128, kWindowed> : FwdTil
 // D = 256: 128 rows on eight waves, two for 32 rows (fa_fwd_pair.h, with what it was measured against).
 template <typename T, bool kWindowed> struct FwdTile<T, 256, kWindowed> : FwdTileOf<256, 8, 32, true> {};
 
-// Half the rows, two workgroups per CU (FwdArgs::half_tiles; dense calls at D <= 128, without a bias or with one of the keys).  A sequence
+// Half the rows, two workgroups per CU (FwdArgs::half_tiles; dense calls at D <= 128).  A sequence
 // is cut finer, so that less of the last tile and of the last round is empty; per row it is 5-15 % slower (K and V
 // are staged once per 128 rows, narrower key tiles).  fwd_small_tiles in fa_api.cpp decides.
 template <int D> struct FwdHalfTile : FwdTileOf<D, 4, D == 64 ? 64 : 32> {};
@@ -894,6 +894,9 @@ hipError_t launch_fwd(const FwdArgs& a, bool windowed, bool bias, bool dropout, 
         return windowed ? launch_fwd_variant<T, D, true, false, false, kPad, false, false, FwdThirdTile>(b, grid, stream)
                         : launch_fwd_variant<T, D, false, false, false, kPad, false, false, FwdThirdTile>(b, grid, stream);
     using Half = FwdHalfTile<D>;
+    if (half && bias && dropout)
+      return windowed ? launch_fwd_variant<T, D, true, true, true, kPad, false, false, Half, true>(b, grid, stream)
+                      : launch_fwd_variant<T, D, false, true, true, kPad, false, false, Half, true>(b, grid, stream);
     switch (half ? (windowed ? 2 : 0) | (dropout ? 1 : 0) : -1) {
       case 0: return launch_fwd_variant<T, D, false, false, false, kPad, false, false, Half>(b, grid, stream);
       case 1: return launch_fwd_variant<T, D, false, false, true, kPad, false, false, Half>(b, grid, stream);
