@@ -46,6 +46,7 @@ EXTRA = {
     'fa_fwd_wide_d128.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form', '-Wno-inline-asm'],
     'fa_bwd_wide_d128.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form', '-Wno-inline-asm'],
     'fa_bwd_pair_d256.hip': ['-Wno-inline-asm'],
+    'fa_bwd_dqs.hip': ['-Wno-inline-asm'],
     'fa_fwd_d256.hip': ['-Wno-inline-asm'],
     'fa_bwd_dq_d128.hip': ['-mllvm', '-amdgpu-mfma-vgpr-form'],
 }

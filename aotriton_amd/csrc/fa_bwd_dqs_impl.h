@@ -8,7 +8,12 @@
 // both dK and dQ are formed from), and this kernel reads it back once and only does
 //   dQ^T (d x queries) += K_tile^T . dS^T      A = K^T from LDS,  B = dS^T from LDS
 // i.e. 5 GEMMs in all, no atomics, one owner per dQ tile, at 2 bytes of HBM traffic each way per
-// visible (query, key) pair.  The kernel is bound by that stream, not by the matrix pipe.
+// visible (query, key) pair.  The kernel is bound by that stream, not by the matrix pipe; calls with few steps by their latency.
+//
+// K and dS go straight into LDS, two steps ahead, counted by hand.  (Through registers, K a step and dS four steps ahead, a wait for
+// K was one for every dS requested before it: memory answers in order.  us, before -> this: 1000 x 1531 D80 43 -> 39, window of 450 of 1801 keys
+// B1 H8 D128 20.8 -> 17.9, B8 H12 S512 D64 with dB 24.9 -> 23.4; window of 1024, B2 H16 S8192 D256 246 -> 230.  Four stages, and 64-key steps at 128
+// columns: level to 2 % slower for whole passes; two stages: 1-2 % slower.)
 //
 // Layout of the stored tiles (written by dkdv_item, kStoreDs): one tile per (batch element, q-head,
 // key tile of 128, query tile of BM = the dK/dV kernel's step) holds 128 x BM values as
@@ -19,16 +24,20 @@
 // copies 1 KB of a tile to LDS as it lies and reads bank-conflict free.
 #pragma once
 #include "fa_bwd_impl.h"
+#include "fa_wide.h"
 
 namespace fa {
 
-template <int D, int BN>
-struct DqsSmem {     // two stages of the K tile (swizzled), then one dS area per wave
+template <int D>
+struct DqsSmem {     // stages of a step's K (swizzled) and of a dS area per wave
   static constexpr int NW = 8;
+  static constexpr int BN = D > 64 ? 32 : 64;        // keys per step
+  static constexpr int STAGES = 3;
   static constexpr int K_BYTES = BN * D * 2;
   static constexpr int DS_WAVE = BN * 32 * 2;
-  static constexpr int DS_OFF = 2 * K_BYTES;
-  static constexpr int BYTES = DS_OFF + NW * DS_WAVE;
+  static constexpr int DS_OFF = STAGES * K_BYTES, DS_STAGE = NW * DS_WAVE;
+  static constexpr int BYTES = DS_OFF + STAGES * DS_STAGE;
+  static_assert(BYTES <= 160 * 1024, "LDS of a CU");
 };
 
 // One Q tile of 256 rows (8 waves x 32 queries) of head h against the key tiles that see it.
@@ -37,19 +46,19 @@ struct DqsSmem {     // two stages of the K tile (swizzled), then one dS area pe
 // where no stored tile is, dB is zero.  The kernel stays bound by its streams, two written or
 // read once instead of one (B8 H12 S512 D64: 25 us for 50 MB in and 50 MB out, with 5 us for the statistics, where
 // the dQ kernel that recomputes S and dP and writes dB took 48).
-template <typename T, int D, int BN, int kPad, bool kDb>
+template <typename T, int D, int kPad, bool kDb>
 __device__ __forceinline__ void dqs_item(const BwdArgs& a, const int h, const int mt, const int z, char* smem_raw) {
   using Tr = Traits<T>;
   using op_t = typename Tr::op_t;
   using q4_t = typename Tr::q4_t;
-  using SM = DqsSmem<D, BN>;
+  using SM = DqsSmem<D>;
+  constexpr int BN = SM::BN, S = SM::STAGES;
   using DT = DsTile<T, D>;
   constexpr int NW = SM::NW, NT = NW * 64, BM = NW * 32;
   constexpr int DB = (kPad ? kPad : D) / 32;
   constexpr int SPT = DT::BN / BN;          // steps per stored tile
   constexpr int KWS = BN / 32;              // 32-key blocks per step
   constexpr int NCK = KWS * 2;              // 1 KB pieces of dS per wave and step
-  constexpr int PD = 4;                     // steps of dS in flight, in registers
   constexpr int LPR = D / 8;                // 16-byte pieces per K row
   constexpr int RPI = NT / LPR;             // rows between two pieces of one thread
   constexpr int CH = (BN * LPR) / NT;       // K pieces per thread and step
@@ -119,66 +128,57 @@ __device__ __forceinline__ void dqs_item(const BwdArgs& a, const int h, const in
     db_lo = jw0;
     db_hi = jw1 < j1 ? jw1 : j1;
 
-    // ---- K tiles: global -> registers -> LDS (swizzled), one step ahead ------------------------
+    // ---- K and dS of a step straight into LDS, S - 1 steps ahead (asm: what is in flight is counted by hand) ----
     const T* kbase = reinterpret_cast<const T*>(a.k) + (int64_t)si.batch_index * a.sk.z + (int64_t)hk * a.sk.h +
                      (int64_t)si.k_start * a.sk.s;
-    const int r0 = tid / LPR, cc0 = tid % LPR;
-    const int k_voff = cc0 * 8 < d_qk ? r0 * (int)a.sk.s * 2 + cc0 * 16 : kVoffOutOfRange;
-    const int k_soff = RPI * (int)a.sk.s * 2;
-    int lds_off[CH];
-#pragma unroll
-    for (int k = 0; k < CH; ++k) lds_off[k] = Swz<D>::addr(r0 + k * RPI, cc0);
-    op_t kreg[CH];
-    auto load_k = [&](int j) {
-      int rows = si.seqlen_k - j * BN;
-      rows = rows < BN ? rows : BN;
-      rows = j <= j1 ? rows : 0;
-      const T* kt = kbase + (int64_t)j * BN * a.sk.s;
-      const auto k_rs = wave_rsrc(kt, rows > 0 ? ((rows - 1) * (int)a.sk.s + d_qk) * 2 : 0);
-#pragma unroll
-      for (int k = 0; k < CH; ++k)
-        kreg[k] = __builtin_bit_cast(op_t, __builtin_amdgcn_raw_buffer_load_b128(k_rs, k_voff, k * k_soff, 0));
-    };
-    auto store_k = [&](int stage) {
-#pragma unroll
-      for (int k = 0; k < CH; ++k) *reinterpret_cast<op_t*>(smem_raw + stage * SM::K_BYTES + lds_off[k]) = kreg[k];
-    };
-
-    // ---- dS pieces: global -> registers (PD steps ahead) -> the wave's LDS area -----------------
+    constexpr int RWI = 64 / LPR;
+    static_assert(RPI % 16 == 0 && RWI * D * 2 == 1024, "the swizzle repeats with every piece, a wave's piece is consecutive");
+    const int r0 = tid / LPR, gch = (tid % LPR) ^ Swz<D>::f(r0);
+    const int k_row = (int)a.sk.s * 2;
+    const int k_voff = gch * 8 < d_qk ? r0 * k_row + gch * 16 : kVoffOutOfRange;
     const char* ws_head = reinterpret_cast<const char*>(a.ds_ws) +
                           ((int64_t)z * a.hq + h) * a.ds_ntk * (int64_t)a.ds_ntq * DT::BYTES;
-    char* ds_area = smem_raw + SM::DS_OFF + wave_u * SM::DS_WAVE;
     const int ds_voff = lane * 16 + qb * DT::QBLOCK_BYTES;
-    op_t dsr[PD][NCK];
-    auto load_ds = [&](auto ring_tag, int j) {
-      constexpr int R = decltype(ring_tag)::value;
-      const int nt = j / SPT, kw0 = (j % SPT) * KWS;
-      const char* tile = ws_head + ((int64_t)nt * a.ds_ntq + pm) * DT::BYTES;
+    const int smem0 = lds_offset(smem_raw);
+    constexpr int LOADS = CH + NCK;          // per wave and step
+    int f_j = j0, f_stage = 0;
+    auto fetch = [&]() __attribute__((always_inline)) {
+      int rows = si.seqlen_k - f_j * BN;
+      rows = rows < BN ? rows : BN;
+      rows = f_j <= j1 ? rows : 0;
+      const auto k_rs = wave_rsrc_words(kbase + (int64_t)f_j * BN * a.sk.s, rows_extent(rows, k_row, d_qk * 2));
+      const int k_at = smem0 + f_stage * SM::K_BYTES + wave_u * 1024;
+      if constexpr (CH == 1) load_to_lds1(k_rs, k_voff, k_at);
+      else load_to_lds(k_rs, k_voff, 0, k_at, k_voff, RPI * k_row, k_at + RPI * D * 2);
       // a wave that has nothing to fetch at this step reads through an empty descriptor: zeros, no traffic
-      const auto rs = wave_rsrc(tile, active(j) ? DT::BYTES : 0);
+      const int nt = f_j / SPT, from = f_j % SPT * KWS * 2048;
+      const auto rs = wave_rsrc_words(ws_head + ((int64_t)nt * a.ds_ntq + pm) * DT::BYTES, active(f_j) ? DT::BYTES : 0);
+      const int ds_at = smem0 + SM::DS_OFF + f_stage * SM::DS_STAGE + wave_u * SM::DS_WAVE;
 #pragma unroll
-      for (int i = 0; i < NCK; ++i)
-        dsr[R][i] = __builtin_bit_cast(op_t, __builtin_amdgcn_raw_buffer_load_b128(
-                                                 rs, ds_voff, kw0 * 2048 + i * 1024, 2));
+      for (int i = 0; i < NCK; i += 2) load_to_lds_once(rs, ds_voff, from + i * 1024, ds_at + i * 1024);
+      ++f_j;
+      f_stage = f_stage == S - 1 ? 0 : f_stage + 1;
     };
+    static_assert(CH <= 2 && NCK % 2 == 0, "pieces in pairs");
 
     // lane constants of the transposing reads: K^T rows of the swizzled tile, dS^T of the wave's area
     const int tr_a0 = Swz<D>::tr_base(lane, 0), tr_a1 = Swz<D>::tr_base(lane, 1);
     const int g16 = (lane >> 4) & 1, il = lane & 15;
     const int ds_rd = g16 * 1024 + ((((4 * hi + (il >> 2)) * 2 + (il & 1)) ^ (g16 << 3)) << 4) + ((il >> 1) & 1) * 8;
 
-    auto step = [&](auto ring_tag, int j) __attribute__((always_inline)) {
-      constexpr int R = decltype(ring_tag)::value;
-      __syncthreads();          // K(j) is in its stage; everybody has left the other one
-      load_k(j + 1);
+    int stage = 0;
+#pragma unroll
+    for (int i = 0; i < S - 1; ++i) fetch();
+#pragma nounroll
+    for (int j = j0; j <= j1; ++j) {
+      // This wave's part of the step has arrived (what was requested for later ones may be under way; stores of dB, which come between, only make the
+      // wait longer) and then everybody's, and everybody has left the stage that is filled next.
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"((S - 2) * LOADS) : "memory");
+      fetch();
+      char* const ds_area = smem_raw + SM::DS_OFF + stage * SM::DS_STAGE + wave_u * SM::DS_WAVE;
       const bool act = active(j);
       if (act) {
-#pragma unroll
-        for (int i = 0; i < NCK; ++i) *reinterpret_cast<op_t*>(ds_area + i * 1024 + lane * 16) = dsr[R][i];
-      }
-      load_ds(ring_tag, j + PD);
-      if (act) {
-        const char* Kb = smem_raw + (j & 1) * SM::K_BYTES;
+        const char* Kb = smem_raw + stage * SM::K_BYTES;
         op_t bs[kDb ? BN / 16 : 1];
 #pragma unroll
         for (int tk = 0; tk < BN / 16; ++tk) {
@@ -206,24 +206,9 @@ __device__ __forceinline__ void dqs_item(const BwdArgs& a, const int h, const in
           }
         }
       }
-      store_k((j + 1) & 1);
-    };
-
-    load_k(j0);
-    load_ds(std::integral_constant<int, 0>{}, j0);
-    load_ds(std::integral_constant<int, 1>{}, j0 + 1);
-    load_ds(std::integral_constant<int, 2>{}, j0 + 2);
-    load_ds(std::integral_constant<int, 3>{}, j0 + 3);
-    store_k(j0 & 1);
-    // whole groups of PD steps, so that the loop body is one straight sequence (steps past the last
-    // one fetch through empty descriptors and compute nothing); with conditional steps the compiler
-    // copies the ring and the accumulators at the loop's end and waits for every load in flight there
-    for (int j = j0; j <= j1; j += PD) {
-      step(std::integral_constant<int, 0>{}, j);
-      step(std::integral_constant<int, 1>{}, j + 1);
-      step(std::integral_constant<int, 2>{}, j + 2);
-      step(std::integral_constant<int, 3>{}, j + 3);
+      stage = stage == S - 1 ? 0 : stage + 1;
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // (LDS belongs to the workgroup no longer than it runs)
   }
 
   if constexpr (kDb) {
@@ -247,7 +232,7 @@ __device__ __forceinline__ void dqs_item(const BwdArgs& a, const int h, const in
 
 // One workgroup per Q tile on a 1-D grid: consecutive ids go round the XCDs, an XCD takes its
 // (batch, q-head) pairs two at a time, the heaviest (last) tile of a causal mask first.
-template <typename T, int D, int BN, int kPad, bool kDb>
+template <typename T, int D, int kPad, bool kDb>
 __global__ __attribute__((amdgpu_flat_work_group_size(512, 512))) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void bwd_dqs_kernel(const BwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
@@ -260,20 +245,19 @@ void bwd_dqs_kernel(const BwdArgs a) {
   const int mt = a.num_m_tiles - 1 - gr / a.zh_group;
   int z, h;
   split_zh(zh, a.num_zh / a.hq, a.hq / a.hk, z, h);
-  dqs_item<T, D, BN, kPad, kDb>(a, h, mt, z, smem_raw);
+  dqs_item<T, D, kPad, kDb>(a, h, mt, z, smem_raw);
 }
 
 template <typename T, int D, int kPad>
 hipError_t launch_bwd_dqs(const BwdArgs& a0, hipStream_t stream) {
-  constexpr int BN = D >= 256 ? 32 : 64;
   BwdArgs a = a0;
   a.num_m_tiles = (a.seq.max_seqlen_q + 255) / 256;
   set_work(a, tile_work(bwd_nseq(a) * a.hq, q_head_group(a.hq, a.hk), a.num_m_tiles));
   dim3 grid((unsigned)(kNumXcd * a.items_per_xcd));
-  constexpr int lds = DqsSmem<D, BN>::BYTES;
+  constexpr int lds = DqsSmem<D>::BYTES;
   const bool db = a.db != nullptr;
-  return db ? launch_with_lds<bwd_dqs_kernel<T, D, BN, kPad, true>>(grid, 512, lds, stream, a)
-            : launch_with_lds<bwd_dqs_kernel<T, D, BN, kPad, false>>(grid, 512, lds, stream, a);
+  return db ? launch_with_lds<bwd_dqs_kernel<T, D, kPad, true>>(grid, 512, lds, stream, a)
+            : launch_with_lds<bwd_dqs_kernel<T, D, kPad, false>>(grid, 512, lds, stream, a);
 }
 
 }  // namespace fa

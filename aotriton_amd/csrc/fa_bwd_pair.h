@@ -46,10 +46,6 @@ struct PairSmem {
   static_assert(STAGE_BYTES % 512 == 0 && TILE_BYTES % 512 == 0, "stage offsets leave the swizzled bits alone");
 };
 
-// A wave's 64 x 16 bytes straight into LDS (see load_to_lds).
-__device__ __forceinline__ void load_to_lds1(u32x4_t rsrc, int voff, int lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" :: "s"(lds), "v"(voff), "s"(rsrc) : "m0");
-}
 // The lane's number, formed where it is used: what is derived from it then does not stay in registers over the steps.
 __device__ __forceinline__ int lane_here() {
   int x;
