@@ -84,3 +84,50 @@ def test_bias_layouts_agree(kind):
         x = b
     got, gl = _forward(q, k, v, x, (100, 30), 1 / 16)
     assert torch.equal(got, want) and torch.equal(gl, wl)
+
+
+@pytest.mark.parametrize('p,causal', [(0.0, False), (0.25, (100, 30))])
+def test_columns_of_a_bias_apart(p, causal):
+    """Columns that lie apart, which the views of the bindings take, go through the units' general step: adjacent columns' results but
+    for the roundings of P."""
+    from aotriton_amd import flash
+    from aotriton_amd.pyaotriton import T4
+    B, H, Sq, Sk = 1, 3, 190, 261
+    q, k, v, b, _ = make_inputs(B, H, H, Sq, Sk, 256, BF, 'cuda', seed=6, bias=True)
+    b = b.contiguous()
+    seed, off = (torch.tensor([x], device='cuda', dtype=torch.uint64) for x in (7, 8))
+    null, out = torch.empty([0], device='cuda', dtype=torch.uint64), []
+    for x in (b, b.transpose(2, 3).contiguous().transpose(2, 3)):
+        o, L = torch.empty_like(q), torch.empty(B * H, Sq, device='cuda')
+        params = flash.fa_forward_op_params()
+        flash._fill_fwd(params, q, k, v, None, 1 / 16, L, o, p, seed, off, 0, null, null, None, causal, null)
+        params.B = T4(x.data_ptr(), tuple(x.size()), x.stride(), flash.cast_dtype(BF))
+        params.varlen_type = 0
+        assert flash.fa_forward_op(params, params.kVersion, flash._stream(), None) == flash.hipError_t.hipSuccess
+        torch.cuda.synchronize()
+        out.append((o.float(), L))
+    (o, L), (o1, L1) = out
+    # P rounded to 16 bits on either side (2^-9 of values that sum to 1 / (1 - p)), the results too
+    assert ((o - o1).abs() <= 2 ** -8 * (1 / (1 - p) * v.float().abs().max() + o.abs())).all()
+    seen = torch.isfinite(L)
+    assert torch.equal(seen, torch.isfinite(L1)) and (L - L1).abs()[seen].max() <= 1e-5
+
+
+@pytest.mark.parametrize('causal', [False, True])
+def test_packed_sequences(causal):
+    """Lengths around tiles and units, walked by level, against 64 bits."""
+    from aotriton_amd.autograd import attention_varlen, AttentionExtraArgs
+    lens, H = [1, 31, 32, 33, 127, 128, 129, 260, 640, 65], 8
+    g = torch.Generator(device='cuda').manual_seed(9)
+    q, k, v = (torch.randn(1, H, sum(lens), 256, device='cuda', generator=g).to(BF) for _ in range(3))
+    got = attention_varlen(q, k, v, lens, lens, causal, 1 / 16, 0.0, AttentionExtraArgs(return_logsumexp=False))[0]
+    at = 0
+    for n in lens:
+        x, y, z = (t[:, :, at:at + n].double() for t in (q, k, v))
+        s = torch.matmul(x, y.transpose(-1, -2).contiguous()) / 16
+        if causal:
+            s = s.masked_fill(torch.ones(n, n, device='cuda', dtype=torch.bool).triu(1), float('-inf'))
+        want = torch.matmul(torch.softmax(s, -1), z)
+        # P rounded to 16 bits, the result rounded
+        assert ((got[:, :, at:at + n].double() - want).norm() / want.norm()).item() < 3 * torch.finfo(BF).eps / 2, n
+        at += n
