@@ -571,8 +571,7 @@ struct FwdPlan {
 // 0.07 us of the whole chip's memory time at D = 128, the second launch 5 us.  Against 665 measured shapes of 1-2048
 // queries and 64-10000 keys (profiles/forward_routes.txt holds a third of them) the estimate of whole tiles is within
 // 25 % for 84 %, that of the rows kernel, which knows no HBM rate, for 63 %; the route taken is the best of
-// the three, or within a tenth of it, for 95 %.  One measured shape is more than 10 % slower than whole tiles on its
-// route (Hq 8, Hk 2, 512 causal, D = 256: 28 -> 33).  The gains it decides on are larger
+// the three, or within a tenth of it, for 95 %.  The gains it decides on are larger
 // (one query, 2051 keys, Hq 32 / Hk 8: 55 -> 11 us; 32 sequences of 8190 keys: 833 -> 189; 80 queries,
 // 3216 keys: 88 -> 35; 1024 queries, 16384 keys: 402 -> 266).  Tiles of 128 rows (fwd_small_tiles below) are not among
 // what is compared: they are asked about where this rule leaves the tiles whole.
@@ -640,7 +639,11 @@ FwdPlan fwd_plan(int dtype, const Shape& s, int causal_type, int window_left, in
   const double load = average * (s.d > 128 ? (double)busy_rounds : (double)busiest / cus);
   const double busy_time = (load > 1 ? load : 1) * steps * t128 + 4 * (double)busy_rounds + 1 + (splits > 1 ? 4 : 0);
   // (the lines: D = 128 and 256 level at 1.1 of these figures, D = 64, whose steps take 0.55 us on two XCDs, at 1.7)
-  r.rows = rows_time < best && busy_time <= (s.d == 64 ? 1.75 : 1.08) * whole;
+  // (D = 256 with more than one row block: its tiles take less than t64 says where a round of them is short.  us, rows / tiles: on the rows' side of
+  // the line 16 heads 256 x 1024 28 / 32, 32 heads 128 x 2000 37 / 54, 4 x 16 heads 128 x 1000 31 / 33; on the other Hq 8 Hk 2 512 causal 32 / 21, 256 causal
+  // 18.6 / 15.8, 8 x 16 heads 64 x 300 19 / 16, 4 x 8 heads 64 x 200 17 / 13, 4 x 16 heads 60 x 60 12.1 / 10.7; one query is never slower in rows)
+  const double line = s.d == 64 ? 1.75 : s.d == 128 || rows <= 32 ? 1.08 : 0.75;
+  r.rows = rows_time < (s.d > 128 && rows > 32 ? 0.75 : 1.0) * best && busy_time <= line * whole;
   int64_t stored;
   if (r.rows) {
     r.splits = (int)splits;

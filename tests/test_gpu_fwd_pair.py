@@ -10,9 +10,17 @@ from test_launch_queries import fwd
 from oracle import fa_ref
 from _util import FUDGE, check, make_inputs
 
-pytestmark = pytest.mark.gpu
-
 BF, HF = torch.bfloat16, torch.float16
+
+
+def test_short_calls_of_several_row_blocks():
+    """tiles where one round of them is shorter than the packed rows' steps; one row block stays packed"""
+    for call in [(1, 8, 2, 512, 512, 256, True), (8, 16, 16, 64, 300, 256), (1, 8, 2, 256, 256, 256, True), (4, 16, 16, 60, 60, 200)]:
+        assert not fwd(*call).flags & 128, call
+    for call in [(1, 16, 4, 256, 1024, 256), (1, 32, 32, 128, 2000, 256), (1, 32, 8, 1, 64, 256), (4, 16, 16, 16, 100, 256), (4, 16, 16, 32, 60, 256)]:
+        assert fwd(*call).flags & 128, call
+
+
 CASES = [
     # B, Hq, Hk, Sq, Sk, D, Dv, dtype, causal, dropout, bias
     (2, 2, 2, 17, 1, 256, 256, BF, False, 0.0, False),             # one key, three row blocks without rows
@@ -31,6 +39,7 @@ CASES = [
 ]
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize('case', CASES, ids=lambda c: '-'.join(str(x).replace('torch.', '') for x in c))
 def test_pairs_meet_the_oracle(case):
     B, Hq, Hk, Sq, Sk, D, Dv, dtype, causal, p, bias = case
@@ -50,6 +59,7 @@ def _forward(q, k, v, b, causal, sm):
     return o, lse.view(q.shape[0], q.shape[1], -1)
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize('dtype,causal,sm,bias', [(BF, False, 1 / 16, False), (HF, True, 1 / 16, True), (BF, False, -1 / 16, False), (HF, False, 1.0, False)])
 def test_references_that_move(dtype, causal, sm, bias):
     """Scores that grow along the keys (every few units the exponentials leave their range and a unit is done in full), for some rows
@@ -68,6 +78,7 @@ def test_references_that_move(dtype, causal, sm, bias):
     assert ((lse - rl.view_as(lse)).abs() <= 1e-5 * (1 + rl.view_as(lse).abs()) + 2e-4).all()
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize('kind', ['offset', 'odd rows', 'broadcast rows'])
 def test_bias_layouts_agree(kind):
     """A bias gives the same bits wherever its rows lie."""
@@ -86,6 +97,7 @@ def test_bias_layouts_agree(kind):
     assert torch.equal(got, want) and torch.equal(gl, wl)
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize('p,causal', [(0.0, False), (0.25, (100, 30))])
 def test_columns_of_a_bias_apart(p, causal):
     """Columns that lie apart, which the views of the bindings take, go through the units' general step: adjacent columns' results but
@@ -113,6 +125,7 @@ def test_columns_of_a_bias_apart(p, causal):
     assert torch.equal(seen, torch.isfinite(L1)) and (L - L1).abs()[seen].max() <= 1e-5
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize('causal', [False, True])
 def test_packed_sequences(causal):
     """Lengths around tiles and units, walked by level, against 64 bits."""
