@@ -126,6 +126,9 @@ __device__ __forceinline__ typename Traits<T>::op_t lds_read_tr8(const T* p, int
 // MFMA operand (16 consecutive rows, same chunk) and the transposing reads (4
 // consecutive rows x 4 consecutive chunks per half-wave).  A tile can therefore
 // serve both as the row operand of one GEMM and as the transposed operand of another.
+// (f moves chunks inside 256 bytes: a kernel that picks operands by an exclusive or with an address instead of an offset into the
+// tile needs its tiles at multiples of that.)
+constexpr int kSwzAlign = 256;
 template <int D>
 struct Swz {
   static constexpr int ROWB = D * 2;

@@ -729,7 +729,8 @@ template <typename T, int D, int NW, int BN, bool kPairs, bool kWindowed, bool k
 __global__ __attribute__((amdgpu_flat_work_group_size(NW * 64, NW * 64)))
 __attribute__((amdgpu_waves_per_eu(kFwdWaves<D, NW, BN>, kFwdWaves<D, NW, BN>)))
 void fwd_kernel(const FwdArgs a) {
-  extern __shared__ __attribute__((aligned(16))) char smem_raw[];
+  extern __shared__ __attribute__((aligned(kPairs ? kSwzAlign : 16))) char smem_raw[];
+  static_assert(!kPairs || __alignof__(smem_raw) >= kSwzAlign, "fwd_item_pair picks operands by exclusive or with addresses");
   if (kDropout && blockIdx.x == 0 && threadIdx.x == 0) {
     // modules/flash/kernel/fwd_kernel.py:199-207
     const uint64_t seed = *a.drop.seed_ptr;

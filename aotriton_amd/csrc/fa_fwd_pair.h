@@ -42,6 +42,7 @@ struct FwdPairSmem {
   static constexpr int BYTES = BIAS_OFF + 2 * 4 * BIAS_BYTES;
   static constexpr int ROW_STR = D * 2 + 16;                             // O rows on their way out, where K and V were
   static_assert(4 * 32 * ROW_STR <= P_OFF, "four waves' rows");
+  static_assert(TILE_BYTES % kSwzAlign == 0 && V_OFF % kSwzAlign == 0, "stages leave the swizzled bits of an address alone");
 };
 
 template <typename T, bool kWindowed, bool kBias, bool kDropout, int kPad>
