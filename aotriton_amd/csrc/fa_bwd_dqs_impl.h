@@ -12,8 +12,16 @@
 //
 // K and dS go straight into LDS, two steps ahead, counted by hand.  (Through registers, K a step and dS four steps ahead, a wait for
 // K was one for every dS requested before it: memory answers in order.  us, before -> this: 1000 x 1531 D80 43 -> 39, window of 450 of 1801 keys
-// B1 H8 D128 20.8 -> 17.9, B8 H12 S512 D64 with dB 24.9 -> 23.4; window of 1024, B2 H16 S8192 D256 246 -> 230.  Four stages, and 64-key steps at 128
-// columns: level to 2 % slower for whole passes; two stages: 1-2 % slower.)
+// B1 H8 D128 19.3 -> 17.7, B8 H12 S512 D64 with dB 26.6 -> 25.2; window of 1024, B2 H16 S8192 D256 246 -> 230.  What is slower that way: at D = 64 with dB
+// where each CU has one workgroup of four steps, two of which are requested at once instead of all, 4000 x 200 17.7 -> 21.2, 4000 x 256 17.8 -> 19.3,
+// B16 H16 S256 17.8 -> 18.9; D256 B2 H16 S4096 causal 182 -> 187.  Four stages: those 20.2, 17.9, 17.7 and 189, but 1-4 % more for other calls with dB; two
+// stages: 1-2 % slower.  Waits that count the stores of dB as well: level.)
+//
+// Keys per step at 128 columns: 64 with dB and where there are fewer workgroups than CUs, else 32.  A step has a barrier and a chain of LDS reads, with dB a
+// turn through LDS as well, which a CU's only workgroup waits out; steps of 32 take half the LDS, so that a CU holds two workgroups.  us, 32 / 64 keys: with dB
+// B2 H8 200 x 4000 113 / 91 (D80 108 / 87), B1 H8 S4096 causal 155 / 134, B2 H16 S2048 causal 102 / 86, B8 H16 S1024 119 / 108, B16 H16 S256 22.9 / 21.7; without,
+// dropout: B1 H8 64 x 2000 26.8 / 22.0, B2 H8 200 x 4000 69 / 58.7, B1 H16 S2048 D80 causal 34.3 / 31.1, B3 H16 1000 x 1531 39.5 / 36.7; from a workgroup per CU
+// on B64 H16 S128 D96 26.9 / 28.1, B32 H16 S128 17.2 / 18.0, B4 H16 1000 x 1531 43-54 / 43-57, B5 H16 with a bias 74-79 / 78-82.
 //
 // Layout of the stored tiles (written by dkdv_item, kStoreDs): one tile per (batch element, q-head,
 // key tile of 128, query tile of BM = the dK/dV kernel's step) holds 128 x BM values as
@@ -28,10 +36,9 @@
 
 namespace fa {
 
-template <int D>
+template <int D, int BN>      // BN: keys per step
 struct DqsSmem {     // stages of a step's K (swizzled) and of a dS area per wave
   static constexpr int NW = 8;
-  static constexpr int BN = D > 64 ? 32 : 64;        // keys per step
   static constexpr int STAGES = 3;
   static constexpr int K_BYTES = BN * D * 2;
   static constexpr int DS_WAVE = BN * 32 * 2;
@@ -46,13 +53,13 @@ struct DqsSmem {     // stages of a step's K (swizzled) and of a dS area per wav
 // where no stored tile is, dB is zero.  The kernel stays bound by its streams, two written or
 // read once instead of one (B8 H12 S512 D64: 25 us for 50 MB in and 50 MB out, with 5 us for the statistics, where
 // the dQ kernel that recomputes S and dP and writes dB took 48).
-template <typename T, int D, int kPad, bool kDb>
+template <typename T, int D, int BN, int kPad, bool kDb>
 __device__ __forceinline__ void dqs_item(const BwdArgs& a, const int h, const int mt, const int z, char* smem_raw) {
   using Tr = Traits<T>;
   using op_t = typename Tr::op_t;
   using q4_t = typename Tr::q4_t;
-  using SM = DqsSmem<D>;
-  constexpr int BN = SM::BN, S = SM::STAGES;
+  using SM = DqsSmem<D, BN>;
+  constexpr int S = SM::STAGES;
   using DT = DsTile<T, D>;
   constexpr int NW = SM::NW, NT = NW * 64, BM = NW * 32;
   constexpr int DB = (kPad ? kPad : D) / 32;
@@ -232,7 +239,7 @@ __device__ __forceinline__ void dqs_item(const BwdArgs& a, const int h, const in
 
 // One workgroup per Q tile on a 1-D grid: consecutive ids go round the XCDs, an XCD takes its
 // (batch, q-head) pairs two at a time, the heaviest (last) tile of a causal mask first.
-template <typename T, int D, int kPad, bool kDb>
+template <typename T, int D, int BN, int kPad, bool kDb>
 __global__ __attribute__((amdgpu_flat_work_group_size(512, 512))) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void bwd_dqs_kernel(const BwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
@@ -245,7 +252,7 @@ void bwd_dqs_kernel(const BwdArgs a) {
   const int mt = a.num_m_tiles - 1 - gr / a.zh_group;
   int z, h;
   split_zh(zh, a.num_zh / a.hq, a.hq / a.hk, z, h);
-  dqs_item<T, D, kPad, kDb>(a, h, mt, z, smem_raw);
+  dqs_item<T, D, BN, kPad, kDb>(a, h, mt, z, smem_raw);
 }
 
 template <typename T, int D, int kPad>
@@ -254,10 +261,12 @@ hipError_t launch_bwd_dqs(const BwdArgs& a0, hipStream_t stream) {
   a.num_m_tiles = (a.seq.max_seqlen_q + 255) / 256;
   set_work(a, tile_work(bwd_nseq(a) * a.hq, q_head_group(a.hq, a.hk), a.num_m_tiles));
   dim3 grid((unsigned)(kNumXcd * a.items_per_xcd));
-  constexpr int lds = DqsSmem<D>::BYTES;
-  const bool db = a.db != nullptr;
-  return db ? launch_with_lds<bwd_dqs_kernel<T, D, kPad, true>>(grid, 512, lds, stream, a)
-            : launch_with_lds<bwd_dqs_kernel<T, D, kPad, false>>(grid, 512, lds, stream, a);
+  constexpr int BN = D >= 256 ? 32 : 64;
+  if (a.db != nullptr) return launch_with_lds<bwd_dqs_kernel<T, D, BN, kPad, true>>(grid, 512, DqsSmem<D, BN>::BYTES, stream, a);
+  if constexpr (D == 128)
+    if ((int64_t)a.num_zh * a.num_m_tiles >= a.num_cu)
+      return launch_with_lds<bwd_dqs_kernel<T, D, 32, kPad, false>>(grid, 512, DqsSmem<D, 32>::BYTES, stream, a);
+  return launch_with_lds<bwd_dqs_kernel<T, D, BN, kPad, false>>(grid, 512, DqsSmem<D, BN>::BYTES, stream, a);
 }
 
 }  // namespace fa
