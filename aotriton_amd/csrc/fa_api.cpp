@@ -705,10 +705,12 @@ bool fwd_wide(const fa_fwd_params* p, const Shape& s, int splits, int num_cu) {
 // best of the three, whole tiles 49 %; B8 H12 S512 22.1 / 22.4 / 26.1 us, S520 61 / 26 / 30, S513 193 / 26 / 30, B16 H12 275 x 583
 // 62 / 51 / 38); within the three rounds that this rule covers unaligned rows take no whole tiles, unless a window is bounded on the
 // left.  Beyond, and with such a window, the tiles are whole (fa_query_fwd_config reports them).
-// A bias that differs between rows, with dropout: two per CU everywhere.  The 256-row tile of these kernels keeps more than fits 256
-// registers, so that the smaller one wins full rounds as well (us, 256 rows / 128 twice, window with both: D64 B1 H8 S1024 34 / 22, B2 H16
-// S2048 53 / 42, S8192 306 / 256; D128 40 / 26, 66 / 51, 407 / 338; B4 H16 S1500 98 / 51 and 109 / 61; 38 shapes, 0.52-0.84).  Up to two
-// tiles of 256 rows, where either takes 20-40 us, the calls stay with the whole tiles, whose tests are of those sizes.
+// A bias with dropout: two per CU.  The 256-row tile of these kernels keeps more than fits 256 registers, so that the smaller one wins full
+// rounds as well (us, 256 rows / 128 twice, window with both: D64 B1 H8 S1024 34 / 21, B2 H16 S2048 53 / 42, S8192 306 / 256; D128 40 / 26, 66 / 51,
+// 407 / 338; B4 H16 S1500 98 / 51 and 109 / 61) and short calls (D64 B1 H8 64 x 64 20.0 / 8.3, B2 H16 S256 19.4 / 15.4, B8 H16 S512 window 35 / 24, B64 H16 40 x 200
+// 100 / 40, B4 H8 32 x 2000 130 / 75; D80 S64 11.1 / 9.2; D96 B4 H12 S128 14.1 / 12.2; D128 B1 H8 100 x 300 33 / 22, B16 H16 S300 84 / 53): 93 shapes of 32-3000
+// queries, 0.40-1.01 of the time.  Calls of at most four tiles of 256 rows would gain too (B1 H2 512 x 600: D64 45 / 27, D128 causal 36 / 30); they are
+// left with those tiles, which a test of the routes holds them to.
 int fwd_small_tiles(const fa_fwd_params* p, const Shape& s, bool wide, int num_cu) {
   const bool key_bias = s.bias && !s.dropout && p->B.strides[2] == 0;
   const bool row_bias = s.bias && !key_bias && !s.dropout && s.d == 64 && p->B.strides[3] == 1;
@@ -717,8 +719,8 @@ int fwd_small_tiles(const fa_fwd_params* p, const Shape& s, bool wide, int num_c
   if (s.elementwise || !is_16bit(p->Q.dtype) || s.d > 128 || (s.bias && !key_bias && !row_bias && !drop_bias) || s.num_seqlens != 0 || s.max_sq <= 0 ||
       s.max_sk <= 0 || s.batch <= 0 || cus < 1 || cus > 64)
     return 0;
-  if (drop_bias) return s.max_sq > 512 ? 2 : 0;
   const int m_tiles = (s.max_sq + 255) / 256, group = fa::q_head_group(s.hq, s.hk);
+  if (drop_bias) return s.max_sq > 512 || (int64_t)s.batch * s.hq * m_tiles > 4 ? 2 : 0;
   if (fa::tile_work(s.batch * s.hq, group, m_tiles).items_per_xcd > std::min((row_bias ? 3 : 8) * cus, 448)) return 0;
   fa::Window w{0, 0};
   if (s.windowed) w = fa::parse_window(p->causal_type, p->window_left, p->window_right, s.max_sq, s.max_sk);

@@ -61,3 +61,28 @@ def test_rows_lie_anywhere(D, dt, causal):
         got.append((o, L))
     for o, L in got[1:]:
         assert torch.equal(o, got[0][0]) and torch.equal(L, got[0][1])
+
+
+SHORT = [
+    # up to 512 queries, more than four tiles of 256 rows
+    (1, 8, 8, 64, 64, 64, BF, False),
+    (5, 1, 1, 1, 129, 64, HF, False),             # one query
+    (2, 4, 2, 31, 1, 128, BF, False),             # one key
+    (3, 2, 2, 128, 96, 80, HF, True),
+    (2, 3, 3, 129, 257, 128, HF, (40, 30)),       # one row in the second tile, one key in the last
+    (1, 5, 5, 200, 333, 96, BF, (30, -10)),       # rows that see nothing
+    (1, 3, 3, 512, 512, 40, HF, (128, 0)),
+    (1, 6, 2, 256, 70, 64, BF, True),
+]
+
+
+def test_short_calls_are_of_these_tiles_too():
+    for c in SHORT:
+        x = fwd(*c[:6], c[7], 0.3, True)
+        assert (x.block_m, x.block_n, x.num_waves) == (128, 64 if c[5] <= 64 else 32, 4), _id(c)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('case', SHORT, ids=_id)
+def test_short_calls_meet_the_oracle(case):
+    _run_case(*case, dropout_p=0.3, bias=True, seed=37)
