@@ -564,14 +564,17 @@ struct FwdPlan {
 };
 
 // The rule compares estimated times in microseconds.  They come from measurements on one box (bf16):
-// fwd_kernel takes a 256-row tile (128 at D = 256) through 64 keys in 1.2 / 1.9 / 2.4 us (D = 64 / 128 /
+// fwd_kernel takes a 256-row tile (128 at D = 256) through 64 keys in 1.2 / 1.9 / 1.9 us (D = 64 / 128 /
 // 256) with all CUs busy (a quarter less on an idle chip, whose clock is higher), one workgroup per
-// CU, and 6 us around that; the rows kernel takes four waves of 32 rows through 4 x 32 keys in
-// 0.9 / 1.2 / 2.6 us, two workgroups of a CU (one at D = 256) taking turns, and 4 us around that; a part's sums of 256 rows cost
-// 0.07 us of the whole chip's memory time at D = 128, the second launch 5 us.  Against 665 measured shapes of 1-2048
-// queries and 64-10000 keys (profiles/forward_routes.txt holds a third of them) the estimate of whole tiles is within
-// 25 % for 84 %, that of the rows kernel, which knows no HBM rate, for 63 %; the route taken is the best of
-// the three, or within a tenth of it, for 95 %.  The gains it decides on are larger
+// CU, and 6 us (7 at D = 256) around that; the rows kernel takes four waves of 32 rows through 4 x 32 keys in
+// 0.9 / 1.2 / 2.6 us, two workgroups of a CU (one at D = 256) taking turns, and 4 us around that (7.2 at D = 256 for full blocks
+// of rows: 32 keys, 4-9 rows 8 us, 64 rows 10.4, 256 rows 11.1); a part's sums of 256 rows cost
+// 0.07 us of the whole chip's memory time at D = 128, the second launch 5 us.  Against 369 measured shapes of 1-2048
+// queries and 2-10000 keys (227 are in profiles/forward_routes.txt) the estimate of whole tiles is within
+// 25 % for 98 %, that of the rows kernel, which knows no HBM rate, for 79 %; the route taken is the best of
+// the three, or within a tenth of it, for 98 %.  Off by more: at D = 64 256 queries of 4096 keys (split 32 us, rows 24) and 1500 causal of Hq 8
+// Hk 2 (rows 32, tiles 28); at D128 B4 Hq 32 Hk 8 100 x 3000 (rows 59, split 53); at D = 256 three calls of one
+// block of 27-32 rows and as many keys (rows 9.7-10.2, tiles 8.7; a test of the routes holds such calls to the rows).  The gains it decides on are larger
 // (one query, 2051 keys, Hq 32 / Hk 8: 55 -> 11 us; 32 sequences of 8190 keys: 833 -> 189; 80 queries,
 // 3216 keys: 88 -> 35; 1024 queries, 16384 keys: 402 -> 266).  Tiles of 128 rows (fwd_small_tiles below) are not among
 // what is compared: they are asked about where this rule leaves the tiles whole.
@@ -598,7 +601,7 @@ FwdPlan fwd_plan(int dtype, const Shape& s, int causal_type, int window_left, in
     most = n > most ? n : most;
     sum += n;
   }
-  const double t64 = s.d == 64 ? 1.2 : s.d == 128 ? 1.9 : 2.4;
+  const double t64 = s.d == 64 ? 1.2 : 1.9, around = s.d > 128 ? 7 : 6;
   auto tile_time = [&](int64_t parts) {
     const double rounds = (double)((tiles * parts + num_cu - 1) / num_cu);
     // tiles of about the same weight go in whole rounds, uneven ones fill each other's gaps
@@ -606,7 +609,7 @@ FwdPlan fwd_plan(int dtype, const Shape& s, int causal_type, int window_left, in
                         (sum * 5 > most * m_tiles * 4 ? rounds * num_cu / (double)(tiles * parts) : 1.0);
     const double longest = (double)((most + parts - 1) / parts);
     const double busy = tiles * parts < num_cu ? (double)(tiles * parts) / num_cu : 1.0;
-    return (even > longest ? even : longest) * t64 * (0.75 + 0.25 * busy) + 6 * rounds +
+    return (even > longest ? even : longest) * t64 * (0.75 + 0.25 * busy) + around * rounds +
            (parts > 1 ? 5 + 0.07 * wide * tiles * parts : 0.0);
   };
   const double whole = tile_time(1);
@@ -624,8 +627,8 @@ FwdPlan fwd_plan(int dtype, const Shape& s, int causal_type, int window_left, in
   const double steps = (double)((blocks + 4 * splits - 1) / (4 * splits));
   const int64_t slots = (s.d > 128 ? 1 : 2) * num_cu, row_rounds = (items * splits + slots - 1) / slots;
   const double per_cu = s.d > 128 ? (double)row_rounds : (double)(items * splits) / num_cu;
-  const double t128 = s.d == 64 ? 0.9 : s.d == 128 ? 1.2 : 2.6;
-  const double rows_time = (per_cu > 1 ? per_cu : 1) * steps * t128 + 4 * (double)row_rounds + 1 + (splits > 1 ? 4 : 0);
+  const double t128 = s.d == 64 ? 0.9 : s.d == 128 ? 1.2 : 2.6, rows_around = s.d > 128 && rows > 32 ? 7.2 : 4;
+  const double rows_time = (per_cu > 1 ? per_cu : 1) * steps * t128 + rows_around * (double)row_rounds + 1 + (splits > 1 ? 4 : 0);
   // The row blocks of a (pair, part) run on one XCD (fwd_rows_kernel), so with fewer than eight of those, or a few more
   // than a multiple of eight, the busiest XCD has more than its share; with many row blocks that decides.  There the
   // blocks take the average tile's keys, and the rows kernel is refused where that is slower than whole tiles (us, whole tiles
@@ -637,13 +640,9 @@ FwdPlan fwd_plan(int dtype, const Shape& s, int causal_type, int window_left, in
   const int64_t busy_rounds = (busiest + slots / num_cu * cus - 1) / (slots / num_cu * cus);
   const double average = most > 0 ? (double)sum / ((double)most * m_tiles) : 1.0;
   const double load = average * (s.d > 128 ? (double)busy_rounds : (double)busiest / cus);
-  const double busy_time = (load > 1 ? load : 1) * steps * t128 + 4 * (double)busy_rounds + 1 + (splits > 1 ? 4 : 0);
+  const double busy_time = (load > 1 ? load : 1) * steps * t128 + rows_around * (double)busy_rounds + 1 + (splits > 1 ? 4 : 0);
   // (the lines: D = 128 and 256 level at 1.1 of these figures, D = 64, whose steps take 0.55 us on two XCDs, at 1.7)
-  // (D = 256 with more than one row block: its tiles take less than t64 says where a round of them is short.  us, rows / tiles: on the rows' side of
-  // the line 16 heads 256 x 1024 28 / 32, 32 heads 128 x 2000 37 / 54, 4 x 16 heads 128 x 1000 31 / 33; on the other Hq 8 Hk 2 512 causal 32 / 21, 256 causal
-  // 18.6 / 15.8, 8 x 16 heads 64 x 300 19 / 16, 4 x 8 heads 64 x 200 17 / 13, 4 x 16 heads 60 x 60 12.1 / 10.7; one query is never slower in rows)
-  const double line = s.d == 64 ? 1.75 : s.d == 128 || rows <= 32 ? 1.08 : 0.75;
-  r.rows = rows_time < (s.d > 128 && rows > 32 ? 0.75 : 1.0) * best && busy_time <= line * whole;
+  r.rows = rows_time < best && busy_time <= (s.d == 64 ? 1.75 : 1.08) * whole;
   int64_t stored;
   if (r.rows) {
     r.splits = (int)splits;

@@ -230,3 +230,14 @@ def test_a_caller_may_name_any_longest_sequence(causal):
         for longest in (1 << 24, 1 << 30, (1 << 31) - 200, (1 << 31) - 1):
             c = packed(slot, lens, lens, 16, 8, 128, causal, longest)
             assert (c.block_m, c.block_n) in ((m, n), (64, 128) if slot == 1 else (128, 64))
+
+
+@pytest.mark.parametrize('call, rows', [
+    ((5, 24, 8, 24, 108, 256), False), ((3, 24, 8, 75, 230, 256), False), ((1, 32, 8, 200, 200, 256), False), ((2, 16, 16, 200, 200, 256), False),
+    ((1, 24, 8, 227, 247, 256), False), ((1, 32, 8, 64, 64, 256, True), False), ((2, 16, 16, 34, 477, 256), True), ((2, 4, 4, 209, 1204, 256), True),
+    ((4, 12, 12, 51, 1968, 256), True), ((1, 8, 2, 256, 4096, 256), True), ((1, 32, 8, 1, 300, 256), True), ((6, 64, 8, 6, 6, 256, True), True),
+])
+def test_packed_rows_at_head_dim_256_where_they_are_sooner(call, rows):
+    """us, rows / tiles: 12.5 / 10.3, 16.0 / 13.8, 15.6 / 13.9, 15.7 / 14.0, 16.1 / 15.3, 11.2 / 9.9; 17.1 / 18.7, 23.5 / 35.2, 34 / 53, 37 / 101,
+    12.0 / 13.7, 10.3 / 14.5"""
+    assert bool(fwd(*call).flags & 128) == rows
