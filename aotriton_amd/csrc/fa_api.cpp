@@ -411,6 +411,13 @@ fa::SeqArgs seq_args(const Shape& s, const fa_tensor1& cu_q, const fa_tensor1& c
   return r;
 }
 
+void bias_args(const fa_bwd_params& p, const Shape& s, fa::BwdArgs* a) {
+  a->bias = p.B.ptr;
+  if (!s.bias) return;
+  a->sb_z = (int64_t)p.B.strides[0]; a->sb_h = (int64_t)p.B.strides[1];
+  a->sb_m = (int64_t)p.B.strides[2]; a->sb_n = (int64_t)p.B.strides[3];
+}
+
 int validate_fwd(const fa_fwd_params* p, int32_t version, const fa_options* opt, Shape* shape) {
   if (p == nullptr) return FA_ERROR_INVALID_VALUE;
   if (version != FA_FWD_PARAMS_VERSION) return FA_ERROR_INVALID_SYMBOL;   // attn_fwd.cc:53-55
@@ -1157,9 +1164,10 @@ int fa_query_bwd_config(const fa_bwd_params* params, const fa_options* options, 
     fit_workspace(room, &need, &parts);
   }
   const bool wide_dkdv = route.wide_dkdv && need == 0 && parts.bytes == 0;
-  const bool pair_dkdv = s.d == 256 && need > 0 &&
-                         (!s.bias || (s.max_sk % 8 == 0 && fa::bias_aligned(params->B.ptr, params->B.strides[0], params->B.strides[1],
-                                                                            params->B.strides[2], params->B.strides[3])));
+  fa::BwdArgs a{};
+  bias_args(*params, s, &a);
+  a.seq = seq_args(s, params->cu_seqlens_q, params->cu_seqlens_k, params->seq_strides_q, params->seq_strides_k, params->varlen_type);
+  const bool pair_dkdv = fa::bwd_dkdv_by_pairs(a, s.d, s.bias, need > 0);
   const fa::TileShape t = rows32 ? fa::f32_rows_tile_shape(s.d)
                           : f32_mfma ? fa::f32_tile_shape(s.d, kernel_slot)
                           : split_d ? fa::d512_tile_shape(kernel_slot)
@@ -1481,16 +1489,13 @@ static int attn_bwd_impl(const fa_bwd_params* p_in, int32_t params_version, void
   }
 
   fa::BwdArgs a{};
-  a.q = p->Q.ptr; a.k = p->K.ptr; a.v = p->V.ptr; a.bias = p->B.ptr;
+  a.q = p->Q.ptr; a.k = p->K.ptr; a.v = p->V.ptr;
+  bias_args(*p, s, &a);
   a.out = p->Out.ptr; a.dout = p->DO.ptr;
   a.dq = p->DQ.ptr; a.dk = p->DK.ptr; a.dv = p->DV.ptr; a.db = p->DB.ptr;
   a.lse = static_cast<const float*>(p->L.ptr);
   a.sq = strides3(p->Q); a.sk = strides3(p->K); a.sv = strides3(p->V); a.so = strides3(p->Out);
   a.sdo = strides3(p->DO); a.sdq = strides3(p->DQ); a.sdk = strides3(p->DK); a.sdv = strides3(p->DV);
-  if (s.bias) {
-    a.sb_z = (int64_t)p->B.strides[0]; a.sb_h = (int64_t)p->B.strides[1];
-    a.sb_m = (int64_t)p->B.strides[2]; a.sb_n = (int64_t)p->B.strides[3];
-  }
   if (p->DB.ptr != nullptr) {
     a.sdb_z = (int64_t)p->DB.strides[0]; a.sdb_h = (int64_t)p->DB.strides[1];
     a.sdb_m = (int64_t)p->DB.strides[2]; a.sdb_n = (int64_t)p->DB.strides[3];
@@ -1592,7 +1597,7 @@ static int attn_bwd_impl(const fa_bwd_params* p_in, int32_t params_version, void
         a.walk_group = route.group_dkdv;
         return fa::run_bwd_dkdv_wide(dt, a, s.windowed, stream);
       }
-      if (a.ds_ws != nullptr && s.d == 256 && (!s.bias || fa::plain_bias(a)))
+      if (fa::bwd_dkdv_by_pairs(a, s.d, s.bias, a.ds_ws != nullptr))
         return fa::run_bwd_dkdv_pair(dt, a, s.windowed, s.bias, s.dropout, stream);
       return (cut ? fa::run_bwd_dkdv_parts : fa::run_bwd_dkdv)(dt, s.d, a, s.windowed, s.bias, s.dropout, stream);
     };

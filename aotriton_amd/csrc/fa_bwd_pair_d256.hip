@@ -6,9 +6,7 @@
 #ifndef FA_PADDED
 #define FA_PADDED 0
 #endif
-#if FA_PADDED == 96
-#define FA_RUN run_bwd_dkdv_pair_d256_cols96
-#elif FA_PADDED
+#if FA_PADDED
 #define FA_RUN run_bwd_dkdv_pair_d256_padded
 #else
 #define FA_RUN run_bwd_dkdv_pair_d256

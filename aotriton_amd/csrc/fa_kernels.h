@@ -59,6 +59,9 @@ inline bool plain_bias(const BwdArgs& a) {
 }
 // The same for items that store dS at head dims above 128, whole or in parts, without a bias or with a plain one: pairs of waves
 // (fa_bwd_pair.h).
+inline bool bwd_dkdv_by_pairs(const BwdArgs& a, int head_dim, bool bias, bool stored_ds) {
+  return stored_ds && head_dim == 256 && (!bias || plain_bias(a));
+}
 hipError_t run_bwd_dkdv_pair(int dtype, const BwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);
 TileShape bwd_pair_shape(bool bias);
 hipError_t run_bwd_dq(int dtype, int head_dim, const BwdArgs& a, bool windowed, bool bias, bool dropout, hipStream_t s);

@@ -241,3 +241,30 @@ def test_packed_rows_at_head_dim_256_where_they_are_sooner(call, rows):
     """us, rows / tiles: 12.5 / 10.3, 16.0 / 13.8, 15.6 / 13.9, 15.7 / 14.0, 16.1 / 15.3, 11.2 / 9.9; 17.1 / 18.7, 23.5 / 35.2, 34 / 53, 37 / 101,
     12.0 / 13.7, 10.3 / 14.5"""
     assert bool(fwd(*call).flags & 128) == rows
+
+
+def _rows(Sk, start=0, apart=1):
+    """strides of a (2, 4, 300, Sk) bias whose rows are `Sk + start` long and whose columns are `apart` apart"""
+    row = (Sk + start) * apart
+    return (4 * 300 * row, 300 * row, row, apart)
+
+
+@pytest.mark.parametrize('Sk, D, bias, at, pairs', [
+    (264, 256, False, 0, True), (131, 256, False, 0, True), (264, 136, False, 0, True), (264, 128, False, 0, False),
+    (264, 256, _rows(264), 0, True), (264, 256, _rows(264), 16, True), (264, 200, _rows(264, 8), 0, True), (264, 256, (0, 0, 0, 1), 0, True),
+    (264, 256, _rows(264), 2, False), (264, 256, _rows(264, 1), 0, False), (260, 256, _rows(260, 4), 0, False), (264, 256, _rows(264, 0, 2), 0, False),
+    (264, 128, _rows(264), 0, False),
+])
+def test_dkdv_by_pairs_of_waves(Sk, D, bias, at, pairs):
+    """head dims above 128 that store dS, without a bias or with one whose rows are whole 16-byte pieces at such places; never recomputing or for
+    packed sequences"""
+    from aotriton_amd._lib import lib
+    shape = lambda c: (c.block_m, c.block_n, c.num_waves)
+    assert (shape(bwd(1, 2, 4, 4, 300, Sk, D, bias=bias, at=at)) == (32, 128, 8)) == pairs
+    lib.fa_set_bwd_workspace_limit(0)
+    try:
+        assert shape(bwd(1, 2, 4, 4, 300, Sk, D, bias=bias, at=at)) != (32, 128, 8)
+    finally:
+        lib.fa_set_bwd_workspace_limit(-1)
+    if not bias:
+        assert packed(1, [100, 200], [100, 200], 4, 4, D).num_waves == 4
