@@ -210,3 +210,32 @@ def test_rows_that_a_bias_hides(D, Sk):
     x = [t.clone().requires_grad_() for t in (q, k, v)]
     attention(*x, b, False, 1 / math.sqrt(D), 0.0)[0].backward(do)
     assert all(torch.isfinite(t.grad).all() for t in x)
+
+
+@pytest.mark.parametrize('D', [64, 96, 128, 200, 256])
+@pytest.mark.parametrize('Sk,dt,causal,p', [(136, BF, False, 0.0), (131, HF, False, 0.0), (264, HF, (150, 30), 0.0), (259, BF, True, 0.2), (136, HF, False, 0.2)])
+def test_gradients_of_rows_that_a_bias_hides(D, Sk, dt, causal, p):
+    """dS is stored.  A row's softmax does not change with a constant in its bias, so such rows have the gradients of a bias of zero; -256 is
+    enough for what stands for keys past the sequence to overflow, and exact in 16 bits (it costs the exponents 2^-16)."""
+    from aotriton_amd import flash
+    from aotriton_amd.autograd import attention, AttentionExtraArgs
+    from oracle import fa_ref
+    from _util import FUDGE, check, keep_mask_from_oracle
+    B, H, Sq = 1, 4, 300
+    q, k, v, b, do = make_inputs(B, H, H, Sq, Sk, D, dt, 'cuda', seed=4, bias=True)
+    b = b.contiguous()
+    assert bwd(1, B, H, H, Sq, Sk, D, causal, p, bias=tuple(b.stride())).flags & 16
+    hidden, zero = b.clone(), b.clone()
+    hidden[:, :, ::2], zero[:, :, ::2] = -256, 0
+    sm, ext = 1 / math.sqrt(D), AttentionExtraArgs(return_logsumexp=True, fillnan=True)
+    x = [t.clone().requires_grad_() for t in (q, k, v)]
+    attention(*x, hidden, causal, sm, p, ext)[0].backward(do)
+    ct, wl, wr = flash.translate_causal(causal)
+    keep = keep_mask_from_oracle(B, H, Sq, Sk, p, ext.philox_seed, ext.philox_offset1 + ext.philox_offset2, 'cuda')
+    f = lambda t: t.float()
+    ro, rl, _ = fa_ref.attn_fwd_ref(f(q), f(k), f(v), f(zero), sm, ct, wl, wr, p, keep)
+    lo, ll, _ = fa_ref.attn_fwd_ref(q, k, v, zero, sm, ct, wl, wr, p, keep)
+    rg = fa_ref.attn_bwd_ref(f(q), f(k), f(v), f(zero), sm, ro, f(do), rl, ct, wl, wr, p, keep)
+    lg = fa_ref.attn_bwd_ref(q, k, v, zero, sm, lo, do, ll.to(dt).float().to(dt), ct, wl, wr, p, keep)
+    for i, n in enumerate(('dq', 'dk', 'dv')):
+        check(n, x[i].grad, rg[i], lg[i], FUDGE[n])
