@@ -832,11 +832,10 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
   // Per q-head the Q tiles come as [masked | full | masked]; each run has its own
   // loop so that the loop bodies are straight-line code.
   const int fb_lo = kParts && br.fb_lo < br.lo ? br.lo : br.fb_lo, fb_hi = kParts && br.fb_hi > br.hi ? br.hi : br.fb_hi;
-  // (Lanes whose key is past the sequence hold nothing that a result needs, but their dS is stored, and the dQ kernel multiplies it by
-  // zero: with a bias that hides a row by a large number their P overflows.  Such tiles are all masked.)
-  const bool whole = fb_lo <= fb_hi && !(kBias && kStoreDs && n0 + BN > si.seqlen_k);
-  const int n_lb = whole ? fb_lo - br.lo : ntq;
-  const int n_fb = whole ? fb_hi - fb_lo + 1 : 0;
+  // (Lanes whose key is past the sequence hold nothing that a result needs: with a bias that hides a row by a large number their P
+  // overflows.  Their dS is stored all the same; the dQ kernel clears it.)
+  const int n_lb = fb_lo <= fb_hi ? fb_lo - br.lo : ntq;
+  const int n_fb = fb_lo <= fb_hi ? fb_hi - fb_lo + 1 : 0;
   int it = 0;
   int g_cur = g_lo, e_cur = 0;
   auto step = [&](auto masked_tag) {
