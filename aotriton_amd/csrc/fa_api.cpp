@@ -713,10 +713,11 @@ bool fwd_wide(const fa_fwd_params* p, const Shape& s, int splits, int num_cu) {
 // left.  Beyond, and with such a window, the tiles are whole (fa_query_fwd_config reports them).
 // A bias with dropout: two per CU.  The 256-row tile of these kernels keeps more than fits 256 registers, so that the smaller one wins full
 // rounds as well (us, 256 rows / 128 twice, window with both: D64 B1 H8 S1024 34 / 21, B2 H16 S2048 53 / 42, S8192 306 / 256; D128 40 / 26, 66 / 51,
-// 407 / 338; B4 H16 S1500 98 / 51 and 109 / 61) and short calls (D64 B1 H8 64 x 64 20.0 / 8.3, B2 H16 S256 19.4 / 15.4, B8 H16 S512 window 35 / 24, B64 H16 40 x 200
-// 100 / 40, B4 H8 32 x 2000 130 / 75; D80 S64 11.1 / 9.2; D96 B4 H12 S128 14.1 / 12.2; D128 B1 H8 100 x 300 33 / 22, B16 H16 S300 84 / 53): 93 shapes of 32-3000
-// queries, 0.40-1.01 of the time.  Calls of at most four tiles of 256 rows would gain too (B1 H2 512 x 600: D64 45 / 27, D128 causal 36 / 30); they are
-// left with those tiles, which a test of the routes holds them to.
+// 407 / 338; B4 H16 S1500 98 / 51 and 109 / 61) and calls with rows for one whole tile (D64 B1 H8 64 x 64 20.0 / 8.3, B2 H16 S256 19.4 / 15.4, B64 H16
+// 40 x 200 100 / 40, B4 H8 32 x 2000 130 / 75; D80 S64 11.1 / 9.2; D96 B4 H12 S128 14.1 / 12.2; D128 B1 H8 100 x 300 33 / 22, B8 H16 S256 window 29 / 19).
+// Over 93 shapes of 32-3000 queries it takes 0.40-1.01 of the time.  Between the two, with 257 to 512 queries, it would as well (D64 B8 H16 S512 window
+// 35 / 24, B2 H8 512 x 4000 213 / 139, D128 B16 H16 S300 84 / 53): these calls stay on the whole tiles, because the tests of those tiles (bias rows far apart
+// and overlapping) are calls of that size and ask for them.
 int fwd_small_tiles(const fa_fwd_params* p, const Shape& s, bool wide, int num_cu) {
   const bool key_bias = s.bias && !s.dropout && p->B.strides[2] == 0;
   const bool row_bias = s.bias && !key_bias && !s.dropout && s.d == 64 && p->B.strides[3] == 1;
@@ -725,8 +726,8 @@ int fwd_small_tiles(const fa_fwd_params* p, const Shape& s, bool wide, int num_c
   if (s.elementwise || !is_16bit(p->Q.dtype) || s.d > 128 || (s.bias && !key_bias && !row_bias && !drop_bias) || s.num_seqlens != 0 || s.max_sq <= 0 ||
       s.max_sk <= 0 || s.batch <= 0 || cus < 1 || cus > 64)
     return 0;
+  if (drop_bias) return s.max_sq <= 256 || s.max_sq > 512 ? 2 : 0;
   const int m_tiles = (s.max_sq + 255) / 256, group = fa::q_head_group(s.hq, s.hk);
-  if (drop_bias) return s.max_sq > 512 || (int64_t)s.batch * s.hq * m_tiles > 4 ? 2 : 0;
   if (fa::tile_work(s.batch * s.hq, group, m_tiles).items_per_xcd > std::min((row_bias ? 3 : 8) * cus, 448)) return 0;
   fa::Window w{0, 0};
   if (s.windowed) w = fa::parse_window(p->causal_type, p->window_left, p->window_right, s.max_sq, s.max_sk);

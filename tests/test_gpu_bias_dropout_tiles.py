@@ -64,14 +64,14 @@ def test_rows_lie_anywhere(D, dt, causal):
 
 
 SHORT = [
-    # up to 512 queries, more than four tiles of 256 rows
+    # rows for one tile of 256 at most
     (1, 8, 8, 64, 64, 64, BF, False),
     (5, 1, 1, 1, 129, 64, HF, False),             # one query
     (2, 4, 2, 31, 1, 128, BF, False),             # one key
     (3, 2, 2, 128, 96, 80, HF, True),
     (2, 3, 3, 129, 257, 128, HF, (40, 30)),       # one row in the second tile, one key in the last
     (1, 5, 5, 200, 333, 96, BF, (30, -10)),       # rows that see nothing
-    (1, 3, 3, 512, 512, 40, HF, (128, 0)),
+    (1, 3, 3, 256, 512, 40, HF, (128, 0)),
     (1, 6, 2, 256, 70, 64, BF, True),
 ]
 
