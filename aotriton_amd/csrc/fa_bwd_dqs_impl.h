@@ -15,7 +15,7 @@
 // B1 H8 D128 19.3 -> 17.7, B8 H12 S512 D64 with dB 26.6 -> 25.2; window of 1024, B2 H16 S8192 D256 246 -> 230.  What is slower that way: at D = 64 with dB
 // where each CU has one workgroup of four steps, two of which are requested at once instead of all, 4000 x 200 17.7 -> 21.2, 4000 x 256 17.8 -> 19.3,
 // B16 H16 S256 17.8 -> 18.9; D256 B2 H16 S4096 causal 182 -> 187.  Four stages: those 20.2, 17.9, 17.7 and 189, but 1-4 % more for other calls with dB; two
-// stages: 1-2 % slower.  Waits that count the stores of dB as well: level.)
+// stages: 1-2 % slower.)
 //
 // Keys per step at 128 columns: 64 with dB and where there are fewer workgroups than CUs, else 32.  A step has a barrier and a chain of LDS reads, with dB a
 // turn through LDS as well, which a CU's only workgroup waits out; steps of 32 take half the LDS, so that a CU holds two workgroups.  us, 32 / 64 keys: with dB

@@ -19,7 +19,8 @@
 // each next to the other wave) are longer than that: with all four in the second wave its step takes 2800 and the first one's 2000; two each, us, window
 // S1801 38.5 -> 37.4, S8192 571 -> 562 (one card; long calls run at the clock that the power leaves, and moving work between the waves gives them less).
 // Level or slower: more operands in flight, wave priorities, the first operands of the next unit read in front of the barrier (a stage
-// more of K), the second waves over 64 columns of all rows (less LDS traffic, 5-8 % slower).
+// more of K), the second waves over 64 columns of all rows (less LDS traffic, 5-8 % slower), the first product of Philox round 2, which the counter's upper
+// word alone decides, kept along a row (19 registers more; S8192 529 -> 525, S4096 causal 365 -> 373).
 //
 // Measured, us, one wave per SIMD with all of it interleaved -> this, one card: B2 H16 S8192 fp16 window 1024, bias and dropout 618 -> 530, B1 H8 S1801
 // 52 -> 38; B2 H16 S4096 with a bias 728 -> 576 (755 -> 955 TFLOP/s); B1 H16 Hk4 S8192 bf16 causal 716 -> 576, B2 S2048 96 -> 77.
