@@ -13,13 +13,13 @@
 // K and dS go straight into LDS, two steps ahead, counted by hand.  (Through registers, K a step and dS four steps ahead, a wait for
 // K was one for every dS requested before it: memory answers in order.  us, before -> this: 1000 x 1531 D80 43 -> 39, window of 450 of 1801 keys
 // B1 H8 D128 19.3 -> 17.7, B8 H12 S512 D64 with dB 26.6 -> 25.2; window of 1024, B2 H16 S8192 D256 246 -> 230.  What is slower that way: at D = 64 with dB
-// where each CU has one workgroup of four steps, two of which are requested at once instead of all, 4000 x 200 17.7 -> 21.2, 4000 x 256 17.8 -> 19.3,
-// B16 H16 S256 17.8 -> 18.9; D256 B2 H16 S4096 causal 182 -> 187.  Four stages: those 20.2, 17.9, 17.7 and 189, but 1-4 % more for other calls with dB; two
-// stages: 1-2 % slower.)
+// where each CU has one workgroup of four steps, two of which are requested at once instead of all, 4000 x 200 17.8 -> 19.5, 4000 x 256 17.8 -> 19.5,
+// B16 H16 S256 17.8 -> 18.8; D256 B2 H16 S4096 causal 181 -> 185.  Four stages: 4000 x 256 17.9, B16 H16 S256 17.7, D256 189, but 1-4 % more for other calls
+// with dB; two stages: 1-2 % slower.)
 //
 // Keys per step at 128 columns: 64 with dB and where there are fewer workgroups than CUs, else 32.  A step has a barrier and a chain of LDS reads, with dB a
 // turn through LDS as well, which a CU's only workgroup waits out; steps of 32 take half the LDS, so that a CU holds two workgroups.  us, 32 / 64 keys: with dB
-// B2 H8 200 x 4000 113 / 91 (D80 108 / 87), B1 H8 S4096 causal 155 / 134, B2 H16 S2048 causal 102 / 86, B8 H16 S1024 119 / 108, B16 H16 S256 22.9 / 21.7; without,
+// B2 H8 200 x 4000 113 / 91-95 (D80 108 / 87-88), B1 H8 S4096 causal 155 / 134, B2 H16 S2048 causal 102 / 86, B8 H16 S1024 119 / 108, B16 H16 S256 22.9 / 21.7; without,
 // dropout: B1 H8 64 x 2000 26.8 / 22.0, B2 H8 200 x 4000 69 / 58.7, B1 H16 S2048 D80 causal 34.3 / 31.1, B3 H16 1000 x 1531 39.5 / 36.7; from a workgroup per CU
 // on B64 H16 S128 D96 26.9 / 28.1, B32 H16 S128 17.2 / 18.0, B4 H16 1000 x 1531 43-54 / 43-57, B5 H16 with a bias 74-79 / 78-82.
 //
@@ -145,11 +145,15 @@ __device__ __forceinline__ void dqs_item(const BwdArgs& a, const int h, const in
     const int k_voff = gch * 8 < d_qk ? r0 * k_row + gch * 16 : kVoffOutOfRange;
     const char* ws_head = reinterpret_cast<const char*>(a.ds_ws) +
                           ((int64_t)z * a.hq + h) * a.ds_ntk * (int64_t)a.ds_ntq * DT::BYTES;
-    const int ds_voff = lane * 16 + qb * DT::QBLOCK_BYTES;
+    // What is stored for keys past the sequence may be infinite or NaN (dkdv_item), and K is zero there: the lanes whose piece is of such a key, piece
+    // (2 c + hi) ^ 8 (t & 1) of each KB, bring zeros.  (Masking such tiles in dK/dV instead costs 2-6 % of that kernel: us, B16 H16 300 x 131 D64 with a
+    // bias 33.5 -> 35.2, B4 H16 1000 x 1531 D80 with dropout 248 -> 258, Hq 64 Hk 8 5000 x 130 D160 280 -> 296.  Asked in every step it costs this kernel
+    // 2-5 %; hence a loop of their own for the last steps.)
+    const int ds_voff = lane * 16 + qb * DT::QBLOCK_BYTES, ds_key[2] = {lane >> 1, (lane ^ 8) >> 1};
     const int smem0 = lds_offset(smem_raw);
     constexpr int LOADS = CH + NCK;          // per wave and step
     int f_j = j0, f_stage = 0;
-    auto fetch = [&]() __attribute__((always_inline)) {
+    auto fetch = [&](auto may_be_last) __attribute__((always_inline)) {
       int rows = si.seqlen_k - f_j * BN;
       rows = rows < BN ? rows : BN;
       rows = f_j <= j1 ? rows : 0;
@@ -162,7 +166,11 @@ __device__ __forceinline__ void dqs_item(const BwdArgs& a, const int h, const in
       const auto rs = wave_rsrc_words(ws_head + ((int64_t)nt * a.ds_ntq + pm) * DT::BYTES, active(f_j) ? DT::BYTES : 0);
       const int ds_at = smem0 + SM::DS_OFF + f_stage * SM::DS_STAGE + wave_u * SM::DS_WAVE;
 #pragma unroll
-      for (int i = 0; i < NCK; i += 2) load_to_lds_once(rs, ds_voff, from + i * 1024, ds_at + i * 1024);
+      for (int i = 0; i < NCK; i += 2) {
+        const int left = si.seqlen_k - f_j * BN - i * 16;
+        load_to_lds_once(rs, !may_be_last || ds_key[0] < left ? ds_voff : kVoffOutOfRange, !may_be_last || ds_key[1] < left ? ds_voff : kVoffOutOfRange,
+                         from + i * 1024, ds_at + i * 1024);
+      }
       ++f_j;
       f_stage = f_stage == S - 1 ? 0 : f_stage + 1;
     };
@@ -175,33 +183,23 @@ __device__ __forceinline__ void dqs_item(const BwdArgs& a, const int h, const in
 
     int stage = 0;
 #pragma unroll
-    for (int i = 0; i < S - 1; ++i) fetch();
-#pragma nounroll
-    for (int j = j0; j <= j1; ++j) {
+    for (int i = 0; i < S - 1; ++i) fetch(std::true_type{});
+    auto step = [&](auto may_be_last, int j) __attribute__((always_inline)) {
       // This wave's part of the step has arrived (what was requested for later ones may be under way; stores of dB, which come between, only make the
       // wait longer) and then everybody's, and everybody has left the stage that is filled next.
       asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"((S - 2) * LOADS) : "memory");
-      fetch();
+      fetch(may_be_last);
       char* const ds_area = smem_raw + SM::DS_OFF + stage * SM::DS_STAGE + wave_u * SM::DS_WAVE;
       const bool act = active(j);
       if (act) {
         const char* Kb = smem_raw + stage * SM::K_BYTES;
-        // What is stored for keys past the sequence may be infinite or NaN (dkdv_item); here K is zero there.  (Masking such tiles in dK/dV
-        // instead costs 2-6 % of that kernel: us, B16 H16 300 x 131 D64 with a bias 33.5 -> 35.2, B4 H16 1000 x 1531 D80 with dropout 248 -> 258, Hq 64 Hk 8
-        // 5000 x 130 D160 280 -> 296; the test here is 0-0.5 us.)
-        const int left = si.seqlen_k - j * BN;
         op_t bs[kDb ? BN / 16 : 1];
 #pragma unroll
         for (int tk = 0; tk < BN / 16; ++tk) {
           const char* p = ds_area + ds_rd + (tk >> 1) * 2048 + (tk & 1) * 512;
           const q4_t lo = Tr::lds_read_tr(reinterpret_cast<const T*>(p));
           const q4_t up = Tr::lds_read_tr(reinterpret_cast<const T*>(p + 256));
-          op_t b = __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7);
-          if (left < BN) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-              if (16 * tk + 4 * hi + 8 * (e / 4) + e % 4 >= left) b[e] = 0;
-          }
+          const op_t b = __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7);
           if constexpr (kDb) bs[tk] = b;
 #pragma unroll
           for (int db = 0; db < DB; ++db) dq[db] = Tr::mfma(swz_read_tr<T, D>(Kb, tr_a0, tr_a1, tk, db), b, dq[db]);
@@ -223,7 +221,12 @@ __device__ __forceinline__ void dqs_item(const BwdArgs& a, const int h, const in
         }
       }
       stage = stage == S - 1 ? 0 : stage + 1;
-    }
+    };
+    int j = j0;
+#pragma nounroll
+    for (; j + S - 1 < j1; ++j) step(std::false_type{}, j);
+#pragma nounroll
+    for (; j <= j1; ++j) step(std::true_type{}, j);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // (LDS belongs to the workgroup no longer than it runs)
   }
 

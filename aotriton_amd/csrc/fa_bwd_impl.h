@@ -833,7 +833,7 @@ __device__ __forceinline__ void dkdv_item(const BwdArgs& a, const int hk, const 
   // loop so that the loop bodies are straight-line code.
   const int fb_lo = kParts && br.fb_lo < br.lo ? br.lo : br.fb_lo, fb_hi = kParts && br.fb_hi > br.hi ? br.hi : br.fb_hi;
   // (Lanes whose key is past the sequence hold nothing that a result needs: with a bias that hides a row by a large number their P
-  // overflows.  Their dS is stored all the same; the dQ kernel clears it.)
+  // overflows.  Their dS is stored all the same; the dQ kernel does not read it.)
   const int n_lb = fb_lo <= fb_hi ? fb_lo - br.lo : ntq;
   const int n_fb = fb_lo <= fb_hi ? fb_hi - fb_lo + 1 : 0;
   int it = 0;

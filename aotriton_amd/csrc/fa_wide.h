@@ -69,10 +69,10 @@ __device__ __forceinline__ void load_to_lds1(u32x4_t rsrc, int voff, int lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" :: "s"(lds), "v"(voff), "s"(rsrc) : "m0");
 }
 // Two consecutive KB that nobody reads again.
-__device__ __forceinline__ void load_to_lds_once(u32x4_t rsrc, int voff, int soff, int lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %2, %3, %4 offen nt lds\n\t"
-               "s_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, %5 offen nt lds"
-               :: "s"(lds), "s"(lds + 1024), "v"(voff), "s"(rsrc), "s"(soff), "s"(soff + 1024) : "m0");
+__device__ __forceinline__ void load_to_lds_once(u32x4_t rsrc, int voff0, int voff1, int soff, int lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %2, %4, %5 offen nt lds\n\t"
+               "s_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %3, %4, %6 offen nt lds"
+               :: "s"(lds), "s"(lds + 1024), "v"(voff0), "v"(voff1), "s"(rsrc), "s"(soff), "s"(soff + 1024) : "m0");
 }
 // Accesses i and i + 1 of the 16 that bring a wave's 64 rows of 128 columns into LDS (swizzled; a lane's row of access 0 is `voff`
 // bytes from the first, the rows of two accesses `step` apart; chunks past column d are zero).
